@@ -360,6 +360,18 @@ int yvex_hip_memcpy_h2d(void *dst, const void *src, uint64_t bytes, yvex_hip_str
  * (yvex_hip_host_alloc) that stays untouched until the stream has passed the copy. */
 int yvex_hip_memcpy_h2d_queued(void *dst, const void *src, uint64_t bytes, yvex_hip_stream stream);
 int yvex_hip_memcpy_d2h(void *dst, const void *src, uint64_t bytes, yvex_hip_stream stream);
+/* The end of a synchronous operation: `publish` enqueues one small launch that writes `bytes` of
+ * device results (a multiple of 4, at most YVEX_HIP_PUBLISH_MAX_BYTES, may be 0) behind the first
+ * YVEX_HIP_PUBLISH_HEAD_BYTES of `host`, the status word into its second word and `sequence` into its
+ * first, and with `clear` resets a raised status word; `await` waits for that sequence number and
+ * returns the status word. `host` is pinned (yvex_hip_host_alloc), 64-byte aligned, and serves one
+ * stream; sequence numbers of successive calls differ. A wait of more than 20 ms turns into a
+ * stream synchronisation. */
+#define YVEX_HIP_PUBLISH_HEAD_BYTES 64u
+#define YVEX_HIP_PUBLISH_MAX_BYTES 65536u
+int yvex_hip_publish(const void *source, uint64_t bytes, int *status, int clear, void *host, uint32_t sequence,
+                     yvex_hip_stream stream);
+int yvex_hip_await(const void *host, uint32_t sequence, int *status, yvex_hip_stream stream);
 int yvex_hip_memcpy_d2d(void *dst, const void *src, uint64_t bytes, yvex_hip_stream stream);
 int yvex_hip_stream_create(yvex_hip_stream *out);
 int yvex_hip_stream_destroy(yvex_hip_stream stream);

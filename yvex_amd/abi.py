@@ -314,7 +314,7 @@ KERNEL_EXPORTS = [
     "yvex_hip_device_count", "yvex_hip_device_info", "yvex_hip_device_clocks", "yvex_hip_malloc", "yvex_hip_free",
     "yvex_hip_host_alloc", "yvex_hip_host_free", "yvex_hip_memcpy_h2d", "yvex_hip_memcpy_h2d_queued", "yvex_hip_memcpy_d2h",
     "yvex_hip_memcpy_d2d", "yvex_hip_stream_create", "yvex_hip_stream_destroy",
-    "yvex_hip_stream_sync", "yvex_hip_kernels_loadable", "yvex_hip_last_error",
+    "yvex_hip_stream_sync", "yvex_hip_publish", "yvex_hip_await", "yvex_hip_kernels_loadable", "yvex_hip_last_error",
 ]
 
 

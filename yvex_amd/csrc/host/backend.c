@@ -64,24 +64,51 @@ int yvex_rocm_status_reset(yvex_rocm_backend *backend, const char *where, yvex_e
     /* row batches whose completion is deferred own the word until their barrier: an operation
      * that runs between them must not erase what they raised (it then reports it as its own) */
     if (backend->pending_completion) return YVEX_OK;
+    if (backend->status_clean) {
+        backend->status_clean = 0;     /* until the operation has been waited for */
+        return YVEX_OK;
+    }
     return yvex_rocm_launch_result(yvex_hip_fill_u32(backend->device_status, 0u, 1u, backend->stream),
                                    where, err);
 }
 
-int yvex_rocm_finish(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err)
+static int finish(yvex_rocm_backend *backend, unsigned long long device_results, unsigned long long bytes,
+                  const unsigned char **results, int clear, const char *where, int *device_status, yvex_error *err)
 {
+    const unsigned int sequence = ++backend->published_sequence;
     int rc;
     *device_status = 0;
+    if (results) *results = NULL;
     if (yvex_rocm_seam("YVEX_TEST_ROCM_SYNC_FAILURE"))
         return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, where, "synchronisation failed (test seam)");
-    /* the copy below synchronises the stream after the last kernel */
-    rc = yvex_hip_memcpy_d2h(device_status, backend->device_status, sizeof(int), backend->stream);
+    rc = yvex_hip_publish((const void *)(uintptr_t)device_results, bytes, backend->device_status, clear,
+                          backend->published, sequence, backend->stream);
+    if (rc == 0) rc = yvex_hip_await(backend->published, sequence, device_status, backend->stream);
     if (rc != 0) {
         backend->status = YVEX_BACKEND_STATUS_FAILED;
         return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, where, yvex_hip_last_error());
     }
+    if (clear) backend->status_clean = 1;
+    if (results) *results = backend->published + YVEX_HIP_PUBLISH_HEAD_BYTES;
     backend->memory.d2h_bytes += sizeof(int);
     return YVEX_OK;
+}
+
+int yvex_rocm_finish(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err)
+{
+    return finish(backend, 0ull, 0ull, NULL, !backend->pending_completion, where, device_status, err);
+}
+
+int yvex_rocm_finish_results(yvex_rocm_backend *backend, unsigned long long device_results, unsigned long long bytes,
+                             const unsigned char **results, const char *where, int *device_status,
+                             yvex_error *err)
+{
+    return finish(backend, device_results, bytes, results, !backend->pending_completion, where, device_status, err);
+}
+
+int yvex_rocm_finish_phase(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err)
+{
+    return finish(backend, 0ull, 0ull, NULL, 1, where, device_status, err);
 }
 
 int yvex_rocm_upload_queued(yvex_rocm_backend *backend, void *device, const void *host,
@@ -112,6 +139,23 @@ int yvex_rocm_upload_queued(yvex_rocm_backend *backend, void *device, const void
         return -1;
     backend->token_staging_cursor += piece;
     return 0;
+}
+
+/* What every session has of its own on the device: a stream, a status word, and pinned memory for
+ * what its synchronous operations publish. Released again where any of it is missing. */
+static int session_open(yvex_rocm_backend *backend)
+{
+    void *status_word = NULL, *published = NULL;
+    if (yvex_hip_stream_create(&backend->stream) != 0 || yvex_hip_malloc(&status_word, 256u) != 0 ||
+        yvex_hip_host_alloc(&published, YVEX_HIP_PUBLISH_HEAD_BYTES + YVEX_HIP_PUBLISH_MAX_BYTES) != 0) {
+        if (status_word) (void)yvex_hip_free(status_word);
+        if (backend->stream) (void)yvex_hip_stream_destroy(backend->stream);
+        return 0;
+    }
+    memset(published, 0, YVEX_HIP_PUBLISH_HEAD_BYTES);
+    backend->device_status = (int *)status_word;
+    backend->published = (unsigned char *)published;
+    return 1;
 }
 
 int yvex_rocm_backend_open(yvex_rocm_backend **out, const yvex_backend_options *options, yvex_error *err)
@@ -146,25 +190,21 @@ int yvex_rocm_backend_open(yvex_rocm_backend **out, const yvex_backend_options *
     backend->host_only = host_only;
     backend->memory.memory_limit_bytes = options->memory_limit_bytes;
     if (!host_only) {
-        void *status_word = NULL;
         char name[64], arch[64];
         uint64_t total = 0, free_bytes = 0;
         int units = 0;
         if (yvex_hip_device_info(device, name, sizeof(name), arch, sizeof(arch), &total,
-                                 &free_bytes, &units) != 0 ||
-            yvex_hip_stream_create(&backend->stream) != 0 ||
-            yvex_hip_malloc(&status_word, 256u) != 0) {
-            if (backend->stream) yvex_hip_stream_destroy(backend->stream);
+                                 &free_bytes, &units) != 0 || !session_open(backend)) {
             free(backend);
             return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, "backend.open", yvex_hip_last_error());
         }
-        backend->device_status = (int *)status_word;
         backend->kernels_available = !yvex_rocm_seam("YVEX_TEST_ROCM_BUNDLE_FAILURE") &&
                                      strncmp(arch, "gfx950", 6) == 0 && yvex_hip_kernels_loadable();
         if (backend->kernels_available &&
             (yvex_hip_fill_u32(backend->device_status, 0u, 1u, backend->stream) != 0 ||
              yvex_hip_stream_sync(backend->stream) != 0))
             backend->kernels_available = 0;
+        backend->status_clean = backend->kernels_available;
     }
     backend->status = backend->kernels_available ? YVEX_BACKEND_STATUS_READY
                                                  : YVEX_BACKEND_STATUS_CONTEXT_READY;
@@ -202,18 +242,16 @@ int yvex_rocm_backend_open_shared(yvex_rocm_backend **out, yvex_rocm_backend *co
     backend->host_only = context_owner->host_only;
     backend->memory.memory_limit_bytes = memory_limit_bytes;
     if (!backend->host_only) {
-        void *status_word = NULL;
-        if (yvex_hip_stream_create(&backend->stream) != 0 || yvex_hip_malloc(&status_word, 256u) != 0) {
-            if (backend->stream) yvex_hip_stream_destroy(backend->stream);
+        if (!session_open(backend)) {
             free(backend);
             return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, "rocm.shared.open", yvex_hip_last_error());
         }
-        backend->device_status = (int *)status_word;
         backend->kernels_available = context_owner->kernels_available;
         if (backend->kernels_available &&
             (yvex_hip_fill_u32(backend->device_status, 0u, 1u, backend->stream) != 0 ||
              yvex_hip_stream_sync(backend->stream) != 0))
             backend->kernels_available = 0;
+        backend->status_clean = backend->kernels_available;
     }
     backend->status = backend->kernels_available ? YVEX_BACKEND_STATUS_READY
                                                  : YVEX_BACKEND_STATUS_CONTEXT_READY;
@@ -250,7 +288,9 @@ int yvex_rocm_backend_close_checked(yvex_rocm_backend **backend_ref, yvex_error 
             backend->token_staging = NULL;
             backend->token_staging_bytes = 0ull;
         }
-        if (yvex_hip_stream_sync(backend->stream) != 0 || backend->token_staging ||
+        if (yvex_hip_stream_sync(backend->stream) == 0 && yvex_hip_host_free(backend->published) == 0)
+            backend->published = NULL;
+        if (yvex_hip_stream_sync(backend->stream) != 0 || backend->token_staging || backend->published ||
             yvex_hip_free(backend->device_status) != 0 ||
             yvex_hip_stream_destroy(backend->stream) != 0) {
             backend->status = YVEX_BACKEND_STATUS_FAILED;

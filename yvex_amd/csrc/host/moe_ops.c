@@ -1192,7 +1192,7 @@ static int moe_complete_rows(yvex_rocm_backend *backend, int barrier_observed,
                                 "MoE completion owner is invalid");
     if (!backend->host_only) {
         started = monotonic_ns();
-        rc = yvex_rocm_finish(backend, "rocm.moe.rows.phase-sync", &device_status, err);
+        rc = yvex_rocm_finish_phase(backend, "rocm.moe.rows.phase-sync", &device_status, err);
         if (rc == YVEX_OK) backend->pending_completion = 0;   /* the barrier was reached: the next phase starts clean */
         if (rc == YVEX_OK && device_status)
             rc = yvex_rocm_refuse(err, device_status == 1 ? YVEX_ERR_FORMAT : YVEX_ERR_BACKEND,

@@ -483,6 +483,7 @@ int yvex_rocm_backend_moe_begin(yvex_rocm_moe_execution **out, yvex_rocm_backend
         }
     }
     expanded_bytes = layer->expanded_width * sizeof(float);
+    if (!backend->pending_completion) backend->status_clean = 0;
     rc = backend->pending_completion   /* deferred row batches own the word until their barrier */
         ? YVEX_OK
         : launched(x, yvex_hip_fill_u32(backend->device_status, 0u, 1u, backend->stream), "rocm.moe.status", err);

@@ -33,7 +33,12 @@ struct yvex_rocm_backend {
     unsigned long long workspace_bytes, workspace_cursor;
     /* device status word shared by the operations of this backend */
     int *device_status;
+    int status_clean;          /* the word is zero: whoever read it last cleared it */
     int pending_completion;
+    /* pinned host memory that a synchronous operation's last launch publishes its status word and
+     * small results in, and the number of the last such launch */
+    unsigned char *published;
+    unsigned int published_sequence;
     /* launch graphs of the row-batch MoE operation, keyed on topology and device addresses */
     struct yvex_rocm_moe_graphs *moe_graphs;
     /* shared sessions (src/backend/cuda/backend.c:1913-2000): a child borrows the device and the
@@ -60,9 +65,18 @@ void yvex_rocm_workspace_reset(yvex_rocm_backend *backend);
 int yvex_rocm_require_kernels(const yvex_rocm_backend *backend, const char *where, yvex_error *err);
 /* Map a launch-level return code (negative yvex_status) to an error. */
 int yvex_rocm_launch_result(int rc, const char *where, yvex_error *err);
-/* Stream synchronise + read the device status word. */
+/* Wait for the stream's work and read the device status word; the word is cleared unless deferred
+ * row batches are waiting for their barrier. */
 int yvex_rocm_finish(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err);
-/* Clear the status word on the stream, unless deferred row batches are waiting for their barrier. */
+/* The same for an operation with small results: `bytes` of device memory (a multiple of 4, at most
+ * YVEX_HIP_PUBLISH_MAX_BYTES) arrive in *results, host memory that is good until the next such call. */
+int yvex_rocm_finish_results(yvex_rocm_backend *backend, unsigned long long device_results, unsigned long long bytes,
+                             const unsigned char **results, const char *where, int *device_status,
+                             yvex_error *err);
+/* The barrier of a phase of deferred row batches: yvex_rocm_finish that clears the word they share. */
+int yvex_rocm_finish_phase(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err);
+/* Make sure the status word is zero on the stream, unless deferred row batches are waiting for their
+ * barrier. */
 int yvex_rocm_status_reset(yvex_rocm_backend *backend, const char *where, yvex_error *err);
 /* Resolve a weight view: device_address if given, else the resident arena mapping. */
 /* Queue `bytes` of caller-owned host memory for upload to `device` on the backend's stream; the

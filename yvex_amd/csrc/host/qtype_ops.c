@@ -145,7 +145,7 @@ int yvex_rocm_encoded_matvec(
     if (rc != YVEX_OK) return rc;
     output->is_written = 1;
     facts->d2h_bytes = sizeof(int);
-    facts->kernel_launches = launches + 1ull;   /* status reset included */
+    facts->kernel_launches = launches + 1ull;   /* the status word's included */
     facts->download_count = 1ull;
     facts->stream_synchronizations = 1ull;
     facts->active_weight_bytes = encoded_bytes;

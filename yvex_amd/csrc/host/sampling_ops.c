@@ -50,11 +50,13 @@ int yvex_rocm_select_greedy_rows(
     rc = yvex_rocm_require_kernels(backend, where, err);
     if (rc != YVEX_OK) return rc;
     yvex_rocm_workspace_reset(backend);
-    if (!yvex_rocm_backend_workspace_acquire(backend, tie_bytes, 256ull, &ties_device) ||
-        !yvex_rocm_backend_workspace_acquire(backend, token_bytes, 256ull, &tokens_device) ||
-        !yvex_rocm_backend_workspace_acquire(backend, selected_bytes, 256ull, &values_device))
+    /* ties, tokens and values end to end: what fits the published results comes back with the status
+     * word in one go */
+    if (!yvex_rocm_backend_workspace_acquire(backend, tie_bytes + token_bytes + selected_bytes, 256ull, &ties_device))
         return yvex_rocm_refuse(err, YVEX_ERR_NOMEM, where,
                                 "greedy row selection needs an attached workspace for its results");
+    tokens_device = ties_device + tie_bytes;
+    values_device = tokens_device + token_bytes;
     /* long rows are shared among the compute units when the workspace has room for the partial
      * results; otherwise one workgroup scans a row */
     scratch_bytes = yvex_hip_argmax_scratch_bytes(row_count, row_width);
@@ -71,15 +73,28 @@ int yvex_rocm_select_greedy_rows(
                                 (uint64_t *)(uintptr_t)ties_device, (void *)(uintptr_t)scratch_device,
                                 scratch_bytes, backend->device_status, backend->stream),
             "rocm.sampling.greedy.launch", err);
+    if (tie_bytes + token_bytes + selected_bytes <= YVEX_HIP_PUBLISH_MAX_BYTES) {
+        const unsigned char *results = NULL;
+        if (rc == YVEX_OK)
+            rc = yvex_rocm_finish_results(backend, ties_device, tie_bytes + token_bytes + selected_bytes, &results,
+                                          "rocm.sampling.greedy.sync", &device_status, err);
+        if (rc == YVEX_OK) {
+            memcpy(tie_counts, results, (size_t)tie_bytes);
+            memcpy(selected_tokens, results + tie_bytes, (size_t)token_bytes);
+            memcpy(selected_values, results + tie_bytes + token_bytes, (size_t)selected_bytes);
+        }
+    } else {
 #define READ(target_, source_, bytes_)                                                         \
-    if (rc == YVEX_OK &&                                                                       \
-        yvex_hip_memcpy_d2h((target_), (const void *)(uintptr_t)(source_), (bytes_), backend->stream) != 0) \
-        rc = yvex_rocm_refuse(err, YVEX_ERR_BACKEND, where, yvex_hip_last_error())
-    READ(selected_tokens, tokens_device, token_bytes);
-    READ(selected_values, values_device, selected_bytes);
-    READ(tie_counts, ties_device, tie_bytes);
+        if (rc == YVEX_OK &&                                                                   \
+            yvex_hip_memcpy_d2h((target_), (const void *)(uintptr_t)(source_), (bytes_), backend->stream) != 0) \
+            rc = yvex_rocm_refuse(err, YVEX_ERR_BACKEND, where, yvex_hip_last_error())
+        READ(selected_tokens, tokens_device, token_bytes);
+        READ(selected_values, values_device, selected_bytes);
+        READ(tie_counts, ties_device, tie_bytes);
 #undef READ
-    if (rc == YVEX_OK) rc = yvex_rocm_finish(backend, "rocm.sampling.greedy.sync", &device_status, err);
+        if (rc == YVEX_OK)
+            rc = yvex_rocm_finish(backend, "rocm.sampling.greedy.sync", &device_status, err);
+    }
     for (row = 0ull; rc == YVEX_OK && row < row_count; ++row)
         if (device_status || selected_tokens[row] >= row_width || !isfinite(selected_values[row]) ||
             !tie_counts[row])
