@@ -1,4 +1,4 @@
-// Decode-width expert sweeps specialised for IQ2_XXS (and, with the same item list, streams and
+// Decode-width expert sweeps specialised for IQ2_XXS (and, with the same pieces, streams and
 // finishing pass, Q4_K rows and the Q2_K rows of a down projection) weights and Q8_K activations
 // on gfx950. The notes below are about IQ2_XXS; what differs for Q4_K rows stands above
 // `Q4kHalf`, for Q2_K rows above `Q2kHalf`.
@@ -23,8 +23,13 @@
 //     computes (double accumulation over the blocks of a row, src/gguf/quant_compute.c:152-172),
 //     so every value that is rounded to bfloat16 afterwards rounds as it does there.
 //
-// A work item is (bucket, tile of up to 32 row iterations, sweep). One workgroup per compute
-// unit stays resident and its waves draw items from the workgroup's share of the list.
+// One workgroup per compute unit stays resident. The rows of all sweeps, weighed by what a sweep
+// costs, are dealt out to the workgroups in one piece each (a piece may end in the middle of a
+// sweep and the next begin there). A workgroup's waves draw short chunks of its piece from a
+// counter in LDS: the older wave of a SIMD is served first and gets through 1.2 to 1.6 times the
+// rows of the younger one. A wave whose next chunk belongs to the same sweep goes on with the
+// activation columns it holds, and asks for that chunk's first rows before it is done with this
+// one's, so that a chunk costs no round trip to memory.
 //
 // IMAGE: the weights come from the backend's own re-packing of the canonical bytes (built once at
 // residency time, the canonical tensor stays the authority), made for this kernel's instruction
@@ -44,10 +49,27 @@ namespace yvex {
 constexpr unsigned kSweepWaves = 8u;           // two per SIMD: the sweep of four pairs needs their registers
 constexpr unsigned kSweepThreads = kSweepWaves * 64u;
 constexpr int kSweepPairs = 4;                 // pairs of one bucket served by one sweep
-constexpr unsigned kSweepIters = 32u;          // weight-row iterations per work item (at most)
 constexpr int kSweepAheadSmall = 1;            // rows requested ahead of the one decoded, sweeps of one or two pairs
-constexpr unsigned kSweepLongPercent = 75u;    // share of the weight rows that goes out in full-length items
-constexpr unsigned kSweepShortDiv = 2u;        // the rest goes out in items of 1 / kSweepShortDiv of that length
+constexpr unsigned kSweepChunkTurns = 16u;     // iterations a wave draws at a time (at most)
+
+// What a weight row costs a sweep that serves n pairs, relative to the other sweeps of the launch:
+// what the workgroups' pieces of a launch are measured in. Fitted to the times of the workgroups of
+// decode launches (23 to 96 rows) against what they had swept: IQ2_XXS 1 : 1.25 : 1.52 : 1.73 (the LDS
+// pipe's share is the same whatever n is, the dot products come on top), Q2_K 1 : 1.17 : 1.34 : 1.48,
+// Q4_K 1 : 0.95 : 1 : 1.03 (it waits for memory).
+template <unsigned QT>
+__device__ __forceinline__ constexpr unsigned sweep_cost(unsigned n)
+{
+    if (QT == QT_IQ2_XXS) return n >= 4u ? 14u : n == 3u ? 12u : n == 2u ? 10u : 8u;
+    if (QT == QT_Q2_K) return n >= 4u ? 12u : n == 3u ? 11u : n == 2u ? 9u : 8u;
+    return n >= 4u ? 13u : 12u;
+}
+// ... and the rows of one matrix with n pairs: sweeps of four and one of what is left.
+template <unsigned QT>
+__device__ __forceinline__ unsigned bucket_cost(unsigned n)
+{
+    return n / 4u * sweep_cost<QT>(4u) + (n % 4u ? sweep_cost<QT>(n % 4u) : 0u);
+}
 
 // LDS map (byte addresses; the dynamic block starts at LDS address 0)
 constexpr unsigned kMagBase = 0u;              // 256 entries x 16 replicas x {+lo, +hi, -lo, -hi}
@@ -60,22 +82,16 @@ constexpr unsigned kParkBase = kTicketAddress + 32u;
 // ([stream][pair][row of the item]) for the SwiGLU pass at its end.
 constexpr unsigned kWindowLines = 16u;
 constexpr unsigned kWindowBytes = kWindowLines * 256u;
-constexpr unsigned kFusedItemRows = 32u;       // weight row pairs per fused work item
+constexpr unsigned kFusedItemRows = 32u;       // weight row pairs of a chunk, at most
 constexpr unsigned kResultBytes = 2u * 4u * kFusedItemRows * 4u;
 constexpr unsigned kParkBytes = kWindowBytes + kResultBytes;
-// Sweeps listed by the number of pairs they serve (4, 3, 2, 1): four class sizes, four class
-// starts (cursors while the list is built) and one word per sweep:
-// {whole problem is one bucket : 1, shared expert's problem : 1, bucket : 14, sweep of the bucket : 16}.
-constexpr unsigned kClassMaxSweeps = 4096u;
-constexpr unsigned kClassCountBase = kParkBase + kSweepWaves * kParkBytes;
-constexpr unsigned kClassWaveBase = kClassCountBase + 32u;    // per wave and class: entries of a turn
-constexpr unsigned kClassListBase = kClassCountBase + 32u + kSweepWaves * 16u;
+constexpr unsigned kMaxSweeps = 4096u;
 // What opens an item without a round trip to memory: expert, first ordered pair and population of
 // every routed bucket, and {source pair, route weight} of every ordered pair when the routed
 // problem has at most kPairCacheMax of them (decode widths; wider batches read them from memory).
-constexpr unsigned kBucketBase = kClassListBase + kClassMaxSweeps * 4u;   // 256 x {expert, first, population}
-constexpr unsigned kPairCacheBase = kBucketBase + 256u * 12u;
-constexpr unsigned kPairCacheMax = 608u;
+constexpr unsigned kBucketBase = kParkBase + kSweepWaves * kParkBytes;     // 256 x {expert, first, population, sweeps before it}
+constexpr unsigned kPairCacheBase = kBucketBase + 256u * 16u;
+constexpr unsigned kPairCacheMax = 1024u;
 constexpr unsigned kSweepLdsBytes = kPairCacheBase + kPairCacheMax * 8u;
 static_assert(kSweepLdsBytes <= 160u * 1024u, "the sweep's tables, lists and caches must fit the LDS of a compute unit");
 
@@ -125,18 +141,22 @@ __device__ __forceinline__ unsigned lds_load_u32(unsigned address)
 #endif
 }
 
-__device__ __forceinline__ void sweep_tables_fill()
+// The codebook digits of a thread's table entries, requested together at kernel start: one round
+// trip to memory, which runs beside the others that open the launch.
+constexpr unsigned kTableTurns = 256u * 16u / kSweepThreads;
+static_assert(256u * 16u % kSweepThreads == 0u && 128u * 32u % kSweepThreads == 0u,
+              "every thread fills the same number of table entries");
+
+__device__ __forceinline__ void sweep_tables_request(unsigned (&digits)[kTableTurns])
 {
-    // (the codebook digits of a thread's entries are requested together: one round trip to
-    // memory, not one per entry)
-    constexpr unsigned kTurns = 256u * 16u / kSweepThreads;
-    static_assert(256u * 16u % kSweepThreads == 0u && 128u * 32u % kSweepThreads == 0u,
-                  "every thread fills the same number of table entries");
-    unsigned digits[kTurns];
 #pragma unroll
-    for (unsigned t = 0; t < kTurns; ++t) digits[t] = k_iq2_digits[(threadIdx.x + t * kSweepThreads) >> 4];
+    for (unsigned t = 0; t < kTableTurns; ++t) digits[t] = k_iq2_digits[(threadIdx.x + t * kSweepThreads) >> 4];
+}
+
+__device__ __forceinline__ void sweep_tables_fill(const unsigned (&digits)[kTableTurns])
+{
 #pragma unroll
-    for (unsigned t = 0; t < kTurns; ++t) {
+    for (unsigned t = 0; t < kTableTurns; ++t) {
         const unsigned i = threadIdx.x + t * kSweepThreads;
         const uint2 m = iq2_magnitude_of_digits(digits[t]);
         // byte-wise negation: every level is >= 8, so (x ^ 0xff) + 1 never carries
@@ -461,16 +481,29 @@ __device__ __forceinline__ void q4k_half_dots(const Q4kHalf (&c)[STREAMS], const
     }
 }
 
-// One sweep over the item's weight rows [row_begin, row_end) for N live pairs.
+// The workgroup's next chunk, for every lane of the wave.
+__device__ __forceinline__ unsigned draw_chunk()
+{
+    unsigned got = 0u;
+    if ((threadIdx.x & 63u) == 0u)
+        got = __hip_atomic_fetch_add(reinterpret_cast<__attribute__((address_space(3))) unsigned *>(kTicketAddress), 1u,
+                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    return (unsigned)__builtin_amdgcn_readfirstlane((int)got);
+}
+
+// One sweep over weight rows [row_begin, row_end) for N live pairs: chunk `chunk` of them
+// (chunk_turns iterations each) and whatever chunks of the same rows this wave draws next; returns
+// the first one drawn that lies behind them (as drawn: the rows' first chunk is number `base`).
 // MODE 0: one weight row group (the rows of one iteration) at a time; MODE 1: a gate row group
 // and the matching up row group, SwiGLU in the finishing pass; MODE 2: two consecutive row groups
 // of one matrix, which share the activation columns as gate and up rows do: the fixed cost of an
 // iteration (requests, waits, reduction, loop control) is spent once per two groups.
 template <int MODE, int N, bool IMAGE, unsigned QT>
-__device__ __forceinline__ void iq2_sweep(const GroupedArgs &a, const GroupedProblem &pr,
-                                          const SweepLane &g, const unsigned char *gate_e,
-                                          const unsigned char *up_e, unsigned long long first_ordered,
-                                          unsigned row_begin, unsigned row_end, bool pairs_in_lds)
+__device__ __forceinline__ unsigned iq2_sweep(const GroupedArgs &a, const GroupedProblem &pr,
+                                              const SweepLane &g, const unsigned char *gate_e,
+                                              const unsigned char *up_e, unsigned long long first_ordered,
+                                              unsigned row_begin, unsigned row_end, bool pairs_in_lds,
+                                              unsigned chunk, unsigned base, unsigned chunk_turns)
 {
     constexpr bool FUSED = MODE == 1;
     constexpr bool TWIN = MODE != 0;     // two streams of weight rows against the same activation columns
@@ -549,7 +582,7 @@ __device__ __forceinline__ void iq2_sweep(const GroupedArgs &a, const GroupedPro
 
     const unsigned rows_per_turn = MODE == 2 ? 2u * g.rows_per_iter : g.rows_per_iter;
     const unsigned rows = row_end - row_begin;               // a multiple of rows_per_turn
-    const unsigned iterations = rows / rows_per_turn;         // <= kSweepIters
+    const unsigned iterations = rows / rows_per_turn;
     // wave-uniform row bases advance by a scalar stride; the lane's place inside an iteration's
     // rows is a constant 32-bit offset
     const unsigned char *gate_rows = gate_e + (unsigned long long)row_begin * pr.row_bytes;
@@ -587,26 +620,22 @@ __device__ __forceinline__ void iq2_sweep(const GroupedArgs &a, const GroupedPro
     constexpr int STREAMS = TWIN ? 2 : 1;
     using Half = typename SweepHalf<QT>::type;
     Half ring[AHEAD + 1][STREAMS];
-    const unsigned last = iterations - 1u;
     auto request = [&](Half (&slot)[STREAMS], unsigned it) {
-        const unsigned clamped = it < last ? it : last;
         if constexpr (Q2) {
-            slot[0].load(gate_rows + clamped * gate_step, gate_codes_at, gate_tail_at, gate_block + 80u);
+            slot[0].load(gate_rows + it * gate_step, gate_codes_at, gate_tail_at, gate_block + 80u);
             if constexpr (TWIN)
-                slot[1].load(up_rows + clamped * up_step, up_codes_at, up_tail_at, up_block + 80u);
+                slot[1].load(up_rows + it * up_step, up_codes_at, up_tail_at, up_block + 80u);
         } else {
-            slot[0].load(gate_rows + clamped * gate_step, gate_codes_at, gate_tail_at);
+            slot[0].load(gate_rows + it * gate_step, gate_codes_at, gate_tail_at);
             if constexpr (TWIN)
-                slot[1].load(up_rows + clamped * up_step, up_codes_at, up_tail_at);
+                slot[1].load(up_rows + it * up_step, up_codes_at, up_tail_at);
         }
     };
-    // The first requests are kept in ring order: the loop's first wait is counted against the
-    // loads issued after the slot it consumes, on the entry path and on the back edge alike.
-#pragma unroll
-    for (int ahead = 0; ahead < AHEAD; ++ahead) {
-        __builtin_amdgcn_sched_barrier(0);
-        request(ring[ahead], (unsigned)ahead);
-    }
+    static_assert(AHEAD == 1, "a chunk's last turn asks for the first rows of the next");
+    const unsigned chunks = (iterations + chunk_turns - 1u) / chunk_turns;
+    unsigned begin = chunk * chunk_turns;
+    __builtin_amdgcn_sched_barrier(0);
+    request(ring[0], begin);
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- the window's row sums: a lane per (line, parity, row of the iteration) adds that
@@ -614,7 +643,7 @@ __device__ __forceinline__ void iq2_sweep(const GroupedArgs &a, const GroupedPro
     // A fused item keeps the sums for the SwiGLU pass at its end; a plain projection rounds to
     // bfloat16 and stores here.
     const unsigned R = g.rows_per_iter;
-    auto flush = [&](unsigned first_iteration, unsigned count) {
+    auto flush = [&](unsigned first_iteration, unsigned count, unsigned chunk_begin) {
         // LDS operations of one wave complete in order, so the terms parked above are visible here
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -638,7 +667,7 @@ __device__ __forceinline__ void iq2_sweep(const GroupedArgs &a, const GroupedPro
             const float row_sum = (float)sum;
             const unsigned iteration = first_iteration + line / (unsigned)PV, v = line % (unsigned)PV;
             if constexpr (FUSED) {
-                const unsigned local = (iteration << g.row_shift) + group;      // < kFusedItemRows
+                const unsigned local = ((iteration - chunk_begin) << g.row_shift) + group;   // < kFusedItemRows
                 lds_store_u32(g.results + ((parity * (unsigned)N + v) * kFusedItemRows + local) * 4u,
                               __float_as_uint(row_sum));
             } else {
@@ -665,14 +694,23 @@ __device__ __forceinline__ void iq2_sweep(const GroupedArgs &a, const GroupedPro
     constexpr unsigned kWindowIters = (kWindowLines / (unsigned)PV) / (AHEAD + 1) * (AHEAD + 1);
     static_assert(kWindowIters >= AHEAD + 1, "a window holds at least one trip's lines");
 
-    for (unsigned window_begin = 0; window_begin < iterations; window_begin += kWindowIters) {
-      const unsigned window_end = window_begin + kWindowIters < iterations ? window_begin + kWindowIters : iterations;
+    for (;;) {
+    // the chunk behind this one, whose rows the last turn below asks for (past the last of these
+    // rows: this chunk's last rows once more, which nobody uses)
+    const unsigned drawn = draw_chunk(), next = drawn - base;
+    const unsigned finish = begin + chunk_turns < iterations ? begin + chunk_turns : iterations;
+    const unsigned padded = begin + ((finish - begin + 1u) & ~1u);
+    const unsigned follow = next < chunks ? next * chunk_turns : finish - 1u;
+    unsigned window_begin = begin;
+    while (window_begin < finish) {
+      const unsigned window_end = window_begin + kWindowIters < finish ? window_begin + kWindowIters : finish;
       unsigned park_at = g.park + g.term_slot;
       for (unsigned it0 = window_begin; it0 < window_end; it0 += AHEAD + 1) {
 #pragma unroll
       for (int turn = 0; turn <= AHEAD; ++turn) {
-        const unsigned it = it0 + (unsigned)turn;   // may run past the last row by AHEAD turns
-        request(ring[(turn + AHEAD) % (AHEAD + 1)], it + AHEAD);
+        const unsigned it = it0 + (unsigned)turn;   // may run past the chunk's last rows by a turn
+        const unsigned ahead = it + 1u;
+        request(ring[(turn + AHEAD) % (AHEAD + 1)], ahead >= padded ? follow : ahead < finish ? ahead : finish - 1u);
         const Half (&now)[STREAMS] = ring[turn];
         int total_gate[N], total_up[N];
         int min_gate[N], min_up[N];          // Q4_K: the sums of the minimum term
@@ -749,14 +787,16 @@ __device__ __forceinline__ void iq2_sweep(const GroupedArgs &a, const GroupedPro
         }
       }
       }
-      flush(window_begin, window_end - window_begin);
+      flush(window_begin, window_end - window_begin, begin);
+      window_begin = window_end;
     }
 
-    // ---- finish a fused item: SwiGLU of the (gate, up) row sums, coalesced stores ----
+    // ---- the end of a fused chunk: SwiGLU of the (gate, up) row sums, coalesced stores ----
     if constexpr (FUSED) {
-        const unsigned outputs = rows * (unsigned)N;
+        const unsigned chunk_rows = (finish - begin) << g.row_shift, chunk_row = row_begin + (begin << g.row_shift);
+        const unsigned outputs = chunk_rows * (unsigned)N;
         for (unsigned o = lane; o < outputs; o += 64u) {
-            const unsigned p = o / rows, local = o % rows;      // consecutive lanes: consecutive rows
+            const unsigned p = o / chunk_rows, local = o % chunk_rows;      // consecutive lanes: consecutive rows
             const float first = __uint_as_float(lds_load_u32(g.results + (p * kFusedItemRows + local) * 4u));
             const float second = __uint_as_float(
                 lds_load_u32(g.results + (((unsigned)N + p) * kFusedItemRows + local) * 4u));
@@ -770,10 +810,24 @@ __device__ __forceinline__ void iq2_sweep(const GroupedArgs &a, const GroupedPro
                 }
             const float value = swiglu_bf16_fast(first, second, rw, a.limit, (float)a.limit);
             if (!finite_f32(value)) raise_status(a.status, 1);
-            else pr.out[oi * a.out_rows + row_begin + local] = value;
+            else pr.out[oi * a.out_rows + chunk_row + local] = value;
         }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
+    if (next >= chunks) return drawn;
+    begin = next * chunk_turns;
+    }
+}
+
+__device__ __forceinline__ unsigned uniform(unsigned v)
+{
+    return (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+}
+__device__ __forceinline__ unsigned long long uniform64(unsigned long long v)
+{
+    return ((unsigned long long)uniform((unsigned)(v >> 32)) << 32) | uniform((unsigned)v);
 }
 
 template <int MODE, bool IMAGE, unsigned QT>
@@ -786,55 +840,32 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
         return;
     }
     const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    // The bucket count and this thread's bucket population are requested before the tables are
-    // built, so that their round trips to memory run under the table fill instead of after it.
     const GroupedProblem &routed = a.problem[0];
     const bool routed_fixed = routed.expert_ids == nullptr;
-    const unsigned buckets = routed_fixed ? 1u : (unsigned)routed.counts[0];
-    unsigned population_here = 0u;
-    if (!routed_fixed && tid < 256u && tid < routed.experts)
-        population_here = (unsigned)routed.bucket_populations[tid];
-    // ... and so are the routed buckets' experts and first pairs and the pairs' sources, which
-    // the items will find in LDS
-    unsigned long long expert_here = 0ull, first_here = 0ull;
-    if (!routed_fixed && tid < 256u && tid < routed.experts) {
-        expert_here = routed.expert_ids[tid];
-        first_here = routed.bucket_offsets[tid];
-    }
     const bool pairs_in_lds = !routed_fixed && routed.order != nullptr && routed.pairs <= kPairCacheMax;
     static_assert(kPairCacheMax <= 2u * kSweepThreads, "two cached pairs a thread");
+    // ---- everything that opens the launch is requested before any of it is used: the tables'
+    // digits, the routed buckets (four a lane, in every wave) and the pairs' sources ----
+    unsigned digits[kTableTurns];
+    if constexpr (QT == QT_IQ2_XXS) sweep_tables_request(digits);     // (the other formats need no tables)
+    const unsigned long long bucket_count = routed_fixed ? 1ull : routed.counts[0];
+    unsigned long long population64[4], expert64[4], first64[4];
+#pragma unroll
+    for (unsigned j = 0; j < 4u; ++j) {
+        const unsigned slot = 4u * lane + j;
+        population64[j] = routed_fixed ? (slot == 0u ? routed.pairs : 0ull) : 0ull;
+        expert64[j] = first64[j] = 0ull;
+        if (!routed_fixed && slot < routed.experts) {
+            population64[j] = routed.bucket_populations[slot];
+            expert64[j] = routed.expert_ids[slot];
+            first64[j] = routed.bucket_offsets[slot];
+        }
+    }
     unsigned long long source_here[2] = {~0ull, ~0ull};
     if (pairs_in_lds) {
 #pragma unroll
         for (unsigned k = 0; k < 2u; ++k)
             if (tid + k * kSweepThreads < routed.pairs) source_here[k] = routed.order[tid + k * kSweepThreads];
-    }
-    if constexpr (QT == QT_IQ2_XXS) sweep_tables_fill();     // (Q4_K rows need no tables)
-    if (tid == 0u) lds_store_u32(kTicketAddress, 0u);
-    if (pairs_in_lds) {
-        float weight_here[2];
-#pragma unroll
-        for (unsigned k = 0; k < 2u; ++k)   // a source outside the problem reads no weight here; the sweep's own checks refuse it
-            weight_here[k] = routed.route_weights && source_here[k] < routed.pairs
-                ? routed.route_weights[source_here[k]] : 1.0f;
-#pragma unroll
-        for (unsigned k = 0; k < 2u; ++k)
-            if (tid + k * kSweepThreads < routed.pairs)
-                lds_store_uint2(kPairCacheBase + 8u * (tid + k * kSweepThreads),
-                                make_uint2(source_here[k] < 0xffffffffull ? (unsigned)source_here[k] : 0xffffffffu,
-                                           __float_as_uint(weight_here[k])));
-    }
-
-    if (!routed_fixed && buckets > 256u) {
-        if (tid == 0u) raise_status(a.status, 2);
-        return;
-    }
-    if (!routed_fixed && tid < buckets) {
-        // (values past 32 bits fail the item's range check through their low words' sum only by
-        // accident, so they are clamped to a value that always fails it)
-        lds_store_u32(kBucketBase + 12u * tid, expert_here < 0xffffffffull ? (unsigned)expert_here : 0xffffffffu);
-        lds_store_u32(kBucketBase + 12u * tid + 4u, first_here < 0xffffffffull ? (unsigned)first_here : 0xffffffffu);
-        lds_store_u32(kBucketBase + 12u * tid + 8u, population_here);
     }
 
     const unsigned units = a.width >> 5;
@@ -863,167 +894,206 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
         g.term_slot = ((lane & 1u) * 32u + (lane / span) * (span / 2u) + (lane % span) / 2u) * 4u;
     }
 
-    // The first part of the weight rows is cut into long items (kSweepIters iterations), the rest
-    // into short ones that come last in the item list: the waves of the grid finish within a short
-    // item of each other instead of a long one, and only the short items pay the fixed cost of an
-    // item (its activation columns, the first requests, the finishing pass) more often.
-    // (a fused item keeps its row sums in LDS until its SwiGLU pass: kFusedItemRows rows)
+    // ---- the launch's work, the same in every wave ----
+    // Slot 0 is the shared expert (no rows of its own when there is none), slot 1 + b bucket b. A
+    // slot of n pairs has n / 4 sweeps of four pairs and one of what is left. Every wave needs the
+    // prefix sums of cost and sweeps over the slots: a scan across its 64 lanes, four slots each,
+    // no barrier and no LDS. (It was a list of all sweeps sorted by their pairs, built by the
+    // workgroup in LDS behind two barriers: 2.5 us of every launch's first 8.5.)
+    const GroupedProblem &extra = a.problem[a.problems > 1u ? 1u : 0u];
+    const unsigned extra_pairs = a.problems > 1u ? extra.pairs : 0u;
+    const unsigned extra_cost = bucket_cost<QT>(extra_pairs), extra_sweeps = (extra_pairs + 3u) / 4u;
+    const unsigned buckets = (unsigned)bucket_count;
+    unsigned population[4], cost_here = 0u, sweeps_here = 0u;
+    bool bad = bucket_count > 256ull;
+#pragma unroll
+    for (unsigned j = 0; j < 4u; ++j) {
+        const bool live = 4u * lane + j < bucket_count;
+        bad |= live && (population64[j] > routed.pairs || expert64[j] >= routed.experts || first64[j] > routed.pairs);
+        population[j] = live ? (unsigned)population64[j] : 0u;
+        cost_here += bucket_cost<QT>(population[j]);
+        sweeps_here += (population[j] + 3u) / 4u;
+    }
+    const unsigned all_pairs = (unsigned)group_sum_i32<64>((int)(population[0] + population[1] + population[2] + population[3]));
+    // (the launch wrapper bounds the pairs, and with them what the packed sums below can hold)
+    if (__ballot(bad) != 0ull || all_pairs > routed.pairs || routed.pairs + extra_pairs > kMaxSweeps) {
+        if (tid == 0u) raise_status(a.status, 2);
+        return;
+    }
+    static_assert(kMaxSweeps * sweep_cost<QT>(4u) < 65536u, "a prefix is two 16-bit sums");
+    const unsigned packed = (sweeps_here << 16) | cost_here;
+    unsigned inclusive = packed;
+    inclusive += (unsigned)dpp_move<0x111, 0xf>((int)inclusive);    // row_shr 1, 2, 4, 8
+    inclusive += (unsigned)dpp_move<0x112, 0xf>((int)inclusive);
+    inclusive += (unsigned)dpp_move<0x114, 0xf>((int)inclusive);
+    inclusive += (unsigned)dpp_move<0x118, 0xf>((int)inclusive);
+    inclusive += (unsigned)dpp_move<0x142, 0xa>((int)inclusive);    // row_bcast15, row_bcast31
+    inclusive += (unsigned)dpp_move<0x143, 0xc>((int)inclusive);
+    const unsigned before = inclusive - packed;
+    const unsigned totals = (unsigned)__builtin_amdgcn_readlane((int)inclusive, 63);
+    const unsigned row_cost = extra_cost + (totals & 0xffffu), all_sweeps = extra_sweeps + (totals >> 16);
 
-    // Work items: sweeps by class, the ones that serve four pairs first (the shared expert's are
-    // all of that kind), then three, two, one; inside a class sweep by sweep, each over its tiles
-    // (neighbouring items are neighbouring tiles of one expert). A sweep's cost grows with its
-    // pairs and workgroup b owns items b, b + grid, ...: listed by class every workgroup gets the
-    // same share of every kind.
-    // Every workgroup must arrive at the same list, so a sweep's place is computed, not drawn:
-    // a bucket of n pairs has n / 4 sweeps of the first class, which start at the number of such
-    // sweeps in the buckets before it (a scan over the bucket slots), and, when n % 4 pairs are
-    // left, one sweep of class 4 - n % 4, whose place is the bucket's rank among the buckets that
-    // have one of that class (ballots and per-wavefront totals). The shared expert's pairs count
-    // as a bucket in front of the routed ones.
-    // list word: {whole problem is one bucket : 1, shared expert's problem : 1, bucket : 14, sweep of the bucket : 16}
-    static_assert(kSweepPairs == 4, "the sweep list has one class per number of pairs served, four of them");
-    unsigned all_sweeps;
-    {
-        const GroupedProblem &extra = a.problem[a.problems > 1u ? 1u : 0u];
-        const unsigned extra_pairs = a.problems > 1u ? extra.pairs : 0u;
-        const unsigned extra_full = extra_pairs / 4u, extra_class = extra_pairs % 4u ? 4u - extra_pairs % 4u : 0u;
-        // this thread's slot: bucket tid of the routed problem (or the whole problem as slot 0)
-        unsigned pairs_here = 0u;
-        if (routed_fixed) pairs_here = tid == 0u ? routed.pairs : 0u;
-        else if (tid < buckets) pairs_here = population_here;
-        const unsigned full = pairs_here / 4u;
-        const unsigned cls = pairs_here % 4u ? 4u - pairs_here % 4u : 0u;     // 0: no partial sweep
-        unsigned inclusive = full;
-#pragma unroll
-        for (int offset = 1; offset < 64; offset <<= 1) {
-            const unsigned below = (unsigned)__shfl_up((int)inclusive, offset, kWave);
-            if ((int)lane >= offset) inclusive += below;
-        }
-        unsigned rank[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (unsigned c = 1; c < 4u; ++c) {
-            const unsigned long long members = __ballot(cls == c);
-            rank[c] = (unsigned)__popcll(members & ((1ull << lane) - 1ull));
-            if (lane == 0u) lds_store_u32(kClassWaveBase + (wave * 4u + c) * 4u, (unsigned)__popcll(members));
-        }
-        if (lane == 63u) lds_store_u32(kClassWaveBase + wave * 16u, inclusive);       // class 0: full sweeps of the wave's slots
-        __syncthreads();
-        unsigned before[4] = {0u, 0u, 0u, 0u}, total[4] = {0u, 0u, 0u, 0u};
-        for (unsigned w = 0; w < kSweepWaves; ++w)
-#pragma unroll
-            for (unsigned c = 0; c < 4u; ++c) {
-                const unsigned n = lds_load_u32(kClassWaveBase + (w * 4u + c) * 4u);
-                if (w < wave) before[c] += n;
-                total[c] += n;
-            }
-        total[0] += extra_full;
-        if (extra_class) total[extra_class] += 1u;
-        all_sweeps = total[0] + total[1] + total[2] + total[3];
-        if (all_sweeps > kClassMaxSweeps) {          // the launch wrapper bounds the pairs
-            if (tid == 0u) raise_status(a.status, 2);
-            return;
-        }
-        unsigned start[4];
-        start[0] = 0u;
-#pragma unroll
-        for (unsigned c = 1; c < 4u; ++c) start[c] = start[c - 1u] + total[c - 1u];
-        const unsigned tag = routed_fixed ? 0x80000000u : tid << 16;
-        {
-            const unsigned at = extra_full + before[0] + inclusive - full;
-            for (unsigned k = 0; k < full; ++k) lds_store_u32(kClassListBase + 4u * (at + k), tag | (k & 0xffffu));
-        }
-        if (cls)
-            lds_store_u32(kClassListBase + 4u * (start[cls] + (extra_class == cls ? 1u : 0u) + before[cls] + rank[cls]),
-                          tag | (full & 0xffffu));
-        // the shared expert's sweeps: in front of their classes
-        for (unsigned k = tid; k < extra_full; k += kSweepThreads)
-            lds_store_u32(kClassListBase + 4u * k, 0xc0000000u | (k & 0xffffu));
-        if (tid == 0u && extra_class)
-            lds_store_u32(kClassListBase + 4u * start[extra_class], 0xc0000000u | (extra_full & 0xffffu));
-        if (tid < 4u) lds_store_u32(kClassCountBase + 4u * tid, total[tid]);
-        __syncthreads();
-    }
-    // A batch of a few rows has few sweeps: its items are made shorter (down to four iterations)
-    // until every wave of the grid has one, which matters more there than an item's fixed cost.
-    unsigned item_rows = FUSED ? kFusedItemRows : kSweepIters * g.rows_per_iter * (MODE == 2 ? 2u : 1u);
-    {
-        const unsigned least = 4u * g.rows_per_iter * (MODE == 2 ? 2u : 1u);
-        const unsigned waves = gridDim.x * kSweepWaves;
-        while (item_rows / 2u >= least && all_sweeps * (a.out_rows / item_rows) < waves) item_rows /= 2u;
-    }
-    const unsigned short_rows = item_rows / kSweepShortDiv;
-    const unsigned long_tiles = (unsigned)((unsigned long long)a.out_rows * kSweepLongPercent / 100u / item_rows);
-    const unsigned long_rows = long_tiles * item_rows;
-    const unsigned short_tiles = (a.out_rows - long_rows + short_rows - 1u) / short_rows;
-    const unsigned total_long = all_sweeps * long_tiles;
-    const unsigned total_items = total_long + all_sweeps * short_tiles;
-    // Workgroup b owns items b, b + grid, b + 2 grid, ...; its waves draw positions in that list
-    // from a counter in LDS, so a wave that met light items takes more of them.
-    auto draw = [&]() -> unsigned {
-        unsigned got = 0u;
-        if (lane == 0u)
-            got = __hip_atomic_fetch_add(
-                reinterpret_cast<__attribute__((address_space(3))) unsigned *>(kTicketAddress), 1u,
-                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        return (unsigned)__builtin_amdgcn_readfirstlane((int)got) * gridDim.x + blockIdx.x;
+    // ---- this workgroup's piece ----
+    const unsigned turn_rows = MODE == 2 ? 2u * g.rows_per_iter : g.rows_per_iter;
+    const unsigned granule = 2u * turn_rows;                       // the ring turns twice a trip through its loop
+    // iterations of a piece: a batch of a few rows leaves a wave a handful of them, and is cut finely
+    const unsigned piece_turns = (unsigned)((unsigned long long)all_sweeps * (a.out_rows / turn_rows) / gridDim.x);
+    auto chunk_turns_of = [&](unsigned n) -> unsigned {
+        unsigned turns = n >= 2u ? kSweepChunkTurns / 2u : kSweepChunkTurns;
+        while (turns > 2u && (turns * (4u * kSweepWaves) > piece_turns || (FUSED && turns * turn_rows > kFusedItemRows)))
+            turns /= 2u;
+        return turns;
     };
-    for (unsigned listed = draw(); listed < total_items; listed = draw()) {
-        const bool is_short = listed >= total_long;
-        const unsigned item = is_short ? listed - total_long : listed;   // within its zone of rows
-        const unsigned tiles = is_short ? short_tiles : long_tiles;
-        const unsigned rows_of_item = is_short ? short_rows : item_rows;
-        // class of the item, then (sweep of the class list, tile)
-        unsigned start = 0u, size = 0u, position = item;
-        bool found = false;
-        for (unsigned c = 0; c < 4u && !found; ++c) {
-            size = lds_load_u32(kClassCountBase + 4u * c);
-            if (position < size * tiles) {
-                found = true;
-            } else {
-                position -= size * tiles;
-                start += size;
+    struct Place {
+        unsigned slot, sweep, row;
+    };
+    const unsigned long long all_cost = (unsigned long long)row_cost * a.out_rows;
+    auto place_of = [&](unsigned who) -> Place {        // where the piece of workgroup `who` begins
+        if (who >= gridDim.x) return Place{buckets + 1u, 0u, 0u};
+        unsigned long long at = uniform64((unsigned long long)((double)all_cost * (double)who / (double)gridDim.x));
+        unsigned slot = 0u, n = extra_pairs;
+        if (at >= (unsigned long long)extra_cost * a.out_rows) {
+            at -= (unsigned long long)extra_cost * a.out_rows;
+            const unsigned long long below = __ballot((unsigned long long)(before & 0xffffu) * a.out_rows <= at);
+            const int holder = 63 - __builtin_clzll(below);
+            at -= (unsigned long long)((unsigned)__builtin_amdgcn_readlane((int)before, holder) & 0xffffu) * a.out_rows;
+            slot = 4u * (unsigned)holder + 1u;
+            n = (unsigned)__builtin_amdgcn_readlane((int)population[0], holder);
+#pragma unroll
+            for (unsigned j = 1; j < 4u; ++j) {
+                const unsigned long long rows = (unsigned long long)bucket_cost<QT>(n) * a.out_rows;
+                const unsigned behind = (unsigned)__builtin_amdgcn_readlane((int)population[j], holder);
+                if (slot == 4u * (unsigned)holder + j && at >= rows) {
+                    at -= rows;
+                    ++slot;
+                    n = behind;
+                }
             }
         }
-        if (!found) {
+        const unsigned full = n / 4u;
+        const unsigned long long sweep_rows = (unsigned long long)sweep_cost<QT>(4u) * a.out_rows;
+        unsigned sweep = uniform((unsigned)((double)at / (double)sweep_rows));
+        if ((unsigned long long)sweep * sweep_rows > at) --sweep;
+        if (sweep > full) sweep = full;
+        at -= (unsigned long long)sweep * sweep_rows;
+        const unsigned weight = sweep < full ? sweep_cost<QT>(4u) : sweep_cost<QT>(n % 4u);
+        unsigned row = uniform((unsigned)at / weight);
+        if (row > a.out_rows) row = a.out_rows;
+        // (the same in every lane: kept in scalar registers, of which the sweeps leave some)
+        return Place{uniform(slot), uniform(sweep), uniform(row & ~(granule - 1u))};
+    };
+    Place now = place_of(blockIdx.x);
+    const Place end = place_of(blockIdx.x + 1u);
+
+    // The first weight rows of the piece start on their way to the caches while the tables are
+    // built (64 bytes apart, so the lanes cover 4 KB of each stream).
+    unsigned warm[2] = {0u, 0u};
+    if (now.slot <= buckets) {
+        const unsigned bucket = now.slot ? now.slot - 1u : 0u;
+        unsigned expert = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)expert64[0], (int)(bucket >> 2));
+#pragma unroll
+        for (unsigned j = 1; j < 4u; ++j) {
+            const unsigned other = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)expert64[j], (int)(bucket >> 2));
+            if ((bucket & 3u) == j) expert = other;
+        }
+        const GroupedProblem &pr = a.problem[now.slot == 0u ? a.problems - 1u : 0u];
+        if (now.slot == 0u) expert = 0u;
+        const unsigned rows_left = a.out_rows - now.row;
+        unsigned long long offset = 64ull * lane;
+        const unsigned long long bytes_left = rows_left * pr.row_bytes;
+        if (bytes_left >= 8ull) {
+            if (offset + 4ull > bytes_left) offset = bytes_left - 4ull;
+            const unsigned char *rows = pr.gate + expert * pr.expert_bytes + now.row * pr.row_bytes;
+            warm[0] = *reinterpret_cast<const unsigned *>(rows + (offset & ~3ull));
+            if (FUSED) {
+                warm[1] = *reinterpret_cast<const unsigned *>(pr.up + expert * pr.up_expert_bytes +
+                                                              now.row * pr.up_row_bytes + (offset & ~3ull));
+            } else if (offset + 4096ull + 4ull <= bytes_left) {
+                warm[1] = *reinterpret_cast<const unsigned *>(rows + 4096u + (offset & ~3ull));
+            }
+        }
+    }
+
+    if constexpr (QT == QT_IQ2_XXS) sweep_tables_fill(digits);
+    if (tid == 0u) lds_store_u32(kTicketAddress, 0u);
+    if (wave == 0u) {
+        unsigned sweeps_before = before >> 16;
+#pragma unroll
+        for (unsigned j = 0; j < 4u; ++j) {
+            lds_store_uint4(kBucketBase + 16u * (4u * lane + j),
+                            make_uint4((unsigned)expert64[j], (unsigned)first64[j], population[j], sweeps_before));
+            sweeps_before += (population[j] + 3u) / 4u;
+        }
+    }
+    if (pairs_in_lds) {
+        float weight_here[2];
+#pragma unroll
+        for (unsigned k = 0; k < 2u; ++k)   // a source outside the problem reads no weight here; the sweep's own checks refuse it
+            weight_here[k] = routed.route_weights && source_here[k] < routed.pairs
+                ? routed.route_weights[source_here[k]] : 1.0f;
+#pragma unroll
+        for (unsigned k = 0; k < 2u; ++k)
+            if (tid + k * kSweepThreads < routed.pairs)
+                lds_store_uint2(kPairCacheBase + 8u * (tid + k * kSweepThreads),
+                                make_uint2(source_here[k] < 0xffffffffull ? (unsigned)source_here[k] : 0xffffffffu,
+                                           __float_as_uint(weight_here[k])));
+    }
+    __syncthreads();
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" ::"v"(warm[0]), "v"(warm[1]));
+#endif
+
+    // ---- the piece: its sweeps one after another, each with the chunks of its rows ----
+    unsigned drawn = draw_chunk(), base = 0u;
+    while (now.slot < end.slot || (now.slot == end.slot &&
+                                   (now.sweep < end.sweep || (now.sweep == end.sweep && now.row < end.row)))) {
+        const unsigned slot = now.slot, sweep = now.sweep, row_begin = now.row;
+        const bool last = slot == end.slot && sweep == end.sweep;
+        const unsigned row_end = last ? end.row : a.out_rows;
+        const bool is_routed = slot != 0u;
+        const GroupedProblem &pr = a.problem[!is_routed && a.problems > 1u ? 1u : 0u];
+        unsigned long long expert = 0ull, first = 0ull;
+        unsigned n = extra_pairs;
+        if (is_routed) {
+            const uint4 bucket = lds_read_uint4(kBucketBase + 16u * (slot - 1u));
+            expert = uniform(bucket.x);
+            first = uniform(bucket.y);
+            n = uniform(bucket.z);
+        }
+        now.row = 0u;
+        if ((sweep + 1u) * 4u < n) {
+            ++now.sweep;
+        } else {
+            now.sweep = 0u;
+            ++now.slot;
+        }
+        if (last) now = end;
+        const unsigned pass = sweep * (unsigned)kSweepPairs;
+        if (pass >= n || row_begin >= row_end) continue;
+        if (first + n > pr.pairs) {
             if (lane == 0u) raise_status(a.status, 2);
             continue;
         }
-        const unsigned tile = position % tiles;
-        const unsigned word = lds_load_u32(kClassListBase + 4u * (start + position / tiles));
-        const GroupedProblem &pr = a.problem[(word & 0x40000000u) && a.problems > 1u ? 1u : 0u];
-        unsigned long long expert = 0ull, first = 0ull, population = pr.pairs;
-        const bool is_routed = !(word & 0x40000000u);
-        if (!(word & 0x80000000u)) {
-            const unsigned bucket = (word >> 16) & 0x3fffu;
-            if (is_routed) {          // the routed problem's buckets were copied at kernel start
-                expert = lds_load_u32(kBucketBase + 12u * bucket);
-                first = lds_load_u32(kBucketBase + 12u * bucket + 4u);
-                population = lds_load_u32(kBucketBase + 12u * bucket + 8u);
-            } else {
-                expert = pr.expert_ids[bucket];
-                first = pr.bucket_offsets[bucket];
-                population = pr.bucket_populations[bucket];
-            }
+        const unsigned live = n - pass < 4u ? n - pass : 4u;
+        const unsigned chunk_turns = chunk_turns_of(live);
+        const unsigned chunk_rows = chunk_turns * turn_rows;
+        const unsigned chunks = (row_end - row_begin + chunk_rows - 1u) / chunk_rows;
+        if (drawn - base < chunks) {
+            const unsigned char *gate_e = pr.gate + expert * pr.expert_bytes;
+            const unsigned char *up_e = FUSED ? pr.up + expert * pr.up_expert_bytes : nullptr;
+            const bool cached = pairs_in_lds && is_routed;
+            const unsigned chunk = drawn - base;
+            static_assert(kSweepPairs == 4, "a sweep serves one to four pairs");
+            if (live == 4u)
+                drawn = iq2_sweep<MODE, 4, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached, chunk, base, chunk_turns);
+            else if (live == 3u)
+                drawn = iq2_sweep<MODE, 3, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached, chunk, base, chunk_turns);
+            else if (live == 2u)
+                drawn = iq2_sweep<MODE, 2, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached, chunk, base, chunk_turns);
+            else
+                drawn = iq2_sweep<MODE, 1, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached, chunk, base, chunk_turns);
         }
-        const unsigned long long pass = (unsigned long long)(word & 0xffffu) * kSweepPairs;
-        if (expert >= pr.experts || first + population > pr.pairs || pass >= population) {
-            if (lane == 0u) raise_status(a.status, 2);
-            continue;
-        }
-        const unsigned char *gate_e = pr.gate + expert * pr.expert_bytes;
-        const unsigned char *up_e = FUSED ? pr.up + expert * pr.up_expert_bytes : nullptr;
-        const unsigned row_begin = (is_short ? long_rows : 0u) + tile * rows_of_item;
-        const unsigned row_end = row_begin + rows_of_item < a.out_rows ? row_begin + rows_of_item : a.out_rows;
-        const unsigned long long live = population - pass;
-        const bool cached = pairs_in_lds && is_routed;
-        if (kSweepPairs >= 4 && live >= 4ull)
-            iq2_sweep<MODE, kSweepPairs >= 4 ? 4 : 1, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached);
-        else if (kSweepPairs >= 3 && live >= 3ull)
-            iq2_sweep<MODE, kSweepPairs >= 3 ? 3 : 1, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached);
-        else if (live >= 2ull)
-            iq2_sweep<MODE, 2, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached);
-        else
-            iq2_sweep<MODE, 1, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached);
+        base += chunks;
     }
 }
 
@@ -1031,7 +1101,7 @@ bool iq2_sweep_supported(unsigned qtype, unsigned width, unsigned out_rows, unsi
 {
     if (qtype != QT_IQ2_XXS && qtype != QT_Q4_K && qtype != QT_Q2_K) return false;
     if (image && qtype != QT_IQ2_XXS) return false;
-    if (pairs > kClassMaxSweeps) return false;            // every sweep serves at least one pair
+    if (pairs > kMaxSweeps) return false;            // every sweep serves at least one pair
     const unsigned lanes_per_row = width / 128u;
     if (width % 256u != 0u || lanes_per_row < 16u || lanes_per_row > 64u) return false;
     // IQ2_XXS rows must start on dword boundaries (Q4_K rows are multiples of 144 bytes, Q2_K rows of 84)
