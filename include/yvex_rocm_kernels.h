@@ -99,6 +99,21 @@ int yvex_hip_matvec_f32_rows_scored(const float *weights, uint64_t row_count, ui
                                     void *scratch, uint64_t scratch_bytes, int *status,
                                     yvex_hip_stream stream);
 
+/* The router of a row batch in two launches: yvex_hip_matvec_f32_rows (split form) followed by
+ * yvex_hip_moe_route_rows on its logits, the joining of the partial sums and the routing in one
+ * launch, a workgroup a row. weights is [row_count <= 256 experts, row_width]. UNSUPPORTED where
+ * yvex_hip_matvec_f32_rows_launches says 1 for the operands. */
+int yvex_hip_matvec_f32_rows_routed(const float *weights, uint64_t row_count, uint64_t row_width,
+                                    const float *input, uint64_t input_rows, uint64_t input_stride,
+                                    float *logits, const float *bias, uint64_t topk, int scoring, int normalize,
+                                    double scaling, uint64_t *selected, float *route_weights, void *scratch,
+                                    uint64_t scratch_bytes, int *status, yvex_hip_stream stream);
+/* yvex_hip_matvec of two Q8_0 matrices of one shape against the same Q8_K input rows, in one launch. */
+int yvex_hip_matvec_q8_0_pair(const uint8_t *first, const uint8_t *second, uint64_t row_count,
+                              uint64_t row_width, uint64_t row_bytes, const void *input_q8k,
+                              uint64_t input_rows, float *out_first, float *out_second, int *status,
+                              yvex_hip_stream stream);
+
 /* Replaces yvex_argmax_f32 (kernels.cu:59-110): for each of row_count (<= 65535) rows of
  * row_width (< 2^32) F32 values the largest value, the lowest index holding it and the number of
  * elements holding it. A non-finite element raises status 1 and its row publishes nothing.
@@ -193,6 +208,14 @@ int yvex_hip_moe_prepare_scored(const float *scores, const float *bias, uint64_t
                                 uint64_t width, uint64_t input_stride, uint8_t *encoded, int *status,
                                 yvex_hip_stream stream);
 
+/* yvex_hip_moe_prepare for rows that are routed already (yvex_hip_matvec_f32_rows_routed): the
+ * worklist and the quantization. rows <= 512. */
+int yvex_hip_moe_prepare_routed(const uint64_t *selected, uint64_t rows, uint64_t experts, uint64_t topk,
+                                uint64_t *order, uint64_t *expert_ids, uint64_t *bucket_offsets,
+                                uint64_t *bucket_populations, uint64_t *sweep_offsets, uint64_t *counts,
+                                const float *values, uint64_t width, uint64_t input_stride, uint8_t *encoded,
+                                int *status, yvex_hip_stream stream);
+
 /* Expert matrices of one MoE layer. routed_* are expert-major: expert e starts at
  * base + e * expert_bytes and holds rows * row_bytes canonical GGUF bytes. gate_up_image /
  * down_image say that those IQ2_XXS matrices are given as the sweep image of
@@ -280,6 +303,13 @@ int yvex_hip_moe_down_rows(const yvex_hip_expert_weights *weights, const void *i
 int yvex_hip_moe_swiglu_rows(const float *gate, const float *up, uint64_t count, double limit,
                              float *out, int *status, yvex_hip_stream stream);
 
+/* yvex_hip_q8k_quantize of `rows` rows and, behind them in the same launch, of `shared_rows` rows whose
+ * values are yvex_hip_moe_swiglu_rows of gate and up sums. width % 256 == 0, F32 operands 16-byte
+ * aligned and dense. A value that is not finite raises status 1. */
+int yvex_hip_q8k_quantize_swiglu(const float *values, uint64_t rows, uint64_t width, uint8_t *encoded,
+                                 const float *gate, const float *up, uint64_t shared_rows, double limit,
+                                 uint8_t *shared_encoded, int *status, yvex_hip_stream stream);
+
 /* Replaces yvex_moe_reduce_rows + yvex_moe_combine_rows (moe_kernels.cu:584-616):
  * routed[row, c] = sum over rank (in rank order, fp32) of pair_outputs[row*topk+rank, c];
  * combined[row, c] = bf16(routed + shared) when shared != NULL and combined != NULL. */
@@ -322,6 +352,13 @@ int yvex_hip_mhc_ingress_encoded(const float *rows, const float *mixes, const vo
 int yvex_hip_mhc_egress(const float *core, const float *rows, const float *post,
                         const float *combination, uint64_t row_count, uint64_t streams,
                         uint64_t width, float *output, int *status, yvex_hip_stream stream);
+/* yvex_hip_moe_reduce_combine and yvex_hip_mhc_egress of its combined rows in one launch, which
+ * publishes the egress only. streams == 4, width % 4 == 0, 16-byte aligned operands (else
+ * UNSUPPORTED). */
+int yvex_hip_moe_combine_egress(const float *pair_outputs, uint64_t row_count, uint64_t topk, uint64_t streams,
+                                uint64_t width, const float *shared, const float *rows, const float *post,
+                                const float *combination, float *output, int *status, yvex_hip_stream stream);
+
 
 /* Bandwidth probe (the reference publishes the same fact at backend start,
  * src/backend/cuda/backend.c:1550): streams `bytes` of device memory through 16-byte loads.

@@ -38,7 +38,17 @@ struct DenseQ80Args {
     unsigned long long out_stride;
     int output_bf16;
     int *status;
+    const unsigned char *encoded_second;     // a second matrix of the same shape (blockIdx.z = 1), or null
+    float *out_second;
 };
+
+__device__ __forceinline__ void choose_matrix(DenseQ80Args &g)
+{
+    if (blockIdx.z) {
+        g.encoded = g.encoded_second;
+        g.out = g.out_second;
+    }
+}
 
 // What a lane needs of one superblock: its half of the eight blocks' codes (their scales lie in
 // the same windows) and its half of one input row's blocks.
@@ -82,6 +92,7 @@ __global__ __launch_bounds__(64 * kPlainWaves) void dense_q8_0_kernel(DenseQ80Ar
     // per wave: the scales of the input rows whose blocks its lanes hold; then the partial tiles
     __shared__ __align__(16) float row_scale[kPlainWaves][32];
     __shared__ double partial[kPlainWaves - 1u][16][64];
+    choose_matrix(g);
     const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const unsigned r = lane & 31u, h = lane >> 5;
     const unsigned long long row0 = (unsigned long long)blockIdx.x * 32ull;
@@ -246,6 +257,7 @@ __global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS) void dense_q8_0_sta
         if (threadIdx.x == 0u) raise_status(g.status, 2);
         return;
     }
+    choose_matrix(g);
     const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const unsigned r = lane & 31u, h = lane >> 5;
     const unsigned row_block = wave % ROW_BLOCKS, token_block = wave / ROW_BLOCKS;
@@ -400,16 +412,18 @@ __global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS) void dense_q8_0_sta
 int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t row_width,
                            uint64_t row_bytes, const void *act_q8k, uint64_t input_rows,
                            const float *additive, float *out, uint64_t out_stride, bool output_bf16,
-                           int *status, hipStream_t stream)
+                           int *status, hipStream_t stream, const uint8_t *encoded_second, float *out_second)
 {
+    const uint64_t matrices = encoded_second ? 2u : 1u;
     if (!row_count || !input_rows || row_width % 256u || row_width / 32u * 34u != row_bytes)
         return ST_BOUNDS;
-    if (((uintptr_t)encoded & 3u) || ((uintptr_t)act_q8k & 3u)) return ST_INVALID_ARG;
+    if ((((uintptr_t)encoded | (uintptr_t)encoded_second) & 3u) || ((uintptr_t)act_q8k & 3u)) return ST_INVALID_ARG;
+    const bool aligned16 = !(((uintptr_t)encoded | (uintptr_t)encoded_second) & 15u);
     const uint64_t row_tiles = (row_count + 31u) / 32u;
     if (row_tiles > 0x7fffffffull || row_width / 256u > 0xffffffffull) return ST_BOUNDS;
     DenseQ80Args g{encoded, row_count, row_bytes, (unsigned)(row_width / 256u),
                    (const unsigned char *)act_q8k, input_rows, additive, out, out_stride,
-                   output_bf16 ? 1 : 0, status};
+                   output_bf16 ? 1 : 0, status, encoded_second, out_second};
     // Which tiles: a pass over the row width costs a workgroup about the same whatever the device's
     // load (measured at 16 superblocks a row, microseconds: 17 unstaged and 27 once two such
     // workgroups share a compute unit, 29 on the 64-row staged tile and 43 once two of them share
@@ -421,33 +435,34 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
     // up to 32 input rows against a matrix with a 256-row tile for every compute unit (an output
     // head at decode width, 129 280 x 7168: 306 us on the 128 x 64 tiles, half of them padding;
     // memory time 173 us)
-    if (!((uintptr_t)encoded & 15u) && input_rows <= 32u && units && (row_count + 255u) / 256u >= units) {
+    if (aligned16 && input_rows <= 32u && units && matrices * ((row_count + 255u) / 256u) >= units) {
         YVEX_ALLOW_DYNAMIC_LDS((dense_q8_0_staged_kernel<8u, 1u>), staged_lds_bytes(8u, 1u));
-        dense_q8_0_staged_kernel<8u, 1u><<<dim3((unsigned)((row_count + 255u) / 256u), 1), 512, staged_lds_bytes(8u, 1u),
+        dense_q8_0_staged_kernel<8u, 1u><<<dim3((unsigned)((row_count + 255u) / 256u), 1, (unsigned)matrices), 512, staged_lds_bytes(8u, 1u),
                                            stream>>>(g);
         return check_launch("dense_q8_0_staged");
     }
-    if (!((uintptr_t)encoded & 15u) && units) {
-        const uint64_t plain = row_tiles * token_tiles32;
-        const uint64_t tall = (row_count + 127u) / 128u * token_tiles64, low = (row_count + 63u) / 64u * token_tiles64;
+    if (aligned16 && units) {
+        const uint64_t plain = matrices * row_tiles * token_tiles32;
+        const uint64_t tall = matrices * ((row_count + 127u) / 128u) * token_tiles64,
+                       low = matrices * ((row_count + 63u) / 64u) * token_tiles64;
         const double plain_cost = plain <= units ? 17.0 : 27.0 * (double)((plain + 2u * units - 1u) / (2u * units));
         const double low_share = 43.0 * (double)low / (double)(2u * units);
         const double low_cost = low <= units ? 29.0 : (low_share > 43.0 ? low_share : 43.0);
         const double tall_cost = 35.0 * (double)((tall + units - 1u) / units);
         if (tall_cost < plain_cost && tall_cost <= low_cost) {
             YVEX_ALLOW_DYNAMIC_LDS(dense_q8_0_staged_kernel<4u>, staged_lds_bytes(4u));
-            dense_q8_0_staged_kernel<4u><<<dim3((unsigned)((row_count + 127u) / 128u), (unsigned)token_tiles64), 512,
+            dense_q8_0_staged_kernel<4u><<<dim3((unsigned)((row_count + 127u) / 128u), (unsigned)token_tiles64, (unsigned)matrices), 512,
                                           staged_lds_bytes(4u), stream>>>(g);
             return check_launch("dense_q8_0_staged");
         }
         if (low_cost < plain_cost) {
             YVEX_ALLOW_DYNAMIC_LDS(dense_q8_0_staged_kernel<2u>, staged_lds_bytes(2u));
-            dense_q8_0_staged_kernel<2u><<<dim3((unsigned)((row_count + 63u) / 64u), (unsigned)token_tiles64), 256,
+            dense_q8_0_staged_kernel<2u><<<dim3((unsigned)((row_count + 63u) / 64u), (unsigned)token_tiles64, (unsigned)matrices), 256,
                                           staged_lds_bytes(2u), stream>>>(g);
             return check_launch("dense_q8_0_staged");
         }
     }
-    dense_q8_0_kernel<<<dim3((unsigned)row_tiles, (unsigned)token_tiles32), 64 * kPlainWaves, 0, stream>>>(g);
+    dense_q8_0_kernel<<<dim3((unsigned)row_tiles, (unsigned)token_tiles32, (unsigned)matrices), 64 * kPlainWaves, 0, stream>>>(g);
     return check_launch("dense_q8_0");
 }
 

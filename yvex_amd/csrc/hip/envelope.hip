@@ -73,6 +73,41 @@ __device__ __forceinline__ float4 coefficient4(const void *values, unsigned qtyp
                        __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
 }
 
+// A double moved by a data-parallel-primitive step (both halves).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v)
+{
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
+    const unsigned low = (unsigned)dpp_move<CTRL, 0xf>((int)(unsigned)bits);
+    const unsigned high = (unsigned)dpp_move<CTRL, 0xf>((int)(unsigned)(bits >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)high << 32) | low));
+}
+
+// Alternating row and column normalisations of a 4 x 4 matrix, one element a lane (4 row + column,
+// repeated in each group of sixteen lanes). The totals are two additions each way inside the row of
+// sixteen lanes, on the vector ALU; sums of four floats of a matrix whose elements lie within a
+// factor of 2^29 are exact in double, so the order of the additions does not show. Gathering the
+// four elements with lane permutes through LDS, one waited for after another, took 0.4 us a turn
+// (twenty of them: 8 of the 18 us of a one-row launch); 0.15 us now.
+__device__ __forceinline__ float sinkhorn4(float m, unsigned iterations, double epsilon, bool &bad)
+{
+    for (unsigned it = 0; it < iterations; ++it) {
+        if (it != 0u) {
+            double across = (double)m;
+            across += dpp_f64<0xb1>(across);       // quad_perm [1, 0, 3, 2]
+            across += dpp_f64<0x4e>(across);       // quad_perm [2, 3, 0, 1]
+            bad |= !finite_f64(across);
+            m = (float)((double)m / (across + epsilon));
+        }
+        double down = (double)m;
+        down += dpp_f64<0x128>(down);              // row_ror 8, row_ror 4
+        down += dpp_f64<0x124>(down);
+        bad |= !finite_f64(down);
+        m = (float)((double)m / (down + epsilon));
+    }
+    return m;
+}
+
 // One workgroup per row. The row is read twice (mean square, then the gated sum of the streams);
 // both passes keep four 16-byte loads per thread in flight, because a row is a short stream and
 // a loop that waits for each load in turn spends its time on latency; long rows take 1024
@@ -155,9 +190,11 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
     // over the row meanwhile.
     const unsigned cells = streams * streams;
     if (tid < 64u) {
-        const bool cell = tid < cells;
-        const unsigned r = cell ? tid / streams : 0u, c = cell ? tid % streams : 0u;
-        const unsigned index = 2u * streams + (cell ? tid : 0u);
+        // (four streams: every group of sixteen lanes holds the matrix)
+        const unsigned held = streams == 4u ? tid & 15u : tid;
+        const bool cell = held < cells;
+        const unsigned r = cell ? held / streams : 0u, c = cell ? held % streams : 0u;
+        const unsigned index = 2u * streams + (cell ? held : 0u);
         float m = (float)((double)mix[index] * inverse * (double)scale[2] + (double)base[index]);
         double maximum = -__builtin_inf(), total = 0.0, mine = 0.0;
         for (unsigned k = 0; k < streams; ++k)
@@ -169,7 +206,8 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
         }
         bad |= cell && (!finite_f64(total) || !(total > 0.0));
         m = (float)((double)(float)mine / total + mhc_epsilon);
-        for (unsigned it = 0; it < iterations; ++it) {
+        if (streams == 4u) m = sinkhorn4(m, iterations, mhc_epsilon, bad);
+        else for (unsigned it = 0; it < iterations; ++it) {
             if (it != 0u) {
                 double across = 0.0;
                 for (unsigned k = 0; k < streams; ++k) across += (double)__shfl(m, (int)(r * streams + k), kWave);
@@ -181,7 +219,7 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
             bad |= cell && !finite_f64(down);
             m = (float)((double)m / (down + mhc_epsilon));
         }
-        if (cell) combination[row * cells + tid] = m;
+        if (tid < cells) combination[row * cells + tid] = m;
     }
 
     // collapsed row: float accumulation over the streams in order, then bf16
@@ -312,6 +350,77 @@ __global__ __launch_bounds__(kEnvelopeThreads) void mhc_egress_kernel(
     if (bad) raise_status(status, 1);
 }
 
+// The rank-ordered sum of the pairs' outputs, the shared expert and the egress in one pass over a
+// row's columns (yvex_hip_moe_reduce_combine followed by yvex_hip_mhc_egress, the same operations in
+// the same order): the combined row never goes to memory, and a decode batch has a launch less
+// (5 us of 11 at one row).
+template <unsigned STREAMS>
+__global__ __launch_bounds__(kEnvelopeThreads) void combine_egress_kernel(
+    const float *__restrict__ pair_outputs, unsigned topk, const float *__restrict__ shared,
+    const float *__restrict__ rows, const float *__restrict__ post, const float *__restrict__ combination,
+    unsigned long long row_count, unsigned width, unsigned blocks_per_row, float *__restrict__ output, int *status)
+{
+    const unsigned long long row = blockIdx.x / blocks_per_row;
+    const unsigned lane = ((blockIdx.x % blocks_per_row) * kEnvelopeThreads + threadIdx.x) * 4u;
+    if (row >= row_count || lane >= width) return;
+    const unsigned expanded = STREAMS * width;
+    const float *in = rows + row * expanded + lane;
+    float4 loaded[STREAMS];
+#pragma unroll
+    for (unsigned s = 0; s < STREAMS; ++s) loaded[s] = *reinterpret_cast<const float4 *>(in + s * width);
+    const float4 base = *reinterpret_cast<const float4 *>(shared + row * width + lane);
+    double gain[STREAMS], weight[STREAMS][STREAMS];
+#pragma unroll
+    for (unsigned t = 0; t < STREAMS; ++t) {
+        gain[t] = (double)post[row * STREAMS + t];
+#pragma unroll
+        for (unsigned s = 0; s < STREAMS; ++s) weight[s][t] = (double)combination[(row * STREAMS + s) * STREAMS + t];
+    }
+    // ranks in order, four of them in flight
+    float total[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const float *source = pair_outputs + row * topk * width + lane;
+    for (unsigned rank = 0; rank < topk; rank += 4u) {
+        float4 part[4];
+#pragma unroll
+        for (unsigned k = 0; k < 4u; ++k)
+            part[k] = *reinterpret_cast<const float4 *>(source + (unsigned long long)(rank + k < topk ? rank + k : topk - 1u) * width);
+#pragma unroll
+        for (unsigned k = 0; k < 4u; ++k) {
+            if (rank + k >= topk) break;
+            total[0] += part[k].x;
+            total[1] += part[k].y;
+            total[2] += part[k].z;
+            total[3] += part[k].w;
+        }
+    }
+    bool bad = false;
+    double value[4];
+    const float shared_lane[4] = {base.x, base.y, base.z, base.w};
+#pragma unroll
+    for (unsigned i = 0; i < 4u; ++i) {
+        const float combined = bf16_round(total[i] + shared_lane[i]);
+        bad |= !finite_f32(total[i]) || !finite_f32(combined);
+        value[i] = (double)combined;
+    }
+#pragma unroll
+    for (unsigned t = 0; t < STREAMS; ++t) {
+        float packed[4];
+#pragma unroll
+        for (unsigned i = 0; i < 4u; ++i) {
+            double sum = gain[t] * value[i];
+#pragma unroll
+            for (unsigned s = 0; s < STREAMS; ++s)
+                sum += weight[s][t] * (double)bf16_round(reinterpret_cast<const float *>(&loaded[s])[i]);
+            const float published = (float)sum;
+            bad |= !finite_f64(sum) || !finite_f32(published);
+            packed[i] = bf16_round(published);
+        }
+        *reinterpret_cast<float4 *>(output + row * expanded + t * width + lane) =
+            make_float4(packed[0], packed[1], packed[2], packed[3]);
+    }
+    if (bad) raise_status(status, 1);
+}
+
 }  // namespace yvex
 
 using namespace yvex;
@@ -417,4 +526,24 @@ extern "C" int yvex_hip_mhc_egress(const float *core, const float *rows, const f
             core, rows, post, combination, row_count, (unsigned)streams, (unsigned)width, blocks_per_row,
             output, status);
     return check_launch("mhc_egress");
+}
+
+// Four streams, widths of whole 16-byte pieces; UNSUPPORTED otherwise (the two launches serve those).
+extern "C" int yvex_hip_moe_combine_egress(const float *pair_outputs, uint64_t row_count, uint64_t topk,
+                                           uint64_t streams, uint64_t width, const float *shared, const float *rows,
+                                           const float *post, const float *combination, float *output, int *status,
+                                           yvex_hip_stream stream)
+{
+    if (!pair_outputs || !shared || !rows || !post || !combination || !output || !status || output == rows || !topk ||
+        topk > 0xffffu)
+        return ST_INVALID_ARG;
+    if (!envelope_shape_ok(row_count, streams, width)) return ST_BOUNDS;
+    if (streams != 4u || width % 4u ||
+        (((uintptr_t)pair_outputs | (uintptr_t)shared | (uintptr_t)rows | (uintptr_t)output) & 15u))
+        return ST_UNSUPPORTED;
+    const unsigned blocks_per_row = (unsigned)((width / 4u + kEnvelopeThreads - 1u) / kEnvelopeThreads);
+    combine_egress_kernel<4><<<(unsigned)(row_count * blocks_per_row), kEnvelopeThreads, 0, as_stream(stream)>>>(
+        pair_outputs, (unsigned)topk, shared, rows, post, combination, row_count, (unsigned)width, blocks_per_row,
+        output, status);
+    return check_launch("moe_combine_egress");
 }

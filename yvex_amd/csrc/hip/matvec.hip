@@ -12,6 +12,7 @@
 #include "common.hpp"
 #include "launch.hpp"
 #include "units.hpp"
+#include "route.hpp"
 
 namespace yvex {
 
@@ -28,6 +29,8 @@ struct MatvecArgs {
     double *parts;           // split projections: [split][input row][weight row] partial sums
     float *scores;           // join of a split projection: the router scores of the outputs as well
     int scoring;
+    const unsigned char *encoded_second = nullptr;   // a second matrix of the same shape (blockIdx.z = 1)
+    float *out_second = nullptr;
 };
 
 __device__ __forceinline__ void matvec_publish(const MatvecArgs &a, unsigned long long in,
@@ -67,6 +70,10 @@ __global__ __launch_bounds__(256) void matvec_block_kernel(MatvecArgs a)
     __shared__ Iq2Tables tables;
     extern __shared__ __align__(16) float4 staged_row[];
     const unsigned long long in0 = (unsigned long long)blockIdx.y * T;
+    if (blockIdx.z) {
+        a.encoded = a.encoded_second;
+        a.out = a.out_second;
+    }
     if constexpr (STAGE) {
         const float4 *source = reinterpret_cast<const float4 *>((const float *)a.input + in0 * a.input_stride);
         const unsigned pieces = (unsigned)(a.row_width >> 2);
@@ -789,6 +796,44 @@ __global__ __launch_bounds__(256) void matvec_f32_join_kernel(MatvecArgs a, unsi
     }
 }
 
+// The second launch of a router's split projection: one workgroup joins a row's partial sums, scores
+// them and routes the row, a thread an expert and then one wavefront (route.hpp). With the rows'
+// routing in workgroups of their own the launch behind this one is left with the worklist; when its
+// one routing workgroup took sixteen rows at a time, 96 rows cost 26 us there, 9 us now.
+__global__ __launch_bounds__(256) void matvec_f32_join_route_kernel(
+    MatvecArgs a, unsigned splits, const float *__restrict__ bias, unsigned topk, int normalize, double scaling,
+    unsigned long long *__restrict__ selected, float *__restrict__ weights)
+{
+    __shared__ float scores[256];
+    const unsigned experts = (unsigned)a.row_count, e = threadIdx.x;
+    const unsigned long long in = blockIdx.x, outputs = a.input_rows * a.row_count, at = in * a.row_count + e;
+    RouteInputs row;
+    if (e < 64u)
+#pragma unroll
+        for (unsigned i = 0; i < 4u; ++i)          // the biases: on their way meanwhile
+            row.bias[i] = bias ? bias[4u * e + i < experts ? 4u * e + i : experts - 1u] : 0.0f;
+    if (e < experts) {
+        double part[16], sum = 0.0;
+#pragma unroll
+        for (unsigned z = 0; z < 16u; ++z) part[z] = z < splits ? a.parts[z * outputs + at] : 0.0;
+        sum = part[0];
+#pragma unroll
+        for (unsigned z = 1; z < 16u; ++z)
+            if (z < splits) sum += part[z];
+        for (unsigned z = 16u; z < splits; ++z) sum += a.parts[z * outputs + at];
+        matvec_publish(a, in, e, (float)sum);
+        const double s = route_score((double)(float)sum, a.scoring);
+        const float published = (float)s;
+        if (!(s == s) || !finite_f32(published)) raise_status(a.status, 1);
+        scores[e] = published;
+    }
+    __syncthreads();
+    if (e >= 64u) return;
+#pragma unroll
+    for (unsigned i = 0; i < 4u; ++i) row.value[i] = scores[4u * e + i < experts ? 4u * e + i : experts - 1u];
+    route_row(row, true, in, e, experts, topk, a.scoring, normalize, scaling, selected, weights, a.status);
+}
+
 // int32 block sums of the Q8_K path, produced by the same unit code the matvec runs.
 template <unsigned QT>
 __global__ __launch_bounds__(256) void block_dots_kernel(
@@ -867,6 +912,7 @@ template <unsigned QT, bool Q8, bool EVEN>
 static int launch_block_even(const MatvecArgs &a, hipStream_t stream)
 {
     const unsigned long long grid_x = (a.row_count + 3ull) / 4ull;
+    const unsigned grid_z = a.encoded_second ? 2u : 1u;
     if (grid_x > 0x7fffffffull) return ST_BOUNDS;
     if (a.input_rows == 1ull) {
         // Q8_K activations: four chunks (8192 columns) in flight for a matrix that takes many
@@ -875,15 +921,15 @@ static int launch_block_even(const MatvecArgs &a, hipStream_t stream)
         const bool deep = Q8 && (a.row_count * a.row_bytes >= (64ull << 20) || a.row_width > 2048ull);
         // one F32 input row of up to 12 288 values (48 KB) is staged in LDS
         const bool stage = !Q8 && a.row_width <= 12288ull && !((uintptr_t)a.input & 15u);
-        if (deep) matvec_block_kernel<QT, Q8, 1, Q8 ? 4 : 1, EVEN><<<dim3((unsigned)grid_x, 1), 256, 0, stream>>>(a);
+        if (deep) matvec_block_kernel<QT, Q8, 1, Q8 ? 4 : 1, EVEN><<<dim3((unsigned)grid_x, 1, grid_z), 256, 0, stream>>>(a);
         else if (stage)
-            matvec_block_kernel<QT, Q8, 1, 1, EVEN, !Q8><<<dim3((unsigned)grid_x, 1), 256,
+            matvec_block_kernel<QT, Q8, 1, 1, EVEN, !Q8><<<dim3((unsigned)grid_x, 1, grid_z), 256,
                                                             (size_t)a.row_width * 4u, stream>>>(a);
-        else matvec_block_kernel<QT, Q8, 1, 1, EVEN><<<dim3((unsigned)grid_x, 1), 256, 0, stream>>>(a);
+        else matvec_block_kernel<QT, Q8, 1, 1, EVEN><<<dim3((unsigned)grid_x, 1, grid_z), 256, 0, stream>>>(a);
     } else {
         const unsigned long long grid_y = (a.input_rows + 3ull) / 4ull;
         if (grid_y > 65535ull) return ST_BOUNDS;
-        matvec_block_kernel<QT, Q8, 4, 1, EVEN><<<dim3((unsigned)grid_x, (unsigned)grid_y), 256, 0, stream>>>(a);
+        matvec_block_kernel<QT, Q8, 4, 1, EVEN><<<dim3((unsigned)grid_x, (unsigned)grid_y, grid_z), 256, 0, stream>>>(a);
     }
     return check_launch("matvec");
 }
@@ -995,6 +1041,15 @@ static int launch_scalar_rows(const MatvecArgs &a, hipStream_t s)
     return check_launch("matvec_f32_tile16");
 }
 
+static bool q8_0_takes_matrix_cores(const uint8_t *encoded, uint64_t row_count, uint64_t row_bytes,
+                                    uint64_t input_rows)
+{
+    const unsigned long long matrix_bytes = row_count * row_bytes;
+    return !((uintptr_t)encoded & 3u) &&
+           (input_rows >= 16ull || (input_rows >= 2ull && matrix_bytes >= (32ull << 20)) ||
+            (input_rows >= 12ull && matrix_bytes >= (8ull << 20)));
+}
+
 extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint64_t row_count,
                                uint64_t row_width, uint64_t row_bytes, const void *input,
                                int input_q8, uint64_t input_rows, uint64_t input_stride,
@@ -1044,10 +1099,7 @@ extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint6
     // but 7168 x 7168 (55 MB) takes 15 us for one row, 21 for two and 66 for fifteen where the
     // matrix cores take 18.5, and an output head of 129 280 x 7168 171 us for one row, 336 for two
     // and 1.5 ms for fifteen where they take 200 to 235
-    const unsigned long long matrix_bytes = row_count * row_bytes;
-    if (qtype == QT_Q8_0 && input_q8 && !((uintptr_t)encoded & 3u) &&
-        (input_rows >= 16ull || (input_rows >= 2ull && matrix_bytes >= (32ull << 20)) ||
-         (input_rows >= 12ull && matrix_bytes >= (8ull << 20))))
+    if (qtype == QT_Q8_0 && input_q8 && q8_0_takes_matrix_cores(encoded, row_count, row_bytes, input_rows))
         return launch_q8_0_rows_dense(encoded, row_count, row_width, row_bytes, input, input_rows, additive, out,
                                       out_stride, output_bf16 != 0, status, s);
     // F32 rows against a batch of F32 input rows: the double-precision matrix cores; rows of F16
@@ -1089,6 +1141,29 @@ extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint6
     case QT_Q2_K: return launch_block_q<QT_Q2_K>(a, input_q8, s);
     default: return ST_UNSUPPORTED;
     }
+}
+
+// Two Q8_0 matrices of one shape against the same Q8_K input rows in one launch (a shared expert's gate
+// and up projections): each offers too few workgroups for the device on its own (2048 x 4096 against
+// 96 rows: 192 of them, 16 us a launch).
+extern "C" int yvex_hip_matvec_q8_0_pair(const uint8_t *first, const uint8_t *second, uint64_t row_count,
+                                         uint64_t row_width, uint64_t row_bytes, const void *input_q8k,
+                                         uint64_t input_rows, float *out_first, float *out_second,
+                                         int *status, yvex_hip_stream stream)
+{
+    if (!first || !second || !input_q8k || !out_first || !out_second || !status || !row_count || !row_width ||
+        !input_rows || (((uintptr_t)input_q8k | (uintptr_t)out_first | (uintptr_t)out_second) & 3u))
+        return ST_INVALID_ARG;
+    if (row_width % 256u || row_width / 32u * 34u != row_bytes || row_width > 0xffffffffull * 32ull) return ST_BOUNDS;
+    // (the kernels address both matrices the same way: the weaker alignment decides)
+    const uint8_t *alignment = (const uint8_t *)((uintptr_t)first | (uintptr_t)second);
+    if (q8_0_takes_matrix_cores(alignment, row_count, row_bytes, input_rows))
+        return launch_q8_0_rows_dense(first, row_count, row_width, row_bytes, input_q8k, input_rows, nullptr,
+                                      out_first, row_count, false, status, as_stream(stream), second, out_second);
+    MatvecArgs a{first, row_count, row_width, row_bytes, input_q8k, input_rows, row_width, nullptr, out_first,
+                 row_count, 0, status, nullptr, nullptr, 0, second, out_second};
+    return ((uintptr_t)alignment & 1u) == 0u ? launch_block_even<QT_Q8_0, true, true>(a, as_stream(stream))
+                                             : launch_block_even<QT_Q8_0, true, false>(a, as_stream(stream));
 }
 
 extern "C" int yvex_hip_block_dots_i32(const uint8_t *encoded, unsigned int qtype,
@@ -1208,6 +1283,7 @@ extern "C" unsigned int yvex_hip_matvec_f32_rows_launches(const float *weights, 
                                   scratch_bytes) ? 2u : 1u;
 }
 
+static int launch_f32_rows_parts(const MatvecArgs &a, yvex_hip_stream stream);
 static int launch_f32_rows_split(const MatvecArgs &a, yvex_hip_stream stream);
 
 extern "C" int yvex_hip_matvec_f32_rows(const float *weights, uint64_t row_count, uint64_t row_width,
@@ -1247,17 +1323,50 @@ extern "C" int yvex_hip_matvec_f32_rows_scored(const float *weights, uint64_t ro
     return launch_f32_rows_split(a, stream);
 }
 
+// The router of a row batch: the split projection whose second launch routes as well. Selections,
+// route weights and logits are those of yvex_hip_matvec_f32_rows followed by yvex_hip_moe_route_rows.
+extern "C" int yvex_hip_matvec_f32_rows_routed(const float *weights, uint64_t row_count, uint64_t row_width,
+                                               const float *input, uint64_t input_rows, uint64_t input_stride,
+                                               float *logits, const float *bias, uint64_t topk, int scoring,
+                                               int normalize, double scaling, uint64_t *selected,
+                                               float *route_weights, void *scratch, uint64_t scratch_bytes,
+                                               int *status, yvex_hip_stream stream)
+{
+    if (!logits || !selected || !route_weights || !status || (scoring != 0 && scoring != 1) || !topk ||
+        topk > 16u || topk > row_count || ((uintptr_t)logits & 3u))
+        return ST_INVALID_ARG;
+    if (row_count > 256u ||
+        !f32_rows_split_applies(weights, row_count, row_width, input, input_rows, input_stride, scratch,
+                                scratch_bytes))
+        return ST_UNSUPPORTED;
+    MatvecArgs a{(const unsigned char *)weights, row_count, row_width, row_width * 4u, input, input_rows,
+                 input_stride, nullptr, logits, row_count, 0, status, (double *)scratch, nullptr, scoring};
+    int rc = launch_f32_rows_parts(a, stream);
+    if (rc) return rc;
+    matvec_f32_join_route_kernel<<<(unsigned)input_rows, 256, 0, as_stream(stream)>>>(
+        a, f32_rows_splits(row_count, row_width, input_rows), bias, (unsigned)topk, normalize, scaling,
+        (unsigned long long *)selected, route_weights);
+    return check_launch("matvec_f32_rows.join_route");
+}
+
+static int launch_f32_rows_parts(const MatvecArgs &a, yvex_hip_stream stream)
+{
+    const uint64_t grid_x = (a.row_count + 15u) / 16u, grid_y = (a.input_rows + 15u) / 16u;
+    if (grid_x > 0x7fffffffull || grid_y > 65535ull) return ST_BOUNDS;
+    matvec_f32_tile16_kernel<4><<<dim3((unsigned)grid_x, (unsigned)grid_y,
+                                       f32_rows_splits(a.row_count, a.row_width, a.input_rows)), 256, 0,
+                                  as_stream(stream)>>>(a);
+    return check_launch("matvec_f32_rows.parts");
+}
+
 static int launch_f32_rows_split(const MatvecArgs &a, yvex_hip_stream stream)
 {
     const uint64_t row_count = a.row_count, input_rows = a.input_rows;
     const unsigned splits = f32_rows_splits(row_count, a.row_width, input_rows);
-    hipStream_t s = as_stream(stream);
-    const uint64_t grid_x = (row_count + 15u) / 16u, grid_y = (input_rows + 15u) / 16u;
     const uint64_t outputs = input_rows * row_count;
-    if (grid_x > 0x7fffffffull || grid_y > 65535ull || (outputs + 255u) / 256u > 0x7fffffffull) return ST_BOUNDS;
-    matvec_f32_tile16_kernel<4><<<dim3((unsigned)grid_x, (unsigned)grid_y, splits), 256, 0, s>>>(a);
-    int rc = check_launch("matvec_f32_rows.parts");
+    if ((outputs + 255u) / 256u > 0x7fffffffull) return ST_BOUNDS;
+    int rc = launch_f32_rows_parts(a, stream);
     if (rc) return rc;
-    matvec_f32_join_kernel<<<(unsigned)((outputs + 255u) / 256u), 256, 0, s>>>(a, splits);
+    matvec_f32_join_kernel<<<(unsigned)((outputs + 255u) / 256u), 256, 0, as_stream(stream)>>>(a, splits);
     return check_launch("matvec_f32_rows.join");
 }

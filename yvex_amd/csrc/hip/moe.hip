@@ -12,6 +12,7 @@
 #include "units.hpp"
 #include "grouped.hpp"
 #include "q8k.hpp"
+#include "route.hpp"
 
 namespace yvex {
 
@@ -28,117 +29,6 @@ __global__ __launch_bounds__(256) void route_scores_kernel(
     const float published = (float)s;
     if (!(s == s) || !finite_f32(published)) raise_status(status, 1);
     scores[i] = published;
-}
-
-// One wavefront per row; each lane scores four experts (experts <= 256).
-// Largest value of the 64 lanes, in every lane: butterflies inside each row of 16 lanes, then the
-// rows' results carried upward (lane 15 into the next row, lane 31 into the upper half) and the
-// last lane read back.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ unsigned dpp_max_u32(unsigned v)
-{
-    const unsigned other = (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROWS, 0xf, false);
-    return other > v ? other : v;
-}
-
-__device__ __forceinline__ unsigned wave_max_u32(unsigned v)
-{
-    v = dpp_max_u32<0xb1, 0xf>(v);    // quad_perm [1, 0, 3, 2]
-    v = dpp_max_u32<0x4e, 0xf>(v);    // quad_perm [2, 3, 0, 1]
-    v = dpp_max_u32<0x141, 0xf>(v);   // row_half_mirror
-    v = dpp_max_u32<0x140, 0xf>(v);   // row_mirror
-    v = dpp_max_u32<0x142, 0xa>(v);   // row_bcast15 into rows 1 and 3
-    v = dpp_max_u32<0x143, 0xc>(v);   // row_bcast31 into rows 2 and 3
-    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
-}
-
-// What a lane reads of one row: the logits (or the scores a launch before this one has
-// published: the float a double-precision score rounds to, what route_row works out from a logit
-// otherwise) and the correction biases of experts 4 lane .. 4 lane + 3. The loads depend on
-// nothing and sit under no condition on the lane (a lane past the last expert reads the last
-// one's again), so a caller can ask for a row's values while it routes the row before: under
-// `if (e < experts)` they were issued, and waited for, one expert after another.
-struct RouteInputs {
-    float value[4], bias[4];
-};
-
-__device__ __forceinline__ void route_inputs_load(RouteInputs &in, const float *__restrict__ values,
-                                                  const float *__restrict__ bias, unsigned long long row,
-                                                  unsigned lane, unsigned experts)
-{
-#pragma unroll
-    for (unsigned i = 0; i < 4u; ++i) {
-        const unsigned e = lane * 4u + i < experts ? lane * 4u + i : experts - 1u;
-        in.value[i] = values[row * experts + e];
-        in.bias[i] = bias ? bias[e] : 0.0f;
-    }
-}
-
-// One row by one wavefront. `published`: in.value holds scores, not logits.
-__device__ __forceinline__ void route_row(
-    const RouteInputs &in, bool published, unsigned long long row, unsigned lane,
-    unsigned experts, unsigned topk, int scoring, int normalize, double scaling,
-    unsigned long long *__restrict__ selected, float *__restrict__ weights, int *status)
-{
-    float score[4];
-    unsigned long long key[4];
-#pragma unroll
-    for (unsigned i = 0; i < 4u; ++i) {
-        const unsigned e = lane * 4u + i;
-        score[i] = 0.0f;
-        key[i] = 0ull;
-        if (e < experts) {
-            if (published) {
-                score[i] = in.value[i];
-            } else {
-                const double s = route_score((double)in.value[i], scoring);
-                score[i] = (float)s;      // (a NaN stays a NaN)
-            }
-            float biased = in.bias[i] + score[i];
-            if (!finite_f32(score[i]) || !finite_f32(biased)) raise_status(status, 1);
-            biased += 0.0f;   // -0 and +0 must compare equal
-            const unsigned bits = __float_as_uint(biased);
-            const unsigned sortable = (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);
-            // larger score first, then the lower expert ordinal; +1 keeps live keys non-zero
-            key[i] = ((unsigned long long)sortable << 32) | (unsigned long long)(0xfffffffeu - e + 1u);
-        }
-    }
-    double total = 0.0;
-    float picked_score = 0.0f;   // lane r keeps the score of rank r
-    for (unsigned rank = 0; rank < topk; ++rank) {
-        unsigned long long best = key[0];
-#pragma unroll
-        for (unsigned i = 1; i < 4u; ++i) best = key[i] > best ? key[i] : best;
-        // The wave's best key in two steps that need no cross-lane permutes through LDS: the
-        // largest score word, then the first lane holding it (a lane's ordinals are below the
-        // next lane's, and its own best already is its lowest ordinal with that score).
-        const unsigned top = wave_max_u32((unsigned)(best >> 32));
-        const unsigned long long holders = __ballot((unsigned)(best >> 32) == top);
-        const unsigned winner = (unsigned)__builtin_ctzll(holders);
-        const unsigned e = 0xffffffffu - (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(best & 0xffffffffull),
-                                                                             (int)winner);
-        float s = 0.0f;
-#pragma unroll
-        for (unsigned i = 0; i < 4u; ++i)
-            if (lane * 4u + i == e) {
-                s = score[i];
-                key[i] = 0ull;
-            }
-        // (the winner's ordinal is the same in every lane: a lane read, no permute through LDS)
-        s = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), (int)(e >> 2)));
-        total += (double)s;                 // rank order, in double (src/graph/moe.c:566-574)
-        if (lane == rank) picked_score = s;
-        if (lane == 0u) selected[row * topk + rank] = e;
-    }
-    if (normalize && !(total > 0.0 && total < 1.0e300)) raise_status(status, 1);
-    if (lane < topk) {
-        double value = (double)picked_score;
-        if (normalize) value /= total;
-        value *= scaling;
-        const float w = (float)value;
-        if (!finite_f32(w)) raise_status(status, 1);
-        weights[row * topk + lane] = w;
-    }
 }
 
 __global__ __launch_bounds__(256) void route_rows_kernel(
@@ -368,6 +258,9 @@ __global__ __launch_bounds__(1024) void worklist_kernel(
 // wavefront a row, sixteen at a time) and then builds the worklist from what it wrote; every
 // other workgroup quantizes sixteen Q8_K blocks of the input rows, which depend on neither.
 constexpr unsigned kPrepareMaxRows = 128u;
+// Rows that are routed already leave the worklist: as long as its bitmap is small enough for the
+// quantizing workgroups, which get the same LDS, to share a compute unit.
+constexpr unsigned kPrepareMaxRoutedRows = 512u;
 
 __global__ __launch_bounds__(1024) void decode_prepare_kernel(
     const float *__restrict__ logits, const float *__restrict__ bias, unsigned rows, unsigned experts,
@@ -390,7 +283,9 @@ __global__ __launch_bounds__(1024) void decode_prepare_kernel(
         return;
     }
     // a wave's rows one after another, the next row's values on their way while this one is routed
+    // (neither logits nor scores: the router's own launch has routed the rows)
     const float *values_in = scores ? scores : logits;
+    if (values_in) {
     RouteInputs current;
     if (wave < rows) route_inputs_load(current, values_in, bias, wave, lane, experts);
     for (unsigned row = wave; row < rows; row += 16u) {
@@ -401,6 +296,7 @@ __global__ __launch_bounds__(1024) void decode_prepare_kernel(
         current = next;
     }
     __syncthreads();   // the selections written above are read back by other waves below
+    }
     worklist_block(selected, rows * topk, topk, experts, order, expert_ids, bucket_offsets,
                    bucket_populations, sweep_offsets, counts, status, shared_words, true);
 }
@@ -981,10 +877,13 @@ static int launch_moe_prepare(const float *logits, const float *scores, const fl
                               uint64_t *counts, const float *values, uint64_t width, uint64_t input_stride,
                               uint8_t *encoded, int *status, yvex_hip_stream stream)
 {
-    if ((!logits && !scores) || !selected || !weights || !order || !expert_ids || !bucket_offsets ||
+    const bool routed = !logits && !scores;
+    if (!selected || (!weights && !routed) || !order || !expert_ids || !bucket_offsets ||
         !bucket_populations || !sweep_offsets || !counts || !status || (scoring != 0 && scoring != 1))
         return ST_INVALID_ARG;
-    if (!yvex_hip_moe_prepare_supported(rows, experts, topk)) return ST_UNSUPPORTED;
+    if (routed ? !rows || rows > kPrepareMaxRoutedRows || !experts || experts > 256u || !topk || topk > 16u || topk > experts
+               : !yvex_hip_moe_prepare_supported(rows, experts, topk))
+        return ST_UNSUPPORTED;
     uint64_t tasks = 0u;
     if (values) {
         if (!encoded || !width || width % 256u || input_stride < width || width / 256u > 0xffffu)
@@ -1028,6 +927,18 @@ extern "C" int yvex_hip_moe_prepare_scored(const float *scores, const float *bia
 {
     if (!scores) return ST_INVALID_ARG;
     return launch_moe_prepare(nullptr, scores, bias, rows, experts, topk, 0, normalize, scaling, selected, weights,
+                              order, expert_ids, bucket_offsets, bucket_populations, sweep_offsets, counts,
+                              values, width, input_stride, encoded, status, stream);
+}
+
+extern "C" int yvex_hip_moe_prepare_routed(const uint64_t *selected, uint64_t rows, uint64_t experts, uint64_t topk,
+                                           uint64_t *order, uint64_t *expert_ids, uint64_t *bucket_offsets,
+                                           uint64_t *bucket_populations, uint64_t *sweep_offsets,
+                                           uint64_t *counts, const float *values, uint64_t width,
+                                           uint64_t input_stride, uint8_t *encoded, int *status,
+                                           yvex_hip_stream stream)
+{
+    return launch_moe_prepare(nullptr, nullptr, nullptr, rows, experts, topk, 0, 0, 1.0, (uint64_t *)selected, nullptr,
                               order, expert_ids, bucket_offsets, bucket_populations, sweep_offsets, counts,
                               values, width, input_stride, encoded, status, stream);
 }

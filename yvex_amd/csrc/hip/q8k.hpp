@@ -6,16 +6,14 @@
 
 namespace yvex {
 
-// x: this lane's four values of the block; out: the block's 292 bytes.
-__device__ __forceinline__ void q8k_quantize_block(const float *__restrict__ x, unsigned char *__restrict__ out,
-                                                   unsigned lane, int *status)
+// v: this lane's four values of the block; out: the block's 292 bytes.
+__device__ __forceinline__ void q8k_quantize_values(const float (&v)[4], unsigned char *__restrict__ out,
+                                                    unsigned lane, int *status)
 {
-    float v[4];
     unsigned long long key = 0ull;
     bool bad = false;
 #pragma unroll
     for (unsigned i = 0; i < 4u; ++i) {
-        v[i] = x[i];
         const unsigned bits = __float_as_uint(v[i]);
         bad |= !finite_f32(v[i]);
         // order by |x|, then by lowest index; the low bit carries the sign of the winner
@@ -46,6 +44,14 @@ __device__ __forceinline__ void q8k_quantize_block(const float *__restrict__ x, 
     *reinterpret_cast<unsigned *>(out + 4u + lane * 4u) = packed;
     sum = group_sum_i32<4>(sum);   // four lanes hold sixteen consecutive values
     if ((lane & 3u) == 0u) *reinterpret_cast<short *>(out + 260u + (lane >> 2) * 2u) = (short)sum;
+}
+
+// x: this lane's four values of the block in memory.
+__device__ __forceinline__ void q8k_quantize_block(const float *__restrict__ x, unsigned char *__restrict__ out,
+                                                   unsigned lane, int *status)
+{
+    const float v[4] = {x[0], x[1], x[2], x[3]};
+    q8k_quantize_values(v, out, lane, status);
 }
 
 }  // namespace yvex

@@ -141,41 +141,37 @@ __device__ __forceinline__ unsigned lds_load_u32(unsigned address)
 #endif
 }
 
-// The codebook digits of a thread's table entries, requested together at kernel start: one round
-// trip to memory, which runs beside the others that open the launch.
-constexpr unsigned kTableTurns = 256u * 16u / kSweepThreads;
-static_assert(256u * 16u % kSweepThreads == 0u && 128u * 32u % kSweepThreads == 0u,
-              "every thread fills the same number of table entries");
+// The lookup tables: the first 256 threads form one codebook entry each and store its sixteen
+// replicas, the others one sign entry in twos, sixteen replicas each. Step t stores the replica
+// after the lane's own by t, so that a store's lanes spread over all banks. (One replica a thread and
+// turn, all turns unrolled, was several kilobytes of code that every launch fetched to run it
+// once, and eight codebook loads a thread: 1.5 us, with it 3 of the 7 us a launch opened with.)
+static_assert(kSweepThreads == 512u, "a thread a codebook entry, two a sign entry");
 
-__device__ __forceinline__ void sweep_tables_request(unsigned (&digits)[kTableTurns])
-{
-#pragma unroll
-    for (unsigned t = 0; t < kTableTurns; ++t) digits[t] = k_iq2_digits[(threadIdx.x + t * kSweepThreads) >> 4];
-}
+__device__ __forceinline__ unsigned sweep_table_digits() { return k_iq2_digits[threadIdx.x & 255u]; }
 
-__device__ __forceinline__ void sweep_tables_fill(const unsigned (&digits)[kTableTurns])
+__device__ __forceinline__ void sweep_tables_fill(unsigned digits)
 {
-#pragma unroll
-    for (unsigned t = 0; t < kTableTurns; ++t) {
-        const unsigned i = threadIdx.x + t * kSweepThreads;
-        const uint2 m = iq2_magnitude_of_digits(digits[t]);
+    if (threadIdx.x < 256u) {
+        const uint2 m = iq2_magnitude_of_digits(digits);
         // byte-wise negation: every level is >= 8, so (x ^ 0xff) + 1 never carries
-        lds_store_uint4(kMagBase + i * 16u,
-                        make_uint4(m.x, m.y, (m.x ^ 0xffffffffu) + 0x01010101u,
-                                   (m.y ^ 0xffffffffu) + 0x01010101u));
-    }
-#pragma unroll
-    for (unsigned i = threadIdx.x; i < 128u * 32u; i += kSweepThreads) {
-        const unsigned s7 = i >> 5;
+        const uint4 entry = make_uint4(m.x, m.y, (m.x ^ 0xffffffffu) + 0x01010101u, (m.y ^ 0xffffffffu) + 0x01010101u);
+#pragma unroll 4
+        for (unsigned t = 0; t < 16u; ++t)
+            lds_store_uint4(kMagBase + threadIdx.x * 256u + ((threadIdx.x + t) & 15u) * 16u, entry);
+    } else {
+        const unsigned s7 = (threadIdx.x - 256u) >> 1, upper = threadIdx.x & 1u;
         const unsigned s = s7 | ((__popc(s7) & 1u) << 7);
         // selector byte k = k (take +level, source 1) or k + 4 (take -level, source 0)
         unsigned lo = 0x03020100u, hi = 0x03020100u;
 #pragma unroll
         for (unsigned l = 0; l < 4u; ++l) {
-            if ((s >> l) & 1u) lo += 4u << (8u * l);
-            if ((s >> (l + 4u)) & 1u) hi += 4u << (8u * l);
+            lo += ((s >> l) & 1u) << (8u * l + 2u);
+            hi += ((s >> (l + 4u)) & 1u) << (8u * l + 2u);
         }
-        lds_store_uint2(kSelBase + i * 8u, make_uint2(lo, hi));
+#pragma unroll 4
+        for (unsigned t = 0; t < 16u; ++t)
+            lds_store_uint2(kSelBase + s7 * 256u + upper * 128u + ((s7 + t) & 15u) * 8u, make_uint2(lo, hi));
     }
 }
 
@@ -846,8 +842,8 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
     static_assert(kPairCacheMax <= 2u * kSweepThreads, "two cached pairs a thread");
     // ---- everything that opens the launch is requested before any of it is used: the tables'
     // digits, the routed buckets (four a lane, in every wave) and the pairs' sources ----
-    unsigned digits[kTableTurns];
-    if constexpr (QT == QT_IQ2_XXS) sweep_tables_request(digits);     // (the other formats need no tables)
+    unsigned digits = 0u;
+    if constexpr (QT == QT_IQ2_XXS) digits = sweep_table_digits();    // (the other formats need no tables)
     const unsigned long long bucket_count = routed_fixed ? 1ull : routed.counts[0];
     unsigned long long population64[4], expert64[4], first64[4];
 #pragma unroll
@@ -947,10 +943,13 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
     struct Place {
         unsigned slot, sweep, row;
     };
+    // (integer arithmetic on the scalar unit, one division for both ends)
     const unsigned long long all_cost = (unsigned long long)row_cost * a.out_rows;
+    const unsigned long long share = uniform64((unsigned long long)((double)all_cost / (double)gridDim.x));
+    const unsigned long long left_over = all_cost - share * gridDim.x;
     auto place_of = [&](unsigned who) -> Place {        // where the piece of workgroup `who` begins
         if (who >= gridDim.x) return Place{buckets + 1u, 0u, 0u};
-        unsigned long long at = uniform64((unsigned long long)((double)all_cost * (double)who / (double)gridDim.x));
+        unsigned long long at = share * who + (who < left_over ? who : left_over);
         unsigned slot = 0u, n = extra_pairs;
         if (at >= (unsigned long long)extra_cost * a.out_rows) {
             at -= (unsigned long long)extra_cost * a.out_rows;
@@ -971,19 +970,27 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
             }
         }
         const unsigned full = n / 4u;
-        const unsigned long long sweep_rows = (unsigned long long)sweep_cost<QT>(4u) * a.out_rows;
-        unsigned sweep = uniform((unsigned)((double)at / (double)sweep_rows));
-        if ((unsigned long long)sweep * sweep_rows > at) --sweep;
-        if (sweep > full) sweep = full;
-        at -= (unsigned long long)sweep * sweep_rows;
-        const unsigned weight = sweep < full ? sweep_cost<QT>(4u) : sweep_cost<QT>(n % 4u);
-        unsigned row = uniform((unsigned)at / weight);
+        const unsigned sweep_rows = sweep_cost<QT>(4u) * a.out_rows;
+        unsigned sweep = 0u;
+        if (full) {
+            sweep = uniform((unsigned)((double)at / (double)sweep_rows));
+            if (sweep > full) sweep = full;
+            at -= (unsigned long long)sweep * sweep_rows;
+        }
+        const unsigned rest = (unsigned)at;
+        unsigned row = sweep < full ? rest / sweep_cost<QT>(4u)
+            : n % 4u == 1u ? rest / sweep_cost<QT>(1u) : n % 4u == 2u ? rest / sweep_cost<QT>(2u)
+                                                                     : rest / sweep_cost<QT>(3u);
         if (row > a.out_rows) row = a.out_rows;
         // (the same in every lane: kept in scalar registers, of which the sweeps leave some)
         return Place{uniform(slot), uniform(sweep), uniform(row & ~(granule - 1u))};
     };
-    Place now = place_of(blockIdx.x);
-    const Place end = place_of(blockIdx.x + 1u);
+    Place now{}, end{};
+#pragma unroll 1
+    for (unsigned ends = 0; ends < 2u; ++ends) {      // (the code of one, run twice)
+        now = end;
+        end = place_of(blockIdx.x + ends);
+    }
 
     // The first weight rows of the piece start on their way to the caches while the tables are
     // built (64 bytes apart, so the lanes cover 4 KB of each stream).

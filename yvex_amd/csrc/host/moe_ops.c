@@ -502,7 +502,7 @@ static int moe_execute_rows(yvex_rocm_backend *backend, const yvex_moe_layer_job
     const float *bias_rows;
     void *combined_target;
     unsigned long long table_address = 0ull;
-    int matrix_allowed = 1, envelope, hash_router, unsupported_width, routed_q8 = 0, shared_q8 = 0, routed_image = 0, shared_image = 0, has_shared, merged, row_batch, shared_row_batch, shared_dense, device_status = 0, rc, defer, scored = 0;
+    int matrix_allowed = 1, envelope, hash_router, unsupported_width, routed_q8 = 0, shared_q8 = 0, routed_image = 0, shared_image = 0, has_shared, merged, row_batch, shared_row_batch, shared_dense, device_status = 0, rc, defer, host_rows, combined_egress, swiglu_quantized, routed_rows = 0;
     void *status;
     yvex_hip_stream stream;
     enum { GRAPH_EAGER = 0, GRAPH_CAPTURE, GRAPH_REPLAY } graph_mode = GRAPH_EAGER;
@@ -700,7 +700,17 @@ static int moe_execute_rows(yvex_rocm_backend *backend, const yvex_moe_layer_job
      * projection. */
     shared_dense = has_shared && shared_q8 && !merged && !shared_row_batch && !shared_image &&
                    shared.gate_qtype == 8u && shared.up_qtype == 8u && shared.down_qtype == 8u &&
-                   layer->shared_intermediate_width <= topk * hidden;
+                   layer->shared_intermediate_width <= topk * hidden && shared.gate_row_bytes == shared.up_row_bytes;
+    /* ... and its SwiGLU products are formed by the launch that quantizes both kinds of intermediate
+     * rows, where they are of one width and their ranges of whole 16-byte pieces */
+    swiglu_quantized = shared_dense && routed_q8 && layer->shared_intermediate_width == layer->expert_intermediate_width;
+    /* The routed sums and, with residual streams around the layer, the combined rows go to memory only
+     * for a caller that asked for host copies of them; otherwise the combine goes straight on into the
+     * egress. */
+    defer = job->device_completion && job->device_completion->defer;
+    host_rows = !defer && (output->routed_rows || output->combined_rows);
+    combined_egress = envelope && streams == 4ull && hidden % 4ull == 0ull && !host_rows &&
+                      !(((uintptr_t)rows->device_rows->data | (uintptr_t)rows->device_outputs->data) & 15u);
     if (yvex_rocm_seam("YVEX_TEST_ROCM_LAUNCH_FAILURE"))
         return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, "rocm.moe.rows.launch",
                                 "kernel launch failed (test seam)");
@@ -737,6 +747,7 @@ static int moe_execute_rows(yvex_rocm_backend *backend, const yvex_moe_layer_job
         key.overflow = 0;
         key_word(&key, row_count);
         key_word(&key, (unsigned long long)row_batch);
+        key_word(&key, (unsigned long long)host_rows);
         key_word(&key, (unsigned long long)(uintptr_t)status);
         key_word(&key, (unsigned long long)(uintptr_t)stream);
         key_word(&key, base);
@@ -769,8 +780,6 @@ sequence:
             if (rc == YVEX_OK) launches++;                              \
         }                                                               \
     } while (0)
-    if (has_shared && !merged)
-        LAUNCH(yvex_hip_fill_u32(AT(shared_outputs), 0u, row_count * hidden, stream), "rocm.moe.rows.zero");
     activations = rows->device_rows->data;
     combined_target = rows->device_outputs->data;
     if (envelope) {
@@ -847,6 +856,16 @@ sequence:
         activations = AT(normalized);
         combined_target = AT(combined);
     }
+    /* a correction bias stored as F32 values is read where it lies; any other encoding is
+     * decoded into the workspace first */
+    bias_rows = NULL;
+    if (!hash_router && layer->requires_correction_bias)
+        bias_rows = views[YVEX_MOE_WEIGHT_ROUTER_BIAS].qtype == YVEX_GGUF_QTYPE_F32 && !(bias_address & 3ull)
+                        ? (const float *)(uintptr_t)bias_address : (const float *)AT(bias);
+    if (bias_rows && bias_rows == (const float *)AT(bias))
+        LAUNCH(yvex_hip_gather((const uint8_t *)(uintptr_t)bias_address, views[YVEX_MOE_WEIGHT_ROUTER_BIAS].qtype,
+                               1ull, experts, views[YVEX_MOE_WEIGHT_ROUTER_BIAS].row_bytes, NULL, 1ull,
+                               (float *)AT(bias), (int *)status, stream), "rocm.moe.rows.bias");
     /* router: logits = router . row (F32 activations, as src/backend/cuda/moe.c:1259-1284). F32
      * router weights over a decode-width batch are split over the whole device; their partial
      * sums use the pair-output range, which nothing else touches before the down projection. */
@@ -858,18 +877,18 @@ sequence:
         unsigned int router_launches = yvex_hip_matvec_f32_rows_launches(
             (const float *)(uintptr_t)router_address, experts, hidden, (const float *)activations, row_count,
             hidden, lend ? AT(pair_outputs) : NULL, lend ? need : 0ull);
-        /* the split projection's second launch publishes the learned router's scores as well
-         * (into the combine's output range, which nothing reads or writes before the combine):
-         * the preparation launch, whose one routing workgroup everything behind it waits for,
-         * then starts from them */
-        scored = router_launches == 2u && !hash_router && hidden >= experts &&
-                 yvex_hip_moe_prepare_supported(row_count, experts, topk);
-        if (scored)
-            LAUNCH(yvex_hip_matvec_f32_rows_scored((const float *)(uintptr_t)router_address, experts, hidden,
+        /* the split projection's second launch routes the rows as well, a workgroup a row: the
+         * preparation launch behind it, whose one routing workgroup everything else would wait
+         * for, is left with the worklist */
+        routed_rows = router_launches == 2u && !hash_router && experts <= 256ull;
+        if (routed_rows)
+            LAUNCH(yvex_hip_matvec_f32_rows_routed((const float *)(uintptr_t)router_address, experts, hidden,
                                                    (const float *)activations, row_count, hidden,
-                                                   (float *)AT(logits), experts, (float *)AT(routed),
-                                                   (int)layer->scoring, AT(pair_outputs), need,
-                                                   (int *)status, stream), "rocm.moe.rows.router");
+                                                   (float *)AT(logits), bias_rows, topk, (int)layer->scoring,
+                                                   layer->normalize_topk_probabilities,
+                                                   layer->routed_scaling_factor, (uint64_t *)AT(selected),
+                                                   (float *)AT(weights), AT(pair_outputs), need, (int *)status,
+                                                   stream), "rocm.moe.rows.router");
         else
         LAUNCH(yvex_hip_matvec_f32_rows((const float *)(uintptr_t)router_address, experts, hidden,
                                         (const float *)activations, row_count, hidden, NULL,
@@ -892,32 +911,18 @@ sequence:
                                             (float *)AT(weights), (int *)status, stream),
                "rocm.moe.rows.route");
     }
-    /* a correction bias stored as F32 values is read where it lies; any other encoding is
-     * decoded into the workspace first */
-    bias_rows = NULL;
-    if (!hash_router && layer->requires_correction_bias)
-        bias_rows = views[YVEX_MOE_WEIGHT_ROUTER_BIAS].qtype == YVEX_GGUF_QTYPE_F32 && !(bias_address & 3ull)
-                        ? (const float *)(uintptr_t)bias_address : (const float *)AT(bias);
-    if (bias_rows && bias_rows == (const float *)AT(bias))
-        LAUNCH(yvex_hip_gather((const uint8_t *)(uintptr_t)bias_address, views[YVEX_MOE_WEIGHT_ROUTER_BIAS].qtype,
-                               1ull, experts, views[YVEX_MOE_WEIGHT_ROUTER_BIAS].row_bytes, NULL, 1ull,
-                               (float *)AT(bias), (int *)status, stream), "rocm.moe.rows.bias");
     /* a decode-width batch with the learned router: routing, worklist and input quantization
      * share one launch */
     const int need_q8 = routed_q8 || (has_shared && shared_q8);
-    if (scored) {
-        LAUNCH(yvex_hip_moe_prepare_scored((const float *)AT(routed),
-                                           bias_rows,
-                                           row_count, experts, topk, layer->normalize_topk_probabilities,
-                                           layer->routed_scaling_factor, (uint64_t *)AT(selected),
-                                           (float *)AT(weights), (uint64_t *)AT(order),
-                                           (uint64_t *)AT(expert_ids), (uint64_t *)AT(bucket_offsets),
-                                           (uint64_t *)AT(bucket_populations),
+    if (routed_rows && row_count <= 512ull) {
+        LAUNCH(yvex_hip_moe_prepare_routed((const uint64_t *)AT(selected), row_count, experts, topk,
+                                           (uint64_t *)AT(order), (uint64_t *)AT(expert_ids),
+                                           (uint64_t *)AT(bucket_offsets), (uint64_t *)AT(bucket_populations),
                                            (uint64_t *)AT(sweep_offsets), (uint64_t *)AT(counts),
                                            need_q8 ? (const float *)activations : NULL, hidden, hidden,
                                            need_q8 ? (uint8_t *)AT(input_q8) : NULL, (int *)status, stream),
                "rocm.moe.rows.prepare");
-    } else if (!hash_router && yvex_hip_moe_prepare_supported(row_count, experts, topk)) {
+    } else if (!routed_rows && !hash_router && yvex_hip_moe_prepare_supported(row_count, experts, topk)) {
         LAUNCH(yvex_hip_moe_prepare((const float *)AT(logits),
                                     bias_rows,
                                     row_count, experts, topk, (int)layer->scoring,
@@ -929,7 +934,7 @@ sequence:
                                     hidden, hidden, need_q8 ? (uint8_t *)AT(input_q8) : NULL,
                                     (int *)status, stream), "rocm.moe.rows.prepare");
     } else {
-        if (!hash_router)
+        if (!hash_router && !routed_rows)
             LAUNCH(yvex_hip_moe_route_rows((const float *)AT(logits),
                                            bias_rows,
                                            row_count, experts, topk, (int)layer->scoring,
@@ -968,24 +973,27 @@ sequence:
                                     1ull, 1ull, layer->activation_limit, (float *)AT(shared_intermediate),
                                     (int *)status, stream), "rocm.moe.rows.shared-up-matrix");
     else if (shared_dense) {
-        LAUNCH(yvex_hip_matvec(shared.gate, shared.gate_qtype, layer->shared_intermediate_width, hidden,
-                               shared.gate_row_bytes, AT(input_q8), 1, row_count, hidden, NULL,
-                               (float *)AT(shared_intermediate), layer->shared_intermediate_width, 0,
-                               (int *)status, stream), "rocm.moe.rows.shared-gate-dense");
-        LAUNCH(yvex_hip_matvec(shared.up, shared.up_qtype, layer->shared_intermediate_width, hidden,
-                               shared.up_row_bytes, AT(input_q8), 1, row_count, hidden, NULL,
-                               (float *)AT(pair_outputs), layer->shared_intermediate_width, 0,
-                               (int *)status, stream), "rocm.moe.rows.shared-up-dense");
-        LAUNCH(yvex_hip_moe_swiglu_rows((const float *)AT(shared_intermediate), (const float *)AT(pair_outputs),
-                                        row_count * layer->shared_intermediate_width, layer->activation_limit,
-                                        (float *)AT(shared_intermediate), (int *)status, stream),
-               "rocm.moe.rows.shared-swiglu");
+        LAUNCH(yvex_hip_matvec_q8_0_pair(shared.gate, shared.up, layer->shared_intermediate_width, hidden,
+                                         shared.gate_row_bytes, AT(input_q8), row_count,
+                                         (float *)AT(shared_intermediate), (float *)AT(pair_outputs), (int *)status,
+                                         stream), "rocm.moe.rows.shared-up-dense");
+        if (!swiglu_quantized)
+            LAUNCH(yvex_hip_moe_swiglu_rows((const float *)AT(shared_intermediate), (const float *)AT(pair_outputs),
+                                            row_count * layer->shared_intermediate_width, layer->activation_limit,
+                                            (float *)AT(shared_intermediate), (int *)status, stream),
+                   "rocm.moe.rows.shared-swiglu");
     } else if (has_shared && !merged)
         LAUNCH(yvex_hip_moe_up(&shared, shared_q8 ? AT(input_q8) : (void *)(uintptr_t)activations,
                                shared_q8, NULL, NULL, NULL, NULL, NULL, NULL, NULL, row_count, 1ull, 1ull,
                                layer->activation_limit, (float *)AT(shared_intermediate), NULL, 0ull, NULL,
                                (int *)status, stream), "rocm.moe.rows.shared-up");
-    if (routed_q8 && has_shared && shared_q8 && ranges.joined_intermediates)
+    if (swiglu_quantized)
+        LAUNCH(yvex_hip_q8k_quantize_swiglu((const float *)AT(intermediate), pairs, layer->expert_intermediate_width,
+                                            (uint8_t *)AT(intermediate_q8), (const float *)AT(shared_intermediate),
+                                            (const float *)AT(pair_outputs), row_count, layer->activation_limit,
+                                            (uint8_t *)AT(shared_intermediate_q8), (int *)status, stream),
+               "rocm.moe.rows.q8-mid");
+    else if (routed_q8 && has_shared && shared_q8 && ranges.joined_intermediates)
         LAUNCH(yvex_hip_q8k_quantize((const float *)AT(intermediate), pairs + row_count,
                                      layer->expert_intermediate_width, layer->expert_intermediate_width,
                                      (uint8_t *)AT(intermediate_q8), (int *)status, stream),
@@ -994,7 +1002,7 @@ sequence:
         LAUNCH(yvex_hip_q8k_quantize((const float *)AT(intermediate), pairs, layer->expert_intermediate_width,
                                      layer->expert_intermediate_width, (uint8_t *)AT(intermediate_q8),
                                      (int *)status, stream), "rocm.moe.rows.q8-mid");
-    if (has_shared && shared_q8 && !(routed_q8 && ranges.joined_intermediates))
+    if (has_shared && shared_q8 && !swiglu_quantized && !(routed_q8 && ranges.joined_intermediates))
         LAUNCH(yvex_hip_q8k_quantize((const float *)AT(shared_intermediate), row_count,
                                      layer->shared_intermediate_width, layer->shared_intermediate_width,
                                      (uint8_t *)AT(shared_intermediate_q8), (int *)status, stream),
@@ -1031,15 +1039,24 @@ sequence:
                "rocm.moe.rows.shared-down");
     if (!has_shared)
         LAUNCH(yvex_hip_fill_u32(AT(shared_outputs), 0u, row_count * hidden, stream), "rocm.moe.rows.zero");
-    LAUNCH(yvex_hip_moe_reduce_combine((const float *)AT(pair_outputs), row_count, topk, hidden,
-                                       (const float *)AT(shared_outputs), (float *)AT(routed),
-                                       (float *)combined_target, (int *)status, stream),
-           "rocm.moe.rows.combine");
-    if (envelope)
-        LAUNCH(yvex_hip_mhc_egress((const float *)AT(combined), (const float *)rows->device_rows->data,
-                                   (const float *)AT(post), (const float *)AT(combination), row_count,
-                                   streams, hidden, (float *)rows->device_outputs->data, (int *)status,
-                                   stream), "rocm.moe.rows.mhc-egress");
+    if (combined_egress)
+        LAUNCH(yvex_hip_moe_combine_egress((const float *)AT(pair_outputs), row_count, topk, streams, hidden,
+                                           (const float *)AT(shared_outputs), (const float *)rows->device_rows->data,
+                                           (const float *)AT(post), (const float *)AT(combination),
+                                           (float *)rows->device_outputs->data, (int *)status, stream),
+               "rocm.moe.rows.combine-egress");
+    else {
+        LAUNCH(yvex_hip_moe_reduce_combine((const float *)AT(pair_outputs), row_count, topk, hidden,
+                                           (const float *)AT(shared_outputs),
+                                           host_rows ? (float *)AT(routed) : NULL,
+                                           (float *)combined_target, (int *)status, stream),
+               "rocm.moe.rows.combine");
+        if (envelope)
+            LAUNCH(yvex_hip_mhc_egress((const float *)AT(combined), (const float *)rows->device_rows->data,
+                                       (const float *)AT(post), (const float *)AT(combination), row_count,
+                                       streams, hidden, (float *)rows->device_outputs->data, (int *)status,
+                                       stream), "rocm.moe.rows.mhc-egress");
+    }
     if (graph_mode == GRAPH_CAPTURE) {
         /* a recording that fails, or holds anything but kernels, is dropped for good and the
          * batch runs eagerly: the stream has executed nothing yet */
@@ -1072,7 +1089,6 @@ sequence:
         return rc;
     }
 
-    defer = job->device_completion && job->device_completion->defer;
     result->graph_launches = graph_mode != GRAPH_EAGER;
     result->graph_captures = graph_mode == GRAPH_CAPTURE;
     result->graph_replays = graph_mode == GRAPH_REPLAY;
