@@ -34,3 +34,153 @@ def test_publish_brings_results_and_status_to_the_host(gpu, nbytes):
     finally:
         torch.cuda.synchronize()
         lib.yvex_hip_host_free(host)
+
+
+def ptr(t):
+    return C.c_void_p(0 if t is None else t.data_ptr())
+
+
+def u64(v):
+    return C.c_uint64(v)
+
+
+def call(name, *args):
+    from yvex_amd import kernels as K
+    K._call(name, *args, C.c_void_p(torch.cuda.current_stream().cuda_stream))
+
+
+def dev(a, device):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(device)
+
+
+def same_bits(a, b):
+    return torch.equal(a.contiguous().view(torch.int32), b.contiguous().view(torch.int32))
+
+
+# a full round of 128 x 128 tiles with ragged edges on both sides, one and three superblocks a row
+@pytest.mark.parametrize("rows,width,inputs", [(2047, 256, 2040), (1921, 768, 2048)])
+def test_q8_0_wide_tiles_are_the_oracles_bits(gpu, oracle, rows, width, inputs):
+    from yvex_amd import kernels as K
+    g = oracle.Generator(42, f"wide.{rows}.{width}.{inputs}")
+    w, x = g.weights(oracle.Q8_0, rows, width), g.normal(inputs * width).reshape(inputs, width)
+    status = K.new_status(gpu)
+    act = K.q8k_quantize(dev(x, gpu), status)
+    got = K.matvec(dev(w, gpu), oracle.Q8_0, rows, width, act, input_q8=True, input_rows=inputs, status=status).cpu().numpy()
+    assert int(status.item()) == 0
+    picked = np.array([0, 1, 31, 32, 63, 64, 127, 128, inputs // 2, inputs - 2, inputs - 1])
+    encoded = oracle.q8k_quantize(x[picked])
+    want = oracle.q8_matvec(oracle.Q8_0, w, rows, width, encoded, picked.size)
+    assert np.array_equal(got[picked].view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,width,inputs", [(34, 512, 1), (128, 256, 5), (2048, 512, 17), (70, 768, 40)])
+def test_q8_0_pair_is_two_projections(gpu, oracle, rows, width, inputs):
+    from yvex_amd import kernels as K
+    g = oracle.Generator(42, f"pair.{rows}.{width}.{inputs}")
+    first, second = (dev(g.weights(oracle.Q8_0, rows, width), gpu) for _ in range(2))
+    status = K.new_status(gpu)
+    act = K.q8k_quantize(dev(g.normal(inputs * width).reshape(inputs, width), gpu), status)
+    out = [torch.full((inputs, rows), 7.0, device=gpu) for _ in range(2)]
+    call("yvex_hip_matvec_q8_0_pair", ptr(first), ptr(second), u64(rows), u64(width), u64(width // 32 * 34), ptr(act),
+         u64(inputs), ptr(out[0]), ptr(out[1]), ptr(status))
+    for w, got in zip((first, second), out):
+        want = K.matvec(w, oracle.Q8_0, rows, width, act, input_q8=True, input_rows=inputs, status=status)
+        assert same_bits(got, want)
+    assert int(status.item()) == 0
+
+
+@pytest.mark.parametrize("rows,experts,topk,width,bias", [(8, 8, 2, 1024, True), (33, 200, 16, 1024, False),
+                                                          (255, 256, 8, 7168, True), (300, 24, 6, 2048, False)])
+def test_router_joins_and_routes_in_one_launch(gpu, oracle, rows, experts, topk, width, bias):
+    from yvex_amd import kernels as K
+    g = oracle.Generator(42, f"routed.{rows}.{experts}")
+    w = dev(g.normal(experts * width, width ** -0.5).reshape(experts, width), gpu)
+    x = dev(g.normal(rows * width).reshape(rows, width), gpu)
+    b = dev(g.normal(experts, 0.1).astype(np.float32), gpu) if bias else None
+    status = K.new_status(gpu)
+    logits = K.matvec_f32_rows(w, x, status)
+    want = K.moe_route_rows(logits, b, topk, K.SIGMOID, True, 1.5, status)
+    lib = K.load_library()
+    lib.yvex_hip_matvec_f32_scratch_bytes.restype = C.c_uint64
+    need = lib.yvex_hip_matvec_f32_scratch_bytes(u64(experts), u64(width), u64(rows))
+    assert need > 0
+    scratch = torch.empty(need, dtype=torch.uint8, device=gpu)
+    got_logits = torch.empty_like(logits)
+    selected, weights = torch.empty_like(want[0]), torch.empty_like(want[1])
+    call("yvex_hip_matvec_f32_rows_routed", ptr(w), u64(experts), u64(width), ptr(x), u64(rows), u64(width), ptr(got_logits),
+         ptr(b), u64(topk), C.c_int(K.SIGMOID), C.c_int(1), C.c_double(1.5), ptr(selected), ptr(weights), ptr(scratch),
+         u64(need), ptr(status))
+    assert same_bits(got_logits, logits) and torch.equal(selected, want[0]) and same_bits(weights, want[1])
+    # ... and the preparation behind it: the worklist and the quantization alone
+    wl, mine = K.worklist_build(selected, experts, status), K.Worklist(rows * topk, experts, gpu)
+    encoded = torch.empty(rows * (width // 256) * 292, dtype=torch.uint8, device=gpu)
+    call("yvex_hip_moe_prepare_routed", ptr(selected), u64(rows), u64(experts), u64(topk), *K._wl_ptrs(mine), ptr(x),
+         u64(width), u64(width), ptr(encoded), ptr(status))
+    for name in ("order", "expert_ids", "bucket_offsets", "bucket_populations", "sweep_offsets", "counts"):
+        assert torch.equal(getattr(mine, name), getattr(wl, name)), name
+    assert torch.equal(encoded, K.q8k_quantize(x, status)) and int(status.item()) == 0
+
+
+@pytest.mark.parametrize("rows,shared,width", [(1, 1, 256), (7, 5, 768), (40, 3, 2048)])
+def test_quantization_forms_the_shared_experts_products(gpu, oracle, rows, shared, width):
+    from yvex_amd import kernels as K
+    g = oracle.Generator(42, f"qswiglu.{rows}.{width}")
+    values = dev(g.normal(rows * width).reshape(rows, width), gpu)
+    gate, up = (dev(g.normal(shared * width, 4.0).reshape(shared, width), gpu) for _ in range(2))
+    status = K.new_status(gpu)
+    products = torch.empty_like(gate)
+    call("yvex_hip_moe_swiglu_rows", ptr(gate), ptr(up), u64(shared * width), C.c_double(7.0), ptr(products), ptr(status))
+    bytes_of = [torch.zeros(n * (width // 256) * 292, dtype=torch.uint8, device=gpu) for n in (rows, shared)]
+    call("yvex_hip_q8k_quantize_swiglu", ptr(values), u64(rows), u64(width), ptr(bytes_of[0]), ptr(gate), ptr(up),
+         u64(shared), C.c_double(7.0), ptr(bytes_of[1]), ptr(status))
+    assert torch.equal(bytes_of[0], K.q8k_quantize(values, status))
+    assert torch.equal(bytes_of[1], K.q8k_quantize(products, status)) and int(status.item()) == 0
+
+
+@pytest.mark.parametrize("rows,topk,width", [(1, 1, 4), (3, 6, 1028), (9, 8, 7168)])
+def test_combine_goes_straight_into_the_egress(gpu, oracle, rows, topk, width):
+    from yvex_amd import kernels as K
+    streams = 4
+    g = oracle.Generator(42, f"egress.{rows}.{width}")
+    pairs = dev(g.normal(rows * topk * width).reshape(rows * topk, width), gpu)
+    shared = dev(g.normal(rows * width).reshape(rows, width), gpu)
+    x = dev(g.normal(rows * streams * width).reshape(rows, streams * width), gpu)
+    post = dev(np.abs(g.normal(rows * streams)).reshape(rows, streams), gpu)
+    mixing = dev(np.abs(g.normal(rows * 16)).reshape(rows, streams, streams), gpu)
+    status = K.new_status(gpu)
+    combined, routed = torch.empty_like(shared), torch.empty_like(shared)
+    K.moe_reduce_combine(pairs, rows, topk, width, shared, routed, combined, status)
+    want = K.mhc_egress(combined, x, post, mixing, streams=streams, width=width, status=status)
+    got = torch.zeros_like(want)
+    call("yvex_hip_moe_combine_egress", ptr(pairs), u64(rows), u64(topk), u64(streams), u64(width), ptr(shared), ptr(x),
+         ptr(post), ptr(mixing), ptr(got), ptr(status))
+    assert same_bits(got, want) and int(status.item()) == 0
+
+
+@pytest.mark.parametrize("qtype,hidden,intermediate,experts,rows,topk", [
+    ("IQ2_XXS", 2048, 2048, 3, 1, 3),          # a handful of iterations a workgroup, whole pieces of some empty
+    ("IQ2_XXS", 7168, 2304, 9, 9, 5),          # one weight row an iteration, buckets of one to nine pairs
+    ("Q4_K", 4096, 2048, 40, 16, 6)])
+def test_sweeps_agree_with_the_matrix_core_kernels(gpu, oracle, qtype, hidden, intermediate, experts, rows, topk):
+    """Wherever a workgroup's piece of the launch begins and ends, the sweeps publish what the matrix-core
+    kernels publish for the same worklist (both are the CPU path's bits)."""
+    from yvex_amd import kernels as K
+    qt = getattr(oracle, qtype)
+    g = oracle.Generator(42, f"pieces.{qtype}.{hidden}.{experts}")
+    tensors = [dev(g.weights(qt, experts * r, w), gpu) for r, w in
+               ((intermediate, hidden), (intermediate, hidden), (hidden, intermediate))]
+    weights = K.expert_weights(*tensors, (qt, qt, qt), hidden, intermediate)
+    status = K.new_status(gpu)
+    logits = dev(g.normal(rows * experts).reshape(rows, experts) - 0.35 * np.arange(experts), gpu)
+    selected, route = K.moe_route_rows(logits.float(), None, topk, K.SIGMOID, True, 1.0, status)
+    wl, pairs = K.worklist_build(selected, experts, status), rows * topk
+    act = K.q8k_quantize(dev(g.normal(rows * hidden).reshape(rows, hidden), gpu), status)
+    mid = [torch.zeros((pairs, intermediate), device=gpu) for _ in range(2)]
+    K.moe_up(weights, act, True, route, wl, pairs, topk, experts, 10.0, mid[0], status)
+    K.moe_up_rows(weights, act, route, wl, pairs, topk, experts, 10.0, mid[1], status)
+    assert same_bits(mid[0], mid[1])
+    mid_q8 = K.q8k_quantize(mid[0], status)
+    out = [torch.zeros((pairs, hidden), device=gpu) for _ in range(2)]
+    K.moe_down(weights, mid_q8, True, wl, pairs, experts, out[0], status)
+    K.moe_down_rows(weights, mid_q8, wl, pairs, experts, out[1], status)
+    assert same_bits(out[0], out[1]) and int(status.item()) == 0

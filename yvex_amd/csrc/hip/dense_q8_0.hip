@@ -407,6 +407,206 @@ __global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS) void dense_q8_0_sta
     if (bad) raise_status(g.status, 1);
 }
 
+// float(sum) of a matrix instruction's sums without a conversion each. The instruction starts from
+// 1.5 * 2^23 as an integer instead of zero; the sums of one block are below 2^20, so the bits of a result
+// are those of the float 12582912 + sum, and one addition, which two waves of a SIMD issue at
+// twice the rate of a conversion, leaves float(sum) exactly. (The constant sits in a vector register: an
+// addition with a scalar or literal operand issues at the conversion's rate.)
+struct FloatBias {
+    v16i start;
+    float minus;
+    __device__ __forceinline__ void set()
+    {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) start[i] = 0x4b400000;
+        minus = -12582912.0f;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm("" : "+v"(minus));
+#endif
+    }
+    __device__ __forceinline__ float value(int sum) const { return __int_as_float(sum) + minus; }
+};
+
+constexpr unsigned kWideRows = 128u, kWideTokens = 128u, kWideThreads = 512u;
+constexpr unsigned kWideWeightBytes = kWideRows * kStagedPitch, kWideActBytes = kWideTokens * kStagedPitch;  // one buffer
+constexpr unsigned kWideActBase = 2u * kWideWeightBytes, kWideScaleBase = kWideActBase + 2u * kWideActBytes;
+constexpr unsigned kWideLdsBytes = kWideScaleBase + 2u * kWideTokens * 4u;
+
+// The same product for batches that fill the device with tiles of 128 weight rows x 128 input rows.
+// Bound by vector-instruction issue: behind one matrix instruction (32 cycles) sixteen results a lane
+// are brought to float, multiplied by their scale and chained. What this kernel does about it:
+//  * FloatBias above in place of the conversions.
+//  * A wave owns 32 weight rows x 64 input rows: a block's codes and scale are read, and the
+//    even blocks shifted into place, once for two matrix instructions, and while the matrix pipe works
+//    on one 32-row block the vector ALU scales the other's results (a wave's own matrix and vector
+//    instructions overlap on this part).
+//  * The input rows' scales lie end to end in LDS: a lane's sixteen are four 16-byte reads, not
+//    sixteen 4-byte ones.
+//  * Copies take a scalar base and a 32-bit offset a lane: a register and no addition each.
+// 4096 x 4096 by 2048 rows 171 -> 138 us (498 TOP/s), 2048 x 7168 124 -> 104 us.
+__global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80Args g)
+{
+    extern __shared__ __align__(16) unsigned char dense_q8_0_lds[];
+    if (lds_address_of(dense_q8_0_lds) != 0u) {   // operands are addressed by absolute LDS offsets
+        if (threadIdx.x == 0u) raise_status(g.status, 2);
+        return;
+    }
+    choose_matrix(g);
+    const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const unsigned r = lane & 31u, h = lane >> 5;
+    const unsigned row_block = wave & 3u, token_pair = wave >> 2;
+    const unsigned long long row0 = (unsigned long long)blockIdx.x * kWideRows;
+    const unsigned long long tok0 = (unsigned long long)blockIdx.y * kWideTokens;
+    const unsigned rows_here = (unsigned)(g.row_count - row0 < kWideRows ? g.row_count - row0 : kWideRows);
+    const unsigned toks_here = (unsigned)(g.input_rows - tok0 < kWideTokens ? g.input_rows - tok0 : kWideTokens);
+    const unsigned act_row_bytes = g.blocks * kQ8KBytes, row_bytes = (unsigned)g.row_bytes;
+
+    // ---- copies: pieces q = tid + 512 k of 128 rows x 17 (a ragged edge repeats the tile's last row;
+    // an input row's seventeenth piece only keeps the pitch); the last 128 pieces of the weights by
+    // waves 0 and 1, of the input rows by waves 2 and 3, the input rows' scales by waves 4 and 5 ----
+    unsigned weight_at[5], act_at[5];
+#pragma unroll
+    for (unsigned k = 0; k < 5u; ++k) {
+        const unsigned q = k < 4u ? tid + kWideThreads * k : 2048u + (tid & 127u);
+        const unsigned row = q / 17u, piece = q - row * 17u;
+        weight_at[k] = (row < rows_here ? row : rows_here - 1u) * row_bytes + 16u * piece;
+        act_at[k] = (row < toks_here ? row : toks_here - 1u) * act_row_bytes + (piece < 16u ? 4u + 16u * piece : 0u);
+    }
+    const unsigned scale_token = tid & 127u;
+    const unsigned scale_at = (scale_token < toks_here ? scale_token : toks_here - 1u) * act_row_bytes;
+    const unsigned char *weights = g.encoded + row0 * g.row_bytes;
+    const unsigned char *acts = g.act + tok0 * act_row_bytes;
+    const unsigned wave_lds = (unsigned)__builtin_amdgcn_readfirstlane((int)(1024u * wave));
+    const unsigned scale_lds = (unsigned)__builtin_amdgcn_readfirstlane((int)(kWideScaleBase + 256u * (wave & 1u)));
+    const unsigned rest_lds = (unsigned)__builtin_amdgcn_readfirstlane((int)(2048u * 16u + 1024u * (wave & 1u)));
+    auto copies = [&](unsigned sb) {
+        const unsigned buffer = sb & 1u;
+        const unsigned char *w = weights + (unsigned long long)sb * 272ull;
+        const unsigned char *a = acts + (unsigned long long)sb * kQ8KBytes;
+        const unsigned w_to = buffer * kWideWeightBytes, a_to = kWideActBase + buffer * kWideActBytes;
+#pragma unroll
+        for (unsigned k = 0; k < 4u; ++k) {
+            copy_to_lds_16_at(w, weight_at[k], w_to + wave_lds + 16u * kWideThreads * k);
+            copy_to_lds_16_at(a, act_at[k], a_to + wave_lds + 16u * kWideThreads * k);
+        }
+        if (wave < 2u) copy_to_lds_16_at(w, weight_at[4], w_to + rest_lds);
+        else if (wave < 4u) copy_to_lds_16_at(a, act_at[4], a_to + rest_lds);
+        else if (wave < 6u) copy_to_lds_4_at(a, scale_at, scale_lds + buffer * (kWideTokens * 4u));
+    };
+
+    FloatBias bias;
+    bias.set();
+    double acc[2][16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.0;
+    copies(0u);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    for (unsigned sb = 0; sb < g.blocks; ++sb) {
+        const unsigned buffer = sb & 1u;
+        if (sb + 1u < g.blocks) copies(sb + 1u);
+        const unsigned w_row = buffer * kWideWeightBytes + (32u * row_block + r) * kStagedPitch;
+        const unsigned a_row = kWideActBase + buffer * kWideActBytes + (64u * token_pair + r) * kStagedPitch + 16u * h;
+        const unsigned scales = kWideScaleBase + buffer * (kWideTokens * 4u) + (64u * token_pair + 4u * h) * 4u;
+        float d_a[2][16], total[2][16];
+        uint4 lo[2], hi[2];
+        v4i tokens[2][2];
+        unsigned scale_bits[2];
+        auto read_block = [&](unsigned c) {
+            const unsigned slot = c % 2u;
+            const unsigned start = c % 2u == 0u ? 34u * c : 34u * c + 2u;      // the lane's window: + 16 h
+            lo[slot] = read16(w_row + 16u * h + (start & ~15u));
+            // (an even block's window is 20 bytes, an odd block's 16: only block 7's fits one piece)
+            hi[slot] = c % 2u == 0u || (start & 15u) ? read16(w_row + 16u * h + (start & ~15u) + 16u) : lo[slot];
+            scale_bits[slot] = lds_read_u16(w_row + 34u * c);
+            tokens[slot][0] = lds_read_v4i(a_row + 32u * c);
+            tokens[slot][1] = lds_read_v4i(a_row + 32u * kStagedPitch + 32u * c);
+        };
+        auto codes_of = [&](unsigned c) -> v4i {
+            const unsigned slot = c % 2u;
+            const unsigned start = c % 2u == 0u ? 34u * c : 34u * c + 2u, at = (start & 15u) / 4u;
+            const unsigned q[8] = {lo[slot].x, lo[slot].y, lo[slot].z, lo[slot].w,
+                                   hi[slot].x, hi[slot].y, hi[slot].z, hi[slot].w};
+            v4i codes;
+#pragma unroll
+            for (unsigned j = 0; j < 4u; ++j)
+                codes[j] = c % 2u == 0u ? (int)__builtin_amdgcn_alignbyte(q[at + j + 1u], q[at + j], 2u) : (int)q[at + j];
+            return codes;
+        };
+        v16i dot[2];
+        float d_w = 0.0f;
+        // (eight results at a time, one kind of instruction after another: a dependent instruction
+        // issues nine cycles behind its producer, and left alone the three of a result follow each other)
+        auto scale = [&](unsigned t, unsigned c) {
+#pragma unroll
+            for (int half = 0; half < 16; half += 8) {
+                float value[8], step[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) step[i] = d_w * d_a[t][half + i];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) value[i] = bias.value(dot[t][half + i]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    total[t][half + i] = c == 0u ? step[i] * value[i] : __builtin_fmaf(step[i], value[i], total[t][half + i]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        read_block(0u);       // (ahead of the scales, which the first matrix instruction does not wait for)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (unsigned t = 0; t < 2u; ++t)
+#pragma unroll
+            for (unsigned q = 0; q < 4u; ++q) {
+                const uint4 d = read16(scales + (32u * t + 8u * q) * 4u);
+                d_a[t][4u * q] = __uint_as_float(d.x); d_a[t][4u * q + 1u] = __uint_as_float(d.y);
+                d_a[t][4u * q + 2u] = __uint_as_float(d.z); d_a[t][4u * q + 3u] = __uint_as_float(d.w);
+            }
+#pragma unroll
+        for (unsigned c = 0; c < 8u; ++c) {
+            if (c + 1u < 8u) read_block(c + 1u);
+            const v4i codes = codes_of(c);
+            dot[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(tokens[c % 2u][0], codes, bias.start, 0, 0, 0);
+            // (the scheduler would put the scaling of the results first and wait for them there)
+            __builtin_amdgcn_sched_barrier(0);
+            if (c) scale(1u, c - 1u);
+            __builtin_amdgcn_sched_barrier(0);
+            d_w = f16_bits_to_float(scale_bits[c % 2u]);
+            dot[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(tokens[c % 2u][1], codes, bias.start, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            scale(0u, c);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        scale(1u, 7u);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            acc[0][i] += (double)total[0][i];
+            acc[1][i] += (double)total[1][i];
+        }
+        // the next superblock's copies have landed and every wave is done with this one's buffers
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+
+    const unsigned long long row = row0 + 32u * row_block + r;
+    if (row >= g.row_count) return;
+    bool bad = false;
+#pragma unroll
+    for (unsigned t = 0; t < 2u; ++t)
+#pragma unroll
+        for (unsigned i = 0; i < 16u; ++i) {
+            const unsigned long long token = tok0 + 64u * token_pair + 32u * t + 8u * (i >> 2) + 4u * h + (i & 3u);
+            if (token >= g.input_rows) continue;
+            const unsigned long long at = token * g.out_stride + row;
+            const float sum = (float)acc[t][i];
+            const float value = g.additive ? sum + g.additive[at] : sum;
+            if (!finite_f32(value)) bad = true;
+            else g.out[at] = g.output_bf16 ? bf16_round(value) : value;
+        }
+    if (bad) raise_status(g.status, 1);
+}
+
 }  // namespace
 
 int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t row_width,
@@ -427,7 +627,8 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
     // Which tiles: a pass over the row width costs a workgroup about the same whatever the device's
     // load (measured at 16 superblocks a row, microseconds: 17 unstaged and 27 once two such
     // workgroups share a compute unit, 29 on the 64-row staged tile and 43 once two of them share
-    // a compute unit, 35 on the 128-row tile), so the choice is the number of rounds each shape needs.
+    // a compute unit, 35 on the 128-row tile, 56 on the 128 x 128 tile), so the choice is the number of
+    // rounds each shape needs.
     const uint64_t token_tiles32 = (input_rows + 31u) / 32u;
     const uint64_t token_tiles64 = (input_rows + 63u) / 64u;
     if (token_tiles32 > 65535ull) return ST_BOUNDS;
@@ -449,6 +650,17 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
         const double low_share = 43.0 * (double)low / (double)(2u * units);
         const double low_cost = low <= units ? 29.0 : (low_share > 43.0 ? low_share : 43.0);
         const double tall_cost = 35.0 * (double)((tall + units - 1u) / units);
+        const uint64_t token_tiles128 = (input_rows + 127u) / 128u;
+        const uint64_t wide = matrices * ((row_count + 127u) / 128u) * token_tiles128;
+        const double wide_cost = 56.0 * (double)((wide + units - 1u) / units);
+        // (32-bit offsets into a tile's rows)
+        if (wide_cost < plain_cost && wide_cost <= low_cost && wide_cost <= tall_cost &&
+            row_bytes <= (1ull << 24) && row_width / 256u * kQ8KBytes <= (1ull << 24)) {
+            YVEX_ALLOW_DYNAMIC_LDS(dense_q8_0_wide_kernel, kWideLdsBytes);
+            dense_q8_0_wide_kernel<<<dim3((unsigned)((row_count + 127u) / 128u), (unsigned)token_tiles128,
+                                          (unsigned)matrices), kWideThreads, kWideLdsBytes, stream>>>(g);
+            return check_launch("dense_q8_0_wide");
+        }
         if (tall_cost < plain_cost && tall_cost <= low_cost) {
             YVEX_ALLOW_DYNAMIC_LDS(dense_q8_0_staged_kernel<4u>, staged_lds_bytes(4u));
             dense_q8_0_staged_kernel<4u><<<dim3((unsigned)((row_count + 127u) / 128u), (unsigned)token_tiles64, (unsigned)matrices), 512,

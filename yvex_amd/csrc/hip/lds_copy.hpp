@@ -97,6 +97,30 @@ __device__ __forceinline__ void copy_to_lds_16(const void *global, unsigned lds_
     (void)lds_base;
 #endif
 }
+// The same with the address as a wave-uniform base and a 32-bit offset a lane: a kernel that walks its
+// operands keeps one register a copy and advances the bases on the scalar unit.
+__device__ __forceinline__ void copy_to_lds_16_at(const void *base, unsigned offset, unsigned lds_base)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :: "s"(lds_base), "v"(offset), "s"(base) : "memory", "m0");
+#else
+    (void)base;
+    (void)offset;
+    (void)lds_base;
+#endif
+}
+__device__ __forceinline__ void copy_to_lds_4_at(const void *base, unsigned offset, unsigned lds_base)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                 :: "s"(lds_base), "v"(offset), "s"(base) : "memory", "m0");
+#else
+    (void)base;
+    (void)offset;
+    (void)lds_base;
+#endif
+}
 __device__ __forceinline__ void copy_to_lds_4(const void *global, unsigned lds_base)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
