@@ -280,9 +280,12 @@ int yvex_hip_moe_down(const yvex_hip_expert_weights *weights, const void *interm
 /* Row-batch (prefill-width) forms of the two sweeps above on the int8 matrix cores; they replace
  * yvex_moe_grouped_up_tensorcore / _down_tensorcore (tensorcore.cu:378-702). Same inputs,
  * outputs and rounding points as yvex_hip_moe_up / yvex_hip_moe_down with act_q8 = 1; weights
- * must be IQ2_XXS. A work item is 64 ordered pairs of one bucket times a tile of 256 weight rows,
- * so buckets of any population are served; expert_ids == NULL is the single-bucket form
- * (shared expert: every pair uses expert 0, order may be NULL for the identity). */
+ * must be IQ2_XXS or Q4_K, for the down projection also Q2_K. A work item is 64 ordered pairs of one
+ * bucket times a tile of weight rows, so buckets of any population are served; expert_ids == NULL
+ * is the single-bucket form (shared expert: every pair uses expert 0, order may be NULL for the
+ * identity). What a bucket holds behind whole tiles, if it is a dozen pairs or so, and small single
+ * buckets run through a second kind of kernel where the rows are Q4_K, Q2_K or IQ2_XXS sweep
+ * images; the functions named ..._launches say how many launches (1 or 2) a call makes. */
 int yvex_hip_moe_up_rows(const yvex_hip_expert_weights *weights, const void *act_q8k,
                          const float *route_weights, const uint64_t *order,
                          const uint64_t *expert_ids, const uint64_t *bucket_offsets,
@@ -294,6 +297,12 @@ int yvex_hip_moe_down_rows(const yvex_hip_expert_weights *weights, const void *i
                            const uint64_t *bucket_offsets, const uint64_t *bucket_populations,
                            const uint64_t *counts, uint64_t pairs, uint64_t experts,
                            float *pair_outputs, int *status, yvex_hip_stream stream);
+unsigned int yvex_hip_moe_up_rows_launches(const yvex_hip_expert_weights *weights, const void *act_q8k,
+                                           const uint64_t *expert_ids, uint64_t pairs, uint64_t topk,
+                                           uint64_t experts, float *intermediate);
+unsigned int yvex_hip_moe_down_rows_launches(const yvex_hip_expert_weights *weights, const void *intermediate_q8k,
+                                             const uint64_t *expert_ids, uint64_t pairs, uint64_t experts,
+                                             float *pair_outputs);
 
 /* The SwiGLU stage of an expert whose gate and up projections ran as dense projections (a shared
  * expert of a format the expert kernels do not take): out[i] = bf16(silu(min(gate[i], limit)) *

@@ -184,3 +184,52 @@ def test_sweeps_agree_with_the_matrix_core_kernels(gpu, oracle, qtype, hidden, i
     K.moe_down(weights, mid_q8, True, wl, pairs, experts, out[0], status)
     K.moe_down_rows(weights, mid_q8, wl, pairs, experts, out[1], status)
     assert same_bits(out[0], out[1]) and int(status.item()) == 0
+
+
+# a pair, a remainder of the largest size the few-pair kernels take at the width and one more, 64-pair
+# tiles with and without such remainders; two, three and 32 superblocks a row, ragged row units
+@pytest.mark.parametrize("up,down,hidden,intermediate,tokens", [
+    ("IQ2_XXS", "Q2_K", 1024, 768, 16), ("IQ2_XXS", "IQ2_XXS", 7168, 512, 12), ("Q4_K", "Q4_K", 768, 1024, 16),
+    ("Q4_K", "Q2_K", 7168, 512, 16), ("IQ2_XXS", "Q4_K", 8192, 256, 8), ("IQ2_XXS", "Q2_K", 512, 2304, 16)])
+def test_few_pair_kernels_agree_with_the_generic_kernel(gpu, oracle, up, down, hidden, intermediate, tokens):
+    """Buckets split between the two row-batch kernels by their remainders, and a matrix alone, hold
+    what the generic grouped kernel (the CPU path's bits) publishes for the same pairs."""
+    from yvex_amd import kernels as K
+    uq, dq = getattr(oracle, up), getattr(oracle, down)
+    populations = [1, tokens, tokens + 1, 64 + tokens, 64, 0, 64 + tokens + 1, 5]
+    experts, pairs = len(populations), sum(populations)
+    g = oracle.Generator(43, f"few.{up}.{down}.{hidden}")
+    tensors = [dev(g.weights(q, experts * r, w), gpu) for q, r, w in
+               ((uq, intermediate, hidden), (uq, intermediate, hidden), (dq, hidden, intermediate))]
+    weights = K.expert_weights(*tensors, (uq, uq, dq), hidden, intermediate)
+    rows_form = K.expert_weights(*tensors, (uq, uq, dq), hidden, intermediate)
+    images = [K.iq2_sweep_image(t) if q == oracle.IQ2_XXS else None for t, q in zip(tensors, (uq, uq, dq))]
+    if images[0] is not None:
+        rows_form.gate, rows_form.up, rows_form.gate_up_image = images[0].data_ptr(), images[1].data_ptr(), 1
+        rows_form.gate_row_bytes = rows_form.up_row_bytes = hidden // 256 * 72
+        rows_form.gate_expert_bytes = rows_form.up_expert_bytes = hidden // 256 * 72 * intermediate
+    if images[2] is not None:
+        rows_form.down, rows_form.down_image = images[2].data_ptr(), 1
+        rows_form.down_row_bytes, rows_form.down_expert_bytes = intermediate // 256 * 72, intermediate // 256 * 72 * hidden
+    status = K.new_status(gpu)
+    selected = torch.repeat_interleave(torch.arange(experts), torch.tensor(populations))
+    selected = selected[torch.randperm(pairs, generator=torch.Generator().manual_seed(3))].reshape(pairs, 1).to(gpu)
+    wl = K.worklist_build(selected, experts, status)
+    route = dev((0.5 + np.abs(g.normal(pairs))).astype(np.float32), gpu)
+    act = K.q8k_quantize(dev(g.normal(pairs * hidden).reshape(pairs, hidden), gpu), status)
+    mid = [torch.zeros((pairs, intermediate), device=gpu) for _ in range(2)]
+    K.moe_up(weights, act, True, route, wl, pairs, 1, experts, 10.0, mid[0], status)
+    K.moe_up_rows(rows_form, act, route, wl, pairs, 1, experts, 10.0, mid[1], status)
+    assert same_bits(mid[0], mid[1])
+    mid_q8 = K.q8k_quantize(mid[0], status)
+    out = [torch.zeros((pairs, hidden), device=gpu) for _ in range(2)]
+    K.moe_down(weights, mid_q8, True, wl, pairs, experts, out[0], status)
+    K.moe_down_rows(rows_form, mid_q8, wl, pairs, experts, out[1], status)
+    assert same_bits(out[0], out[1])
+    for alone in (tokens + 3, 257):                     # one matrix for all rows: either kernel
+        some = K.q8k_quantize(dev(g.normal(alone * hidden).reshape(alone, hidden), gpu), status)
+        mid = [torch.zeros((alone, intermediate), device=gpu) for _ in range(2)]
+        K.moe_up(weights, some, True, None, None, alone, 1, 1, 10.0, mid[0], status)
+        K.moe_up_rows(rows_form, some, None, None, alone, 1, 1, 10.0, mid[1], status)
+        assert same_bits(mid[0], mid[1])
+    assert int(status.item()) == 0

@@ -157,9 +157,18 @@ bool iq2_sweep_supported(unsigned qtype, unsigned width, unsigned out_rows, unsi
 int launch_iq2_sweep(const GroupedArgs &a, unsigned qtype, bool fused, bool image, hipStream_t stream);
 
 // Row-batch expert kernels on the int8 matrix cores (rows_q4k.hip): Q4_K weights, fused gate/up
-// or a plain projection; Q2_K weights, a plain projection (the down experts).
+// or a plain projection; Q2_K weights, a plain projection (the down experts). A bucket's last tile of
+// up to `left` pairs is left to the kernels below.
 int launch_q4k_rows_grouped(const GroupedProblem &problem, unsigned qtype, bool fused, uint64_t width,
-                            uint64_t out_rows, double limit, int *status, hipStream_t stream);
+                            uint64_t out_rows, unsigned left, double limit, int *status, hipStream_t stream);
+
+// The same problems where few pairs meet (rows16.hip): IQ2_XXS sweep images and Q4_K rows, fused
+// gate/up or plain; Q2_K rows, plain. The first: pairs of a full tile, 0 for a problem the kernels do
+// not serve. The second serves whole buckets (`behind` 0), or what a bucket holds behind whole tiles
+// of `behind` pairs where that fits one tile.
+unsigned rows16_tokens(const GroupedProblem &problem, unsigned qtype, bool fused, uint64_t width, uint64_t out_rows);
+int launch_rows16_grouped(const GroupedProblem &problem, unsigned qtype, bool fused, unsigned width,
+                          unsigned out_rows, unsigned behind, double limit, int *status, hipStream_t stream);
 
 static inline bool same_shape(const yvex_hip_expert_weights *a, const yvex_hip_expert_weights *b)
 {

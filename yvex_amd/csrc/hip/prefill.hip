@@ -49,6 +49,7 @@
 #include "launch.hpp"
 #include "grouped.hpp"
 #include "lds_copy.hpp"
+#include "iq2_limbs.hpp"
 
 namespace yvex {
 
@@ -92,54 +93,17 @@ struct MfmaArgs {
     int *status;
     int plain_output;        // plain projection: outputs stay fp32 instead of being rounded to bf16
     int image;               // weights are the sweep image (72-byte records) instead of canonical bytes
+    unsigned left;           // a bucket's last tile of up to this many pairs is not this launch's (rows16.hip)
 };
-
-// Limb pair of one magnitude: low limb in bits 0-7, high limb in bits 8-15.
-__device__ __forceinline__ unsigned iq2_limbs(unsigned level, unsigned factor)
-{
-    const unsigned magnitude = level * factor;
-    unsigned hi = (magnitude + 64u) >> 7;
-    if (hi == 0u) hi = 1u;
-    const int lo = (int)magnitude - 128 * (int)hi;
-    return ((unsigned)lo & 255u) | (hi << 8);
-}
 
 __device__ __forceinline__ void mfma_tables_fill()
 {
-    // level codes: byte l of the entry is 0, 1 or 2 for level 8, 25 or 43 of weight l
-    for (unsigned index = threadIdx.x; index < 256u * 16u; index += blockDim.x) {
-        const uint2 m = iq2_magnitude_entry(index >> 4);
-        uint2 codes = make_uint2(0u, 0u);
-#pragma unroll
-        for (unsigned l = 0; l < 4u; ++l) {
-            const unsigned a = (m.x >> (8u * l)) & 255u, b = (m.y >> (8u * l)) & 255u;
-            codes.x |= (a == 8u ? 0u : a == 25u ? 1u : 2u) << (8u * l);
-            codes.y |= (b == 8u ? 0u : b == 25u ? 1u : 2u) << (8u * l);
-        }
-        lds_write_uint2(kCodeBase + (index >> 4) * 256u + (index & 15u) * 8u, codes);
-    }
-    // sign selectors: byte l is 4 when weight l is negative (7 stored bits + parity)
-    for (unsigned index = threadIdx.x; index < 128u * 16u; index += blockDim.x) {
-        const uint2 m = iq2_signmask_entry(index >> 4);
-        lds_write_uint2(kSelBase + (index >> 4) * 256u + (index & 15u) * 8u,
-                        make_uint2(m.x & 0x04040404u, m.y & 0x04040404u));
-    }
-    // limb words of scale s: {+lo, -lo, +hi, -hi}, byte c = limb of level code c
-    for (unsigned index = threadIdx.x; index < 16u * 16u; index += blockDim.x) {
-        const unsigned factor = 2u * (index >> 4) + 1u;
-        unsigned lo = 0u, hi = 0u;
-        const unsigned levels[3] = {8u, 25u, 43u};
-#pragma unroll
-        for (unsigned c = 0; c < 3u; ++c) {
-            const unsigned pair = iq2_limbs(levels[c], factor);
-            lo |= (pair & 255u) << (8u * c);
-            hi |= (pair >> 8) << (8u * c);
-        }
-        // byte-wise negation: no limb is zero, so (x ^ 0xff) + 1 never carries; byte 3 stays 0
-        const unsigned neg_lo = ((lo ^ 0x00ffffffu) + 0x00010101u) & 0x00ffffffu;
-        const unsigned neg_hi = ((hi ^ 0x00ffffffu) + 0x00010101u) & 0x00ffffffu;
-        lds_write_uint4(kLutBase + index * 16u, make_uint4(lo, neg_lo, hi, neg_hi));
-    }
+    for (unsigned index = threadIdx.x; index < 256u * 16u; index += blockDim.x)
+        lds_write_uint2(kCodeBase + (index >> 4) * 256u + (index & 15u) * 8u, iq2_level_codes(index >> 4));
+    for (unsigned index = threadIdx.x; index < 128u * 16u; index += blockDim.x)
+        lds_write_uint2(kSelBase + (index >> 4) * 256u + (index & 15u) * 8u, iq2_sign_selectors(index >> 4));
+    for (unsigned index = threadIdx.x; index < 16u * 16u; index += blockDim.x)
+        lds_write_uint4(kLutBase + index * 16u, iq2_limb_words(index >> 4));
 }
 
 // What one work item needs to know about its place in the problem.
@@ -675,11 +639,10 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
     const bool fixed = pr.expert_ids == nullptr;
     const unsigned buckets = fixed ? 1u : (unsigned)pr.counts[0];
 
-    // The buckets' populations are requested before the tables are built (one round trip to
-    // memory under the fill instead of one per bucket after it).
+    // The buckets' populations are requested together (one round trip to memory instead of one per
+    // bucket), and the tables built only where there is an item.
     unsigned long long population_here = 0ull;
     if (tid < 256u && tid < buckets) population_here = fixed ? pr.pairs : pr.bucket_populations[tid];
-    mfma_tables_fill();
     // Full 64-pair tiles come first in the item list, then the partial last tiles by size,
     // largest first: every workgroup, walking the list with the grid's stride, gets the same
     // share of each kind of item, and the short items come last. Bucket b's first full tile is
@@ -690,7 +653,7 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
         const unsigned lane = tid & 63u, wave = tid >> 6;
         const unsigned full = tid < 256u ? (unsigned)(population_here / kTileTokens) : 0u;
         const unsigned rest = tid < 256u ? (unsigned)(population_here % kTileTokens) : 0u;
-        const unsigned cls = rest == 0u ? 2u : rest > 32u ? 0u : 1u;
+        const unsigned cls = rest <= a.left ? 2u : rest > 32u ? 0u : 1u;
         unsigned inclusive = full;
 #pragma unroll
         for (int offset = 1; offset < 64; offset <<= 1) {
@@ -739,6 +702,9 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
         members[c] = lds_read_u32(kClassCountBase + 4u * c);
         items += (unsigned long long)members[c] * row_tiles;
     }
+    if (blockIdx.x >= items) return;
+    mfma_tables_fill();
+    __syncthreads();
 
     // ---- which bucket, row tile and token tile an item is: the bucket's record is requested... ----
     auto request_item = [&](unsigned long long item) {
@@ -857,6 +823,41 @@ static int launch_mfma(const MfmaArgs &a, hipStream_t stream)
                    : launch_mfma_variant<FUSED_UP, false>(a, stream);
 }
 
+// Expert matrices against the buckets of a worklist. Where the few-pair kernels serve the rows
+// (IQ2_XXS sweep images, Q4_K and Q2_K rows), they take what a bucket holds behind its whole
+// 64-pair tiles if that fits one of their tiles (12 pairs at width 7168, 16 up to about 5000): such a tile
+// takes them 1.4 us of the whole device for the 2 x 2048 x 4096 IQ2_XXS rows of an expert, and the 64-pair
+// kernels, which pay for 32 token columns, 2.3 us; with two of theirs (from 17 pairs on, 2.8 us) it
+// is the other way round. A matrix that is alone (no worklist) is theirs up to 256 rows, where the
+// other kernels have fewer items than there are compute units.
+struct RowsPlan {
+    unsigned few;            // pairs of a full tile of the few-pair kernel, 0: it does not run
+    bool many;               // the 64-pair kernel runs
+};
+
+static RowsPlan plan_rows(const GroupedProblem &pr, unsigned qtype, bool fused, int image, uint64_t width, uint64_t out_rows)
+{
+    constexpr unsigned kAloneRows = 256u;
+    const bool alone = pr.expert_ids == nullptr, readable = qtype != QT_IQ2_XXS || image;
+    const unsigned few = readable && !(alone && pr.pairs > kAloneRows) ? rows16_tokens(pr, qtype, fused, width, out_rows) : 0u;
+    return {few, !few || (!alone && pr.pairs > few)};
+}
+
+template <bool FUSED_UP>
+static int launch_rows(MfmaArgs &a, unsigned qtype, hipStream_t stream)
+{
+    const RowsPlan plan = plan_rows(a.pr, qtype, FUSED_UP, a.image, a.width, a.out_rows);
+    a.left = plan.few;
+    if (plan.many) {
+        const int rc = qtype == QT_IQ2_XXS
+            ? launch_mfma<FUSED_UP>(a, stream)
+            : launch_q4k_rows_grouped(a.pr, qtype, FUSED_UP, a.width, a.out_rows, plan.few, a.limit, a.status, stream);
+        if (rc || !plan.few) return rc;
+    }
+    return launch_rows16_grouped(a.pr, qtype, FUSED_UP, a.width, a.out_rows, a.pr.expert_ids ? kTileTokens : 0u, a.limit,
+                                 a.status, stream);
+}
+
 // A plain projection through the row-batch kernel: every input row in one bucket of expert 0.
 int launch_iq2_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t row_width,
                           uint64_t row_bytes, const void *act_q8k, uint64_t input_rows, float *out,
@@ -888,6 +889,30 @@ int launch_iq2_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t r
 using namespace yvex;
 
 
+extern "C" unsigned yvex_hip_moe_up_rows_launches(const yvex_hip_expert_weights *w, const void *act_q8k,
+                                                  const uint64_t *expert_ids, uint64_t pairs, uint64_t topk,
+                                                  uint64_t experts, float *intermediate)
+{
+    if (!w || pairs > 0xffffffffull) return 1u;
+    GroupedProblem pr{};
+    const WorklistView wl{nullptr, expert_ids, nullptr, nullptr, nullptr, nullptr};
+    fill_up_problem(pr, w, act_q8k, 1, nullptr, wl, pairs, topk, experts, intermediate);
+    const RowsPlan plan = plan_rows(pr, w->gate_qtype, true, w->gate_up_image, w->hidden, w->intermediate);
+    return (plan.few ? 1u : 0u) + (plan.many ? 1u : 0u);
+}
+
+extern "C" unsigned yvex_hip_moe_down_rows_launches(const yvex_hip_expert_weights *w, const void *intermediate_q8k,
+                                                    const uint64_t *expert_ids, uint64_t pairs, uint64_t experts,
+                                                    float *pair_outputs)
+{
+    if (!w || pairs > 0xffffffffull) return 1u;
+    GroupedProblem pr{};
+    const WorklistView wl{nullptr, expert_ids, nullptr, nullptr, nullptr, nullptr};
+    fill_down_problem(pr, w, intermediate_q8k, 1, wl, pairs, experts, pair_outputs);
+    const RowsPlan plan = plan_rows(pr, w->down_qtype, false, w->down_image, w->intermediate, w->hidden);
+    return (plan.few ? 1u : 0u) + (plan.many ? 1u : 0u);
+}
+
 extern "C" int yvex_hip_moe_up_rows(const yvex_hip_expert_weights *w, const void *act_q8k,
                                     const float *route_weights, const uint64_t *order,
                                     const uint64_t *expert_ids, const uint64_t *bucket_offsets,
@@ -910,14 +935,12 @@ extern "C" int yvex_hip_moe_up_rows(const yvex_hip_expert_weights *w, const void
     MfmaArgs a{};
     const WorklistView wl{order, expert_ids, bucket_offsets, bucket_populations, nullptr, counts};
     fill_up_problem(a.pr, w, act_q8k, 1, route_weights, wl, pairs, topk, experts, intermediate);
-    if (w->gate_qtype == QT_Q4_K)
-        return launch_q4k_rows_grouped(a.pr, QT_Q4_K, true, w->hidden, w->intermediate, limit, status, as_stream(stream));
     a.width = (unsigned)w->hidden;
     a.out_rows = (unsigned)w->intermediate;
     a.limit = limit;
     a.status = status;
     a.image = w->gate_up_image != 0;
-    return launch_mfma<true>(a, as_stream(stream));
+    return launch_rows<true>(a, w->gate_qtype, as_stream(stream));
 }
 
 extern "C" int yvex_hip_moe_down_rows(const yvex_hip_expert_weights *w, const void *intermediate_q8k,
@@ -939,13 +962,10 @@ extern "C" int yvex_hip_moe_down_rows(const yvex_hip_expert_weights *w, const vo
     MfmaArgs a{};
     const WorklistView wl{order, expert_ids, bucket_offsets, bucket_populations, nullptr, counts};
     fill_down_problem(a.pr, w, intermediate_q8k, 1, wl, pairs, experts, pair_outputs);
-    if (w->down_qtype == QT_Q4_K || w->down_qtype == QT_Q2_K)
-        return launch_q4k_rows_grouped(a.pr, w->down_qtype, false, w->intermediate, w->hidden, 1.0, status,
-                                       as_stream(stream));
     a.width = (unsigned)w->intermediate;
     a.out_rows = (unsigned)w->hidden;
     a.limit = 1.0;
     a.status = status;
     a.image = w->down_image != 0;
-    return launch_mfma<false>(a, as_stream(stream));
+    return launch_rows<false>(a, w->down_qtype, as_stream(stream));
 }

@@ -41,12 +41,11 @@
 #include "launch.hpp"
 #include "grouped.hpp"
 #include "lds_copy.hpp"
+#include "kquant_limbs.hpp"
 
 namespace yvex {
 
 namespace {
-
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 // One 16-byte LDS read (as a vector value, so that it stays one instruction).
 __device__ __forceinline__ uint4 read16(unsigned address)
@@ -77,53 +76,10 @@ struct RowsQ4kArgs {
     int *status;
     // plain projection (one bucket holding every input row): out[token * out_stride + row]
     int plain, output_bf16;
+    unsigned left;           // a bucket's last tile of up to this many pairs is not this launch's (rows16.hip)
     const float *additive;
     unsigned long long out_stride;
 };
-
-// Two int8 limbs of sc * nibble for the four nibbles of one dword, value = 8 hi + lo (see
-// dense_q4k.hip).
-__device__ __forceinline__ void q4k_limbs(unsigned x, unsigned sc, unsigned &lo, unsigned &hi)
-{
-    const unsigned nibbles = x & 0x0f0f0f0fu;
-    const unsigned low = (sc & 7u) * 0x00010001u, high = ((sc >> 3) & 7u) * 0x00010001u;
-    lo = __builtin_bit_cast(unsigned, __builtin_bit_cast(u16x2, nibbles) * __builtin_bit_cast(u16x2, low));
-    hi = __builtin_bit_cast(unsigned, __builtin_bit_cast(u16x2, nibbles) * __builtin_bit_cast(u16x2, high));
-}
-
-// Pair sums of the 16 int16 block sums as two int8 limbs (value = 128 hi + lo, lo in 0..127).
-__device__ __forceinline__ void q4k_bsum_limbs(const uint4 (&b)[2], uint2 &lo, uint2 &hi)
-{
-    const unsigned w[8] = {b[0].x, b[0].y, b[0].z, b[0].w, b[1].x, b[1].y, b[1].z, b[1].w};
-    unsigned l[2] = {0u, 0u}, u[2] = {0u, 0u};
-#pragma unroll
-    for (unsigned s = 0; s < 8u; ++s) {
-        const int pair = (int)(short)(w[s] & 0xffffu) + ((int)w[s] >> 16);
-        l[s >> 2] |= ((unsigned)pair & 127u) << (8u * (s & 3u));
-        u[s >> 2] |= ((unsigned)(pair >> 7) & 255u) << (8u * (s & 3u));
-    }
-    lo = make_uint2(l[0], l[1]);
-    hi = make_uint2(u[0], u[1]);
-}
-
-// The sixteen int16 block sums as two int8 limbs (value = 128 hi + lo, lo in 0..127), in order.
-__device__ __forceinline__ void q2k_bsum_limbs(const uint4 (&b)[2], v4i &lo, v4i &hi)
-{
-    const unsigned w[8] = {b[0].x, b[0].y, b[0].z, b[0].w, b[1].x, b[1].y, b[1].z, b[1].w};
-#pragma unroll
-    for (unsigned i = 0; i < 4u; ++i) {
-        unsigned l = 0u, u = 0u;
-#pragma unroll
-        for (unsigned k = 0; k < 4u; ++k) {
-            const unsigned word = w[2u * i + k / 2u];
-            const int sum = k % 2u ? (int)word >> 16 : (int)(short)(word & 0xffffu);
-            l |= ((unsigned)sum & 127u) << (8u * k);
-            u |= ((unsigned)(sum >> 7) & 255u) << (8u * k);
-        }
-        lo[i] = (int)l;
-        hi[i] = (int)u;
-    }
-}
 
 struct Q4Tile {
     unsigned long long expert, first;
@@ -275,13 +231,9 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
                     const unsigned c = 4u * p + sft;
                     // scale byte 2 c + h: word c / 2, byte (2 c) % 4 + h
                     const unsigned sc = (scale_words[c >> 1] >> (8u * ((2u * c) & 3u) + 8u * h)) & 15u;
-                    const u16x2 twice = __builtin_bit_cast(u16x2, sc * 0x00010001u);
                     v4i a;
 #pragma unroll
-                    for (unsigned i = 0; i < 4u; ++i)
-                        // two bytes a 16-bit lane: (code * sc) stays inside its byte
-                        a[i] = (int)__builtin_bit_cast(unsigned,
-                                                       __builtin_bit_cast(u16x2, (q[i] >> (2u * sft)) & 0x03030303u) * twice);
+                    for (unsigned i = 0; i < 4u; ++i) a[i] = (int)q2k_limb(q[i] >> (2u * sft), sc);
 #pragma unroll
                     for (unsigned nt = 0; nt < NT; ++nt) {
                         const v4i b = lds_read_v4i(a_at + nt * 32u * 256u + 16u * ((2u * c + h) ^ (r & 15u)));
@@ -471,7 +423,7 @@ __global__ __launch_bounds__(kQ4Threads, 2) void rows_q4k_kernel(RowsQ4kArgs g)
     } else {
         const unsigned buckets = (unsigned)pr.counts[0];
         const unsigned long long population = threadIdx.x < buckets ? pr.bucket_populations[threadIdx.x] : 0ull;
-        const unsigned tiles = (unsigned)((population + kQ4Tokens - 1ull) / kQ4Tokens);
+        const unsigned tiles = (unsigned)(population / kQ4Tokens) + (population % kQ4Tokens > g.left ? 1u : 0u);
         unsigned inclusive = tiles;
 #pragma unroll
         for (int offset = 1; offset < 64; offset <<= 1) {
@@ -520,7 +472,7 @@ int launch_rows_q4k(const RowsQ4kArgs &g, dim3 grid, hipStream_t stream)
 }  // namespace
 
 int launch_q4k_rows_grouped(const GroupedProblem &problem, unsigned qtype, bool fused, uint64_t width,
-                            uint64_t out_rows, double limit, int *status, hipStream_t stream)
+                            uint64_t out_rows, unsigned left, double limit, int *status, hipStream_t stream)
 {
     if (qtype != QT_Q4_K && !(qtype == QT_Q2_K && !fused)) return ST_UNSUPPORTED;
     if (!width || width % 256u || !out_rows || out_rows > 0x7fffffffull) return ST_BOUNDS;
@@ -535,11 +487,13 @@ int launch_q4k_rows_grouped(const GroupedProblem &problem, unsigned qtype, bool 
         return ST_INVALID_ARG;
     if (problem.experts > 256u && problem.expert_ids) return ST_BOUNDS;
     const uint64_t row_tiles = (out_rows + (fused ? 63u : 127u)) / (fused ? 64u : 128u);
-    // token tiles: every bucket may end in a partial tile
-    const uint64_t token_tiles = problem.expert_ids ? (uint64_t)problem.pairs / kQ4Tokens + problem.experts
+    // token tiles: every bucket of more than `left` pairs may end in a partial tile
+    const uint64_t partial = (uint64_t)problem.pairs / (left + 1u);
+    const uint64_t token_tiles = problem.expert_ids ? (uint64_t)problem.pairs / kQ4Tokens +
+                                                          (partial < problem.experts ? partial : problem.experts)
                                                     : ((uint64_t)problem.pairs + kQ4Tokens - 1u) / kQ4Tokens;
     if (row_tiles > 0x7fffffffull || token_tiles > 65535ull) return ST_BOUNDS;
-    RowsQ4kArgs g{problem, (unsigned)(width / 256u), (unsigned)out_rows, limit, status, 0, 0, nullptr, 0ull};
+    RowsQ4kArgs g{problem, (unsigned)(width / 256u), (unsigned)out_rows, limit, status, 0, 0, left, nullptr, 0ull};
     const dim3 grid((unsigned)row_tiles, (unsigned)token_tiles);
     if (qtype == QT_Q2_K) return launch_rows_q4k<QT_Q2_K, false>(g, grid, stream);
     return fused ? launch_rows_q4k<QT_Q4_K, true>(g, grid, stream) : launch_rows_q4k<QT_Q4_K, false>(g, grid, stream);
@@ -570,7 +524,7 @@ int launch_q4k_rows_staged(const uint8_t *encoded, uint64_t row_count, uint64_t 
     const uint64_t token_tiles = (input_rows + kQ4Tokens - 1u) / kQ4Tokens;
     if (token_tiles > 65535ull) return ST_BOUNDS;
     RowsQ4kArgs g{problem, (unsigned)(row_width / 256u), (unsigned)row_count, 0.0, status, 1, output_bf16 ? 1 : 0,
-                  additive, out_stride};
+                  0u, additive, out_stride};
     return launch_rows_q4k<QT_Q4_K, false>(g, dim3((unsigned)row_tiles, (unsigned)token_tiles), stream);
 }
 

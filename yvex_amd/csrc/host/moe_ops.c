@@ -502,6 +502,7 @@ static int moe_execute_rows(yvex_rocm_backend *backend, const yvex_moe_layer_job
     const float *bias_rows;
     void *combined_target;
     unsigned long long table_address = 0ull;
+    unsigned int matrix_launches[4] = {0};   /* routed up and down, shared up and down */
     int matrix_allowed = 1, envelope, hash_router, unsupported_width, routed_q8 = 0, shared_q8 = 0, routed_image = 0, shared_image = 0, has_shared, merged, row_batch, shared_row_batch, shared_dense, device_status = 0, rc, defer, host_rows, combined_egress, swiglu_quantized, routed_rows = 0;
     void *status;
     yvex_hip_stream stream;
@@ -679,17 +680,24 @@ static int moe_execute_rows(yvex_rocm_backend *backend, const yvex_moe_layer_job
         fill_expert_weights(&shared, &views[YVEX_MOE_WEIGHT_SHARED_GATE], &views[YVEX_MOE_WEIGHT_SHARED_UP],
                             &views[YVEX_MOE_WEIGHT_SHARED_DOWN], addresses[3], addresses[4], addresses[5],
                             hidden, layer->shared_intermediate_width, shared_image);
-    /* Row batches whose buckets average six pairs or more (four with Q4_K gate and up rows) go to
-     * the int8 matrix-core kernels (IQ2_XXS or Q4_K weights, Q8_K activations); below that the decode
-     * sweeps, which read an expert's bytes once per four pairs, are faster: with 256 experts and
-     * top-8 the two families cross at about 170 rows (IQ2_XXS) and 128 rows (Q4_K). The
+    /* Row batches whose buckets average three pairs or more go to the int8 matrix-core kernels
+     * (IQ2_XXS or Q4_K weights, Q8_K activations; IQ2_XXS as canonical bytes, which the few-pair kernels
+     * among them do not read, from six pairs on); below that the decode sweeps, which read an expert's
+     * bytes once per four pairs, are faster. Gate/up and down launches of 256 experts, uniform
+     * routing: 7168 wide, top-8, 96 rows IQ2_XXS 824 us as sweeps and 858 as tiles, 112 rows 939 and 871;
+     * Q4_K 96 rows 1334 and 1306; 4096 wide, top-6, Q2_K down, 128 rows 485 and 527, 160 rows 568 and 543.
+     * A skewed routing is a little better off as tiles (96 rows at 7168, a Zipf exponent of 1.1: 430 us
+     * and 400). Layers of fewer than 32 experts keep the line at six (four with Q4_K rows), where
+     * the published launch facts have had it: their launches are 20-50 us either way. The
      * reference switches its tensor-core kernels on from 16 input rows
      * (src/backend/cuda/private.h:461-464). Both kernel families read the sweep image of
      * IQ2_XXS experts as well as canonical bytes, and both publish the same bits (a row's terms
      * are added in double in block order in either), so the choice is one of speed only; a
      * sealed worklist policy can keep the matrix-core regime off (matrix_allowed). */
     row_batch = matrix_allowed && routed_q8 && matrix_core_qtypes(&routed) &&
-                pairs >= (routed.gate_qtype == 12u ? 4ull : 6ull) * experts;
+                pairs >= (experts >= 32ull && (routed.gate_qtype == 12u || routed.gate_up_image) ? 3ull
+                          : routed.gate_qtype == 12u                                             ? 4ull
+                                                                                                 : 6ull) * experts;
     shared_row_batch = row_batch && has_shared && shared_q8 && matrix_core_qtypes(&shared);
     merged = !row_batch && has_shared && shared_q8 == routed_q8 && same_expert_shape(&routed, &shared);
     /* A Q8_0 shared expert (the format the reference's model file keeps it in, its default for every
@@ -773,6 +781,23 @@ sequence:
         backend->moe_graphs->refused = 1;
         graph_mode = GRAPH_EAGER;
     }
+    /* (the matrix-core wrappers make one launch or two) */
+    if (row_batch) {
+        matrix_launches[0] = yvex_hip_moe_up_rows_launches(&routed, AT(input_q8), (const uint64_t *)AT(expert_ids), pairs,
+                                                           topk, experts, (float *)AT(intermediate));
+        matrix_launches[1] = yvex_hip_moe_down_rows_launches(&routed, AT(intermediate_q8), (const uint64_t *)AT(expert_ids),
+                                                             pairs, experts, (float *)AT(pair_outputs));
+    }
+    if (shared_row_batch) {
+        matrix_launches[2] = yvex_hip_moe_up_rows_launches(&shared, AT(input_q8), NULL, row_count, 1ull, 1ull,
+                                                           (float *)AT(shared_intermediate));
+        matrix_launches[3] = yvex_hip_moe_down_rows_launches(&shared, AT(shared_intermediate_q8), NULL, row_count, 1ull,
+                                                             (float *)AT(shared_outputs));
+    }
+#define COUNTED(index)                                                  \
+    do {                                                                \
+        if (rc == YVEX_OK && graph_mode != GRAPH_REPLAY) launches += matrix_launches[index] - 1u; \
+    } while (0)
 #define LAUNCH(call, where)                                             \
     do {                                                                \
         if (rc == YVEX_OK && graph_mode != GRAPH_REPLAY) {              \
@@ -951,7 +976,7 @@ sequence:
             LAUNCH(yvex_hip_q8k_quantize((const float *)activations, row_count, hidden, hidden,
                                          (uint8_t *)AT(input_q8), (int *)status, stream), "rocm.moe.rows.q8");
     }
-    if (row_batch)
+    if (row_batch) {
         LAUNCH(yvex_hip_moe_up_rows(&routed, AT(input_q8), (const float *)AT(weights),
                                     (const uint64_t *)AT(order), (const uint64_t *)AT(expert_ids),
                                     (const uint64_t *)AT(bucket_offsets),
@@ -959,7 +984,8 @@ sequence:
                                     pairs, topk, experts, layer->activation_limit,
                                     (float *)AT(intermediate), (int *)status, stream),
                "rocm.moe.rows.up-matrix");
-    else
+        COUNTED(0);
+    } else
     LAUNCH(yvex_hip_moe_up(&routed, routed_q8 ? AT(input_q8) : (void *)(uintptr_t)activations, routed_q8,
                            (const float *)AT(weights), (const uint64_t *)AT(order),
                            (const uint64_t *)AT(expert_ids), (const uint64_t *)AT(bucket_offsets),
@@ -968,11 +994,12 @@ sequence:
                            (float *)AT(intermediate), merged ? &shared : NULL, merged ? row_count : 0ull,
                            merged ? (float *)AT(shared_intermediate) : NULL, (int *)status, stream),
            "rocm.moe.rows.up");
-    if (shared_row_batch)
+    if (shared_row_batch) {
         LAUNCH(yvex_hip_moe_up_rows(&shared, AT(input_q8), NULL, NULL, NULL, NULL, NULL, NULL, row_count,
                                     1ull, 1ull, layer->activation_limit, (float *)AT(shared_intermediate),
                                     (int *)status, stream), "rocm.moe.rows.shared-up-matrix");
-    else if (shared_dense) {
+        COUNTED(2);
+    } else if (shared_dense) {
         LAUNCH(yvex_hip_matvec_q8_0_pair(shared.gate, shared.up, layer->shared_intermediate_width, hidden,
                                          shared.gate_row_bytes, AT(input_q8), row_count,
                                          (float *)AT(shared_intermediate), (float *)AT(pair_outputs), (int *)status,
@@ -1007,13 +1034,14 @@ sequence:
                                      layer->shared_intermediate_width, layer->shared_intermediate_width,
                                      (uint8_t *)AT(shared_intermediate_q8), (int *)status, stream),
                "rocm.moe.rows.q8-shared-mid");
-    if (row_batch)
+    if (row_batch) {
         LAUNCH(yvex_hip_moe_down_rows(&routed, AT(intermediate_q8), (const uint64_t *)AT(order),
                                       (const uint64_t *)AT(expert_ids), (const uint64_t *)AT(bucket_offsets),
                                       (const uint64_t *)AT(bucket_populations), (const uint64_t *)AT(counts),
                                       pairs, experts, (float *)AT(pair_outputs), (int *)status, stream),
                "rocm.moe.rows.down-matrix");
-    else
+        COUNTED(1);
+    } else
     LAUNCH(yvex_hip_moe_down(&routed, routed_q8 ? AT(intermediate_q8) : AT(intermediate), routed_q8,
                              (const uint64_t *)AT(order), (const uint64_t *)AT(expert_ids),
                              (const uint64_t *)AT(bucket_offsets), (const uint64_t *)AT(bucket_populations),
@@ -1023,11 +1051,12 @@ sequence:
                              merged ? (shared_q8 ? AT(shared_intermediate_q8) : AT(shared_intermediate)) : NULL,
                              merged ? (float *)AT(shared_outputs) : NULL, (int *)status, stream),
            "rocm.moe.rows.down");
-    if (shared_row_batch)
+    if (shared_row_batch) {
         LAUNCH(yvex_hip_moe_down_rows(&shared, AT(shared_intermediate_q8), NULL, NULL, NULL, NULL, NULL,
                                       row_count, 1ull, (float *)AT(shared_outputs), (int *)status, stream),
                "rocm.moe.rows.shared-down-matrix");
-    else if (shared_dense)
+        COUNTED(3);
+    } else if (shared_dense)
         LAUNCH(yvex_hip_matvec(shared.down, shared.down_qtype, hidden, layer->shared_intermediate_width,
                                shared.down_row_bytes, AT(shared_intermediate_q8), 1, row_count,
                                layer->shared_intermediate_width, NULL, (float *)AT(shared_outputs), hidden, 1,
@@ -1097,7 +1126,7 @@ sequence:
     result->row_count = row_count;
     result->row_expert_pairs = pairs;
     result->kernel_launches = launches + status_launches;
-    result->tensor_core_launches = (row_batch ? 2ull : 0ull) + (shared_row_batch ? 2ull : 0ull);
+    result->tensor_core_launches = matrix_launches[0] + matrix_launches[1] + matrix_launches[2] + matrix_launches[3];
     result->shared_expert_operations = has_shared ? row_count : 0ull;
     result->grouped_expert_operations = pairs;
     result->active_weight_base_bytes = views[YVEX_MOE_WEIGHT_ROUTER].encoded_bytes +
@@ -1162,6 +1191,7 @@ sequence:
     }
 #undef DOWNLOAD
 #undef LAUNCH
+#undef COUNTED
 #undef AT
     if (rc != YVEX_OK) {
         memset(result, 0, sizeof(*result));
