@@ -188,10 +188,12 @@ def test_sweeps_agree_with_the_matrix_core_kernels(gpu, oracle, qtype, hidden, i
 
 # a pair, a remainder of the largest size the few-pair kernels take at the width and one more, 64-pair
 # tiles with and without such remainders; two, three and 32 superblocks a row, ragged row units
-@pytest.mark.parametrize("up,down,hidden,intermediate,tokens", [
-    ("IQ2_XXS", "Q2_K", 1024, 768, 16), ("IQ2_XXS", "IQ2_XXS", 7168, 512, 12), ("Q4_K", "Q4_K", 768, 1024, 16),
-    ("Q4_K", "Q2_K", 7168, 512, 16), ("IQ2_XXS", "Q4_K", 8192, 256, 8), ("IQ2_XXS", "Q2_K", 512, 2304, 16)])
-def test_few_pair_kernels_agree_with_the_generic_kernel(gpu, oracle, up, down, hidden, intermediate, tokens):
+@pytest.mark.parametrize("up,down,hidden,intermediate,tokens,image", [
+    ("IQ2_XXS", "Q2_K", 1024, 768, 16, True), ("IQ2_XXS", "IQ2_XXS", 7168, 512, 12, True),
+    ("IQ2_XXS", "IQ2_XXS", 7168, 512, 12, False), ("IQ2_XXS", "IQ2_XXS", 512, 1024, 16, False),
+    ("Q4_K", "Q4_K", 768, 1024, 16, False), ("Q4_K", "Q2_K", 7168, 512, 16, False),
+    ("IQ2_XXS", "Q4_K", 8192, 256, 8, True), ("IQ2_XXS", "Q2_K", 512, 2304, 16, True)])
+def test_few_pair_kernels_agree_with_the_generic_kernel(gpu, oracle, up, down, hidden, intermediate, tokens, image):
     """Buckets split between the two row-batch kernels by their remainders, and a matrix alone, hold
     what the generic grouped kernel (the CPU path's bits) publishes for the same pairs."""
     from yvex_amd import kernels as K
@@ -203,7 +205,7 @@ def test_few_pair_kernels_agree_with_the_generic_kernel(gpu, oracle, up, down, h
                ((uq, intermediate, hidden), (uq, intermediate, hidden), (dq, hidden, intermediate))]
     weights = K.expert_weights(*tensors, (uq, uq, dq), hidden, intermediate)
     rows_form = K.expert_weights(*tensors, (uq, uq, dq), hidden, intermediate)
-    images = [K.iq2_sweep_image(t) if q == oracle.IQ2_XXS else None for t, q in zip(tensors, (uq, uq, dq))]
+    images = [K.iq2_sweep_image(t) if image and q == oracle.IQ2_XXS else None for t, q in zip(tensors, (uq, uq, dq))]
     if images[0] is not None:
         rows_form.gate, rows_form.up, rows_form.gate_up_image = images[0].data_ptr(), images[1].data_ptr(), 1
         rows_form.gate_row_bytes = rows_form.up_row_bytes = hidden // 256 * 72
@@ -226,7 +228,7 @@ def test_few_pair_kernels_agree_with_the_generic_kernel(gpu, oracle, up, down, h
     K.moe_down(weights, mid_q8, True, wl, pairs, experts, out[0], status)
     K.moe_down_rows(rows_form, mid_q8, wl, pairs, experts, out[1], status)
     assert same_bits(out[0], out[1])
-    for alone in (tokens + 3, 257):                     # one matrix for all rows: either kernel
+    for alone in (tokens + 3, 257):                     # one matrix for all rows
         some = K.q8k_quantize(dev(g.normal(alone * hidden).reshape(alone, hidden), gpu), status)
         mid = [torch.zeros((alone, intermediate), device=gpu) for _ in range(2)]
         K.moe_up(weights, some, True, None, None, alone, 1, 1, 10.0, mid[0], status)

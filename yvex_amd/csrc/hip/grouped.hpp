@@ -162,13 +162,17 @@ int launch_iq2_sweep(const GroupedArgs &a, unsigned qtype, bool fused, bool imag
 int launch_q4k_rows_grouped(const GroupedProblem &problem, unsigned qtype, bool fused, uint64_t width,
                             uint64_t out_rows, unsigned left, double limit, int *status, hipStream_t stream);
 
-// The same problems where few pairs meet (rows16.hip): IQ2_XXS sweep images and Q4_K rows, fused
-// gate/up or plain; Q2_K rows, plain. The first: pairs of a full tile, 0 for a problem the kernels do
-// not serve. The second serves whole buckets (`behind` 0), or what a bucket holds behind whole tiles
-// of `behind` pairs where that fits one tile.
-unsigned rows16_tokens(const GroupedProblem &problem, unsigned qtype, bool fused, uint64_t width, uint64_t out_rows);
-int launch_rows16_grouped(const GroupedProblem &problem, unsigned qtype, bool fused, unsigned width,
-                          unsigned out_rows, unsigned behind, double limit, int *status, hipStream_t stream);
+// The same problems where few pairs meet (rows16.hip): IQ2_XXS (canonical bytes, or the sweep image) and
+// Q4_K rows, fused gate/up or plain; Q2_K rows, plain. The first: pairs of a full tile, 0 for a problem
+// the kernels do not serve. The second serves whole buckets (`behind` 0), or what a bucket holds
+// behind whole tiles of `behind` pairs where that fits one tile; a plain projection's sums are rounded
+// to bfloat16 where `round` says so.
+unsigned rows16_tokens(const GroupedProblem &problem, unsigned qtype, bool image, bool fused, uint64_t width,
+                       uint64_t out_rows);
+// Whether a matrix alone comes out at one round of the kernels' waves.
+bool rows16_one_round(const GroupedProblem &problem, unsigned qtype, bool fused, unsigned tokens, uint64_t out_rows);
+int launch_rows16_grouped(const GroupedProblem &problem, unsigned qtype, bool image, bool fused, unsigned width,
+                          unsigned out_rows, unsigned behind, bool round, double limit, int *status, hipStream_t stream);
 
 static inline bool same_shape(const yvex_hip_expert_weights *a, const yvex_hip_expert_weights *b)
 {

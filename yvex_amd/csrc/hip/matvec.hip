@@ -1076,10 +1076,14 @@ extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint6
     // IQ2_XXS rows against a batch of Q8_K input rows: the int8 matrix-core kernel of the
     // row-batch expert path, as one bucket that holds every input row (the reference turns its
     // tensor-core kernels on from 16 input rows, src/backend/cuda/private.h:461-464; measured
-    // here the sweep below stays faster up to 31 rows: 17 us against 22 us for 7168 x 2048 at 16). Same exact
+    // here against the sweep below, whose time grows with the products: 4096 x 4096 by 16 rows 20.5 us
+    // there and 22.4 here, by 24 28 and 22; 7168 x 2048 by 8 11.7 and 14.4, by 16 19.7 and 14.6;
+    // 2048 x 7168 by 24 25.6 and 32.4). Same exact
     // int32 superblock sums and the same float terms as the sweep below, added in double in
     // superblock order there and here: the same bits.
-    if (qtype == QT_IQ2_XXS && input_q8 && input_rows >= 32ull && !additive &&
+    const bool iq2_batch = input_rows >= 32ull || (input_rows >= 8ull && row_width >= 512ull && row_count <= 32768ull &&
+                                                   input_rows * row_count >= 73728ull);
+    if (qtype == QT_IQ2_XXS && input_q8 && iq2_batch && !additive &&
         out_stride == row_count && row_count % 4ull == 0ull && !((uintptr_t)encoded & 3u) &&
         !(row_bytes & 3ull) && row_width / 32ull <= 64ull * 4ull && !((uintptr_t)out & 15u))
         return launch_iq2_rows_dense(encoded, row_count, row_width, row_bytes, input, input_rows, out,

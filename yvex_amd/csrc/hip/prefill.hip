@@ -823,13 +823,14 @@ static int launch_mfma(const MfmaArgs &a, hipStream_t stream)
                    : launch_mfma_variant<FUSED_UP, false>(a, stream);
 }
 
-// Expert matrices against the buckets of a worklist. Where the few-pair kernels serve the rows
-// (IQ2_XXS sweep images, Q4_K and Q2_K rows), they take what a bucket holds behind its whole
-// 64-pair tiles if that fits one of their tiles (12 pairs at width 7168, 16 up to about 5000): such a tile
+// Expert matrices against the buckets of a worklist. The few-pair kernels (rows16.hip) take what a
+// bucket holds behind its whole 64-pair tiles if that fits one of their tiles (12 pairs at width 7168, 16 up to about 5000): such a tile
 // takes them 1.4 us of the whole device for the 2 x 2048 x 4096 IQ2_XXS rows of an expert, and the 64-pair
 // kernels, which pay for 32 token columns, 2.3 us; with two of theirs (from 17 pairs on, 2.8 us) it
-// is the other way round. A matrix that is alone (no worklist) is theirs up to 256 rows, where the
-// other kernels have fewer items than there are compute units.
+// is the other way round. A matrix that is alone (no worklist) is theirs where they come out at one round of
+// their waves: 16 superblocks take 22 to 31 us then, and 45 us as 64-pair items, which are fewer than the
+// compute units up to 1024 rows (4096 x 4096 IQ2_XXS by 128 rows 44 -> 24 us, 2048 x 7168 69 -> 35; 7168 x
+// 7168 by 256 rows, two rounds, 102 us against 70).
 struct RowsPlan {
     unsigned few;            // pairs of a full tile of the few-pair kernel, 0: it does not run
     bool many;               // the 64-pair kernel runs
@@ -837,9 +838,9 @@ struct RowsPlan {
 
 static RowsPlan plan_rows(const GroupedProblem &pr, unsigned qtype, bool fused, int image, uint64_t width, uint64_t out_rows)
 {
-    constexpr unsigned kAloneRows = 256u;
-    const bool alone = pr.expert_ids == nullptr, readable = qtype != QT_IQ2_XXS || image;
-    const unsigned few = readable && !(alone && pr.pairs > kAloneRows) ? rows16_tokens(pr, qtype, fused, width, out_rows) : 0u;
+    const bool alone = pr.expert_ids == nullptr;
+    unsigned few = rows16_tokens(pr, qtype, image != 0, fused, width, out_rows);
+    if (alone && few && !rows16_one_round(pr, qtype, fused, few, out_rows)) few = 0u;
     return {few, !few || (!alone && pr.pairs > few)};
 }
 
@@ -854,8 +855,8 @@ static int launch_rows(MfmaArgs &a, unsigned qtype, hipStream_t stream)
             : launch_q4k_rows_grouped(a.pr, qtype, FUSED_UP, a.width, a.out_rows, plan.few, a.limit, a.status, stream);
         if (rc || !plan.few) return rc;
     }
-    return launch_rows16_grouped(a.pr, qtype, FUSED_UP, a.width, a.out_rows, a.pr.expert_ids ? kTileTokens : 0u, a.limit,
-                                 a.status, stream);
+    return launch_rows16_grouped(a.pr, qtype, a.image != 0, FUSED_UP, a.width, a.out_rows, a.pr.expert_ids ? kTileTokens : 0u,
+                                 !a.plain_output, a.limit, a.status, stream);
 }
 
 // A plain projection through the row-batch kernel: every input row in one bucket of expert 0.
@@ -881,7 +882,7 @@ int launch_iq2_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t r
     a.limit = 1.0;
     a.status = status;
     a.plain_output = round_bf16 ? 0 : 1;
-    return launch_mfma<false>(a, stream);
+    return launch_rows<false>(a, QT_IQ2_XXS, stream);
 }
 
 }  // namespace yvex

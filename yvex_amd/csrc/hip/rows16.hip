@@ -1,5 +1,5 @@
 // Expert projections of row batches whose buckets hold few pairs, on the int8 matrix cores of
-// gfx950: IQ2_XXS rows as the sweep image, Q4_K rows and the Q2_K rows of a down projection
+// gfx950: IQ2_XXS rows (canonical bytes or the sweep image), Q4_K rows and the Q2_K rows of a down projection
 // (src/backend/cuda/tensorcore.cu:378-702 is the reference's counterpart, for its own formats).
 //
 // With a handful of pairs to an expert the cost of the row-batch kernels (prefill.hip,
@@ -42,6 +42,7 @@ constexpr unsigned kSlots16 = 16u;                        // token columns of a 
 constexpr unsigned kMaxBlocks16 = 32u;                    // superblocks of a row
 constexpr unsigned kBatchTiles = 8u;                      // tiles in LDS at a time
 constexpr unsigned kLds16 = 160u * 1024u;
+constexpr unsigned kIq2Image = 0x100u;                    // IQ2_XXS rows as the sweep image (no format number)
 
 // LDS map (byte addresses; the dynamic block starts at LDS address 0). The IQ2_XXS tables come
 // first: entry e owns the 256 bytes at 256 e, sixteen replicas of the level codes of codebook
@@ -57,7 +58,7 @@ constexpr unsigned kLds16 = 160u * 1024u;
 // reads. The payload stands piece-major, [superblock][piece][token slot] with a multiple of four
 // slots: 4.1 cycles instead of the 8.0 of token rows with XOR-ed piece positions.
 template <unsigned QT> struct Map16 {
-    static constexpr bool kIq2 = QT == QT_IQ2_XXS;
+    static constexpr bool kIq2 = QT == QT_IQ2_XXS || QT == kIq2Image;
     static constexpr unsigned kWaves = kIq2 ? 12u : 8u;
     static constexpr unsigned kThreads = 64u * kWaves;
     static constexpr unsigned kLimbs = 65536u;
@@ -80,6 +81,7 @@ struct Rows16Args {
     unsigned blocks;         // superblocks per weight row
     unsigned out_rows;       // weight rows per expert
     unsigned tokens;         // of a full tile
+    bool round;              // a plain projection's sums are rounded to bfloat16
     unsigned behind;         // what is served of a bucket: all of it (0), or its pairs behind whole tiles of
                              // this many, where they fit one tile here
     double limit;
@@ -98,14 +100,31 @@ struct Tile16 {
 // ---- formats: a lane's bytes of one row's superblock ----
 template <unsigned QT> struct Record16;
 
-template <> struct Record16<QT_IQ2_XXS> {
+template <> struct Record16<kIq2Image> {
     static constexpr unsigned kBytes = 72u;
     unsigned head;           // fp16 scale | the four group scales of the lane's half << 16
     v4i body;                // groups 2 q and 2 q + 1: codebook bytes, sign bytes
-    __device__ __forceinline__ void load(const unsigned char *base, unsigned row, const Lane16 &l)
+    __device__ __forceinline__ void load(const unsigned char *base, unsigned row, bool, const Lane16 &l)
     {
         head = *reinterpret_cast<const unsigned *>(base + (row + 36u * (l.q >> 1)));
         body = *reinterpret_cast<const v4i_dword *>(base + (row + (36u * (l.q >> 1) + 16u * (l.q & 1u) + 4u)));
+    }
+};
+
+// Canonical superblocks are 66 bytes and rows whole dwords, so the lane's sixteen bytes start two bytes
+// into a dword in even superblocks and on one in odd ones: a window of five dwords, of which the odd
+// superblocks use four (their fifth, which may lie behind the matrix, repeats the fourth).
+template <> struct Record16<QT_IQ2_XXS> {
+    static constexpr unsigned kBytes = 66u;
+    v4i window;
+    unsigned fifth;
+    unsigned short scale;
+    __device__ __forceinline__ void load(const unsigned char *base, unsigned row, bool odd, const Lane16 &l)
+    {
+        const unsigned at = row + (odd ? 2u : 0u) + 16u * l.q;
+        window = *reinterpret_cast<const v4i_dword *>(base + at);
+        fifth = *reinterpret_cast<const unsigned *>(base + (at + (odd ? 12u : 16u)));
+        scale = *reinterpret_cast<const unsigned short *>(base + row);
     }
 };
 
@@ -113,7 +132,7 @@ template <> struct Record16<QT_Q4_K> {
     static constexpr unsigned kBytes = 144u;
     v4i head;                // d | dmin << 16, the 12 scale bytes
     v4i codes[2];            // the 32 bytes of sub-blocks 2 q (low nibbles) and 2 q + 1
-    __device__ __forceinline__ void load(const unsigned char *base, unsigned row, const Lane16 &l)
+    __device__ __forceinline__ void load(const unsigned char *base, unsigned row, bool, const Lane16 &l)
     {
         head = *reinterpret_cast<const v4i_dword *>(base + row);
         codes[0] = *reinterpret_cast<const v4i_dword *>(base + (row + (32u * l.q + 16u)));
@@ -127,7 +146,7 @@ template <> struct Record16<QT_Q2_K> {
     v4i scales;              // (scale | minimum << 4) of the sixteen sub-blocks
     v4i codes;               // bytes 16 (q % 2) .. + 15 of code half q / 2
     unsigned dd;             // d | dmin << 16
-    __device__ __forceinline__ void load(const unsigned char *base, unsigned row, const Lane16 &l)
+    __device__ __forceinline__ void load(const unsigned char *base, unsigned row, bool, const Lane16 &l)
     {
         scales = *reinterpret_cast<const v4i_dword *>(base + row);
         codes = *reinterpret_cast<const v4i_dword *>(base + (row + (16u * l.q + 16u)));
@@ -183,9 +202,24 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
     // ---- this workgroup's piece of the tiles' row units ----
     constexpr unsigned kUnitRows = FUSED ? 16u : 32u;
     const unsigned units = (a.out_rows + kUnitRows - 1u) / kUnitRows;
-    const unsigned long long total = (unsigned long long)uniform(lds_read_u32(M::kStarts + 4u * buckets)) * units;
-    unsigned long long at = total * blockIdx.x / gridDim.x;
-    const unsigned long long end = total * (blockIdx.x + 1u) / gridDim.x;
+    const unsigned all_tiles = uniform(lds_read_u32(M::kStarts + 4u * buckets));
+    if (!all_tiles) return;
+    // A short piece that runs into a second tile takes twice its time where the two do not fit the LDS
+    // together. So where a tile has several workgroups to itself and they come out at two rounds of
+    // their waves or less, pieces end with their tiles (4096 x 4096 by 48 rows, three tiles: 39 -> 23 us);
+    // longer ones are cut to equal lengths across tiles.
+    const unsigned shares = gridDim.x / all_tiles;              // workgroups a tile
+    unsigned long long at, end;
+    if (shares && (units + shares - 1u) / shares <= 2u * M::kWaves) {
+        const unsigned tile = blockIdx.x / shares, share = blockIdx.x % shares;
+        if (tile >= all_tiles) return;
+        at = (unsigned long long)tile * units + (unsigned long long)units * share / shares;
+        end = (unsigned long long)tile * units + (unsigned long long)units * (share + 1u) / shares;
+    } else {
+        const unsigned long long total = (unsigned long long)all_tiles * units;
+        at = total * blockIdx.x / gridDim.x;
+        end = total * (blockIdx.x + 1u) / gridDim.x;
+    }
     if (at == end) return;
     if constexpr (kIq2) {
         for (unsigned index = tid; index < 256u * 16u; index += M::kThreads)
@@ -360,7 +394,8 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
             const unsigned block = (past ? sb - a.blocks : sb) * Record16<QT>::kBytes;
 #pragma unroll
             for (unsigned u = 0; u < 2u; ++u)
-                into[u].load(past ? ahead.base[u] : here.base[u], (past ? ahead.row[u] : here.row[u]) + block, l);
+                into[u].load(past ? ahead.base[u] : here.base[u], (past ? ahead.row[u] : here.row[u]) + block,
+                             ((past ? sb - a.blocks : sb) & 1u) != 0u, l);
         };
         request(rec[0], 0u);
         request(rec[1], 1u);
@@ -385,25 +420,45 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
             v4i lo[2] = {zero, zero}, hi[2] = {zero, zero};
             if constexpr (kIq2) {
                 // lanes of odd quarters look signs up first
-                const bool odd = (l.q & 1u) != 0u;
+                const bool odd = QT == kIq2Image && (l.q & 1u) != 0u;
                 const unsigned first_lane = l.r * 8u + (odd ? 128u : 0u), second_lane = first_lane ^ 128u;
                 const unsigned lut_lane = M::kLimbs + l.r * 16u;
                 const unsigned nibble = 8u + 8u * (l.q & 1u);
-                unsigned first[2][2], second[2][2];              // [tile][group]
+                unsigned first[2][2], second[2][2];              // [tile][group]: codebook and sign words
+                unsigned scale16[2];
 #pragma unroll
-                for (unsigned u = 0; u < 2u; ++u)
+                for (unsigned u = 0; u < 2u; ++u) {
+                    if constexpr (QT == kIq2Image) {
+                        scale16[u] = w[u].head & 0xffffu;
 #pragma unroll
-                    for (unsigned g = 0; g < 2u; ++g) {
-                        const unsigned grids = (unsigned)w[u].body[2u * g], aux = (unsigned)w[u].body[2u * g + 1u];
-                        first[u][g] = odd ? aux : grids;
-                        second[u][g] = odd ? grids : aux;
+                        for (unsigned g = 0; g < 2u; ++g) {
+                            const unsigned grids = (unsigned)w[u].body[2u * g], aux = (unsigned)w[u].body[2u * g + 1u];
+                            first[u][g] = odd ? aux : grids;
+                            second[u][g] = odd ? grids : aux;
+                        }
+                    } else {
+                        scale16[u] = w[u].scale;
+                        const unsigned shift = sb & 1u ? 0u : 2u;
+                        const unsigned d[5] = {(unsigned)w[u].window[0], (unsigned)w[u].window[1], (unsigned)w[u].window[2],
+                                               (unsigned)w[u].window[3], w[u].fifth};
+#pragma unroll
+                        for (unsigned g = 0; g < 2u; ++g) {
+                            first[u][g] = __builtin_amdgcn_alignbyte(d[2u * g + 1u], d[2u * g], shift);
+                            second[u][g] = __builtin_amdgcn_alignbyte(d[2u * g + 2u], d[2u * g + 1u], shift);
+                        }
                     }
+                }
 #pragma unroll
                 for (unsigned u = 0; u < 2u; ++u)
-                    lds_write_u32(scratch + 64u * u + 4u * l.r, __float_as_uint(0.125f * f16_bits_to_float(w[u].head & 0xffffu)));
+                    lds_write_u32(scratch + 64u * u + 4u * l.r, __float_as_uint(0.125f * f16_bits_to_float(scale16[u])));
                 uint2 codes[2][2][2], signs[2][2][2];            // [chunk & 1][tile][subgroup]
                 uint4 limbs[2][2];                               // [group & 1][tile]
                 v4i frag[2];
+                // the scale of a group in bits 8-11
+                auto limb_field = [&](unsigned u, unsigned g) -> unsigned {
+                    if constexpr (QT == kIq2Image) return w[u].head >> (nibble + 4u * g);
+                    else return second[u][g] >> 20;
+                };
                 auto lookup = [&](unsigned m) {
                     frag[m & 1u] = lds_read_v4i(frag_at + m * frag_step);
 #pragma unroll
@@ -413,12 +468,14 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
                             const unsigned pick = 0x0c0c0400u + ((2u * (m & 1u) + i) << 8);
                             codes[m & 1u][u][i] =
                                 lds_read_uint2(__builtin_amdgcn_perm(first[u][m >> 1], first_lane, pick));
-                            signs[m & 1u][u][i] =
-                                lds_read_uint2(__builtin_amdgcn_perm(second[u][m >> 1], second_lane, pick));
+                            // (the image's sign fields have bytes of their own, the canonical ones seven bits each)
+                            const unsigned j = 2u * (m & 1u) + i, word = second[u][m >> 1];
+                            signs[m & 1u][u][i] = lds_read_uint2(
+                                QT == kIq2Image ? __builtin_amdgcn_perm(word, second_lane, pick)
+                                                : ((j == 0u ? word << 8 : j == 1u ? word << 1 : word >> (7u * j - 8u)) & 0x7f00u) | second_lane);
                         }
                         if ((m & 1u) == 0u)
-                            limbs[(m >> 1) & 1u][u] =
-                                lds_read_uint4(((w[u].head >> (nibble + 4u * (m >> 1))) & 0xf00u) | lut_lane);
+                            limbs[(m >> 1) & 1u][u] = lds_read_uint4((limb_field(u, m >> 1) & 0xf00u) | lut_lane);
                     }
                 };
                 lookup(0u);
@@ -562,7 +619,7 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
                     } else {
                         value[i] = (float)acc[u][i];
                         good &= finite_f32(value[i]);
-                        value[i] = bf16_round_number(value[i]);       // (a NaN has just been noted)
+                        if (a.round) value[i] = bf16_round_number(value[i]);      // (a NaN has just been noted)
                     }
                     good &= finite_f32(value[i]);
                 }
@@ -614,13 +671,14 @@ template <unsigned QT> unsigned tile_tokens16(unsigned blocks)
 
 }  // namespace
 
-unsigned rows16_tokens(const GroupedProblem &problem, unsigned qtype, bool fused, uint64_t width, uint64_t out_rows)
+unsigned rows16_tokens(const GroupedProblem &problem, unsigned qtype, bool image, bool fused, uint64_t width,
+                       uint64_t out_rows)
 {
-    const uint64_t blocks = width / 256u, superblock = qtype == QT_IQ2_XXS ? 72u : qtype == QT_Q4_K ? 144u : 84u;
+    const uint64_t blocks = width / 256u, superblock = qtype == QT_IQ2_XXS ? (image ? 72u : 66u) : qtype == QT_Q4_K ? 144u : 84u;
     // superblocks are requested two ahead, across one unit's end
     if (width % 256u || blocks < 2u || blocks > kMaxBlocks16 || (qtype == QT_Q2_K && fused)) return 0u;
     // a lane addresses its rows with 32-bit offsets inside an expert and stores four rows at a time
-    if (!out_rows || out_rows % 4u || problem.row_bytes != blocks * superblock ||
+    if (!out_rows || out_rows % 4u || problem.row_bytes != blocks * superblock || (problem.row_bytes & 3u) ||
         (fused && problem.up_row_bytes != problem.row_bytes) || out_rows * problem.row_bytes > 0xffffffffull)
         return 0u;
     if ((((uintptr_t)problem.gate | (uintptr_t)problem.up | (uintptr_t)problem.activations | problem.expert_bytes |
@@ -632,15 +690,24 @@ unsigned rows16_tokens(const GroupedProblem &problem, unsigned qtype, bool fused
          : qtype == QT_Q2_K    ? tile_tokens16<QT_Q2_K>((unsigned)blocks) : 0u;
 }
 
-int launch_rows16_grouped(const GroupedProblem &problem, unsigned qtype, bool fused, unsigned width,
-                          unsigned out_rows, unsigned behind, double limit, int *status, hipStream_t stream)
+bool rows16_one_round(const GroupedProblem &problem, unsigned qtype, bool fused, unsigned tokens, uint64_t out_rows)
 {
-    const Rows16Args a{problem, width / 256u, out_rows, rows16_tokens(problem, qtype, fused, width, out_rows), behind,
-                       limit, status};
+    const uint64_t units = (out_rows + (fused ? 15u : 31u)) / (fused ? 16u : 32u);
+    const unsigned waves = qtype == QT_IQ2_XXS ? Map16<QT_IQ2_XXS>::kWaves : Map16<QT_Q4_K>::kWaves;
+    return (problem.pairs + (uint64_t)tokens - 1u) / tokens * units <= (uint64_t)waves * compute_units();
+}
+
+int launch_rows16_grouped(const GroupedProblem &problem, unsigned qtype, bool image, bool fused, unsigned width,
+                          unsigned out_rows, unsigned behind, bool round, double limit, int *status, hipStream_t stream)
+{
+    const Rows16Args a{problem, width / 256u, out_rows, rows16_tokens(problem, qtype, image, fused, width, out_rows), round,
+                       behind, limit, status};
     if (!a.tokens) return ST_UNSUPPORTED;
     if (qtype == QT_Q2_K) return launch_rows16<QT_Q2_K, false>(a, stream);
     if (qtype == QT_Q4_K)
         return fused ? launch_rows16<QT_Q4_K, true>(a, stream) : launch_rows16<QT_Q4_K, false>(a, stream);
+    if (image)
+        return fused ? launch_rows16<kIq2Image, true>(a, stream) : launch_rows16<kIq2Image, false>(a, stream);
     return fused ? launch_rows16<QT_IQ2_XXS, true>(a, stream) : launch_rows16<QT_IQ2_XXS, false>(a, stream);
 }
 

@@ -681,9 +681,8 @@ static int moe_execute_rows(yvex_rocm_backend *backend, const yvex_moe_layer_job
                             &views[YVEX_MOE_WEIGHT_SHARED_DOWN], addresses[3], addresses[4], addresses[5],
                             hidden, layer->shared_intermediate_width, shared_image);
     /* Row batches whose buckets average three pairs or more go to the int8 matrix-core kernels
-     * (IQ2_XXS or Q4_K weights, Q8_K activations; IQ2_XXS as canonical bytes, which the few-pair kernels
-     * among them do not read, from six pairs on); below that the decode sweeps, which read an expert's
-     * bytes once per four pairs, are faster. Gate/up and down launches of 256 experts, uniform
+     * (IQ2_XXS or Q4_K weights, Q8_K activations); below that the decode sweeps, which read an
+     * expert's bytes once per four pairs, are faster. Gate/up and down launches of 256 experts, uniform
      * routing: 7168 wide, top-8, 96 rows IQ2_XXS 824 us as sweeps and 858 as tiles, 112 rows 939 and 871;
      * Q4_K 96 rows 1334 and 1306; 4096 wide, top-6, Q2_K down, 128 rows 485 and 527, 160 rows 568 and 543.
      * A skewed routing is a little better off as tiles (96 rows at 7168, a Zipf exponent of 1.1: 430 us
@@ -695,9 +694,7 @@ static int moe_execute_rows(yvex_rocm_backend *backend, const yvex_moe_layer_job
      * are added in double in block order in either), so the choice is one of speed only; a
      * sealed worklist policy can keep the matrix-core regime off (matrix_allowed). */
     row_batch = matrix_allowed && routed_q8 && matrix_core_qtypes(&routed) &&
-                pairs >= (experts >= 32ull && (routed.gate_qtype == 12u || routed.gate_up_image) ? 3ull
-                          : routed.gate_qtype == 12u                                             ? 4ull
-                                                                                                 : 6ull) * experts;
+                pairs >= (experts >= 32ull ? 3ull : routed.gate_qtype == 12u ? 4ull : 6ull) * experts;
     shared_row_batch = row_batch && has_shared && shared_q8 && matrix_core_qtypes(&shared);
     merged = !row_batch && has_shared && shared_q8 == routed_q8 && same_expert_shape(&routed, &shared);
     /* A Q8_0 shared expert (the format the reference's model file keeps it in, its default for every
