@@ -702,7 +702,12 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
         members[c] = lds_read_u32(kClassCountBase + 4u * c);
         items += (unsigned long long)members[c] * row_tiles;
     }
-    if (blockIdx.x >= items) return;
+    // Neighbouring items read the same weights (a bucket's token tiles of one row tile), so they go to
+    // workgroups of one XCD (workgroups are dealt to the eight XCDs in turn), whose L2 then fetches them
+    // once: 2048 rows of 7168 with uneven experts, gate/up 1506 -> 1480 us; even experts, whose
+    // buckets are single tiles, are indifferent.
+    const unsigned start = gridDim.x % 8u ? blockIdx.x : (blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
+    if (start >= items) return;
     mfma_tables_fill();
     __syncthreads();
 
@@ -786,7 +791,7 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
         out.it.tokens = left < kTileTokens ? (unsigned)left : kTileTokens;
     };
 
-    unsigned long long item = blockIdx.x;
+    unsigned long long item = start;
     MfmaNextItem current;
     resolve_item(request_item(item), current);
     bool prefetched = false;
