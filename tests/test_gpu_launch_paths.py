@@ -235,3 +235,18 @@ def test_few_pair_kernels_agree_with_the_generic_kernel(gpu, oracle, up, down, h
         K.moe_up_rows(rows_form, some, None, None, alone, 1, 1, 10.0, mid[1], status)
         assert same_bits(mid[0], mid[1])
     assert int(status.item()) == 0
+
+
+# 16, 32 and 64 input rows a workgroup of the staged kernel (on 256 compute units), ragged on both sides,
+# one chunk and several
+@pytest.mark.parametrize("rows,width,inputs", [(250, 384, 345), (256, 128, 850), (249, 256, 2045)])
+def test_router_blocks_of_every_size_are_sums_in_double(gpu, rows, width, inputs):
+    from yvex_amd import kernels as K
+    gen = torch.Generator().manual_seed(rows)
+    w, x = torch.randn((rows, width), generator=gen), torch.randn((inputs, width), generator=gen)
+    status = K.new_status(gpu)
+    got = K.matvec(w.to(gpu).view(torch.uint8), 0, rows, width, x.to(gpu), status=status).cpu()
+    want = (x.double() @ w.double().t()).float()
+    # sums in double in another order differ by under 1e-13 of the terms: the float is the same or, next
+    # to a rounding boundary, its neighbour
+    assert torch.all((got - want).abs() <= want.abs() * 2.0 ** -23 + 1e-12) and int(status.item()) == 0

@@ -665,43 +665,51 @@ __global__ __launch_bounds__(WAVES * 64) void matvec_f32_tile16_kernel(MatvecArg
     }
 }
 
-// The same product for a batch of 256 input rows or more (the router projection of a prefill
+// The same product for a batch of several hundred input rows or more (the router projection of a prefill
 // batch): with one 16 x 16 tile a workgroup every wave loads its own operands, four bytes for
-// every matrix-core flop, and the launch runs at what the caches deliver (33 TFLOP/s where the
-// instruction alone sustains 75). Here a workgroup of eight waves (two a SIMD, so that one
-// multiplies while the other waits) owns 32 weight rows x 64 input rows and stages 128 columns
-// of both in LDS (a 528-byte pitch keeps the sixteen rows that one 16-byte read phase touches
-// on sixteen different bank groups), the next chunk's loads in flight while the current one is
-// multiplied; wave w multiplies the 16-row half w % 2 of the weight block by input rows
-// 16 (w / 2) .. + 15. Sums and rounding as above.
+// every matrix-core flop, and the launch runs at what the caches deliver (27 TFLOP/s where the
+// instruction alone sustains 75). Here a workgroup of sixteen waves, four a SIMD, owns 32 weight rows x
+// INPUTS input rows and stages 128 columns of both in LDS (a 528-byte pitch keeps the sixteen rows that one
+// 16-byte read phase touches on sixteen different bank groups), the next chunk's loads in flight while the
+// current one is multiplied. Two 16-row halves of the weights times INPUTS / 16 blocks of input rows are the
+// tiles; the waves of a tile share a chunk's eight steps out among themselves and their sums are added
+// at the end, in wave order. (One wave a tile, two a SIMD, left the matrix pipe idle half the time:
+// 256 x 7168 by 2048 rows 205 us, 165 now; the matrix instructions alone are 104.)
 constexpr unsigned kF32BlockColumns = 128u, kF32BlockPitch = kF32BlockColumns * 4u + 16u;
-constexpr unsigned kF32BlockWeightRows = 32u, kF32BlockInputRows = 64u;
-constexpr unsigned kF32BlockLdsBytes = 2u * (kF32BlockWeightRows + kF32BlockInputRows) * kF32BlockPitch;
+constexpr unsigned kF32BlockWeightRows = 32u, kF32BlockWaves = 16u;
+constexpr unsigned f32_block_lds(unsigned inputs) { return 2u * (kF32BlockWeightRows + inputs) * kF32BlockPitch; }
 
-template <unsigned QT>
-__global__ __launch_bounds__(512) void matvec_f32_block_kernel(MatvecArgs a)
+template <unsigned QT, unsigned INPUTS>
+__global__ __launch_bounds__(64 * kF32BlockWaves) void matvec_f32_block_kernel(MatvecArgs a)
 {
     typedef double v4d __attribute__((ext_vector_type(4)));
     typedef float v4f __attribute__((ext_vector_type(4)));
-    constexpr unsigned kRows = kF32BlockWeightRows + kF32BlockInputRows;
+    constexpr unsigned kRows = kF32BlockWeightRows + INPUTS;
     constexpr unsigned kPieces = kF32BlockColumns / 4u;                   // 16-byte pieces a row
-    constexpr unsigned kHeld = kRows * kPieces / 512u;
+    constexpr unsigned kThreads = 64u * kF32BlockWaves;
+    constexpr unsigned kHeld = (kRows * kPieces + kThreads - 1u) / kThreads;
+    constexpr unsigned kTiles = INPUTS / 8u, kSplits = kF32BlockWaves / kTiles;      // waves a tile
+    constexpr unsigned kSteps = kF32BlockColumns / 16u / kSplits;         // of a chunk, a wave
+    static_assert(kSteps * kSplits * 16u == kF32BlockColumns && kRows * kPieces % 512u == 0u, "whole shares");
+    static_assert((kSplits - 1u) * kTiles * 4u * 64u * 8u <= f32_block_lds(INPUTS), "the partial sums fit the stages");
     extern __shared__ __align__(16) unsigned char staged[];               // [2][kRows * kF32BlockPitch]
     const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const unsigned i16 = lane & 15u, q = lane >> 4;
-    // staging: piece p = threadIdx.x + 512 j of the chunk is columns 4 (p % 32) .. + 3 of staged
-    // row p / 32 (weight rows first, then input rows); 32 lanes read one row's 512 bytes
-    const unsigned char *source[kHeld];       // (weight rows: F32, F16 or BF16 values; input rows: F32)
+    // staging: piece p = threadIdx.x + 1024 j of the chunk is columns 4 (p % 32) .. + 3 of staged
+    // row p / 32 (weight rows first, then input rows); 32 lanes read one row's 512 bytes. Threads whose
+    // last piece lies behind the rows repeat the last row's.
+    const unsigned char *source[kHeld];       // (weight rows: F32, F16, BF16 or Q8_0 values; input rows: F32)
     unsigned target[kHeld];
 #pragma unroll
     for (unsigned j = 0; j < kHeld; ++j) {
-        const unsigned p = threadIdx.x + 512u * j, row = p / kPieces, piece = p % kPieces;
+        const unsigned p = threadIdx.x + kThreads * j, piece = p % kPieces;
+        const unsigned row = p / kPieces < kRows ? p / kPieces : kRows - 1u;
         if (row < kF32BlockWeightRows) {
             unsigned long long wrow = (unsigned long long)blockIdx.x * kF32BlockWeightRows + row;
             if (wrow >= a.row_count) wrow = a.row_count - 1ull;          // a ragged edge repeats the last row
             source[j] = a.encoded + wrow * a.row_bytes;       // (a weight row: columns from 4 * piece on)
         } else {
-            unsigned long long in = (unsigned long long)blockIdx.y * kF32BlockInputRows + (row - kF32BlockWeightRows);
+            unsigned long long in = (unsigned long long)blockIdx.y * INPUTS + (row - kF32BlockWeightRows);
             if (in >= a.input_rows) in = a.input_rows - 1ull;
             source[j] = (const unsigned char *)((const float *)a.input + in * a.input_stride + 4u * piece);
         }
@@ -710,28 +718,31 @@ __global__ __launch_bounds__(512) void matvec_f32_block_kernel(MatvecArgs a)
     const unsigned chunks = (unsigned)(a.row_width / kF32BlockColumns);
     v4f held[kHeld];
     unsigned bad = 0u;
-    // piece j of this thread is a piece of a weight row for the first two j, of an input row after
+    // piece 0 of every thread is a piece of a weight row, the others are of input rows
+    static_assert(kF32BlockWeightRows * kPieces == kThreads, "the weight rows are the threads' first pieces");
     auto fetch = [&](unsigned j, unsigned chunk) -> v4f {
-        if (512u * (j + 1u) <= kF32BlockWeightRows * kPieces) {
-            const unsigned piece = (threadIdx.x + 512u * j) % kPieces;
-            const float4 w = scalar_weights4<QT>(source[j], (unsigned long long)chunk * kF32BlockColumns + 4u * piece);
+        if (j == 0u) {
+            const float4 w = scalar_weights4<QT>(source[0], (unsigned long long)chunk * kF32BlockColumns + 4u * (threadIdx.x % kPieces));
             return v4f{w.x, w.y, w.z, w.w};
         }
         return *reinterpret_cast<const v4f *>(source[j] + (unsigned long long)chunk * kF32BlockColumns * 4ull);
     };
+    auto stage = [&](unsigned char *to) {
+        // (a non-finite weight is reported by the thread that stages it, once, not by the sixteen
+        // lanes that multiply it)
+        bad |= (unsigned)!finite_f32(held[0][0]) | (unsigned)!finite_f32(held[0][1]) |
+               (unsigned)!finite_f32(held[0][2]) | (unsigned)!finite_f32(held[0][3]);
+#pragma unroll
+        for (unsigned j = 0; j < kHeld; ++j) *reinterpret_cast<v4f *>(to + target[j]) = held[j];
+    };
 #pragma unroll
     for (unsigned j = 0; j < kHeld; ++j) held[j] = fetch(j, 0u);
-#pragma unroll
-    for (unsigned j = 0; j < kHeld; ++j) {
-        if (512u * (j + 1u) <= kF32BlockWeightRows * kPieces)
-            bad |= (unsigned)!finite_f32(held[j][0]) | (unsigned)!finite_f32(held[j][1]) |
-                   (unsigned)!finite_f32(held[j][2]) | (unsigned)!finite_f32(held[j][3]);
-        *reinterpret_cast<v4f *>(&staged[target[j]]) = held[j];
-    }
+    stage(staged);
     __syncthreads();
     v4d acc = {0.0, 0.0, 0.0, 0.0};
-    const unsigned weight_at = (16u * (wave & 1u) + i16) * kF32BlockPitch + 16u * q;
-    const unsigned input_at = (kF32BlockWeightRows + 16u * (wave >> 1) + i16) * kF32BlockPitch + 16u * q;
+    const unsigned tile = wave % kTiles, split = wave / kTiles;
+    const unsigned weight_at = (16u * (tile & 1u) + i16) * kF32BlockPitch + 16u * q + 64u * kSteps * split;
+    const unsigned input_at = (kF32BlockWeightRows + 16u * (tile >> 1) + i16) * kF32BlockPitch + 16u * q + 64u * kSteps * split;
     for (unsigned chunk = 0; chunk < chunks; ++chunk) {
         // (the last turn asks for its own chunk again and stages it where nobody reads it: no
         // branch around the loads, whose registers would otherwise be kept in scratch memory)
@@ -740,22 +751,8 @@ __global__ __launch_bounds__(512) void matvec_f32_block_kernel(MatvecArgs a)
         for (unsigned j = 0; j < kHeld; ++j)
             held[j] = fetch(j, ahead);
         const unsigned char *now = staged + (chunk & 1u) * (kRows * kF32BlockPitch);
-        unsigned char *next = staged + ((chunk + 1u) & 1u) * (kRows * kF32BlockPitch);
 #pragma unroll
-        for (unsigned step = 0; step < kF32BlockColumns / 16u; ++step) {
-            if (step == kF32BlockColumns / 32u) {
-                // half way: the loads have had four steps to arrive, and the stores have four
-                // more to land before the barrier
-#pragma unroll
-                for (unsigned j = 0; j < kHeld; ++j) {
-                    // (the weight rows are the first pieces: a non-finite weight is reported by
-                    // the thread that stages it, once, not by the sixteen lanes that multiply it)
-                    if (512u * (j + 1u) <= kF32BlockWeightRows * kPieces)
-                        bad |= (unsigned)!finite_f32(held[j][0]) | (unsigned)!finite_f32(held[j][1]) |
-                               (unsigned)!finite_f32(held[j][2]) | (unsigned)!finite_f32(held[j][3]);
-                    *reinterpret_cast<v4f *>(next + target[j]) = held[j];
-                }
-            }
+        for (unsigned step = 0; step < kSteps; ++step) {
             const v4f x = *reinterpret_cast<const v4f *>(now + input_at + 64u * step);
             const v4f w = *reinterpret_cast<const v4f *>(now + weight_at + 64u * step);
             acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)w[0], (double)x[0], acc, 0, 0, 0);
@@ -763,16 +760,28 @@ __global__ __launch_bounds__(512) void matvec_f32_block_kernel(MatvecArgs a)
             acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)w[2], (double)x[2], acc, 0, 0, 0);
             acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)w[3], (double)x[3], acc, 0, 0, 0);
         }
+        stage(staged + ((chunk + 1u) & 1u) * (kRows * kF32BlockPitch));
         // the next chunk is complete, and nobody reads this one any more when it is overwritten
         __syncthreads();
     }
     if (bad) raise_status(a.status, 1);
-    const unsigned long long in = (unsigned long long)blockIdx.y * kF32BlockInputRows + 16u * (wave >> 1) + i16;
+    // the other waves' sums of a tile through the stages' memory (the barrier above: nobody reads it any more)
+    double *const partial = reinterpret_cast<double *>(staged);
+    if (split) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) partial[(((split - 1u) * kTiles + tile) * 4u + k) * 64u + lane] = acc[k];
+    }
+    __syncthreads();
+    if (split) return;
+    const unsigned long long in = (unsigned long long)blockIdx.y * INPUTS + 16u * (tile >> 1) + i16;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         // accumulator k of lane (i, q): weight row 4 k + q of the tile, input row i
-        const unsigned long long row = (unsigned long long)blockIdx.x * kF32BlockWeightRows + 16u * (wave & 1u) + 4u * k + q;
-        if (row < a.row_count && in < a.input_rows) matvec_publish(a, in, row, (float)acc[k]);
+        const unsigned long long row = (unsigned long long)blockIdx.x * kF32BlockWeightRows + 16u * (tile & 1u) + 4u * k + q;
+        double sum = acc[k];
+#pragma unroll
+        for (unsigned other = 0; other + 1u < kSplits; ++other) sum += partial[((other * kTiles + tile) * 4u + k) * 64u + lane];
+        if (row < a.row_count && in < a.input_rows) matvec_publish(a, in, row, (float)sum);
     }
 }
 
@@ -1014,6 +1023,17 @@ static int launch_block_q(const MatvecArgs &a, bool q8, hipStream_t stream)
 
 using namespace yvex;
 
+template <unsigned QT, unsigned INPUTS>
+static int launch_scalar_block(const MatvecArgs &a, hipStream_t s)
+{
+    const unsigned long long block_y = (a.input_rows + INPUTS - 1ull) / INPUTS;
+    if (block_y > 65535ull) return ST_BOUNDS;
+    YVEX_ALLOW_DYNAMIC_LDS((matvec_f32_block_kernel<QT, INPUTS>), f32_block_lds(INPUTS));
+    matvec_f32_block_kernel<QT, INPUTS><<<dim3((unsigned)((a.row_count + kF32BlockWeightRows - 1ull) / kF32BlockWeightRows),
+                                           (unsigned)block_y), 64u * kF32BlockWaves, f32_block_lds(INPUTS), s>>>(a);
+    return check_launch("matvec_f32_block");
+}
+
 // Rows of F32, F16 or BF16 values against eight or more F32 input rows: 16 x 16 tiles on the
 // double-precision matrix cores; a small batch offers few tiles, so sixteen waves split the row
 // width, a large one has tiles enough for four, or for the staged kernel.
@@ -1022,19 +1042,27 @@ static int launch_scalar_rows(const MatvecArgs &a, hipStream_t s)
 {
     const unsigned long long grid_x = (a.row_count + 15ull) / 16ull, grid_y = (a.input_rows + 15ull) / 16ull;
     if (grid_x > 0x7fffffffull || grid_y > 65535ull) return ST_BOUNDS;
+    const unsigned long long block_rows = (a.row_count + kF32BlockWeightRows - 1ull) / kF32BlockWeightRows;
+    // The staged kernel's launch takes as long as its rounds of workgroups, one a compute unit: 51, 93 and
+    // 165 us a round with 16, 32 and 64 input rows a workgroup (7168 columns); the small tiles take 30 us
+    // for a workgroup a compute unit, 45 at least. So 256 weight rows by 512
+    // input rows take 51 us (60 with small tiles), by 850 93 (110), by 2048 165 (211), but by 1111 the
+    // small tiles' 136 (157).
+    const unsigned long long cus = compute_units();
+    auto rounds = [&](unsigned long long inputs) {
+        return (block_rows * ((a.input_rows + inputs - 1ull) / inputs) + cus - 1ull) / cus;
+    };
+    const unsigned long long small_tiles = 30ull * ((grid_x * grid_y + cus - 1ull) / cus);
+    const unsigned long long cost[4] = {small_tiles > 45ull ? small_tiles : 45ull, 51ull * rounds(16ull), 93ull * rounds(32ull),
+                                        165ull * rounds(64ull)};
+    unsigned best = 0u;
+    for (unsigned i = 1u; i < 4u; ++i)
+        if (cost[i] < cost[best]) best = i;
     if (a.input_rows < 256ull) {
         matvec_f32_tile16_kernel<16, QT><<<dim3((unsigned)grid_x, (unsigned)grid_y), 1024, 0, s>>>(a);
-    } else if (a.row_width % kF32BlockColumns == 0ull &&
-               (a.row_count + kF32BlockWeightRows - 1ull) / kF32BlockWeightRows *
-                   ((a.input_rows + kF32BlockInputRows - 1ull) / kF32BlockInputRows) >= 3ull * compute_units() / 4ull) {
-        // (a block a compute unit or close to it: the staged kernel walks the row width
-        // chunk by chunk, 3 us each, and is behind the small tiles on a grid that leaves
-        // most of the device idle: 161 us against 46 us for 256 rows by 256)
-        const unsigned long long block_y = (a.input_rows + kF32BlockInputRows - 1ull) / kF32BlockInputRows;
-        if (block_y > 65535ull) return ST_BOUNDS;
-        YVEX_ALLOW_DYNAMIC_LDS(matvec_f32_block_kernel<QT>, kF32BlockLdsBytes);
-        matvec_f32_block_kernel<QT><<<dim3((unsigned)((a.row_count + kF32BlockWeightRows - 1ull) / kF32BlockWeightRows),
-                                       (unsigned)block_y), 512, kF32BlockLdsBytes, s>>>(a);
+    } else if (a.row_width % kF32BlockColumns == 0ull && best) {
+        return best == 1u ? launch_scalar_block<QT, 16>(a, s) : best == 2u ? launch_scalar_block<QT, 32>(a, s)
+                                                                           : launch_scalar_block<QT, 64>(a, s);
     } else {
         matvec_f32_tile16_kernel<4, QT><<<dim3((unsigned)grid_x, (unsigned)grid_y), 256, 0, s>>>(a);
     }
