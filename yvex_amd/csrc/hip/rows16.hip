@@ -7,15 +7,16 @@
 // a barrier a superblock: 256 experts with eight pairs each cost what they cost with 32. Here a
 // tile is up to sixteen pairs of one bucket, and
 //   * their whole Q8_K rows are resident in LDS, so nothing is staged inside the loop and no
-//     wave waits for another: sixteen waves a workgroup, four a SIMD, cover each other's latency;
+//     wave waits for another: twelve waves a workgroup (eight for Q4_K and Q2_K rows) cover each
+//     other's latency;
 //   * a wave owns 32 weight rows (16 gate rows and the matching up rows when the SwiGLU is
 //     fused) and walks them superblock by superblock, records coming straight into registers
 //     ahead of their use, across row units as well;
 //   * the products are V_MFMA_I32_16X16X64_I8: lane (r, q) = (lane % 16, lane / 16) owns weight
 //     row r and a quarter of the superblock, four K chunks of sixteen values, in an order of K
 //     that is the format's own (both operands follow it). One B fragment serves both row tiles.
-//   * tiles times row units, in order, are cut into one piece of equal length a workgroup; the
-//     waves of a workgroup draw units of its piece from a counter.
+//   * tiles times row units, in order, are cut into one piece of equal length a workgroup (short
+//     ones end with their tiles); the waves of a workgroup draw units of its piece from a counter.
 // Measured (256 experts, uniform routing; the row-batch kernels before, these after): gate/up of 4096 x 2048
 // IQ2_XXS, eight pairs an expert, 620 -> 357 us, Q2_K down 358 -> 196; 7168 x 2048 IQ2_XXS, six pairs, 890 ->
 // 608 and 503 -> 307; Q4_K 1115 -> 950 and 624 -> 509 (4.5 TB/s). IQ2_XXS is bound by its loads: with
@@ -52,7 +53,7 @@ constexpr unsigned kIq2Image = 0x100u;                    // IQ2_XXS rows as the
 // [superblock][token], the minimum operands and the int8 payload.
 //
 // LDS reads: 64 banks, and a 16-byte read takes lanes 0-3, 12-15, 20-23 and 24-27 (and so on)
-// together. The table lookups of eight bytes use all banks because the lanes of odd quarters read
+// together. With the image the table lookups of eight bytes use all banks: the lanes of odd quarters read
 // the sign selectors with the instruction that reads codes for the even ones, and the codes with
 // the other (the two are OR-ed): 2.3 cycles an instruction instead of 4.0, measured in a loop of such
 // reads. The payload stands piece-major, [superblock][piece][token slot] with a multiple of four
