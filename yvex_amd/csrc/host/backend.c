@@ -64,17 +64,20 @@ int yvex_rocm_status_reset(yvex_rocm_backend *backend, const char *where, yvex_e
     /* row batches whose completion is deferred own the word until their barrier: an operation
      * that runs between them must not erase what they raised (it then reports it as its own) */
     if (backend->pending_completion) return YVEX_OK;
-    if (backend->status_clean) {
-        backend->status_clean = 0;     /* until the operation has been waited for */
-        return YVEX_OK;
+    if (backend->status_state != YVEX_ROCM_STATUS_CLEAN) {
+        int rc = yvex_rocm_launch_result(yvex_hip_fill_u32(backend->device_status, 0u, 1u, backend->stream),
+                                         where, err);
+        if (rc != YVEX_OK) return rc;
     }
-    return yvex_rocm_launch_result(yvex_hip_fill_u32(backend->device_status, 0u, 1u, backend->stream),
-                                   where, err);
+    backend->status_state = YVEX_ROCM_STATUS_OWNED;     /* until the operation has been waited for */
+    return YVEX_OK;
 }
 
 static int finish(yvex_rocm_backend *backend, unsigned long long device_results, unsigned long long bytes,
-                  const unsigned char **results, int clear, const char *where, int *device_status, yvex_error *err)
+                  const unsigned char **results, int whole_phase, const char *where, int *device_status,
+                  yvex_error *err)
 {
+    const int clear = backend->status_state == YVEX_ROCM_STATUS_OWNED && (whole_phase || !backend->pending_completion);
     const unsigned int sequence = ++backend->published_sequence;
     int rc;
     *device_status = 0;
@@ -88,7 +91,7 @@ static int finish(yvex_rocm_backend *backend, unsigned long long device_results,
         backend->status = YVEX_BACKEND_STATUS_FAILED;
         return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, where, yvex_hip_last_error());
     }
-    if (clear) backend->status_clean = 1;
+    if (clear) backend->status_state = YVEX_ROCM_STATUS_CLEAN;
     if (results) *results = backend->published + YVEX_HIP_PUBLISH_HEAD_BYTES;
     backend->memory.d2h_bytes += sizeof(int);
     return YVEX_OK;
@@ -96,14 +99,14 @@ static int finish(yvex_rocm_backend *backend, unsigned long long device_results,
 
 int yvex_rocm_finish(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err)
 {
-    return finish(backend, 0ull, 0ull, NULL, !backend->pending_completion, where, device_status, err);
+    return finish(backend, 0ull, 0ull, NULL, 0, where, device_status, err);
 }
 
 int yvex_rocm_finish_results(yvex_rocm_backend *backend, unsigned long long device_results, unsigned long long bytes,
                              const unsigned char **results, const char *where, int *device_status,
                              yvex_error *err)
 {
-    return finish(backend, device_results, bytes, results, !backend->pending_completion, where, device_status, err);
+    return finish(backend, device_results, bytes, results, 0, where, device_status, err);
 }
 
 int yvex_rocm_finish_phase(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err)
@@ -204,7 +207,7 @@ int yvex_rocm_backend_open(yvex_rocm_backend **out, const yvex_backend_options *
             (yvex_hip_fill_u32(backend->device_status, 0u, 1u, backend->stream) != 0 ||
              yvex_hip_stream_sync(backend->stream) != 0))
             backend->kernels_available = 0;
-        backend->status_clean = backend->kernels_available;
+        backend->status_state = backend->kernels_available ? YVEX_ROCM_STATUS_CLEAN : YVEX_ROCM_STATUS_UNKNOWN;
     }
     backend->status = backend->kernels_available ? YVEX_BACKEND_STATUS_READY
                                                  : YVEX_BACKEND_STATUS_CONTEXT_READY;
@@ -251,7 +254,7 @@ int yvex_rocm_backend_open_shared(yvex_rocm_backend **out, yvex_rocm_backend *co
             (yvex_hip_fill_u32(backend->device_status, 0u, 1u, backend->stream) != 0 ||
              yvex_hip_stream_sync(backend->stream) != 0))
             backend->kernels_available = 0;
-        backend->status_clean = backend->kernels_available;
+        backend->status_state = backend->kernels_available ? YVEX_ROCM_STATUS_CLEAN : YVEX_ROCM_STATUS_UNKNOWN;
     }
     backend->status = backend->kernels_available ? YVEX_BACKEND_STATUS_READY
                                                  : YVEX_BACKEND_STATUS_CONTEXT_READY;

@@ -119,7 +119,8 @@ static int weight_address_in(yvex_rocm_moe_execution *x, const yvex_moe_weight_v
     return rc;
 }
 
-/* Stream synchronisation and the kernels' status word (moe.c:277-296). */
+/* Stream synchronisation and the kernels' status word (moe.c:277-296), which is read and left: the
+ * execution goes on launching after its first wait, and others may be open beside it. */
 static int sync_status(yvex_rocm_moe_execution *x, const char *where, yvex_error *err)
 {
     int device_status = 0, rc;
@@ -483,7 +484,7 @@ int yvex_rocm_backend_moe_begin(yvex_rocm_moe_execution **out, yvex_rocm_backend
         }
     }
     expanded_bytes = layer->expanded_width * sizeof(float);
-    if (!backend->pending_completion) backend->status_clean = 0;
+    backend->status_state = YVEX_ROCM_STATUS_UNKNOWN;     /* from here on this execution's kernels may raise it */
     rc = backend->pending_completion   /* deferred row batches own the word until their barrier */
         ? YVEX_OK
         : launched(x, yvex_hip_fill_u32(backend->device_status, 0u, 1u, backend->stream), "rocm.moe.status", err);
@@ -548,6 +549,7 @@ int yvex_rocm_backend_moe_add_expert(yvex_rocm_moe_execution *x, const yvex_moe_
         rc = weight_address_in(x, down, width, layer->hidden_width, x->stage_offset[2],
                                x->stage_capacity[2], &address[2], "rocm.moe.expert-down", err);
     if (rc != YVEX_OK) return rc;
+    x->backend->status_state = YVEX_ROCM_STATUS_UNKNOWN;
     fill_weights(&w, gate, up, down, address, layer->hidden_width, width);
     if (!shared) {
         unsigned int bits;
@@ -600,6 +602,7 @@ int yvex_rocm_backend_moe_finish(yvex_rocm_moe_execution *x, yvex_moe_layer_resu
     stream = x->backend->stream;
     status = x->backend->device_status;
     evidence = !x->job->device_output || x->job->evidence_level == YVEX_ATTENTION_EVIDENCE_FULL;
+    x->backend->status_state = YVEX_ROCM_STATUS_UNKNOWN;
     /* routed = experts in the order added, combined = bf16(routed + shared): moe.c:752-770 */
     rc = launched(x, yvex_hip_moe_reduce_combine((const float *)AT(pair_outputs), 1ull,
                                                  x->routed_added ? x->routed_added : 1ull, hidden,

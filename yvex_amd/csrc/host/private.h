@@ -33,7 +33,7 @@ struct yvex_rocm_backend {
     unsigned long long workspace_bytes, workspace_cursor;
     /* device status word shared by the operations of this backend */
     int *device_status;
-    int status_clean;          /* the word is zero: whoever read it last cleared it */
+    int status_state;          /* YVEX_ROCM_STATUS_*: what the host knows of the word */
     int pending_completion;
     /* pinned host memory that a synchronous operation's last launch publishes its status word and
      * small results in, and the number of the last such launch */
@@ -65,18 +65,27 @@ void yvex_rocm_workspace_reset(yvex_rocm_backend *backend);
 int yvex_rocm_require_kernels(const yvex_rocm_backend *backend, const char *where, yvex_error *err);
 /* Map a launch-level return code (negative yvex_status) to an error. */
 int yvex_rocm_launch_result(int rc, const char *where, yvex_error *err);
-/* Wait for the stream's work and read the device status word; the word is cleared unless deferred
- * row batches are waiting for their barrier. */
+/* What the host knows of the status word. Only the operation whose own reset found or made it zero
+ * may clear it again when it reads it, and only then is it known to be clean: kernels of a token-local
+ * execution may raise it at any time between begin and finish, and what they raise is theirs to report. */
+enum {
+    YVEX_ROCM_STATUS_UNKNOWN = 0,   /* may have been raised, or may be raised yet, by somebody else's kernels */
+    YVEX_ROCM_STATUS_CLEAN,         /* zero, and nothing was launched since that could raise it */
+    YVEX_ROCM_STATUS_OWNED          /* reset for an operation that has not been waited for */
+};
+/* Wait for the stream's work and read the device status word. The word is cleared where the waiting
+ * operation owns it and no deferred row batches are waiting for their barrier, and left as it is else. */
 int yvex_rocm_finish(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err);
 /* The same for an operation with small results: `bytes` of device memory (a multiple of 4, at most
  * YVEX_HIP_PUBLISH_MAX_BYTES) arrive in *results, host memory that is good until the next such call. */
 int yvex_rocm_finish_results(yvex_rocm_backend *backend, unsigned long long device_results, unsigned long long bytes,
                              const unsigned char **results, const char *where, int *device_status,
                              yvex_error *err);
-/* The barrier of a phase of deferred row batches: yvex_rocm_finish that clears the word they share. */
+/* The barrier of a phase of deferred row batches: the word they share is cleared where the phase still
+ * owns it. */
 int yvex_rocm_finish_phase(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err);
-/* Make sure the status word is zero on the stream, unless deferred row batches are waiting for their
- * barrier. */
+/* Make sure the status word is zero on the stream and take it for the calling operation, unless deferred
+ * row batches are waiting for their barrier. */
 int yvex_rocm_status_reset(yvex_rocm_backend *backend, const char *where, yvex_error *err);
 /* Resolve a weight view: device_address if given, else the resident arena mapping. */
 /* Queue `bytes` of caller-owned host memory for upload to `device` on the backend's stream; the
