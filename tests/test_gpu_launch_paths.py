@@ -250,3 +250,25 @@ def test_router_blocks_of_every_size_are_sums_in_double(gpu, rows, width, inputs
     # sums in double in another order differ by under 1e-13 of the terms: the float is the same or, next
     # to a rounding boundary, its neighbour
     assert torch.all((got - want).abs() <= want.abs() * 2.0 ** -23 + 1e-12) and int(status.item()) == 0
+
+
+# a row below and at the line between the sweeps and the tiles: the constant part and the cap of each rule
+@pytest.mark.parametrize("qtype,shared,hidden,experts,at", [
+    ("IQ2_XXS", True, 512, 8, 62), ("IQ2_XXS", True, 512, 4, 36), ("IQ2_XXS", True, 5632, 8, 60), ("IQ2_XXS", "Q8_0", 512, 16, 41),
+    ("IQ2_XXS", False, 512, 8, 24), ("Q4_K", True, 512, 24, 45), ("Q4_K", True, 512, 4, 8), ("Q4_K", False, 512, 8, 11)])
+def test_row_batches_either_side_of_the_matrix_core_line(gpu, oracle, qtype, shared, hidden, experts, at):
+    from backend_helpers import Backend
+    from test_gpu_backend import MoeCase, same_as_cpu
+    for rows in (at - 1, at):
+        b = Backend()
+        try:
+            case = MoeCase(b, oracle, qtype=qtype, hidden=hidden, experts=experts, topk=2, rows=rows, shared=bool(shared),
+                           shared_qtype=shared if isinstance(shared, str) else None)
+            b.workspace(case.workspace_bytes)
+            assert case.execute() == 0, case.err.message
+            assert (case.result.tensor_core_launches > 0) == (rows == at)
+            want = case.oracle_layer(act_q8=True)
+            assert np.array_equal(case.sel.reshape(rows, 2), want["selected"])
+            same_as_cpu(case.combined, want["combined"])
+        finally:
+            assert b.close() == 0

@@ -342,6 +342,41 @@ static int same_expert_shape(const yvex_hip_expert_weights *a, const yvex_hip_ex
            a->down_image == b->down_image;
 }
 
+/* Routed pairs from which a batch goes to the int8 matrix-core kernels (IQ2_XXS or Q4_K gate and up rows,
+ * Q8_K activations); below, the decode sweeps, which read an expert's bytes once per four pairs, are
+ * faster. The lines lie where whole layers of 4 to 256 experts cross under uniform routing, intermediate
+ * rows 2048 wide. A shared expert of the routed experts' shape (`rides`) goes along in the sweeps'
+ * launches and takes launches of its own beside the tiles, so the lines have a constant part.
+ *   IQ2_XXS, rides: crossings at 3.0, 3.5, 4.2 and 4.6 pairs an expert for 256, 128, 64 and 32 experts 7168
+ *     wide, 3.4, 4.3, 4.8 and 5.7 at 4096, 3.8, -, 5.5 and 6.5 at 2048; about 6.5 to 9 for 8 to 24
+ *     experts. 256 experts at 4096: 3.0 pairs 568 us as sweeps and 604 as tiles, 4.0 pairs 704 and 640;
+ *     at 7168: 2.5 pairs 867 and 920, 3.5 pairs 1117 and 998. With four experts every bucket has its
+ *     columns full at the cap.
+ *   IQ2_XXS alone: 3.1 to 3.6 pairs for 256 experts of any width, 2.8 to 3.9 for 32 and 64 (256 at 4096 with
+ *     Q2_K down rows: 3.0 pairs 610 and 660, 4.0 pairs 746 and 685).
+ *   Q4_K, rides: 2.7, 2.8, 3.2 and 3.4 (256 at 7168: 2.5 pairs 1380 and 1421, 3.0 pairs 1532 and 1461), 3.7 to
+ *     4.8 for 8 to 24 experts. Q4_K alone: 2.8 for 256 experts, under 2.5 for fewer.
+ * Sums of few pairs are flat around the line: within a quarter of it the slower side costs under 10 %.
+ * A skewed routing crosses earlier (an exponent of 0.4 at 2.3 to 3.5 pairs, of 0.8 at under 2.5), but the
+ * host does not know the routing. */
+static unsigned long long matrix_core_pairs(const yvex_hip_expert_weights *routed, unsigned long long experts,
+                                            int rides)
+{
+    unsigned long long line, cap;
+    if (routed->gate_qtype == 12u) {
+        line = rides ? experts * 5ull / 2ull + 30ull : experts * 11ull / 4ull;
+        cap = experts * 4ull;
+    } else if (rides) {
+        /* between the widths measured on either side the line is drawn half way */
+        line = (routed->hidden < 5632ull ? experts * 3ull : experts * 13ull / 5ull) + 100ull;
+        cap = experts * 18ull;
+    } else {
+        line = experts * 13ull / 4ull + 30ull;
+        cap = experts * 6ull;
+    }
+    return line < cap ? line : cap;
+}
+
 /* ---- launch graphs -------------------------------------------------------------------------
  * The launch sequence of a row batch depends only on facts the host knows before the first
  * kernel: the layer's geometry and policies, the weight views, the row count, and the device
@@ -680,23 +715,16 @@ static int moe_execute_rows(yvex_rocm_backend *backend, const yvex_moe_layer_job
         fill_expert_weights(&shared, &views[YVEX_MOE_WEIGHT_SHARED_GATE], &views[YVEX_MOE_WEIGHT_SHARED_UP],
                             &views[YVEX_MOE_WEIGHT_SHARED_DOWN], addresses[3], addresses[4], addresses[5],
                             hidden, layer->shared_intermediate_width, shared_image);
-    /* Row batches whose buckets average three pairs or more go to the int8 matrix-core kernels
-     * (IQ2_XXS or Q4_K weights, Q8_K activations); below that the decode sweeps, which read an
-     * expert's bytes once per four pairs, are faster. Gate/up and down launches of 256 experts, uniform
-     * routing: 7168 wide, top-8, 96 rows IQ2_XXS 824 us as sweeps and 858 as tiles, 112 rows 939 and 871;
-     * Q4_K 96 rows 1334 and 1306; 4096 wide, top-6, Q2_K down, 128 rows 485 and 527, 160 rows 568 and 543.
-     * A skewed routing is a little better off as tiles (96 rows at 7168, a Zipf exponent of 1.1: 430 us
-     * and 400). Layers of fewer than 32 experts keep the line at six (four with Q4_K rows), where
-     * the published launch facts have had it: their launches are 20-50 us either way. The
-     * reference switches its tensor-core kernels on from 16 input rows
-     * (src/backend/cuda/private.h:461-464). Both kernel families read the sweep image of
+    /* The reference switches its tensor-core kernels on from 16 input rows
+     * (src/backend/cuda/private.h:461-464); here the pairs decide. Both kernel families read the sweep image of
      * IQ2_XXS experts as well as canonical bytes, and both publish the same bits (a row's terms
      * are added in double in block order in either), so the choice is one of speed only; a
      * sealed worklist policy can keep the matrix-core regime off (matrix_allowed). */
+    merged = has_shared && shared_q8 == routed_q8 && same_expert_shape(&routed, &shared);
     row_batch = matrix_allowed && routed_q8 && matrix_core_qtypes(&routed) &&
-                pairs >= (experts >= 32ull ? 3ull : routed.gate_qtype == 12u ? 4ull : 6ull) * experts;
+                pairs >= matrix_core_pairs(&routed, experts, merged);
     shared_row_batch = row_batch && has_shared && shared_q8 && matrix_core_qtypes(&shared);
-    merged = !row_batch && has_shared && shared_q8 == routed_q8 && same_expert_shape(&routed, &shared);
+    merged = merged && !row_batch;
     /* A Q8_0 shared expert (the format the reference's model file keeps it in, its default for every
      * tensor outside the routed experts: src/graph/families/deepseek_v4.c:1550-1557) is three dense
      * projections of every row, and the dense Q8_0 kernels give the CPU path's bits at any number of
