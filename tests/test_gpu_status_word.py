@@ -94,3 +94,27 @@ def test_an_execution_reports_what_its_kernels_raised(backend, oracle, between):
     assert t.close() == 0
     backend.workspace(8 << 20)
     assert next_operation(backend, case, "matvec") == 0
+
+
+def test_a_phase_counts_the_launches_it_makes(backend, oracle):  # noqa: F811
+    """The batches of a phase launch the same kernels; the word is cleared before the first only where somebody
+    else may have raised it, and published once at the barrier."""
+    case = MoeCase(backend, oracle, rows=3, streams=4, act=abi.ACT_DEVICE_F32)
+    backend.workspace(max(case.workspace_bytes, 8 << 20))
+
+    def phase(batches):
+        counts = []
+        for _ in range(batches):
+            assert deferred(case) == 0, case.err.message
+            counts.append(case.result.kernel_launches)
+        done = abi.RowBatchResult()
+        assert case.ops.complete_rows(backend.handle, 0, C.byref(done), C.byref(case.err)) == 0
+        return counts, done.kernel_launches
+    (first, second, third), published = phase(3)
+    assert first == second == third and published == 1
+    out, case.out = case.out, abi.RowBatchOutput()      # (no host copies, whose rows would come from other kernels)
+    assert case.execute() == 0 and case.result.kernel_launches == first + published
+    case.out = out
+    assert opened(case).close() == 0
+    (first, second), published = phase(2)
+    assert first == second + 1 and published == 1

@@ -59,7 +59,8 @@ int yvex_rocm_require_kernels(const yvex_rocm_backend *backend, const char *wher
     return YVEX_OK;
 }
 
-int yvex_rocm_status_reset(yvex_rocm_backend *backend, const char *where, yvex_error *err)
+int yvex_rocm_status_reset(yvex_rocm_backend *backend, unsigned long long *launches, const char *where,
+                           yvex_error *err)
 {
     /* row batches whose completion is deferred own the word until their barrier: an operation
      * that runs between them must not erase what they raised (it then reports it as its own) */
@@ -68,6 +69,7 @@ int yvex_rocm_status_reset(yvex_rocm_backend *backend, const char *where, yvex_e
         int rc = yvex_rocm_launch_result(yvex_hip_fill_u32(backend->device_status, 0u, 1u, backend->stream),
                                          where, err);
         if (rc != YVEX_OK) return rc;
+        if (launches) (*launches)++;
     }
     backend->status_state = YVEX_ROCM_STATUS_OWNED;     /* until the operation has been waited for */
     return YVEX_OK;

@@ -760,9 +760,8 @@ static int moe_execute_rows(yvex_rocm_backend *backend, const yvex_moe_layer_job
      * completion is deferred leaves what it raised for the barrier to find, whatever runs behind
      * it (the word only ever changes from zero). Like the token ids, outside any graph. */
     if (!backend->pending_completion) {
-        rc = yvex_rocm_status_reset(backend, "rocm.moe.rows.status", err);
+        rc = yvex_rocm_status_reset(backend, &status_launches, "rocm.moe.rows.status", err);
         if (rc != YVEX_OK) return rc;
-        status_launches = 1ull;
     }
     if (!job->eager_execution && !(backend->moe_graphs && backend->moe_graphs->refused)) {
         graph_key key;
@@ -1179,6 +1178,7 @@ sequence:
     {
         unsigned long long sync_started = monotonic_ns();
         rc = yvex_rocm_finish(backend, "rocm.moe.rows.sync", &device_status, err);
+        if (rc == YVEX_OK) result->kernel_launches++;      /* it published the word */
         result->synchronization_ns = monotonic_ns() - sync_started;
     }
     d2h += sizeof(int);
@@ -1275,6 +1275,7 @@ static int moe_complete_rows(yvex_rocm_backend *backend, int barrier_observed,
     result->completed = 1;
     result->execution_class = YVEX_EXECUTION_CLASS_DEVICE_NATIVE;
     result->stream_synchronizations = barrier_observed ? 0ull : 1ull;
+    result->kernel_launches = backend->host_only ? 0ull : 1ull;      /* it published the word */
     result->synchronization_ns = started ? monotonic_ns() - started : 0ull;
     yvex_rocm_error_clear(err);
     return YVEX_OK;

@@ -85,8 +85,10 @@ int yvex_rocm_finish_results(yvex_rocm_backend *backend, unsigned long long devi
  * owns it. */
 int yvex_rocm_finish_phase(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err);
 /* Make sure the status word is zero on the stream and take it for the calling operation, unless deferred
- * row batches are waiting for their barrier. */
-int yvex_rocm_status_reset(yvex_rocm_backend *backend, const char *where, yvex_error *err);
+ * row batches are waiting for their barrier. *launches, where asked for, counts the launch this took: none
+ * where the word was clean. */
+int yvex_rocm_status_reset(yvex_rocm_backend *backend, unsigned long long *launches, const char *where,
+                           yvex_error *err);
 /* Resolve a weight view: device_address if given, else the resident arena mapping. */
 /* Queue `bytes` of caller-owned host memory for upload to `device` on the backend's stream; the
  * caller's buffer may be reused as soon as this returns. */

@@ -110,7 +110,7 @@ int yvex_rocm_encoded_matvec(
     if (yvex_rocm_seam("YVEX_TEST_ROCM_LAUNCH_FAILURE"))
         return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, "rocm.encoded-matvec.launch",
                                 "kernel launch failed (test seam)");
-    rc = yvex_rocm_status_reset(backend, where, err);
+    rc = yvex_rocm_status_reset(backend, NULL, where, err);
     activations = input->data;
     if (rc == YVEX_OK && split_input) {
         rc = yvex_rocm_launch_result(
@@ -196,7 +196,7 @@ int yvex_rocm_encoded_gather(
     if (yvex_hip_memcpy_h2d((void *)(uintptr_t)ids_address, row_ids, selected_rows * sizeof(unsigned int),
                             backend->stream) != 0)
         return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, where, yvex_hip_last_error());
-    rc = yvex_rocm_status_reset(backend, where, err);
+    rc = yvex_rocm_status_reset(backend, NULL, where, err);
     if (rc == YVEX_OK)
         rc = yvex_rocm_launch_result(
             yvex_hip_gather((const uint8_t *)(uintptr_t)device_address, qtype, row_count, row_width,

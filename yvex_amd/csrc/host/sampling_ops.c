@@ -65,7 +65,7 @@ int yvex_rocm_select_greedy_rows(
     if (yvex_rocm_seam("YVEX_TEST_ROCM_LAUNCH_FAILURE"))
         return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, "rocm.sampling.greedy.launch",
                                 "kernel launch failed (test seam)");
-    rc = yvex_rocm_status_reset(backend, where, err);
+    rc = yvex_rocm_status_reset(backend, NULL, where, err);
     if (rc == YVEX_OK)
         rc = yvex_rocm_launch_result(
             yvex_hip_argmax_f32((const float *)logits->data, row_count, row_width,
