@@ -272,3 +272,44 @@ def test_row_batches_either_side_of_the_matrix_core_line(gpu, oracle, qtype, sha
             same_as_cpu(case.combined, want["combined"])
         finally:
             assert b.close() == 0
+
+
+# the layer as a decoder runs it, deferred and without host copies, whose combine goes straight into the egress; the
+# caller alternates with batches that ask for host copies, each kind eager, captured and replayed
+@pytest.mark.parametrize("down,shared,rows", [(None, None, 1), ("Q2_K", "Q8_0", 5), ("Q2_K", "Q8_0", 75)])
+def test_deferred_layers_with_streams_are_the_oracles(gpu, oracle, down, shared, rows):
+    from backend_helpers import Backend
+    from test_gpu_backend import MoeCase, same_as_cpu
+    from yvex_amd import abi
+    b = Backend()
+    try:
+        case = MoeCase(b, oracle, hidden=512, intermediate=512, rows=rows, streams=4, down_qtype=down, shared_qtype=shared)
+        b.workspace(case.workspace_bytes)
+        want, host, done = case.oracle_layer(act_q8=True), case.out, abi.RowBatchResult()
+        empty, zeros = abi.RowBatchOutput(), np.zeros_like(case.x)
+        completion = abi.DeviceCompletion(1, None)
+        for sight in range(3):
+            for kind in ("host copies", "deferred", "no copies"):
+                assert b.lib.yvex_rocm_backend_tensor_write(b.handle, case.rows_out, zeros.ctypes.data, zeros.nbytes,
+                                                            C.byref(case.err)) == 0
+                case.combined.fill(0.0)
+                case.out = host if kind == "host copies" else empty
+                case.job.device_completion = C.pointer(completion) if kind == "deferred" else None
+                assert case.execute() == 0, case.err.message
+                if kind == "deferred":
+                    assert case.ops.complete_rows(b.handle, 0, C.byref(done), C.byref(case.err)) == 0, case.err.message
+                # (deferred or not, batches without host copies are one topology)
+                assert case.result.graph_replays == (sight == 2 or (sight == 1 and kind != "host copies"))
+                if kind == "host copies":
+                    assert np.max(np.abs(case.post - want["post"])) <= 1e-6
+                    assert np.max(np.abs(case.comb - want["combination"])) <= 1e-6
+                    same_as_cpu(case.combined, want["combined"])
+                    # the egress of the CPU's combined rows with the device's own gates is exact
+                    rc, egress = oracle.mhc_post(want["combined"], case.x, case.post, case.comb, streams=4, width=512)
+                    assert rc == 0
+                else:
+                    assert not case.combined.any()
+                got = b.read_f32(case.rows_out, case.x.size).reshape(case.x.shape)
+                assert np.array_equal(got.view(np.uint32), egress.view(np.uint32)), kind
+    finally:
+        assert b.close() == 0
