@@ -313,3 +313,21 @@ def test_deferred_layers_with_streams_are_the_oracles(gpu, oracle, down, shared,
                 assert np.array_equal(got.view(np.uint32), egress.view(np.uint32)), kind
     finally:
         assert b.close() == 0
+
+
+# matrices past 32 768 rows against few input rows: one round of the 16-token tiles, and more than one
+@pytest.mark.parametrize("rows,inputs", [(32772, 8), (50004, 17), (99332, 9)])
+def test_iq2_rows_of_tall_matrices_are_the_sweeps_bits(gpu, oracle, rows, inputs):
+    from yvex_amd import kernels as K
+    width = 512
+    g = oracle.Generator(44, f"tall.{rows}")
+    w = dev(g.weights(oracle.IQ2_XXS, rows, width), gpu)
+    x = dev(g.normal(inputs * width).reshape(inputs, width), gpu)
+    status = K.new_status(gpu)
+    got = K.matvec(w, oracle.IQ2_XXS, rows, width, K.q8k_quantize(x, status), input_q8=True, input_rows=inputs, status=status)
+    for at in range(0, inputs, 7):                     # (fewer than eight input rows: the sweep)
+        some = x[at:at + 7].contiguous()
+        want = K.matvec(w, oracle.IQ2_XXS, rows, width, K.q8k_quantize(some, status), input_q8=True,
+                        input_rows=some.shape[0], status=status)
+        assert same_bits(got[at:at + 7], want)
+    assert int(status.item()) == 0
