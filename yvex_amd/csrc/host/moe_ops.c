@@ -347,16 +347,16 @@ static int same_expert_shape(const yvex_hip_expert_weights *a, const yvex_hip_ex
  * faster. The lines lie where whole layers of 4 to 256 experts cross under uniform routing, intermediate
  * rows 2048 wide. A shared expert of the routed experts' shape (`rides`) goes along in the sweeps'
  * launches and takes launches of its own beside the tiles, so the lines have a constant part.
- *   IQ2_XXS, rides: crossings at 3.0, 3.5, 4.2 and 4.6 pairs an expert for 256, 128, 64 and 32 experts 7168
- *     wide, 3.4, 4.3, 4.8 and 5.7 at 4096, 3.8, -, 5.5 and 6.5 at 2048; about 6.5 to 9 for 8 to 24
- *     experts. 256 experts at 4096: 3.0 pairs 568 us as sweeps and 604 as tiles, 4.0 pairs 704 and 640;
- *     at 7168: 2.5 pairs 867 and 920, 3.5 pairs 1117 and 998. With four experts every bucket has its
- *     columns full at the cap.
+ *   IQ2_XXS, rides: crossings at 3.0, 3.4, 4.2 and 4.6 pairs an expert for 256, 128, 64 and 32 experts 7168
+ *     wide, 3.4, 4.3, 4.8 and 5.7 at 4096, 3.8, -, 5.5 and over 6 at 2048; from 6 to over 20 for 24 to 4
+ *     experts, where buckets past a tile's sixteen columns put the tiles behind once more. 256 experts at
+ *     4096: 3.0 pairs 568 us as sweeps and 604 as tiles, 4.0 pairs 704 and 640; at 7168: 2.5 pairs 867 and 920,
+ *     3.5 pairs 1117 and 998. The cap is where sealed policies of four-expert layers expect the tiles.
  *   IQ2_XXS alone: 3.1 to 3.6 pairs for 256 experts of any width, 2.8 to 3.9 for 32 and 64 (256 at 4096 with
  *     Q2_K down rows: 3.0 pairs 610 and 660, 4.0 pairs 746 and 685).
  *   Q4_K, rides: 2.7, 2.8, 3.2 and 3.4 (256 at 7168: 2.5 pairs 1380 and 1421, 3.0 pairs 1532 and 1461), 3.7 to
  *     4.8 for 8 to 24 experts. Q4_K alone: 2.8 for 256 experts, under 2.5 for fewer.
- * Sums of few pairs are flat around the line: within a quarter of it the slower side costs under 10 %.
+ * Between a crossing and its line the slower side costs under 10 % with 32 experts and more.
  * A skewed routing crosses earlier (an exponent of 0.4 at 2.3 to 3.5 pairs, of 0.8 at under 2.5), but the
  * host does not know the routing. */
 static unsigned long long matrix_core_pairs(const yvex_hip_expert_weights *routed, unsigned long long experts,
@@ -368,7 +368,7 @@ static unsigned long long matrix_core_pairs(const yvex_hip_expert_weights *route
         cap = experts * 4ull;
     } else if (rides) {
         /* between the widths measured on either side the line is drawn half way */
-        line = (routed->hidden < 5632ull ? experts * 3ull : experts * 13ull / 5ull) + 100ull;
+        line = routed->hidden < 5632ull ? experts * 3ull + 100ull : experts * 13ull / 5ull + 85ull;
         cap = experts * 18ull;
     } else {
         line = experts * 13ull / 4ull + 30ull;
