@@ -443,7 +443,8 @@ constexpr unsigned kWideLdsBytes = kWideScaleBase + 2u * kWideTokens * 4u;
 //  * The input rows' scales lie end to end in LDS: a lane's sixteen are four 16-byte reads, not
 //    sixteen 4-byte ones.
 //  * Copies take a scalar base and a 32-bit offset a lane: a register and no addition each.
-// 4096 x 4096 by 2048 rows 171 -> 138 us (498 TOP/s), 2048 x 7168 124 -> 104 us.
+// 4096 x 4096 by 2048 rows 171 -> 138 us (498 TOP/s), 2048 x 7168 124 -> 104 us. Counters of the former: vector ALU
+// 79 % busy, LDS 20 %, matrix cores 11 %.
 __global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80Args g)
 {
     extern __shared__ __align__(16) unsigned char dense_q8_0_lds[];

@@ -19,9 +19,10 @@
 //     ones end with their tiles); the waves of a workgroup draw units of its piece from a counter.
 // Measured (256 experts, uniform routing; the row-batch kernels before, these after): gate/up of 4096 x 2048
 // IQ2_XXS, eight pairs an expert, 620 -> 357 us, Q2_K down 358 -> 196; 7168 x 2048 IQ2_XXS, six pairs, 890 ->
-// 608 and 503 -> 307; Q4_K 1115 -> 950 and 624 -> 509 (4.5 TB/s). IQ2_XXS is bound by its loads: with
-// all of them hitting the first cache and nothing computed the launch takes 245 us, from memory 330;
-// scaling, matrix instructions and lookups hide behind them. Coalescing four lanes to a row and passing
+// 608 and 503 -> 307; Q4_K 1115 -> 950 and 624 -> 509 (4.5 TB/s). IQ2_XXS has no pipe full (counters, 4096 x 2048 by
+// eight pairs, 358 us: 1.21 GB or 3.4 TB/s, vector ALU 62 % busy, LDS 31 %, matrix cores 16 %; a wave waits for data
+// 38 % of its time and for its turn to issue 29 %): load latency that three waves a SIMD do not cover, and
+// more do not fit the registers. Coalescing four lanes to a row and passing
 // the records through LDS, requesting four superblocks ahead, eight or sixteen waves (spills) were no faster.
 // The arithmetic is that of the kernels named above, term by term: int8 limbs whose product sums
 // are exact, one float term a superblock, added in double in superblock order, rounded to float
