@@ -237,6 +237,44 @@ def test_few_pair_kernels_agree_with_the_generic_kernel(gpu, oracle, up, down, h
     assert int(status.item()) == 0
 
 
+# one more pair than a tile of the few-pair kernels, two tiles' pairs, one more; as many such buckets as their second tiles
+# are for and one more; rows of four, five and 28 superblocks (two at a time, one, one and twelve pairs a tile)
+@pytest.mark.parametrize("hidden,intermediate,tokens", [(1024, 1024, 16), (1280, 512, 16), (7168, 256, 12)])
+@pytest.mark.parametrize("extra", [0, 1])
+@pytest.mark.parametrize("tail", ["within", "beyond"])
+def test_few_pair_kernels_take_second_tiles(gpu, oracle, hidden, intermediate, tokens, extra, tail):
+    """What the 64-pair kernels leave and the few-pair kernels take is each pair once, whichever side of
+    the rule for second tiles a batch is on."""
+    from yvex_amd import kernels as K
+    uq, dq = oracle.IQ2_XXS, oracle.Q2_K
+    populations = [tokens + 1 + (i * 3) % tokens for i in range(16 + extra)] + [2 * tokens + (tail == "beyond"), 1, tokens]
+    populations = populations[1:]                       # sixteen buckets past a tile, or seventeen
+    experts, pairs = len(populations), sum(populations)
+    g = oracle.Generator(44, f"second.{hidden}")
+    tensors = [dev(g.weights(q, experts * r, w), gpu) for q, r, w in
+               ((uq, intermediate, hidden), (uq, intermediate, hidden), (dq, hidden, intermediate))]
+    weights = K.expert_weights(*tensors, (uq, uq, dq), hidden, intermediate)
+    rows_form = K.expert_weights(*tensors, (uq, uq, dq), hidden, intermediate)
+    images = [K.iq2_sweep_image(t) for t in tensors[:2]]
+    rows_form.gate, rows_form.up, rows_form.gate_up_image = images[0].data_ptr(), images[1].data_ptr(), 1
+    rows_form.gate_row_bytes = rows_form.up_row_bytes = hidden // 256 * 72
+    rows_form.gate_expert_bytes = rows_form.up_expert_bytes = hidden // 256 * 72 * intermediate
+    status = K.new_status(gpu)
+    selected = torch.repeat_interleave(torch.arange(experts), torch.tensor(populations)).reshape(pairs, 1).to(gpu)
+    wl = K.worklist_build(selected, experts, status)
+    route = dev((0.5 + np.abs(g.normal(pairs))).astype(np.float32), gpu)
+    act = K.q8k_quantize(dev(g.normal(pairs * hidden).reshape(pairs, hidden), gpu), status)
+    mid = [torch.full((pairs, intermediate), float("nan"), device=gpu) for _ in range(2)]
+    K.moe_up(weights, act, True, route, wl, pairs, 1, experts, 10.0, mid[0], status)
+    K.moe_up_rows(rows_form, act, route, wl, pairs, 1, experts, 10.0, mid[1], status)
+    assert same_bits(mid[0], mid[1])
+    mid_q8 = K.q8k_quantize(mid[0], status)
+    out = [torch.full((pairs, hidden), float("nan"), device=gpu) for _ in range(2)]
+    K.moe_down(weights, mid_q8, True, wl, pairs, experts, out[0], status)
+    K.moe_down_rows(rows_form, mid_q8, wl, pairs, experts, out[1], status)
+    assert same_bits(out[0], out[1]) and int(status.item()) == 0
+
+
 # 16, 32 and 64 input rows a workgroup of the staged kernel (on 256 compute units), ragged on both sides,
 # one chunk and several
 @pytest.mark.parametrize("rows,width,inputs", [(250, 384, 345), (256, 128, 850), (249, 256, 2045)])

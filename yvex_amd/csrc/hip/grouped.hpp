@@ -4,6 +4,7 @@
 
 #include "common.hpp"
 #include "launch.hpp"
+#include "lds_copy.hpp"
 
 namespace yvex {
 
@@ -156,16 +157,36 @@ static inline void fill_down_problem(GroupedProblem &p, const yvex_hip_expert_we
 bool iq2_sweep_supported(unsigned qtype, unsigned width, unsigned out_rows, unsigned long long pairs, bool image);
 int launch_iq2_sweep(const GroupedArgs &a, unsigned qtype, bool fused, bool image, hipStream_t stream);
 
+// Pairs behind a bucket's whole 64-pair tiles that are the few-pair kernels' (rows16.hip), by the same rule there and
+// in the 64-pair kernels. A tile of theirs takes `few`. Where that leaves the 64-pair kernels with nothing but a few
+// buckets' single tiles, two tiles of theirs take those too: a launch of the 64-pair kernels is one tile's time however
+// few it holds (54 us of gate/up and 28 us of Q2_K down rows at width 4096 for one bucket or sixteen), a bucket in two
+// tiles 2.6 and 1.5 us of the whole device. Two tiles in every bucket of 256 are the slower way: 665 us
+// against 600 (width 4096, 24 pairs), 1148 against 935 (7168, fourteen); and beside a launch that is long anyway
+// they gain nothing (1111 uneven rows of Q4_K 2570 us without, 2650 with). Every thread of a block calls this, a thread a
+// bucket, those without one with 0; `lds` is the address of four words of LDS that hold nothing (the kernels leave no
+// room for static LDS).
+constexpr unsigned kFewPairSeconds = 16u;
+__device__ __forceinline__ unsigned few_pair_limit(unsigned few, unsigned long long population, unsigned lds)
+{
+    const unsigned seconds = (unsigned)__popcll(__ballot(population > few && population <= 2u * few));
+    const unsigned members = __ballot(population > 2u * few) ? kFewPairSeconds + 1u : seconds, wave = threadIdx.x >> 6;
+    if ((threadIdx.x & 63u) == 0u && wave < 4u) lds_write_u32(lds + 4u * wave, members);
+    __syncthreads();
+    const unsigned all = lds_read_u32(lds) + lds_read_u32(lds + 4u) + lds_read_u32(lds + 8u) + lds_read_u32(lds + 12u);
+    return all <= kFewPairSeconds ? 2u * few : few;
+}
+
 // Row-batch expert kernels on the int8 matrix cores (rows_q4k.hip): Q4_K weights, fused gate/up
-// or a plain projection; Q2_K weights, a plain projection (the down experts). A bucket's last tile of
-// up to `left` pairs is left to the kernels below.
+// or a plain projection; Q2_K weights, a plain projection (the down experts). A bucket's last tile is left to
+// the kernels below where few_pair_limit says so.
 int launch_q4k_rows_grouped(const GroupedProblem &problem, unsigned qtype, bool fused, uint64_t width,
-                            uint64_t out_rows, unsigned left, double limit, int *status, hipStream_t stream);
+                            uint64_t out_rows, unsigned few, double limit, int *status, hipStream_t stream);
 
 // The same problems where few pairs meet (rows16.hip): IQ2_XXS (canonical bytes, or the sweep image) and
 // Q4_K rows, fused gate/up or plain; Q2_K rows, plain. The first: pairs of a full tile, 0 for a problem
 // the kernels do not serve. The second serves whole buckets (`behind` 0), or what a bucket holds
-// behind whole tiles of `behind` pairs where that fits one tile; a plain projection's sums are rounded
+// behind whole tiles of `behind` pairs where few_pair_limit admits that; a plain projection's sums are rounded
 // to bfloat16 where `round` says so.
 unsigned rows16_tokens(const GroupedProblem &problem, unsigned qtype, bool image, bool fused, uint64_t width,
                        uint64_t out_rows);

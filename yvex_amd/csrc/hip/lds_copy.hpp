@@ -18,6 +18,15 @@ __device__ __forceinline__ void lds_write_uint4(unsigned address, uint4 v)
     (void)v;
 #endif
 }
+__device__ __forceinline__ void lds_write_v4i(unsigned address, v4i v)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    *reinterpret_cast<__attribute__((address_space(3))) v4i *>(address) = v;
+#else
+    (void)address;
+    (void)v;
+#endif
+}
 __device__ __forceinline__ void lds_write_uint2(unsigned address, uint2 v)
 {
 #if defined(__HIP_DEVICE_COMPILE__)

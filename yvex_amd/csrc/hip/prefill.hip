@@ -93,7 +93,7 @@ struct MfmaArgs {
     int *status;
     int plain_output;        // plain projection: outputs stay fp32 instead of being rounded to bf16
     int image;               // weights are the sweep image (72-byte records) instead of canonical bytes
-    unsigned left;           // a bucket's last tile of up to this many pairs is not this launch's (rows16.hip)
+    unsigned few;            // pairs of a tile of the few-pair kernel (rows16.hip), which has a part of the buckets' last tiles
 };
 
 __device__ __forceinline__ void mfma_tables_fill()
@@ -653,7 +653,7 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
         const unsigned lane = tid & 63u, wave = tid >> 6;
         const unsigned full = tid < 256u ? (unsigned)(population_here / kTileTokens) : 0u;
         const unsigned rest = tid < 256u ? (unsigned)(population_here % kTileTokens) : 0u;
-        const unsigned cls = rest <= a.left ? 2u : rest > 32u ? 0u : 1u;
+        const unsigned cls = rest <= few_pair_limit(a.few, population_here, kTrashBase + 48u) ? 2u : rest > 32u ? 0u : 1u;
         unsigned inclusive = full;
 #pragma unroll
         for (int offset = 1; offset < 64; offset <<= 1) {
@@ -829,9 +829,9 @@ static int launch_mfma(const MfmaArgs &a, hipStream_t stream)
 }
 
 // Expert matrices against the buckets of a worklist. The few-pair kernels (rows16.hip) take what a
-// bucket holds behind its whole 64-pair tiles if that fits one of their tiles (12 pairs at width 7168, 16 up to about 5000): such a tile
-// takes them 1.4 us of the whole device for the 2 x 2048 x 4096 IQ2_XXS rows of an expert, and the 64-pair
-// kernels, which pay for 32 token columns, 2.3 us; with two of theirs (from 17 pairs on, 2.8 us) it
+// bucket holds behind its whole 64-pair tiles if that fits one of their tiles (12 pairs at width 7168, 16 up to about 5000; two tiles
+// where few_pair_limit says so): such a tile takes them 1.3 us of the whole device for the 2 x 2048 x 4096 IQ2_XXS
+// rows of an expert, and the 64-pair kernels, which pay for 32 token columns, 2.3 us; with two of theirs (2.6 us) it
 // is the other way round. A matrix that is alone (no worklist) is theirs where they come out at one round of
 // their waves: 16 superblocks take 22 to 31 us then, and 45 us as 64-pair items, which are fewer than the
 // compute units up to 1024 rows (4096 x 4096 IQ2_XXS by 128 rows 44 -> 24 us, 2048 x 7168 69 -> 35; 7168 x
@@ -853,7 +853,7 @@ template <bool FUSED_UP>
 static int launch_rows(MfmaArgs &a, unsigned qtype, hipStream_t stream)
 {
     const RowsPlan plan = plan_rows(a.pr, qtype, FUSED_UP, a.image, a.width, a.out_rows);
-    a.left = plan.few;
+    a.few = plan.few;
     if (plan.many) {
         const int rc = qtype == QT_IQ2_XXS
             ? launch_mfma<FUSED_UP>(a, stream)

@@ -10,20 +10,22 @@
 //     wave waits for another: twelve waves a workgroup (eight for Q4_K and Q2_K rows) cover each
 //     other's latency;
 //   * a wave owns 32 weight rows (16 gate rows and the matching up rows when the SwiGLU is
-//     fused) and walks them superblock by superblock, records coming straight into registers
-//     ahead of their use, across row units as well;
+//     fused) and walks them superblock by superblock, their bytes loaded in runs ahead of their use (Run16 below),
+//     across row units as well;
 //   * the products are V_MFMA_I32_16X16X64_I8: lane (r, q) = (lane % 16, lane / 16) owns weight
 //     row r and a quarter of the superblock, four K chunks of sixteen values, in an order of K
 //     that is the format's own (both operands follow it). One B fragment serves both row tiles.
+//   * IQ2_XXS table lookups run one step (a K chunk of a row tile) ahead of their use, the next superblock's
+//     first ones ahead of this one's scaling; the scaling starts from sums that are floats already (kBias);
 //   * tiles times row units, in order, are cut into one piece of equal length a workgroup (short
 //     ones end with their tiles); the waves of a workgroup draw units of its piece from a counter.
-// Measured (256 experts, uniform routing; the row-batch kernels before, these after): gate/up of 4096 x 2048
-// IQ2_XXS, eight pairs an expert, 620 -> 357 us, Q2_K down 358 -> 196; 7168 x 2048 IQ2_XXS, six pairs, 890 ->
-// 608 and 503 -> 307; Q4_K 1115 -> 950 and 624 -> 509 (4.5 TB/s). IQ2_XXS has no pipe full (counters, 4096 x 2048 by
-// eight pairs, 358 us: 1.21 GB or 3.4 TB/s, vector ALU 62 % busy, LDS 31 %, matrix cores 16 %; a wave waits for data
-// 38 % of its time and for its turn to issue 29 %): load latency that three waves a SIMD do not cover, and
-// more do not fit the registers. Coalescing four lanes to a row and passing
-// the records through LDS, requesting four superblocks ahead, eight or sixteen waves (spills) were no faster.
+// Measured (256 experts, uniform routing; lanes loading their own records before, runs after): gate/up of 4096 x 2048
+// IQ2_XXS, nine pairs an expert, 370 -> 325 us, Q2_K down 208 -> 198; 7168 x 2048 IQ2_XXS, eight pairs, 592 -> 580 and
+// 312 -> 292; Q4_K 947 -> 860 and 535 -> 505. Loads of the old kind with nothing computed took 314 us for the first of
+// these (3.8 TB/s), in runs 209 (5.8). What bounds the IQ2_XXS rows now is the vector ALU: 237 instructions a wave and
+// superblock at 4.7 cycles each with three waves a SIMD, 1190 of 1310 to 1490 cycles; the rest is the
+// ends of tiles that do not fit the LDS together, where waves wait for each other. (Eight waves: two a SIMD, 5.0 cycles an
+// instruction, 3 % behind; units cut at whole rounds of the waves: 1 % behind.)
 // The arithmetic is that of the kernels named above, term by term: int8 limbs whose product sums
 // are exact, one float term a superblock, added in double in superblock order, rounded to float
 // once, so all kernel families publish the same bits.
@@ -46,6 +48,51 @@ constexpr unsigned kBatchTiles = 8u;                      // tiles in LDS at a t
 constexpr unsigned kLds16 = 160u * 1024u;
 constexpr unsigned kIq2Image = 0x100u;                    // IQ2_XXS rows as the sweep image (no format number)
 
+// How weight bytes arrive: a run is the bytes of S superblocks of a row: pieces of sixteen bytes that hold codes, at the
+// offsets that a lane's record begins at, and what else the superblocks have. The lanes of a load take consecutive
+// pieces of consecutive rows, few cache lines an instruction (a lane loading its own record touches another
+// row's lines than its neighbour, and the memory pipeline takes about two cycles a line). The pieces of sixteen
+// rows pass through a window of LDS of the wave's own, piece k of row r at slot r ^ swizzle(k) of line k: writes of
+// neighbouring rows and reads of sixteen both spread over the banks.
+// IQ2_XXS runs of one superblock have their windows in the halves of the table entries from 128 on that hold no sign
+// selectors, half the banks: without LDS of their own twelve pairs fit behind the tables at width 7168 (eight with it). Up to
+// width 4096, where sixteen fit either way, the image comes two superblocks at a time through windows of their own:
+// a load touches half the lines and all banks serve it (256 experts of nine pairs, gate/up of 4096 x 2048 325 us, 349
+// one at a time; the other way round at 7168, ten pairs: 585, and 924 in the 64-pair kernels).
+template <unsigned QT, unsigned S> struct Run16 {
+    static constexpr bool kIq2 = QT == QT_IQ2_XXS || QT == kIq2Image, kAmongTables = kIq2 && S == 1u;
+    static constexpr unsigned kPieces = (QT == QT_Q4_K ? 8u : 4u) * S;
+    static constexpr unsigned kRows = 64u / kPieces, kLoads = 16u / kRows;      // of a load, for sixteen rows
+    // behind the codes: Q4_K the superblock's first sixteen bytes, Q2_K scales, then d and dmin, of both row tiles
+    static constexpr unsigned kExtra = 256u * kPieces, kWords = kExtra + 512u * S;
+    static constexpr unsigned kWindow = kIq2 ? 2048u : kExtra + (QT == QT_Q4_K ? 512u : 640u * S);
+    // Canonical IQ2_XXS superblocks are 66 bytes and rows whole dwords: an odd one's codes start on a dword, an even
+    // one's two bytes into one, where the pieces start on the dword before.
+    __device__ static __forceinline__ unsigned offset(unsigned run)
+    {
+        if constexpr (QT == QT_IQ2_XXS) return 66u * run + 2u * (run & 1u);
+        else return S * (QT == QT_Q4_K ? 144u : QT == QT_Q2_K ? 84u : 72u) * run;
+    }
+    __device__ static __forceinline__ unsigned piece(unsigned k)
+    {
+        if constexpr (QT == kIq2Image) return 36u * (k >> 1) + 16u * (k & 1u) + 4u;
+        else if constexpr (QT == QT_IQ2_XXS) return 16u * k;
+        else if constexpr (QT == QT_Q4_K) return 16u * k + 16u;
+        else return 84u * (k >> 2) + 16u * (k & 3u) + 16u;
+    }
+    __device__ static __forceinline__ unsigned place(unsigned window, unsigned k, unsigned row)
+    {
+        if constexpr (kAmongTables) {
+            const unsigned slot = row ^ (4u * k);
+            return window + 512u * k + 256u * (slot >> 3) + 16u * (slot & 7u);
+        } else {
+            // (a Q4_K lane reads pieces 2 q and 2 q + 1)
+            const unsigned swizzle = QT == QT_Q4_K ? 8u * (k >> 2) + 4u * (k & 1u) + (k & 2u) : 16u / kPieces * k;
+            return window + 256u * k + 16u * (row ^ swizzle);
+        }
+    }
+};
+
 // LDS map (byte addresses; the dynamic block starts at LDS address 0). The IQ2_XXS tables come
 // first: entry e owns the 256 bytes at 256 e, sixteen replicas of the level codes of codebook
 // entry e in the first half; the second halves hold the sign selectors of fields 0-127, then the
@@ -59,7 +106,7 @@ constexpr unsigned kIq2Image = 0x100u;                    // IQ2_XXS rows as the
 // the other (the two are OR-ed): 2.3 cycles an instruction instead of 4.0, measured in a loop of such
 // reads. The payload stands piece-major, [superblock][piece][token slot] with a multiple of four
 // slots: 4.1 cycles instead of the 8.0 of token rows with XOR-ed piece positions.
-template <unsigned QT> struct Map16 {
+template <unsigned QT, unsigned S> struct Map16 {
     static constexpr bool kIq2 = QT == QT_IQ2_XXS || QT == kIq2Image;
     static constexpr unsigned kWaves = kIq2 ? 12u : 8u;
     static constexpr unsigned kThreads = 64u * kWaves;
@@ -69,7 +116,15 @@ template <unsigned QT> struct Map16 {
     static constexpr unsigned kDrawn = kMisc + 64u, kBatch = kMisc + 68u; // units drawn; {tiles, units, units passed}
     static constexpr unsigned kTiles = kMisc + 112u;                      // Tile16 of every tile at hand
     static constexpr unsigned kScratch = kTiles + kBatchTiles * 32u;      // Q4_K, Q2_K: [wave][tile][d, dmin][16] f32
-    static constexpr unsigned kAreas = (kScratch + (kIq2 ? 0u : kWaves * 256u) + 255u) & ~255u;
+    // a run of the waves' rows
+    static constexpr bool kAmongTables = Run16<QT, S>::kAmongTables;
+    static constexpr unsigned kUnused = 128u * 256u + 128u;               // first of the unused half entries of the tables
+    static constexpr unsigned kBehind = (kScratch + (kIq2 ? 0u : kWaves * 256u) + 255u) & ~255u;
+    static constexpr unsigned kWindows = kAmongTables ? kUnused : kBehind;
+    // IQ2_XXS, in unused half entries: the words before the halves of the image's records (canonical: the one dword of
+    // a superblock that its pieces leave out), [row][half]; then the waves' row scales, [tile][16] f32
+    static constexpr unsigned kHeads = kUnused + (kAmongTables ? kWaves * 2048u : 0u), kRowScales = kHeads + kWaves * S * 256u;
+    static constexpr unsigned kAreas = kBehind + (kAmongTables ? 0u : kWaves * Run16<QT, S>::kWindow);
     // minimum operands of a superblock: Q4_K lo | hi limbs of a token's pair sums, Q2_K three pieces a token
     static constexpr unsigned kSumBytes = kIq2 ? 0u : QT == QT_Q4_K ? 256u : 768u;
     __host__ __device__ static constexpr unsigned area_bytes(unsigned blocks, unsigned slots)
@@ -85,7 +140,7 @@ struct Rows16Args {
     unsigned tokens;         // of a full tile
     bool round;              // a plain projection's sums are rounded to bfloat16
     unsigned behind;         // what is served of a bucket: all of it (0), or its pairs behind whole tiles of
-                             // this many, where they fit one tile here
+                             // this many, where few_pair_limit admits them
     double limit;
     int *status;
 };
@@ -99,68 +154,65 @@ struct Tile16 {
     unsigned start, first_unit, expert, pair0, live, area;
 };
 
-// ---- formats: a lane's bytes of one row's superblock ----
-template <unsigned QT> struct Record16;
+// ---- formats: a lane's bytes of one row's superblock, out of the wave's window ----
+template <unsigned QT, unsigned S> struct Record16;
 
-template <> struct Record16<kIq2Image> {
-    static constexpr unsigned kBytes = 72u;
+template <unsigned S> struct Record16<kIq2Image, S> {
     unsigned head;           // fp16 scale | the four group scales of the lane's half << 16
     v4i body;                // groups 2 q and 2 q + 1: codebook bytes, sign bytes
-    __device__ __forceinline__ void load(const unsigned char *base, unsigned row, bool, const Lane16 &l)
+    __device__ __forceinline__ void read(unsigned window, unsigned heads, unsigned, unsigned s, const Lane16 &l)
     {
-        head = *reinterpret_cast<const unsigned *>(base + (row + 36u * (l.q >> 1)));
-        body = *reinterpret_cast<const v4i_dword *>(base + (row + (36u * (l.q >> 1) + 16u * (l.q & 1u) + 4u)));
+        const unsigned word = 2u * (S * l.r + s) + (l.q >> 1);
+        head = lds_read_u32(heads + 256u * (word >> 5) + 4u * (word & 31u));
+        body = lds_read_v4i(Run16<kIq2Image, S>::place(window, 4u * s + l.q, l.r));
     }
 };
 
-// Canonical superblocks are 66 bytes and rows whole dwords, so the lane's sixteen bytes start two bytes
-// into a dword in even superblocks and on one in odd ones: a window of five dwords, of which the odd
-// superblocks use four (their fifth, which may lie behind the matrix, repeats the fourth).
-template <> struct Record16<QT_IQ2_XXS> {
-    static constexpr unsigned kBytes = 66u;
+// A window of five dwords of which odd superblocks use four.
+template <unsigned S> struct Record16<QT_IQ2_XXS, S> {
     v4i window;
     unsigned fifth;
-    unsigned short scale;
-    __device__ __forceinline__ void load(const unsigned char *base, unsigned row, bool odd, const Lane16 &l)
+    unsigned scale;
+    __device__ __forceinline__ void read(unsigned at, unsigned heads, unsigned, unsigned parity, const Lane16 &l)
     {
-        const unsigned at = row + (odd ? 2u : 0u) + 16u * l.q;
-        window = *reinterpret_cast<const v4i_dword *>(base + at);
-        fifth = *reinterpret_cast<const unsigned *>(base + (at + (odd ? 12u : 16u)));
-        scale = *reinterpret_cast<const unsigned short *>(base + row);
+        using Run = Run16<QT_IQ2_XXS, S>;
+        window = lds_read_v4i(Run::place(at, l.q, l.r));
+        fifth = parity ? 0u : lds_read_u32(l.q == 3u ? heads + 4u * l.r : Run::place(at, l.q + 1u, l.r));
+        scale = parity ? lds_read_u16(heads + 4u * l.r + 2u) : lds_read_u16(Run::place(at, 0u, l.r));
     }
 };
 
-template <> struct Record16<QT_Q4_K> {
-    static constexpr unsigned kBytes = 144u;
+template <unsigned S> struct Record16<QT_Q4_K, S> {
     v4i head;                // d | dmin << 16, the 12 scale bytes
     v4i codes[2];            // the 32 bytes of sub-blocks 2 q (low nibbles) and 2 q + 1
-    __device__ __forceinline__ void load(const unsigned char *base, unsigned row, bool, const Lane16 &l)
+    __device__ __forceinline__ void read(unsigned window, unsigned, unsigned u, unsigned, const Lane16 &l)
     {
-        head = *reinterpret_cast<const v4i_dword *>(base + row);
-        codes[0] = *reinterpret_cast<const v4i_dword *>(base + (row + (32u * l.q + 16u)));
-        codes[1] = *reinterpret_cast<const v4i_dword *>(base + (row + (32u * l.q + 32u)));
+        using Run = Run16<QT_Q4_K, S>;
+        head = lds_read_v4i(window + Run::kExtra + 256u * u + 16u * l.r);
+        codes[0] = lds_read_v4i(Run::place(window, 2u * l.q, l.r));
+        codes[1] = lds_read_v4i(Run::place(window, 2u * l.q + 1u, l.r));
     }
     __device__ __forceinline__ unsigned scales_word() const { return (unsigned)head[0]; }
 };
 
-template <> struct Record16<QT_Q2_K> {
-    static constexpr unsigned kBytes = 84u;
+template <unsigned S> struct Record16<QT_Q2_K, S> {
     v4i scales;              // (scale | minimum << 4) of the sixteen sub-blocks
     v4i codes;               // bytes 16 (q % 2) .. + 15 of code half q / 2
     unsigned dd;             // d | dmin << 16
-    __device__ __forceinline__ void load(const unsigned char *base, unsigned row, bool, const Lane16 &l)
+    __device__ __forceinline__ void read(unsigned window, unsigned, unsigned u, unsigned s, const Lane16 &l)
     {
-        scales = *reinterpret_cast<const v4i_dword *>(base + row);
-        codes = *reinterpret_cast<const v4i_dword *>(base + (row + (16u * l.q + 16u)));
-        dd = *reinterpret_cast<const unsigned *>(base + (row + 80u));
+        using Run = Run16<QT_Q2_K, S>;
+        scales = lds_read_v4i(window + Run::kExtra + 256u * (S * u + s) + 16u * l.r);
+        codes = lds_read_v4i(Run::place(window, 4u * s + l.q, l.r));
+        dd = lds_read_u32(window + Run::kWords + 64u * (S * u + s) + 4u * l.r);
     }
     __device__ __forceinline__ unsigned scales_word() const { return dd; }
 };
 
-template <unsigned QT, bool FUSED>
-__global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args a)
+template <unsigned QT, bool FUSED, unsigned S>
+__global__ __launch_bounds__((Map16<QT, S>::kThreads)) void rows16_kernel(Rows16Args a)
 {
-    using M = Map16<QT>;
+    using M = Map16<QT, S>;
     constexpr bool kIq2 = M::kIq2;
     extern __shared__ __align__(16) unsigned char rows16_lds[];
     if (lds_address_of(rows16_lds) != 0u) {      // operands are addressed by absolute LDS offsets
@@ -179,7 +231,8 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
     if (tid < 256u && tid < buckets) population_here = fixed ? pr.pairs : pr.bucket_populations[tid];
     {
         const unsigned long long served = a.behind ? population_here % a.behind : population_here;
-        const unsigned tiles = tid >= 256u || (a.behind && served > a.tokens) ? 0u
+        const unsigned limit = a.behind ? few_pair_limit(a.tokens, population_here, M::kMisc + 16u) : 0u;
+        const unsigned tiles = tid >= 256u || (a.behind && served > limit) ? 0u
                                                                              : (unsigned)((served + a.tokens - 1u) / a.tokens);
         unsigned inclusive = tiles;
 #pragma unroll
@@ -231,9 +284,23 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
         if (tid < 256u)
             lds_write_uint4(M::kLimbs + 16u * tid, iq2_limb_words(tid >> 4));
     }
-    const unsigned scratch = kIq2 ? (160u + wave) * 256u + 128u : M::kScratch + wave * 256u;
+    const unsigned scratch = (kIq2 ? M::kRowScales : M::kScratch) + wave * 256u;
     auto source_of = [&](unsigned long long ordered) { return pr.order ? pr.order[ordered] : ordered; };
 
+    using Run = Run16<QT, S>;
+    const unsigned window = uniform(M::kWindows + wave * Run::kWindow), heads = uniform(M::kHeads + wave * S * 256u);
+    // the lane's pieces of sixteen rows' run: piece lane % kPieces of every kRows-th row; the rest of its bytes
+    unsigned place[Run::kLoads], piece_at[Run::kLoads], head_at = 0u;
+#pragma unroll
+    for (unsigned i = 0; i < Run::kLoads; ++i) {
+        const unsigned k = lane % Run::kPieces, row = Run::kRows * i + lane / Run::kPieces;
+        place[i] = Run::place(window, k, row);
+        piece_at[i] = row * (unsigned)pr.row_bytes + Run::piece(k);
+    }
+    if constexpr (QT == kIq2Image) head_at = (lane / (2u * S) & 15u) * (unsigned)pr.row_bytes + 36u * (lane % (2u * S));
+    if constexpr (QT == QT_IQ2_XXS) head_at = l.r * (unsigned)pr.row_bytes;
+    if constexpr (QT == QT_Q4_K) head_at = (FUSED ? l.r : lane & 31u) * (unsigned)pr.row_bytes;
+    if constexpr (QT == QT_Q2_K) head_at = (l.r + 16u * (lane / (16u * S) & 1u)) * (unsigned)pr.row_bytes + 84u * (l.q & (S - 1u));
     while (at < end) {
         // ---- the next tiles of the piece, as many as fit the LDS together: between them nobody
         // waits for anybody ----
@@ -254,8 +321,8 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
                     else high = middle;
                 }
                 const unsigned long long population = fixed ? pr.pairs : pr.bucket_populations[low];
-                const unsigned long long inside = a.behind ? population - population % a.behind
-                    : (unsigned long long)(tile - lds_read_u32(M::kStarts + 4u * low)) * a.tokens;
+                const unsigned long long inside = (a.behind ? population - population % a.behind : 0ull) +
+                                                  (unsigned long long)(tile - lds_read_u32(M::kStarts + 4u * low)) * a.tokens;
                 const unsigned long long pair0 = (fixed ? 0ull : pr.bucket_offsets[low]) + inside;
                 const unsigned long long expert = fixed ? 0ull : pr.expert_ids[low];
                 if (inside >= population || expert >= pr.experts || pair0 + (population - inside) > pr.pairs) {
@@ -362,25 +429,25 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
             if (lane == 0u) drawn = atomicAdd(reinterpret_cast<unsigned *>(rows16_lds + M::kDrawn), 1u);
             return uniform(drawn);
         };
-        // where a unit's rows lie: its expert's matrices and the lane's row of either row tile
+        // where the row tiles of a unit lie (a ragged edge takes rows that the unit before has, too: the same bits)
         struct Rows {
             const unsigned char *base[2];
-            unsigned row[2];
+        };
+        auto first_row = [&](const Tile16 &t, unsigned unit) {
+            return min((t.first_unit + unit - t.start) * kUnitRows, a.out_rows - kUnitRows);
         };
         unsigned tile_index = 0u;                               // of the unit drawn last (they ascend)
         Tile16 drawn_tile = tile_of(0u);
+        unsigned tile_end = tiles > 1u ? uniform(lds_read_u32(M::kTiles + 32u)) : drawable;
         auto locate = [&](unsigned unit) {
-            while (tile_index + 1u < tiles && uniform(lds_read_u32(M::kTiles + 32u * (tile_index + 1u))) <= unit) ++tile_index;
-            drawn_tile = tile_of(tile_index);
-            Rows rows;
-            rows.base[0] = pr.gate + drawn_tile.expert * pr.expert_bytes;
-            rows.base[1] = FUSED ? pr.up + drawn_tile.expert * pr.up_expert_bytes : rows.base[0];
-#pragma unroll
-            for (unsigned u = 0; u < 2u; ++u) {
-                unsigned row = (drawn_tile.first_unit + unit - drawn_tile.start) * kUnitRows + (FUSED ? 0u : 16u * u) + l.r;
-                if (row >= a.out_rows) row = a.out_rows - 1u;       // a ragged edge repeats the last row
-                rows.row[u] = row * (unsigned)pr.row_bytes;
+            while (unit >= tile_end) {
+                drawn_tile = tile_of(++tile_index);
+                tile_end = tile_index + 1u < tiles ? uniform(lds_read_u32(M::kTiles + 32u * (tile_index + 1u))) : drawable;
             }
+            const unsigned long long row = (unsigned long long)first_row(drawn_tile, unit) * pr.row_bytes;
+            Rows rows;
+            rows.base[0] = pr.gate + drawn_tile.expert * pr.expert_bytes + row;
+            rows.base[1] = FUSED ? pr.up + drawn_tile.expert * pr.up_expert_bytes + row : rows.base[0] + 16u * pr.row_bytes;
             return rows;
         };
         unsigned unit = wave;
@@ -390,25 +457,56 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
         unsigned next = draw();
         Rows ahead = here;
         if (next < drawable) ahead = locate(next);
-        Record16<QT> rec[2][2];                  // [parity of the stream][row tile]
-        auto request = [&](Record16<QT> (&into)[2], unsigned sb) {
-            const bool past = sb >= a.blocks;
-            const unsigned block = (past ? sb - a.blocks : sb) * Record16<QT>::kBytes;
+        // the run that comes next
+        struct Staged {
+            v4i piece[2][Run::kLoads], head;
+            unsigned word[2];
+        } staged;
+        const unsigned runs = a.blocks / S;
+        auto request = [&](unsigned run) {       // of the unit at hand, or behind its end of the one drawn before
+            const bool past = run >= runs;
+            const unsigned here_run = past ? run - runs : run, from = Run::offset(here_run);
+            const unsigned char *const base[2] = {(past ? ahead.base[0] : here.base[0]) + from,
+                                                  (past ? ahead.base[1] : here.base[1]) + from};
 #pragma unroll
-            for (unsigned u = 0; u < 2u; ++u)
-                into[u].load(past ? ahead.base[u] : here.base[u], (past ? ahead.row[u] : here.row[u]) + block,
-                             ((past ? sb - a.blocks : sb) & 1u) != 0u, l);
+            for (unsigned u = 0; u < 2u; ++u) {
+                if constexpr (kIq2)
+                    staged.word[u] = *reinterpret_cast<const unsigned *>(base[u] + (QT == kIq2Image ? 0 : here_run & 1u ? -4 : 64) + head_at);
+#pragma unroll
+                for (unsigned i = 0; i < Run::kLoads; ++i)
+                    staged.piece[u][i] = *reinterpret_cast<const v4i_dword *>(base[u] + piece_at[i]);
+            }
+            if constexpr (QT == QT_Q4_K) {
+                // gate heads on the lanes of the even quarters, up heads on the others (plain rows: of both row tiles)
+                const unsigned long long to_up = FUSED && (l.q & 1u) ? (unsigned long long)(base[1] - base[0]) : 0ull;
+                staged.head = *reinterpret_cast<const v4i_dword *>(base[0] + to_up + head_at);
+            }
+            if constexpr (QT == QT_Q2_K) {
+                staged.head = *reinterpret_cast<const v4i_dword *>(base[0] + head_at);
+                staged.word[0] = *reinterpret_cast<const unsigned *>(base[0] + (head_at + 80u));
+            }
         };
-        request(rec[0], 0u);
-        request(rec[1], 1u);
+        request(0u);
 
-        unsigned column, frag_pitch, frag_step, frag_at, sb = 0u;
+        // where a tile's activations stand for a lane. Lanes behind the last token, whose results nobody takes, read
+        // what their neighbours read, with which they share the banks' cycle.
+        struct Columns {
+            unsigned column, pitch, frag_at, scale_at;     // pitch: from piece to piece
+        };
+        auto columns_of = [&](const Tile16 &t) {
+            const bool lives = l.r < t.live;
+            const unsigned q = lives ? l.q : l.q & 2u;
+            Columns c;
+            c.column = lives ? l.r : 0u;
+            c.pitch = 16u * ((t.live + 3u) & ~3u);
+            c.frag_at = t.area + payload_at + (lives ? l.r : l.r & 3u) * 16u + c.pitch * (QT == QT_Q2_K ? 8u * (q >> 1) + (q & 1u) : 4u * q);
+            c.scale_at = t.area + scales_at + 4u * c.column;
+            return c;
+        };
+        Columns c = columns_of(tile), c_ahead = columns_of(drawn_tile);
+        unsigned sb = 0u;
         double acc[2][4];
-        auto begin = [&]() {                     // the unit at hand, `tile`
-            column = l.r < tile.live ? l.r : 0u;                    // padding repeats the first token
-            frag_pitch = 16u * ((tile.live + 3u) & ~3u);            // from piece to piece
-            frag_step = QT == QT_Q2_K ? 2u * frag_pitch : frag_pitch;       // from K chunk to K chunk
-            frag_at = tile.area + payload_at + column * 16u + frag_pitch * (QT == QT_Q2_K ? 8u * (l.q >> 1) + (l.q & 1u) : 4u * l.q);
+        auto begin = [&]() {                     // the unit at hand
             sb = 0u;
 #pragma unroll
             for (unsigned u = 0; u < 2u; ++u)
@@ -416,112 +514,174 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
                 for (unsigned i = 0; i < 4u; ++i) acc[u][i] = 0.0;
         };
         begin();
-        const v4i zero = {0, 0, 0, 0};
+        // The IQ2_XXS limbs' sums start from the bits of 1.5 * 2^23: |sum| stays below 2^22 (low limbs 256 * 64 * 127), so
+        // a result's bits are the float 1.5 * 2^23 + sum.
+        constexpr float kBias = 12582912.0f;
+        const int start_bits = kIq2 ? __float_as_int(kBias) : 0;
+        const v4i start = {start_bits, start_bits, start_bits, start_bits}, zero = {0, 0, 0, 0};
 
-        auto superblock = [&](Record16<QT> (&w)[2]) {
-            v4i lo[2] = {zero, zero}, hi[2] = {zero, zero};
+        // A superblock's sums (int32, exact) and the scales that make its float terms of them.
+        struct Sums {
+            v4i lo[2], hi[2], min_lo[2], min_hi[2];
+        };
+        struct Scales {
+            float token;
+            v4i d[2], dmin[2];
+        };
+        auto scales_here = [&]() {
+            Scales r;
+            r.token = __uint_as_float(lds_read_u32(c.scale_at + 64u * sb));
+#pragma unroll
+            for (unsigned u = 0; u < 2u; ++u) {
+                r.d[u] = lds_read_v4i(scratch + (kIq2 ? 64u : 128u) * u + 16u * l.q);
+                if constexpr (!kIq2) r.dmin[u] = lds_read_v4i(scratch + 128u * u + 64u + 16u * l.q);
+            }
+            return r;
+        };
+        auto settle = [&](const Sums &x, const Scales &r) {
+#pragma unroll
+            for (unsigned u = 0; u < 2u; ++u)
+#pragma unroll
+                for (unsigned i = 0; i < 4u; ++i) {
+                    if constexpr (kIq2) {
+                        // 128 hi - kBias is exact, and so the float of 128 hi + lo comes from one rounding
+                        const float sum = __builtin_fmaf(__int_as_float(x.hi[u][i]), 128.0f, -129.0f * kBias) + __int_as_float(x.lo[u][i]);
+                        const float term = __int_as_float(r.d[u][i]) * r.token * sum;      // each product rounded to float
+                        acc[u][i] += (double)term;
+                    } else {
+                        const int dot = QT == QT_Q2_K ? x.lo[u][i] : (x.hi[u][i] << 3) + x.lo[u][i];
+                        const int low = QT == QT_Q2_K ? x.min_lo[u][i] : (x.min_hi[u][i] << 7) + x.min_lo[u][i];
+                        const float left = (r.token * __int_as_float(r.d[u][i])) * (float)dot;
+                        const float right = (r.token * __int_as_float(r.dmin[u][i])) * (float)low;
+                        acc[u][i] += (double)(left - right);
+                    }
+                }
+        };
+
+        // IQ2_XXS: a superblock's table words and the lookups in flight.
+        // Lanes of odd quarters look signs up first.
+        const bool odd_quarter = QT == kIq2Image && (l.q & 1u) != 0u;
+        const unsigned first_lane = l.r * 8u + (odd_quarter ? 128u : 0u), second_lane = first_lane ^ 128u;
+        const unsigned lut_lane = M::kLimbs + l.r * 16u;
+        const unsigned nibble = 8u + 8u * (l.q & 1u);
+        unsigned first[2][2], second[2][2], words[2];            // [tile][group]: codebook and sign words
+        uint2 codes[2][2], signs[2][2];                          // [row tile][subgroup]
+        v4i limbs[2][2];                                         // [group & 1][tile]
+        v4i frag[kIq2 ? 2 : 4];
+        unsigned frag_at = c.frag_at, pitch = c.pitch;           // of the superblock that is ready
+        const unsigned chunk_pieces = QT == QT_Q2_K ? 2u : 1u;   // from K chunk to K chunk
+        auto lookup = [&](unsigned step) {                       // K chunk step / 2 of row tile step % 2
+            const unsigned m = step >> 1, u = step & 1u;
+            if (u == 0u) frag[m & 1u] = lds_read_v4i(frag_at + m * pitch);
+            // the scale of a group in bits 8-11
+            if ((m & 1u) == 0u) {
+                const unsigned field = QT == kIq2Image ? words[u] >> (nibble + 4u * (m >> 1)) : second[u][m >> 1] >> 20;
+                limbs[(m >> 1) & 1u][u] = lds_read_v4i((field & 0xf00u) | lut_lane);
+            }
+#pragma unroll
+            for (unsigned i = 0; i < 2u; ++i) {
+                const unsigned j = 2u * (m & 1u) + i, pick = 0x0c0c0400u + (j << 8), word = second[u][m >> 1];
+                codes[u][i] = lds_read_uint2(__builtin_amdgcn_perm(first[u][m >> 1], first_lane, pick));
+                // (the image's sign fields have bytes of their own, the canonical ones seven bits each)
+                signs[u][i] = lds_read_uint2(
+                    QT == kIq2Image ? __builtin_amdgcn_perm(word, second_lane, pick)
+                                    : ((j == 0u ? word << 8 : j == 1u ? word << 1 : word >> (7u * j - 8u)) & 0x7f00u) | second_lane);
+            }
+        };
+        // A superblock is next: its row scales where the lanes that will hold its sums find them, its first lookups.
+        auto ready = [&](const Record16<QT, S> (&w)[2], unsigned parity) {
             if constexpr (kIq2) {
-                // lanes of odd quarters look signs up first
-                const bool odd = QT == kIq2Image && (l.q & 1u) != 0u;
-                const unsigned first_lane = l.r * 8u + (odd ? 128u : 0u), second_lane = first_lane ^ 128u;
-                const unsigned lut_lane = M::kLimbs + l.r * 16u;
-                const unsigned nibble = 8u + 8u * (l.q & 1u);
-                unsigned first[2][2], second[2][2];              // [tile][group]: codebook and sign words
-                unsigned scale16[2];
 #pragma unroll
                 for (unsigned u = 0; u < 2u; ++u) {
+                    unsigned scale16;
                     if constexpr (QT == kIq2Image) {
-                        scale16[u] = w[u].head & 0xffffu;
+                        words[u] = w[u].head;
+                        scale16 = w[u].head & 0xffffu;
 #pragma unroll
                         for (unsigned g = 0; g < 2u; ++g) {
                             const unsigned grids = (unsigned)w[u].body[2u * g], aux = (unsigned)w[u].body[2u * g + 1u];
-                            first[u][g] = odd ? aux : grids;
-                            second[u][g] = odd ? grids : aux;
+                            first[u][g] = odd_quarter ? aux : grids;
+                            second[u][g] = odd_quarter ? grids : aux;
                         }
                     } else {
-                        scale16[u] = w[u].scale;
-                        const unsigned shift = sb & 1u ? 0u : 2u;
+                        scale16 = w[u].scale;
                         const unsigned d[5] = {(unsigned)w[u].window[0], (unsigned)w[u].window[1], (unsigned)w[u].window[2],
                                                (unsigned)w[u].window[3], w[u].fifth};
 #pragma unroll
                         for (unsigned g = 0; g < 2u; ++g) {
-                            first[u][g] = __builtin_amdgcn_alignbyte(d[2u * g + 1u], d[2u * g], shift);
-                            second[u][g] = __builtin_amdgcn_alignbyte(d[2u * g + 2u], d[2u * g + 1u], shift);
+                            first[u][g] = parity ? d[2u * g] : __builtin_amdgcn_alignbyte(d[2u * g + 1u], d[2u * g], 2u);
+                            second[u][g] = parity ? d[2u * g + 1u] : __builtin_amdgcn_alignbyte(d[2u * g + 2u], d[2u * g + 1u], 2u);
                         }
                     }
+                    lds_write_u32(scratch + 64u * u + 4u * l.r, __float_as_uint(0.125f * f16_bits_to_float(scale16)));
                 }
-#pragma unroll
-                for (unsigned u = 0; u < 2u; ++u)
-                    lds_write_u32(scratch + 64u * u + 4u * l.r, __float_as_uint(0.125f * f16_bits_to_float(scale16[u])));
-                uint2 codes[2][2][2], signs[2][2][2];            // [chunk & 1][tile][subgroup]
-                uint4 limbs[2][2];                               // [group & 1][tile]
-                v4i frag[2];
-                // the scale of a group in bits 8-11
-                auto limb_field = [&](unsigned u, unsigned g) -> unsigned {
-                    if constexpr (QT == kIq2Image) return w[u].head >> (nibble + 4u * g);
-                    else return second[u][g] >> 20;
-                };
-                auto lookup = [&](unsigned m) {
-                    frag[m & 1u] = lds_read_v4i(frag_at + m * frag_step);
-#pragma unroll
-                    for (unsigned u = 0; u < 2u; ++u) {
-#pragma unroll
-                        for (unsigned i = 0; i < 2u; ++i) {
-                            const unsigned pick = 0x0c0c0400u + ((2u * (m & 1u) + i) << 8);
-                            codes[m & 1u][u][i] =
-                                lds_read_uint2(__builtin_amdgcn_perm(first[u][m >> 1], first_lane, pick));
-                            // (the image's sign fields have bytes of their own, the canonical ones seven bits each)
-                            const unsigned j = 2u * (m & 1u) + i, word = second[u][m >> 1];
-                            signs[m & 1u][u][i] = lds_read_uint2(
-                                QT == kIq2Image ? __builtin_amdgcn_perm(word, second_lane, pick)
-                                                : ((j == 0u ? word << 8 : j == 1u ? word << 1 : word >> (7u * j - 8u)) & 0x7f00u) | second_lane);
-                        }
-                        if ((m & 1u) == 0u)
-                            limbs[(m >> 1) & 1u][u] = lds_read_uint4((limb_field(u, m >> 1) & 0xf00u) | lut_lane);
-                    }
-                };
                 lookup(0u);
-#pragma unroll
-                for (unsigned m = 0; m < 4u; ++m) {
-                    if (m < 3u) lookup(m + 1u);
-#pragma unroll
-                    for (unsigned u = 0; u < 2u; ++u) {
-                        const uint4 lw = limbs[(m >> 1) & 1u][u];
-                        v4i a_lo, a_hi;
-#pragma unroll
-                        for (unsigned i = 0; i < 4u; ++i) {
-                            const uint2 c = codes[m & 1u][u][i >> 1], s = signs[m & 1u][u][i >> 1];
-                            const unsigned selector = i & 1u ? c.y | s.y : c.x | s.x;
-                            a_lo[i] = (int)__builtin_amdgcn_perm(lw.y, lw.x, selector);
-                            a_hi[i] = (int)__builtin_amdgcn_perm(lw.w, lw.z, selector);
-                        }
-                        lo[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_lo, frag[m & 1u], lo[u], 0, 0, 0);
-                        hi[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_hi, frag[m & 1u], hi[u], 0, 0, 0);
-                    }
-                }
-                request(w, sb + 2u);
-                const float ts = __uint_as_float(lds_read_u32(tile.area + scales_at + 64u * sb + 4u * column));
-#pragma unroll
-                for (unsigned u = 0; u < 2u; ++u) {
-                    const v4i rs = lds_read_v4i(scratch + 64u * u + 16u * l.q);
-#pragma unroll
-                    for (unsigned i = 0; i < 4u; ++i) {
-                        const int sum = (hi[u][i] << 7) + lo[u][i];
-                        const float term = __int_as_float(rs[i]) * ts * (float)sum;      // each product rounded to float
-                        acc[u][i] += (double)term;
-                    }
-                }
             } else {
-                // d and dmin of the rows, for the lanes that hold their sums
 #pragma unroll
                 for (unsigned u = 0; u < 2u; ++u) {
                     const unsigned dd = w[u].scales_word();
                     lds_write_u32(scratch + 128u * u + 4u * l.r, __float_as_uint(f16_bits_to_float(dd & 0xffffu)));
                     lds_write_u32(scratch + 128u * u + 64u + 4u * l.r, __float_as_uint(f16_bits_to_float(dd >> 16)));
                 }
-                v4i min_lo[2], min_hi[2];
+            }
+        };
+
+        // The staged run through the window into the lanes' records, and the one behind it requested.
+        Record16<QT, S> rec[S][2];
+        unsigned run = 0u;                       // of the unit at hand
+        auto turn_over = [&](unsigned behind, [[maybe_unused]] unsigned parity) {
+            if constexpr (QT == QT_Q4_K) lds_write_v4i(window + Run::kExtra + 16u * (lane & 31u), staged.head);
+            if constexpr (QT == QT_Q2_K) {
+                lds_write_v4i(window + Run::kExtra + 16u * (lane % (32u * S)), staged.head);
+                lds_write_u32(window + Run::kWords + 4u * (lane % (32u * S)), staged.word[0]);
+            }
+#pragma unroll
+            for (unsigned u = 0; u < 2u; ++u) {
+#pragma unroll
+                for (unsigned i = 0; i < Run::kLoads; ++i) lds_write_v4i(place[i], staged.piece[u][i]);
+                if constexpr (kIq2) lds_write_u32(heads + 256u * (S - 1u) * (lane >> 5) + 4u * (lane & (QT == kIq2Image ? 31u : 15u)), staged.word[u]);
+#pragma unroll
+                for (unsigned s = 0; s < S; ++s) rec[s][u].read(window, heads, u, QT == QT_IQ2_XXS ? parity : s, l);
+            }
+            request(behind);
+        };
+        // One superblock, an odd one by `parity`; `turn` if it is its run's last.
+        auto superblock = [&](const Record16<QT, S> (&record)[2], bool turn, unsigned parity) {
+            [[maybe_unused]] const Record16<QT, S> w[2] = {record[0], record[1]};
+            Sums x;
+#pragma unroll
+            for (unsigned u = 0; u < 2u; ++u) {
+                x.lo[u] = x.hi[u] = start;
+                x.min_lo[u] = x.min_hi[u] = zero;
+            }
+            if constexpr (kIq2) {
+#pragma unroll
+                for (unsigned step = 0; step < 8u; ++step) {
+                    const unsigned m = step >> 1, u = step & 1u;
+                    if (step < 7u) lookup(step + 1u);
+                    else if (turn) turn_over(run + 2u, parity ^ 1u);
+                    __builtin_amdgcn_sched_barrier(0);
+                    const v4i lw = limbs[(m >> 1) & 1u][u];
+                    v4i a_lo, a_hi;
+#pragma unroll
+                    for (unsigned i = 0; i < 4u; ++i) {
+                        const uint2 code = codes[u][i >> 1], sign = signs[u][i >> 1];
+                        const unsigned selector = i & 1u ? code.y | sign.y : code.x | sign.x;
+                        a_lo[i] = (int)__builtin_amdgcn_perm((unsigned)lw[1], (unsigned)lw[0], selector);
+                        a_hi[i] = (int)__builtin_amdgcn_perm((unsigned)lw[3], (unsigned)lw[2], selector);
+                    }
+                    x.lo[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_lo, frag[m & 1u], x.lo[u], 0, 0, 0);
+                    x.hi[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_hi, frag[m & 1u], x.hi[u], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+                const v4i sums = lds_read_v4i(tile.area + sums_at + M::kSumBytes * sb + (QT == QT_Q2_K ? 256u * (l.q < 2u ? l.q : 2u) : 0u)
+                                              + 16u * c.column);
+#pragma unroll
+                for (unsigned m = 0; m < 4u; ++m) frag[m] = lds_read_v4i(frag_at + m * chunk_pieces * pitch);
+                if (turn) turn_over(run + 2u, parity ^ 1u);
+                __builtin_amdgcn_sched_barrier(0);
                 if constexpr (QT == QT_Q4_K) {
-                    const v4i sums = lds_read_v4i(tile.area + sums_at + 256u * sb + 16u * column);
                     unsigned scales[2];
 #pragma unroll
                     for (unsigned u = 0; u < 2u; ++u) {
@@ -532,12 +692,11 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
                         // pair sums (dwords 0-1 of `sums`), then against the high ones (dwords 2-3)
                         const int mn0 = l.q ? 0 : (int)(s1 & 0x3f3f3f3fu);
                         const int mn1 = l.q ? 0 : (int)(((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u));
-                        min_lo[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v4i{mn0, mn1, 0, 0}, sums, zero, 0, 0, 0);
-                        min_hi[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v4i{0, 0, mn0, mn1}, sums, zero, 0, 0, 0);
+                        x.min_lo[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v4i{mn0, mn1, 0, 0}, sums, zero, 0, 0, 0);
+                        x.min_hi[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v4i{0, 0, mn0, mn1}, sums, zero, 0, 0, 0);
                     }
 #pragma unroll
                     for (unsigned m = 0; m < 4u; ++m) {
-                        const v4i frag = lds_read_v4i(frag_at + m * frag_step);
 #pragma unroll
                         for (unsigned u = 0; u < 2u; ++u) {
                             const unsigned sc = (scales[u] >> (8u * (m >> 1))) & 255u;
@@ -549,14 +708,13 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
                                 a_lo[i] = (int)low_limbs;
                                 a_hi[i] = (int)high_limbs;
                             }
-                            lo[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_lo, frag, lo[u], 0, 0, 0);
-                            hi[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_hi, frag, hi[u], 0, 0, 0);
+                            x.lo[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_lo, frag[m], x.lo[u], 0, 0, 0);
+                            x.hi[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_hi, frag[m], x.hi[u], 0, 0, 0);
                         }
                     }
                 } else {
                     // quarter 0 holds the minimums against the sums' low three bits, quarters 1 and 2 hold
                     // eight times the minimums against the two halves of the rest
-                    const v4i sums = lds_read_v4i(tile.area + sums_at + 768u * sb + 256u * (l.q < 2u ? l.q : 2u) + 16u * column);
                     unsigned scales[2][2];
 #pragma unroll
                     for (unsigned u = 0; u < 2u; ++u) {
@@ -566,51 +724,35 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
                             const unsigned four = ((unsigned)w[u].scales[i] >> 4) & 0x0f0f0f0fu;
                             mn[i] = (int)(l.q == 3u ? 0u : four << (l.q ? 3u : 0u));
                         }
-                        min_lo[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(mn, sums, zero, 0, 0, 0);
-                        min_hi[u] = zero;
+                        x.min_lo[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(mn, sums, zero, 0, 0, 0);
 #pragma unroll
                         for (unsigned i = 0; i < 2u; ++i)      // sub-blocks 8 (q / 2) + 4 i .. + 3: every other byte from q % 2 on
                             scales[u][i] = (unsigned)(l.q >> 1 ? w[u].scales[2u + i] : w[u].scales[i]) >> (8u * (l.q & 1u));
                     }
 #pragma unroll
                     for (unsigned m = 0; m < 4u; ++m) {
-                        const v4i frag = lds_read_v4i(frag_at + m * frag_step);
 #pragma unroll
                         for (unsigned u = 0; u < 2u; ++u) {
                             const unsigned sc = (scales[u][m >> 1] >> (16u * (m & 1u))) & 15u;
                             v4i limb;
 #pragma unroll
                             for (unsigned i = 0; i < 4u; ++i) limb[i] = (int)q2k_limb((unsigned)w[u].codes[i] >> (2u * m), sc);
-                            lo[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(limb, frag, lo[u], 0, 0, 0);
+                            x.lo[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(limb, frag[m], x.lo[u], 0, 0, 0);
                         }
                     }
                 }
-                request(w, sb + 2u);
-                const float ts = __uint_as_float(lds_read_u32(tile.area + scales_at + 64u * sb + 4u * column));
-#pragma unroll
-                for (unsigned u = 0; u < 2u; ++u) {
-                    const v4i d = lds_read_v4i(scratch + 128u * u + 16u * l.q);
-                    const v4i dmin = lds_read_v4i(scratch + 128u * u + 64u + 16u * l.q);
-#pragma unroll
-                    for (unsigned i = 0; i < 4u; ++i) {
-                        const int dot = QT == QT_Q2_K ? lo[u][i] : (hi[u][i] << 3) + lo[u][i];
-                        const int low = QT == QT_Q2_K ? min_lo[u][i] : (min_hi[u][i] << 7) + min_lo[u][i];
-                        const float left = (ts * __int_as_float(d[i])) * (float)dot;
-                        const float right = (ts * __int_as_float(dmin[i])) * (float)low;
-                        acc[u][i] += (double)(left - right);
-                    }
-                }
             }
+            return x;
         };
         // Lane (token, q) holds the sums of rows 4 q .. 4 q + 3 of either row tile: sixteen bytes a store.
         auto publish = [&]() {
-            const uint2 info = lds_read_uint2(tile.area + 8u * column);
+            const uint2 info = lds_read_uint2(tile.area + 8u * c.column);
             float *const out_row = pr.out + (unsigned long long)info.x * a.out_rows;
             const float limit_f32 = (float)a.limit;
             bool bad = false;
 #pragma unroll
             for (unsigned u = 0; u < (FUSED ? 1u : 2u); ++u) {
-                const unsigned row = (tile.first_unit + unit - tile.start) * kUnitRows + 16u * u + 4u * l.q;
+                const unsigned row = first_row(tile, unit) + 16u * u + 4u * l.q;
                 float value[4];
                 bool good = true;
 #pragma unroll
@@ -625,51 +767,76 @@ __global__ __launch_bounds__(Map16<QT>::kThreads) void rows16_kernel(Rows16Args 
                     }
                     good &= finite_f32(value[i]);
                 }
-                const bool kept = (l.r < tile.live) & (row < a.out_rows);
+                const bool kept = l.r < tile.live;
                 bad |= kept & !good;
                 if (kept & good) *reinterpret_cast<float4 *>(out_row + row) = make_float4(value[0], value[1], value[2], value[3]);
             }
             if (bad) raise_status(a.status, 1);
         };
-        // Behind a superblock: on to the next, at a unit's end its results and the unit drawn before.
-        // False when there is none.
-        auto advance = [&]() -> bool {
-            frag_at += 16u * frag_pitch;
-            if (++sb < a.blocks) return true;
-            publish();
-            if (next >= drawable) return false;
-            unit = next;
-            here = ahead;
-            tile = drawn_tile;
-            begin();
-            next = draw();
-            if (next < drawable) ahead = locate(next);
+        // Behind a run's last superblock: its successor made ready while the sums settle, at a unit's end that of the
+        // next unit; the results go out then. False when no unit is left.
+        auto advance = [&](const Sums &x, unsigned parity) -> bool {
+            const bool ends = ++run == runs;
+            const Scales r = scales_here();
+            frag_at = ends ? c_ahead.frag_at : frag_at + 16u * pitch;
+            pitch = ends ? c_ahead.pitch : pitch;
+            ready(rec[0], parity);
+            settle(x, r);
+            ++sb;
+            if (ends) {
+                publish();
+                if (next >= drawable) return false;
+                unit = next;
+                here = ahead;
+                tile = drawn_tile;
+                c = c_ahead;
+                run = 0u;
+                begin();
+                next = draw();
+                if (next < drawable) {
+                    ahead = locate(next);
+                    c_ahead = columns_of(drawn_tile);
+                }
+            }
             return true;
         };
+        turn_over(1u, 0u);
+        ready(rec[0], 0u);
         for (;;) {
-            superblock(rec[0]);
-            if (!advance()) break;
-            superblock(rec[1]);
-            if (!advance()) break;
+            const Sums x = superblock(rec[0], S == 1u, 0u);
+            if constexpr (S == 1u) {
+                if (!advance(x, 1u)) break;
+            } else {
+                const Scales r = scales_here();
+                frag_at += 16u * pitch;
+                ready(rec[1], 1u);
+                settle(x, r);
+                ++sb;
+            }
+            if (!advance(superblock(rec[S - 1u], true, 1u), 0u)) break;
         }
     }
 }
 
-template <unsigned QT, bool FUSED>
+template <unsigned QT, bool FUSED, unsigned S>
 int launch_rows16(const Rows16Args &a, hipStream_t stream)
 {
-    YVEX_ALLOW_DYNAMIC_LDS((rows16_kernel<QT, FUSED>), kLds16);
-    rows16_kernel<QT, FUSED><<<compute_units(), Map16<QT>::kThreads, kLds16, stream>>>(a);
+    YVEX_ALLOW_DYNAMIC_LDS((rows16_kernel<QT, FUSED, S>), kLds16);
+    rows16_kernel<QT, FUSED, S><<<compute_units(), (Map16<QT, S>::kThreads), kLds16, stream>>>(a);
     return check_launch("moe_rows16");
 }
 
 // Pairs of a full tile: as many Q8_K rows as the LDS holds, at most sixteen.
-template <unsigned QT> unsigned tile_tokens16(unsigned blocks)
+template <unsigned QT, unsigned S> unsigned tile_tokens16(unsigned blocks)
 {
+    using M = Map16<QT, S>;
     unsigned tokens = kSlots16;
-    while (tokens && Map16<QT>::kAreas + Map16<QT>::area_bytes(blocks, tokens) > kLds16) tokens -= 4u;
+    while (tokens && M::kAreas + M::area_bytes(blocks, tokens) > kLds16) tokens -= 4u;
     return tokens;
 }
+
+// Image rows that come two superblocks a run.
+bool two_at_a_time(uint64_t blocks) { return blocks % 2u == 0u && blocks >= 4u && blocks <= 16u; }
 
 }  // namespace
 
@@ -677,25 +844,26 @@ unsigned rows16_tokens(const GroupedProblem &problem, unsigned qtype, bool image
                        uint64_t out_rows)
 {
     const uint64_t blocks = width / 256u, superblock = qtype == QT_IQ2_XXS ? (image ? 72u : 66u) : qtype == QT_Q4_K ? 144u : 84u;
-    // superblocks are requested two ahead, across one unit's end
-    if (width % 256u || blocks < 2u || blocks > kMaxBlocks16 || (qtype == QT_Q2_K && fused)) return 0u;
+    // two runs are asked for ahead of their use, the second of them at a unit's end of the unit behind it
+    if (width % 256u || blocks < (qtype == QT_Q2_K && !(blocks & 1u) ? 4u : 2u) || blocks > kMaxBlocks16 || (qtype == QT_Q2_K && fused)) return 0u;
     // a lane addresses its rows with 32-bit offsets inside an expert and stores four rows at a time
-    if (!out_rows || out_rows % 4u || problem.row_bytes != blocks * superblock || (problem.row_bytes & 3u) ||
+    if (out_rows < (fused ? 16u : 32u) || out_rows % 4u || problem.row_bytes != blocks * superblock || (problem.row_bytes & 3u) ||
         (fused && problem.up_row_bytes != problem.row_bytes) || out_rows * problem.row_bytes > 0xffffffffull)
         return 0u;
     if ((((uintptr_t)problem.gate | (uintptr_t)problem.up | (uintptr_t)problem.activations | problem.expert_bytes |
           problem.up_expert_bytes | problem.act_stride) & 3u) || ((uintptr_t)problem.out & 15u))
         return 0u;
     if (problem.experts > 256u && problem.expert_ids) return 0u;
-    return qtype == QT_IQ2_XXS ? tile_tokens16<QT_IQ2_XXS>((unsigned)blocks)
-         : qtype == QT_Q4_K    ? tile_tokens16<QT_Q4_K>((unsigned)blocks)
-         : qtype == QT_Q2_K    ? tile_tokens16<QT_Q2_K>((unsigned)blocks) : 0u;
+    return qtype == QT_IQ2_XXS && image && two_at_a_time(blocks) ? tile_tokens16<kIq2Image, 2u>((unsigned)blocks)
+         : qtype == QT_IQ2_XXS ? tile_tokens16<kIq2Image, 1u>((unsigned)blocks)
+         : qtype == QT_Q4_K    ? tile_tokens16<QT_Q4_K, 1u>((unsigned)blocks)
+         : qtype == QT_Q2_K    ? tile_tokens16<QT_Q2_K, 2u>((unsigned)blocks) : 0u;
 }
 
 bool rows16_one_round(const GroupedProblem &problem, unsigned qtype, bool fused, unsigned tokens, uint64_t out_rows)
 {
     const uint64_t units = (out_rows + (fused ? 15u : 31u)) / (fused ? 16u : 32u);
-    const unsigned waves = qtype == QT_IQ2_XXS ? Map16<QT_IQ2_XXS>::kWaves : Map16<QT_Q4_K>::kWaves;
+    const unsigned waves = qtype == QT_IQ2_XXS ? Map16<kIq2Image, 1u>::kWaves : Map16<QT_Q4_K, 1u>::kWaves;
     return (problem.pairs + (uint64_t)tokens - 1u) / tokens * units <= (uint64_t)waves * compute_units();
 }
 
@@ -705,12 +873,16 @@ int launch_rows16_grouped(const GroupedProblem &problem, unsigned qtype, bool im
     const Rows16Args a{problem, width / 256u, out_rows, rows16_tokens(problem, qtype, image, fused, width, out_rows), round,
                        behind, limit, status};
     if (!a.tokens) return ST_UNSUPPORTED;
-    if (qtype == QT_Q2_K) return launch_rows16<QT_Q2_K, false>(a, stream);
+    // (a run of two Q2_K superblocks fills a load; a row of an odd number of them comes one at a time)
+    if (qtype == QT_Q2_K)
+        return a.blocks & 1u ? launch_rows16<QT_Q2_K, false, 1u>(a, stream) : launch_rows16<QT_Q2_K, false, 2u>(a, stream);
     if (qtype == QT_Q4_K)
-        return fused ? launch_rows16<QT_Q4_K, true>(a, stream) : launch_rows16<QT_Q4_K, false>(a, stream);
+        return fused ? launch_rows16<QT_Q4_K, true, 1u>(a, stream) : launch_rows16<QT_Q4_K, false, 1u>(a, stream);
+    if (image && two_at_a_time(a.blocks))
+        return fused ? launch_rows16<kIq2Image, true, 2u>(a, stream) : launch_rows16<kIq2Image, false, 2u>(a, stream);
     if (image)
-        return fused ? launch_rows16<kIq2Image, true>(a, stream) : launch_rows16<kIq2Image, false>(a, stream);
-    return fused ? launch_rows16<QT_IQ2_XXS, true>(a, stream) : launch_rows16<QT_IQ2_XXS, false>(a, stream);
+        return fused ? launch_rows16<kIq2Image, true, 1u>(a, stream) : launch_rows16<kIq2Image, false, 1u>(a, stream);
+    return fused ? launch_rows16<QT_IQ2_XXS, true, 1u>(a, stream) : launch_rows16<QT_IQ2_XXS, false, 1u>(a, stream);
 }
 
 }  // namespace yvex

@@ -76,7 +76,7 @@ struct RowsQ4kArgs {
     int *status;
     // plain projection (one bucket holding every input row): out[token * out_stride + row]
     int plain, output_bf16;
-    unsigned left;           // a bucket's last tile of up to this many pairs is not this launch's (rows16.hip)
+    unsigned few;            // pairs of a tile of the few-pair kernel, which has a part of the buckets' last tiles
     const float *additive;
     unsigned long long out_stride;
 };
@@ -423,7 +423,8 @@ __global__ __launch_bounds__(kQ4Threads, 2) void rows_q4k_kernel(RowsQ4kArgs g)
     } else {
         const unsigned buckets = (unsigned)pr.counts[0];
         const unsigned long long population = threadIdx.x < buckets ? pr.bucket_populations[threadIdx.x] : 0ull;
-        const unsigned tiles = (unsigned)(population / kQ4Tokens) + (population % kQ4Tokens > g.left ? 1u : 0u);
+        const unsigned rest = (unsigned)(population % kQ4Tokens), left = few_pair_limit(g.few, population, kQ4MetaBase + 48u);
+        const unsigned tiles = (unsigned)(population / kQ4Tokens) + (rest > left ? 1u : 0u);
         unsigned inclusive = tiles;
 #pragma unroll
         for (int offset = 1; offset < 64; offset <<= 1) {
@@ -472,7 +473,7 @@ int launch_rows_q4k(const RowsQ4kArgs &g, dim3 grid, hipStream_t stream)
 }  // namespace
 
 int launch_q4k_rows_grouped(const GroupedProblem &problem, unsigned qtype, bool fused, uint64_t width,
-                            uint64_t out_rows, unsigned left, double limit, int *status, hipStream_t stream)
+                            uint64_t out_rows, unsigned few, double limit, int *status, hipStream_t stream)
 {
     if (qtype != QT_Q4_K && !(qtype == QT_Q2_K && !fused)) return ST_UNSUPPORTED;
     if (!width || width % 256u || !out_rows || out_rows > 0x7fffffffull) return ST_BOUNDS;
@@ -487,13 +488,13 @@ int launch_q4k_rows_grouped(const GroupedProblem &problem, unsigned qtype, bool 
         return ST_INVALID_ARG;
     if (problem.experts > 256u && problem.expert_ids) return ST_BOUNDS;
     const uint64_t row_tiles = (out_rows + (fused ? 63u : 127u)) / (fused ? 64u : 128u);
-    // token tiles: every bucket of more than `left` pairs may end in a partial tile
-    const uint64_t partial = (uint64_t)problem.pairs / (left + 1u);
+    // token tiles: every bucket of more than `few` pairs may end in a partial tile
+    const uint64_t partial = (uint64_t)problem.pairs / (few + 1u);
     const uint64_t token_tiles = problem.expert_ids ? (uint64_t)problem.pairs / kQ4Tokens +
                                                           (partial < problem.experts ? partial : problem.experts)
                                                     : ((uint64_t)problem.pairs + kQ4Tokens - 1u) / kQ4Tokens;
     if (row_tiles > 0x7fffffffull || token_tiles > 65535ull) return ST_BOUNDS;
-    RowsQ4kArgs g{problem, (unsigned)(width / 256u), (unsigned)out_rows, limit, status, 0, 0, left, nullptr, 0ull};
+    RowsQ4kArgs g{problem, (unsigned)(width / 256u), (unsigned)out_rows, limit, status, 0, 0, few, nullptr, 0ull};
     const dim3 grid((unsigned)row_tiles, (unsigned)token_tiles);
     if (qtype == QT_Q2_K) return launch_rows_q4k<QT_Q2_K, false>(g, grid, stream);
     return fused ? launch_rows_q4k<QT_Q4_K, true>(g, grid, stream) : launch_rows_q4k<QT_Q4_K, false>(g, grid, stream);
