@@ -9,8 +9,8 @@
 //     dot_b = sum_i q_i * a_i                              (int32, exact: one K step of V_MFMA_I32_32X32X32_I8)
 //     total = fmaf(d_b * d_a, float(dot_b), total)         b = 0 .. 7 in order, floats, from zero
 //     row  += double(total)                                superblock by superblock, rounded to float once
-// A block has a scale of its own, so every matrix instruction starts from zero and its sixteen
-// results a lane are converted, scaled and chained on the vector ALU (three instructions each).
+// A block has a scale of its own, so every matrix instruction starts anew and its sixteen
+// results a lane are brought to float, scaled and chained on the vector ALU (three instructions each).
 //
 // A workgroup owns 32 weight rows x 32 input rows; its four waves take every fourth superblock
 // (eight blocks, 272 bytes a row) and their partial tiles are added in wave order, so results do
@@ -50,137 +50,205 @@ __device__ __forceinline__ void choose_matrix(DenseQ80Args &g)
     }
 }
 
-// What a lane needs of one superblock: its half of the eight blocks' codes (their scales lie in
-// the same windows) and its half of one input row's blocks.
-struct Q80Inputs {
-    uint4 codes[8];         // even blocks: the aligned window two bytes in front of the codes
-    unsigned tail[4];       // even blocks: the dword behind the window
-    uint4 a[8];
-    float act_scale;
-};
+// float(sum) of a matrix instruction's sums without a conversion each. The instruction starts from the bits of
+// 1 / (2 pi) as an integer instead of zero, which its encoding holds as an inline constant; the sums of one
+// block are below 2^20 and the constant's mantissa is 2 292 099 above its binade's first, 6 096 508 below its last, so the
+// bits of a result are those of the float kStart + 2^-26 sum, and one subtraction, which the vector ALU issues at twice the
+// rate of a conversion, leaves 2^-26 float(sum) exactly.
+constexpr unsigned kStartBits = 0x3e22f983u;
 
-__device__ __forceinline__ void q80_load(const unsigned char *wrow, const unsigned char *arow, unsigned sb,
-                                         unsigned h, Q80Inputs &in)
+// The block's sums from kStartBits on, as floats. Written out because the compiler puts a start other than zero into
+// sixteen registers. The results are in their registers behind the last wait states (eleven for a matrix
+// instruction of eight passes), so that whatever follows may read or reuse them; the first ones cover operands that vector
+// instructions have just written.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ v16f block_sums(v4i tokens, v4i codes)
 {
-    const unsigned char *w = wrow + (unsigned long long)sb * 272ull;     // dword-aligned
+    v16f dot;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("s_nop 1\n\t"
+        "v_mfma_i32_32x32x32_i8 %0, %1, %2, 0.15915494\n\t"
+        "s_nop 12"
+        : "=&v"(dot) : "v"(tokens), "v"(codes));
+#else
+    (void)tokens;
+    (void)codes;
+    for (int i = 0; i < 16; ++i) dot[i] = 0.0f;
+#endif
+    return dot;
+}
+#pragma clang diagnostic pop
+
+__device__ __forceinline__ uint4 read16(unsigned address)
+{
+    const v4i v = lds_read_v4i(address);
+    return make_uint4((unsigned)v[0], (unsigned)v[1], (unsigned)v[2], (unsigned)v[3]);
+}
+
+constexpr unsigned kStagedPitch = 272u;
+
+// One superblock out of LDS: lane (r, h)'s weight row at `w_row` (272 bytes), its input row's codes, of which it holds
+// sixteen bytes a block, at `a_row`, and the scales of the input rows that it has sums of, four at a time, at `scales`.
+__device__ __forceinline__ void q80_superblock(unsigned w_row, unsigned a_row, unsigned scales, unsigned h, float minus, double (&acc)[16])
+{
+    float d_a[16], total[16];
+    uint4 lo[2], hi[2] = {};
+    v4i tokens[2];
+    unsigned scale_bits[2];
+    auto read_block = [&](unsigned c) {
+        const unsigned slot = c % 2u;
+        const unsigned start_at = c % 2u == 0u ? 34u * c : 34u * c + 2u;      // the lane's window: + 16 h
+        lo[slot] = read16(w_row + 16u * h + (start_at & ~15u));
+        // (an even block's window is 20 bytes, an odd block's 16: what of it lies in the next piece)
+        const unsigned behind = w_row + 16u * h + (start_at & ~15u) + 16u, words = (start_at & 15u) / 4u + (c % 2u == 0u ? 1u : 0u);
+        if (words == 1u) hi[slot].x = lds_read_u32(behind);
+        else if (words == 2u) {
+            const uint2 two = lds_read_uint2(behind);
+            hi[slot].x = two.x;
+            hi[slot].y = two.y;
+        } else if (words) hi[slot] = read16(behind);
+        scale_bits[slot] = lds_read_u16(w_row + 34u * c);
+        tokens[slot] = lds_read_v4i(a_row + 32u * c);
+    };
+    auto codes_of = [&](unsigned c) -> v4i {
+        const unsigned slot = c % 2u;
+        const unsigned start_at = c % 2u == 0u ? 34u * c : 34u * c + 2u, at = (start_at & 15u) / 4u;
+        const unsigned q[8] = {lo[slot].x, lo[slot].y, lo[slot].z, lo[slot].w,
+                               hi[slot].x, hi[slot].y, hi[slot].z, hi[slot].w};
+        v4i codes;
+#pragma unroll
+        for (unsigned j = 0; j < 4u; ++j)
+            codes[j] = c % 2u == 0u ? (int)__builtin_amdgcn_alignbyte(q[at + j + 1u], q[at + j], 2u) : (int)q[at + j];
+        return codes;
+    };
+    read_block(0u);
+#pragma unroll
+    for (unsigned q = 0; q < 4u; ++q) {
+        const uint4 d = read16(scales + 32u * q);
+        d_a[4u * q] = __uint_as_float(d.x); d_a[4u * q + 1u] = __uint_as_float(d.y);
+        d_a[4u * q + 2u] = __uint_as_float(d.z); d_a[4u * q + 3u] = __uint_as_float(d.w);
+    }
 #pragma unroll
     for (unsigned c = 0; c < 8u; ++c) {
-        // block c starts at 34 c: two bytes past a dword boundary when c is odd
-        const unsigned codes = 34u * c + 2u + 16u * h;
-        if (c % 2u == 0u) {
-            const unsigned *p = reinterpret_cast<const unsigned *>(w + codes - 2u);
-            in.codes[c] = make_uint4(p[0], p[1], p[2], p[3]);
-            in.tail[c / 2u] = p[4];
-        } else {
-            const unsigned *p = reinterpret_cast<const unsigned *>(w + codes);
-            in.codes[c] = make_uint4(p[0], p[1], p[2], p[3]);
+        const v4i codes = codes_of(c);
+        const float d_w = f16_bits_to_float(scale_bits[c % 2u]) * 67108864.0f;       // (what the sums lack)
+        if (c + 1u < 8u) read_block(c + 1u);
+        __builtin_amdgcn_sched_barrier(0);
+        const v16f dot = block_sums(tokens[c % 2u], codes);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float step = d_w * d_a[i], value = dot[i] + minus;
+            total[i] = c == 0u ? step * value : __builtin_fmaf(step, value, total[i]);
         }
-    }
-    const unsigned char *a = arow + (unsigned long long)sb * kQ8KBytes;
-    in.act_scale = *reinterpret_cast<const float *>(a);
+        // (the compiler would sink all of it behind the last block, and keep every block's sums until then)
+#if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-    for (unsigned c = 0; c < 8u; ++c) {
-        const unsigned *p = reinterpret_cast<const unsigned *>(a + 4u + 32u * c + 16u * h);
-        in.a[c] = make_uint4(p[0], p[1], p[2], p[3]);
+        for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(total[i]));
+#endif
+        __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] += (double)total[i];
+}
+
+// What the sums start from, in a vector register (a subtraction with a constant operand issues at a conversion's rate).
+__device__ __forceinline__ float minus_start()
+{
+    float minus = -__uint_as_float(kStartBits);
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(minus));
+#endif
+    return minus;
 }
 
 constexpr unsigned kPlainWaves = 4u;
+// LDS of a wave: its 32 weight rows' superblock, its 32 input rows' codes (both 272 bytes a row), their scales
+constexpr unsigned kPlainAct = 32u * kStagedPitch, kPlainScales = 2u * kPlainAct, kPlainWindow = kPlainScales + 128u;
+constexpr unsigned kPlainLdsBytes = kPlainWaves * kPlainWindow;        // (the partial tiles take their place in the end)
 
+// 32 weight rows x 32 input rows a workgroup, a superblock in four a wave. Every lane used to load its own pieces of 16
+// bytes, 33 instructions of 64 cache lines a superblock at two cycles a line: waves stood before the memory pipeline half
+// their time and the vector ALU was 19 % busy. The lanes of a load take consecutive pieces of consecutive rows now, a
+// superblock ahead, and the bytes pass through a window of LDS of the wave's own. 4096 x 4096 by 32 / 96 rows
+// 17.0 / 25.6 -> 14.2 / 18.3 us, 2048 x 7168 by 32 / 256 21.2 / 34.1 -> 18.3 / 25.9. (Eight waves, two superblocks each, are
+// 1 to 1.5 us behind: the reduction is longer and the device no fuller.)
 __global__ __launch_bounds__(64 * kPlainWaves) void dense_q8_0_kernel(DenseQ80Args g)
 {
-    // per wave: the scales of the input rows whose blocks its lanes hold; then the partial tiles
-    __shared__ __align__(16) float row_scale[kPlainWaves][32];
-    __shared__ double partial[kPlainWaves - 1u][16][64];
+    extern __shared__ __align__(16) unsigned char dense_q8_0_plain_lds[];
+    if (lds_address_of(dense_q8_0_plain_lds) != 0u) {   // operands are addressed by absolute LDS offsets
+        if (threadIdx.x == 0u) raise_status(g.status, 2);
+        return;
+    }
     choose_matrix(g);
     const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const unsigned r = lane & 31u, h = lane >> 5;
     const unsigned long long row0 = (unsigned long long)blockIdx.x * 32ull;
     const unsigned long long tok0 = (unsigned long long)blockIdx.y * 32ull;
-    unsigned long long wr = row0 + r;
-    if (wr >= g.row_count) wr = g.row_count - 1ull;              // a ragged edge repeats the last row
-    const unsigned char *wrow = g.encoded + wr * g.row_bytes;
-    unsigned long long t = tok0 + r;
-    if (t >= g.input_rows) t = g.input_rows - 1ull;
-    const unsigned char *arow = g.act + t * ((unsigned long long)g.blocks * kQ8KBytes);
+    const unsigned rows_here = (unsigned)(g.row_count - row0 < 32ull ? g.row_count - row0 : 32ull);
+    const unsigned toks_here = (unsigned)(g.input_rows - tok0 < 32ull ? g.input_rows - tok0 : 32ull);
+    const unsigned long long act_row_bytes = (unsigned long long)g.blocks * kQ8KBytes;
+    const unsigned char *const weights = g.encoded + row0 * g.row_bytes, *const acts = g.act + tok0 * act_row_bytes;
+    // pieces 64 k + lane of 32 rows x 17 and of 32 rows x 16 (a ragged edge repeats the last row)
+    const unsigned char *weight_at[9], *act_at[8];
+#pragma unroll
+    for (unsigned k = 0; k < 9u; ++k) {
+        const unsigned piece = k < 8u ? 64u * k + lane : 512u + r, row = piece / 17u;
+        weight_at[k] = weights + (row < rows_here ? row : rows_here - 1u) * g.row_bytes + 16u * (piece - 17u * row);
+    }
+#pragma unroll
+    for (unsigned k = 0; k < 8u; ++k) {
+        const unsigned row = 4u * k + (lane >> 4);
+        act_at[k] = acts + (row < toks_here ? row : toks_here - 1u) * act_row_bytes + 4u + 16u * (lane & 15u);
+    }
+    const unsigned char *const scale_from = acts + (r < toks_here ? r : toks_here - 1u) * act_row_bytes;
+    struct {
+        v4i weights[9], acts[8];
+        unsigned scale;
+    } ahead;
+    typedef v4i v4i_dword __attribute__((aligned(4)));
+    auto request = [&](unsigned sb) {
+        const unsigned long long w = sb * 272ull, a = (unsigned long long)sb * kQ8KBytes;
+#pragma unroll
+        for (unsigned k = 0; k < 9u; ++k) ahead.weights[k] = *reinterpret_cast<const v4i_dword *>(weight_at[k] + w);
+#pragma unroll
+        for (unsigned k = 0; k < 8u; ++k) ahead.acts[k] = *reinterpret_cast<const v4i_dword *>(act_at[k] + a);
+        ahead.scale = *reinterpret_cast<const unsigned *>(scale_from + a);
+    };
+    const unsigned window = kPlainWindow * wave;
+    const float minus = minus_start();
     double acc[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.0;
-
-    Q80Inputs cur;
-    q80_load(wrow, arow, wave < g.blocks ? wave : 0u, h, cur);
+    if (wave < g.blocks) request(wave);
     for (unsigned sb = wave; sb < g.blocks; sb += kPlainWaves) {
+        // (LDS operations of one wave complete in order)
+#pragma unroll
+        for (unsigned k = 0; k < 8u; ++k) {
+            lds_write_v4i(window + 1024u * k + 16u * lane, ahead.weights[k]);
+            lds_write_v4i(window + kPlainAct + 4u * kStagedPitch * k + kStagedPitch * (lane >> 4) + 16u * (lane & 15u), ahead.acts[k]);
+        }
+        lds_write_v4i(window + 8192u + 16u * r, ahead.weights[8]);
+        lds_write_u32(window + kPlainScales + 4u * r, ahead.scale);
         // the next superblock's bytes travel while this one is worked on
-        Q80Inputs nxt;
-        q80_load(wrow, arow, sb + kPlainWaves < g.blocks ? sb + kPlainWaves : sb, h, nxt);
-
-        // The block scales lie in the windows already: an even block's in front of its codes (the
-        // low half of the first dword of the lane with h = 0), an odd block's behind the codes of
-        // the block before it (the high half of the tail dword of the lane with h = 1). Each half
-        // packs its four and takes the other half's from the lane 32 away.
-        unsigned mine[2], theirs[2];
-#pragma unroll
-        for (unsigned j = 0; j < 2u; ++j) {
-            const unsigned first = h ? cur.tail[2u * j] >> 16 : cur.codes[4u * j].x & 0xffffu;
-            const unsigned second = h ? cur.tail[2u * j + 1u] >> 16 : cur.codes[4u * j + 2u].x & 0xffffu;
-            mine[j] = first | (second << 16);
-            theirs[j] = (unsigned)__shfl_xor((int)mine[j], 32, 64);
-        }
-        float d_w[8];
-#pragma unroll
-        for (unsigned c = 0; c < 8u; ++c) {
-            const unsigned pack = (c % 2u == h) ? mine[c / 4u] : theirs[c / 4u];     // blocks c with c % 2 == h are mine
-            d_w[c] = f16_bits_to_float((c / 2u) % 2u ? pack >> 16 : pack & 0xffffu);
-        }
-        // the input rows' scales to the lanes that hold their sums
-        row_scale[wave][r] = cur.act_scale;
+        request(sb + kPlainWaves < g.blocks ? sb + kPlainWaves : sb);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-        float d_a[16], total[16];       // the input rows' scales; the superblock's chain of eight terms
-#pragma unroll
-        for (unsigned q4 = 0; q4 < 4u; ++q4) {
-            const float4 d = *reinterpret_cast<const float4 *>(&row_scale[wave][8u * q4 + 4u * h]);
-            d_a[4u * q4] = d.x; d_a[4u * q4 + 1u] = d.y; d_a[4u * q4 + 2u] = d.z; d_a[4u * q4 + 3u] = d.w;
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) total[i] = 0.0f;
-#pragma unroll
-        for (unsigned c = 0; c < 8u; ++c) {
-            v4i codes;
-            if (c % 2u == 0u) {
-                const uint4 q = cur.codes[c];
-                codes[0] = (int)__builtin_amdgcn_alignbyte(q.y, q.x, 2u);
-                codes[1] = (int)__builtin_amdgcn_alignbyte(q.z, q.y, 2u);
-                codes[2] = (int)__builtin_amdgcn_alignbyte(q.w, q.z, 2u);
-                codes[3] = (int)__builtin_amdgcn_alignbyte(cur.tail[c / 2u], q.w, 2u);
-            } else {
-                codes[0] = (int)cur.codes[c].x; codes[1] = (int)cur.codes[c].y;
-                codes[2] = (int)cur.codes[c].z; codes[3] = (int)cur.codes[c].w;
-            }
-            v16i zero;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) zero[i] = 0;
-            const v4i tokens = {(int)cur.a[c].x, (int)cur.a[c].y, (int)cur.a[c].z, (int)cur.a[c].w};
-            const v16i dot = __builtin_amdgcn_mfma_i32_32x32x32_i8(tokens, codes, zero, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) total[i] = __builtin_fmaf(d_w[c] * d_a[i], (float)dot[i], total[i]);
-            // (left alone the scheduler issues the matrix instructions of all blocks first and
-            // keeps their results)
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] += (double)total[i];
-        // (the next superblock's scales are not written before every lane has read these)
+        q80_superblock(window + r * kStagedPitch, window + kPlainAct + r * kStagedPitch + 16u * h, window + kPlainScales + 16u * h, h,
+                       minus, acc);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        cur = nxt;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
 
+    // (the partial tiles of waves 1 to 3 take the windows' place)
+    __syncthreads();
+    double *const partial = reinterpret_cast<double *>(dense_q8_0_plain_lds);
     if (wave) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) partial[wave - 1u][i][lane] = acc[i];
+        for (int i = 0; i < 16; ++i) partial[((wave - 1u) * 16u + i) * 64u + lane] = acc[i];
     }
     __syncthreads();
     if (wave) return;
@@ -192,7 +260,7 @@ __global__ __launch_bounds__(64 * kPlainWaves) void dense_q8_0_kernel(DenseQ80Ar
         const unsigned long long token = tok0 + 8u * (i >> 2) + 4u * h + (i & 3);
         double wide = acc[i];
 #pragma unroll
-        for (unsigned w = 0; w + 1u < kPlainWaves; ++w) wide += partial[w][i][lane];
+        for (unsigned w = 0; w + 1u < kPlainWaves; ++w) wide += partial[(w * 16u + i) * 64u + lane];
         const float sum = (float)wide;
         if (row >= g.row_count || token >= g.input_rows) continue;
         const unsigned long long at = token * g.out_stride + row;
@@ -224,17 +292,11 @@ __global__ __launch_bounds__(64 * kPlainWaves) void dense_q8_0_kernel(DenseQ80Ar
 // TOKEN_BLOCKS = 1 (with ROW_BLOCKS = 8: 256 weight rows x 32 input rows, 153 KB): batches of up to
 // 32 input rows against a matrix too large for the caches, an output head at decode width, where
 // the second block of input rows would be padding and half of every wave's work with it.
-constexpr unsigned kStagedPitch = 272u;
 constexpr unsigned staged_lds_bytes(unsigned row_blocks, unsigned token_blocks = 2u)
 {
     return 2u * (32u * row_blocks + 32u * token_blocks) * kStagedPitch;
 }
 
-__device__ __forceinline__ uint4 read16(unsigned address)
-{
-    const v4i v = lds_read_v4i(address);
-    return make_uint4((unsigned)v[0], (unsigned)v[1], (unsigned)v[2], (unsigned)v[3]);
-}
 
 template <unsigned ROW_BLOCKS, unsigned TOKEN_BLOCKS = 2u>
 __global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS) void dense_q8_0_staged_kernel(DenseQ80Args g)
@@ -337,7 +399,7 @@ __global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS) void dense_q8_0_sta
         // scaling of the results one after the other: in step k the operands of block k are
         // read, block k - 1 is multiplied and the results of block k - 2 are scaled (vector
         // instructions that issue while the matrix pipe works).
-        uint4 lo[2], hi[2];
+        uint4 lo[2], hi[2] = {};
         v4i tokens[2];
         unsigned scale_bits[2];
         v16i dot[2];
@@ -407,27 +469,7 @@ __global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS) void dense_q8_0_sta
     if (bad) raise_status(g.status, 1);
 }
 
-// float(sum) of a matrix instruction's sums without a conversion each. The instruction starts from
-// 1.5 * 2^23 as an integer instead of zero; the sums of one block are below 2^20, so the bits of a result
-// are those of the float 12582912 + sum, and one addition, which two waves of a SIMD issue at
-// twice the rate of a conversion, leaves float(sum) exactly. (The constant sits in a vector register: an
-// addition with a scalar or literal operand issues at the conversion's rate.)
-struct FloatBias {
-    v16i start;
-    float minus;
-    __device__ __forceinline__ void set()
-    {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) start[i] = 0x4b400000;
-        minus = -12582912.0f;
-#if defined(__HIP_DEVICE_COMPILE__)
-        asm("" : "+v"(minus));
-#endif
-    }
-    __device__ __forceinline__ float value(int sum) const { return __int_as_float(sum) + minus; }
-};
-
-constexpr unsigned kWideRows = 128u, kWideTokens = 128u, kWideThreads = 512u;
+constexpr unsigned kWideRows = 128u, kWideTokens = 128u, kWideThreads = 1024u;
 constexpr unsigned kWideWeightBytes = kWideRows * kStagedPitch, kWideActBytes = kWideTokens * kStagedPitch;  // one buffer
 constexpr unsigned kWideActBase = 2u * kWideWeightBytes, kWideScaleBase = kWideActBase + 2u * kWideActBytes;
 constexpr unsigned kWideLdsBytes = kWideScaleBase + 2u * kWideTokens * 4u;
@@ -435,16 +477,15 @@ constexpr unsigned kWideLdsBytes = kWideScaleBase + 2u * kWideTokens * 4u;
 // The same product for batches that fill the device with tiles of 128 weight rows x 128 input rows.
 // Bound by vector-instruction issue: behind one matrix instruction (32 cycles) sixteen results a lane
 // are brought to float, multiplied by their scale and chained. What this kernel does about it:
-//  * FloatBias above in place of the conversions.
-//  * A wave owns 32 weight rows x 64 input rows: a block's codes and scale are read, and the
-//    even blocks shifted into place, once for two matrix instructions, and while the matrix pipe works
-//    on one 32-row block the vector ALU scales the other's results (a wave's own matrix and vector
-//    instructions overlap on this part).
-//  * The input rows' scales lie end to end in LDS: a lane's sixteen are four 16-byte reads, not
-//    sixteen 4-byte ones.
+//  * kStartBits above in place of the conversions.
+//  * A wave owns 32 weight rows x 32 input rows on 128 registers, so that sixteen of them, four a SIMD, cover each
+//    other's waits and the rate of one wave's instructions (one in 5.5 cycles on this part; two waves issue 4-cycle
+//    instructions in 5.0 cycles each, four in 4.4).
 //  * Copies take a scalar base and a 32-bit offset a lane: a register and no addition each.
-// 4096 x 4096 by 2048 rows 171 -> 138 us (498 TOP/s), 2048 x 7168 124 -> 104 us. Counters of the former: vector ALU
-// 79 % busy, LDS 20 %, matrix cores 11 %.
+// 4096 x 4096 by 2048 rows 136 -> 129 us (528 TOP/s; eight waves of 32 x 64, two a SIMD, before). Counters of the old one: vector
+// ALU 60 instructions a wave and block at 3 cycles, half the time; of the new one 2.4 cycles each, and the LDS, which serves
+// twice the weight reads, 40 % busy, is the other half. The products of the scales as one V_MFMA_F32_32X32X2_F32 a block (the
+// same bits): 137 us, it does not run beside vector instructions. Whole 16-byte reads of a window's end: 131 us.
 __global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80Args g)
 {
     extern __shared__ __align__(16) unsigned char dense_q8_0_lds[];
@@ -455,20 +496,20 @@ __global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80A
     choose_matrix(g);
     const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const unsigned r = lane & 31u, h = lane >> 5;
-    const unsigned row_block = wave & 3u, token_pair = wave >> 2;
+    const unsigned row_block = wave & 3u, token_block = wave >> 2;
     const unsigned long long row0 = (unsigned long long)blockIdx.x * kWideRows;
     const unsigned long long tok0 = (unsigned long long)blockIdx.y * kWideTokens;
     const unsigned rows_here = (unsigned)(g.row_count - row0 < kWideRows ? g.row_count - row0 : kWideRows);
     const unsigned toks_here = (unsigned)(g.input_rows - tok0 < kWideTokens ? g.input_rows - tok0 : kWideTokens);
     const unsigned act_row_bytes = g.blocks * kQ8KBytes, row_bytes = (unsigned)g.row_bytes;
 
-    // ---- copies: pieces q = tid + 512 k of 128 rows x 17 (a ragged edge repeats the tile's last row;
+    // ---- copies: pieces q = tid + 1024 k of 128 rows x 17 (a ragged edge repeats the tile's last row;
     // an input row's seventeenth piece only keeps the pitch); the last 128 pieces of the weights by
     // waves 0 and 1, of the input rows by waves 2 and 3, the input rows' scales by waves 4 and 5 ----
-    unsigned weight_at[5], act_at[5];
+    unsigned weight_at[3], act_at[3];
 #pragma unroll
-    for (unsigned k = 0; k < 5u; ++k) {
-        const unsigned q = k < 4u ? tid + kWideThreads * k : 2048u + (tid & 127u);
+    for (unsigned k = 0; k < 3u; ++k) {
+        const unsigned q = k < 2u ? tid + kWideThreads * k : 2048u + (tid & 127u);
         const unsigned row = q / 17u, piece = q - row * 17u;
         weight_at[k] = (row < rows_here ? row : rows_here - 1u) * row_bytes + 16u * piece;
         act_at[k] = (row < toks_here ? row : toks_here - 1u) * act_row_bytes + (piece < 16u ? 4u + 16u * piece : 0u);
@@ -486,105 +527,28 @@ __global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80A
         const unsigned char *a = acts + (unsigned long long)sb * kQ8KBytes;
         const unsigned w_to = buffer * kWideWeightBytes, a_to = kWideActBase + buffer * kWideActBytes;
 #pragma unroll
-        for (unsigned k = 0; k < 4u; ++k) {
+        for (unsigned k = 0; k < 2u; ++k) {
             copy_to_lds_16_at(w, weight_at[k], w_to + wave_lds + 16u * kWideThreads * k);
             copy_to_lds_16_at(a, act_at[k], a_to + wave_lds + 16u * kWideThreads * k);
         }
-        if (wave < 2u) copy_to_lds_16_at(w, weight_at[4], w_to + rest_lds);
-        else if (wave < 4u) copy_to_lds_16_at(a, act_at[4], a_to + rest_lds);
+        if (wave < 2u) copy_to_lds_16_at(w, weight_at[2], w_to + rest_lds);
+        else if (wave < 4u) copy_to_lds_16_at(a, act_at[2], a_to + rest_lds);
         else if (wave < 6u) copy_to_lds_4_at(a, scale_at, scale_lds + buffer * (kWideTokens * 4u));
     };
 
-    FloatBias bias;
-    bias.set();
-    double acc[2][16];
+    const float minus = minus_start();
+    double acc[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.0;
+    for (int i = 0; i < 16; ++i) acc[i] = 0.0;
     copies(0u);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     for (unsigned sb = 0; sb < g.blocks; ++sb) {
         const unsigned buffer = sb & 1u;
         if (sb + 1u < g.blocks) copies(sb + 1u);
-        const unsigned w_row = buffer * kWideWeightBytes + (32u * row_block + r) * kStagedPitch;
-        const unsigned a_row = kWideActBase + buffer * kWideActBytes + (64u * token_pair + r) * kStagedPitch + 16u * h;
-        const unsigned scales = kWideScaleBase + buffer * (kWideTokens * 4u) + (64u * token_pair + 4u * h) * 4u;
-        float d_a[2][16], total[2][16];
-        uint4 lo[2], hi[2];
-        v4i tokens[2][2];
-        unsigned scale_bits[2];
-        auto read_block = [&](unsigned c) {
-            const unsigned slot = c % 2u;
-            const unsigned start = c % 2u == 0u ? 34u * c : 34u * c + 2u;      // the lane's window: + 16 h
-            lo[slot] = read16(w_row + 16u * h + (start & ~15u));
-            // (an even block's window is 20 bytes, an odd block's 16: only block 7's fits one piece)
-            hi[slot] = c % 2u == 0u || (start & 15u) ? read16(w_row + 16u * h + (start & ~15u) + 16u) : lo[slot];
-            scale_bits[slot] = lds_read_u16(w_row + 34u * c);
-            tokens[slot][0] = lds_read_v4i(a_row + 32u * c);
-            tokens[slot][1] = lds_read_v4i(a_row + 32u * kStagedPitch + 32u * c);
-        };
-        auto codes_of = [&](unsigned c) -> v4i {
-            const unsigned slot = c % 2u;
-            const unsigned start = c % 2u == 0u ? 34u * c : 34u * c + 2u, at = (start & 15u) / 4u;
-            const unsigned q[8] = {lo[slot].x, lo[slot].y, lo[slot].z, lo[slot].w,
-                                   hi[slot].x, hi[slot].y, hi[slot].z, hi[slot].w};
-            v4i codes;
-#pragma unroll
-            for (unsigned j = 0; j < 4u; ++j)
-                codes[j] = c % 2u == 0u ? (int)__builtin_amdgcn_alignbyte(q[at + j + 1u], q[at + j], 2u) : (int)q[at + j];
-            return codes;
-        };
-        v16i dot[2];
-        float d_w = 0.0f;
-        // (eight results at a time, one kind of instruction after another: a dependent instruction
-        // issues nine cycles behind its producer, and left alone the three of a result follow each other)
-        auto scale = [&](unsigned t, unsigned c) {
-#pragma unroll
-            for (int half = 0; half < 16; half += 8) {
-                float value[8], step[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) step[i] = d_w * d_a[t][half + i];
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) value[i] = bias.value(dot[t][half + i]);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    total[t][half + i] = c == 0u ? step[i] * value[i] : __builtin_fmaf(step[i], value[i], total[t][half + i]);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        };
-        read_block(0u);       // (ahead of the scales, which the first matrix instruction does not wait for)
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (unsigned t = 0; t < 2u; ++t)
-#pragma unroll
-            for (unsigned q = 0; q < 4u; ++q) {
-                const uint4 d = read16(scales + (32u * t + 8u * q) * 4u);
-                d_a[t][4u * q] = __uint_as_float(d.x); d_a[t][4u * q + 1u] = __uint_as_float(d.y);
-                d_a[t][4u * q + 2u] = __uint_as_float(d.z); d_a[t][4u * q + 3u] = __uint_as_float(d.w);
-            }
-#pragma unroll
-        for (unsigned c = 0; c < 8u; ++c) {
-            if (c + 1u < 8u) read_block(c + 1u);
-            const v4i codes = codes_of(c);
-            dot[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(tokens[c % 2u][0], codes, bias.start, 0, 0, 0);
-            // (the scheduler would put the scaling of the results first and wait for them there)
-            __builtin_amdgcn_sched_barrier(0);
-            if (c) scale(1u, c - 1u);
-            __builtin_amdgcn_sched_barrier(0);
-            d_w = f16_bits_to_float(scale_bits[c % 2u]);
-            dot[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(tokens[c % 2u][1], codes, bias.start, 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            scale(0u, c);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        scale(1u, 7u);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            acc[0][i] += (double)total[0][i];
-            acc[1][i] += (double)total[1][i];
-        }
+        q80_superblock(buffer * kWideWeightBytes + (32u * row_block + r) * kStagedPitch,
+                       kWideActBase + buffer * kWideActBytes + (32u * token_block + r) * kStagedPitch + 16u * h,
+                       kWideScaleBase + buffer * (kWideTokens * 4u) + (32u * token_block + 4u * h) * 4u, h, minus, acc);
         // the next superblock's copies have landed and every wave is done with this one's buffers
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
@@ -594,17 +558,15 @@ __global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80A
     if (row >= g.row_count) return;
     bool bad = false;
 #pragma unroll
-    for (unsigned t = 0; t < 2u; ++t)
-#pragma unroll
-        for (unsigned i = 0; i < 16u; ++i) {
-            const unsigned long long token = tok0 + 64u * token_pair + 32u * t + 8u * (i >> 2) + 4u * h + (i & 3u);
-            if (token >= g.input_rows) continue;
-            const unsigned long long at = token * g.out_stride + row;
-            const float sum = (float)acc[t][i];
-            const float value = g.additive ? sum + g.additive[at] : sum;
-            if (!finite_f32(value)) bad = true;
-            else g.out[at] = g.output_bf16 ? bf16_round(value) : value;
-        }
+    for (unsigned i = 0; i < 16u; ++i) {
+        const unsigned long long token = tok0 + 32u * token_block + 8u * (i >> 2) + 4u * h + (i & 3u);
+        if (token >= g.input_rows) continue;
+        const unsigned long long at = token * g.out_stride + row;
+        const float sum = (float)acc[i];
+        const float value = g.additive ? sum + g.additive[at] : sum;
+        if (!finite_f32(value)) bad = true;
+        else g.out[at] = g.output_bf16 ? bf16_round(value) : value;
+    }
     if (bad) raise_status(g.status, 1);
 }
 
@@ -626,9 +588,9 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
                    (const unsigned char *)act_q8k, input_rows, additive, out, out_stride,
                    output_bf16 ? 1 : 0, status, encoded_second, out_second};
     // Which tiles: a pass over the row width costs a workgroup about the same whatever the device's
-    // load (measured at 16 superblocks a row, microseconds: 17 unstaged and 27 once two such
+    // load (measured at 16 superblocks a row, microseconds: 14 on the 32-row tile and 18.5 once two such
     // workgroups share a compute unit, 29 on the 64-row staged tile and 43 once two of them share
-    // a compute unit, 35 on the 128-row tile, 56 on the 128 x 128 tile), so the choice is the number of
+    // a compute unit, 35 on the 128-row tile, 54 on the 128 x 128 tile), so the choice is the number of
     // rounds each shape needs.
     const uint64_t token_tiles32 = (input_rows + 31u) / 32u;
     const uint64_t token_tiles64 = (input_rows + 63u) / 64u;
@@ -647,13 +609,13 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
         const uint64_t plain = matrices * row_tiles * token_tiles32;
         const uint64_t tall = matrices * ((row_count + 127u) / 128u) * token_tiles64,
                        low = matrices * ((row_count + 63u) / 64u) * token_tiles64;
-        const double plain_cost = plain <= units ? 17.0 : 27.0 * (double)((plain + 2u * units - 1u) / (2u * units));
+        const double plain_cost = plain <= units ? 14.0 : 18.5 * (double)((plain + 2u * units - 1u) / (2u * units));
         const double low_share = 43.0 * (double)low / (double)(2u * units);
         const double low_cost = low <= units ? 29.0 : (low_share > 43.0 ? low_share : 43.0);
         const double tall_cost = 35.0 * (double)((tall + units - 1u) / units);
         const uint64_t token_tiles128 = (input_rows + 127u) / 128u;
         const uint64_t wide = matrices * ((row_count + 127u) / 128u) * token_tiles128;
-        const double wide_cost = 56.0 * (double)((wide + units - 1u) / units);
+        const double wide_cost = 54.0 * (double)((wide + units - 1u) / units);
         // (32-bit offsets into a tile's rows)
         if (wide_cost < plain_cost && wide_cost <= low_cost && wide_cost <= tall_cost &&
             row_bytes <= (1ull << 24) && row_width / 256u * kQ8KBytes <= (1ull << 24)) {
@@ -675,7 +637,9 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
             return check_launch("dense_q8_0_staged");
         }
     }
-    dense_q8_0_kernel<<<dim3((unsigned)row_tiles, (unsigned)token_tiles32, (unsigned)matrices), 64 * kPlainWaves, 0, stream>>>(g);
+    YVEX_ALLOW_DYNAMIC_LDS(dense_q8_0_kernel, kPlainLdsBytes);
+    dense_q8_0_kernel<<<dim3((unsigned)row_tiles, (unsigned)token_tiles32, (unsigned)matrices), 64 * kPlainWaves, kPlainLdsBytes,
+                        stream>>>(g);
     return check_launch("dense_q8_0");
 }
 
