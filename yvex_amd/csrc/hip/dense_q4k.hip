@@ -264,76 +264,114 @@ __global__ __launch_bounds__(256) void dense_q4k_kernel(DenseQ4kArgs g)
     }
 }
 
-// The same product for 16 to 32 input rows on V_MFMA_I32_16X16X64_I8: a workgroup owns 16
-// weight rows x 16 or 32 tokens, so a batch of 16 wastes no token slot and twice as many
-// workgroups share the matrix; eight waves (two per SIMD) take every eighth superblock. One K
+// LDS of a wave of the kernel below: 16 weight rows' superblock (144 bytes a row), 16 input rows' codes, sums and scale
+// (256, 32 and 4 bytes of 304 a row, which spreads the rows over the banks).
+constexpr unsigned kSmallWeights = 16u * 144u, kSmallActPitch = 304u, kSmallWindow = kSmallWeights + 16u * kSmallActPitch;
+
+// The same product for few input rows on V_MFMA_I32_16X16X64_I8: a workgroup owns 16
+// weight rows x 16 tokens, so a batch of 16 wastes no token slot and twice as many
+// workgroups share the matrix; its waves take every eighth superblock, or every fourth. One K
 // step is a 64-value nibble group, i.e. two sub-blocks, which is fine because the limbs already
 // carry their sub-block's scale. Lane (r, q) holds bytes 16q..16q+15 of weight row r's group as
 // the A operand (q = 0, 1: low nibbles of nibble bytes 16q.., the first sub-block; q = 2, 3:
 // high nibbles of nibble bytes 16(q-2).., the second) and the same positions of token r's
 // activations as the B operand; accumulator i of that lane is weight row 4 q + i against token r.
-template <unsigned NT>
-__global__ __launch_bounds__(512) void dense_q4k16_kernel(DenseQ4kArgs g)
+// Lanes that loaded their own pieces took twenty instructions of 16 to 32 cache lines a superblock, at two cycles
+// a line 12 of the 14 us of 2048 x 7168 by 19. Loads take consecutive pieces of consecutive rows now, a superblock ahead,
+// and the bytes pass through a window of LDS of the wave's own. 2048 x 7168 by 19 rows 13.6 -> 8.2 us, by 4
+// 8.8 -> 7.7, 4096 x 4096 by 32 12.4 -> 9.2.
+template <unsigned WAVES>
+__global__ __launch_bounds__(64 * WAVES) void dense_q4k16_kernel(DenseQ4kArgs g)
 {
     typedef int v4s __attribute__((ext_vector_type(4)));
-    __shared__ __align__(16) float row_scale[8][2][16];
-    __shared__ double partial[7][NT][4][64];
-    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    typedef int v4i_dword __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr unsigned kActPieces = 18u, kActLoads = (16u * kActPieces + 63u) / 64u;        // of 16 rows: 4.5 instructions
+    __shared__ __align__(16) float row_scale[WAVES][2][16];
+    __shared__ __align__(16) unsigned char windows[WAVES * kSmallWindow + 1024u];    // (and where lanes without a piece write)
+    double (*const partial)[4][64] = reinterpret_cast<double (*)[4][64]>(windows);     // when the superblocks are done
+    static_assert((WAVES - 1u) * 4u * 64u * sizeof(double) <= WAVES * kSmallWindow, "the partial tiles fit the windows");
+    const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const unsigned r = lane & 15u, q = lane >> 4;
     const unsigned long long row0 = (unsigned long long)blockIdx.x * 16ull;
-    const unsigned long long tok0 = (unsigned long long)blockIdx.y * (16ull * NT);
-    unsigned long long wr = row0 + r;
-    if (wr >= g.row_count) wr = g.row_count - 1ull;
-    const unsigned char *wrow = g.encoded + wr * g.row_bytes;
-    const unsigned char *arow[NT];
+    const unsigned long long tok0 = (unsigned long long)blockIdx.y * 16ull;
+    const unsigned rows_here = (unsigned)(g.row_count - row0 < 16ull ? g.row_count - row0 : 16ull);
+    const unsigned toks_here = (unsigned)(g.input_rows - tok0 < 16ull ? g.input_rows - tok0 : 16ull);
     const unsigned long long act_row_bytes = (unsigned long long)g.blocks * kQ8KBytes;
-#pragma unroll
-    for (unsigned nt = 0; nt < NT; ++nt) {
-        unsigned long long t = tok0 + 16ull * nt + r;
-        if (t >= g.input_rows) t = g.input_rows - 1ull;
-        arow[nt] = g.act + t * act_row_bytes;
-    }
-    double acc[NT][4];
-#pragma unroll
-    for (unsigned nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[nt][i] = 0.0;
+    const unsigned char *const weights = g.encoded + row0 * g.row_bytes, *const acts = g.act + tok0 * act_row_bytes;
+    unsigned char *const window = windows + wave * kSmallWindow, *const spare = windows + WAVES * kSmallWindow + 16u * lane;
 
-    for (unsigned sb = wave; sb < g.blocks; sb += 8u) {
-        const unsigned char *w = wrow + (unsigned long long)sb * 144ull;
-        const unsigned head = *reinterpret_cast<const unsigned *>(w);
-        const uint3 scales = *reinterpret_cast<const uint3 *>(w + 4u);
+    // the lane's pieces (a ragged edge repeats the last row) and their places in the window
+    const unsigned char *weight_at[3], *act_at[kActLoads];
+    unsigned char *act_to[kActLoads];
+#pragma unroll
+    for (unsigned k = 0; k < 3u; ++k) {
+        const unsigned piece = k < 2u ? 64u * k + lane : 128u + r, row = piece / 9u;
+        weight_at[k] = weights + (row < rows_here ? row : rows_here - 1u) * g.row_bytes + 16u * (piece - 9u * row);
+    }
+#pragma unroll
+    for (unsigned k = 0; k < kActLoads; ++k) {
+        const unsigned piece = 64u * k + lane, held = piece < 16u * kActPieces ? piece : 16u * kActPieces - 1u;
+        const unsigned token = held / kActPieces, part = held - kActPieces * token;
+        act_at[k] = acts + (token < toks_here ? token : toks_here - 1u) * act_row_bytes + 4u + 16u * part;
+        act_to[k] = piece == held ? window + kSmallWeights + token * kSmallActPitch + 16u * part : spare;
+    }
+    const unsigned char *const scale_at = acts + (r < toks_here ? r : toks_here - 1u) * act_row_bytes;
+    unsigned char *const scale_to = lane < 16u ? window + kSmallWeights + lane * kSmallActPitch + 288u : spare;
+    struct {
+        v4i weights[3], acts[kActLoads];
+        unsigned scale;
+    } ahead;
+    auto request = [&](unsigned sb) {
+        const unsigned long long w = sb * 144ull, a = (unsigned long long)sb * kQ8KBytes;
+#pragma unroll
+        for (unsigned k = 0; k < 3u; ++k) ahead.weights[k] = *reinterpret_cast<const v4i_dword *>(weight_at[k] + w);
+#pragma unroll
+            for (unsigned k = 0; k < kActLoads; ++k) ahead.acts[k] = *reinterpret_cast<const v4i_dword *>(act_at[k] + a);
+        ahead.scale = *reinterpret_cast<const unsigned *>(scale_at + a);
+    };
+
+    double acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = 0.0;
+
+    if (wave < g.blocks) request(wave);
+    for (unsigned sb = wave; sb < g.blocks; sb += WAVES) {
+        // (LDS operations of one wave complete in order)
+#pragma unroll
+        for (unsigned k = 0; k < 2u; ++k) *reinterpret_cast<v4i *>(window + 1024u * k + 16u * lane) = ahead.weights[k];
+        *reinterpret_cast<v4i *>(window + 2048u + 16u * r) = ahead.weights[2];
+#pragma unroll
+        for (unsigned k = 0; k < kActLoads; ++k) *reinterpret_cast<v4i *>(act_to[k]) = ahead.acts[k];
+        *reinterpret_cast<unsigned *>(scale_to) = ahead.scale;
+        request(sb + WAVES < g.blocks ? sb + WAVES : sb);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const unsigned char *const w = window + 144u * r;
+        const uint4 opening = *reinterpret_cast<const uint4 *>(w);
+        const unsigned head = opening.x;
         uint4 qs[4];
 #pragma unroll
         for (unsigned j = 0; j < 4u; ++j)
             qs[j] = *reinterpret_cast<const uint4 *>(w + 16u + 32u * j + 16u * (q & 1u));
-        uint4 a[NT][4], bsums[NT][2];
-        float da[NT];
+        uint4 a[4], bsums[2];
+        float da;
+        const unsigned char *ab = window + kSmallWeights + r * kSmallActPitch;
+        da = *reinterpret_cast<const float *>(ab + 288u);
 #pragma unroll
-        for (unsigned nt = 0; nt < NT; ++nt) {
-            const unsigned char *ab = arow[nt] + (unsigned long long)sb * kQ8KBytes;
-            da[nt] = *reinterpret_cast<const float *>(ab);
-#pragma unroll
-            for (unsigned j = 0; j < 4u; ++j) {
-                const unsigned *p = reinterpret_cast<const unsigned *>(ab + 4u + 64u * j + 16u * q);
-                a[nt][j] = make_uint4(p[0], p[1], p[2], p[3]);
-            }
-            const unsigned *b = reinterpret_cast<const unsigned *>(ab + 260u);
-            bsums[nt][0] = make_uint4(b[0], b[1], b[2], b[3]);
-            bsums[nt][1] = make_uint4(b[4], b[5], b[6], b[7]);
-        }
-        const unsigned s0 = scales.x, s1 = scales.y, s2 = scales.z;
+        for (unsigned j = 0; j < 4u; ++j) a[j] = *reinterpret_cast<const uint4 *>(ab + 64u * j + 16u * q);
+        bsums[0] = *reinterpret_cast<const uint4 *>(ab + 256u);
+        bsums[1] = *reinterpret_cast<const uint4 *>(ab + 272u);
+        const unsigned s0 = opening.y, s1 = opening.z, s2 = opening.w;
         const unsigned sc_pack[2] = {s0 & 0x3f3f3f3fu, (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u)};
         const unsigned mn_pack[2] = {s1 & 0x3f3f3f3fu, ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u)};
         if (q == 0u) {
             row_scale[wave][0][r] = f16_bits_to_float(head & 0xffffu);
             row_scale[wave][1][r] = f16_bits_to_float(head >> 16);
         }
-        v4s lo_sum[NT], hi_sum[NT];
+        v4s lo_sum, hi_sum;
 #pragma unroll
-        for (unsigned nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) lo_sum[nt][i] = hi_sum[nt][i] = 0;
+        for (int i = 0; i < 4; ++i) lo_sum[i] = hi_sum[i] = 0;
         const unsigned high = q >> 1;                          // this lane decodes the high nibbles
 #pragma unroll
         for (unsigned j = 0; j < 4u; ++j) {
@@ -346,32 +384,26 @@ __global__ __launch_bounds__(512) void dense_q4k16_kernel(DenseQ4kArgs g)
             limbs(qs[j].y >> shift, sc, lo, hi); a_lo[1] = (int)lo; a_hi[1] = (int)hi;
             limbs(qs[j].z >> shift, sc, lo, hi); a_lo[2] = (int)lo; a_hi[2] = (int)hi;
             limbs(qs[j].w >> shift, sc, lo, hi); a_lo[3] = (int)lo; a_hi[3] = (int)hi;
-#pragma unroll
-            for (unsigned nt = 0; nt < NT; ++nt) {
-                const v4i b = as_v4i(a[nt][j]);
-                lo_sum[nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_lo, b, lo_sum[nt], 0, 0, 0);
-                hi_sum[nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_hi, b, hi_sum[nt], 0, 0, 0);
-            }
+            const v4i b = as_v4i(a[j]);
+            lo_sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_lo, b, lo_sum, 0, 0, 0);
+            hi_sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(a_hi, b, hi_sum, 0, 0, 0);
         }
         v4i m_op = {0, 0, 0, 0};
         if (q == 0u) {
             m_op[0] = (int)mn_pack[0];
             m_op[1] = (int)mn_pack[1];
         }
-        v4s min_lo[NT], min_hi[NT];
-#pragma unroll
-        for (unsigned nt = 0; nt < NT; ++nt) {
-            uint2 bl, bh;
-            bsum_limbs(bsums[nt], bl, bh);
-            v4i b_lo = {0, 0, 0, 0}, b_hi = {0, 0, 0, 0};
-            if (q == 0u) {
-                b_lo[0] = (int)bl.x; b_lo[1] = (int)bl.y;
-                b_hi[0] = (int)bh.x; b_hi[1] = (int)bh.y;
-            }
-            const v4s zero = {0, 0, 0, 0};
-            min_lo[nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(m_op, b_lo, zero, 0, 0, 0);
-            min_hi[nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(m_op, b_hi, zero, 0, 0, 0);
+        v4s min_lo, min_hi;
+        uint2 bl, bh;
+        bsum_limbs(bsums, bl, bh);
+        v4i b_lo = {0, 0, 0, 0}, b_hi = {0, 0, 0, 0};
+        if (q == 0u) {
+            b_lo[0] = (int)bl.x; b_lo[1] = (int)bl.y;
+            b_hi[0] = (int)bh.x; b_hi[1] = (int)bh.y;
         }
+        const v4s zero = {0, 0, 0, 0};
+        min_lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(m_op, b_lo, zero, 0, 0, 0);
+        min_hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(m_op, b_hi, zero, 0, 0, 0);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -381,41 +413,35 @@ __global__ __launch_bounds__(512) void dense_q4k16_kernel(DenseQ4kArgs g)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (unsigned nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int dot = (hi_sum[nt][i] << 3) + lo_sum[nt][i];
-                const int minimum = (min_hi[nt][i] << 7) + min_lo[nt][i];
-                const float left = (da[nt] * d_of[i]) * (float)dot;
-                const float right = (da[nt] * dmin_of[i]) * (float)minimum;
-                acc[nt][i] += (double)(left - right);
-            }
+        for (int i = 0; i < 4; ++i) {
+            const int dot = (hi_sum[i] << 3) + lo_sum[i];
+            const int minimum = (min_hi[i] << 7) + min_lo[i];
+            const float left = (da * d_of[i]) * (float)dot;
+            const float right = (da * dmin_of[i]) * (float)minimum;
+            acc[i] += (double)(left - right);
+        }
     }
 
+    __syncthreads();
     if (wave) {
 #pragma unroll
-        for (unsigned nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) partial[wave - 1u][nt][i][lane] = acc[nt][i];
+        for (int i = 0; i < 4; ++i) partial[wave - 1u][i][lane] = acc[i];
     }
     __syncthreads();
     if (wave) return;
+    const unsigned long long token = tok0 + r;
 #pragma unroll
-    for (unsigned nt = 0; nt < NT; ++nt) {
-        const unsigned long long token = tok0 + 16ull * nt + r;
+    for (int i = 0; i < 4; ++i) {
+        const unsigned long long row = row0 + 4u * q + (unsigned)i;
+        double wide = acc[i];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const unsigned long long row = row0 + 4u * q + (unsigned)i;
-            double wide = acc[nt][i];
-#pragma unroll
-            for (unsigned wv = 0; wv < 7u; ++wv) wide += partial[wv][nt][i][lane];
-            const float sum = (float)wide;
-            if (row >= g.row_count || token >= g.input_rows) continue;
-            const unsigned long long at = token * g.out_stride + row;
-            const float value = g.additive ? sum + g.additive[at] : sum;
-            if (!finite_f32(value)) raise_status(g.status, 1);
-            else g.out[at] = g.output_bf16 ? bf16_round(value) : value;
-        }
+        for (unsigned wv = 0; wv + 1u < WAVES; ++wv) wide += partial[wv][i][lane];
+        const float sum = (float)wide;
+        if (row >= g.row_count || token >= g.input_rows) continue;
+        const unsigned long long at = token * g.out_stride + row;
+        const float value = g.additive ? sum + g.additive[at] : sum;
+        if (!finite_f32(value)) raise_status(g.status, 1);
+        else g.out[at] = g.output_bf16 ? bf16_round(value) : value;
     }
 }
 
@@ -434,27 +460,26 @@ int launch_q4k_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t r
     DenseQ4kArgs g{encoded, row_count, row_bytes, (unsigned)(row_width / 256u),
                    (const unsigned char *)act_q8k, input_rows, additive, out, out_stride,
                    output_bf16 ? 1 : 0, status};
-    if (input_rows <= 32u) {
-        const uint64_t small_tiles = (row_count + 15u) / 16u;
-        if (small_tiles > 0x7fffffffull) return ST_BOUNDS;
-        if (input_rows <= 16u) dense_q4k16_kernel<1><<<dim3((unsigned)small_tiles, 1), 512, 0, stream>>>(g);
-        else dense_q4k16_kernel<2><<<dim3((unsigned)small_tiles, 1), 512, 0, stream>>>(g);
+    // 16 x 16 tiles, on four waves where several workgroups share a compute unit (7168 x 7168 by 32 rows 23.2 us, on
+    // eight 26.8; 7168 x 2048 by 32 9.8 and 13.1), up to 32 input rows and beyond them while tiles of twice the tokens would fit
+    // the device in one round (2048 x 7168 by 64 rows 12.7 us, on the 32 x 32 tiles 16.7).
+    const uint64_t units = (uint64_t)compute_units(), small_tiles = (row_count + 15u) / 16u;
+    const uint64_t token_tiles16 = (input_rows + 15u) / 16u, token_tiles32 = (input_rows + 31u) / 32u;
+    if (input_rows <= 32u || small_tiles * token_tiles32 <= units) {
+        if (small_tiles > 0x7fffffffull || token_tiles16 > 65535ull) return ST_BOUNDS;
+        const dim3 grid((unsigned)small_tiles, (unsigned)token_tiles16);
+        if (small_tiles * token_tiles16 <= units) dense_q4k16_kernel<8><<<grid, 512, 0, stream>>>(g);
+        else dense_q4k16_kernel<4><<<grid, 256, 0, stream>>>(g);
     } else {
         const uint64_t token_tiles = (input_rows + 63u) / 64u;
-        if (token_tiles > 65535ull) return ST_BOUNDS;
         // enough (128 rows x 64 tokens) tiles for every compute unit: operands staged through LDS
-        if ((row_count + 127u) / 128u * token_tiles >= compute_units())
+        if ((row_count + 127u) / 128u * token_tiles >= units)
             return launch_q4k_rows_staged(encoded, row_count, row_width, row_bytes, act_q8k, input_rows,
                                           additive, out, out_stride, output_bf16, status, stream);
         // A workgroup's pass over the row width takes about as long on a full device as on an
         // empty one, so while the smaller tiles still fit the device in one round they are the
-        // faster ones (2048 x 7168 at 64 rows: 25 us on 32 x 64 tiles, 17 us on 32 x 32, 16 us on
-        // 16 x 32; at 256 rows 29, 33 and 49 us).
-        const uint64_t token_tiles32 = (input_rows + 31u) / 32u, small_tiles = (row_count + 15u) / 16u;
-        const uint64_t units = (uint64_t)compute_units();
-        if (small_tiles * token_tiles32 <= units)
-            dense_q4k16_kernel<2><<<dim3((unsigned)small_tiles, (unsigned)token_tiles32), 512, 0, stream>>>(g);
-        else if (row_tiles * token_tiles32 <= units)
+        // faster ones (2048 x 7168 at 96 rows: 17 us on 32 x 32 tiles, 21 on 16 x 32; at 256 rows 27 us on 32 x 64).
+        if (row_tiles * token_tiles32 <= units)
             dense_q4k_kernel<1><<<dim3((unsigned)row_tiles, (unsigned)token_tiles32), 256, 0, stream>>>(g);
         else
             dense_q4k_kernel<2><<<dim3((unsigned)row_tiles, (unsigned)token_tiles), 256, 0, stream>>>(g);
