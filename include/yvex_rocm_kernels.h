@@ -68,7 +68,7 @@ int yvex_hip_concat_rows_bf16(const float *head, const float *tail, uint64_t row
                               uint64_t head_width, uint64_t tail_width, float *out, int *status,
                               yvex_hip_stream stream);
 
-/* yvex_hip_matvec for F32 weight rows and a decode-width batch of F32 input rows (8 to 255: the
+/* yvex_hip_matvec for F32 weight rows and a batch of F32 input rows (8 or more: the
  * router projection of the MoE row batch, src/backend/cuda/moe.c:1259-1284), given scratch memory
  * (8-byte aligned): the row width is split between workgroups so that the whole device takes
  * part, the partial sums (doubles) go to scratch and a second launch adds them in split order

@@ -387,3 +387,32 @@ def test_iq2_rows_of_tall_matrices_are_the_sweeps_bits(gpu, oracle, rows, inputs
                         input_rows=some.shape[0], status=status)
         assert same_bits(got[at:at + 7], want)
     assert int(status.item()) == 0
+
+
+# the 32-row tiles of the F32 projection: ragged on both sides, fewer columns than waves, one launch and split, 16 and 32
+# input rows a tile; formats other than F32 (one launch)
+@pytest.mark.parametrize("qtype,rows,width,inputs", [
+    ("F32", 1, 128, 257), ("F32", 250, 1024, 1570), ("F32", 33, 16512, 17), ("F32", 65, 2176, 301), ("F32", 255, 4096, 97),
+    ("F16", 31, 64, 256), ("BF16", 33, 320, 511), ("Q8_0", 97, 448, 289)])
+def test_f32_tiles_of_32_weight_rows_match_float64(gpu, oracle, qtype, rows, width, inputs):
+    """Sums of exact products in double, rounded once: half a unit in the last place and the double
+    sums' own error, which a sum of `width` terms bounds by width 2^-52 of the terms' magnitudes."""
+    from yvex_amd import kernels as K
+    qt = getattr(oracle, qtype)
+    g = oracle.Generator(42, f"tile32.{qtype}.{rows}.{width}.{inputs}")
+    x = g.normal(inputs * width).reshape(inputs, width)
+    if qtype in ("F16", "BF16"):
+        half = torch.from_numpy(g.normal(rows * width)).to(torch.float16 if qtype == "F16" else torch.bfloat16)
+        w = half.view(torch.uint8).numpy()
+    else:
+        w = g.weights(qt, rows, width)
+    values = oracle.decode_rows(qt, w, width).reshape(rows, width).astype(np.float64)
+    status = K.new_status(gpu)
+    want = x.astype(np.float64) @ values.T
+    slack = np.abs(want) * 2.0 ** -24 + width * 2.0 ** -52 * (np.abs(x.astype(np.float64)) @ np.abs(values).T)
+    one = K.matvec(dev(w, gpu), qt, rows, width, dev(x, gpu), status=status).cpu().numpy()
+    assert np.all(np.abs(one - want) <= slack)
+    if qtype == "F32":
+        split = K.matvec_f32_rows(dev(w.view(np.float32).reshape(rows, width), gpu), dev(x, gpu), status).cpu().numpy()
+        assert np.all(np.abs(split - want) <= slack)
+    assert int(status.item()) == 0

@@ -14,7 +14,8 @@
 //
 // A workgroup owns 32 weight rows x 32 input rows; its four waves take every fourth superblock
 // (eight blocks, 272 bytes a row) and their partial tiles are added in wave order, so results do
-// not depend on timing. The input rows are the A operand and the weight rows the B operand: lane (r, h) holds bytes 16 h .. 16 h + 15 of input row r's block and
+// not depend on timing. The input rows are the A operand and the weight rows the B operand: lane (r, h) holds bytes
+// 16 h .. 16 h + 15 of input row r's block and
 // of weight row r's block, and accumulator i of that lane is weight row r against input row
 // 8 (i / 4) + 4 h + i % 4, so a block's scale is one value a lane. Blocks start on 2-byte
 // boundaries (34 bytes each): the codes of an even block are read as five aligned dwords and

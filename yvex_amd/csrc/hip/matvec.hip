@@ -665,123 +665,122 @@ __global__ __launch_bounds__(WAVES * 64) void matvec_f32_tile16_kernel(MatvecArg
     }
 }
 
-// The same product for a batch of several hundred input rows or more (the router projection of a prefill
-// batch): with one 16 x 16 tile a workgroup every wave loads its own operands, four bytes for
-// every matrix-core flop, and the launch runs at what the caches deliver (27 TFLOP/s where the
-// instruction alone sustains 75). Here a workgroup of sixteen waves, four a SIMD, owns 32 weight rows x
-// INPUTS input rows and stages 128 columns of both in LDS (a 528-byte pitch keeps the sixteen rows that one
-// 16-byte read phase touches on sixteen different bank groups), the next chunk's loads in flight while the
-// current one is multiplied. Two 16-row halves of the weights times INPUTS / 16 blocks of input rows are the
-// tiles; the waves of a tile share a chunk's eight steps out among themselves and their sums are added
-// at the end, in wave order. (One wave a tile, two a SIMD, left the matrix pipe idle half the time:
-// 256 x 7168 by 2048 rows 205 us, 165 now; the matrix instructions alone are 104.)
-constexpr unsigned kF32BlockColumns = 128u, kF32BlockPitch = kF32BlockColumns * 4u + 16u;
-constexpr unsigned kF32BlockWeightRows = 32u, kF32BlockWaves = 16u;
-constexpr unsigned f32_block_lds(unsigned inputs) { return 2u * (kF32BlockWeightRows + inputs) * kF32BlockPitch; }
+// The same product for a batch of input rows on tiles of 32 weight rows x INPUTS input rows whose waves split the row
+// width (and workgroups do: blockIdx.z, as above). The matrix instructions bound it: 64 cycles each, 54 us of the
+// device for 256 x 7168 by 1111 rows. So the operands must come at half the bytes and a quarter of the cache lines that
+// a 16 x 16 tile asks for: a wave loads 32 columns of its tile's rows as consecutive 16-byte pieces, eight lanes a row,
+// 32 columns ahead, passes them through a window of LDS of its own (144 bytes a row: the sixteen rows that a read
+// touches lie on different banks) and needs no barrier before the sums are added.
+// 256 x 7168 by 64 / 256 / 512 / 1111 / 2048 rows 18.7 / 38.6 / 62.6 / 136 / 168 us -> 14.0 / 25.0 / 40.8 / 87.0 / 131, with
+// the join.
+constexpr unsigned kTile32Columns = 32u, kTile32Pitch = kTile32Columns * 4u + 16u, kTile32Waves = 8u;
 
 template <unsigned QT, unsigned INPUTS>
-__global__ __launch_bounds__(64 * kF32BlockWaves) void matvec_f32_block_kernel(MatvecArgs a)
+__global__ __launch_bounds__(kTile32Waves * 64) void matvec_f32_tile32_kernel(MatvecArgs a)
 {
+    constexpr unsigned WAVES = kTile32Waves;
     typedef double v4d __attribute__((ext_vector_type(4)));
     typedef float v4f __attribute__((ext_vector_type(4)));
-    constexpr unsigned kRows = kF32BlockWeightRows + INPUTS;
-    constexpr unsigned kPieces = kF32BlockColumns / 4u;                   // 16-byte pieces a row
-    constexpr unsigned kThreads = 64u * kF32BlockWaves;
-    constexpr unsigned kHeld = (kRows * kPieces + kThreads - 1u) / kThreads;
-    constexpr unsigned kTiles = INPUTS / 8u, kSplits = kF32BlockWaves / kTiles;      // waves a tile
-    constexpr unsigned kSteps = kF32BlockColumns / 16u / kSplits;         // of a chunk, a wave
-    static_assert(kSteps * kSplits * 16u == kF32BlockColumns && kRows * kPieces % 512u == 0u, "whole shares");
-    static_assert((kSplits - 1u) * kTiles * 4u * 64u * 8u <= f32_block_lds(INPUTS), "the partial sums fit the stages");
-    extern __shared__ __align__(16) unsigned char staged[];               // [2][kRows * kF32BlockPitch]
-    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    constexpr unsigned kRows = 32u + INPUTS, kWindow = kRows * kTile32Pitch, kTiles = INPUTS / 8u;
+    constexpr unsigned kInputLoads = INPUTS / 8u;
+    static_assert((WAVES - 1u) * kTiles * 4u * 64u * 8u <= WAVES * kWindow, "the partial sums fit the windows");
+    __shared__ __align__(16) unsigned char windows[WAVES * kWindow];
+    const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const unsigned i16 = lane & 15u, q = lane >> 4;
-    // staging: piece p = threadIdx.x + 1024 j of the chunk is columns 4 (p % 32) .. + 3 of staged
-    // row p / 32 (weight rows first, then input rows); 32 lanes read one row's 512 bytes. Threads whose
-    // last piece lies behind the rows repeat the last row's.
-    const unsigned char *source[kHeld];       // (weight rows: F32, F16, BF16 or Q8_0 values; input rows: F32)
-    unsigned target[kHeld];
+    const unsigned long long row0 = (unsigned long long)blockIdx.x * 32ull, in0 = (unsigned long long)blockIdx.y * INPUTS;
+    const unsigned weights_here = (unsigned)(a.row_count - row0 < 32ull ? a.row_count - row0 : 32ull);
+    const unsigned inputs_here = (unsigned)(a.input_rows - in0 < INPUTS ? a.input_rows - in0 : INPUTS);
+    unsigned char *const window = windows + wave * kWindow;
+    // the lane's pieces: columns 4 (lane % 8) .. + 3 of rows lane / 8 + 8 k (a ragged edge repeats the last row)
+    const unsigned piece = lane & 7u;
+    const unsigned char *weight_at[4];
+    const float *input_at[kInputLoads];
 #pragma unroll
-    for (unsigned j = 0; j < kHeld; ++j) {
-        const unsigned p = threadIdx.x + kThreads * j, piece = p % kPieces;
-        const unsigned row = p / kPieces < kRows ? p / kPieces : kRows - 1u;
-        if (row < kF32BlockWeightRows) {
-            unsigned long long wrow = (unsigned long long)blockIdx.x * kF32BlockWeightRows + row;
-            if (wrow >= a.row_count) wrow = a.row_count - 1ull;          // a ragged edge repeats the last row
-            source[j] = a.encoded + wrow * a.row_bytes;       // (a weight row: columns from 4 * piece on)
-        } else {
-            unsigned long long in = (unsigned long long)blockIdx.y * INPUTS + (row - kF32BlockWeightRows);
-            if (in >= a.input_rows) in = a.input_rows - 1ull;
-            source[j] = (const unsigned char *)((const float *)a.input + in * a.input_stride + 4u * piece);
-        }
-        target[j] = row * kF32BlockPitch + 16u * piece;
+    for (unsigned k = 0; k < 4u; ++k) {
+        const unsigned row = 8u * k + (lane >> 3);
+        weight_at[k] = a.encoded + (row0 + (row < weights_here ? row : weights_here - 1u)) * a.row_bytes;
     }
-    const unsigned chunks = (unsigned)(a.row_width / kF32BlockColumns);
-    v4f held[kHeld];
+#pragma unroll
+    for (unsigned k = 0; k < kInputLoads; ++k) {
+        const unsigned row = 8u * k + (lane >> 3);
+        input_at[k] = (const float *)a.input + (in0 + (row < inputs_here ? row : inputs_here - 1u)) * a.input_stride + 4u * piece;
+    }
+    unsigned char *const to = window + (lane >> 3) * kTile32Pitch + 16u * piece;
+    const unsigned char *const from = window + i16 * kTile32Pitch + 16u * q;
+    const unsigned chunks = (unsigned)(a.row_width / kTile32Columns), shares = gridDim.z * WAVES;
+    const unsigned share = blockIdx.z * WAVES + wave;
+    const unsigned begin = (unsigned)((unsigned long long)chunks * share / shares);
+    const unsigned end = (unsigned)((unsigned long long)chunks * (share + 1u) / shares);
+    v4f weights[4], inputs[kInputLoads];
     unsigned bad = 0u;
-    // piece 0 of every thread is a piece of a weight row, the others are of input rows
-    static_assert(kF32BlockWeightRows * kPieces == kThreads, "the weight rows are the threads' first pieces");
-    auto fetch = [&](unsigned j, unsigned chunk) -> v4f {
-        if (j == 0u) {
-            const float4 w = scalar_weights4<QT>(source[0], (unsigned long long)chunk * kF32BlockColumns + 4u * (threadIdx.x % kPieces));
-            return v4f{w.x, w.y, w.z, w.w};
+    auto request = [&](unsigned chunk) {
+#pragma unroll
+        for (unsigned k = 0; k < 4u; ++k) {
+            const float4 w = scalar_weights4<QT>(weight_at[k], (unsigned long long)chunk * kTile32Columns + 4u * piece);
+            weights[k] = v4f{w.x, w.y, w.z, w.w};
         }
-        return *reinterpret_cast<const v4f *>(source[j] + (unsigned long long)chunk * kF32BlockColumns * 4ull);
+#pragma unroll
+        for (unsigned k = 0; k < kInputLoads; ++k)
+            inputs[k] = *reinterpret_cast<const v4f *>(input_at[k] + (unsigned long long)chunk * kTile32Columns);
     };
-    auto stage = [&](unsigned char *to) {
-        // (a non-finite weight is reported by the thread that stages it, once, not by the sixteen
-        // lanes that multiply it)
-        bad |= (unsigned)!finite_f32(held[0][0]) | (unsigned)!finite_f32(held[0][1]) |
-               (unsigned)!finite_f32(held[0][2]) | (unsigned)!finite_f32(held[0][3]);
+    v4d acc[kTiles];
 #pragma unroll
-        for (unsigned j = 0; j < kHeld; ++j) *reinterpret_cast<v4f *>(to + target[j]) = held[j];
-    };
+    for (unsigned t = 0; t < kTiles; ++t) acc[t] = v4d{0.0, 0.0, 0.0, 0.0};
+    if (begin < end) request(begin);
+    for (unsigned chunk = begin; chunk < end; ++chunk) {
 #pragma unroll
-    for (unsigned j = 0; j < kHeld; ++j) held[j] = fetch(j, 0u);
-    stage(staged);
-    __syncthreads();
-    v4d acc = {0.0, 0.0, 0.0, 0.0};
-    const unsigned tile = wave % kTiles, split = wave / kTiles;
-    const unsigned weight_at = (16u * (tile & 1u) + i16) * kF32BlockPitch + 16u * q + 64u * kSteps * split;
-    const unsigned input_at = (kF32BlockWeightRows + 16u * (tile >> 1) + i16) * kF32BlockPitch + 16u * q + 64u * kSteps * split;
-    for (unsigned chunk = 0; chunk < chunks; ++chunk) {
-        // (the last turn asks for its own chunk again and stages it where nobody reads it: no
-        // branch around the loads, whose registers would otherwise be kept in scratch memory)
-        const unsigned ahead = chunk + 1u < chunks ? chunk + 1u : chunk;
-#pragma unroll
-        for (unsigned j = 0; j < kHeld; ++j)
-            held[j] = fetch(j, ahead);
-        const unsigned char *now = staged + (chunk & 1u) * (kRows * kF32BlockPitch);
-#pragma unroll
-        for (unsigned step = 0; step < kSteps; ++step) {
-            const v4f x = *reinterpret_cast<const v4f *>(now + input_at + 64u * step);
-            const v4f w = *reinterpret_cast<const v4f *>(now + weight_at + 64u * step);
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)w[0], (double)x[0], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)w[1], (double)x[1], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)w[2], (double)x[2], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)w[3], (double)x[3], acc, 0, 0, 0);
+        for (unsigned k = 0; k < 4u; ++k) {
+            bad |= (unsigned)!finite_f32(weights[k][0]) | (unsigned)!finite_f32(weights[k][1]) |
+                   (unsigned)!finite_f32(weights[k][2]) | (unsigned)!finite_f32(weights[k][3]);
+            *reinterpret_cast<v4f *>(to + 8u * k * kTile32Pitch) = weights[k];
         }
-        stage(staged + ((chunk + 1u) & 1u) * (kRows * kF32BlockPitch));
-        // the next chunk is complete, and nobody reads this one any more when it is overwritten
-        __syncthreads();
+#pragma unroll
+        for (unsigned k = 0; k < kInputLoads; ++k) *reinterpret_cast<v4f *>(to + (32u + 8u * k) * kTile32Pitch) = inputs[k];
+        request(chunk + 1u < end ? chunk + 1u : chunk);       // (the last turn's are not used)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (unsigned step = 0; step < kTile32Columns / 16u; ++step) {
+            v4f w[2], x[INPUTS / 16u];
+#pragma unroll
+            for (unsigned m = 0; m < 2u; ++m) w[m] = *reinterpret_cast<const v4f *>(from + 16u * m * kTile32Pitch + 64u * step);
+#pragma unroll
+            for (unsigned n = 0; n < INPUTS / 16u; ++n)
+                x[n] = *reinterpret_cast<const v4f *>(from + (32u + 16u * n) * kTile32Pitch + 64u * step);
+#pragma unroll
+            for (unsigned c = 0; c < 4u; ++c)
+#pragma unroll
+                for (unsigned t = 0; t < kTiles; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)w[t & 1u][c], (double)x[t >> 1][c], acc[t], 0, 0, 0);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
     if (bad) raise_status(a.status, 1);
-    // the other waves' sums of a tile through the stages' memory (the barrier above: nobody reads it any more)
-    double *const partial = reinterpret_cast<double *>(staged);
-    if (split) {
+    __syncthreads();
+    double *const partial = reinterpret_cast<double *>(windows);
+    if (wave) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) partial[(((split - 1u) * kTiles + tile) * 4u + k) * 64u + lane] = acc[k];
+        for (unsigned t = 0; t < kTiles; ++t)
+#pragma unroll
+            for (unsigned k = 0; k < 4u; ++k) partial[(((wave - 1u) * kTiles + t) * 4u + k) * 64u + lane] = acc[t][k];
     }
     __syncthreads();
-    if (split) return;
-    const unsigned long long in = (unsigned long long)blockIdx.y * INPUTS + 16u * (tile >> 1) + i16;
+    if (wave) return;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        // accumulator k of lane (i, q): weight row 4 k + q of the tile, input row i
-        const unsigned long long row = (unsigned long long)blockIdx.x * kF32BlockWeightRows + 16u * (tile & 1u) + 4u * k + q;
-        double sum = acc[k];
+    for (unsigned t = 0; t < kTiles; ++t) {
+        const unsigned long long in = in0 + 16u * (t >> 1) + i16;
 #pragma unroll
-        for (unsigned other = 0; other + 1u < kSplits; ++other) sum += partial[((other * kTiles + tile) * 4u + k) * 64u + lane];
-        if (row < a.row_count && in < a.input_rows) matvec_publish(a, in, row, (float)sum);
+        for (unsigned k = 0; k < 4u; ++k) {
+            // accumulator k of lane (i, q): weight row 4 k + q of the tile, input row i
+            const unsigned long long row = row0 + 16u * (t & 1u) + 4u * k + q;
+            double sum = acc[t][k];
+#pragma unroll
+            for (unsigned other = 0; other + 1u < WAVES; ++other) sum += partial[((other * kTiles + t) * 4u + k) * 64u + lane];
+            if (row >= a.row_count || in >= a.input_rows) continue;
+            if (a.parts) a.parts[((unsigned long long)blockIdx.z * a.input_rows + in) * a.row_count + row] = sum;
+            else matvec_publish(a, in, row, (float)sum);
+        }
     }
 }
 
@@ -1023,49 +1022,58 @@ static int launch_block_q(const MatvecArgs &a, bool q8, hipStream_t stream)
 
 using namespace yvex;
 
-template <unsigned QT, unsigned INPUTS>
-static int launch_scalar_block(const MatvecArgs &a, hipStream_t s)
+// How the tiles of 32 weight rows take a projection: input rows a tile, and workgroups that share a tile's row width.
+struct ScalarTiles {
+    unsigned inputs, splits;
+    double us;
+};
+
+// The launch takes as long as the workgroups of the fullest compute unit: 65 us for 32 x 32 outputs of 7168 columns,
+// 35 for 32 x 16. A split costs the join 0.3 us and its sums, written and read, 16 bytes an output at the
+// 10 TB/s of the caches; the join itself is a launch. Measured, 256 weight rows: 1111 input rows in 1, 2, 3 and 4 splits 129, 101, 93
+// and 89 us; 4096 columns by 96 in 4 and 8 splits of 16-row tiles 12.5 and 14.2, of 32-row tiles 17.2 and 14.6.
+static ScalarTiles scalar_tiles(uint64_t row_count, uint64_t row_width, uint64_t input_rows,
+                                unsigned least, unsigned most)
 {
-    const unsigned long long block_y = (a.input_rows + INPUTS - 1ull) / INPUTS;
-    if (block_y > 65535ull) return ST_BOUNDS;
-    YVEX_ALLOW_DYNAMIC_LDS((matvec_f32_block_kernel<QT, INPUTS>), f32_block_lds(INPUTS));
-    matvec_f32_block_kernel<QT, INPUTS><<<dim3((unsigned)((a.row_count + kF32BlockWeightRows - 1ull) / kF32BlockWeightRows),
-                                           (unsigned)block_y), 64u * kF32BlockWaves, f32_block_lds(INPUTS), s>>>(a);
-    return check_launch("matvec_f32_block");
+    const uint64_t cus = (uint64_t)compute_units(), rows = (row_count + 31u) / 32u, chunks = row_width / kTile32Columns;
+    const double split_us = 0.3 + (double)row_count * (double)input_rows * 1.6e-6;
+    ScalarTiles best{0u, 0u, 0.0};
+    for (unsigned inputs = 16u; inputs <= 32u; inputs += 16u) {
+        const uint64_t tiles = rows * ((input_rows + inputs - 1u) / inputs);
+        const double chunk_us = inputs == 16u ? 35.0 / 28.0 : 65.0 / 28.0;      // of a wave: 28 are 7168 columns
+        // (every wave has columns)
+        for (unsigned z = least; z <= most && (z == least || (uint64_t)z * kTile32Waves <= chunks); ++z) {
+            const uint64_t waves = (uint64_t)z * kTile32Waves;
+            const double us = chunk_us * (double)((tiles * z + cus - 1u) / cus) * (double)((chunks + waves - 1u) / waves) +
+                              (z > 1u ? 4.0 + split_us * z : 0.0);
+            if (!best.inputs || us < best.us) best = ScalarTiles{inputs, z, us};
+        }
+    }
+    return best;
 }
 
-// Rows of F32, F16 or BF16 values against eight or more F32 input rows: 16 x 16 tiles on the
-// double-precision matrix cores; a small batch offers few tiles, so sixteen waves split the row
-// width, a large one has tiles enough for four, or for the staged kernel.
+template <unsigned QT>
+static int launch_scalar_tiles(const MatvecArgs &a, ScalarTiles tiles, hipStream_t s)
+{
+    const uint64_t grid_x = (a.row_count + 31ull) / 32ull, grid_y = (a.input_rows + tiles.inputs - 1ull) / tiles.inputs;
+    if (grid_x > 0x3fffffffull || (a.input_rows + 15ull) / 16ull > 65535ull) return ST_BOUNDS;
+    const dim3 grid((unsigned)grid_x, (unsigned)grid_y, tiles.splits);
+    if (tiles.inputs == 16u) matvec_f32_tile32_kernel<QT, 16><<<grid, 64u * kTile32Waves, 0, s>>>(a);
+    else matvec_f32_tile32_kernel<QT, 32><<<grid, 64u * kTile32Waves, 0, s>>>(a);
+    return check_launch("matvec_f32_tile32");
+}
+
+// Rows of F32, F16 or BF16 values against eight or more F32 input rows on the double-precision matrix cores:
+// a small batch offers few tiles, so sixteen waves of a 16 x 16 tile split the row width, a larger one runs on the
+// 32-row tiles.
 template <unsigned QT>
 static int launch_scalar_rows(const MatvecArgs &a, hipStream_t s)
 {
+    if (a.input_rows >= 256ull)
+        return launch_scalar_tiles<QT>(a, scalar_tiles(a.row_count, a.row_width, a.input_rows, 1u, 1u), s);
     const unsigned long long grid_x = (a.row_count + 15ull) / 16ull, grid_y = (a.input_rows + 15ull) / 16ull;
     if (grid_x > 0x7fffffffull || grid_y > 65535ull) return ST_BOUNDS;
-    const unsigned long long block_rows = (a.row_count + kF32BlockWeightRows - 1ull) / kF32BlockWeightRows;
-    // The staged kernel's launch takes as long as its rounds of workgroups, one a compute unit: 51, 93 and
-    // 165 us a round with 16, 32 and 64 input rows a workgroup (7168 columns); the small tiles take 30 us
-    // for a workgroup a compute unit, 45 at least. So 256 weight rows by 512
-    // input rows take 51 us (60 with small tiles), by 850 93 (110), by 2048 165 (211), but by 1111 the
-    // small tiles' 136 (157).
-    const unsigned long long cus = compute_units();
-    auto rounds = [&](unsigned long long inputs) {
-        return (block_rows * ((a.input_rows + inputs - 1ull) / inputs) + cus - 1ull) / cus;
-    };
-    const unsigned long long small_tiles = 30ull * ((grid_x * grid_y + cus - 1ull) / cus);
-    const unsigned long long cost[4] = {small_tiles > 45ull ? small_tiles : 45ull, 51ull * rounds(16ull), 93ull * rounds(32ull),
-                                        165ull * rounds(64ull)};
-    unsigned best = 0u;
-    for (unsigned i = 1u; i < 4u; ++i)
-        if (cost[i] < cost[best]) best = i;
-    if (a.input_rows < 256ull) {
-        matvec_f32_tile16_kernel<16, QT><<<dim3((unsigned)grid_x, (unsigned)grid_y), 1024, 0, s>>>(a);
-    } else if (a.row_width % kF32BlockColumns == 0ull && best) {
-        return best == 1u ? launch_scalar_block<QT, 16>(a, s) : best == 2u ? launch_scalar_block<QT, 32>(a, s)
-                                                                           : launch_scalar_block<QT, 64>(a, s);
-    } else {
-        matvec_f32_tile16_kernel<4, QT><<<dim3((unsigned)grid_x, (unsigned)grid_y), 256, 0, s>>>(a);
-    }
+    matvec_f32_tile16_kernel<16, QT><<<dim3((unsigned)grid_x, (unsigned)grid_y), 1024, 0, s>>>(a);
     return check_launch("matvec_f32_tile16");
 }
 
@@ -1266,27 +1274,45 @@ extern "C" int yvex_hip_row_dot(const uint8_t *encoded, unsigned int qtype, cons
     return check_launch("row_dot");
 }
 
-// Splits of an F32 projection over a decode-width batch: per-wave shares of 128 columns. A larger
-// batch against a few weight rows (the mixing projection of a prefill batch: 24 rows) is split
-// too, as often as brings its 16 x 16 tiles to about two thousand.
-static unsigned f32_rows_splits(uint64_t row_count, uint64_t row_width, uint64_t input_rows)
+// Splits of the 16 x 16 tiles: 512 columns a split (128 a wave) where that gives 2 to 64 splits; a wider row takes
+// the most splits up to 64 that leave every wave a multiple of 16 columns.
+static unsigned f32_rows_column_splits(uint64_t row_width)
 {
-    if (input_rows < 8u || row_width % 128u) return 0u;
-    if (input_rows >= 256u) {
-        const uint64_t tiles = (row_count + 15u) / 16u * ((input_rows + 15u) / 16u);
-        if (tiles >= 1024u) return 0u;
-        for (unsigned splits = (unsigned)(2048u / tiles < 16u ? 2048u / tiles : 16u); splits >= 2u; --splits)
-            if (row_width % (64ull * splits) == 0u) return splits;
-        return 0u;
-    }
-    // 512 columns a split (128 a wave) where that gives 2 to 64 splits; a wider row takes the
-    // most splits up to 64 that leave every wave a multiple of 16 columns
     if (row_width % 512u == 0u && row_width / 512u >= 2u && row_width / 512u <= 64u)
         return (unsigned)(row_width / 512u);
     if (row_width < 64u * 512u) return 0u;
     for (unsigned splits = 64u; splits >= 2u; --splits)
         if (row_width % (64ull * splits) == 0u) return splits;
     return 0u;
+}
+
+// The 16 x 16 tiles keep up to 16 input rows, and a decode batch whose workgroups, sixteen splits at most, have a compute
+// unit each: 256 x 7168 by 10 rows 11.5 us (on the 32-row tiles 12.5), by 23 13.5 (12.9); 256 x 4096 by 32 10.4 (10.8), by
+// 96 14.3 (12.3); 24 x 16384 by 32, 32 splits, 15.2 (14.4).
+static bool f32_rows_wide(uint64_t row_count, uint64_t row_width, uint64_t input_rows)
+{
+    if (input_rows <= 16u || row_width % 128u) return false;
+    const uint64_t splits = f32_rows_column_splits(row_width);
+    return input_rows >= 256u || splits > 16u ||
+           (row_count + 15u) / 16u * ((input_rows + 15u) / 16u) * splits > (uint64_t)compute_units();
+}
+
+// A batch of fewer tiles is always split (a router's second launch then routes its rows as well), a larger one where that
+// is faster.
+static ScalarTiles f32_rows_tiles(uint64_t row_count, uint64_t row_width, uint64_t input_rows)
+{
+    const bool few = input_rows < 256u || (row_count + 15u) / 16u * ((input_rows + 15u) / 16u) < 1024u;
+    return scalar_tiles(row_count, row_width, input_rows, few ? 2u : 1u, 16u);
+}
+
+// Splits of an F32 projection over a row batch; 0 where it is one launch: a row of too few columns at decode width.
+static unsigned f32_rows_splits(uint64_t row_count, uint64_t row_width, uint64_t input_rows)
+{
+    if (input_rows < 8u || row_width % 128u) return 0u;
+    const unsigned columns = f32_rows_column_splits(row_width);
+    if (!f32_rows_wide(row_count, row_width, input_rows)) return columns;
+    const unsigned splits = f32_rows_tiles(row_count, row_width, input_rows).splits;
+    return splits > 1u ? splits : 0u;
 }
 
 extern "C" uint64_t yvex_hip_matvec_f32_scratch_bytes(uint64_t row_count, uint64_t row_width,
@@ -1385,6 +1411,8 @@ extern "C" int yvex_hip_matvec_f32_rows_routed(const float *weights, uint64_t ro
 
 static int launch_f32_rows_parts(const MatvecArgs &a, yvex_hip_stream stream)
 {
+    if (f32_rows_wide(a.row_count, a.row_width, a.input_rows))
+        return launch_scalar_tiles<QT_F32>(a, f32_rows_tiles(a.row_count, a.row_width, a.input_rows), as_stream(stream));
     const uint64_t grid_x = (a.row_count + 15u) / 16u, grid_y = (a.input_rows + 15u) / 16u;
     if (grid_x > 0x7fffffffull || grid_y > 65535ull) return ST_BOUNDS;
     matvec_f32_tile16_kernel<4><<<dim3((unsigned)grid_x, (unsigned)grid_y,
