@@ -108,6 +108,15 @@ int yvex_hip_matvec_f32_rows_routed(const float *weights, uint64_t row_count, ui
                                     float *logits, const float *bias, uint64_t topk, int scoring, int normalize,
                                     double scaling, uint64_t *selected, float *route_weights, void *scratch,
                                     uint64_t scratch_bytes, int *status, yvex_hip_stream stream);
+/* yvex_hip_q8k_quantize of a few F32 input rows followed by yvex_hip_matvec, in one launch and without the quantized rows
+ * in memory: the same bits. `_supported` says whether it serves a projection (Q8_0 rows on even addresses); the call
+ * itself answers UNSUPPORTED where it does not. */
+int yvex_hip_matvec_quantizing_supported(const uint8_t *encoded, unsigned int qtype, uint64_t row_count,
+                                         uint64_t row_width, uint64_t row_bytes, uint64_t input_rows);
+int yvex_hip_matvec_quantizing(const uint8_t *encoded, unsigned int qtype, uint64_t row_count, uint64_t row_width,
+                               uint64_t row_bytes, const float *input, uint64_t input_rows, uint64_t input_stride,
+                               const float *additive, float *out, uint64_t out_stride, int output_bf16, int *status,
+                               yvex_hip_stream stream);
 /* yvex_hip_matvec of two Q8_0 matrices of one shape against the same Q8_K input rows, in one launch. */
 int yvex_hip_matvec_q8_0_pair(const uint8_t *first, const uint8_t *second, uint64_t row_count,
                               uint64_t row_width, uint64_t row_bytes, const void *input_q8k,

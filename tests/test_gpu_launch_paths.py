@@ -73,6 +73,44 @@ def test_q8_0_wide_tiles_are_the_oracles_bits(gpu, oracle, rows, width, inputs):
     assert np.array_equal(got[picked].view(np.uint32), want.view(np.uint32))
 
 
+# one launch that quantizes its input rows: fewer rows than waves, rows whose blocks fill the lanes' chunks or not,
+# rows on dword boundaries and between them, more weight rows than a round of waves
+@pytest.mark.parametrize("rows,width,inputs,offset", [(1, 256, 1, 0), (17, 2048, 2, 2), (33, 2304, 1, 0), (100, 4096, 2, 0),
+                                                      (130, 4352, 1, 2), (4099, 7168, 2, 0), (4100, 14336, 1, 2), (9000, 512, 2, 0)])
+def test_quantizing_projection_is_quantization_and_projection(gpu, oracle, rows, width, inputs, offset):
+    from yvex_amd import kernels as K
+    g = oracle.Generator(42, f"quantizing.{rows}.{width}.{inputs}")
+    held = torch.zeros(rows * width // 32 * 34 + offset, dtype=torch.uint8, device=gpu)
+    held[offset:] = dev(g.weights(oracle.Q8_0, rows, width), gpu)
+    w = held[offset:]
+    x, add = (dev(g.normal(inputs * n).reshape(inputs, n), gpu) for n in (width, rows))
+    status = K.new_status(gpu)
+    lib, row_bytes = K.load_library(), width // 32 * 34
+    assert lib.yvex_hip_matvec_quantizing_supported(ptr(w), C.c_uint(oracle.Q8_0), u64(rows), u64(width), u64(row_bytes), u64(inputs))
+
+    def run(values, additive, bf16):
+        out = torch.full((inputs, rows + 3), 7.0, device=gpu)
+        call("yvex_hip_matvec_quantizing", ptr(w), C.c_uint(oracle.Q8_0), u64(rows), u64(width), u64(row_bytes), ptr(values),
+             u64(inputs), u64(width), ptr(additive), ptr(out), u64(rows + 3), C.c_int(bf16), ptr(status))
+        assert torch.all(out[:, rows:] == 7.0)
+        return out[:, :rows]
+    act = K.q8k_quantize(x, status)
+    for additive, bf16 in ((None, 0), (add, 1)):
+        padded = torch.zeros((inputs, rows + 3), device=gpu)
+        if additive is not None:
+            padded[:, :rows] = additive
+        want = K.matvec(w, oracle.Q8_0, rows, width, act, input_q8=True, input_rows=inputs, status=status,
+                        additive=additive, output_bf16=bool(bf16))
+        assert same_bits(run(x, None if additive is None else padded, bf16), want)
+    assert int(status.item()) == 0
+    x[inputs - 1, width - 1] = float("nan")
+    run(x, None, 0)
+    assert int(status.item()) == 1
+    # what it does not serve it refuses: three rows, rows on odd addresses, another format
+    for at, qtype, n in ((w, oracle.Q8_0, 3), (held[offset + 1:], oracle.Q8_0, inputs), (w, oracle.Q4_K, inputs)):
+        assert not lib.yvex_hip_matvec_quantizing_supported(ptr(at), C.c_uint(qtype), u64(rows), u64(width), u64(row_bytes), u64(n))
+
+
 # 16 x 16 tiles on eight waves and on four, and the 32 x 32 Q8_0 tiles: ragged on both sides, fewer superblocks than
 # waves, a superblock more than a round of them, one row against many
 @pytest.mark.parametrize("qtype,rows,width,inputs", [

@@ -13,6 +13,7 @@
 #include "launch.hpp"
 #include "units.hpp"
 #include "route.hpp"
+#include "q8_0_rows.hpp"
 
 namespace yvex {
 
@@ -183,6 +184,45 @@ __global__ __launch_bounds__(256) void matvec_block_kernel(MatvecArgs a)
                                          a.row_width, QT);
         }
         if (lane == 0u) matvec_publish(a, in, row, sum);
+    }
+}
+
+// A few F32 input rows against Q8_0 rows on even addresses, quantized on the way (q8_0_rows.hpp). The first weight row's
+// bytes are on their way while the input rows are quantized.
+template <int T, int U>
+__global__ __launch_bounds__(kHeldThreads) void matvec_q8_0_quantizing_kernel(MatvecArgs a)
+{
+    extern __shared__ __align__(16) unsigned char held[];
+    const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const unsigned units = (unsigned)(a.row_width >> 5), blocks = units >> 3;
+    const unsigned input_rows = (unsigned)a.input_rows, tasks = input_rows * blocks;
+    auto values_of = [&](unsigned task, float (&v)[4]) {
+        const unsigned in = task / blocks;
+        const float *x = (const float *)a.input + in * a.input_stride + 256u * (task - in * blocks) + 4u * lane;
+#pragma unroll
+        for (unsigned i = 0; i < 4u; ++i) v[i] = x[i];
+    };
+    float v[4];
+    values_of(wave < tasks ? wave : tasks - 1u, v);
+    unsigned long long row = (unsigned long long)blockIdx.x * kHeldWaves + wave;
+    HeldBlockBytes raw[U];
+    const unsigned char *at = a.encoded + (row < a.row_count ? row : a.row_count - 1ull) * a.row_bytes;
+    held_request_row<U>(at, 0u, units, lane, raw);
+    for (unsigned task = wave; task < tasks; task += kHeldWaves) {
+        hold_block(v, held + task * kHeldBlock, lane, a.status);
+        if (task + kHeldWaves < tasks) values_of(task + kHeldWaves, v);
+    }
+    __syncthreads();
+    while (row < a.row_count) {
+        float sums[T];
+        held_row<T, U>(at, units, lane, raw, held, blocks * kHeldBlock, sums);
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+            if (lane == 0u && (unsigned)t < input_rows) matvec_publish(a, (unsigned)t, row, sums[t]);
+        row += (unsigned long long)gridDim.x * kHeldWaves;
+        if (row >= a.row_count) break;
+        at = a.encoded + row * a.row_bytes;
+        held_request_row<U>(at, 0u, units, lane, raw);
     }
 }
 
@@ -1188,6 +1228,49 @@ extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint6
 // Two Q8_0 matrices of one shape against the same Q8_K input rows in one launch (a shared expert's gate
 // and up projections): each offers too few workgroups for the device on its own (2048 x 4096 against
 // 96 rows: 192 of them, 16 us a launch).
+// Whether F32 input rows are multiplied by the launch that quantizes them. Every workgroup quantizes all of them, a
+// block a wave at a time, so up to two rows, and as many blocks as the workgroup has waves or twice that while the rest of
+// the launch is short. Two launches and one, us: 4096 x 4096 by 1 and 2 rows 9.8 and 7.2, 12.2 and 9.0 (by 3 12.4 and
+// 11.9, by 4 12.7 and 12.8); 7168 x 7168 18.2 and 15.7, 22.5 and 18.5; 50 000 x 4096 57.9 and 45.7, 87 and 47;
+// 129 280 x 7168 184.7 and 184.1, 206 and 196; 64 x 256 4.5 and 3.1; but 1024 x 7168 by 2 10.3 and 11.6, 2048 x 8192 by 1
+// 9.7 and 10.2, 256 x 16384 11.3 and 13.8.
+extern "C" int yvex_hip_matvec_quantizing_supported(const uint8_t *encoded, unsigned int qtype, uint64_t row_count,
+                                                    uint64_t row_width, uint64_t row_bytes, uint64_t input_rows)
+{
+    if (qtype != QT_Q8_0 || !input_rows || input_rows > 2u || !row_count || !row_width || row_width > 14336u ||
+        row_width % 256u || row_width / 32u * 34u != row_bytes || ((uintptr_t)encoded & 1u))
+        return 0;
+    const uint64_t tasks = input_rows * (row_width / 256u);
+    return (tasks <= 32u && row_width <= 7168u) || (tasks <= 56u && row_count >= 4096u);
+}
+
+template <int T>
+static int launch_quantizing(const MatvecArgs &a, hipStream_t s)
+{
+    const unsigned long long groups = (a.row_count + kHeldWaves - 1ull) / kHeldWaves, most = (unsigned long long)compute_units();
+    const unsigned grid = (unsigned)(groups < most ? groups : most);
+    const unsigned lds = (unsigned)held_bytes(T, a.row_width / 256ull);
+    if (a.row_width <= 2048ull) matvec_q8_0_quantizing_kernel<T, 1><<<grid, kHeldThreads, lds, s>>>(a);
+    else if (a.row_width <= 4096ull) matvec_q8_0_quantizing_kernel<T, 2><<<grid, kHeldThreads, lds, s>>>(a);
+    else matvec_q8_0_quantizing_kernel<T, 4><<<grid, kHeldThreads, lds, s>>>(a);
+    return check_launch("matvec_quantizing");
+}
+
+extern "C" int yvex_hip_matvec_quantizing(const uint8_t *encoded, unsigned int qtype, uint64_t row_count,
+                                          uint64_t row_width, uint64_t row_bytes, const float *input,
+                                          uint64_t input_rows, uint64_t input_stride, const float *additive, float *out,
+                                          uint64_t out_stride, int output_bf16, int *status, yvex_hip_stream stream)
+{
+    if (!encoded || !input || !out || !status || out_stride < row_count || input_stride < row_width ||
+        (((uintptr_t)input | (uintptr_t)out) & 3u))
+        return ST_INVALID_ARG;
+    if (!yvex_hip_matvec_quantizing_supported(encoded, qtype, row_count, row_width, row_bytes, input_rows))
+        return ST_UNSUPPORTED;
+    MatvecArgs a{encoded, row_count, row_width, row_bytes, input, input_rows, input_stride, additive, out, out_stride,
+                 output_bf16, status, nullptr, nullptr, 0};
+    return input_rows == 1u ? launch_quantizing<1>(a, as_stream(stream)) : launch_quantizing<2>(a, as_stream(stream));
+}
+
 extern "C" int yvex_hip_matvec_q8_0_pair(const uint8_t *first, const uint8_t *second, uint64_t row_count,
                                          uint64_t row_width, uint64_t row_bytes, const void *input_q8k,
                                          uint64_t input_rows, float *out_first, float *out_second,

@@ -6,9 +6,8 @@
 
 namespace yvex {
 
-// v: this lane's four values of the block; out: the block's 292 bytes.
-__device__ __forceinline__ void q8k_quantize_values(const float (&v)[4], unsigned char *__restrict__ out,
-                                                    unsigned lane, int *status)
+// v: this lane's four values of the block; returns their codes, the block's scale (in every lane) and the lane's codes' sum.
+__device__ __forceinline__ unsigned q8k_codes(const float (&v)[4], unsigned lane, float &scale, int &sum, int *status)
 {
     unsigned long long key = 0ull;
     bool bad = false;
@@ -31,9 +30,9 @@ __device__ __forceinline__ void q8k_quantize_values(const float (&v)[4], unsigne
     const float magnitude = __uint_as_float((unsigned)(key >> 32));
     const float signed_max = (key & 1ull) ? -magnitude : magnitude;
     const float inverse = magnitude == 0.0f ? 0.0f : -127.0f / signed_max;
-    if (lane == 0u) *reinterpret_cast<float *>(out) = inverse == 0.0f ? 0.0f : 1.0f / inverse;
+    scale = inverse == 0.0f ? 0.0f : 1.0f / inverse;
     unsigned packed = 0u;
-    int sum = 0;
+    sum = 0;
 #pragma unroll
     for (unsigned i = 0; i < 4u; ++i) {
         int q = inverse == 0.0f ? 0 : __float2int_rn(inverse * v[i]);
@@ -41,6 +40,17 @@ __device__ __forceinline__ void q8k_quantize_values(const float (&v)[4], unsigne
         sum += q;
         packed |= ((unsigned)q & 255u) << (8u * i);
     }
+    return packed;
+}
+
+// out: the block's 292 bytes.
+__device__ __forceinline__ void q8k_quantize_values(const float (&v)[4], unsigned char *__restrict__ out,
+                                                    unsigned lane, int *status)
+{
+    float scale;
+    int sum;
+    const unsigned packed = q8k_codes(v, lane, scale, sum, status);
+    if (lane == 0u) *reinterpret_cast<float *>(out) = scale;
     *reinterpret_cast<unsigned *>(out + 4u + lane * 4u) = packed;
     sum = group_sum_i32<4>(sum);   // four lanes hold sixteen consecutive values
     if ((lane & 3u) == 0u) *reinterpret_cast<short *>(out + 260u + (lane >> 2) * 2u) = (short)sum;

@@ -121,7 +121,19 @@ int yvex_rocm_encoded_matvec(
         if (rc == YVEX_OK) launches++;
         activations = (const void *)(uintptr_t)joined_address;
     }
-    if (rc == YVEX_OK && q8_path) {
+    /* a row or two of a format the product's own launch can quantize them for */
+    const int quantizing = q8_path && yvex_hip_matvec_quantizing_supported(
+        (const uint8_t *)(uintptr_t)device_address, qtype, row_count, row_width, row_bytes, input_rows);
+    if (rc == YVEX_OK && quantizing) {
+        rc = yvex_rocm_launch_result(
+            yvex_hip_matvec_quantizing((const uint8_t *)(uintptr_t)device_address, qtype, row_count, row_width, row_bytes,
+                                       (const float *)input->data, input_rows, row_width,
+                                       additive ? (const float *)additive->data : NULL, (float *)output->data, row_count, 0,
+                                       backend->device_status, backend->stream),
+            "rocm.encoded-matvec.launch", err);
+        if (rc == YVEX_OK) launches++;
+    }
+    if (rc == YVEX_OK && q8_path && !quantizing) {
         rc = yvex_rocm_launch_result(
             yvex_hip_q8k_quantize((const float *)input->data, input_rows, row_width, row_width,
                                   (uint8_t *)(uintptr_t)q8_address, backend->device_status,
@@ -129,7 +141,7 @@ int yvex_rocm_encoded_matvec(
             "rocm.encoded-matvec.q8", err);
         if (rc == YVEX_OK) launches++;
     }
-    if (rc == YVEX_OK) {
+    if (rc == YVEX_OK && !quantizing) {
         rc = yvex_rocm_launch_result(
             yvex_hip_matvec((const uint8_t *)(uintptr_t)device_address, qtype, row_count, row_width,
                             row_bytes, q8_path ? (const void *)(uintptr_t)q8_address : activations,
