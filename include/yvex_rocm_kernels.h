@@ -207,6 +207,22 @@ int yvex_hip_moe_prepare(const float *logits, const float *bias, uint64_t rows, 
                          uint64_t *bucket_populations, uint64_t *sweep_offsets, uint64_t *counts,
                          const float *values, uint64_t width, uint64_t input_stride, uint8_t *encoded,
                          int *status, yvex_hip_stream stream);
+/* Two Q8_0 matrices of one shape and where their products with some input rows go (dense). */
+typedef struct {
+    const uint8_t *first, *second;
+    uint64_t row_count, row_bytes;
+    float *out_first, *out_second;
+} yvex_hip_projection_pair;
+/* yvex_hip_moe_prepare that also multiplies the quantized input rows (one or two) by a pair of matrices, as
+ * yvex_hip_matvec_q8_0_pair behind it would: the same bits, a launch less. `_supported` says whether it serves a pair on
+ * even addresses; the call itself answers UNSUPPORTED where it does not. */
+int yvex_hip_moe_prepare_projecting_supported(const yvex_hip_projection_pair *pair, uint64_t rows, uint64_t width);
+int yvex_hip_moe_prepare_projecting(const float *logits, const float *bias, uint64_t rows, uint64_t experts,
+                                    uint64_t topk, int scoring, int normalize, double scaling, uint64_t *selected,
+                                    float *weights, uint64_t *order, uint64_t *expert_ids, uint64_t *bucket_offsets,
+                                    uint64_t *bucket_populations, uint64_t *sweep_offsets, uint64_t *counts,
+                                    const float *values, uint64_t width, uint64_t input_stride, uint8_t *encoded,
+                                    const yvex_hip_projection_pair *pair, int *status, yvex_hip_stream stream);
 /* yvex_hip_moe_prepare over scores that yvex_hip_matvec_f32_rows_scored has published
  * (rows x experts floats) in place of the logits: same outputs bit for bit. */
 int yvex_hip_moe_prepare_scored(const float *scores, const float *bias, uint64_t rows, uint64_t experts,
@@ -327,6 +343,16 @@ int yvex_hip_moe_swiglu_rows(const float *gate, const float *up, uint64_t count,
 int yvex_hip_q8k_quantize_swiglu(const float *values, uint64_t rows, uint64_t width, uint8_t *encoded,
                                  const float *gate, const float *up, uint64_t shared_rows, double limit,
                                  uint8_t *shared_encoded, int *status, yvex_hip_stream stream);
+
+/* yvex_hip_q8k_quantize_swiglu followed by the Q8_0 projection of the shared rows (one or two) with bf16 outputs, without
+ * their quantized form in memory: the same bits, a launch less. `_supported` says whether it serves a matrix (on an even
+ * address); the call itself answers UNSUPPORTED where it does not. */
+int yvex_hip_q8k_quantize_swiglu_projecting_supported(const uint8_t *down, uint64_t row_count, uint64_t row_bytes,
+                                                      uint64_t shared_rows, uint64_t width);
+int yvex_hip_q8k_quantize_swiglu_projecting(const float *values, uint64_t rows, uint64_t width, uint8_t *encoded,
+                                            const float *gate, const float *up, uint64_t shared_rows, double limit,
+                                            const uint8_t *down, uint64_t row_count, uint64_t row_bytes, float *out,
+                                            int *status, yvex_hip_stream stream);
 
 /* Replaces yvex_moe_reduce_rows + yvex_moe_combine_rows (moe_kernels.cu:584-616):
  * routed[row, c] = sum over rank (in rank order, fp32) of pair_outputs[row*topk+rank, c];

@@ -454,3 +454,60 @@ def test_f32_tiles_of_32_weight_rows_match_float64(gpu, oracle, qtype, rows, wid
         split = K.matvec_f32_rows(dev(w.view(np.float32).reshape(rows, width), gpu), dev(x, gpu), status).cpu().numpy()
         assert np.all(np.abs(split - want) <= slack)
     assert int(status.item()) == 0
+
+
+# the shared expert's Q8_0 products beside preparation and quantization: the separate launches' bits, at one and two rows,
+# fewer weight rows than a workgroup has waves, rows between dword boundaries, several rows a wave
+@pytest.mark.parametrize("rows,hidden,middle,experts,topk,offset", [(1, 256, 256, 4, 2, 0), (2, 2048, 768, 16, 4, 2),
+                                                                    (1, 7168, 2048, 256, 8, 0), (2, 4352, 5120, 33, 3, 2)])
+def test_shared_products_ride_along(gpu, oracle, rows, hidden, middle, experts, topk, offset):
+    from yvex_amd import kernels as K
+    g = oracle.Generator(42, f"ride.{rows}.{hidden}.{middle}")
+    lib, Q = K.load_library(), oracle.Q8_0
+
+    def matrix(n, width):
+        held = torch.zeros(n * width // 32 * 34 + offset, dtype=torch.uint8, device=gpu)
+        held[offset:] = dev(g.weights(Q, n, width), gpu)
+        return held[offset:]
+    gate, up, down = matrix(middle, hidden), matrix(middle, hidden), matrix(hidden, middle)
+    x = dev(g.normal(rows * hidden).reshape(rows, hidden), gpu)
+    logits = dev(g.normal(rows * experts).reshape(rows, experts), gpu)
+    routed = dev(g.normal(rows * topk * middle).reshape(rows * topk, middle), gpu)
+    status = K.new_status(gpu)
+    wl = K.Worklist(rows * topk, experts, gpu)
+    q8 = torch.zeros(rows * (hidden // 256) * 292, dtype=torch.uint8, device=gpu)
+    sel, weights = K.moe_prepare(logits, None, topk, K.SIGMOID, True, 1.5, status, wl, x, q8)
+    want = [K.matvec(w, Q, middle, hidden, q8, input_q8=True, input_rows=rows, status=status) for w in (gate, up)]
+    mid = [torch.zeros(n * (middle // 256) * 292, dtype=torch.uint8, device=gpu) for n in (rows * topk, rows)]
+    limit = 3.0
+    call("yvex_hip_q8k_quantize_swiglu", ptr(routed), u64(rows * topk), u64(middle), ptr(mid[0]), ptr(want[0]), ptr(want[1]),
+         u64(rows), C.c_double(limit), ptr(mid[1]), ptr(status))
+    want_down = K.matvec(down, Q, hidden, middle, mid[1], input_q8=True, input_rows=rows, output_bf16=True, status=status)
+
+    class Pair(C.Structure):
+        _fields_ = [("first", C.c_void_p), ("second", C.c_void_p), ("row_count", C.c_uint64), ("row_bytes", C.c_uint64),
+                    ("out_first", C.c_void_p), ("out_second", C.c_void_p)]
+    got = [torch.full((rows, middle), 7.0, device=gpu) for _ in range(2)]
+    pair = Pair(gate.data_ptr(), up.data_ptr(), middle, hidden // 32 * 34, got[0].data_ptr(), got[1].data_ptr())
+    assert lib.yvex_hip_moe_prepare_projecting_supported(C.byref(pair), u64(rows), u64(hidden))
+    wl2, q82 = K.Worklist(rows * topk, experts, gpu), torch.zeros_like(q8)
+    sel2, weights2 = torch.zeros_like(sel), torch.zeros_like(weights)
+    call("yvex_hip_moe_prepare_projecting", ptr(logits), None, u64(rows), u64(experts), u64(topk), C.c_int(K.SIGMOID), C.c_int(1),
+         C.c_double(1.5), ptr(sel2), ptr(weights2), ptr(wl2.order), ptr(wl2.expert_ids), ptr(wl2.bucket_offsets),
+         ptr(wl2.bucket_populations), ptr(wl2.sweep_offsets), ptr(wl2.counts), ptr(x), u64(hidden), u64(hidden), ptr(q82),
+         C.byref(pair), ptr(status))
+    assert torch.equal(sel2, sel) and same_bits(weights2, weights) and torch.equal(q82, q8)
+    assert torch.equal(wl2.order, wl.order) and torch.equal(wl2.counts, wl.counts)
+    assert same_bits(got[0], want[0]) and same_bits(got[1], want[1])
+    assert lib.yvex_hip_q8k_quantize_swiglu_projecting_supported(ptr(down), u64(hidden), u64(middle // 32 * 34), u64(rows), u64(middle))
+    mid2, got_down = torch.zeros_like(mid[0]), torch.full((rows, hidden), 7.0, device=gpu)
+    call("yvex_hip_q8k_quantize_swiglu_projecting", ptr(routed), u64(rows * topk), u64(middle), ptr(mid2), ptr(want[0]),
+         ptr(want[1]), u64(rows), C.c_double(limit), ptr(down), u64(hidden), u64(middle // 32 * 34), ptr(got_down), ptr(status))
+    assert torch.equal(mid2, mid[0]) and same_bits(got_down, want_down)
+    assert int(status.item()) == 0
+    # three rows and matrices on odd addresses are refused
+    assert not lib.yvex_hip_moe_prepare_projecting_supported(C.byref(pair), u64(3), u64(hidden))
+    pair.second += 1
+    assert not lib.yvex_hip_moe_prepare_projecting_supported(C.byref(pair), u64(rows), u64(hidden))
+    assert not lib.yvex_hip_q8k_quantize_swiglu_projecting_supported(C.c_void_p(down.data_ptr() + 1), u64(hidden),
+                                                                     u64(middle // 32 * 34), u64(rows), u64(middle))

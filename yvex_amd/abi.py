@@ -304,7 +304,7 @@ KERNEL_EXPORTS = [
     "yvex_hip_q8k_quantize", "yvex_hip_concat_rows_bf16", "yvex_hip_row_dot", "yvex_hip_matvec", "yvex_hip_matvec_f32_rows", "yvex_hip_matvec_f32_scratch_bytes", "yvex_hip_matvec_f32_rows_launches", "yvex_hip_matvec_f32_rows_scored", "yvex_hip_matvec_f32_rows_routed", "yvex_hip_matvec_q8_0_pair", "yvex_hip_matvec_quantizing", "yvex_hip_matvec_quantizing_supported", "yvex_hip_moe_up_rows_launches", "yvex_hip_moe_down_rows_launches", "yvex_hip_q8k_quantize_swiglu", "yvex_hip_block_dots_i32", "yvex_hip_gather",
     "yvex_hip_argmax_f32", "yvex_hip_argmax_scratch_bytes", "yvex_hip_argmax_f32_static",
     "yvex_hip_argmax_static_capacity",
-    "yvex_hip_moe_route_rows", "yvex_hip_moe_route_scores", "yvex_hip_moe_route_hash_rows", "yvex_hip_worklist_build", "yvex_hip_moe_prepare", "yvex_hip_moe_prepare_scored", "yvex_hip_moe_prepare_routed", "yvex_hip_moe_combine_egress",
+    "yvex_hip_moe_route_rows", "yvex_hip_moe_route_scores", "yvex_hip_moe_route_hash_rows", "yvex_hip_worklist_build", "yvex_hip_moe_prepare", "yvex_hip_moe_prepare_scored", "yvex_hip_moe_prepare_projecting", "yvex_hip_moe_prepare_projecting_supported", "yvex_hip_q8k_quantize_swiglu_projecting", "yvex_hip_q8k_quantize_swiglu_projecting_supported", "yvex_hip_moe_prepare_routed", "yvex_hip_moe_combine_egress",
     "yvex_hip_moe_prepare_supported", "yvex_hip_moe_up", "yvex_hip_moe_down", "yvex_hip_iq2_sweep_image_bytes", "yvex_hip_iq2_sweep_image_build",
     "yvex_hip_moe_up_rows", "yvex_hip_moe_down_rows", "yvex_hip_moe_swiglu_rows",
     "yvex_hip_moe_reduce_combine", "yvex_hip_mhc_ingress", "yvex_hip_mhc_ingress_encoded", "yvex_hip_mhc_egress",

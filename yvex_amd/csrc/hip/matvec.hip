@@ -193,37 +193,13 @@ template <int T, int U>
 __global__ __launch_bounds__(kHeldThreads) void matvec_q8_0_quantizing_kernel(MatvecArgs a)
 {
     extern __shared__ __align__(16) unsigned char held[];
-    const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const unsigned units = (unsigned)(a.row_width >> 5), blocks = units >> 3;
-    const unsigned input_rows = (unsigned)a.input_rows, tasks = input_rows * blocks;
-    auto values_of = [&](unsigned task, float (&v)[4]) {
-        const unsigned in = task / blocks;
-        const float *x = (const float *)a.input + in * a.input_stride + 256u * (task - in * blocks) + 4u * lane;
-#pragma unroll
-        for (unsigned i = 0; i < 4u; ++i) v[i] = x[i];
-    };
-    float v[4];
-    values_of(wave < tasks ? wave : tasks - 1u, v);
-    unsigned long long row = (unsigned long long)blockIdx.x * kHeldWaves + wave;
-    HeldBlockBytes raw[U];
-    const unsigned char *at = a.encoded + (row < a.row_count ? row : a.row_count - 1ull) * a.row_bytes;
-    held_request_row<U>(at, 0u, units, lane, raw);
-    for (unsigned task = wave; task < tasks; task += kHeldWaves) {
-        hold_block(v, held + task * kHeldBlock, lane, a.status);
-        if (task + kHeldWaves < tasks) values_of(task + kHeldWaves, v);
-    }
-    __syncthreads();
-    while (row < a.row_count) {
-        float sums[T];
-        held_row<T, U>(at, units, lane, raw, held, blocks * kHeldBlock, sums);
-#pragma unroll
-        for (int t = 0; t < T; ++t)
-            if (lane == 0u && (unsigned)t < input_rows) matvec_publish(a, (unsigned)t, row, sums[t]);
-        row += (unsigned long long)gridDim.x * kHeldWaves;
-        if (row >= a.row_count) break;
-        at = a.encoded + row * a.row_bytes;
-        held_request_row<U>(at, 0u, units, lane, raw);
-    }
+    const unsigned units = (unsigned)(a.row_width >> 5), input_rows = (unsigned)a.input_rows;
+    HoldRows hold{(const float *)a.input, a.input_stride, units >> 3, input_rows * (units >> 3), a.status, {}};
+    held_rows<T, U>(a.row_count, blockIdx.x, gridDim.x, units, held,
+                    [&](unsigned long long row) { return a.encoded + row * a.row_bytes; }, hold,
+                    [&](unsigned in, unsigned long long row, float sum) {
+                        if (in < input_rows) matvec_publish(a, in, row, sum);
+                    });
 }
 
 // A unit against 32 int8 activations held in registers; `sums` = the two 16-value sums of the

@@ -122,4 +122,55 @@ __device__ __forceinline__ void held_row(const unsigned char *row, unsigned unit
     }
 }
 
+// The rows [wave of the launch's `groups` workgroups] of up to two matrices (the second's rows count on behind the first's)
+// against T held rows, with the first row's bytes requested ahead by the caller's `hold`, which quantizes the input rows.
+template <int T, int U, typename At, typename Hold, typename Publish>
+__device__ __forceinline__ void held_rows(unsigned long long rows, unsigned group, unsigned groups, unsigned units,
+                                          unsigned char *held, At at, Hold hold, Publish publish)
+{
+    const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    unsigned long long row = (unsigned long long)group * kHeldWaves + wave;
+    HeldBlockBytes raw[U];
+    const unsigned char *from = at(row < rows ? row : rows - 1ull);
+    hold.request(wave);
+    held_request_row<U>(from, 0u, units, lane, raw);
+    hold.finish(wave, held);
+    __syncthreads();
+    while (row < rows) {
+        float sums[T];
+        held_row<T, U>(from, units, lane, raw, held, (units >> 3) * kHeldBlock, sums);
+        if (lane == 0u) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) publish((unsigned)t, row, sums[t]);
+        }
+        row += (unsigned long long)groups * kHeldWaves;
+        if (row >= rows) break;
+        from = at(row);
+        held_request_row<U>(from, 0u, units, lane, raw);
+    }
+}
+
+// Input rows as they lie in memory.
+struct HoldRows {
+    const float *input;
+    unsigned long long stride;
+    unsigned blocks, tasks;          // Q8_K blocks a row, and of all rows
+    int *status;
+    float v[4];
+    __device__ __forceinline__ void request(unsigned task)
+    {
+        const unsigned here = task < tasks ? task : tasks - 1u, in = here / blocks;
+        const float *x = input + in * stride + 256u * (here - in * blocks) + 4u * (threadIdx.x & 63u);
+#pragma unroll
+        for (unsigned i = 0; i < 4u; ++i) v[i] = x[i];
+    }
+    __device__ __forceinline__ void finish(unsigned wave, unsigned char *held)
+    {
+        for (unsigned task = wave; task < tasks; task += kHeldWaves) {
+            hold_block(v, held + task * kHeldBlock, threadIdx.x & 63u, status);
+            if (task + kHeldWaves < tasks) request(task + kHeldWaves);
+        }
+    }
+};
+
 }  // namespace yvex

@@ -963,6 +963,15 @@ sequence:
     /* a decode-width batch with the learned router: routing, worklist and input quantization
      * share one launch */
     const int need_q8 = routed_q8 || (has_shared && shared_q8);
+    /* a row or two: the shared expert's products ride along with the launches that prepare and that quantize */
+    const yvex_hip_projection_pair shared_pair = {shared.gate, shared.up, layer->shared_intermediate_width,
+                                                  shared.gate_row_bytes, (float *)AT(shared_intermediate),
+                                                  (float *)AT(pair_outputs)};
+    const int shared_rides = swiglu_quantized && !routed_rows && !hash_router &&
+                             yvex_hip_moe_prepare_supported(row_count, experts, topk) &&
+                             yvex_hip_moe_prepare_projecting_supported(&shared_pair, row_count, hidden) &&
+                             yvex_hip_q8k_quantize_swiglu_projecting_supported(
+                                 shared.down, hidden, shared.down_row_bytes, row_count, layer->shared_intermediate_width);
     if (routed_rows && row_count <= 512ull) {
         LAUNCH(yvex_hip_moe_prepare_routed((const uint64_t *)AT(selected), row_count, experts, topk,
                                            (uint64_t *)AT(order), (uint64_t *)AT(expert_ids),
@@ -971,6 +980,15 @@ sequence:
                                            need_q8 ? (const float *)activations : NULL, hidden, hidden,
                                            need_q8 ? (uint8_t *)AT(input_q8) : NULL, (int *)status, stream),
                "rocm.moe.rows.prepare");
+    } else if (shared_rides) {
+        LAUNCH(yvex_hip_moe_prepare_projecting((const float *)AT(logits), bias_rows, row_count, experts, topk,
+                                               (int)layer->scoring, layer->normalize_topk_probabilities,
+                                               layer->routed_scaling_factor, (uint64_t *)AT(selected),
+                                               (float *)AT(weights), (uint64_t *)AT(order), (uint64_t *)AT(expert_ids),
+                                               (uint64_t *)AT(bucket_offsets), (uint64_t *)AT(bucket_populations),
+                                               (uint64_t *)AT(sweep_offsets), (uint64_t *)AT(counts),
+                                               (const float *)activations, hidden, hidden, (uint8_t *)AT(input_q8),
+                                               &shared_pair, (int *)status, stream), "rocm.moe.rows.prepare");
     } else if (!routed_rows && !hash_router && yvex_hip_moe_prepare_supported(row_count, experts, topk)) {
         LAUNCH(yvex_hip_moe_prepare((const float *)AT(logits),
                                     bias_rows,
@@ -1023,7 +1041,7 @@ sequence:
                                     1ull, 1ull, layer->activation_limit, (float *)AT(shared_intermediate),
                                     (int *)status, stream), "rocm.moe.rows.shared-up-matrix");
         COUNTED(2);
-    } else if (shared_dense) {
+    } else if (shared_dense && !shared_rides) {
         LAUNCH(yvex_hip_matvec_q8_0_pair(shared.gate, shared.up, layer->shared_intermediate_width, hidden,
                                          shared.gate_row_bytes, AT(input_q8), row_count,
                                          (float *)AT(shared_intermediate), (float *)AT(pair_outputs), (int *)status,
@@ -1033,12 +1051,20 @@ sequence:
                                             row_count * layer->shared_intermediate_width, layer->activation_limit,
                                             (float *)AT(shared_intermediate), (int *)status, stream),
                    "rocm.moe.rows.shared-swiglu");
-    } else if (has_shared && !merged)
+    } else if (has_shared && !merged && !shared_rides)
         LAUNCH(yvex_hip_moe_up(&shared, shared_q8 ? AT(input_q8) : (void *)(uintptr_t)activations,
                                shared_q8, NULL, NULL, NULL, NULL, NULL, NULL, NULL, row_count, 1ull, 1ull,
                                layer->activation_limit, (float *)AT(shared_intermediate), NULL, 0ull, NULL,
                                (int *)status, stream), "rocm.moe.rows.shared-up");
-    if (swiglu_quantized)
+    if (shared_rides)
+        LAUNCH(yvex_hip_q8k_quantize_swiglu_projecting((const float *)AT(intermediate), pairs,
+                                                       layer->expert_intermediate_width, (uint8_t *)AT(intermediate_q8),
+                                                       (const float *)AT(shared_intermediate),
+                                                       (const float *)AT(pair_outputs), row_count,
+                                                       layer->activation_limit, shared.down, hidden,
+                                                       shared.down_row_bytes, (float *)AT(shared_outputs),
+                                                       (int *)status, stream), "rocm.moe.rows.q8-mid");
+    else if (swiglu_quantized)
         LAUNCH(yvex_hip_q8k_quantize_swiglu((const float *)AT(intermediate), pairs, layer->expert_intermediate_width,
                                             (uint8_t *)AT(intermediate_q8), (const float *)AT(shared_intermediate),
                                             (const float *)AT(pair_outputs), row_count, layer->activation_limit,
@@ -1080,12 +1106,12 @@ sequence:
                                       row_count, 1ull, (float *)AT(shared_outputs), (int *)status, stream),
                "rocm.moe.rows.shared-down-matrix");
         COUNTED(3);
-    } else if (shared_dense)
+    } else if (shared_dense && !shared_rides)
         LAUNCH(yvex_hip_matvec(shared.down, shared.down_qtype, hidden, layer->shared_intermediate_width,
                                shared.down_row_bytes, AT(shared_intermediate_q8), 1, row_count,
                                layer->shared_intermediate_width, NULL, (float *)AT(shared_outputs), hidden, 1,
                                (int *)status, stream), "rocm.moe.rows.shared-down-dense");
-    else if (has_shared && !merged)
+    else if (has_shared && !merged && !shared_rides)
         LAUNCH(yvex_hip_moe_down(&shared, shared_q8 ? AT(shared_intermediate_q8) : AT(shared_intermediate),
                                  shared_q8, NULL, NULL, NULL, NULL, NULL, NULL, row_count, 1ull,
                                  (float *)AT(shared_outputs), NULL, 0ull, NULL, NULL, (int *)status, stream),
