@@ -347,15 +347,15 @@ static int same_expert_shape(const yvex_hip_expert_weights *a, const yvex_hip_ex
  * faster. The lines lie where whole layers of 4 to 256 experts cross under uniform routing, intermediate
  * rows 2048 wide. A shared expert of the routed experts' shape (`rides`) goes along in the sweeps'
  * launches and takes launches of its own beside the tiles, so the lines have a constant part.
- *   IQ2_XXS, rides: crossings at 3.0, 3.4, 4.2 and 4.6 pairs an expert for 256, 128, 64 and 32 experts 7168
- *     wide, 3.4, 4.3, 4.8 and 5.7 at 4096, 3.8, -, 5.5 and over 6 at 2048; from 6 to over 20 for 24 to 4
+ *   IQ2_XXS, rides: crossings at 2.8 and 3.8 pairs an expert for 256 and 64 experts 7168 wide, 3.0, 3.45, 4.3 and
+ *     over 5 for 256, 128, 64 and 32 at 4096, 3.3 and 5.3 for 256 and 64 at 2048; from 6 to over 20 for 24 to 4
  *     experts, where buckets past a tile's sixteen columns put the tiles behind once more. 256 experts at
- *     4096: 3.0 pairs 568 us as sweeps and 604 as tiles, 4.0 pairs 704 and 640; at 7168: 2.5 pairs 867 and 920,
- *     3.5 pairs 1117 and 998. The cap is where sealed policies of four-expert layers expect the tiles.
- *   IQ2_XXS alone: 3.1 to 3.6 pairs for 256 experts of any width, 2.8 to 3.9 for 32 and 64 (256 at 4096 with
- *     Q2_K down rows: 3.0 pairs 610 and 660, 4.0 pairs 746 and 685).
- *   Q4_K, rides: 2.7, 2.8, 3.2 and 3.4 (256 at 7168: 2.5 pairs 1380 and 1421, 3.0 pairs 1532 and 1461), 3.7 to
- *     4.8 for 8 to 24 experts. Q4_K alone: 2.8 for 256 experts, under 2.5 for fewer.
+ *     4096: 2.7 pairs 526 us as sweeps and 541 as tiles, 3.2 pairs 585 and 567; at 7168: 2.5 pairs 826 and 867,
+ *     3.0 pairs 933 and 899. The cap is where sealed policies of four-expert layers expect the tiles.
+ *   IQ2_XXS alone: 3.0, 3.15, 3.05 and 3.3 pairs for 256, 128, 64 and 32 experts at 4096 with Q2_K down rows (256:
+ *     2.7 pairs 519 and 538, 3.2 pairs 597 and 573), 3.0 for 256 at 2048.
+ *   Q4_K, rides: 2.27, 2.27, 2.4, 2.65, 3.5 and 4.5 for 256, 128, 64, 32, 16 and 8 (256 at 7168: 2.0 pairs 1175 and
+ *     1176, 2.5 pairs 1292 and 1254). Q4_K alone: 2.25 for 256 experts.
  * Between a crossing and its line the slower side costs under 10 % with 32 experts and more.
  * A skewed routing crosses earlier (an exponent of 0.4 at 2.3 to 3.5 pairs, of 0.8 at under 2.5), but the
  * host does not know the routing. */
@@ -364,14 +364,15 @@ static unsigned long long matrix_core_pairs(const yvex_hip_expert_weights *route
 {
     unsigned long long line, cap;
     if (routed->gate_qtype == 12u) {
-        line = rides ? experts * 5ull / 2ull + 30ull : experts * 11ull / 4ull;
+        line = rides ? experts * 17ull / 8ull + 38ull : experts * 9ull / 4ull + 4ull;
         cap = experts * 4ull;
     } else if (rides) {
         /* between the widths measured on either side the line is drawn half way */
-        line = routed->hidden < 5632ull ? experts * 3ull + 100ull : experts * 13ull / 5ull + 85ull;
+        line = routed->hidden < 3072ull ? experts * 3ull + 100ull
+             : routed->hidden < 5632ull ? experts * 21ull / 8ull + 100ull : experts * 13ull / 5ull + 85ull;
         cap = experts * 18ull;
     } else {
-        line = experts * 13ull / 4ull + 30ull;
+        line = experts * 3ull + 33ull;
         cap = experts * 6ull;
     }
     return line < cap ? line : cap;
