@@ -352,8 +352,11 @@ __global__ __launch_bounds__(kEnvelopeThreads) void mhc_egress_kernel(
 
 // The rank-ordered sum of the pairs' outputs, the shared expert and the egress in one pass over a
 // row's columns (yvex_hip_moe_reduce_combine followed by yvex_hip_mhc_egress, the same operations in
-// the same order): the combined row never goes to memory, and a decode batch has a launch less
-// (5 us of 11 at one row).
+// the same order): the combined row never goes to memory, and a decode batch has a launch less.
+// A thread has one column: a few hundred instructions follow its loads, most of them double-precision, and a wave
+// issues one in five cycles at best, so four columns a thread kept the few waves of a decode batch busy for longer than the
+// memory took, and 87 registers kept a larger batch to five waves a SIMD. 4096 columns, six ranks, by 1 / 96 / 333 rows
+// 8.4 / 12.7 / 27.5 us with four columns, 5.8 / 11.0 / 23.8 with two, 4.4 / 9.0 / 23.5 with one.
 template <unsigned STREAMS>
 __global__ __launch_bounds__(kEnvelopeThreads) void combine_egress_kernel(
     const float *__restrict__ pair_outputs, unsigned topk, const float *__restrict__ shared,
@@ -361,14 +364,14 @@ __global__ __launch_bounds__(kEnvelopeThreads) void combine_egress_kernel(
     unsigned long long row_count, unsigned width, unsigned blocks_per_row, float *__restrict__ output, int *status)
 {
     const unsigned long long row = blockIdx.x / blocks_per_row;
-    const unsigned lane = ((blockIdx.x % blocks_per_row) * kEnvelopeThreads + threadIdx.x) * 4u;
-    if (row >= row_count || lane >= width) return;
+    const unsigned column = (blockIdx.x % blocks_per_row) * kEnvelopeThreads + threadIdx.x;
+    if (row >= row_count || column >= width) return;
     const unsigned expanded = STREAMS * width;
-    const float *in = rows + row * expanded + lane;
-    float4 loaded[STREAMS];
+    const float *in = rows + row * expanded + column;
+    float residual[STREAMS];
 #pragma unroll
-    for (unsigned s = 0; s < STREAMS; ++s) loaded[s] = *reinterpret_cast<const float4 *>(in + s * width);
-    const float4 base = *reinterpret_cast<const float4 *>(shared + row * width + lane);
+    for (unsigned s = 0; s < STREAMS; ++s) residual[s] = in[s * width];
+    const float base = shared[row * width + column];
     double gain[STREAMS], weight[STREAMS][STREAMS];
 #pragma unroll
     for (unsigned t = 0; t < STREAMS; ++t) {
@@ -377,46 +380,30 @@ __global__ __launch_bounds__(kEnvelopeThreads) void combine_egress_kernel(
         for (unsigned s = 0; s < STREAMS; ++s) weight[s][t] = (double)combination[(row * STREAMS + s) * STREAMS + t];
     }
     // ranks in order, four of them in flight
-    float total[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    const float *source = pair_outputs + row * topk * width + lane;
+    float total = 0.0f;
+    const float *source = pair_outputs + row * topk * width + column;
     for (unsigned rank = 0; rank < topk; rank += 4u) {
-        float4 part[4];
+        float part[4];
 #pragma unroll
         for (unsigned k = 0; k < 4u; ++k)
-            part[k] = *reinterpret_cast<const float4 *>(source + (unsigned long long)(rank + k < topk ? rank + k : topk - 1u) * width);
+            part[k] = source[(unsigned long long)(rank + k < topk ? rank + k : topk - 1u) * width];
 #pragma unroll
         for (unsigned k = 0; k < 4u; ++k) {
             if (rank + k >= topk) break;
-            total[0] += part[k].x;
-            total[1] += part[k].y;
-            total[2] += part[k].z;
-            total[3] += part[k].w;
+            total += part[k];
         }
     }
-    bool bad = false;
-    double value[4];
-    const float shared_lane[4] = {base.x, base.y, base.z, base.w};
-#pragma unroll
-    for (unsigned i = 0; i < 4u; ++i) {
-        const float combined = bf16_round(total[i] + shared_lane[i]);
-        bad |= !finite_f32(total[i]) || !finite_f32(combined);
-        value[i] = (double)combined;
-    }
+    const float combined = bf16_round(total + base);
+    bool bad = !finite_f32(total) || !finite_f32(combined);
+    const double value = (double)combined;
 #pragma unroll
     for (unsigned t = 0; t < STREAMS; ++t) {
-        float packed[4];
+        double sum = gain[t] * value;
 #pragma unroll
-        for (unsigned i = 0; i < 4u; ++i) {
-            double sum = gain[t] * value[i];
-#pragma unroll
-            for (unsigned s = 0; s < STREAMS; ++s)
-                sum += weight[s][t] * (double)bf16_round(reinterpret_cast<const float *>(&loaded[s])[i]);
-            const float published = (float)sum;
-            bad |= !finite_f64(sum) || !finite_f32(published);
-            packed[i] = bf16_round(published);
-        }
-        *reinterpret_cast<float4 *>(output + row * expanded + t * width + lane) =
-            make_float4(packed[0], packed[1], packed[2], packed[3]);
+        for (unsigned s = 0; s < STREAMS; ++s) sum += weight[s][t] * (double)bf16_round(residual[s]);
+        const float published = (float)sum;
+        bad |= !finite_f64(sum) || !finite_f32(published);
+        output[row * expanded + t * width + column] = bf16_round(published);
     }
     if (bad) raise_status(status, 1);
 }
@@ -541,7 +528,7 @@ extern "C" int yvex_hip_moe_combine_egress(const float *pair_outputs, uint64_t r
     if (streams != 4u || width % 4u ||
         (((uintptr_t)pair_outputs | (uintptr_t)shared | (uintptr_t)rows | (uintptr_t)output) & 15u))
         return ST_UNSUPPORTED;
-    const unsigned blocks_per_row = (unsigned)((width / 4u + kEnvelopeThreads - 1u) / kEnvelopeThreads);
+    const unsigned blocks_per_row = (unsigned)((width + kEnvelopeThreads - 1u) / kEnvelopeThreads);
     combine_egress_kernel<4><<<(unsigned)(row_count * blocks_per_row), kEnvelopeThreads, 0, as_stream(stream)>>>(
         pair_outputs, (unsigned)topk, shared, rows, post, combination, row_count, (unsigned)width, blocks_per_row,
         output, status);
