@@ -511,3 +511,27 @@ def test_shared_products_ride_along(gpu, oracle, rows, hidden, middle, experts, 
     assert not lib.yvex_hip_moe_prepare_projecting_supported(C.byref(pair), u64(rows), u64(hidden))
     assert not lib.yvex_hip_q8k_quantize_swiglu_projecting_supported(C.c_void_p(down.data_ptr() + 1), u64(hidden),
                                                                      u64(middle // 32 * 34), u64(rows), u64(middle))
+
+
+# two workgroups a row (as many rows as the device leaves two compute units each) against one: the row in registers, rows too
+# long for them, a width that is no multiple of four, other numbers of streams
+@pytest.mark.parametrize("streams,width", [(4, 4096), (4, 7168), (4, 8448), (4, 510), (2, 256), (3, 4100), (7, 1024)])
+def test_ingress_of_few_rows_is_that_of_many(gpu, oracle, streams, width):
+    """The mean squares are sums in double whose order depends on the number of workgroups: the floats that
+    follow are the same or neighbours."""
+    from yvex_amd import kernels as K
+    units = torch.cuda.get_device_properties(gpu).multi_processor_count
+    g, count, mixing = oracle.Generator(42, f"ingress.{streams}.{width}"), units // 2 + 1, (streams + 2) * streams
+    rows, mixes = (dev(g.normal(count * n).reshape(count, n), gpu) for n in (streams * width, mixing))
+    scale, base, norm = (dev(g.normal(n), gpu) for n in (3, mixing, width))
+    kw = dict(streams=streams, width=width, iterations=20, rms_epsilon=1e-6, mhc_epsilon=1e-6, post_multiplier=2.0)
+    status = K.new_status(gpu)
+    many = K.mhc_ingress(rows, mixes, scale, base, norm, status=status, **kw)
+    for few in (1, units // 2):
+        got = K.mhc_ingress(rows[:few].contiguous(), mixes[:few].contiguous(), scale, base, norm, status=status, **kw)
+        for a, b, step in zip(got, many, (2.0 ** -7, 2.0 ** -22, 2.0 ** -22)):      # (bf16 values; floats)
+            assert torch.all((a - b[:few]).abs() <= b[:few].abs() * step)
+    assert int(status.item()) == 0
+    rows[0, streams * width - 1] = float("inf")
+    K.mhc_ingress(rows[:1].contiguous(), mixes[:1].contiguous(), scale, base, norm, status=status, **kw)
+    assert int(status.item()) == 1

@@ -26,14 +26,28 @@ __device__ __forceinline__ bool finite_f64(double v)
     return (__double_as_longlong(v) & 0x7ff0000000000000ll) != 0x7ff0000000000000ll;
 }
 
+// A double moved by a data-parallel-primitive step (both halves).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v)
+{
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
+    const unsigned low = (unsigned)dpp_move<CTRL, 0xf>((int)(unsigned)bits);
+    const unsigned high = (unsigned)dpp_move<CTRL, 0xf>((int)(unsigned)(bits >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)high << 32) | low));
+}
+
 // Sum over the workgroup, the same value in every thread: a butterfly inside each wavefront,
 // then the wavefront totals in order. The order is fixed, so a row's result does not depend on
 // where it runs.
 template <unsigned WAVES>
 __device__ __forceinline__ double workgroup_sum(double v, double *slots)
 {
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, kWave);
+    v += __shfl_xor(v, 32, kWave);
+    v += __shfl_xor(v, 16, kWave);
+    v += dpp_f64<0x128>(v);        // row_ror 8, 4, 2, 1: what they fetch is what the butterfly's lanes hold by then,
+    v += dpp_f64<0x124>(v);        // without a permute through LDS each
+    v += dpp_f64<0x122>(v);
+    v += dpp_f64<0x121>(v);
     if ((threadIdx.x & 63u) == 0u) slots[threadIdx.x >> 6] = v;
     __syncthreads();
     double total = slots[0];
@@ -73,16 +87,6 @@ __device__ __forceinline__ float4 coefficient4(const void *values, unsigned qtyp
                        __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
 }
 
-// A double moved by a data-parallel-primitive step (both halves).
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v)
-{
-    const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
-    const unsigned low = (unsigned)dpp_move<CTRL, 0xf>((int)(unsigned)bits);
-    const unsigned high = (unsigned)dpp_move<CTRL, 0xf>((int)(unsigned)(bits >> 32));
-    return __longlong_as_double((long long)(((unsigned long long)high << 32) | low));
-}
-
 // Alternating row and column normalisations of a 4 x 4 matrix, one element a lane (4 row + column,
 // repeated in each group of sixteen lanes). The totals are two additions each way inside the row of
 // sixteen lanes, on the vector ALU; sums of four floats of a matrix whose elements lie within a
@@ -108,11 +112,16 @@ __device__ __forceinline__ float sinkhorn4(float m, unsigned iterations, double 
     return m;
 }
 
-// One workgroup per row. The row is read twice (mean square, then the gated sum of the streams);
-// both passes keep four 16-byte loads per thread in flight, because a row is a short stream and
-// a loop that waits for each load in turn spends its time on latency; long rows take 1024
-// threads for the same reason. Rows whose width is not a multiple of four take the scalar loops.
-template <unsigned THREADS>
+// One workgroup per row. The row is passed over twice (mean square, then the gated sum of the streams); four 16-byte
+// loads per thread are in flight, because a row is a short stream and a loop that waits for each load in turn spends its
+// time on latency; long rows take 1024 threads for the same reason. Rows whose width is not a multiple of four take the
+// scalar loops.
+// SPLIT, where a batch leaves every row two compute units: a second workgroup forms the mean square as well and then the
+// mixing matrix, whose chain of divisions so runs beside the second pass and not ahead of the sum that ends it, and the
+// row's values stay in registers for the second pass. A one-row launch of four streams of 4096 values is 2.6 us of
+// getting there and back and then waits of one workgroup for itself: 11.9 -> 9.0 us, 96 rows 13.5 -> 11.2. In a batch
+// of more rows two workgroups share a compute unit, which those registers would not let them (333 rows 23 and 28 us).
+template <unsigned THREADS, bool SPLIT>
 __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
     const float *__restrict__ rows, const float *__restrict__ mixes, const void *__restrict__ scale_values,
     const void *__restrict__ base_values, const void *__restrict__ norm, unsigned scale_qtype,
@@ -125,18 +134,44 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
     extern __shared__ __align__(16) float collapsed[];   // width values
     __shared__ double slots[THREADS / 64u];
     __shared__ double gate[8];
-    constexpr unsigned kBatch = 4;
-    constexpr unsigned kWorkers = THREADS - 64u;     // the second pass leaves the first wavefront out
+    constexpr unsigned kBatch = 4, kHeld = SPLIT ? 2 : 0;    // (two workgroups share a compute unit on fewer registers)
+    constexpr unsigned kSpared = SPLIT ? 0u : 64u;           // the second pass leaves the first wavefront out
+    constexpr unsigned kWorkers = THREADS - kSpared;
     const unsigned tid = threadIdx.x;
-    const unsigned long long row = blockIdx.x;
+    const unsigned long long row = SPLIT ? blockIdx.x >> 1 : blockIdx.x;
+    const bool mixes_only = SPLIT && (blockIdx.x & 1u) != 0u, mixes_here = !SPLIT || mixes_only;
     const unsigned expanded = streams * width, mixing_rows = (streams + 2u) * streams;
     const float *in = rows + row * expanded;
     const float *mix = mixes + row * mixing_rows;
     bool bad = false;    // quads: width is a multiple of four and every row starts 16-byte aligned
 
-    // mean square of the bf16-rounded residual
+    // mean square of the bf16-rounded residual (a value that is not finite makes the sum not finite)
     double squares = 0.0;
-    if (quads) {
+    const bool held = kHeld != 0u && quads && streams <= kBatch && width <= kHeld * 4u * kWorkers;   // a worker's columns stay in registers
+    float4 mine[kHeld ? kHeld : 1u][kBatch];
+    if (held) {
+        const float4 *in4 = reinterpret_cast<const float4 *>(in);
+        const unsigned count = width >> 2;
+#pragma unroll
+        for (unsigned u = 0; u < kHeld; ++u) {
+            const unsigned at = tid - kSpared + u * kWorkers;          // (behind the row's end where tid < kSpared)
+#pragma unroll
+            for (unsigned s = 0; s < kBatch; ++s)
+                mine[u][s] = at < count && s < streams ? in4[s * count + at] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+#pragma unroll
+        for (unsigned u = 0; u < kHeld; ++u) {
+            if (u != 0u && u * kWorkers >= count) break;
+#pragma unroll
+            for (unsigned s = 0; s < kBatch; ++s) {
+                const float4 r = mine[u][s] = bf16_round4(mine[u][s]);
+                squares += (double)r.x * (double)r.x;
+                squares += (double)r.y * (double)r.y;
+                squares += (double)r.z * (double)r.z;
+                squares += (double)r.w * (double)r.w;
+            }
+        }
+    } else if (quads) {
         const float4 *in4 = reinterpret_cast<const float4 *>(in);
         const unsigned count = expanded >> 2;
         for (unsigned first = tid; first < count; first += THREADS * kBatch) {
@@ -149,7 +184,6 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
 #pragma unroll
             for (unsigned u = 0; u < kBatch; ++u) {
                 const float4 r = bf16_round4(v[u]);
-                bad |= !finite_f32(r.x) || !finite_f32(r.y) || !finite_f32(r.z) || !finite_f32(r.w);
                 squares += (double)r.x * (double)r.x;
                 squares += (double)r.y * (double)r.y;
                 squares += (double)r.z * (double)r.z;
@@ -159,10 +193,10 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
     } else {
         for (unsigned lane = tid; lane < expanded; lane += THREADS) {
             const float v = bf16_round(in[lane]);
-            bad |= !finite_f32(v);
             squares += (double)v * (double)v;
         }
     }
+    bad |= !finite_f64(squares);
     if (tid < mixing_rows) {
         base[tid] = coefficient(base_values, base_qtype, tid);
         bad |= !finite_f32(base[tid]) || !finite_f32(mix[tid]);
@@ -175,11 +209,14 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
     const double inverse = 1.0 / sqrt(workgroup_sum<THREADS / 64u>(squares, slots) / (double)expanded + rms_epsilon);
     bad |= !finite_f64(inverse);
 
-    if (tid < streams) {
+    // (the two sigmoids of a stream in different wavefronts)
+    if (!mixes_only && tid < streams) {
         const double pre = sigmoid_f64((double)mix[tid] * inverse * (double)scale[0] + (double)base[tid]);
         gate[tid] = pre + mhc_epsilon;
-        post[row * streams + tid] = (float)(post_multiplier * sigmoid_f64(
-            (double)mix[streams + tid] * inverse * (double)scale[1] + (double)base[streams + tid]));
+    } else if (!mixes_only && tid >= 64u && tid < 64u + streams) {
+        const unsigned s = tid - 64u;
+        post[row * streams + s] = (float)(post_multiplier * sigmoid_f64(
+            (double)mix[streams + s] * inverse * (double)scale[1] + (double)base[streams + s]));
     }
     __syncthreads();
 
@@ -189,21 +226,18 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
     // dependent divisions several microseconds long, so the other wavefronts run the second pass
     // over the row meanwhile.
     const unsigned cells = streams * streams;
-    if (tid < 64u) {
+    if (mixes_here && tid < 64u) {
         // (four streams: every group of sixteen lanes holds the matrix)
         const unsigned held = streams == 4u ? tid & 15u : tid;
         const bool cell = held < cells;
         const unsigned r = cell ? held / streams : 0u, c = cell ? held % streams : 0u;
         const unsigned index = 2u * streams + (cell ? held : 0u);
         float m = (float)((double)mix[index] * inverse * (double)scale[2] + (double)base[index]);
-        double maximum = -__builtin_inf(), total = 0.0, mine = 0.0;
+        double maximum = -__builtin_inf(), total = 0.0;
         for (unsigned k = 0; k < streams; ++k)
             maximum = fmax(maximum, (double)__shfl(m, (int)(r * streams + k), kWave));
-        for (unsigned k = 0; k < streams; ++k) {
-            const double value = exp((double)__shfl(m, (int)(r * streams + k), kWave) - maximum);
-            total += value;
-            if (k == c) mine = value;
-        }
+        const double mine = exp((double)m - maximum);          // an exponential a lane; a row's are added in their order
+        for (unsigned k = 0; k < streams; ++k) total += __shfl(mine, (int)(r * streams + k), kWave);
         bad |= cell && (!finite_f64(total) || !(total > 0.0));
         m = (float)((double)(float)mine / total + mhc_epsilon);
         if (streams == 4u) m = sinkhorn4(m, iterations, mhc_epsilon, bad);
@@ -221,28 +255,27 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
         }
         if (tid < cells) combination[row * cells + tid] = m;
     }
+    if (mixes_only) {
+        if (bad) raise_status(status, 1);
+        return;
+    }
 
     // collapsed row: float accumulation over the streams in order, then bf16
     double collapsed_squares = 0.0;
-    if (tid < 64u) {
+    if (tid < kSpared) {
         // busy with the mixing matrix above
     } else if (quads && streams <= kBatch) {
         const float4 *in4 = reinterpret_cast<const float4 *>(in);
         const unsigned count = width >> 2;
-        for (unsigned at = tid - 64u; at < count; at += kWorkers) {
-            float4 v[kBatch];
-#pragma unroll
-            for (unsigned s = 0; s < kBatch; ++s)
-                v[s] = s < streams ? in4[s * count + at] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        auto collapse = [&](unsigned at, const float4 (&rounded)[kBatch]) {
             float4 total = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
             for (unsigned s = 0; s < kBatch; ++s) {
                 if (s < streams) {
-                    const float4 r = bf16_round4(v[s]);
-                    total.x += (float)(gate[s] * (double)r.x);
-                    total.y += (float)(gate[s] * (double)r.y);
-                    total.z += (float)(gate[s] * (double)r.z);
-                    total.w += (float)(gate[s] * (double)r.w);
+                    total.x += (float)(gate[s] * (double)rounded[s].x);
+                    total.y += (float)(gate[s] * (double)rounded[s].y);
+                    total.z += (float)(gate[s] * (double)rounded[s].z);
+                    total.w += (float)(gate[s] * (double)rounded[s].w);
                 }
             }
             bad |= !finite_f32(total.x) || !finite_f32(total.y) || !finite_f32(total.z) || !finite_f32(total.w);
@@ -252,9 +285,24 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
             collapsed_squares += (double)published.y * (double)published.y;
             collapsed_squares += (double)published.z * (double)published.z;
             collapsed_squares += (double)published.w * (double)published.w;
+        };
+        if (held) {
+#pragma unroll
+            for (unsigned u = 0; u < kHeld; ++u)
+                if (tid - kSpared + u * kWorkers < count) collapse(tid - kSpared + u * kWorkers, mine[u]);
+        } else {
+            for (unsigned at = tid - kSpared; at < count; at += kWorkers) {
+                float4 v[kBatch];
+#pragma unroll
+                for (unsigned s = 0; s < kBatch; ++s)
+                    v[s] = s < streams ? in4[s * count + at] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+                for (unsigned s = 0; s < kBatch; ++s) v[s] = bf16_round4(v[s]);
+                collapse(at, v);
+            }
         }
     } else {
-        for (unsigned lane = tid - 64u; lane < width; lane += kWorkers) {
+        for (unsigned lane = tid - kSpared; lane < width; lane += kWorkers) {
             float total = 0.0f;
             for (unsigned s = 0; s < streams; ++s)
                 total += (float)(gate[s] * (double)bf16_round(in[s * width + lane]));
@@ -441,11 +489,11 @@ static int launch_mhc_ingress(const float *rows, const float *mixes, const void 
     static std::once_flag once;
     static bool prepared = false;
     std::call_once(once, [] {
-        prepared =
-            hipFuncSetAttribute((const void *)mhc_ingress_kernel<256>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(kEnvelopeMaxWidth * sizeof(float))) == hipSuccess &&
-            hipFuncSetAttribute((const void *)mhc_ingress_kernel<1024>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(kEnvelopeMaxWidth * sizeof(float))) == hipSuccess;
+        prepared = true;
+        for (const void *kernel : {(const void *)mhc_ingress_kernel<256, false>, (const void *)mhc_ingress_kernel<256, true>,
+                                   (const void *)mhc_ingress_kernel<1024, false>, (const void *)mhc_ingress_kernel<1024, true>})
+            prepared = prepared && hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       (int)(kEnvelopeMaxWidth * sizeof(float))) == hipSuccess;
         if (!prepared) (void)hipGetLastError();
     });
     if (!prepared) {
@@ -455,16 +503,12 @@ static int launch_mhc_ingress(const float *rows, const float *mixes, const void 
     const int quads = width % 4u == 0u && !(((uintptr_t)rows | (uintptr_t)normalized) & 15u) &&
                       !((uintptr_t)norm & (norm_qtype == QT_F32 ? 15u : 7u));
     const unsigned lds = (unsigned)(width * sizeof(float));
-    if (streams * width >= 8192u)
-        mhc_ingress_kernel<1024><<<(unsigned)row_count, 1024, lds, as_stream(stream)>>>(
-            rows, mixes, scale, base, norm, scale_qtype, base_qtype, norm_qtype, (unsigned)streams,
-            (unsigned)width, (unsigned)iterations, rms_epsilon, mhc_epsilon, post_multiplier, normalized, post,
-            combination, quads, status);
-    else
-        mhc_ingress_kernel<256><<<(unsigned)row_count, 256, lds, as_stream(stream)>>>(
-            rows, mixes, scale, base, norm, scale_qtype, base_qtype, norm_qtype, (unsigned)streams,
-            (unsigned)width, (unsigned)iterations, rms_epsilon, mhc_epsilon, post_multiplier, normalized, post,
-            combination, quads, status);
+    const bool split = 2u * row_count <= (uint64_t)compute_units(), wide = streams * width >= 8192u;
+    const auto kernel = wide ? (split ? mhc_ingress_kernel<1024, true> : mhc_ingress_kernel<1024, false>)
+                             : (split ? mhc_ingress_kernel<256, true> : mhc_ingress_kernel<256, false>);
+    kernel<<<(unsigned)(split ? 2u * row_count : row_count), wide ? 1024 : 256, lds, as_stream(stream)>>>(
+        rows, mixes, scale, base, norm, scale_qtype, base_qtype, norm_qtype, (unsigned)streams, (unsigned)width,
+        (unsigned)iterations, rms_epsilon, mhc_epsilon, post_multiplier, normalized, post, combination, quads, status);
     return check_launch("mhc_ingress");
 }
 
