@@ -67,9 +67,10 @@ __device__ __forceinline__ bool finite_f32(float v)
 // softplus. `sigmoid` is YVEX_HIP_SCORING_SIGMOID of the launch-level header.
 __device__ __forceinline__ double route_score(double v, int scoring)
 {
-    if (scoring == 1)
-        return v >= 0.0 ? 1.0 / (1.0 + exp(-v)) : exp(v) / (1.0 + exp(v));
-    const double softplus = v > 0.0 ? v + log1p(exp(-v)) : log1p(exp(v));
+    // (one exponential whatever the sign: lanes of both signs would run a branch each)
+    const double e = exp(-fabs(v));
+    if (scoring == 1) return (v >= 0.0 ? 1.0 : e) / (1.0 + e);
+    const double l = log1p(e), softplus = v > 0.0 ? v + l : l;
     return sqrt(softplus);
 }
 

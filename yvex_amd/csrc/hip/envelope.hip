@@ -59,9 +59,8 @@ __device__ __forceinline__ double workgroup_sum(double v, double *slots)
 
 __device__ __forceinline__ double sigmoid_f64(double value)
 {
-    if (value >= 0.0) return 1.0 / (1.0 + exp(-value));
-    const double direct = exp(value);
-    return direct / (1.0 + direct);
+    const double e = exp(-fabs(value));
+    return (value >= 0.0 ? 1.0 : e) / (1.0 + e);
 }
 
 __device__ __forceinline__ float4 bf16_round4(float4 v)

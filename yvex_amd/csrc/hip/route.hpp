@@ -48,19 +48,20 @@ __device__ __forceinline__ void route_inputs_load(RouteInputs &in, const float *
     }
 }
 
-// One row by one wavefront. `published`: in.value holds scores, not logits.
+// One row by one wavefront. `published`: in.value holds scores, not logits. `chosen`: the selection for the workgroup's
+// own use as well.
 __device__ __forceinline__ void route_row(
     const RouteInputs &in, bool published, unsigned long long row, unsigned lane,
     unsigned experts, unsigned topk, int scoring, int normalize, double scaling,
-    unsigned long long *__restrict__ selected, float *__restrict__ weights, int *status)
+    unsigned long long *__restrict__ selected, float *__restrict__ weights, int *status, unsigned *chosen = nullptr)
 {
     float score[4];
-    unsigned long long key[4];
+    unsigned key[4];       // ordered as the biased scores are; zero: no expert, or one that is taken
 #pragma unroll
     for (unsigned i = 0; i < 4u; ++i) {
         const unsigned e = lane * 4u + i;
         score[i] = 0.0f;
-        key[i] = 0ull;
+        key[i] = 0u;
         if (e < experts) {
             if (published) {
                 score[i] = in.value[i];
@@ -72,37 +73,35 @@ __device__ __forceinline__ void route_row(
             if (!finite_f32(score[i]) || !finite_f32(biased)) raise_status(status, 1);
             biased += 0.0f;   // -0 and +0 must compare equal
             const unsigned bits = __float_as_uint(biased);
-            const unsigned sortable = (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);
-            // larger score first, then the lower expert ordinal; +1 keeps live keys non-zero
-            key[i] = ((unsigned long long)sortable << 32) | (unsigned long long)(0xfffffffeu - e + 1u);
+            key[i] = (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);       // (zero for a NaN only)
         }
     }
     double total = 0.0;
     float picked_score = 0.0f;   // lane r keeps the score of rank r
     for (unsigned rank = 0; rank < topk; ++rank) {
-        unsigned long long best = key[0];
-#pragma unroll
-        for (unsigned i = 1; i < 4u; ++i) best = key[i] > best ? key[i] : best;
-        // The wave's best key in two steps that need no cross-lane permutes through LDS: the
-        // largest score word, then the first lane holding it (a lane's ordinals are below the
-        // next lane's, and its own best already is its lowest ordinal with that score).
-        const unsigned top = wave_max_u32((unsigned)(best >> 32));
-        const unsigned long long holders = __ballot((unsigned)(best >> 32) == top);
+        // The largest key of the wave, then the lowest ordinal that has it: the first lane (a lane's ordinals are
+        // below the next lane's), and in the lane the first of its four. No cross-lane permutes through LDS.
+        const unsigned first = key[0] > key[1] ? key[0] : key[1], second = key[2] > key[3] ? key[2] : key[3];
+        const unsigned top = wave_max_u32(first > second ? first : second);
+        const unsigned place = key[0] == top ? 0u : key[1] == top ? 1u : key[2] == top ? 2u : 3u;
+        const unsigned long long holders = __ballot(key[0] == top || key[1] == top || key[2] == top || key[3] == top);
         const unsigned winner = (unsigned)__builtin_ctzll(holders);
-        const unsigned e = 0xffffffffu - (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(best & 0xffffffffull),
-                                                                             (int)winner);
+        const unsigned e = 4u * winner + (unsigned)__builtin_amdgcn_readlane((int)place, (int)winner);
         float s = 0.0f;
 #pragma unroll
         for (unsigned i = 0; i < 4u; ++i)
             if (lane * 4u + i == e) {
                 s = score[i];
-                key[i] = 0ull;
+                key[i] = 0u;
             }
         // (the winner's ordinal is the same in every lane: a lane read, no permute through LDS)
         s = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), (int)(e >> 2)));
         total += (double)s;                 // rank order, in double (src/graph/moe.c:566-574)
         if (lane == rank) picked_score = s;
-        if (lane == 0u) selected[row * topk + rank] = e;
+        if (lane == 0u) {
+            selected[row * topk + rank] = e;
+            if (chosen) chosen[rank] = e;
+        }
     }
     if (normalize && !(total > 0.0 && total < 1.0e300)) raise_status(status, 1);
     if (lane < topk) {
