@@ -428,9 +428,10 @@ def test_iq2_rows_of_tall_matrices_are_the_sweeps_bits(gpu, oracle, rows, inputs
 
 
 # the 32-row tiles of the F32 projection: ragged on both sides, fewer columns than waves, one launch and split, 16 and 32
-# input rows a tile; formats other than F32 (one launch)
+# input rows a tile; formats other than F32 (one launch); below eight input rows, sixteen waves a weight row
 @pytest.mark.parametrize("qtype,rows,width,inputs", [
     ("F32", 1, 128, 257), ("F32", 250, 1024, 1570), ("F32", 33, 16512, 17), ("F32", 65, 2176, 301), ("F32", 255, 4096, 97),
+    ("F32", 200, 6148, 5), ("F32", 129, 6400, 6), ("F32", 250, 7168, 7), ("F32", 24, 16388, 7), ("F32", 3, 33000, 2),
     ("F16", 31, 64, 256), ("BF16", 33, 320, 511), ("Q8_0", 97, 448, 289)])
 def test_f32_tiles_of_32_weight_rows_match_float64(gpu, oracle, qtype, rows, width, inputs):
     """Sums of exact products in double, rounded once: half a unit in the last place and the double

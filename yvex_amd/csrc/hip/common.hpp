@@ -110,6 +110,29 @@ __device__ __forceinline__ int dpp_move(int v)
     return __builtin_amdgcn_update_dpp(0, v, CTRL, ROW_MASK, 0xf, false);
 }
 
+// A double moved by a data-parallel-primitive step (both halves).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v)
+{
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
+    const unsigned low = (unsigned)dpp_move<CTRL, 0xf>((int)(unsigned)bits);
+    const unsigned high = (unsigned)dpp_move<CTRL, 0xf>((int)(unsigned)(bits >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)high << 32) | low));
+}
+
+// Sum of the 64 lanes, in every lane: the butterfly over lanes 32, 16, 8, 4, 2 and 1 apart. Inside sixteen lanes
+// row_ror 8, 4, 2, 1 fetch what the butterfly's lanes hold by then, without a permute through LDS each.
+__device__ __forceinline__ double wave_sum_f64(double v)
+{
+    v += __shfl_xor(v, 32, kWave);
+    v += __shfl_xor(v, 16, kWave);
+    v += dpp_f64<0x128>(v);
+    v += dpp_f64<0x124>(v);
+    v += dpp_f64<0x122>(v);
+    v += dpp_f64<0x121>(v);
+    return v;
+}
+
 template <int WIDTH>
 __device__ __forceinline__ int group_sum_i32(int v)
 {

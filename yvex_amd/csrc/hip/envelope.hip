@@ -26,28 +26,13 @@ __device__ __forceinline__ bool finite_f64(double v)
     return (__double_as_longlong(v) & 0x7ff0000000000000ll) != 0x7ff0000000000000ll;
 }
 
-// A double moved by a data-parallel-primitive step (both halves).
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v)
-{
-    const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
-    const unsigned low = (unsigned)dpp_move<CTRL, 0xf>((int)(unsigned)bits);
-    const unsigned high = (unsigned)dpp_move<CTRL, 0xf>((int)(unsigned)(bits >> 32));
-    return __longlong_as_double((long long)(((unsigned long long)high << 32) | low));
-}
-
 // Sum over the workgroup, the same value in every thread: a butterfly inside each wavefront,
 // then the wavefront totals in order. The order is fixed, so a row's result does not depend on
 // where it runs.
 template <unsigned WAVES>
 __device__ __forceinline__ double workgroup_sum(double v, double *slots)
 {
-    v += __shfl_xor(v, 32, kWave);
-    v += __shfl_xor(v, 16, kWave);
-    v += dpp_f64<0x128>(v);        // row_ror 8, 4, 2, 1: what they fetch is what the butterfly's lanes hold by then,
-    v += dpp_f64<0x124>(v);        // without a permute through LDS each
-    v += dpp_f64<0x122>(v);
-    v += dpp_f64<0x121>(v);
+    v = wave_sum_f64(v);
     if ((threadIdx.x & 63u) == 0u) slots[threadIdx.x >> 6] = v;
     __syncthreads();
     double total = slots[0];

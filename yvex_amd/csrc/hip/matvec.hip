@@ -447,17 +447,21 @@ __global__ __launch_bounds__(256) void matvec_scalar_kernel(MatvecArgs a, unsign
 // step), DEPTH steps of weight and input loads are in flight before the first product, and the
 // four waves' double-precision sums are joined through LDS in wave order. Products and sums in
 // double as above.
-// WAVE_ROW: a wave a weight row (four rows a workgroup, no barrier) for matrices of many rows,
-// where the device is full either way and a workgroup a row is a launch and a barrier a row.
-template <unsigned QT, int T, int DEPTH, bool WAVE_ROW>
-__global__ __launch_bounds__(256) void matvec_scalar_few_kernel(MatvecArgs a)
+// ROW_WAVES: waves that share a row. One (four rows a workgroup, no barrier) for matrices of many rows, where the device
+// is full either way and a workgroup a row is a launch and a barrier a row; sixteen where a row has a piece for each of
+// their threads: the products are double-precision and one wave issues an instruction in five cycles, so four waves, one a
+// SIMD, took longer over a row than the memory (256 x 7168
+// by 3 / 5 / 7 rows 7.1 / 8.8 / 9.3 -> 5.7 / 6.7 / 8.0 us, 24 x 16384 by 1 / 3 / 7 4.8 / 8.9 / 9.0 -> 4.2 / 6.7 / 6.8).
+template <unsigned QT, int T, int DEPTH, unsigned ROW_WAVES>
+__global__ __launch_bounds__(ROW_WAVES == 1u ? 256u : 64u * ROW_WAVES) void matvec_scalar_few_kernel(MatvecArgs a)
 {
-    constexpr unsigned kSpan = WAVE_ROW ? 64u : 256u;       // threads that share a row
+    constexpr bool WAVE_ROW = ROW_WAVES == 1u;
+    constexpr unsigned kSpan = 64u * ROW_WAVES;             // threads that share a row
     typedef float v4f __attribute__((ext_vector_type(4)));
     typedef unsigned v4u __attribute__((ext_vector_type(4)));
     constexpr int kColumns = QT == QT_F32 ? 4 : 8;           // weights in a 16-byte piece
     constexpr int kInputs = kColumns / 4;                    // 16-byte pieces of an input row beside it
-    __shared__ double partial[3][T];
+    __shared__ double partial[ROW_WAVES][T];
     const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const unsigned long long row = WAVE_ROW ? (unsigned long long)blockIdx.x * 4ull + wave : blockIdx.x;
     const unsigned long long in0 = (unsigned long long)blockIdx.y * T;
@@ -525,9 +529,8 @@ __global__ __launch_bounds__(256) void matvec_scalar_few_kernel(MatvecArgs a)
     if (bad) raise_status(a.status, 1);
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-#pragma unroll
-        for (int offset = 32; offset > 0; offset >>= 1) acc[t] += __shfl_xor(acc[t], offset, kWave);
-        if (!WAVE_ROW && wave && lane == 0u) partial[wave - 1u][t] = acc[t];
+        acc[t] = wave_sum_f64(acc[t]);
+        if (!WAVE_ROW && lane == 0u) partial[wave][t] = acc[t];
     }
     if constexpr (WAVE_ROW) {
         if (lane != 0u) return;
@@ -537,26 +540,35 @@ __global__ __launch_bounds__(256) void matvec_scalar_few_kernel(MatvecArgs a)
         return;
     }
     __syncthreads();
-    if (threadIdx.x != 0u) return;
+    const unsigned t = threadIdx.x;          // a thread an input row
+    if (t >= (unsigned)T || in0 + t >= a.input_rows) return;
+    double sum = partial[0][t];
 #pragma unroll
-    for (int t = 0; t < T; ++t) {
-        if (in0 + t >= a.input_rows) continue;
-        const double sum = acc[t] + partial[0][t] + partial[1][t] + partial[2][t];
-        matvec_publish(a, in0 + t, row, (float)sum);
-    }
+    for (unsigned w = 1; w < ROW_WAVES; ++w) sum += partial[w][t];
+    matvec_publish(a, in0 + t, row, (float)sum);
 }
 
-template <unsigned QT, bool WAVE_ROW>
+template <unsigned QT, unsigned ROW_WAVES>
 static int launch_scalar_few_rows(const MatvecArgs &a, hipStream_t s)
 {
-    const unsigned long long grid_x = WAVE_ROW ? (a.row_count + 3ull) / 4ull : a.row_count;
+    constexpr unsigned kThreads = ROW_WAVES == 1u ? 256u : 64u * ROW_WAVES;
+    constexpr int kDeep = ROW_WAVES == 16u ? 4 : 8;
+    const unsigned long long grid_x = ROW_WAVES == 1u ? (a.row_count + 3ull) / 4ull : a.row_count;
     if (a.input_rows == 1ull)
-        matvec_scalar_few_kernel<QT, 1, 8, WAVE_ROW><<<dim3((unsigned)grid_x, 1), 256, 0, s>>>(a);
+        matvec_scalar_few_kernel<QT, 1, kDeep, ROW_WAVES><<<dim3((unsigned)grid_x, 1), kThreads, 0, s>>>(a);
     else if (a.input_rows == 2ull)
-        matvec_scalar_few_kernel<QT, 2, 8, WAVE_ROW><<<dim3((unsigned)grid_x, 1), 256, 0, s>>>(a);
-    else
-        matvec_scalar_few_kernel<QT, 4, 4, WAVE_ROW><<<dim3((unsigned)grid_x, (unsigned)((a.input_rows + 3ull) / 4ull)),
-                                                       256, 0, s>>>(a);
+        matvec_scalar_few_kernel<QT, 2, kDeep, ROW_WAVES><<<dim3((unsigned)grid_x, 1), kThreads, 0, s>>>(a);
+    else if (ROW_WAVES == 16u && a.input_rows > 4ull && 2ull * a.row_count > (unsigned long long)compute_units()) {
+        // (all of them a workgroup, and its weight row once, unless two workgroups a row have a compute unit each)
+        if constexpr (ROW_WAVES == 16u) {
+            if (a.input_rows == 5ull) matvec_scalar_few_kernel<QT, 5, 2, 16><<<(unsigned)grid_x, kThreads, 0, s>>>(a);
+            else if (a.input_rows == 6ull) matvec_scalar_few_kernel<QT, 6, 2, 16><<<(unsigned)grid_x, kThreads, 0, s>>>(a);
+            else if (a.input_rows == 7ull) matvec_scalar_few_kernel<QT, 7, 2, 16><<<(unsigned)grid_x, kThreads, 0, s>>>(a);
+            else return ST_BOUNDS;
+        }
+    } else
+        matvec_scalar_few_kernel<QT, 4, kDeep / 2, ROW_WAVES><<<dim3((unsigned)grid_x, (unsigned)((a.input_rows + 3ull) / 4ull)),
+                                                                kThreads, 0, s>>>(a);
     return check_launch("matvec_scalar_few");
 }
 
@@ -564,7 +576,14 @@ template <unsigned QT>
 static int launch_scalar_few(const MatvecArgs &a, hipStream_t s)
 {
     // (sixteen waves a compute unit either way from 4096 rows on)
-    return a.row_count >= 4096ull ? launch_scalar_few_rows<QT, true>(a, s) : launch_scalar_few_rows<QT, false>(a, s);
+    if (a.row_count >= 4096ull) return launch_scalar_few_rows<QT, 1>(a, s);
+    // sixteen waves a row while every row has a compute unit and its columns are work for them (four and sixteen: 256 x
+    // 7168 by 2 rows 4.8 and 5.3 us, by 3 6.5 and 5.8; 256 x 4096 by 5 5.4 and 6.9; 1000 x 4096 by 1 6.7 and 9.1)
+    if constexpr (QT == QT_F32)
+        if (a.row_count <= (unsigned long long)compute_units() &&
+            (a.row_width >= 16384ull || (a.row_width >= 6144ull && a.input_rows >= 3ull)))
+            return launch_scalar_few_rows<QT, 16>(a, s);
+    return launch_scalar_few_rows<QT, 4>(a, s);
 }
 
 // F32 weight rows against a batch of F32 input rows (a router or mixing projection over a row
