@@ -5,27 +5,6 @@
 
 namespace yvex {
 
-// Largest value of the 64 lanes, in every lane: butterflies inside each row of 16 lanes, then the
-// rows' results carried upward (lane 15 into the next row, lane 31 into the upper half) and the
-// last lane read back.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ unsigned dpp_max_u32(unsigned v)
-{
-    const unsigned other = (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROWS, 0xf, false);
-    return other > v ? other : v;
-}
-
-__device__ __forceinline__ unsigned wave_max_u32(unsigned v)
-{
-    v = dpp_max_u32<0xb1, 0xf>(v);    // quad_perm [1, 0, 3, 2]
-    v = dpp_max_u32<0x4e, 0xf>(v);    // quad_perm [2, 3, 0, 1]
-    v = dpp_max_u32<0x141, 0xf>(v);   // row_half_mirror
-    v = dpp_max_u32<0x140, 0xf>(v);   // row_mirror
-    v = dpp_max_u32<0x142, 0xa>(v);   // row_bcast15 into rows 1 and 3
-    v = dpp_max_u32<0x143, 0xc>(v);   // row_bcast31 into rows 2 and 3
-    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
-}
-
 // What a lane reads of one row: the logits (or the scores a launch before this one has
 // published: the float a double-precision score rounds to, what route_row works out from a logit
 // otherwise) and the correction biases of experts 4 lane .. 4 lane + 3. The loads depend on
