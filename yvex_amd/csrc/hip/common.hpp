@@ -131,6 +131,18 @@ __device__ __forceinline__ unsigned wave_max_u32(unsigned v)
     return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
 }
 
+// Sums over the lanes up to and with one's own: inside each row of 16 lanes, then the rows' totals carried upward.
+__device__ __forceinline__ unsigned wave_inclusive_sum_u32(unsigned v)
+{
+    v += (unsigned)dpp_move<0x111, 0xf>((int)v);    // row_shr 1, 2, 4, 8
+    v += (unsigned)dpp_move<0x112, 0xf>((int)v);
+    v += (unsigned)dpp_move<0x114, 0xf>((int)v);
+    v += (unsigned)dpp_move<0x118, 0xf>((int)v);
+    v += (unsigned)dpp_move<0x142, 0xa>((int)v);    // row_bcast15, row_bcast31
+    v += (unsigned)dpp_move<0x143, 0xc>((int)v);
+    return v;
+}
+
 // A double moved by a data-parallel-primitive step (both halves).
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v)

@@ -169,10 +169,7 @@ __global__ __launch_bounds__(256) void matvec_block_kernel(MatvecArgs a)
     for (int t = 0; t < T; ++t) {
         float sum;
         if constexpr (kWide) {
-            double wide = acc[t];
-#pragma unroll
-            for (int offset = 32; offset > 0; offset >>= 1) wide += __shfl_xor(wide, offset, kWave);
-            sum = (float)wide;
+            sum = (float)wave_sum_f64(acc[t]);
         } else {
             sum = group_sum_f32<64>(acc[t]);
         }

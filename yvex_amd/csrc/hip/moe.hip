@@ -166,24 +166,16 @@ __device__ __forceinline__ void worklist_block(
     }
     __syncthreads();
     // Inclusive prefix sums over the experts (<= 256: the first four wavefronts) of population,
-    // sweep count and occupancy: a shuffle scan inside each wavefront, the wavefronts' totals
+    // sweep count and occupancy: a scan inside each wavefront, the wavefronts' totals
     // through LDS (one barrier); every expert then publishes its own bucket.
     unsigned *scan = slot + experts;                       // [4][3] wavefront totals; [1536] running maximum
     const unsigned n_mine = tid < experts ? population[tid] : 0u;
     unsigned sum_n = n_mine, sum_sweeps = (n_mine + (unsigned)kPass - 1u) / (unsigned)kPass,
              sum_used = n_mine ? 1u : 0u;
     if (tid < 256u) {
-#pragma unroll
-        for (int step = 1; step < 64; step <<= 1) {
-            const unsigned a = (unsigned)__shfl_up((int)sum_n, step, kWave);
-            const unsigned b = (unsigned)__shfl_up((int)sum_sweeps, step, kWave);
-            const unsigned c = (unsigned)__shfl_up((int)sum_used, step, kWave);
-            if ((int)(tid & 63u) >= step) {
-                sum_n += a;
-                sum_sweeps += b;
-                sum_used += c;
-            }
-        }
+        sum_n = wave_inclusive_sum_u32(sum_n);
+        sum_sweeps = wave_inclusive_sum_u32(sum_sweeps);
+        sum_used = wave_inclusive_sum_u32(sum_used);
         if ((tid & 63u) == 63u) {
             scan[3u * (tid >> 6)] = sum_n;
             scan[3u * (tid >> 6) + 1u] = sum_sweeps;
@@ -233,12 +225,7 @@ __device__ __forceinline__ void worklist_block(
     }
     // largest population: one atomic per wave after a wave-wide maximum
     {
-        unsigned n = tid < experts ? population[tid] : 0u;
-#pragma unroll
-        for (int offset_lanes = 32; offset_lanes > 0; offset_lanes >>= 1) {
-            const unsigned other = (unsigned)__shfl_xor((int)n, offset_lanes, kWave);
-            n = other > n ? other : n;
-        }
+        const unsigned n = wave_max_u32(tid < experts ? population[tid] : 0u);
         if ((tid & 63u) == 0u && tid < 256u) atomicMax(&scan[1536u], n);
     }
     __syncthreads();

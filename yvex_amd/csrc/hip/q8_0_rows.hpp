@@ -115,10 +115,7 @@ __device__ __forceinline__ void held_row(const unsigned char *row, unsigned unit
     }
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-        double wide = acc[t];
-#pragma unroll
-        for (int offset = 32; offset > 0; offset >>= 1) wide += __shfl_xor(wide, offset, kWave);
-        sums[t] = (float)wide;
+        sums[t] = (float)wave_sum_f64(acc[t]);
     }
 }
 

@@ -918,13 +918,7 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
     }
     static_assert(kMaxSweeps * sweep_cost<QT>(4u) < 65536u, "a prefix is two 16-bit sums");
     const unsigned packed = (sweeps_here << 16) | cost_here;
-    unsigned inclusive = packed;
-    inclusive += (unsigned)dpp_move<0x111, 0xf>((int)inclusive);    // row_shr 1, 2, 4, 8
-    inclusive += (unsigned)dpp_move<0x112, 0xf>((int)inclusive);
-    inclusive += (unsigned)dpp_move<0x114, 0xf>((int)inclusive);
-    inclusive += (unsigned)dpp_move<0x118, 0xf>((int)inclusive);
-    inclusive += (unsigned)dpp_move<0x142, 0xa>((int)inclusive);    // row_bcast15, row_bcast31
-    inclusive += (unsigned)dpp_move<0x143, 0xc>((int)inclusive);
+    const unsigned inclusive = wave_inclusive_sum_u32(packed);
     const unsigned before = inclusive - packed;
     const unsigned totals = (unsigned)__builtin_amdgcn_readlane((int)inclusive, 63);
     const unsigned row_cost = extra_cost + (totals & 0xffffu), all_sweeps = extra_sweeps + (totals >> 16);
