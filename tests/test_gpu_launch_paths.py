@@ -111,11 +111,12 @@ def test_quantizing_projection_is_quantization_and_projection(gpu, oracle, rows,
         assert not lib.yvex_hip_matvec_quantizing_supported(ptr(at), C.c_uint(qtype), u64(rows), u64(width), u64(row_bytes), u64(n))
 
 
-# 16 x 16 tiles on eight waves and on four, and the 32 x 32 Q8_0 tiles: ragged on both sides, fewer superblocks than
+# 16 x 16 tiles on eight waves and on four, and the 32 x 32 and 16 x 16 Q8_0 tiles, the latter between 16-byte boundaries: ragged on both sides, fewer superblocks than
 # waves, a superblock more than a round of them, one row against many
 @pytest.mark.parametrize("qtype,rows,width,inputs", [
     ("Q4_K", 1, 256, 61), ("Q4_K", 17, 2304, 33), ("Q4_K", 4094, 1280, 19), ("Q4_K", 2065, 512, 31), ("Q4_K", 500, 2816, 66),
-    ("Q8_0", 1, 256, 61), ("Q8_0", 17, 1280, 33), ("Q8_0", 2047, 1792, 95)])
+    ("Q8_0", 1, 256, 61), ("Q8_0", 17, 1280, 33), ("Q8_0", 2047, 1792, 95), ("Q8_0", 8201, 1024, 2),
+    ("Q8_0", 1, 256, 12), ("Q8_0", 33, 2304, 16), ("Q8_0", 1001, 2816, 31), ("Q8_0", 4095, 512, 11)])
 def test_dense_tiles_with_ragged_edges_are_the_oracles_bits(gpu, oracle, qtype, rows, width, inputs):
     from yvex_amd import kernels as K
     qt = getattr(oracle, qtype)
@@ -123,10 +124,13 @@ def test_dense_tiles_with_ragged_edges_are_the_oracles_bits(gpu, oracle, qtype, 
     w, x = g.weights(qt, rows, width), g.normal(inputs * width).reshape(inputs, width)
     status = K.new_status(gpu)
     act = K.q8k_quantize(dev(x, gpu), status)
-    got = K.matvec(dev(w, gpu), qt, rows, width, act, input_q8=True, input_rows=inputs, status=status).cpu().numpy()
-    assert int(status.item()) == 0
-    want = oracle.q8_matvec(qt, w, rows, width, oracle.q8k_quantize(x), inputs)
-    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    held = torch.zeros(w.size + 4, dtype=torch.uint8, device=gpu)
+    held[4:] = dev(w, gpu)
+    for weights in (dev(w, gpu),) if qtype == "Q4_K" else (dev(w, gpu), held[4:]):
+        got = K.matvec(weights, qt, rows, width, act, input_q8=True, input_rows=inputs, status=status).cpu().numpy()
+        assert int(status.item()) == 0
+        want = oracle.q8_matvec(qt, w, rows, width, oracle.q8k_quantize(x), inputs)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
 @pytest.mark.parametrize("rows,width,inputs", [(34, 512, 1), (128, 256, 5), (2048, 512, 17), (70, 768, 40)])

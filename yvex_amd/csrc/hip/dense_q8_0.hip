@@ -271,6 +271,126 @@ __global__ __launch_bounds__(64 * kPlainWaves) void dense_q8_0_kernel(DenseQ80Ar
     }
 }
 
+constexpr unsigned kSmallWaves = 8u;
+// LDS of a wave: 16 weight rows' superblock, 16 input rows' codes (both 272 bytes a row), their scales
+constexpr unsigned kSmallAct = 16u * kStagedPitch, kSmallScales = 2u * kSmallAct, kSmallWindow = kSmallScales + 64u;
+constexpr unsigned kSmallLdsBytes = kSmallWaves * kSmallWindow;        // (the partial tiles take their place in the end)
+
+// 16 weight rows x 16 input rows a workgroup, a superblock in eight a wave, on V_MFMA_I32_16X16X32_I8: twice the workgroups
+// of the 32 x 32 tiles and no token slot wasted on a batch of sixteen. Loads in runs, a superblock ahead, through LDS as
+// above. Lane (r, q) holds bytes 8 q .. 8 q + 7 of input row r's block (A) and of weight row r's block (B); accumulator
+// i is weight row r against input row 4 q + i. 4096 x 4096 by 4 / 8 / 16 rows 10.2 / 14.4 / 12.8 us (the first two on
+// matvec_block_kernel, the third on the 32 x 32 tiles) -> 7.9 / 8.1 / 8.9, 2048 x 7168 by 4 / 16 / 32 9.9 / 17.2 / 18.3 ->
+// 8.7 / 10.2 / 10.0, 1024 x 4096 by 64 13.0 -> 7.4.
+__global__ __launch_bounds__(64 * kSmallWaves) void dense_q8_0_small_kernel(DenseQ80Args g)
+{
+    typedef int v4s __attribute__((ext_vector_type(4)));
+    typedef v4i v4i_dword __attribute__((aligned(4)));
+    extern __shared__ __align__(16) unsigned char dense_q8_0_small_lds[];
+    if (lds_address_of(dense_q8_0_small_lds) != 0u) {   // operands are addressed by absolute LDS offsets
+        if (threadIdx.x == 0u) raise_status(g.status, 2);
+        return;
+    }
+    choose_matrix(g);
+    const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const unsigned r = lane & 15u, q = lane >> 4;
+    const unsigned long long row0 = (unsigned long long)blockIdx.x * 16ull, tok0 = (unsigned long long)blockIdx.y * 16ull;
+    const unsigned rows_here = (unsigned)(g.row_count - row0 < 16ull ? g.row_count - row0 : 16ull);
+    const unsigned toks_here = (unsigned)(g.input_rows - tok0 < 16ull ? g.input_rows - tok0 : 16ull);
+    const unsigned long long act_row_bytes = (unsigned long long)g.blocks * kQ8KBytes;
+    const unsigned char *const weights = g.encoded + row0 * g.row_bytes, *const acts = g.act + tok0 * act_row_bytes;
+    // pieces 64 k + lane of 16 rows x 17 and of 16 rows x 16 (a ragged edge repeats the last row)
+    const unsigned char *weight_at[5], *act_at[4];
+#pragma unroll
+    for (unsigned k = 0; k < 5u; ++k) {
+        const unsigned piece = k < 4u ? 64u * k + lane : 256u + r, row = piece / 17u;
+        weight_at[k] = weights + (row < rows_here ? row : rows_here - 1u) * g.row_bytes + 16u * (piece - 17u * row);
+    }
+#pragma unroll
+    for (unsigned k = 0; k < 4u; ++k) {
+        const unsigned row = 4u * k + q;
+        act_at[k] = acts + (row < toks_here ? row : toks_here - 1u) * act_row_bytes + 4u + 16u * r;
+    }
+    const unsigned char *const scale_from = acts + (r < toks_here ? r : toks_here - 1u) * act_row_bytes;
+    struct {
+        v4i weights[5], acts[4];
+        unsigned scale;
+    } ahead;
+    auto request = [&](unsigned sb) {
+        const unsigned long long w = sb * 272ull, a = (unsigned long long)sb * kQ8KBytes;
+#pragma unroll
+        for (unsigned k = 0; k < 5u; ++k) ahead.weights[k] = *reinterpret_cast<const v4i_dword *>(weight_at[k] + w);
+#pragma unroll
+        for (unsigned k = 0; k < 4u; ++k) ahead.acts[k] = *reinterpret_cast<const v4i_dword *>(act_at[k] + a);
+        ahead.scale = *reinterpret_cast<const unsigned *>(scale_from + a);
+    };
+    const unsigned window = kSmallWindow * wave;
+    const unsigned w_row = window + r * kStagedPitch, a_row = window + kSmallAct + r * kStagedPitch + 8u * q;
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    if (wave < g.blocks) request(wave);
+    for (unsigned sb = wave; sb < g.blocks; sb += kSmallWaves) {
+        // (LDS operations of one wave complete in order)
+#pragma unroll
+        for (unsigned k = 0; k < 4u; ++k) {
+            lds_write_v4i(window + 1024u * k + 16u * lane, ahead.weights[k]);
+            lds_write_v4i(window + kSmallAct + (4u * k + q) * kStagedPitch + 16u * r, ahead.acts[k]);
+        }
+        lds_write_v4i(window + 4096u + 16u * r, ahead.weights[4]);
+        lds_write_u32(window + kSmallScales + 4u * r, ahead.scale);
+        request(sb + kSmallWaves < g.blocks ? sb + kSmallWaves : sb);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const uint4 d4 = read16(window + kSmallScales + 16u * q);
+        const float d_a[4] = {__uint_as_float(d4.x), __uint_as_float(d4.y), __uint_as_float(d4.z), __uint_as_float(d4.w)};
+        float total[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (unsigned c = 0; c < 8u; ++c) {
+            // (an even block's codes start two bytes into a dword)
+            const unsigned at = w_row + ((34u * c + 2u) & ~3u) + 8u * q;
+            unsigned words[3] = {lds_read_u32(at), lds_read_u32(at + 4u), c % 2u == 0u ? lds_read_u32(at + 8u) : 0u};
+            if (c % 2u == 0u) {
+                words[0] = __builtin_amdgcn_alignbyte(words[1], words[0], 2u);
+                words[1] = __builtin_amdgcn_alignbyte(words[2], words[1], 2u);
+            }
+            const uint2 tokens = lds_read_uint2(a_row + 32u * c);
+            const float d_w = f16_bits_to_float(lds_read_u16(w_row + 34u * c));
+            const long a = (long)(((unsigned long long)tokens.y << 32) | tokens.x);
+            const long b = (long)(((unsigned long long)words[1] << 32) | words[0]);
+            const v4s dot = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, v4s{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) total[i] = __builtin_fmaf(d_w * d_a[i], (float)dot[i], total[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] += (double)total[i];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    __syncthreads();
+    double *const partial = reinterpret_cast<double *>(dense_q8_0_small_lds);
+    if (wave) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) partial[((wave - 1u) * 4u + i) * 64u + lane] = acc[i];
+    }
+    __syncthreads();
+    if (wave) return;
+    const unsigned long long row = row0 + r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const unsigned long long token = tok0 + 4u * q + i;
+        double wide = acc[i];
+#pragma unroll
+        for (unsigned w = 0; w + 1u < kSmallWaves; ++w) wide += partial[(w * 4u + i) * 64u + lane];
+        const float sum = (float)wide;
+        if (row >= g.row_count || token >= g.input_rows) continue;
+        const unsigned long long at = token * g.out_stride + row;
+        const float value = g.additive ? sum + g.additive[at] : sum;
+        if (!finite_f32(value)) raise_status(g.status, 1);
+        else g.out[at] = g.output_bf16 ? bf16_round(value) : value;
+    }
+}
+
 // The same product for batches that offer every compute unit a tile of 128 weight rows x 64
 // input rows: the operands of one superblock pass through LDS. GLOBAL_LOAD_LDS instructions whose
 // lanes walk consecutive 16-byte pieces of consecutive rows (a dozen cache lines an instruction
@@ -589,7 +709,8 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
                    (const unsigned char *)act_q8k, input_rows, additive, out, out_stride,
                    output_bf16 ? 1 : 0, status, encoded_second, out_second};
     // Which tiles: a pass over the row width costs a workgroup about the same whatever the device's
-    // load (measured at 16 superblocks a row, microseconds: 14 on the 32-row tile and 18.5 once two such
+    // load (measured at 16 superblocks a row, microseconds: 9 on the 16 x 16 tile and 3.8 more for every such workgroup
+    // that a compute unit has besides, 14 on the 32-row tile and 18.5 once two such
     // workgroups share a compute unit, 29 on the 64-row staged tile and 43 once two of them share
     // a compute unit, 35 on the 128-row tile, 54 on the 128 x 128 tile), so the choice is the number of
     // rounds each shape needs.
@@ -606,11 +727,20 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
                                            stream>>>(g);
         return check_launch("dense_q8_0_staged");
     }
+    const uint64_t token_tiles16 = (input_rows + 15u) / 16u, small = matrices * ((row_count + 15u) / 16u) * token_tiles16;
+    const uint64_t plain = matrices * row_tiles * token_tiles32;
+    const double plain_cost = !units || plain <= units ? 14.0 : 18.5 * (double)((plain + 2u * units - 1u) / (2u * units));
+    const double small_cost = !units || small <= units ? 9.0 : 4.0 + 3.8 * (double)small / (double)units;
+    // (a batch that offers the staged tiles more than these is not theirs: they take 29 us at least)
+    if (small_cost < plain_cost && small_cost < 29.0 && token_tiles16 <= 65535u && (row_count + 15u) / 16u <= 0x7fffffffull) {
+        YVEX_ALLOW_DYNAMIC_LDS(dense_q8_0_small_kernel, kSmallLdsBytes);
+        dense_q8_0_small_kernel<<<dim3((unsigned)((row_count + 15u) / 16u), (unsigned)token_tiles16, (unsigned)matrices),
+                                  64 * kSmallWaves, kSmallLdsBytes, stream>>>(g);
+        return check_launch("dense_q8_0_small");
+    }
     if (aligned16 && units) {
-        const uint64_t plain = matrices * row_tiles * token_tiles32;
         const uint64_t tall = matrices * ((row_count + 127u) / 128u) * token_tiles64,
                        low = matrices * ((row_count + 63u) / 64u) * token_tiles64;
-        const double plain_cost = plain <= units ? 14.0 : 18.5 * (double)((plain + 2u * units - 1u) / (2u * units));
         const double low_share = 43.0 * (double)low / (double)(2u * units);
         const double low_cost = low <= units ? 29.0 : (low_share > 43.0 ? low_share : 43.0);
         const double tall_cost = 35.0 * (double)((tall + units - 1u) / units);

@@ -1114,8 +1114,8 @@ static bool q8_0_takes_matrix_cores(const uint8_t *encoded, uint64_t row_count, 
 {
     const unsigned long long matrix_bytes = row_count * row_bytes;
     return !((uintptr_t)encoded & 3u) &&
-           (input_rows >= 16ull || (input_rows >= 2ull && matrix_bytes >= (32ull << 20)) ||
-            (input_rows >= 12ull && matrix_bytes >= (8ull << 20)));
+           (input_rows >= (matrix_bytes < (2ull << 20) ? 12ull : 10ull) ||
+            (input_rows >= 2ull && matrix_bytes >= (8ull << 20)));
 }
 
 extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint64_t row_count,
@@ -1166,13 +1166,11 @@ extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint6
         !(input_rows < 4ull && dense_fewrows_applies<QT_Q4_K>(a)))
         return launch_q4k_rows_dense(encoded, row_count, row_width, row_bytes, input, input_rows, additive,
                                      out, out_stride, output_bf16 != 0, status, s);
-    // Q8_0 rows against a batch of Q8_K input rows: matrix cores from the reference's threshold on
-    // (src/backend/cuda/private.h:461-464); below it the lane-strided kernel, which reads the
-    // matrix once per input row: fine while the matrix stays in the caches (4096 x 4096, 18 MB:
-    // 10 us up to four rows, 12.5 at eight, 19 at fifteen; the matrix cores 13.5 us throughout),
-    // but 7168 x 7168 (55 MB) takes 15 us for one row, 21 for two and 66 for fifteen where the
-    // matrix cores take 18.5, and an output head of 129 280 x 7168 171 us for one row, 336 for two
-    // and 1.5 ms for fifteen where they take 200 to 235
+    // Q8_0 rows against a batch of Q8_K input rows: matrix cores (the reference's threshold is 16 rows,
+    // src/backend/cuda/private.h:461-464); the lane-strided kernel reads the matrix once per four input rows, which
+    // matrices of under 8 MB bear up to nine (lane-strided and matrix cores: 1024 x 4096 by 4 / 8 / 10 / 12 rows 5.3 / 6.0 /
+    // 7.0 / 7.2 and 6.5 / 6.7 / 6.9 / 7.1 us, 512 x 2048 by 10 4.4 and 4.7), larger ones not from two on (2048 x 4096 by 4 6.9
+    // and 6.8, 4096 x 4096 by 2 / 8 9.8 / 14.7 and 7.7 / 8.1, 7168 x 7168 by 2 19.2 and 16.6)
     if (qtype == QT_Q8_0 && input_q8 && q8_0_takes_matrix_cores(encoded, row_count, row_bytes, input_rows))
         return launch_q8_0_rows_dense(encoded, row_count, row_width, row_bytes, input, input_rows, additive, out,
                                       out_stride, output_bf16 != 0, status, s);
