@@ -73,6 +73,23 @@ def test_q8_0_wide_tiles_are_the_oracles_bits(gpu, oracle, rows, width, inputs):
     assert np.array_equal(got[picked].view(np.uint32), want.view(np.uint32))
 
 
+# IQ2_XXS tiles whose waves share the row width: ragged on both sides, fewer superblocks than waves and a round of them and
+# some, the last superblock of the matrix, either side of the line to the row-batch kernels
+@pytest.mark.parametrize("rows,width,inputs", [(4, 512, 6), (20, 1024, 17), (132, 2560, 40), (500, 4608, 33), (1028, 8192, 16),
+                                               (2048, 512, 96), (2048, 512, 97), (4100, 4096, 50)])
+def test_iq2_tiles_of_small_matrices_are_the_oracles_bits(gpu, oracle, rows, width, inputs):
+    from yvex_amd import kernels as K
+    qt, g = oracle.IQ2_XXS, oracle.Generator(42, f"iq2.small.{rows}.{width}.{inputs}")
+    w, x = g.weights(qt, rows, width), g.normal(inputs * width).reshape(inputs, width)
+    status = K.new_status(gpu)
+    act = K.q8k_quantize(dev(x, gpu), status)
+    got = K.matvec(dev(w, gpu), qt, rows, width, act, input_q8=True, input_rows=inputs, status=status)
+    rounded = K.matvec(dev(w, gpu), qt, rows, width, act, input_q8=True, input_rows=inputs, output_bf16=True, status=status)
+    want = torch.from_numpy(oracle.q8_matvec(qt, w, rows, width, oracle.q8k_quantize(x), inputs)).to(gpu)
+    assert same_bits(got, want) and same_bits(rounded, want.to(torch.bfloat16).float())
+    assert int(status.item()) == 0
+
+
 # one launch that quantizes its input rows: fewer rows than waves, rows whose blocks fill the lanes' chunks or not,
 # rows on dword boundaries and between them, more weight rows than a round of waves
 @pytest.mark.parametrize("rows,width,inputs,offset", [(1, 256, 1, 0), (17, 2048, 2, 2), (33, 2304, 1, 0), (100, 4096, 2, 0),

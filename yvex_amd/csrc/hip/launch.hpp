@@ -47,6 +47,12 @@ int launch_iq2_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t r
                           uint64_t row_bytes, const void *act_q8k, uint64_t input_rows, float *out,
                           bool round_bf16, int *status, hipStream_t stream);
 
+// The same where the matrix is small (dense_iq2.hip), and whether it is.
+bool iq2_rows_small(uint64_t row_count, uint64_t row_width, uint64_t input_rows);
+int launch_iq2_rows_small(const uint8_t *encoded, uint64_t row_count, uint64_t row_width, uint64_t row_bytes,
+                          const void *act_q8k, uint64_t input_rows, float *out, bool output_bf16, int *status,
+                          hipStream_t stream);
+
 // Q8_0 rows x Q8_K input rows on the int8 matrix cores (dense_q8_0.hip); with a second matrix of the
 // same shape both products in one launch.
 int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t row_width,

@@ -1141,17 +1141,16 @@ extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint6
         if (input_stride < row_width) return ST_INVALID_ARG;
         if (!scalar && (((uintptr_t)input & 15u) || (input_stride & 3u))) return ST_INVALID_ARG;
     }
-    // IQ2_XXS rows against a batch of Q8_K input rows: the int8 matrix-core kernels of the
+    // IQ2_XXS rows against a batch of Q8_K input rows: 16 x 16 tiles whose waves share the row width where the matrix is
+    // small (dense_iq2.hip has the line), else the int8 matrix-core kernels of the
     // row-batch expert path, as one bucket that holds every input row (the reference turns its
     // tensor-core kernels on from 16 input rows, src/backend/cuda/private.h:461-464). The time of the sweep
     // below grows with the products, theirs stands while the tiles come out at one round, so below 32
-    // input rows the line lies at a number of products (sweep and these, us): 4096 x 2048 by 16 13.0 and
-    // 14.7, by 20 15.7 and 14.7; 4096 x 4096 by 16 21.4 and 22.7, by 20 25.5 and 22.0; 8192 x 4096 by 8 20.8 and
-    // 22.0, by 12 28.4 and 22.3; 7168 x 7168 by 8 31.7 and 32.0, by 12 45.1 and 32.6. Matrices of many rows are
-    // further behind it: 32 768 x 4096 by 8 72 and 27, by 31 260 and 32; 129 280 x 7168 by 8 508 and 118, by 31
+    // input rows their line lies at a number of products (sweep and these, us): 7168 x 7168 by 8 31.7 and 32.0, by 12 45.1 and
+    // 32.6; 32 768 x 4096 by 8 72 and 27, by 31 260 and 32; 129 280 x 7168 by 8 508 and 118, by 31
     // 1813 and 125. Same exact int32 superblock sums and the same float terms as the sweep, added in
-    // double in superblock order there and here: the same bits.
-    const bool iq2_batch = input_rows >= 32ull || (input_rows >= 8ull && row_width >= 512ull &&
+    // double there and here: the same bits.
+    const bool iq2_batch = input_rows >= 32ull || iq2_rows_small(row_count, row_width, input_rows) || (input_rows >= 8ull && row_width >= 512ull &&
                                                    row_count >= (73728ull + input_rows - 1ull) / input_rows);
     if (qtype == QT_IQ2_XXS && input_q8 && iq2_batch && !additive &&
         out_stride == row_count && row_count % 4ull == 0ull && !((uintptr_t)encoded & 3u) &&

@@ -872,6 +872,8 @@ int launch_iq2_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t r
     int rc = check_matrix(QT_IQ2_XXS, row_width, row_bytes);
     if (rc) return rc;
     if (input_rows > 0xffffffffull || row_count > 0xffffffffull || row_count % 4u) return ST_BOUNDS;
+    if (iq2_rows_small(row_count, row_width, input_rows))
+        return launch_iq2_rows_small(encoded, row_count, row_width, row_bytes, act_q8k, input_rows, out, round_bf16, status, stream);
     yvex_hip_expert_weights w{};
     w.down = encoded;
     w.down_qtype = QT_IQ2_XXS;
