@@ -654,12 +654,7 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
         const unsigned full = tid < 256u ? (unsigned)(population_here / kTileTokens) : 0u;
         const unsigned rest = tid < 256u ? (unsigned)(population_here % kTileTokens) : 0u;
         const unsigned cls = rest <= few_pair_limit(a.few, population_here, kTrashBase + 48u) ? 2u : rest > 32u ? 0u : 1u;
-        unsigned inclusive = full;
-#pragma unroll
-        for (int offset = 1; offset < 64; offset <<= 1) {
-            const unsigned below = (unsigned)__shfl_up((int)inclusive, offset, kWave);
-            if ((int)lane >= offset) inclusive += below;
-        }
+        unsigned inclusive = wave_inclusive_sum_u32(full);
         unsigned rank[2];
 #pragma unroll
         for (unsigned c = 0; c < 2u; ++c) {

@@ -234,12 +234,7 @@ __global__ __launch_bounds__((Map16<QT, S>::kThreads)) void rows16_kernel(Rows16
         const unsigned limit = a.behind ? few_pair_limit(a.tokens, population_here, M::kMisc + 16u) : 0u;
         const unsigned tiles = tid >= 256u || (a.behind && served > limit) ? 0u
                                                                              : (unsigned)((served + a.tokens - 1u) / a.tokens);
-        unsigned inclusive = tiles;
-#pragma unroll
-        for (int offset = 1; offset < 64; offset <<= 1) {
-            const unsigned below = (unsigned)__shfl_up((int)inclusive, offset, kWave);
-            if ((int)lane >= offset) inclusive += below;
-        }
+        unsigned inclusive = wave_inclusive_sum_u32(tiles);
         if (lane == 63u && wave < 4u) lds_write_u32(M::kMisc + 4u * wave, inclusive);
         __syncthreads();
         if (tid < 256u) {

@@ -425,12 +425,7 @@ __global__ __launch_bounds__(kQ4Threads, 2) void rows_q4k_kernel(RowsQ4kArgs g)
         const unsigned long long population = threadIdx.x < buckets ? pr.bucket_populations[threadIdx.x] : 0ull;
         const unsigned rest = (unsigned)(population % kQ4Tokens), left = few_pair_limit(g.few, population, kQ4MetaBase + 48u);
         const unsigned tiles = (unsigned)(population / kQ4Tokens) + (rest > left ? 1u : 0u);
-        unsigned inclusive = tiles;
-#pragma unroll
-        for (int offset = 1; offset < 64; offset <<= 1) {
-            const unsigned below = __shfl_up(inclusive, offset, kWave);
-            if ((int)lane >= offset) inclusive += below;
-        }
+        unsigned inclusive = wave_inclusive_sum_u32(tiles);
         if (lane == 63u) lds_write_u32(kQ4MetaBase + 32u + 4u * wave, inclusive);
         __syncthreads();
         unsigned before = 0u;
@@ -488,11 +483,13 @@ int launch_q4k_rows_grouped(const GroupedProblem &problem, unsigned qtype, bool 
         return ST_INVALID_ARG;
     if (problem.experts > 256u && problem.expert_ids) return ST_BOUNDS;
     const uint64_t row_tiles = (out_rows + (fused ? 63u : 127u)) / (fused ? 64u : 128u);
-    // token tiles: every bucket of more than `few` pairs may end in a partial tile
+    // token tiles: every bucket of more than `few` pairs may end in a partial tile, and no tile holds fewer than that
     const uint64_t partial = (uint64_t)problem.pairs / (few + 1u);
-    const uint64_t token_tiles = problem.expert_ids ? (uint64_t)problem.pairs / kQ4Tokens +
-                                                          (partial < problem.experts ? partial : problem.experts)
-                                                    : ((uint64_t)problem.pairs + kQ4Tokens - 1u) / kQ4Tokens;
+    uint64_t token_tiles = ((uint64_t)problem.pairs + kQ4Tokens - 1u) / kQ4Tokens;
+    if (problem.expert_ids) {
+        token_tiles = (uint64_t)problem.pairs / kQ4Tokens + (partial < problem.experts ? partial : problem.experts);
+        if (few && few < kQ4Tokens && partial && partial < token_tiles) token_tiles = partial;
+    }
     if (row_tiles > 0x7fffffffull || token_tiles > 65535ull) return ST_BOUNDS;
     RowsQ4kArgs g{problem, (unsigned)(width / 256u), (unsigned)out_rows, limit, status, 0, 0, few, nullptr, 0ull};
     const dim3 grid((unsigned)row_tiles, (unsigned)token_tiles);
