@@ -73,6 +73,32 @@ def test_q8_0_wide_tiles_are_the_oracles_bits(gpu, oracle, rows, width, inputs):
     assert np.array_equal(got[picked].view(np.uint32), want.view(np.uint32))
 
 
+# a shape of each Q8_0 kernel: the lane chain, 16 x 16, 32 x 32, 256 x 32, 64 x 64, 128 x 64 and 128 x 128 tiles
+@pytest.mark.parametrize("rows,width,inputs", [(33, 1024, 1), (100, 768, 20), (2047, 512, 95), (65300, 256, 9), (4090, 256, 200),
+                                               (8190, 256, 230), (2047, 512, 2040)])
+@pytest.mark.parametrize("scales,magnitude", [("largest", 2.0 ** 95), ("subnormal", 2.0 ** -108)])
+def test_q8_0_block_scales_reach_as_far_as_floats(gpu, oracle, rows, width, inputs, scales, magnitude):
+    """Products of a weight and an input block's scale near either end of the float range, the sums of some
+    blocks zero: the oracle's bits at every batch size."""
+    from yvex_amd import kernels as K
+    g = oracle.Generator(42, f"range.{scales}.{rows}.{width}.{inputs}")
+    w = g.weights(oracle.Q8_0, rows, width)
+    blocks = w.reshape(-1, 34)
+    # (2^15, or the fp16 subnormals by turns)
+    bits = np.full(len(blocks), 0x7800) if scales == "largest" else 1 + np.arange(len(blocks)) * 7 % 1023
+    blocks[:, 0], blocks[:, 1] = bits & 255, bits >> 8
+    blocks[::5, 2:] = 0
+    x = g.normal(inputs * width).reshape(inputs, width)
+    x = (x / np.abs(x).max() * magnitude).astype(np.float32)
+    status = K.new_status(gpu)
+    act = K.q8k_quantize(dev(x, gpu), status)
+    got = K.matvec(dev(w, gpu), oracle.Q8_0, rows, width, act, input_q8=True, input_rows=inputs, status=status).cpu().numpy()
+    assert int(status.item()) == 0
+    picked = np.unique([0, inputs // 3, inputs // 2, max(inputs - 2, 0), inputs - 1])
+    want = oracle.q8_matvec(oracle.Q8_0, w, rows, width, oracle.q8k_quantize(x[picked]), picked.size)
+    assert np.all(np.isfinite(want)) and np.array_equal(got[picked].view(np.uint32), want.view(np.uint32))
+
+
 # IQ2_XXS tiles whose waves share the row width: ragged on both sides, fewer superblocks than waves and a round of them and
 # some, the last superblock of the matrix, either side of the line to the row-batch kernels
 @pytest.mark.parametrize("rows,width,inputs", [(4, 512, 6), (20, 1024, 17), (132, 2560, 40), (500, 4608, 33), (1028, 8192, 16),

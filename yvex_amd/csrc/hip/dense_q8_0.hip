@@ -54,9 +54,21 @@ __device__ __forceinline__ void choose_matrix(DenseQ80Args &g)
 // float(sum) of a matrix instruction's sums without a conversion each. The instruction starts from the bits of
 // 1 / (2 pi) as an integer instead of zero, which its encoding holds as an inline constant; the sums of one
 // block are below 2^20 and the constant's mantissa is 2 292 099 above its binade's first, 6 096 508 below its last, so the
-// bits of a result are those of the float kStart + 2^-26 sum, and one subtraction, which the vector ALU issues at twice the
-// rate of a conversion, leaves 2^-26 float(sum) exactly.
+// bits of a result are those of the float kStart + 2^-26 sum, and one multiply-add, which the vector ALU issues at twice the
+// rate of a conversion, leaves float(sum) exactly: 2^26 (kStart + 2^-26 sum) - 2^26 kStart. (Not a subtraction with the
+// 2^26 left to a block's scale: that scale times a row's reaches neither as far up nor as far down as a float's range then.)
 constexpr unsigned kStartBits = 0x3e22f983u;
+
+// The 2^26, in a vector register: the multiply-add then holds the 2^26 kStart in its encoding. 4096 x 4096 by 2048 rows on the
+// 128 x 128 tiles 124.8 us so, 127.9 with both in registers, 125.3 with the factor in the encoding (means of 18 runs).
+__device__ __forceinline__ float sum_scale()
+{
+    float scale = 67108864.0f;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(scale));
+#endif
+    return scale;
+}
 
 // The block's sums from kStartBits on, as floats. Written out because the compiler puts a start other than zero into
 // sixteen registers. The results are in their registers behind the last wait states (eleven for a matrix
@@ -91,7 +103,7 @@ constexpr unsigned kStagedPitch = 272u;
 
 // One superblock out of LDS: lane (r, h)'s weight row at `w_row` (272 bytes), its input row's codes, of which it holds
 // sixteen bytes a block, at `a_row`, and the scales of the input rows that it has sums of, four at a time, at `scales`.
-__device__ __forceinline__ void q80_superblock(unsigned w_row, unsigned a_row, unsigned scales, unsigned h, float minus, double (&acc)[16])
+__device__ __forceinline__ void q80_superblock(unsigned w_row, unsigned a_row, unsigned scales, unsigned h, float scale, double (&acc)[16])
 {
     float d_a[16], total[16];
     uint4 lo[2], hi[2] = {};
@@ -133,14 +145,14 @@ __device__ __forceinline__ void q80_superblock(unsigned w_row, unsigned a_row, u
 #pragma unroll
     for (unsigned c = 0; c < 8u; ++c) {
         const v4i codes = codes_of(c);
-        const float d_w = f16_bits_to_float(scale_bits[c % 2u]) * 67108864.0f;       // (what the sums lack)
+        const float d_w = f16_bits_to_float(scale_bits[c % 2u]);
         if (c + 1u < 8u) read_block(c + 1u);
         __builtin_amdgcn_sched_barrier(0);
         const v16f dot = block_sums(tokens[c % 2u], codes);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const float step = d_w * d_a[i], value = dot[i] + minus;
+            const float step = d_w * d_a[i], value = __builtin_fmaf(dot[i], scale, -67108864.0f * __uint_as_float(kStartBits));
             total[i] = c == 0u ? step * value : __builtin_fmaf(step, value, total[i]);
         }
         // (the compiler would sink all of it behind the last block, and keep every block's sums until then)
@@ -152,16 +164,6 @@ __device__ __forceinline__ void q80_superblock(unsigned w_row, unsigned a_row, u
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] += (double)total[i];
-}
-
-// What the sums start from, in a vector register (a subtraction with a constant operand issues at a conversion's rate).
-__device__ __forceinline__ float minus_start()
-{
-    float minus = -__uint_as_float(kStartBits);
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm("" : "+v"(minus));
-#endif
-    return minus;
 }
 
 constexpr unsigned kPlainWaves = 4u;
@@ -218,7 +220,7 @@ __global__ __launch_bounds__(64 * kPlainWaves) void dense_q8_0_kernel(DenseQ80Ar
         ahead.scale = *reinterpret_cast<const unsigned *>(scale_from + a);
     };
     const unsigned window = kPlainWindow * wave;
-    const float minus = minus_start();
+    const float scale = sum_scale();
     double acc[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.0;
@@ -238,7 +240,7 @@ __global__ __launch_bounds__(64 * kPlainWaves) void dense_q8_0_kernel(DenseQ80Ar
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         q80_superblock(window + r * kStagedPitch, window + kPlainAct + r * kStagedPitch + 16u * h, window + kPlainScales + 16u * h, h,
-                       minus, acc);
+                       scale, acc);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -657,7 +659,7 @@ __global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80A
         else if (wave < 6u) copy_to_lds_4_at(a, scale_at, scale_lds + buffer * (kWideTokens * 4u));
     };
 
-    const float minus = minus_start();
+    const float scale = sum_scale();
     double acc[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.0;
@@ -669,7 +671,7 @@ __global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80A
         if (sb + 1u < g.blocks) copies(sb + 1u);
         q80_superblock(buffer * kWideWeightBytes + (32u * row_block + r) * kStagedPitch,
                        kWideActBase + buffer * kWideActBytes + (32u * token_block + r) * kStagedPitch + 16u * h,
-                       kWideScaleBase + buffer * (kWideTokens * 4u) + (32u * token_block + 4u * h) * 4u, h, minus, acc);
+                       kWideScaleBase + buffer * (kWideTokens * 4u) + (32u * token_block + 4u * h) * 4u, h, scale, acc);
         // the next superblock's copies have landed and every wave is done with this one's buffers
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
