@@ -20,6 +20,8 @@ namespace yvex {
 constexpr unsigned kEnvelopeThreads = 256;
 constexpr unsigned kEnvelopeMaxStreams = 7;       // (streams + 2) * streams <= 64 mixing rows
 constexpr unsigned kEnvelopeMaxWidth = 16384;     // the reference's bound (src/graph/moe.c:453-455)
+constexpr unsigned kEnvelopeLdsBytes = 147456;    // a row of floats and what else fits
+static_assert(kEnvelopeMaxWidth * sizeof(float) <= kEnvelopeLdsBytes, "the collapsed row");
 
 __device__ __forceinline__ bool finite_f64(double v)
 {
@@ -53,6 +55,19 @@ __device__ __forceinline__ float4 bf16_round4(float4 v)
     return make_float4(bf16_round(v.x), bf16_round(v.y), bf16_round(v.z), bf16_round(v.w));
 }
 
+// Four values that bf16 holds, as it holds them, and back.
+__device__ __forceinline__ uint2 bf16_pack4(float4 v)
+{
+    return make_uint2(__builtin_amdgcn_perm(__float_as_uint(v.y), __float_as_uint(v.x), 0x07060302u),
+                      __builtin_amdgcn_perm(__float_as_uint(v.w), __float_as_uint(v.z), 0x07060302u));
+}
+
+__device__ __forceinline__ float4 bf16_unpack4(uint2 v)
+{
+    return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u),
+                       __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
+}
+
 // A coefficient vector (scale, base, norm) as the layer stores it, F32 or BF16 values, decoded
 // where they are used (the reference decodes them into F32 buffers with launches of their own,
 // src/backend/cuda/moe.c:1226-1240; the decoded value is the same float).
@@ -66,9 +81,7 @@ __device__ __forceinline__ float coefficient(const void *values, unsigned qtype,
 __device__ __forceinline__ float4 coefficient4(const void *values, unsigned qtype, unsigned quad)
 {
     if (qtype == QT_F32) return static_cast<const float4 *>(values)[quad];
-    const uint2 v = static_cast<const uint2 *>(values)[quad];
-    return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u),
-                       __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
+    return bf16_unpack4(static_cast<const uint2 *>(values)[quad]);
 }
 
 // Alternating row and column normalisations of a 4 x 4 matrix, one element a lane (4 row + column,
@@ -102,9 +115,11 @@ __device__ __forceinline__ float sinkhorn4(float m, unsigned iterations, double 
 // scalar loops.
 // SPLIT, where a batch leaves every row two compute units: a second workgroup forms the mean square as well and then the
 // mixing matrix, whose chain of divisions so runs beside the second pass and not ahead of the sum that ends it, and the
-// row's values stay in registers for the second pass. A one-row launch of four streams of 4096 values is 2.6 us of
-// getting there and back and then waits of one workgroup for itself: 11.9 -> 9.0 us, 96 rows 13.5 -> 11.2. In a batch
-// of more rows two workgroups share a compute unit, which those registers would not let them (333 rows 23 and 28 us).
+// first pass leaves the rounded values in LDS for the second (`held`: unless the row is too long). Which thread adds which
+// squares is the same either way, so a row's results do not depend on its batch. Four streams of 4096 values, where a
+// one-row launch is 2.6 us of getting there and back and then waits of one workgroup for itself, by 1 / 96 / 128 rows
+// 9.6 / 11.0 / 11.4 -> 7.7 / 9.8 / 10.4 us, of 7168 values 13.7 / 15.4 / 16.0 -> 10.7 / 13.7 / 15.2. Where two workgroups
+// have to share a compute unit the second pass over the row costs what it gave: 160 rows 11.8 and 14.7, 16.6 and 24.4.
 template <unsigned THREADS, bool SPLIT>
 __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
     const float *__restrict__ rows, const float *__restrict__ mixes, const void *__restrict__ scale_values,
@@ -112,15 +127,14 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
     unsigned base_qtype, unsigned norm_qtype, unsigned streams, unsigned width,
     unsigned iterations, double rms_epsilon, double mhc_epsilon, double post_multiplier,
     float *__restrict__ normalized, float *__restrict__ post, float *__restrict__ combination,
-    int quads, int *status)
+    int quads, int held, int *status)
 {
     __shared__ float base[64], scale[3];      // (streams + 2) * streams <= 63 mixing rows
-    extern __shared__ __align__(16) float collapsed[];   // width values
+    extern __shared__ __align__(16) float collapsed[];   // width values; behind them, where held, the row as bf16
     __shared__ double slots[THREADS / 64u];
     __shared__ double gate[8];
-    constexpr unsigned kBatch = 4, kHeld = SPLIT ? 2 : 0;    // (two workgroups share a compute unit on fewer registers)
-    constexpr unsigned kSpared = SPLIT ? 0u : 64u;           // the second pass leaves the first wavefront out
-    constexpr unsigned kWorkers = THREADS - kSpared;
+    constexpr unsigned kBatch = 4, kAhead = SPLIT ? 8 : 4;   // (two workgroups share a compute unit on fewer registers)
+    constexpr unsigned kWorkers = THREADS - 64u;             // the second pass leaves the first wavefront out
     const unsigned tid = threadIdx.x;
     const unsigned long long row = SPLIT ? blockIdx.x >> 1 : blockIdx.x;
     const bool mixes_only = SPLIT && (blockIdx.x & 1u) != 0u, mixes_here = !SPLIT || mixes_only;
@@ -131,47 +145,27 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
 
     // mean square of the bf16-rounded residual (a value that is not finite makes the sum not finite)
     double squares = 0.0;
-    const bool held = kHeld != 0u && quads && streams <= kBatch && width <= kHeld * 4u * kWorkers;   // a worker's columns stay in registers
-    float4 mine[kHeld ? kHeld : 1u][kBatch];
-    if (held) {
-        const float4 *in4 = reinterpret_cast<const float4 *>(in);
-        const unsigned count = width >> 2;
-#pragma unroll
-        for (unsigned u = 0; u < kHeld; ++u) {
-            const unsigned at = tid - kSpared + u * kWorkers;          // (behind the row's end where tid < kSpared)
-#pragma unroll
-            for (unsigned s = 0; s < kBatch; ++s)
-                mine[u][s] = at < count && s < streams ? in4[s * count + at] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
-#pragma unroll
-        for (unsigned u = 0; u < kHeld; ++u) {
-            if (u != 0u && u * kWorkers >= count) break;
-#pragma unroll
-            for (unsigned s = 0; s < kBatch; ++s) {
-                const float4 r = mine[u][s] = bf16_round4(mine[u][s]);
-                squares += (double)r.x * (double)r.x;
-                squares += (double)r.y * (double)r.y;
-                squares += (double)r.z * (double)r.z;
-                squares += (double)r.w * (double)r.w;
-            }
-        }
-    } else if (quads) {
+    uint2 *const row_held = reinterpret_cast<uint2 *>(collapsed + width);
+    const bool hold = SPLIT && held != 0 && !mixes_only;
+    if (quads) {
         const float4 *in4 = reinterpret_cast<const float4 *>(in);
         const unsigned count = expanded >> 2;
-        for (unsigned first = tid; first < count; first += THREADS * kBatch) {
-            float4 v[kBatch];
+        for (unsigned first = tid; first < count; first += THREADS * kAhead) {
+            float4 v[kAhead];
 #pragma unroll
-            for (unsigned u = 0; u < kBatch; ++u) {
+            for (unsigned u = 0; u < kAhead; ++u) {
                 const unsigned at = first + u * THREADS;
                 v[u] = at < count ? in4[at] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             }
 #pragma unroll
-            for (unsigned u = 0; u < kBatch; ++u) {
+            for (unsigned u = 0; u < kAhead; ++u) {
+                if (SPLIT && first - tid + u * THREADS >= count) break;
                 const float4 r = bf16_round4(v[u]);
                 squares += (double)r.x * (double)r.x;
                 squares += (double)r.y * (double)r.y;
                 squares += (double)r.z * (double)r.z;
                 squares += (double)r.w * (double)r.w;
+                if (hold && first + u * THREADS < count) row_held[first + u * THREADS] = bf16_pack4(r);
             }
         }
     } else {
@@ -246,20 +240,31 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
 
     // collapsed row: float accumulation over the streams in order, then bf16
     double collapsed_squares = 0.0;
-    if (tid < kSpared) {
+    if (tid < 64u) {
         // busy with the mixing matrix above
     } else if (quads && streams <= kBatch) {
         const float4 *in4 = reinterpret_cast<const float4 *>(in);
         const unsigned count = width >> 2;
-        auto collapse = [&](unsigned at, const float4 (&rounded)[kBatch]) {
+        for (unsigned at = tid - 64u; at < count; at += kWorkers) {
+            float4 v[kBatch];
+            if (hold) {
+#pragma unroll
+                for (unsigned s = 0; s < kBatch; ++s) v[s] = bf16_unpack4(row_held[s < streams ? s * count + at : at]);
+            } else {
+#pragma unroll
+                for (unsigned s = 0; s < kBatch; ++s)
+                    v[s] = s < streams ? in4[s * count + at] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+                for (unsigned s = 0; s < kBatch; ++s) v[s] = bf16_round4(v[s]);
+            }
             float4 total = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
             for (unsigned s = 0; s < kBatch; ++s) {
                 if (s < streams) {
-                    total.x += (float)(gate[s] * (double)rounded[s].x);
-                    total.y += (float)(gate[s] * (double)rounded[s].y);
-                    total.z += (float)(gate[s] * (double)rounded[s].z);
-                    total.w += (float)(gate[s] * (double)rounded[s].w);
+                    total.x += (float)(gate[s] * (double)v[s].x);
+                    total.y += (float)(gate[s] * (double)v[s].y);
+                    total.z += (float)(gate[s] * (double)v[s].z);
+                    total.w += (float)(gate[s] * (double)v[s].w);
                 }
             }
             bad |= !finite_f32(total.x) || !finite_f32(total.y) || !finite_f32(total.z) || !finite_f32(total.w);
@@ -269,24 +274,9 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
             collapsed_squares += (double)published.y * (double)published.y;
             collapsed_squares += (double)published.z * (double)published.z;
             collapsed_squares += (double)published.w * (double)published.w;
-        };
-        if (held) {
-#pragma unroll
-            for (unsigned u = 0; u < kHeld; ++u)
-                if (tid - kSpared + u * kWorkers < count) collapse(tid - kSpared + u * kWorkers, mine[u]);
-        } else {
-            for (unsigned at = tid - kSpared; at < count; at += kWorkers) {
-                float4 v[kBatch];
-#pragma unroll
-                for (unsigned s = 0; s < kBatch; ++s)
-                    v[s] = s < streams ? in4[s * count + at] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll
-                for (unsigned s = 0; s < kBatch; ++s) v[s] = bf16_round4(v[s]);
-                collapse(at, v);
-            }
         }
     } else {
-        for (unsigned lane = tid - kSpared; lane < width; lane += kWorkers) {
+        for (unsigned lane = tid - 64u; lane < width; lane += kWorkers) {
             float total = 0.0f;
             for (unsigned s = 0; s < streams; ++s)
                 total += (float)(gate[s] * (double)bf16_round(in[s * width + lane]));
@@ -477,7 +467,7 @@ static int launch_mhc_ingress(const float *rows, const float *mixes, const void 
         for (const void *kernel : {(const void *)mhc_ingress_kernel<256, false>, (const void *)mhc_ingress_kernel<256, true>,
                                    (const void *)mhc_ingress_kernel<1024, false>, (const void *)mhc_ingress_kernel<1024, true>})
             prepared = prepared && hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       (int)(kEnvelopeMaxWidth * sizeof(float))) == hipSuccess;
+                                                       (int)kEnvelopeLdsBytes) == hipSuccess;
         if (!prepared) (void)hipGetLastError();
     });
     if (!prepared) {
@@ -486,13 +476,16 @@ static int launch_mhc_ingress(const float *rows, const float *mixes, const void 
     }
     const int quads = width % 4u == 0u && !(((uintptr_t)rows | (uintptr_t)normalized) & 15u) &&
                       !((uintptr_t)norm & (norm_qtype == QT_F32 ? 15u : 7u));
-    const unsigned lds = (unsigned)(width * sizeof(float));
     const bool split = 2u * row_count <= (uint64_t)compute_units(), wide = streams * width >= 8192u;
+    const unsigned collapsed_bytes = (unsigned)(width * sizeof(float)), row_bytes = (unsigned)(2u * streams * width);
+    const int held = split && quads && streams <= 4u && collapsed_bytes + row_bytes <= kEnvelopeLdsBytes;
+    const unsigned lds = collapsed_bytes + (held ? row_bytes : 0u);
     const auto kernel = wide ? (split ? mhc_ingress_kernel<1024, true> : mhc_ingress_kernel<1024, false>)
                              : (split ? mhc_ingress_kernel<256, true> : mhc_ingress_kernel<256, false>);
     kernel<<<(unsigned)(split ? 2u * row_count : row_count), wide ? 1024 : 256, lds, as_stream(stream)>>>(
         rows, mixes, scale, base, norm, scale_qtype, base_qtype, norm_qtype, (unsigned)streams, (unsigned)width,
-        (unsigned)iterations, rms_epsilon, mhc_epsilon, post_multiplier, normalized, post, combination, quads, status);
+        (unsigned)iterations, rms_epsilon, mhc_epsilon, post_multiplier, normalized, post, combination, quads, held,
+        status);
     return check_launch("mhc_ingress");
 }
 
