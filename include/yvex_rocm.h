@@ -357,7 +357,9 @@ typedef struct yvex_rocm_operation_facts {
 
 /* Replaces yvex_backend_cuda_encoded_matvec (include/yvex/internal/backend.h:332-337,
  * src/backend/cuda/qtype.c:220-405). output[in, row] = dot(encoded row, input row in)
- * (+ additive). activation_q8 = 1 quantizes the F32 input rows to Q8_K on device first.
+ * (+ additive). activation_q8 = 1 quantizes the F32 input rows to Q8_K on device first; the attached
+ * workspace must hold rows * width / 256 * 292 bytes for them (temporary_bytes counts these), also where
+ * the launch that multiplies keeps them to itself.
  * Refusals: activation_q8 not 0/1 -> INVALID_ARG; qtype unknown, removed, outside the baseline
  * or without device compute -> UNSUPPORTED (on the host, before any launch); geometry, byte
  * count, ownership, unwritten input, additive aliasing output, resident MISS -> FORMAT; kernels

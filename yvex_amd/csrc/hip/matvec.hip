@@ -1214,9 +1214,6 @@ extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint6
     }
 }
 
-// Two Q8_0 matrices of one shape against the same Q8_K input rows in one launch (a shared expert's gate
-// and up projections): each offers too few workgroups for the device on its own (2048 x 4096 against
-// 96 rows: 192 of them, 16 us a launch).
 // Whether F32 input rows are multiplied by the launch that quantizes them. Every workgroup quantizes all of them, a
 // block a wave at a time, so up to two rows, and as many blocks as the workgroup has waves or twice that while the rest of
 // the launch is short. Two launches and one, us: 4096 x 4096 by 1 and 2 rows 9.8 and 7.2, 12.2 and 9.0 (by 3 12.4 and
@@ -1260,6 +1257,9 @@ extern "C" int yvex_hip_matvec_quantizing(const uint8_t *encoded, unsigned int q
     return input_rows == 1u ? launch_quantizing<1>(a, as_stream(stream)) : launch_quantizing<2>(a, as_stream(stream));
 }
 
+// Two Q8_0 matrices of one shape against the same Q8_K input rows in one launch (a shared expert's gate
+// and up projections): each offers too few workgroups for the device on its own (2048 x 4096 against
+// 96 rows: 192 of them, 16 us a launch).
 extern "C" int yvex_hip_matvec_q8_0_pair(const uint8_t *first, const uint8_t *second, uint64_t row_count,
                                          uint64_t row_width, uint64_t row_bytes, const void *input_q8k,
                                          uint64_t input_rows, float *out_first, float *out_second,

@@ -94,6 +94,8 @@ int yvex_rocm_encoded_matvec(
     rc = yvex_rocm_require_kernels(backend, where, err);
     if (rc != YVEX_OK) return rc;
     yvex_rocm_workspace_reset(backend);
+    /* asked for and counted whichever launches follow, the one that quantizes for itself among them: what a call
+     * needs does not depend on its route */
     if (q8_path) {
         if (!mul_u64(input_rows * (row_width / 256ull), 292ull, &q8_bytes))
             return yvex_rocm_refuse(err, YVEX_ERR_BOUNDS, where, "Q8 activation workspace exceeds bounds");
