@@ -143,6 +143,15 @@ __device__ __forceinline__ unsigned wave_inclusive_sum_u32(unsigned v)
     return v;
 }
 
+// Between what a wave's lanes write to LDS for one another and their reads, and the other way round (a wave's LDS operations
+// complete in order: this keeps the compiler to it).
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // A double moved by a data-parallel-primitive step (both halves).
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v)

@@ -44,7 +44,6 @@ constexpr unsigned kIq2LdsBytes = kWindowBase + kIq2Waves * kIq2Window;
 __global__ __launch_bounds__(kIq2Threads) void dense_iq2_kernel(DenseIq2Args g)
 {
     typedef int v4s __attribute__((ext_vector_type(4)));
-    typedef v4i v4i_dword __attribute__((aligned(4)));
     extern __shared__ __align__(16) unsigned char dense_iq2_lds[];
     if (lds_address_of(dense_iq2_lds) != 0u) {   // operands are addressed by absolute LDS offsets
         if (threadIdx.x == 0u) raise_status(g.status, 2);
@@ -57,31 +56,21 @@ __global__ __launch_bounds__(kIq2Threads) void dense_iq2_kernel(DenseIq2Args g)
     const unsigned toks_here = (unsigned)(g.input_rows - tok0 < 16ull ? g.input_rows - tok0 : 16ull);
     const unsigned long long act_row_bytes = (unsigned long long)g.blocks * kQ8KBytes;
     const unsigned char *const weights = g.encoded + row0 * g.row_bytes, *const acts = g.act + tok0 * act_row_bytes;
-    // dwords 64 k + lane of 16 rows x 17, pieces 64 k + lane of 16 rows x 16 (a ragged edge repeats the last row)
-    const unsigned char *weight_at[5], *act_at[4];
+    // dwords 64 k + lane of 16 rows x 17 (a ragged edge repeats the last row)
+    const unsigned char *weight_at[5];
 #pragma unroll
     for (unsigned k = 0; k < 5u; ++k) {
         const unsigned piece = k < 4u ? 64u * k + lane : 256u + r, row = piece / kRowDwords;
         weight_at[k] = weights + (row < rows_here ? row : rows_here - 1u) * g.row_bytes + 4u * (piece - kRowDwords * row);
     }
-#pragma unroll
-    for (unsigned k = 0; k < 4u; ++k) {
-        const unsigned row = 4u * k + q;
-        act_at[k] = acts + (row < toks_here ? row : toks_here - 1u) * act_row_bytes + 4u + 16u * r;
-    }
-    const unsigned char *const scale_from = acts + (r < toks_here ? r : toks_here - 1u) * act_row_bytes;
-    struct {
-        unsigned weights[5], scale;
-        v4i acts[4];
-    } ahead;
+    InputRows16 inputs(acts, act_row_bytes, toks_here, lane);
+    unsigned ahead[5];
     auto request = [&](unsigned sb) {
         // (rows are whole dwords and an even number of superblocks: the aligned dwords around the last one end with the row)
-        const unsigned long long w = (sb * 66ull) & ~3ull, a = (unsigned long long)sb * kQ8KBytes;
+        const unsigned long long w = (sb * 66ull) & ~3ull;
 #pragma unroll
-        for (unsigned k = 0; k < 5u; ++k) ahead.weights[k] = *reinterpret_cast<const unsigned *>(weight_at[k] + w);
-#pragma unroll
-        for (unsigned k = 0; k < 4u; ++k) ahead.acts[k] = *reinterpret_cast<const v4i_dword *>(act_at[k] + a);
-        ahead.scale = *reinterpret_cast<const unsigned *>(scale_from + a);
+        for (unsigned k = 0; k < 5u; ++k) ahead[k] = *reinterpret_cast<const unsigned *>(weight_at[k] + w);
+        inputs.request(sb);
     };
     if (wave < g.blocks) request(wave);
     // the tables, while the first superblock is on its way
@@ -104,16 +93,11 @@ __global__ __launch_bounds__(kIq2Threads) void dense_iq2_kernel(DenseIq2Args g)
     for (unsigned sb = wave; sb < g.blocks; sb += kIq2Waves) {
         // (LDS operations of one wave complete in order)
 #pragma unroll
-        for (unsigned k = 0; k < 4u; ++k) {
-            lds_write_u32(window + 256u * k + 4u * lane, ahead.weights[k]);
-            lds_write_v4i(window + kIq2Act + (4u * k + q) * kIq2ActPitch + 16u * r, ahead.acts[k]);
-        }
-        lds_write_u32(window + 1024u + 4u * r, ahead.weights[4]);
-        lds_write_u32(window + kIq2Scales + 4u * r, ahead.scale);
+        for (unsigned k = 0; k < 4u; ++k) lds_write_u32(window + 256u * k + 4u * lane, ahead[k]);
+        lds_write_u32(window + 1024u + 4u * r, ahead[4]);
+        inputs.write(window + kIq2Act, kIq2ActPitch, window + kIq2Scales, lane);
         request(sb + kIq2Waves < g.blocks ? sb + kIq2Waves : sb);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
         // an even superblock starts on a dword (its records two bytes behind), an odd one two bytes behind one
         const unsigned shift = sb & 1u ? 0u : 2u, first = sb & 1u ? 1u : 0u;
         const unsigned head = lds_read_u32(w_row);
@@ -140,9 +124,7 @@ __global__ __launch_bounds__(kIq2Threads) void dense_iq2_kernel(DenseIq2Args g)
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[i] += (double)(d * d_a[i] * (float)total[i]);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
     }
     __syncthreads();
     double *const partial = reinterpret_cast<double *>(dense_iq2_lds);

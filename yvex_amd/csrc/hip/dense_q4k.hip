@@ -210,9 +210,7 @@ __global__ __launch_bounds__(256) void dense_q4k_kernel(DenseQ4kArgs g)
             min_hi[nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(m_op, b_hi, zero, 0, 0, 0);
         }
         // d and dmin of the sixteen rows this lane accumulates (written above by the wave itself)
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
         float d_of[16], dmin_of[16];
 #pragma unroll
         for (unsigned q4 = 0; q4 < 4u; ++q4) {
@@ -344,9 +342,7 @@ __global__ __launch_bounds__(64 * WAVES) void dense_q4k16_kernel(DenseQ4kArgs g)
         for (unsigned k = 0; k < kActLoads; ++k) *reinterpret_cast<v4i *>(act_to[k]) = ahead.acts[k];
         *reinterpret_cast<unsigned *>(scale_to) = ahead.scale;
         request(sb + WAVES < g.blocks ? sb + WAVES : sb);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
         const unsigned char *const w = window + 144u * r;
         const uint4 opening = *reinterpret_cast<const uint4 *>(w);
         const unsigned head = opening.x;
@@ -404,9 +400,7 @@ __global__ __launch_bounds__(64 * WAVES) void dense_q4k16_kernel(DenseQ4kArgs g)
         const v4s zero = {0, 0, 0, 0};
         min_lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(m_op, b_lo, zero, 0, 0, 0);
         min_hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(m_op, b_hi, zero, 0, 0, 0);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
         const float4 d4 = *reinterpret_cast<const float4 *>(&row_scale[wave][0][4u * q]);
         const float4 m4 = *reinterpret_cast<const float4 *>(&row_scale[wave][1][4u * q]);
         const float d_of[4] = {d4.x, d4.y, d4.z, d4.w}, dmin_of[4] = {m4.x, m4.y, m4.z, m4.w};

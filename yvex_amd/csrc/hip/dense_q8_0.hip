@@ -236,14 +236,10 @@ __global__ __launch_bounds__(64 * kPlainWaves) void dense_q8_0_kernel(DenseQ80Ar
         lds_write_u32(window + kPlainScales + 4u * r, ahead.scale);
         // the next superblock's bytes travel while this one is worked on
         request(sb + kPlainWaves < g.blocks ? sb + kPlainWaves : sb);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
         q80_superblock(window + r * kStagedPitch, window + kPlainAct + r * kStagedPitch + 16u * h, window + kPlainScales + 16u * h, h,
                        scale, acc);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
     }
 
     // (the partial tiles of waves 1 to 3 take the windows' place)
@@ -301,30 +297,20 @@ __global__ __launch_bounds__(64 * kSmallWaves) void dense_q8_0_small_kernel(Dens
     const unsigned toks_here = (unsigned)(g.input_rows - tok0 < 16ull ? g.input_rows - tok0 : 16ull);
     const unsigned long long act_row_bytes = (unsigned long long)g.blocks * kQ8KBytes;
     const unsigned char *const weights = g.encoded + row0 * g.row_bytes, *const acts = g.act + tok0 * act_row_bytes;
-    // pieces 64 k + lane of 16 rows x 17 and of 16 rows x 16 (a ragged edge repeats the last row)
-    const unsigned char *weight_at[5], *act_at[4];
+    // pieces 64 k + lane of 16 rows x 17 (a ragged edge repeats the last row)
+    const unsigned char *weight_at[5];
 #pragma unroll
     for (unsigned k = 0; k < 5u; ++k) {
         const unsigned piece = k < 4u ? 64u * k + lane : 256u + r, row = piece / 17u;
         weight_at[k] = weights + (row < rows_here ? row : rows_here - 1u) * g.row_bytes + 16u * (piece - 17u * row);
     }
-#pragma unroll
-    for (unsigned k = 0; k < 4u; ++k) {
-        const unsigned row = 4u * k + q;
-        act_at[k] = acts + (row < toks_here ? row : toks_here - 1u) * act_row_bytes + 4u + 16u * r;
-    }
-    const unsigned char *const scale_from = acts + (r < toks_here ? r : toks_here - 1u) * act_row_bytes;
-    struct {
-        v4i weights[5], acts[4];
-        unsigned scale;
-    } ahead;
+    InputRows16 inputs(acts, act_row_bytes, toks_here, lane);
+    v4i ahead[5];
     auto request = [&](unsigned sb) {
-        const unsigned long long w = sb * 272ull, a = (unsigned long long)sb * kQ8KBytes;
+        const unsigned long long w = sb * 272ull;
 #pragma unroll
-        for (unsigned k = 0; k < 5u; ++k) ahead.weights[k] = *reinterpret_cast<const v4i_dword *>(weight_at[k] + w);
-#pragma unroll
-        for (unsigned k = 0; k < 4u; ++k) ahead.acts[k] = *reinterpret_cast<const v4i_dword *>(act_at[k] + a);
-        ahead.scale = *reinterpret_cast<const unsigned *>(scale_from + a);
+        for (unsigned k = 0; k < 5u; ++k) ahead[k] = *reinterpret_cast<const v4i_dword *>(weight_at[k] + w);
+        inputs.request(sb);
     };
     const unsigned window = kSmallWindow * wave;
     const unsigned w_row = window + r * kStagedPitch, a_row = window + kSmallAct + r * kStagedPitch + 8u * q;
@@ -333,16 +319,11 @@ __global__ __launch_bounds__(64 * kSmallWaves) void dense_q8_0_small_kernel(Dens
     for (unsigned sb = wave; sb < g.blocks; sb += kSmallWaves) {
         // (LDS operations of one wave complete in order)
 #pragma unroll
-        for (unsigned k = 0; k < 4u; ++k) {
-            lds_write_v4i(window + 1024u * k + 16u * lane, ahead.weights[k]);
-            lds_write_v4i(window + kSmallAct + (4u * k + q) * kStagedPitch + 16u * r, ahead.acts[k]);
-        }
-        lds_write_v4i(window + 4096u + 16u * r, ahead.weights[4]);
-        lds_write_u32(window + kSmallScales + 4u * r, ahead.scale);
+        for (unsigned k = 0; k < 4u; ++k) lds_write_v4i(window + 1024u * k + 16u * lane, ahead[k]);
+        lds_write_v4i(window + 4096u + 16u * r, ahead[4]);
+        inputs.write(window + kSmallAct, kStagedPitch, window + kSmallScales, lane);
         request(sb + kSmallWaves < g.blocks ? sb + kSmallWaves : sb);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
         const uint4 d4 = read16(window + kSmallScales + 16u * q);
         const float d_a[4] = {__uint_as_float(d4.x), __uint_as_float(d4.y), __uint_as_float(d4.z), __uint_as_float(d4.w)};
         float total[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -365,9 +346,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void dense_q8_0_small_kernel(Dens
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[i] += (double)total[i];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
     }
     __syncthreads();
     double *const partial = reinterpret_cast<double *>(dense_q8_0_small_lds);

@@ -85,6 +85,39 @@ __device__ __forceinline__ unsigned lds_read_u32(unsigned address)
 #endif
 }
 
+// A superblock of sixteen input rows (Q8_K) on its way into a wave's window of LDS: the lanes load consecutive 16-byte pieces
+// of consecutive rows into registers and write them behind the superblock that is being worked on, codes `pitch` bytes a
+// row, the sixteen scales at `scales`. Rows from `count` on repeat the last one.
+struct InputRows16 {
+    const unsigned char *codes_at[4], *scale_at;
+    v4i codes[4];
+    unsigned scale;
+    __device__ __forceinline__ InputRows16(const unsigned char *rows, unsigned long long row_bytes, unsigned count, unsigned lane)
+    {
+        const unsigned r = lane & 15u;
+#pragma unroll
+        for (unsigned k = 0; k < 4u; ++k) {
+            const unsigned row = 4u * k + (lane >> 4);
+            codes_at[k] = rows + (row < count ? row : count - 1u) * row_bytes + 4u + 16u * r;
+        }
+        scale_at = rows + (r < count ? r : count - 1u) * row_bytes;
+    }
+    __device__ __forceinline__ void request(unsigned superblock)
+    {
+        typedef v4i v4i_dword __attribute__((aligned(4)));
+        const unsigned long long at = (unsigned long long)superblock * kQ8KBytes;
+#pragma unroll
+        for (unsigned k = 0; k < 4u; ++k) codes[k] = *reinterpret_cast<const v4i_dword *>(codes_at[k] + at);
+        scale = *reinterpret_cast<const unsigned *>(scale_at + at);
+    }
+    __device__ __forceinline__ void write(unsigned window, unsigned pitch, unsigned scales, unsigned lane) const
+    {
+#pragma unroll
+        for (unsigned k = 0; k < 4u; ++k) lds_write_v4i(window + (4u * k + (lane >> 4)) * pitch + 16u * (lane & 15u), codes[k]);
+        lds_write_u32(scales + 4u * (lane & 15u), scale);
+    }
+};
+
 // The copies below write m0. The compiler reserves m0 and reloads it before every use of its
 // own, but it may merge two of its own loads of the same value across code that sits between
 // them; naming m0 as written by the assembly keeps it from doing that across a copy. It answers

@@ -555,9 +555,7 @@ __device__ __forceinline__ void grouped_sweep(
 #pragma unroll
                     for (int p = 0; p < N; ++p)
                         terms[(w * N + p) * 64 + lane] = row_live[r] ? sums[r][w][p] : 0.0f;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                wave_lds_fence();
                 if (row_live[r] && g.seg == 0u) {
 #pragma unroll
                     for (int w = 0; w < kStreams; ++w)
@@ -569,9 +567,7 @@ __device__ __forceinline__ void grouped_sweep(
                             sums[r][w][p] = (float)sum;
                         }
                 }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                wave_lds_fence();
             } else {
                 // F32 activations: the lanes' double sums added in double, rounded once
                 // (the CPU row dot: src/gguf/quant_compute.c:152-172)

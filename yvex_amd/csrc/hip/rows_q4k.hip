@@ -277,9 +277,7 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
             }
         }
         // d and dmin of the sixteen rows this lane accumulates (written above by the wave itself)
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
 #pragma unroll
         for (unsigned nt = 0; nt < NT; ++nt) {
             const unsigned token = nt * 32u + r;

@@ -641,9 +641,7 @@ __device__ __forceinline__ unsigned iq2_sweep(const GroupedArgs &a, const Groupe
     const unsigned R = g.rows_per_iter;
     auto flush = [&](unsigned first_iteration, unsigned count, unsigned chunk_begin) {
         // LDS operations of one wave complete in order, so the terms parked above are visible here
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
         const unsigned sums = (count * (unsigned)PV * 2u) << g.row_shift;
         const unsigned segment_bytes = 128u >> g.row_shift;       // a row's terms of one parity
         for (unsigned s = lane; s < sums; s += 64u) {
@@ -682,9 +680,7 @@ __device__ __forceinline__ unsigned iq2_sweep(const GroupedArgs &a, const Groupe
                 }
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
     };
     // iterations a window holds (a multiple of the turns of one trip through the loop below)
     constexpr unsigned kWindowIters = (kWindowLines / (unsigned)PV) / (AHEAD + 1) * (AHEAD + 1);
@@ -808,9 +804,7 @@ __device__ __forceinline__ unsigned iq2_sweep(const GroupedArgs &a, const Groupe
             if (!finite_f32(value)) raise_status(a.status, 1);
             else pr.out[oi * a.out_rows + chunk_row + local] = value;
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
     }
     if (next >= chunks) return drawn;
     begin = next * chunk_turns;
