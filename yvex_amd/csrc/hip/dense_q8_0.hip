@@ -577,17 +577,19 @@ constexpr unsigned kWideActBase = 2u * kWideWeightBytes, kWideScaleBase = kWideA
 constexpr unsigned kWideLdsBytes = kWideScaleBase + 2u * kWideTokens * 4u;
 
 // The same product for batches that fill the device with tiles of 128 weight rows x 128 input rows.
-// Bound by vector-instruction issue: behind one matrix instruction (32 cycles) sixteen results a lane
-// are brought to float, multiplied by their scale and chained. What this kernel does about it:
+// Behind one matrix instruction (32 cycles) sixteen results a lane are brought to float, multiplied by their scale and
+// chained: the vector ALU has most of the work, and no wave may be alone with its waits. What this kernel does about it:
 //  * kStartBits above in place of the conversions.
 //  * A wave owns 32 weight rows x 32 input rows on 128 registers, so that sixteen of them, four a SIMD, cover each
 //    other's waits and the rate of one wave's instructions (one in 5.5 cycles on this part; two waves issue 4-cycle
 //    instructions in 5.0 cycles each, four in 4.4).
 //  * Copies take a scalar base and a 32-bit offset a lane: a register and no addition each.
-// 4096 x 4096 by 2048 rows 136 -> 129 us (528 TOP/s; eight waves of 32 x 64, two a SIMD, before). Counters of the old one: vector
-// ALU 60 instructions a wave and block at 3 cycles, half the time; of the new one 2.4 cycles each, and the LDS, which serves
-// twice the weight reads, 40 % busy, is the other half. The products of the scales as one V_MFMA_F32_32X32X2_F32 a block (the
-// same bits): 137 us, it does not run beside vector instructions. Whole 16-byte reads of a window's end: 131 us.
+// 4096 x 4096 by 2048 rows 136 -> 129 us (532 TOP/s; eight waves of 32 x 64, two a SIMD, before). No pipe is full: the
+// vector ALU is issued to 66 % of the time, the LDS is busy 40 %, nearly half of it bank conflicts (at a pitch of 272 bytes
+// rows r and r + 16 start on one bank, which the reads of less than 16 bytes meet on), the matrix cores 12 %; a wave waits for
+// data 42 % of its time, copies behind a full wait and a barrier a superblock. The products of the scales as one
+// V_MFMA_F32_32X32X2_F32 a block (the same bits): 137 us, it does not run beside vector instructions. Whole 16-byte reads of a
+// window's end: 131 us.
 __global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80Args g)
 {
     extern __shared__ __align__(16) unsigned char dense_q8_0_lds[];

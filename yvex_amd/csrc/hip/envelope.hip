@@ -377,8 +377,10 @@ __global__ __launch_bounds__(kEnvelopeThreads) void mhc_egress_kernel(
 // the same order): the combined row never goes to memory, and a decode batch has a launch less.
 // A thread has one column: a few hundred instructions follow its loads, most of them double-precision, and a wave
 // issues one in five cycles at best, so four columns a thread kept the few waves of a decode batch busy for longer than the
-// memory took, and 87 registers kept a larger batch to five waves a SIMD. 4096 columns, six ranks, by 1 / 96 / 333 rows
-// 8.4 / 12.7 / 27.5 us with four columns, 5.8 / 11.0 / 23.8 with two, 4.4 / 9.0 / 23.5 with one.
+// memory took, and 87 registers kept a larger batch to five waves a SIMD. 4096 columns, six ranks, by 1 / 96 / 333 / 700 /
+// 1111 / 2048 rows 7.5 / 13.8 / 30.7 / 50.6 / 70.7 / 114.5 us with four columns, 3.8 / 10.2 / 25.2 / 47.2 / 69.9 / 117.1 with one;
+// eight ranks of 7168 columns by 2048 rows 209 and 213. The 2 % that 16-byte loads are ahead by at 2048 rows are not worth a
+// second kernel.
 template <unsigned STREAMS>
 __global__ __launch_bounds__(kEnvelopeThreads) void combine_egress_kernel(
     const float *__restrict__ pair_outputs, unsigned topk, const float *__restrict__ shared,
