@@ -723,7 +723,7 @@ def main() -> int:
     harness_ms, harness_mode = step_ms, launch_mode
     # The step a caller of include/yvex_rocm.h gets: execute_rows on the backend's own stream
     # (router projection included), completion deferred to one complete_rows per phase. Its
-    # launch graph is built by the library. This is the headline; the stage harness above only
+    # launch graph, if it takes one, is built by the library. This is the headline; the stage harness above only
     # serves the per-kernel timings.
     stage_rows = layer.run(x, logits).clone()
     torch.cuda.synchronize()
@@ -742,9 +742,9 @@ def main() -> int:
               f"vs {unique}, identical rows {abi_same})", file=sys.stderr)
         return 1
     step_ms = min(abi_graph_ms, abi_eager_ms)
-    launch_mode = ("execute_rows, library launch graph, completion deferred to the phase barrier"
-                   if abi_graph_ms <= abi_eager_ms else
-                   "execute_rows, eager launches, completion deferred to the phase barrier")
+    graph_mode = "library launch graph" if graph_facts[0] else "eager launches"
+    launch_mode = (f"execute_rows, {graph_mode if abi_graph_ms <= abi_eager_ms else 'eager launches'}, "
+                   "completion deferred to the phase barrier")
     # The same step with the experts resident as the decode sweeps' image: a caller's residency
     # step plans it (derived_layout_plan, 72 bytes a superblock instead of 66) and builds it on the
     # device from the canonical bytes; execute_rows takes DERIVED_BACKEND views of it. The rows
@@ -783,7 +783,7 @@ def main() -> int:
         if min(image_graph_ms, image_eager_ms) < step_ms:
             step_ms = min(image_graph_ms, image_eager_ms)
             launch_mode = ("execute_rows over the sweep image, " +
-                           ("library launch graph" if image_graph_ms <= image_eager_ms else "eager launches") +
+                           (graph_mode if image_graph_ms <= image_eager_ms else "eager launches") +
                            ", completion deferred to the phase barrier")
             sweeps_ms = image_sweeps_ms
     weight_bytes = (unique + 1) * EXPERT_BYTES

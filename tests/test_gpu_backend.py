@@ -1090,6 +1090,23 @@ def test_execute_rows_graph_key_follows_addresses(backend, oracle):
     assert not np.array_equal(first, got)
 
 
+# 6 488 064 bytes an expert, the shared one included: 30.9 and 37.1 MiB about the line of 32
+@pytest.mark.parametrize("topk,replays", [(4, 1), (5, 0)])
+def test_execute_rows_launches_large_layers_one_by_one(backend, oracle, topk, replays):
+    b = backend
+    case = MoeCase(b, oracle, rows=1, hidden=4096, intermediate=2048, experts=topk, topk=topk)
+    b.workspace(case.workspace_bytes)
+    rows = []
+    for _ in range(4):
+        assert case.execute() == 0, case.err.message
+        rows.append(b.read_f32(case.rows_out, case.hidden).copy())
+    assert (case.result.graph_launches, case.result.graph_replays) == (replays, replays)
+    case.job.eager_execution = 1
+    assert case.execute() == 0 and case.result.graph_launches == 0
+    rows.append(b.read_f32(case.rows_out, case.hidden))
+    assert all(np.array_equal(r.view(np.uint32), rows[0].view(np.uint32)) for r in rows)
+
+
 # ---- token-local operation: src/backend/cuda/moe.c:516-842 --------------------------------------
 
 class TokenLocal:

@@ -386,8 +386,16 @@ static unsigned long long matrix_core_pairs(const yvex_hip_expert_weights *route
  * execution (moe.c:1650-1681). Here a key seen for the first time runs eagerly, the second time
  * it is captured and launched, and from then on it is replayed; sixteen keys are kept, the least
  * recently used one making room. Everything a kernel argument is computed from is in the key,
- * so a replay submits exactly the launches the eager sequence would. */
+ * so a replay submits exactly the launches the eager sequence would.
+ *
+ * A replay keeps the stream 4.5 to 6 us longer than the same launches made one by one (its first and last packets
+ * wait for and signal the whole queue) and takes the host as long: 20 us a layer, 20 to 40 us for the six to twelve
+ * launches. Three layers, us, replayed and launched: one row of 4096 x 2048 by six experts in the model file's formats
+ * 218 and 203, five rows of 7168 x 2048 by eight 456 and 442, 96 rows 1537 and 1525; one row of 4096 x 2048 by two
+ * experts 140 and 125, where the host was busy with the launches for 70 to 105 us of them. So a graph is for layers so
+ * small that a slow host would keep the device waiting: those whose row needs less than 32 MB of weights. */
 enum { GRAPH_SLOTS = 16, GRAPH_KEY_WORDS = 176 };
+static const unsigned long long graph_weight_bytes = 32ull << 20;
 
 typedef struct {
     unsigned long long words[GRAPH_KEY_WORDS];
@@ -408,6 +416,14 @@ struct yvex_rocm_moe_graphs {
     unsigned long long clock;
     int refused;                       /* a capture failed: this backend stays eager */
 };
+
+/* What one row reads of the experts. */
+static unsigned long long row_weight_bytes(const yvex_hip_expert_weights *routed, unsigned long long topk,
+                                           const yvex_hip_expert_weights *shared)
+{
+    const unsigned long long bytes = topk * (routed->gate_expert_bytes + routed->up_expert_bytes + routed->down_expert_bytes);
+    return shared ? bytes + shared->gate_expert_bytes + shared->up_expert_bytes + shared->down_expert_bytes : bytes;
+}
 
 static void key_word(graph_key *key, unsigned long long value)
 {
@@ -764,7 +780,8 @@ static int moe_execute_rows(yvex_rocm_backend *backend, const yvex_moe_layer_job
         rc = yvex_rocm_status_reset(backend, &status_launches, "rocm.moe.rows.status", err);
         if (rc != YVEX_OK) return rc;
     }
-    if (!job->eager_execution && !(backend->moe_graphs && backend->moe_graphs->refused)) {
+    if (!job->eager_execution && row_weight_bytes(&routed, topk, has_shared ? &shared : NULL) < graph_weight_bytes &&
+        !(backend->moe_graphs && backend->moe_graphs->refused)) {
         graph_key key;
         unsigned long long slot_address[YVEX_MOE_WEIGHT_COUNT] = {0};
         int k;
