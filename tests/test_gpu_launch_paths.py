@@ -57,6 +57,49 @@ def same_bits(a, b):
     return torch.equal(a.contiguous().view(torch.int32), b.contiguous().view(torch.int32))
 
 
+# every kernel whose launch ends the operation by itself: the product that quantizes, the Q8_0 and IQ2_XXS 16 x 16 tiles, the
+# Q4_K ones on eight and on four waves, a row and a few of superblock formats, the 256 x 32 tiles of an output head; one
+# workgroup, fewer than counters, ragged numbers of them. `launches`: 1 where that is all, 2 with the quantizer's
+@pytest.mark.parametrize("qtype,weight_rows,width,inputs,launches", [
+    ("Q8_0", 1, 256, 1, 1), ("Q8_0", 4099, 512, 2, 1), ("Q8_0", 4096, 2304, 3, 2), ("Q8_0", 37, 256, 17, 2), ("Q8_0", 65281, 256, 3, 2),
+    ("Q4_K", 250, 512, 19, 2), ("Q4_K", 8200, 256, 33, 3), ("Q4_K", 8200, 256, 31, 2), ("Q4_K", 9, 768, 1, 2), ("Q4_K", 1030, 512, 3, 2),
+    ("IQ2_XXS", 52, 1024, 9, 2), ("IQ2_XXS", 300, 512, 1, 2), ("IQ2_XXS", 301, 1024, 4, 2), ("Q2_K", 70, 512, 2, 2)])
+def test_projections_that_publish_for_themselves(gpu, oracle, qtype, weight_rows, width, inputs, launches):
+    from backend_helpers import Backend
+    from yvex_amd import abi, kernels as K
+    qt, g, b = getattr(oracle, qtype), oracle.Generator(17, "publishing"), Backend()
+    encoded = g.weights(qt, weight_rows, width)
+    at = 80 if qtype == "Q2_K" else 0
+    encoded[at:at + 2] = (0x53, 0x7b)           # a block scale of 60 000: rows of 3e38 overflow, in the product
+    x = g.normal(inputs * width).reshape(inputs, width)
+    try:
+        _, base = b.resident(encoded)
+        b.workspace(inputs * (width // 256) * 292 + 4096)
+        out, facts, err = b.empty_f32(inputs * weight_rows), abi.OperationFacts(), abi.Error()
+        good, huge = b.f32(x), b.f32(np.full_like(x, 3e38))
+
+        def run(rows_in):
+            return b.lib.yvex_rocm_encoded_matvec(b.handle, base, encoded.nbytes, qt, weight_rows, width, encoded.nbytes // weight_rows,
+                                                  inputs, rows_in, None, 0, None, out, 1, C.byref(facts), C.byref(err))
+        st = K.new_status(gpu)
+
+        def product(rows_in):
+            return K.matvec(dev(encoded, gpu), qt, weight_rows, width, K.q8k_quantize(dev(rows_in, gpu), st), input_q8=True,
+                            input_rows=inputs, status=st).cpu().numpy()
+        want = product(x)
+        assert int(st.item()) == 0
+        for _ in range(2):
+            for _ in range(3):
+                assert run(good) == 0, err.message
+                assert facts.kernel_launches == launches
+                got = b.read_f32(out, inputs * weight_rows).reshape(inputs, weight_rows)
+                assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+            # what the product raises is this operation's, and the next one's word is clean
+            assert run(huge) == abi.FORMAT
+    finally:
+        b.close()
+
+
 # a full round of 128 x 128 tiles with ragged edges on both sides, one and three superblocks a row
 @pytest.mark.parametrize("rows,width,inputs", [(2047, 256, 2040), (1921, 768, 2048)])
 def test_q8_0_wide_tiles_are_the_oracles_bits(gpu, oracle, rows, width, inputs):

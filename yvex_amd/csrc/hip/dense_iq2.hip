@@ -16,6 +16,7 @@
 #include "common.hpp"
 #include "launch.hpp"
 #include "lds_copy.hpp"
+#include "publish.hpp"
 
 namespace yvex {
 
@@ -30,6 +31,7 @@ struct DenseIq2Args {
     float *out;
     int output_bf16;
     int *status;
+    Publication publication;
 };
 
 constexpr unsigned kIq2Waves = 8u, kIq2Threads = 64u * kIq2Waves;
@@ -47,6 +49,7 @@ __global__ __launch_bounds__(kIq2Threads) void dense_iq2_kernel(DenseIq2Args g)
     extern __shared__ __align__(16) unsigned char dense_iq2_lds[];
     if (lds_address_of(dense_iq2_lds) != 0u) {   // operands are addressed by absolute LDS offsets
         if (threadIdx.x == 0u) raise_status(g.status, 2);
+        publish_when_last(g.publication, g.status, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
         return;
     }
     const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -133,10 +136,10 @@ __global__ __launch_bounds__(kIq2Threads) void dense_iq2_kernel(DenseIq2Args g)
         for (int i = 0; i < 4; ++i) partial[((wave - 1u) * 4u + i) * 64u + lane] = acc[i];
     }
     __syncthreads();
-    if (wave) return;
     const unsigned long long row = row0 + r;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+        if (wave) break;
         const unsigned long long token = tok0 + 4u * q + i;
         double wide = acc[i];
 #pragma unroll
@@ -144,8 +147,9 @@ __global__ __launch_bounds__(kIq2Threads) void dense_iq2_kernel(DenseIq2Args g)
         if (row >= g.row_count || token >= g.input_rows) continue;
         const float sum = (float)wide, value = g.output_bf16 ? bf16_round(sum) : sum;
         if (!finite_f32(value)) raise_status(g.status, 1);
-        else g.out[token * g.row_count + row] = value;
+        else store_published(g.publication, g.out + token * g.row_count + row, value);
     }
+    publish_when_last(g.publication, g.status, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
 }
 
 }  // namespace
@@ -163,7 +167,7 @@ bool iq2_rows_small(uint64_t row_count, uint64_t row_width, uint64_t input_rows)
 
 int launch_iq2_rows_small(const uint8_t *encoded, uint64_t row_count, uint64_t row_width, uint64_t row_bytes,
                           const void *act_q8k, uint64_t input_rows, float *out, bool output_bf16, int *status,
-                          hipStream_t stream)
+                          hipStream_t stream, Publisher *publisher)
 {
     const uint64_t row_tiles = (row_count + 15u) / 16u, token_tiles = (input_rows + 15u) / 16u;
     if (!row_count || !input_rows || row_width % 512u || row_width / 256u * 66u != row_bytes || row_tiles > 0x7fffffffull ||
@@ -173,7 +177,7 @@ int launch_iq2_rows_small(const uint8_t *encoded, uint64_t row_count, uint64_t r
     YVEX_ALLOW_DYNAMIC_LDS(dense_iq2_kernel, kIq2LdsBytes);
     dense_iq2_kernel<<<dim3((unsigned)row_tiles, (unsigned)token_tiles), kIq2Threads, kIq2LdsBytes, stream>>>(
         DenseIq2Args{encoded, row_count, row_bytes, (unsigned)(row_width / 256u), (const unsigned char *)act_q8k, input_rows,
-                     out, output_bf16 ? 1 : 0, status});
+                     out, output_bf16 ? 1 : 0, status, take_publication(publisher, row_tiles * token_tiles)});
     return check_launch("dense_iq2");
 }
 

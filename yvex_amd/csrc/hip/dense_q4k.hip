@@ -26,6 +26,7 @@
 #include "common.hpp"
 #include "launch.hpp"
 #include "grouped.hpp"
+#include "publish.hpp"
 
 namespace yvex {
 
@@ -45,6 +46,7 @@ struct DenseQ4kArgs {
     unsigned long long out_stride;
     int output_bf16;
     int *status;
+    Publication publication;
 };
 
 // What one wave needs of one superblock: the weight row's block and NT token blocks.
@@ -422,10 +424,10 @@ __global__ __launch_bounds__(64 * WAVES) void dense_q4k16_kernel(DenseQ4kArgs g)
         for (int i = 0; i < 4; ++i) partial[wave - 1u][i][lane] = acc[i];
     }
     __syncthreads();
-    if (wave) return;
     const unsigned long long token = tok0 + r;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+        if (wave) break;
         const unsigned long long row = row0 + 4u * q + (unsigned)i;
         double wide = acc[i];
 #pragma unroll
@@ -435,8 +437,9 @@ __global__ __launch_bounds__(64 * WAVES) void dense_q4k16_kernel(DenseQ4kArgs g)
         const unsigned long long at = token * g.out_stride + row;
         const float value = g.additive ? sum + g.additive[at] : sum;
         if (!finite_f32(value)) raise_status(g.status, 1);
-        else g.out[at] = g.output_bf16 ? bf16_round(value) : value;
+        else store_published(g.publication, g.out + at, g.output_bf16 ? bf16_round(value) : value);
     }
+    publish_when_last(g.publication, g.status, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
 }
 
 }  // namespace
@@ -444,7 +447,7 @@ __global__ __launch_bounds__(64 * WAVES) void dense_q4k16_kernel(DenseQ4kArgs g)
 int launch_q4k_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t row_width,
                           uint64_t row_bytes, const void *act_q8k, uint64_t input_rows,
                           const float *additive, float *out, uint64_t out_stride, bool output_bf16,
-                          int *status, hipStream_t stream)
+                          int *status, hipStream_t stream, Publisher *publisher)
 {
     if (!row_count || !input_rows || row_width % 256u || row_width / 256u * 144u != row_bytes)
         return ST_BOUNDS;
@@ -453,7 +456,7 @@ int launch_q4k_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t r
     if (row_tiles > 0x7fffffffull || row_width / 256u > 0xffffffffull) return ST_BOUNDS;
     DenseQ4kArgs g{encoded, row_count, row_bytes, (unsigned)(row_width / 256u),
                    (const unsigned char *)act_q8k, input_rows, additive, out, out_stride,
-                   output_bf16 ? 1 : 0, status};
+                   output_bf16 ? 1 : 0, status, {}};
     // 16 x 16 tiles, on four waves where several workgroups share a compute unit (7168 x 7168 by 32 rows 23.2 us, on
     // eight 26.8; 7168 x 2048 by 32 9.8 and 13.1), up to 32 input rows and beyond them while tiles of twice the tokens would fit
     // the device in one round (2048 x 7168 by 64 rows 12.7 us, on the 32 x 32 tiles 16.7).
@@ -462,6 +465,7 @@ int launch_q4k_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t r
     if (input_rows <= 32u || small_tiles * token_tiles32 <= units) {
         if (small_tiles > 0x7fffffffull || token_tiles16 > 65535ull) return ST_BOUNDS;
         const dim3 grid((unsigned)small_tiles, (unsigned)token_tiles16);
+        g.publication = take_publication(publisher, small_tiles * token_tiles16);
         if (small_tiles * token_tiles16 <= units) dense_q4k16_kernel<8><<<grid, 512, 0, stream>>>(g);
         else dense_q4k16_kernel<4><<<grid, 256, 0, stream>>>(g);
     } else {

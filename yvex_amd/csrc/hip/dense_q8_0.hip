@@ -23,6 +23,7 @@
 #include "common.hpp"
 #include "launch.hpp"
 #include "lds_copy.hpp"
+#include "publish.hpp"
 
 namespace yvex {
 
@@ -41,6 +42,7 @@ struct DenseQ80Args {
     int *status;
     const unsigned char *encoded_second;     // a second matrix of the same shape (blockIdx.z = 1), or null
     float *out_second;
+    Publication publication;
 };
 
 __device__ __forceinline__ void choose_matrix(DenseQ80Args &g)
@@ -287,6 +289,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void dense_q8_0_small_kernel(Dens
     extern __shared__ __align__(16) unsigned char dense_q8_0_small_lds[];
     if (lds_address_of(dense_q8_0_small_lds) != 0u) {   // operands are addressed by absolute LDS offsets
         if (threadIdx.x == 0u) raise_status(g.status, 2);
+        publish_when_last(g.publication, g.status, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
         return;
     }
     choose_matrix(g);
@@ -355,10 +358,10 @@ __global__ __launch_bounds__(64 * kSmallWaves) void dense_q8_0_small_kernel(Dens
         for (int i = 0; i < 4; ++i) partial[((wave - 1u) * 4u + i) * 64u + lane] = acc[i];
     }
     __syncthreads();
-    if (wave) return;
     const unsigned long long row = row0 + r;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+        if (wave) break;
         const unsigned long long token = tok0 + 4u * q + i;
         double wide = acc[i];
 #pragma unroll
@@ -368,8 +371,9 @@ __global__ __launch_bounds__(64 * kSmallWaves) void dense_q8_0_small_kernel(Dens
         const unsigned long long at = token * g.out_stride + row;
         const float value = g.additive ? sum + g.additive[at] : sum;
         if (!finite_f32(value)) raise_status(g.status, 1);
-        else g.out[at] = g.output_bf16 ? bf16_round(value) : value;
+        else store_published(g.publication, g.out + at, g.output_bf16 ? bf16_round(value) : value);
     }
+    publish_when_last(g.publication, g.status, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
 }
 
 // The same product for batches that offer every compute unit a tile of 128 weight rows x 64
@@ -419,6 +423,7 @@ __global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS) void dense_q8_0_sta
     extern __shared__ __align__(16) unsigned char dense_q8_0_lds[];
     if (lds_address_of(dense_q8_0_lds) != 0u) {   // operands are addressed by absolute LDS offsets
         if (threadIdx.x == 0u) raise_status(g.status, 2);
+        if constexpr (TOKEN_BLOCKS == 1u) publish_when_last(g.publication, g.status, blockIdx.x, gridDim.x);
         return;
     }
     choose_matrix(g);
@@ -556,19 +561,20 @@ __global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS) void dense_q8_0_sta
     // lane (r, h): weight row r of the wave's 32 against sixteen input rows; a store instruction
     // writes 32 consecutive floats of two output rows
     const unsigned long long row = row0 + 32u * row_block + r;
-    if (row >= g.row_count) return;
     bool bad = false;
 #pragma unroll
     for (unsigned i = 0; i < 16u; ++i) {
         const unsigned long long token = tok0 + 32u * token_block + 8u * (i >> 2) + 4u * h + (i & 3u);
-        if (token >= g.input_rows) continue;
+        if (row >= g.row_count || token >= g.input_rows) continue;
         const unsigned long long at = token * g.out_stride + row;
         const float sum = (float)acc[i];
         const float value = g.additive ? sum + g.additive[at] : sum;
         if (!finite_f32(value)) bad = true;
+        else if (TOKEN_BLOCKS == 1u) store_published(g.publication, g.out + at, g.output_bf16 ? bf16_round(value) : value);
         else g.out[at] = g.output_bf16 ? bf16_round(value) : value;
     }
     if (bad) raise_status(g.status, 1);
+    if constexpr (TOKEN_BLOCKS == 1u) publish_when_last(g.publication, g.status, blockIdx.x, gridDim.x);
 }
 
 constexpr unsigned kWideRows = 128u, kWideTokens = 128u, kWideThreads = 1024u;
@@ -679,7 +685,8 @@ __global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80A
 int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t row_width,
                            uint64_t row_bytes, const void *act_q8k, uint64_t input_rows,
                            const float *additive, float *out, uint64_t out_stride, bool output_bf16,
-                           int *status, hipStream_t stream, const uint8_t *encoded_second, float *out_second)
+                           int *status, hipStream_t stream, const uint8_t *encoded_second, float *out_second,
+                           Publisher *publisher)
 {
     const uint64_t matrices = encoded_second ? 2u : 1u;
     if (!row_count || !input_rows || row_width % 256u || row_width / 32u * 34u != row_bytes)
@@ -690,7 +697,8 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
     if (row_tiles > 0x7fffffffull || row_width / 256u > 0xffffffffull) return ST_BOUNDS;
     DenseQ80Args g{encoded, row_count, row_bytes, (unsigned)(row_width / 256u),
                    (const unsigned char *)act_q8k, input_rows, additive, out, out_stride,
-                   output_bf16 ? 1 : 0, status, encoded_second, out_second};
+                   output_bf16 ? 1 : 0, status, encoded_second, out_second, {}};
+    if (matrices > 1u) publisher = nullptr;       // (workgroups are counted over one matrix)
     // Which tiles: a pass over the row width costs a workgroup about the same whatever the device's
     // load (measured at 16 superblocks a row, microseconds: 9 on the 16 x 16 tile and 3.8 more for every such workgroup
     // that a compute unit has besides, 14 on the 32-row tile and 18.5 once two such
@@ -706,6 +714,7 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
     // memory time 173 us)
     if (aligned16 && input_rows <= 32u && units && matrices * ((row_count + 255u) / 256u) >= units) {
         YVEX_ALLOW_DYNAMIC_LDS((dense_q8_0_staged_kernel<8u, 1u>), staged_lds_bytes(8u, 1u));
+        g.publication = take_publication(publisher, (row_count + 255u) / 256u);
         dense_q8_0_staged_kernel<8u, 1u><<<dim3((unsigned)((row_count + 255u) / 256u), 1, (unsigned)matrices), 512, staged_lds_bytes(8u, 1u),
                                            stream>>>(g);
         return check_launch("dense_q8_0_staged");
@@ -717,6 +726,7 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
     // (a batch that offers the staged tiles more than these is not theirs: they take 29 us at least)
     if (small_cost < plain_cost && small_cost < 29.0 && token_tiles16 <= 65535u && (row_count + 15u) / 16u <= 0x7fffffffull) {
         YVEX_ALLOW_DYNAMIC_LDS(dense_q8_0_small_kernel, kSmallLdsBytes);
+        g.publication = take_publication(publisher, small);
         dense_q8_0_small_kernel<<<dim3((unsigned)((row_count + 15u) / 16u), (unsigned)token_tiles16, (unsigned)matrices),
                                   64 * kSmallWaves, kSmallLdsBytes, stream>>>(g);
         return check_launch("dense_q8_0_small");

@@ -42,16 +42,18 @@ int compute_units();
         });                                                                                     \
     } while (0)
 
+struct Publisher;       // publish.hpp: a launch that may end a synchronous operation by itself
+
 // IQ2_XXS rows x Q8_K input rows on the int8 matrix cores as a plain projection (prefill.hip).
 int launch_iq2_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t row_width,
                           uint64_t row_bytes, const void *act_q8k, uint64_t input_rows, float *out,
-                          bool round_bf16, int *status, hipStream_t stream);
+                          bool round_bf16, int *status, hipStream_t stream, Publisher *publisher = nullptr);
 
 // The same where the matrix is small (dense_iq2.hip), and whether it is.
 bool iq2_rows_small(uint64_t row_count, uint64_t row_width, uint64_t input_rows);
 int launch_iq2_rows_small(const uint8_t *encoded, uint64_t row_count, uint64_t row_width, uint64_t row_bytes,
                           const void *act_q8k, uint64_t input_rows, float *out, bool output_bf16, int *status,
-                          hipStream_t stream);
+                          hipStream_t stream, Publisher *publisher);
 
 // Q8_0 rows x Q8_K input rows on the int8 matrix cores (dense_q8_0.hip); with a second matrix of the
 // same shape both products in one launch.
@@ -59,13 +61,13 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
                            uint64_t row_bytes, const void *act_q8k, uint64_t input_rows,
                            const float *additive, float *out, uint64_t out_stride, bool output_bf16,
                            int *status, hipStream_t stream, const uint8_t *encoded_second = nullptr,
-                           float *out_second = nullptr);
+                           float *out_second = nullptr, Publisher *publisher = nullptr);
 
 // Q4_K rows x Q8_K input rows on the int8 matrix cores (dense_q4k.hip).
 int launch_q4k_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t row_width,
                           uint64_t row_bytes, const void *act_q8k, uint64_t input_rows,
                           const float *additive, float *out, uint64_t out_stride, bool output_bf16,
-                          int *status, hipStream_t stream);
+                          int *status, hipStream_t stream, Publisher *publisher = nullptr);
 // The same product with its operands staged through LDS, for batches that fill every compute
 // unit with (128 rows x 64 tokens) tiles (rows_q4k.hip).
 int launch_q4k_rows_staged(const uint8_t *encoded, uint64_t row_count, uint64_t row_width,

@@ -13,6 +13,7 @@
 #include "launch.hpp"
 #include "units.hpp"
 #include "route.hpp"
+#include "publish.hpp"
 #include "q8_0_rows.hpp"
 
 namespace yvex {
@@ -32,6 +33,7 @@ struct MatvecArgs {
     int scoring;
     const unsigned char *encoded_second = nullptr;   // a second matrix of the same shape (blockIdx.z = 1)
     float *out_second = nullptr;
+    Publication publication = {nullptr, nullptr, 0u, 0};
 };
 
 __device__ __forceinline__ void matvec_publish(const MatvecArgs &a, unsigned long long in,
@@ -40,7 +42,7 @@ __device__ __forceinline__ void matvec_publish(const MatvecArgs &a, unsigned lon
     const unsigned long long at = in * a.out_stride + row;
     float value = a.additive ? sum + a.additive[at] : sum;
     if (!finite_f32(value)) raise_status(a.status, 1);
-    else a.out[at] = a.output_bf16 ? bf16_round(value) : value;
+    else store_published(a.publication, a.out + at, a.output_bf16 ? bf16_round(value) : value);
 }
 
 // Slow exact path for a row whose F32 sum overflowed before opposite terms cancelled
@@ -197,6 +199,7 @@ __global__ __launch_bounds__(kHeldThreads) void matvec_q8_0_quantizing_kernel(Ma
                     [&](unsigned in, unsigned long long row, float sum) {
                         if (in < input_rows) matvec_publish(a, in, row, sum);
                     });
+    publish_when_last(a.publication, a.status, blockIdx.x, gridDim.x);
 }
 
 // A unit against 32 int8 activations held in registers; `sums` = the two 16-value sums of the
@@ -319,6 +322,7 @@ __global__ __launch_bounds__(256) void dense_row_q8k_kernel(MatvecArgs a)
     }
     acc = group_sum_f64_last<L>(acc);
     if (row_live && slot == (unsigned)L - 1u) matvec_publish(a, 0ull, row, (float)acc);
+    publish_when_last(a.publication, a.status, blockIdx.x, gridDim.x);
 }
 
 // The same for a few Q8_K input rows (rows of up to 8192 columns, which L lanes hold whole): the
@@ -396,6 +400,7 @@ __global__ __launch_bounds__(256) void dense_fewrows_q8k_kernel(MatvecArgs a)
         if (row_live && slot == (unsigned)L - 1u) matvec_publish(a, in, row, (float)sum);
         current = next;
     }
+    publish_when_last(a.publication, a.status, blockIdx.x, gridDim.x);
 }
 
 // F32 / F16 / BF16 weight rows: lanes stride the row element-wise. Products and sums run in
@@ -975,10 +980,11 @@ static int launch_block_even(const MatvecArgs &a, hipStream_t stream)
 }
 
 template <unsigned QT, int L>
-static int launch_dense_row(const MatvecArgs &a, hipStream_t stream)
+static int launch_dense_row(MatvecArgs &a, hipStream_t stream, Publisher *publisher)
 {
     const unsigned long long grid = (a.row_count + 4ull * (64u / L) - 1ull) / (4ull * (64u / L));
     if (grid > 0x7fffffffull) return ST_BOUNDS;
+    a.publication = take_publication(publisher, grid);
     dense_row_q8k_kernel<QT, L><<<(unsigned)grid, 256, 0, stream>>>(a);
     return check_launch("matvec.row");
 }
@@ -994,10 +1000,11 @@ static bool dense_row_applies(const MatvecArgs &a)
 }
 
 template <unsigned QT, int L>
-static int launch_dense_fewrows(const MatvecArgs &a, hipStream_t stream)
+static int launch_dense_fewrows(MatvecArgs &a, hipStream_t stream, Publisher *publisher)
 {
     const unsigned long long grid = (a.row_count + 4ull * (64u / L) - 1ull) / (4ull * (64u / L));
     if (grid > 0x7fffffffull) return ST_BOUNDS;
+    a.publication = take_publication(publisher, grid);
     dense_fewrows_q8k_kernel<QT, L><<<(unsigned)grid, 256, 0, stream>>>(a);
     return check_launch("matvec.fewrows");
 }
@@ -1014,40 +1021,40 @@ static bool dense_fewrows_applies(const MatvecArgs &a)
 }
 
 template <unsigned QT>
-static int launch_dense_fewrows_width(const MatvecArgs &a, hipStream_t stream)
+static int launch_dense_fewrows_width(MatvecArgs &a, hipStream_t stream, Publisher *publisher)
 {
     const unsigned long long halves = a.row_width >> 7;
-    if (halves <= 8ull) return launch_dense_fewrows<QT, 8>(a, stream);
-    if (halves <= 16ull) return launch_dense_fewrows<QT, 16>(a, stream);
-    if (halves <= 32ull) return launch_dense_fewrows<QT, 32>(a, stream);
-    return launch_dense_fewrows<QT, 64>(a, stream);
+    if (halves <= 8ull) return launch_dense_fewrows<QT, 8>(a, stream, publisher);
+    if (halves <= 16ull) return launch_dense_fewrows<QT, 16>(a, stream, publisher);
+    if (halves <= 32ull) return launch_dense_fewrows<QT, 32>(a, stream, publisher);
+    return launch_dense_fewrows<QT, 64>(a, stream, publisher);
 }
 
 template <unsigned QT>
-static int launch_dense_row_width(const MatvecArgs &a, hipStream_t stream)
+static int launch_dense_row_width(MatvecArgs &a, hipStream_t stream, Publisher *publisher)
 {
     const unsigned long long halves = a.row_width >> 7;
-    if (halves <= 8ull) return launch_dense_row<QT, 8>(a, stream);
-    if (halves <= 16ull) return launch_dense_row<QT, 16>(a, stream);
-    if (halves <= 32ull) return launch_dense_row<QT, 32>(a, stream);
-    return launch_dense_row<QT, 64>(a, stream);
+    if (halves <= 8ull) return launch_dense_row<QT, 8>(a, stream, publisher);
+    if (halves <= 16ull) return launch_dense_row<QT, 16>(a, stream, publisher);
+    if (halves <= 32ull) return launch_dense_row<QT, 32>(a, stream, publisher);
+    return launch_dense_row<QT, 64>(a, stream, publisher);
 }
 
 template <unsigned QT, bool Q8>
-static int launch_block(const MatvecArgs &a, hipStream_t stream)
+static int launch_block(MatvecArgs &a, hipStream_t stream, Publisher *publisher)
 {
     if constexpr (Q8 && UnitTraits<QT>::kIntegerCombine) {
-        if (dense_row_applies<QT>(a)) return launch_dense_row_width<QT>(a, stream);
-        if (dense_fewrows_applies<QT>(a)) return launch_dense_fewrows_width<QT>(a, stream);
+        if (dense_row_applies<QT>(a)) return launch_dense_row_width<QT>(a, stream, publisher);
+        if (dense_fewrows_applies<QT>(a)) return launch_dense_fewrows_width<QT>(a, stream, publisher);
     }
     const bool even = (((unsigned long long)a.encoded | a.row_bytes) & 1ull) == 0ull;
     return even ? launch_block_even<QT, Q8, true>(a, stream) : launch_block_even<QT, Q8, false>(a, stream);
 }
 
 template <unsigned QT>
-static int launch_block_q(const MatvecArgs &a, bool q8, hipStream_t stream)
+static int launch_block_q(MatvecArgs &a, bool q8, hipStream_t stream, Publisher *publisher)
 {
-    return q8 ? launch_block<QT, true>(a, stream) : launch_block<QT, false>(a, stream);
+    return q8 ? launch_block<QT, true>(a, stream, publisher) : launch_block<QT, false>(a, stream, publisher);
 }
 
 }  // namespace yvex
@@ -1118,11 +1125,11 @@ static bool q8_0_takes_matrix_cores(const uint8_t *encoded, uint64_t row_count, 
             (input_rows >= 2ull && matrix_bytes >= (8ull << 20)));
 }
 
-extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint64_t row_count,
-                               uint64_t row_width, uint64_t row_bytes, const void *input,
-                               int input_q8, uint64_t input_rows, uint64_t input_stride,
-                               const float *additive, float *out, uint64_t out_stride,
-                               int output_bf16, int *status, yvex_hip_stream stream)
+static int launch_matvec(const uint8_t *encoded, unsigned int qtype, uint64_t row_count,
+                         uint64_t row_width, uint64_t row_bytes, const void *input,
+                         int input_q8, uint64_t input_rows, uint64_t input_stride,
+                         const float *additive, float *out, uint64_t out_stride,
+                         int output_bf16, int *status, yvex_hip_stream stream, Publisher *publisher)
 {
     unsigned block, bytes;
     if (!encoded || !input || !out || !status || !row_count || !row_width || !input_rows ||
@@ -1156,7 +1163,7 @@ extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint6
         out_stride == row_count && row_count % 4ull == 0ull && !((uintptr_t)encoded & 3u) &&
         !(row_bytes & 3ull) && row_width / 32ull <= 64ull * 4ull && !((uintptr_t)out & 15u))
         return launch_iq2_rows_dense(encoded, row_count, row_width, row_bytes, input, input_rows, out,
-                                     output_bf16 != 0, status, s);
+                                     output_bf16 != 0, status, s, publisher);
     // Q4_K rows against two or more Q8_K input rows: matrix cores (the reference's threshold is 16
     // input rows; here the 16-token tiles beat the general kernel below from two rows on, 10.5 us
     // against 12.2 us at 2 and 19.7 us at 15 rows for 2048 x 7168; the few-rows kernel, where it
@@ -1164,7 +1171,7 @@ extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint6
     if (qtype == QT_Q4_K && input_q8 && input_rows >= 2ull && !((uintptr_t)encoded & 15u) &&
         !(input_rows < 4ull && dense_fewrows_applies<QT_Q4_K>(a)))
         return launch_q4k_rows_dense(encoded, row_count, row_width, row_bytes, input, input_rows, additive,
-                                     out, out_stride, output_bf16 != 0, status, s);
+                                     out, out_stride, output_bf16 != 0, status, s, publisher);
     // Q8_0 rows against a batch of Q8_K input rows: matrix cores (the reference's threshold is 16 rows,
     // src/backend/cuda/private.h:461-464); the lane-strided kernel reads the matrix once per four input rows, which
     // matrices of under 8 MB bear up to nine (lane-strided and matrix cores: 1024 x 4096 by 4 / 8 / 10 / 12 rows 5.3 / 6.0 /
@@ -1172,7 +1179,7 @@ extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint6
     // and 6.8, 4096 x 4096 by 2 / 8 9.8 / 14.7 and 7.7 / 8.1, 7168 x 7168 by 2 19.2 and 16.6)
     if (qtype == QT_Q8_0 && input_q8 && q8_0_takes_matrix_cores(encoded, row_count, row_bytes, input_rows))
         return launch_q8_0_rows_dense(encoded, row_count, row_width, row_bytes, input, input_rows, additive, out,
-                                      out_stride, output_bf16 != 0, status, s);
+                                      out_stride, output_bf16 != 0, status, s, nullptr, nullptr, publisher);
     // F32 rows against a batch of F32 input rows: the double-precision matrix cores; rows of F16
     // and BF16 values take the same kernels (the conversion to double is exact for them as well),
     // and so do Q8_0 rows against F32 input rows (a caller that switched the Q8 activation policy
@@ -1206,12 +1213,35 @@ extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint6
         return check_launch("matvec_scalar");
     }
     switch (qtype) {
-    case QT_IQ2_XXS: return launch_block_q<QT_IQ2_XXS>(a, input_q8, s);
-    case QT_Q8_0: return launch_block_q<QT_Q8_0>(a, input_q8, s);
-    case QT_Q4_K: return launch_block_q<QT_Q4_K>(a, input_q8, s);
-    case QT_Q2_K: return launch_block_q<QT_Q2_K>(a, input_q8, s);
+    case QT_IQ2_XXS: return launch_block_q<QT_IQ2_XXS>(a, input_q8, s, publisher);
+    case QT_Q8_0: return launch_block_q<QT_Q8_0>(a, input_q8, s, publisher);
+    case QT_Q4_K: return launch_block_q<QT_Q4_K>(a, input_q8, s, publisher);
+    case QT_Q2_K: return launch_block_q<QT_Q2_K>(a, input_q8, s, publisher);
     default: return ST_UNSUPPORTED;
     }
+}
+
+extern "C" int yvex_hip_matvec(const uint8_t *encoded, unsigned int qtype, uint64_t row_count,
+                               uint64_t row_width, uint64_t row_bytes, const void *input,
+                               int input_q8, uint64_t input_rows, uint64_t input_stride,
+                               const float *additive, float *out, uint64_t out_stride,
+                               int output_bf16, int *status, yvex_hip_stream stream)
+{
+    return launch_matvec(encoded, qtype, row_count, row_width, row_bytes, input, input_q8, input_rows, input_stride,
+                         additive, out, out_stride, output_bf16, status, stream, nullptr);
+}
+
+int yvex_hip_matvec_publishing(const uint8_t *encoded, unsigned int qtype, uint64_t row_count, uint64_t row_width,
+                               uint64_t row_bytes, const void *input, int input_q8, uint64_t input_rows,
+                               uint64_t input_stride, const float *additive, float *out, uint64_t out_stride,
+                               int output_bf16, int *status, const yvex_hip_publication *publication, int *published,
+                               yvex_hip_stream stream)
+{
+    Publisher publisher = publisher_of(*publication);
+    const int rc = launch_matvec(encoded, qtype, row_count, row_width, row_bytes, input, input_q8, input_rows, input_stride,
+                                 additive, out, out_stride, output_bf16, status, stream, &publisher);
+    *published = publisher.taken;
+    return rc;
 }
 
 // Whether F32 input rows are multiplied by the launch that quantizes them. Every workgroup quantizes all of them, a
@@ -1231,21 +1261,22 @@ extern "C" int yvex_hip_matvec_quantizing_supported(const uint8_t *encoded, unsi
 }
 
 template <int T>
-static int launch_quantizing(const MatvecArgs &a, hipStream_t s)
+static int launch_quantizing(MatvecArgs &a, hipStream_t s, Publisher *publisher)
 {
     const unsigned long long groups = (a.row_count + kHeldWaves - 1ull) / kHeldWaves, most = (unsigned long long)compute_units();
     const unsigned grid = (unsigned)(groups < most ? groups : most);
     const unsigned lds = (unsigned)held_bytes(T, a.row_width / 256ull);
+    a.publication = take_publication(publisher, grid);
     if (a.row_width <= 2048ull) matvec_q8_0_quantizing_kernel<T, 1><<<grid, kHeldThreads, lds, s>>>(a);
     else if (a.row_width <= 4096ull) matvec_q8_0_quantizing_kernel<T, 2><<<grid, kHeldThreads, lds, s>>>(a);
     else matvec_q8_0_quantizing_kernel<T, 4><<<grid, kHeldThreads, lds, s>>>(a);
     return check_launch("matvec_quantizing");
 }
 
-extern "C" int yvex_hip_matvec_quantizing(const uint8_t *encoded, unsigned int qtype, uint64_t row_count,
+static int launch_matvec_quantizing(const uint8_t *encoded, unsigned int qtype, uint64_t row_count,
                                           uint64_t row_width, uint64_t row_bytes, const float *input,
                                           uint64_t input_rows, uint64_t input_stride, const float *additive, float *out,
-                                          uint64_t out_stride, int output_bf16, int *status, yvex_hip_stream stream)
+                                          uint64_t out_stride, int output_bf16, int *status, yvex_hip_stream stream, Publisher *publisher)
 {
     if (!encoded || !input || !out || !status || out_stride < row_count || input_stride < row_width ||
         (((uintptr_t)input | (uintptr_t)out) & 3u))
@@ -1254,7 +1285,29 @@ extern "C" int yvex_hip_matvec_quantizing(const uint8_t *encoded, unsigned int q
         return ST_UNSUPPORTED;
     MatvecArgs a{encoded, row_count, row_width, row_bytes, input, input_rows, input_stride, additive, out, out_stride,
                  output_bf16, status, nullptr, nullptr, 0};
-    return input_rows == 1u ? launch_quantizing<1>(a, as_stream(stream)) : launch_quantizing<2>(a, as_stream(stream));
+    return input_rows == 1u ? launch_quantizing<1>(a, as_stream(stream), publisher) : launch_quantizing<2>(a, as_stream(stream), publisher);
+}
+
+extern "C" int yvex_hip_matvec_quantizing(const uint8_t *encoded, unsigned int qtype, uint64_t row_count,
+                                          uint64_t row_width, uint64_t row_bytes, const float *input,
+                                          uint64_t input_rows, uint64_t input_stride, const float *additive, float *out,
+                                          uint64_t out_stride, int output_bf16, int *status, yvex_hip_stream stream)
+{
+    return launch_matvec_quantizing(encoded, qtype, row_count, row_width, row_bytes, input, input_rows, input_stride, additive,
+                                    out, out_stride, output_bf16, status, stream, nullptr);
+}
+
+int yvex_hip_matvec_quantizing_publishing(const uint8_t *encoded, unsigned int qtype, uint64_t row_count,
+                                          uint64_t row_width, uint64_t row_bytes, const float *input,
+                                          uint64_t input_rows, uint64_t input_stride, const float *additive, float *out,
+                                          uint64_t out_stride, int output_bf16, int *status,
+                                          const yvex_hip_publication *publication, int *published, yvex_hip_stream stream)
+{
+    Publisher publisher = publisher_of(*publication);
+    const int rc = launch_matvec_quantizing(encoded, qtype, row_count, row_width, row_bytes, input, input_rows, input_stride,
+                                            additive, out, out_stride, output_bf16, status, stream, &publisher);
+    *published = publisher.taken;
+    return rc;
 }
 
 // Two Q8_0 matrices of one shape against the same Q8_K input rows in one launch (a shared expert's gate

@@ -862,13 +862,14 @@ static int launch_rows(MfmaArgs &a, unsigned qtype, hipStream_t stream)
 // A plain projection through the row-batch kernel: every input row in one bucket of expert 0.
 int launch_iq2_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t row_width,
                           uint64_t row_bytes, const void *act_q8k, uint64_t input_rows, float *out,
-                          bool round_bf16, int *status, hipStream_t stream)
+                          bool round_bf16, int *status, hipStream_t stream, Publisher *publisher)
 {
     int rc = check_matrix(QT_IQ2_XXS, row_width, row_bytes);
     if (rc) return rc;
     if (input_rows > 0xffffffffull || row_count > 0xffffffffull || row_count % 4u) return ST_BOUNDS;
     if (iq2_rows_small(row_count, row_width, input_rows))
-        return launch_iq2_rows_small(encoded, row_count, row_width, row_bytes, act_q8k, input_rows, out, round_bf16, status, stream);
+        return launch_iq2_rows_small(encoded, row_count, row_width, row_bytes, act_q8k, input_rows, out, round_bf16, status, stream,
+                                     publisher);
     yvex_hip_expert_weights w{};
     w.down = encoded;
     w.down_qtype = QT_IQ2_XXS;

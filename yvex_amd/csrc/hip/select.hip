@@ -12,6 +12,7 @@
 // side.
 #include "common.hpp"
 #include "launch.hpp"
+#include "publish.hpp"
 
 namespace yvex {
 
@@ -159,23 +160,41 @@ __device__ __forceinline__ Candidate span_candidate(const float *row, unsigned l
     return all;
 }
 
+// Where a row's results go: to device memory, and for a launch that publishes behind the head of its host memory as well,
+// ties, tokens and values of all rows end to end.
+struct Selection {
+    unsigned *tokens;
+    float *values;
+    unsigned long long *ties, row_count;
+    Publication publication;
+};
+
+__device__ __forceinline__ void selection_store(const Selection &s, unsigned long long row, const Candidate &c)
+{
+    store_published(s.publication, s.tokens + row, c.index);
+    store_published(s.publication, s.values + row, c.best);
+    store_published(s.publication, s.ties + row, c.ties);
+    if (!s.publication.host) return;
+    unsigned *const results = s.publication.host + YVEX_HIP_PUBLISH_HEAD_BYTES / 4u;
+    const unsigned words[4] = {(unsigned)c.ties, (unsigned)(c.ties >> 32), c.index, __float_as_uint(c.best)};
+    const unsigned long long at[4] = {2ull * row, 2ull * row + 1ull, 2ull * s.row_count + row, 3ull * s.row_count + row};
+#pragma unroll
+    for (unsigned i = 0; i < 4u; ++i)
+        __hip_atomic_store(results + at[i], words[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 constexpr unsigned kSelectThreads = 1024u;    // one workgroup per row
 constexpr unsigned kSpanThreads = 256u;       // several workgroups per row
 constexpr unsigned kSpanElements = 8192u;
 
 __global__ __launch_bounds__(kSelectThreads) void argmax_rows_kernel(
-    const float *values, unsigned long long row_count, unsigned long long row_width,
-    unsigned *selected_tokens, float *selected_values, unsigned long long *tie_counts, int *status)
+    const float *values, unsigned long long row_width, Selection selection, int *status)
 {
     const unsigned long long row = blockIdx.x;
-    if (row >= row_count) return;
     bool ok;
     const Candidate all = span_candidate<kSelectThreads>(values + row * row_width, 0ull, row_width, status, ok);
-    if (threadIdx.x == 0u && ok) {
-        selected_tokens[row] = all.index;
-        selected_values[row] = all.best;
-        tie_counts[row] = all.ties;
-    }
+    if (threadIdx.x == 0u && ok) selection_store(selection, row, all);
+    publish_when_last(selection.publication, status, blockIdx.x, gridDim.x);
 }
 
 // A long row split over blockIdx.x spans of kSpanElements: partial candidates into scratch
@@ -202,11 +221,9 @@ __global__ __launch_bounds__(kSpanThreads) void argmax_spans_kernel(
 }
 
 __global__ __launch_bounds__(64) void argmax_merge_kernel(
-    const SpanResult *partial, unsigned spans, unsigned long long row_count, unsigned *selected_tokens,
-    float *selected_values, unsigned long long *tie_counts)
+    const SpanResult *partial, unsigned spans, Selection selection, int *status)
 {
     const unsigned long long row = blockIdx.x;
-    if (row >= row_count) return;
     const unsigned lane = threadIdx.x;
     Candidate mine{-3.402823466e+38F, 0xffffffffu, 0ull};
     bool bad = false;         // a span that met a non-finite value counts no element at all
@@ -217,7 +234,7 @@ __global__ __launch_bounds__(64) void argmax_merge_kernel(
     }
     // only the row that holds the bad value publishes nothing, as when one workgroup scans a row;
     // a status left by other work on the stream does not silence the rows of this launch
-    if (__any(bad)) return;
+    const bool kept = !__any(bad);
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) {
         Candidate other;
@@ -226,11 +243,8 @@ __global__ __launch_bounds__(64) void argmax_merge_kernel(
         other.ties = (unsigned long long)__shfl_xor((long long)mine.ties, offset, kWave);
         candidate_merge(mine, other);
     }
-    if (lane == 0u) {
-        selected_tokens[row] = mine.index;
-        selected_values[row] = mine.best;
-        tie_counts[row] = mine.ties;
-    }
+    if (lane == 0u && kept) selection_store(selection, row, mine);
+    publish_when_last(selection.publication, status, blockIdx.x, gridDim.x);
 }
 
 // Span results for callers that cannot allocate: one array per device, held until the process
@@ -278,10 +292,9 @@ extern "C" uint64_t yvex_hip_argmax_scratch_bytes(uint64_t row_count, uint64_t r
     return spans > 1u ? row_count * spans * sizeof(SpanResult) : 0u;
 }
 
-extern "C" int yvex_hip_argmax_f32(const float *values, uint64_t row_count, uint64_t row_width,
-                                   uint32_t *selected_tokens, float *selected_values,
-                                   uint64_t *tie_counts, void *scratch, uint64_t scratch_bytes,
-                                   int *status, yvex_hip_stream stream)
+static int launch_argmax(const float *values, uint64_t row_count, uint64_t row_width, uint32_t *selected_tokens,
+                         float *selected_values, uint64_t *tie_counts, void *scratch, uint64_t scratch_bytes, int *status,
+                         yvex_hip_stream stream, Publisher *publisher)
 {
     if (!values || !row_count || !row_width || !selected_tokens || !selected_values || !tie_counts ||
         !status)
@@ -290,6 +303,10 @@ extern "C" int yvex_hip_argmax_f32(const float *values, uint64_t row_count, uint
     if (((uintptr_t)values & 3u) || ((uintptr_t)scratch & 7u)) return ST_INVALID_ARG;
     const uint64_t need = yvex_hip_argmax_scratch_bytes(row_count, row_width);
     hipStream_t s = as_stream(stream);
+    // (what crosses to the host is bounded like what a publishing launch of its own brings there)
+    if (row_count * 16u > YVEX_HIP_PUBLISH_MAX_BYTES) publisher = nullptr;
+    const Selection selection{selected_tokens, selected_values, (unsigned long long *)tie_counts, row_count,
+                              take_publication(publisher, row_count)};
     if (need && scratch && scratch_bytes >= need) {
         const unsigned spans = (unsigned)((row_width + kSpanElements - 1u) / kSpanElements);
         argmax_spans_kernel<<<dim3(spans, (unsigned)row_count), kSpanThreads, 0, s>>>(
@@ -297,14 +314,33 @@ extern "C" int yvex_hip_argmax_f32(const float *values, uint64_t row_count, uint
         int rc = check_launch("argmax_f32.spans");
         if (rc) return rc;
         argmax_merge_kernel<<<(unsigned)row_count, 64, 0, s>>>(
-            (const SpanResult *)scratch, spans, row_count, selected_tokens, selected_values,
-            (unsigned long long *)tie_counts);
+            (const SpanResult *)scratch, spans, selection, status);
         return check_launch("argmax_f32.merge");
     }
     argmax_rows_kernel<<<(unsigned)row_count, kSelectThreads, 0, s>>>(
-        values, row_count, row_width, selected_tokens, selected_values,
-        (unsigned long long *)tie_counts, status);
+        values, row_width, selection, status);
     return check_launch("argmax_f32");
+}
+
+extern "C" int yvex_hip_argmax_f32(const float *values, uint64_t row_count, uint64_t row_width,
+                                   uint32_t *selected_tokens, float *selected_values,
+                                   uint64_t *tie_counts, void *scratch, uint64_t scratch_bytes,
+                                   int *status, yvex_hip_stream stream)
+{
+    return launch_argmax(values, row_count, row_width, selected_tokens, selected_values, tie_counts, scratch, scratch_bytes,
+                         status, stream, nullptr);
+}
+
+int yvex_hip_argmax_f32_publishing(const float *values, uint64_t row_count, uint64_t row_width, uint32_t *selected_tokens,
+                                   float *selected_values, uint64_t *tie_counts, void *scratch, uint64_t scratch_bytes,
+                                   int *status, const yvex_hip_publication *publication, int *published,
+                                   yvex_hip_stream stream)
+{
+    Publisher publisher = publisher_of(*publication);
+    const int rc = launch_argmax(values, row_count, row_width, selected_tokens, selected_values, tie_counts, scratch,
+                                 scratch_bytes, status, stream, &publisher);
+    *published = publisher.taken;
+    return rc;
 }
 
 extern "C" uint64_t yvex_hip_argmax_static_capacity(void) { return sizeof(scratch); }

@@ -75,45 +75,57 @@ int yvex_rocm_status_reset(yvex_rocm_backend *backend, unsigned long long *launc
     return YVEX_OK;
 }
 
-static int finish(yvex_rocm_backend *backend, unsigned long long device_results, unsigned long long bytes,
-                  const unsigned char **results, int whole_phase, const char *where, int *device_status,
-                  yvex_error *err)
+static void publication_open(yvex_rocm_backend *backend, int whole_phase, yvex_hip_publication *publication)
 {
-    const int clear = backend->status_state == YVEX_ROCM_STATUS_OWNED && (whole_phase || !backend->pending_completion);
-    const unsigned int sequence = ++backend->published_sequence;
-    int rc;
+    publication->arrivals = backend->arrivals;
+    publication->host = (uint32_t *)backend->published;
+    publication->sequence = ++backend->published_sequence;
+    publication->clear = backend->status_state == YVEX_ROCM_STATUS_OWNED && (whole_phase || !backend->pending_completion);
+}
+
+void yvex_rocm_publication_open(yvex_rocm_backend *backend, yvex_hip_publication *publication)
+{
+    publication_open(backend, 0, publication);
+}
+
+int yvex_rocm_finish_published(yvex_rocm_backend *backend, const yvex_hip_publication *publication, int published,
+                               unsigned long long device_results, unsigned long long bytes, const unsigned char **results,
+                               const char *where, int *device_status, yvex_error *err)
+{
+    int rc = 0;
     *device_status = 0;
     if (results) *results = NULL;
     if (yvex_rocm_seam("YVEX_TEST_ROCM_SYNC_FAILURE"))
         return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, where, "synchronisation failed (test seam)");
-    rc = yvex_hip_publish((const void *)(uintptr_t)device_results, bytes, backend->device_status, clear,
-                          backend->published, sequence, backend->stream);
-    if (rc == 0) rc = yvex_hip_await(backend->published, sequence, device_status, backend->stream);
+    if (!published)
+        rc = yvex_hip_publish((const void *)(uintptr_t)device_results, bytes, backend->device_status, publication->clear,
+                              backend->published, publication->sequence, backend->stream);
+    if (rc == 0) rc = yvex_hip_await(backend->published, publication->sequence, device_status, backend->stream);
     if (rc != 0) {
         backend->status = YVEX_BACKEND_STATUS_FAILED;
         return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, where, yvex_hip_last_error());
     }
-    if (clear) backend->status_state = YVEX_ROCM_STATUS_CLEAN;
+    if (publication->clear) backend->status_state = YVEX_ROCM_STATUS_CLEAN;
     if (results) *results = backend->published + YVEX_HIP_PUBLISH_HEAD_BYTES;
     backend->memory.d2h_bytes += sizeof(int);
     return YVEX_OK;
 }
 
-int yvex_rocm_finish(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err)
+static int finish(yvex_rocm_backend *backend, int whole_phase, const char *where, int *device_status, yvex_error *err)
 {
-    return finish(backend, 0ull, 0ull, NULL, 0, where, device_status, err);
+    yvex_hip_publication publication;
+    publication_open(backend, whole_phase, &publication);
+    return yvex_rocm_finish_published(backend, &publication, 0, 0ull, 0ull, NULL, where, device_status, err);
 }
 
-int yvex_rocm_finish_results(yvex_rocm_backend *backend, unsigned long long device_results, unsigned long long bytes,
-                             const unsigned char **results, const char *where, int *device_status,
-                             yvex_error *err)
+int yvex_rocm_finish(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err)
 {
-    return finish(backend, device_results, bytes, results, 0, where, device_status, err);
+    return finish(backend, 0, where, device_status, err);
 }
 
 int yvex_rocm_finish_phase(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err)
 {
-    return finish(backend, 0ull, 0ull, NULL, 1, where, device_status, err);
+    return finish(backend, 1, where, device_status, err);
 }
 
 int yvex_rocm_upload_queued(yvex_rocm_backend *backend, void *device, const void *host,
@@ -148,10 +160,12 @@ int yvex_rocm_upload_queued(yvex_rocm_backend *backend, void *device, const void
 
 /* What every session has of its own on the device: a stream, a status word, and pinned memory for
  * what its synchronous operations publish. Released again where any of it is missing. */
+enum { SESSION_WORDS_BYTES = 256 + YVEX_HIP_ARRIVAL_BYTES };     /* the status word, then the counters */
+
 static int session_open(yvex_rocm_backend *backend)
 {
     void *status_word = NULL, *published = NULL;
-    if (yvex_hip_stream_create(&backend->stream) != 0 || yvex_hip_malloc(&status_word, 256u) != 0 ||
+    if (yvex_hip_stream_create(&backend->stream) != 0 || yvex_hip_malloc(&status_word, SESSION_WORDS_BYTES) != 0 ||
         yvex_hip_host_alloc(&published, YVEX_HIP_PUBLISH_HEAD_BYTES + YVEX_HIP_PUBLISH_MAX_BYTES) != 0) {
         if (status_word) (void)yvex_hip_free(status_word);
         if (backend->stream) (void)yvex_hip_stream_destroy(backend->stream);
@@ -159,6 +173,7 @@ static int session_open(yvex_rocm_backend *backend)
     }
     memset(published, 0, YVEX_HIP_PUBLISH_HEAD_BYTES);
     backend->device_status = (int *)status_word;
+    backend->arrivals = (uint32_t *)((unsigned char *)status_word + 256u);
     backend->published = (unsigned char *)published;
     return 1;
 }
@@ -206,7 +221,7 @@ int yvex_rocm_backend_open(yvex_rocm_backend **out, const yvex_backend_options *
         backend->kernels_available = !yvex_rocm_seam("YVEX_TEST_ROCM_BUNDLE_FAILURE") &&
                                      strncmp(arch, "gfx950", 6) == 0 && yvex_hip_kernels_loadable();
         if (backend->kernels_available &&
-            (yvex_hip_fill_u32(backend->device_status, 0u, 1u, backend->stream) != 0 ||
+            (yvex_hip_fill_u32(backend->device_status, 0u, SESSION_WORDS_BYTES / 4u, backend->stream) != 0 ||
              yvex_hip_stream_sync(backend->stream) != 0))
             backend->kernels_available = 0;
         backend->status_state = backend->kernels_available ? YVEX_ROCM_STATUS_CLEAN : YVEX_ROCM_STATUS_UNKNOWN;
@@ -253,7 +268,7 @@ int yvex_rocm_backend_open_shared(yvex_rocm_backend **out, yvex_rocm_backend *co
         }
         backend->kernels_available = context_owner->kernels_available;
         if (backend->kernels_available &&
-            (yvex_hip_fill_u32(backend->device_status, 0u, 1u, backend->stream) != 0 ||
+            (yvex_hip_fill_u32(backend->device_status, 0u, SESSION_WORDS_BYTES / 4u, backend->stream) != 0 ||
              yvex_hip_stream_sync(backend->stream) != 0))
             backend->kernels_available = 0;
         backend->status_state = backend->kernels_available ? YVEX_ROCM_STATUS_CLEAN : YVEX_ROCM_STATUS_UNKNOWN;

@@ -8,6 +8,7 @@
 
 #include "yvex_rocm.h"
 #include "yvex_rocm_kernels.h"
+#include "publication.h"
 
 struct yvex_rocm_backend {
     yvex_backend_kind kind;
@@ -33,6 +34,7 @@ struct yvex_rocm_backend {
     unsigned long long workspace_bytes, workspace_cursor;
     /* device status word shared by the operations of this backend */
     int *device_status;
+    uint32_t *arrivals;        /* counters of launches that publish by themselves, in the word's allocation */
     int status_state;          /* YVEX_ROCM_STATUS_*: what the host knows of the word */
     int pending_completion;
     /* pinned host memory that a synchronous operation's last launch publishes its status word and
@@ -76,11 +78,14 @@ enum {
 /* Wait for the stream's work and read the device status word. The word is cleared where the waiting
  * operation owns it and no deferred row batches are waiting for their barrier, and left as it is else. */
 int yvex_rocm_finish(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err);
-/* The same for an operation with small results: `bytes` of device memory (a multiple of 4, at most
- * YVEX_HIP_PUBLISH_MAX_BYTES) arrive in *results, host memory that is good until the next such call. */
-int yvex_rocm_finish_results(yvex_rocm_backend *backend, unsigned long long device_results, unsigned long long bytes,
-                             const unsigned char **results, const char *where, int *device_status,
-                             yvex_error *err);
+/* The same for an operation whose last launch may publish by itself and may have small results: `publication` is what that
+ * launch takes, filled in ahead of it and behind the status word's reset, `published` says whether it did, and `bytes` of
+ * device memory (a multiple of 4, at most YVEX_HIP_PUBLISH_MAX_BYTES) arrive in *results, host memory that is good
+ * until the next such call. */
+void yvex_rocm_publication_open(yvex_rocm_backend *backend, yvex_hip_publication *publication);
+int yvex_rocm_finish_published(yvex_rocm_backend *backend, const yvex_hip_publication *publication, int published,
+                               unsigned long long device_results, unsigned long long bytes, const unsigned char **results,
+                               const char *where, int *device_status, yvex_error *err);
 /* The barrier of a phase of deferred row batches: the word they share is cleared where the phase still
  * owns it. */
 int yvex_rocm_finish_phase(yvex_rocm_backend *backend, const char *where, int *device_status, yvex_error *err);

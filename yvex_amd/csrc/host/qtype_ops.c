@@ -54,7 +54,8 @@ int yvex_rocm_encoded_matvec(
     unsigned long long total_bytes, q8_bytes = 0ull, q8_address = 0ull, launches = 0ull;
     unsigned long long head_bytes, tail_bytes = 0ull, joined_bytes = 0ull, joined_address = 0ull;
     const void *activations;
-    int q8_path, device_status = 0, rc, split_input = input_tail != NULL;
+    yvex_hip_publication publication;
+    int q8_path, device_status = 0, rc, split_input = input_tail != NULL, published = 0;
     if (facts) memset(facts, 0, sizeof(*facts));
     if (activation_q8 != 0 && activation_q8 != 1)
         return yvex_rocm_refuse(err, YVEX_ERR_INVALID_ARG, "rocm.encoded-matvec.activation",
@@ -113,6 +114,7 @@ int yvex_rocm_encoded_matvec(
         return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, "rocm.encoded-matvec.launch",
                                 "kernel launch failed (test seam)");
     rc = yvex_rocm_status_reset(backend, NULL, where, err);
+    yvex_rocm_publication_open(backend, &publication);
     activations = input->data;
     if (rc == YVEX_OK && split_input) {
         rc = yvex_rocm_launch_result(
@@ -128,10 +130,11 @@ int yvex_rocm_encoded_matvec(
         (const uint8_t *)(uintptr_t)device_address, qtype, row_count, row_width, row_bytes, input_rows);
     if (rc == YVEX_OK && quantizing) {
         rc = yvex_rocm_launch_result(
-            yvex_hip_matvec_quantizing((const uint8_t *)(uintptr_t)device_address, qtype, row_count, row_width, row_bytes,
-                                       (const float *)input->data, input_rows, row_width,
-                                       additive ? (const float *)additive->data : NULL, (float *)output->data, row_count, 0,
-                                       backend->device_status, backend->stream),
+            yvex_hip_matvec_quantizing_publishing((const uint8_t *)(uintptr_t)device_address, qtype, row_count, row_width,
+                                                  row_bytes, (const float *)input->data, input_rows, row_width,
+                                                  additive ? (const float *)additive->data : NULL, (float *)output->data,
+                                                  row_count, 0, backend->device_status, &publication, &published,
+                                                  backend->stream),
             "rocm.encoded-matvec.launch", err);
         if (rc == YVEX_OK) launches++;
     }
@@ -145,21 +148,24 @@ int yvex_rocm_encoded_matvec(
     }
     if (rc == YVEX_OK && !quantizing) {
         rc = yvex_rocm_launch_result(
-            yvex_hip_matvec((const uint8_t *)(uintptr_t)device_address, qtype, row_count, row_width,
-                            row_bytes, q8_path ? (const void *)(uintptr_t)q8_address : activations,
-                            q8_path, input_rows, row_width, additive ? (const float *)additive->data : NULL,
-                            (float *)output->data, row_count, 0, backend->device_status, backend->stream),
+            yvex_hip_matvec_publishing((const uint8_t *)(uintptr_t)device_address, qtype, row_count, row_width,
+                                       row_bytes, q8_path ? (const void *)(uintptr_t)q8_address : activations,
+                                       q8_path, input_rows, row_width, additive ? (const float *)additive->data : NULL,
+                                       (float *)output->data, row_count, 0, backend->device_status, &publication,
+                                       &published, backend->stream),
             "rocm.encoded-matvec.launch", err);
         if (rc == YVEX_OK) launches++;
     }
-    if (rc == YVEX_OK) rc = yvex_rocm_finish(backend, "rocm.encoded-matvec.sync", &device_status, err);
+    if (rc == YVEX_OK)
+        rc = yvex_rocm_finish_published(backend, &publication, published, 0ull, 0ull, NULL, "rocm.encoded-matvec.sync",
+                                        &device_status, err);
     if (rc == YVEX_OK && device_status)
         rc = yvex_rocm_refuse(err, YVEX_ERR_FORMAT, where,
                               "encoded projection produced invalid numerics");
     if (rc != YVEX_OK) return rc;
     output->is_written = 1;
     facts->d2h_bytes = sizeof(int);
-    facts->kernel_launches = launches + 1ull;   /* the status word's included */
+    facts->kernel_launches = launches + (published ? 0ull : 1ull);   /* the status word's, where it took one */
     facts->download_count = 1ull;
     facts->stream_synchronizations = 1ull;
     facts->active_weight_bytes = encoded_bytes;

@@ -29,7 +29,8 @@ int yvex_rocm_select_greedy_rows(
     unsigned long long value_count, value_bytes, token_bytes, selected_bytes, tie_bytes;
     unsigned long long temporary_bytes, tokens_device = 0ull, values_device = 0ull, ties_device = 0ull, row;
     unsigned long long scratch_bytes, scratch_device = 0ull;
-    int device_status = 0, rc;
+    yvex_hip_publication publication;
+    int device_status = 0, rc, published = 0;
     if (facts) memset(facts, 0, sizeof(*facts));
     if (!backend || backend->kind != YVEX_BACKEND_KIND_ROCM || !logits || !selected_tokens ||
         !selected_values || !tie_counts || !facts || !row_count || !row_width ||
@@ -66,18 +67,21 @@ int yvex_rocm_select_greedy_rows(
         return yvex_rocm_refuse(err, YVEX_ERR_BACKEND, "rocm.sampling.greedy.launch",
                                 "kernel launch failed (test seam)");
     rc = yvex_rocm_status_reset(backend, NULL, where, err);
+    yvex_rocm_publication_open(backend, &publication);
     if (rc == YVEX_OK)
         rc = yvex_rocm_launch_result(
-            yvex_hip_argmax_f32((const float *)logits->data, row_count, row_width,
-                                (uint32_t *)(uintptr_t)tokens_device, (float *)(uintptr_t)values_device,
-                                (uint64_t *)(uintptr_t)ties_device, (void *)(uintptr_t)scratch_device,
-                                scratch_bytes, backend->device_status, backend->stream),
+            yvex_hip_argmax_f32_publishing((const float *)logits->data, row_count, row_width,
+                                           (uint32_t *)(uintptr_t)tokens_device, (float *)(uintptr_t)values_device,
+                                           (uint64_t *)(uintptr_t)ties_device, (void *)(uintptr_t)scratch_device,
+                                           scratch_bytes, backend->device_status, &publication, &published,
+                                           backend->stream),
             "rocm.sampling.greedy.launch", err);
     if (tie_bytes + token_bytes + selected_bytes <= YVEX_HIP_PUBLISH_MAX_BYTES) {
         const unsigned char *results = NULL;
         if (rc == YVEX_OK)
-            rc = yvex_rocm_finish_results(backend, ties_device, tie_bytes + token_bytes + selected_bytes, &results,
-                                          "rocm.sampling.greedy.sync", &device_status, err);
+            rc = yvex_rocm_finish_published(backend, &publication, published, ties_device,
+                                            tie_bytes + token_bytes + selected_bytes, &results,
+                                            "rocm.sampling.greedy.sync", &device_status, err);
         if (rc == YVEX_OK) {
             memcpy(tie_counts, results, (size_t)tie_bytes);
             memcpy(selected_tokens, results + tie_bytes, (size_t)token_bytes);
@@ -93,7 +97,8 @@ int yvex_rocm_select_greedy_rows(
         READ(tie_counts, ties_device, tie_bytes);
 #undef READ
         if (rc == YVEX_OK)
-            rc = yvex_rocm_finish(backend, "rocm.sampling.greedy.sync", &device_status, err);
+            rc = yvex_rocm_finish_published(backend, &publication, published, 0ull, 0ull, NULL,
+                                            "rocm.sampling.greedy.sync", &device_status, err);
     }
     for (row = 0ull; rc == YVEX_OK && row < row_count; ++row)
         if (device_status || selected_tokens[row] >= row_width || !isfinite(selected_values[row]) ||
