@@ -1,0 +1,49 @@
+"""Superblock sums, scales and minimums at the ends of their ranges: the matrix-core kernels publish what
+the sweeps and the generic kernel (the CPU path's bits) publish for the same pairs."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(array, device):
+    return torch.from_numpy(np.ascontiguousarray(array)).to(device)
+
+
+# both token blocks of a tile, one, a tile of one pair more than the few-pair kernels take, and a remainder of theirs
+POPULATIONS = [64 + 40, 33, 17, 5]
+
+
+@pytest.mark.parametrize("qtype", ["Q4_K", "Q2_K"])
+@pytest.mark.parametrize("scales,magnitude", [("ordinary", 1.0), ("largest", 2.0 ** 80), ("subnormal", 2.0 ** -108)])
+def test_scales_and_minimums_reach_as_far_as_floats(gpu, oracle, qtype, scales, magnitude):
+    """Sub-block scales and minimums at their largest against rows whose codes all have the largest magnitude and one sign,
+    (the largest sums there are), with block scales whose products are ordinary, huge or denormal."""
+    from yvex_amd import kernels as K
+    qt, hidden, intermediate = getattr(oracle, qtype), 256, 512
+    block, heads = {"Q4_K": (144, slice(4, 16)), "Q2_K": (84, slice(0, 16))}[qtype]
+    at = 0 if qtype == "Q4_K" else 80
+    experts, pairs = len(POPULATIONS), sum(POPULATIONS)
+    g = oracle.Generator(45, f"limits.{qtype}")
+    up = dev(g.weights(oracle.Q4_K, experts * intermediate, hidden), gpu)
+    down = g.weights(qt, experts * hidden, intermediate)
+    blocks = down.reshape(-1, block)
+    blocks[::2, heads] = 255
+    if scales != "ordinary":
+        bits = (np.full(len(blocks), 0x7800) if scales == "largest" else 1 + np.arange(len(blocks)) * 7 % 1023).astype(np.uint16)
+        for offset in (at, at + 2):
+            blocks[:, offset], blocks[:, offset + 1] = bits & 255, bits >> 8
+    weights = K.expert_weights(up, up, dev(down, gpu), (oracle.Q4_K, oracle.Q4_K, qt), hidden, intermediate)
+    status = K.new_status(gpu)
+    selected = torch.repeat_interleave(torch.arange(experts), torch.tensor(POPULATIONS)).reshape(pairs, 1).to(gpu)
+    wl = K.worklist_build(selected, experts, status)
+    x = g.normal(pairs * intermediate).reshape(pairs, intermediate)
+    x[::3], x[1::3] = 1.0, -1.0
+    x = (x / np.abs(x).max(axis=1, keepdims=True) * magnitude).astype(np.float32)
+    act = K.q8k_quantize(dev(x, gpu), status)
+    out = [torch.full((pairs, hidden), float("nan"), device=gpu) for _ in range(2)]
+    K.moe_down(weights, act, True, wl, pairs, experts, out[0], status)
+    K.moe_down_rows(weights, act, wl, pairs, experts, out[1], status)
+    assert int(status.item()) == 0 and bool(torch.isfinite(out[0]).all())
+    assert torch.equal(out[0].view(torch.int32), out[1].view(torch.int32))

@@ -9,13 +9,12 @@ namespace yvex {
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 // Two int8 limbs of sc * nibble for the four nibbles of one dword, value = 8 hi + lo (see
-// dense_q4k.hip).
-__device__ __forceinline__ void q4k_limbs(unsigned x, unsigned sc, unsigned &lo, unsigned &hi)
+// dense_q4k.hip): sc = 8 high + low.
+__device__ __forceinline__ void q4k_limbs(unsigned x, unsigned short low, unsigned short high, unsigned &lo, unsigned &hi)
 {
     const unsigned nibbles = x & 0x0f0f0f0fu;
-    const unsigned low = (sc & 7u) * 0x00010001u, high = ((sc >> 3) & 7u) * 0x00010001u;
-    lo = __builtin_bit_cast(unsigned, __builtin_bit_cast(u16x2, nibbles) * __builtin_bit_cast(u16x2, low));
-    hi = __builtin_bit_cast(unsigned, __builtin_bit_cast(u16x2, nibbles) * __builtin_bit_cast(u16x2, high));
+    lo = __builtin_bit_cast(unsigned, __builtin_bit_cast(u16x2, nibbles) * u16x2{low, low});
+    hi = __builtin_bit_cast(unsigned, __builtin_bit_cast(u16x2, nibbles) * u16x2{high, high});
 }
 
 // Pair sums of the 16 int16 block sums as two int8 limbs (value = 128 hi + lo, lo in 0..127).
@@ -33,26 +32,58 @@ __device__ __forceinline__ void q4k_bsum_limbs(const uint4 (&b)[2], uint2 &lo, u
     hi = make_uint2(u[0], u[1]);
 }
 
-// The sixteen int16 block sums as two int8 limbs (value = 128 hi + lo, lo in 0..127), in order.
-__device__ __forceinline__ void q2k_bsum_limbs(const uint4 (&b)[2], v4i &lo, v4i &hi)
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
+static_assert(sizeof(f16x8) == 16, "an operand of a matrix instruction");
+
+// Minimum terms on the f16 matrix instructions. A minimum is at most 63 and a sum of sixteen int8 values at
+// most 2048 in magnitude, both whole numbers that f16 holds; their products and sums stay below 2^21, so the float a matrix
+// core publishes is the exact sum, with nothing to join or convert.
+
+// Eight bytes (at most 127) as f16: the byte below the high byte of 1024.0 is 1024 + byte.
+__device__ __forceinline__ f16x8 bytes_to_f16(unsigned first, unsigned second)
 {
-    const unsigned w[8] = {b[0].x, b[0].y, b[0].z, b[0].w, b[1].x, b[1].y, b[1].z, b[1].w};
+    const f16x2 bias = {(_Float16)1024.0f, (_Float16)1024.0f};
+    f16x2 pair[4];
 #pragma unroll
     for (unsigned i = 0; i < 4u; ++i) {
-        unsigned l = 0u, u = 0u;
-#pragma unroll
-        for (unsigned k = 0; k < 4u; ++k) {
-            const unsigned word = w[2u * i + k / 2u];
-            const int sum = k % 2u ? (int)word >> 16 : (int)(short)(word & 0xffffu);
-            l |= ((unsigned)sum & 127u) << (8u * k);
-            u |= ((unsigned)(sum >> 7) & 255u) << (8u * k);
-        }
-        lo[i] = (int)l;
-        hi[i] = (int)u;
+        const unsigned bits = __builtin_amdgcn_perm(0x64646464u, i < 2u ? first : second, i & 1u ? 0x04030402u : 0x04010400u);
+        pair[i] = __builtin_bit_cast(f16x2, bits) - bias;
     }
+    return f16x8{pair[0][0], pair[0][1], pair[1][0], pair[1][1], pair[2][0], pair[2][1], pair[3][0], pair[3][1]};
 }
 
-// The same sums as operands whose products with {m, 8 m, 8 m} add up to m * sum in one sum: the low
+// Q4_K: a minimum per 32 values. The sums of two neighbours (at most 4096 in magnitude) in two parts f16 holds, each on
+// half of the K step: multiples of 32 for lanes of half 0, what is left for those of half 1.
+__device__ __forceinline__ f16x8 q4k_bsum_operand(const uint4 &b0, const uint4 &b1, unsigned half)
+{
+    const unsigned w[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+    const int part = half ? 31 : ~31;
+    f16x8 out;
+#pragma unroll
+    for (unsigned s = 0; s < 8u; ++s) {
+        const int pair = (int)(short)(w[s] & 0xffffu) + ((int)w[s] >> 16);
+        out[s] = (_Float16)(short)(pair & part);
+    }
+    return out;
+}
+
+// Q2_K: a minimum per 16 values, eight of the sixteen sums a lane.
+__device__ __forceinline__ f16x8 q2k_bsum_operand(const uint4 &b)
+{
+    const unsigned w[4] = {b.x, b.y, b.z, b.w};
+    f16x8 out;
+#pragma unroll
+    for (unsigned s = 0; s < 4u; ++s) {
+        out[2u * s] = (_Float16)(short)(w[s] & 0xffffu);
+        out[2u * s + 1u] = (_Float16)(short)(w[s] >> 16);
+    }
+    return out;
+}
+
+// The sixteen int16 block sums as operands whose products with {m, 8 m, 8 m} add up to m * sum in one sum: the low
 // three bits, and the rest (-256 .. 254) in two halves that fit int8.
 __device__ __forceinline__ void q2k_bsum_pieces(const uint4 (&b)[2], v4i (&piece)[3])
 {

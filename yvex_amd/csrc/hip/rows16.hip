@@ -699,7 +699,8 @@ __global__ __launch_bounds__((Map16<QT, S>::kThreads)) void rows16_kernel(Rows16
 #pragma unroll
                             for (unsigned i = 0; i < 4u; ++i) {
                                 unsigned low_limbs, high_limbs;
-                                q4k_limbs((unsigned)w[u].codes[m & 1u][i] >> (4u * (m >> 1)), sc, low_limbs, high_limbs);
+                                q4k_limbs((unsigned)w[u].codes[m & 1u][i] >> (4u * (m >> 1)), (unsigned short)(sc & 7u),
+                                          (unsigned short)(sc >> 3), low_limbs, high_limbs);
                                 a_lo[i] = (int)low_limbs;
                                 a_hi[i] = (int)high_limbs;
                             }

@@ -4,12 +4,21 @@
 //
 // Arithmetic per 256-value superblock as in dense_q4k.hip: the weight operand carries
 // sc_j * nibble as two int8 limbs of base 8, one K step of V_MFMA_I32_32X32X32_I8 is one 32-value
-// sub-block, the int32 accumulators run over the whole superblock, the minimum term is one more
-// K step of depth 8, and
+// sub-block, the int32 accumulators run over the whole superblock, and
 //     value = (d_a * d) * float(dot) - (d_a * dmin) * float(minimum)
 // (a float, every operation rounded) is added to the row sums in double, superblock by
 // superblock, and a sum is rounded to float once when it is published: the row dot the CPU path
 // forms (double accumulation over a row's blocks, src/gguf/quant_compute.c:152-172).
+//
+// The vector ALU is what these kernels wait for first, and half of what it did was that line, so
+// all of it that is a product of a row's and a token's number runs on the matrix cores, which had
+// two thirds of their time left: the minimum term is one K step on f16 operands, whose float sums
+// are exact (kquant_limbs.hpp; on int8 limbs it took an instruction to join them and one to convert), and
+// d_a d and d_a dmin are the two outer products of one V_MFMA_F32_32X32X1_2B_F32: a product
+// of two floats rounded once, bit for bit what V_MUL_F32 gives (denormals and infinities too), and
+// the row scales need no place in LDS. The sums are kept from being rounded in every turn of the loop
+// for the sake of its last (what the compiler made of it). 600 -> 453 vector instructions a superblock and wave of 64 tokens; 1111
+// rows of 7168 by eight of 256 Q4_K experts with uneven routing 2530 -> 2213 us.
 //
 // What differs is how the operands arrive. A lane that fetches its own 16-byte pieces of a
 // 144-byte weight block and of a 292-byte activation block touches up to 64 cache lines per load
@@ -35,8 +44,7 @@
 // tensor-core down kernel serves this format only, src/backend/cuda/tensorcore.cu:628-702) run
 // through the same tiles, copies and publication. Their operand is simpler: a 2-bit code times its
 // sub-block's 4-bit scale is at most 45, one int8 limb, so a K step (two 16-value sub-blocks) is
-// one matrix instruction a token block; the minimum term is a K step of depth 16 against the
-// Q8_K block's sixteen sums; rows are copied as dwords (84-byte superblocks), pitch 21 dwords.
+// one matrix instruction a token block; the minimum term is a K step of the Q8_K block's sixteen sums; rows are copied as dwords (84-byte superblocks), pitch 21 dwords.
 #include "common.hpp"
 #include "launch.hpp"
 #include "grouped.hpp"
@@ -63,8 +71,7 @@ constexpr unsigned kQ4WeightBase = 0u;                                          
 constexpr unsigned kQ4ActBase = kQ4WeightBase + kQ4Waves * 2u * kQ4WeightBytes; // [buffer][token][256]
 constexpr unsigned kQ4ScaleBase = kQ4ActBase + 2u * kQ4Tokens * 256u;           // [buffer][token] f32
 constexpr unsigned kQ4BsumBase = kQ4ScaleBase + 2u * kQ4Tokens * 4u;            // [buffer][token][32]
-constexpr unsigned kQ4RowScaleBase = kQ4BsumBase + 2u * kQ4Tokens * 32u;        // [wave][d, dmin][32] f32
-constexpr unsigned kQ4MetaBase = kQ4RowScaleBase + kQ4Waves * 2u * 32u * 4u;    // tile lookup
+constexpr unsigned kQ4MetaBase = kQ4BsumBase + 2u * kQ4Tokens * 32u;            // tile lookup
 constexpr unsigned kQ4TrashBase = kQ4MetaBase + 64u;                            // 1 KB nobody reads
 constexpr unsigned kQ4LdsBytes = kQ4TrashBase + 1024u;
 
@@ -191,7 +198,6 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
 
-    const unsigned row_scale_at = kQ4RowScaleBase + wave * 256u;
     for (unsigned sb = 0; sb < g.blocks; ++sb) {
         const unsigned buffer = sb & 1u;
         if (sb + 1u < g.blocks) copies(sb + 1u);
@@ -204,7 +210,8 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
         for (unsigned nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int i = 0; i < 16; ++i) lo_sum[nt][i] = hi_sum[nt][i] = 0;
-        v4i m_op = {0, 0, 0, 0};         // the minimums of the row's sub-blocks, on the h = 0 half
+        f16x8 m_op;                      // the minimums of the row's sub-blocks: their K step's operand
+        unsigned scales16;               // d | dmin << 16
         if constexpr (QT == QT_Q2_K) {
             // Public ggml block_q2_K (src/backend/cuda/kernel_primitives.h:314-341 is the product):
             // sixteen bytes (scale | minimum << 4) of the 16-value sub-blocks, 64 bytes of 2-bit
@@ -214,13 +221,10 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
             // instruction per step and token block.
             const unsigned scale_words[4] = {lds_read_u32(w_at), lds_read_u32(w_at + 4u), lds_read_u32(w_at + 8u),
                                              lds_read_u32(w_at + 12u)};
-            const unsigned dd = lds_read_u32(w_at + 80u);
-            if (h == 0u) {
-                lds_write_u32(row_scale_at + 4u * r, __float_as_uint(f16_bits_to_float(dd & 0xffffu)));
-                lds_write_u32(row_scale_at + 128u + 4u * r, __float_as_uint(f16_bits_to_float(dd >> 16)));
-#pragma unroll
-                for (unsigned i = 0; i < 4u; ++i) m_op[i] = (int)((scale_words[i] >> 4) & 0x0f0f0f0fu);
-            }
+            scales16 = lds_read_u32(w_at + 80u);
+            // lane (r, h): the minimums of sub-blocks 8 h .. 8 h + 7
+            m_op = bytes_to_f16((h ? scale_words[2] : scale_words[0]) >> 4 & 0x0f0f0f0fu,
+                                (h ? scale_words[3] : scale_words[1]) >> 4 & 0x0f0f0f0fu);
 #pragma unroll
             for (unsigned p = 0; p < 2u; ++p) {
                 unsigned q[4];
@@ -246,27 +250,25 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
             const unsigned s0 = head.y, s1 = head.z, s2 = head.w;
             const unsigned sc_pack[2] = {s0 & 0x3f3f3f3fu, (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u)};
             const unsigned mn_pack[2] = {s1 & 0x3f3f3f3fu, ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u)};
-            if (h == 0u) {
-                lds_write_u32(row_scale_at + 4u * r, __float_as_uint(f16_bits_to_float(head.x & 0xffffu)));
-                lds_write_u32(row_scale_at + 128u + 4u * r, __float_as_uint(f16_bits_to_float(head.x >> 16)));
-                // minimum term: m_j (bytes 0..7 of the h = 0 half, zeros elsewhere) against the pair sums
-                m_op[0] = (int)mn_pack[0];
-                m_op[1] = (int)mn_pack[1];
-            }
+            const unsigned sc_low[2] = {sc_pack[0] & 0x07070707u, sc_pack[1] & 0x07070707u};
+            const unsigned sc_high[2] = {sc_pack[0] >> 3 & 0x07070707u, sc_pack[1] >> 3 & 0x07070707u};
+            scales16 = head.x;
+            m_op = bytes_to_f16(mn_pack[0], mn_pack[1]);     // the same on both halves, against the two parts of the sums
 #pragma unroll
             for (unsigned j = 0; j < 4u; ++j) {
                 const uint4 q = read16(w_at + 16u + 32u * j + 16u * h);
 #pragma unroll
                 for (unsigned half = 0; half < 2u; ++half) {
                     const unsigned c = 2u * j + half;
-                    const unsigned sc = (sc_pack[c >> 2] >> (8u * (c & 3u))) & 255u;
+                    const unsigned short low = (unsigned short)(sc_low[c >> 2] >> (8u * (c & 3u)) & 255u);
+                    const unsigned short high = (unsigned short)(sc_high[c >> 2] >> (8u * (c & 3u)) & 255u);
                     const unsigned shift = 4u * half;
                     v4i a_lo, a_hi;
                     unsigned lo, hi;
-                    q4k_limbs(q.x >> shift, sc, lo, hi); a_lo[0] = (int)lo; a_hi[0] = (int)hi;
-                    q4k_limbs(q.y >> shift, sc, lo, hi); a_lo[1] = (int)lo; a_hi[1] = (int)hi;
-                    q4k_limbs(q.z >> shift, sc, lo, hi); a_lo[2] = (int)lo; a_hi[2] = (int)hi;
-                    q4k_limbs(q.w >> shift, sc, lo, hi); a_lo[3] = (int)lo; a_hi[3] = (int)hi;
+                    q4k_limbs(q.x >> shift, low, high, lo, hi); a_lo[0] = (int)lo; a_hi[0] = (int)hi;
+                    q4k_limbs(q.y >> shift, low, high, lo, hi); a_lo[1] = (int)lo; a_hi[1] = (int)hi;
+                    q4k_limbs(q.z >> shift, low, high, lo, hi); a_lo[2] = (int)lo; a_hi[2] = (int)hi;
+                    q4k_limbs(q.w >> shift, low, high, lo, hi); a_lo[3] = (int)lo; a_hi[3] = (int)hi;
 #pragma unroll
                     for (unsigned nt = 0; nt < NT; ++nt) {
                         const v4i b = lds_read_v4i(a_at + nt * 32u * 256u + 16u * ((2u * c + h) ^ (r & 15u)));
@@ -276,53 +278,41 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
                 }
             }
         }
-        // d and dmin of the sixteen rows this lane accumulates (written above by the wave itself)
-        wave_lds_fence();
+        // Block scales (d in the h = 0 half, dmin in the other) against the tokens': a product of two
+        // floats rounded once is what the matrix core forms of one K step from zero.
+        const float row_scale = f16_bits_to_float(scales16 >> (16u * h) & 0xffffu);
 #pragma unroll
         for (unsigned nt = 0; nt < NT; ++nt) {
             const unsigned token = nt * 32u + r;
             const float da = __uint_as_float(lds_read_u32(kQ4ScaleBase + buffer * kQ4Tokens * 4u + 4u * token));
-            v4i b_lo = {0, 0, 0, 0}, b_hi = {0, 0, 0, 0};
-            if (h == 0u) {
-                const unsigned at = kQ4BsumBase + buffer * kQ4Tokens * 32u + 32u * token;
-                const uint4 bsums[2] = {read16(at), read16(at + 16u)};
-                if constexpr (QT == QT_Q2_K) {
-                    q2k_bsum_limbs(bsums, b_lo, b_hi);       // a minimum per 16 values: the sums as they are
-                } else {
-                    uint2 bl, bh;
-                    q4k_bsum_limbs(bsums, bl, bh);
-                    b_lo[0] = (int)bl.x; b_lo[1] = (int)bl.y;
-                    b_hi[0] = (int)bh.x; b_hi[1] = (int)bh.y;
-                }
-            }
-            v16i zero;
+            const unsigned at = kQ4BsumBase + buffer * kQ4Tokens * 32u + 32u * token;
+            f16x8 sums;
+            if constexpr (QT == QT_Q2_K) sums = q2k_bsum_operand(read16(at + 16u * h));  // a minimum per 16 values: the sums as they are
+            else sums = q4k_bsum_operand(read16(at), read16(at + 16u), h);
+            v16f zero16;
+            v32f zero32;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) zero[i] = 0;
-            const v16i min_lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(m_op, b_lo, zero, 0, 0, 0);
-            const v16i min_hi = __builtin_amdgcn_mfma_i32_32x32x32_i8(m_op, b_hi, zero, 0, 0, 0);
+            for (int i = 0; i < 16; ++i) zero16[i] = zero32[i] = zero32[i + 16] = 0.0f;
+            const v16f minimum = __builtin_amdgcn_mfma_f32_32x32x16_f16(m_op, sums, zero16, 0, 0, 0);
+            const v32f scale = __builtin_amdgcn_mfma_f32_32x32x1f32(row_scale, da, zero32, 0, 0, 0);
 #pragma unroll
-            for (unsigned q4 = 0; q4 < 4u; ++q4) {
-                const uint4 d = read16(row_scale_at + 4u * (8u * q4 + 4u * h));
-                const uint4 mn = read16(row_scale_at + 128u + 4u * (8u * q4 + 4u * h));
-                const float d_of[4] = {__uint_as_float(d.x), __uint_as_float(d.y), __uint_as_float(d.z),
-                                       __uint_as_float(d.w)};
-                const float dmin_of[4] = {__uint_as_float(mn.x), __uint_as_float(mn.y), __uint_as_float(mn.z),
-                                          __uint_as_float(mn.w)};
-#pragma unroll
-                for (unsigned k = 0; k < 4u; ++k) {
-                    const unsigned i = 4u * q4 + k;
-                    const int dot = QT == QT_Q2_K ? lo_sum[nt][i] : (hi_sum[nt][i] << 3) + lo_sum[nt][i];
-                    const int minimum = (min_hi[i] << 7) + min_lo[i];
-                    const float left = (da * d_of[k]) * (float)dot;
-                    const float right = (da * dmin_of[k]) * (float)minimum;
-                    acc[nt][i] += (double)(left - right);
-                }
+            for (unsigned i = 0; i < 16u; ++i) {
+                const int dot = QT == QT_Q2_K ? lo_sum[nt][i] : (hi_sum[nt][i] << 3) + lo_sum[nt][i];
+                const float left = scale[i] * (float)dot;
+                const float right = scale[i + 16u] * minimum[i];
+                acc[nt][i] += (double)(left - right);
             }
         }
         // the next superblock's copies have landed and every wave is done with this one's buffers
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
     }
+
+    // (the sums are rounded when they are published: the compiler would round them in every turn of the loop)
+#pragma unroll
+    for (unsigned nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (unsigned i = 0; i < 16u; ++i) asm volatile("" : "+v"(acc[nt][i]));
 
     // ---- publish: lane (token r, half h) holds rows 8 (i / 4) + 4 h + i % 4 of the wave's 32 ----
     // Four rows at a time, 16 bytes a lane where the output's geometry allows it (the two halves
