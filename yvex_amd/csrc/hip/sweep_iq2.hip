@@ -50,7 +50,7 @@ constexpr unsigned kSweepWaves = 8u;           // two per SIMD: the sweep of fou
 constexpr unsigned kSweepThreads = kSweepWaves * 64u;
 constexpr int kSweepPairs = 4;                 // pairs of one bucket served by one sweep
 constexpr int kSweepAheadSmall = 1;            // rows requested ahead of the one decoded, sweeps of one or two pairs
-constexpr unsigned kSweepChunkTurns = 16u;     // iterations a wave draws at a time (at most)
+constexpr unsigned kSweepChunkShift = 4u;      // iterations a wave draws at a time (at most), as a power of two
 
 // What a weight row costs a sweep that serves n pairs, relative to the other sweeps of the launch:
 // what the workgroups' pieces of a launch are measured in. Fitted to the times of the workgroups of
@@ -75,7 +75,9 @@ __device__ __forceinline__ unsigned bucket_cost(unsigned n)
 constexpr unsigned kMagBase = 0u;              // 256 entries x 16 replicas x {+lo, +hi, -lo, -hi}
 constexpr unsigned kSelBase = 65536u;          // 128 entries x 32 replicas x {selector lo, hi}
 constexpr unsigned kTicketAddress = kSelBase + 128u * 32u * 8u;   // work-item counter of the workgroup
-constexpr unsigned kParkBase = kTicketAddress + 32u;
+constexpr unsigned kPlaceAddress = kTicketAddress + 32u;          // what wave kPlacingWave found out for the workgroup
+constexpr unsigned kPlacingWave = 4u;
+constexpr unsigned kParkBase = kPlaceAddress + 32u;
 // Per wave: a window of kWindowLines lines of 64 float terms (one line per iteration and packed
 // value: even lanes' terms in the first 32 words, odd lanes' in the last 32, a weight row's
 // terms next to each other in superblock order), then the (gate, up) row sums of a fused item
@@ -89,7 +91,7 @@ constexpr unsigned kMaxSweeps = 4096u;
 // What opens an item without a round trip to memory: expert, first ordered pair and population of
 // every routed bucket, and {source pair, route weight} of every ordered pair when the routed
 // problem has at most kPairCacheMax of them (decode widths; wider batches read them from memory).
-constexpr unsigned kBucketBase = kParkBase + kSweepWaves * kParkBytes;     // 256 x {expert, first, population, sweeps before it}
+constexpr unsigned kBucketBase = kParkBase + kSweepWaves * kParkBytes;     // 256 x {expert, first, population, -}
 constexpr unsigned kPairCacheBase = kBucketBase + 256u * 16u;
 constexpr unsigned kPairCacheMax = 1024u;
 constexpr unsigned kSweepLdsBytes = kPairCacheBase + kPairCacheMax * 8u;
@@ -150,29 +152,30 @@ static_assert(kSweepThreads == 512u, "a thread a codebook entry, two a sign entr
 
 __device__ __forceinline__ unsigned sweep_table_digits() { return k_iq2_digits[threadIdx.x & 255u]; }
 
-__device__ __forceinline__ void sweep_tables_fill(unsigned digits)
+__device__ __forceinline__ void sweep_levels_fill(unsigned digits)       // threads 0 .. 255
 {
-    if (threadIdx.x < 256u) {
-        const uint2 m = iq2_magnitude_of_digits(digits);
-        // byte-wise negation: every level is >= 8, so (x ^ 0xff) + 1 never carries
-        const uint4 entry = make_uint4(m.x, m.y, (m.x ^ 0xffffffffu) + 0x01010101u, (m.y ^ 0xffffffffu) + 0x01010101u);
+    const uint2 m = iq2_magnitude_of_digits(digits);
+    // byte-wise negation: every level is >= 8, so (x ^ 0xff) + 1 never carries
+    const uint4 entry = make_uint4(m.x, m.y, (m.x ^ 0xffffffffu) + 0x01010101u, (m.y ^ 0xffffffffu) + 0x01010101u);
 #pragma unroll 4
-        for (unsigned t = 0; t < 16u; ++t)
-            lds_store_uint4(kMagBase + threadIdx.x * 256u + ((threadIdx.x + t) & 15u) * 16u, entry);
-    } else {
-        const unsigned s7 = (threadIdx.x - 256u) >> 1, upper = threadIdx.x & 1u;
-        const unsigned s = s7 | ((__popc(s7) & 1u) << 7);
-        // selector byte k = k (take +level, source 1) or k + 4 (take -level, source 0)
-        unsigned lo = 0x03020100u, hi = 0x03020100u;
+    for (unsigned t = 0; t < 16u; ++t)
+        lds_store_uint4(kMagBase + threadIdx.x * 256u + ((threadIdx.x + t) & 15u) * 16u, entry);
+}
+
+__device__ __forceinline__ void sweep_signs_fill()                       // threads 256 .. 511
+{
+    const unsigned s7 = (threadIdx.x - 256u) >> 1, upper = threadIdx.x & 1u;
+    const unsigned s = s7 | ((__popc(s7) & 1u) << 7);
+    // selector byte k = k (take +level, source 1) or k + 4 (take -level, source 0)
+    unsigned lo = 0x03020100u, hi = 0x03020100u;
 #pragma unroll
-        for (unsigned l = 0; l < 4u; ++l) {
-            lo += ((s >> l) & 1u) << (8u * l + 2u);
-            hi += ((s >> (l + 4u)) & 1u) << (8u * l + 2u);
-        }
-#pragma unroll 4
-        for (unsigned t = 0; t < 16u; ++t)
-            lds_store_uint2(kSelBase + s7 * 256u + upper * 128u + ((s7 + t) & 15u) * 8u, make_uint2(lo, hi));
+    for (unsigned l = 0; l < 4u; ++l) {
+        lo += ((s >> l) & 1u) << (8u * l + 2u);
+        hi += ((s >> (l + 4u)) & 1u) << (8u * l + 2u);
     }
+#pragma unroll 4
+    for (unsigned t = 0; t < 16u; ++t)
+        lds_store_uint2(kSelBase + s7 * 256u + upper * 128u + ((s7 + t) & 15u) * 8u, make_uint2(lo, hi));
 }
 
 // A lane's share of one IQ2_XXS weight row: half a superblock, 32 packed bytes plus the scale.
@@ -488,7 +491,7 @@ __device__ __forceinline__ unsigned draw_chunk()
 }
 
 // One sweep over weight rows [row_begin, row_end) for N live pairs: chunk `chunk` of them
-// (chunk_turns iterations each) and whatever chunks of the same rows this wave draws next; returns
+// (1 << chunk_shift iterations each) and whatever chunks of the same rows this wave draws next; returns
 // the first one drawn that lies behind them (as drawn: the rows' first chunk is number `base`).
 // MODE 0: one weight row group (the rows of one iteration) at a time; MODE 1: a gate row group
 // and the matching up row group, SwiGLU in the finishing pass; MODE 2: two consecutive row groups
@@ -499,7 +502,7 @@ __device__ __forceinline__ unsigned iq2_sweep(const GroupedArgs &a, const Groupe
                                               const SweepLane &g, const unsigned char *gate_e,
                                               const unsigned char *up_e, unsigned long long first_ordered,
                                               unsigned row_begin, unsigned row_end, bool pairs_in_lds,
-                                              unsigned chunk, unsigned base, unsigned chunk_turns)
+                                              unsigned chunk, unsigned base, unsigned chunk_shift)
 {
     constexpr bool FUSED = MODE == 1;
     constexpr bool TWIN = MODE != 0;     // two streams of weight rows against the same activation columns
@@ -578,7 +581,7 @@ __device__ __forceinline__ unsigned iq2_sweep(const GroupedArgs &a, const Groupe
 
     const unsigned rows_per_turn = MODE == 2 ? 2u * g.rows_per_iter : g.rows_per_iter;
     const unsigned rows = row_end - row_begin;               // a multiple of rows_per_turn
-    const unsigned iterations = rows / rows_per_turn;
+    const unsigned iterations = rows >> (g.row_shift + (MODE == 2 ? 1u : 0u)), chunk_turns = 1u << chunk_shift;
     // wave-uniform row bases advance by a scalar stride; the lane's place inside an iteration's
     // rows is a constant 32-bit offset
     const unsigned char *gate_rows = gate_e + (unsigned long long)row_begin * pr.row_bytes;
@@ -628,8 +631,8 @@ __device__ __forceinline__ unsigned iq2_sweep(const GroupedArgs &a, const Groupe
         }
     };
     static_assert(AHEAD == 1, "a chunk's last turn asks for the first rows of the next");
-    const unsigned chunks = (iterations + chunk_turns - 1u) / chunk_turns;
-    unsigned begin = chunk * chunk_turns;
+    const unsigned chunks = (iterations + chunk_turns - 1u) >> chunk_shift;
+    unsigned begin = chunk << chunk_shift;
     __builtin_amdgcn_sched_barrier(0);
     request(ring[0], begin);
     __builtin_amdgcn_sched_barrier(0);
@@ -692,7 +695,7 @@ __device__ __forceinline__ unsigned iq2_sweep(const GroupedArgs &a, const Groupe
     const unsigned drawn = draw_chunk(), next = drawn - base;
     const unsigned finish = begin + chunk_turns < iterations ? begin + chunk_turns : iterations;
     const unsigned padded = begin + ((finish - begin + 1u) & ~1u);
-    const unsigned follow = next < chunks ? next * chunk_turns : finish - 1u;
+    const unsigned follow = next < chunks ? next << chunk_shift : finish - 1u;
     unsigned window_begin = begin;
     while (window_begin < finish) {
       const unsigned window_end = window_begin + kWindowIters < finish ? window_begin + kWindowIters : finish;
@@ -807,7 +810,7 @@ __device__ __forceinline__ unsigned iq2_sweep(const GroupedArgs &a, const Groupe
         wave_lds_fence();
     }
     if (next >= chunks) return drawn;
-    begin = next * chunk_turns;
+    begin = next << chunk_shift;
     }
 }
 
@@ -829,26 +832,36 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
         if (threadIdx.x == 0u) raise_status(a.status, 2);
         return;
     }
-    const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const unsigned tid = threadIdx.x, lane = tid & 63u, wave = uniform(tid >> 6);
     const GroupedProblem &routed = a.problem[0];
     const bool routed_fixed = routed.expert_ids == nullptr;
     const bool pairs_in_lds = !routed_fixed && routed.order != nullptr && routed.pairs <= kPairCacheMax;
     static_assert(kPairCacheMax <= 2u * kSweepThreads, "two cached pairs a thread");
-    // ---- everything that opens the launch is requested before any of it is used: the tables'
-    // digits, the routed buckets (four a lane, in every wave) and the pairs' sources ----
+    // ---- what opens the launch. Everything is requested before any of it is used: the tables' digits by the waves that
+    // form the codebook entries, the routed buckets (four a lane) by the wave that finds the workgroup's piece, the
+    // pairs' sources by all; the sign entries need nothing and are stored meanwhile. Every wave used to find the piece, with
+    // divisions, and to fill its part of the tables behind that: 5.7 us to the first sweep of a gate/up launch and 4.9 of a
+    // down launch of one row, 4.6 and 4.0 now, of which 2.3 pass before the buckets are there; launches of one row over IQ2_XXS
+    // and Q2_K 18.6 and 11.7 -> 18.1 and 11.3 us, of 96 rows 257 -> 254. (A second wave for the piece's end is another 0.5 us,
+    // but costs the loops their registers: Q4_K 434 -> 454.) ----
     unsigned digits = 0u;
-    if constexpr (QT == QT_IQ2_XXS) digits = sweep_table_digits();    // (the other formats need no tables)
-    const unsigned long long bucket_count = routed_fixed ? 1ull : routed.counts[0];
-    unsigned long long population64[4], expert64[4], first64[4];
+    if constexpr (QT == QT_IQ2_XXS) {                                 // (the other formats need no tables)
+        if (wave < 4u) digits = sweep_table_digits();
+    }
+    const bool placing = wave == kPlacingWave;
+    unsigned long long bucket_count = 0ull, population64[4], expert64[4], first64[4];
+    if (placing) {
+        bucket_count = routed_fixed ? 1ull : routed.counts[0];
 #pragma unroll
-    for (unsigned j = 0; j < 4u; ++j) {
-        const unsigned slot = 4u * lane + j;
-        population64[j] = routed_fixed ? (slot == 0u ? routed.pairs : 0ull) : 0ull;
-        expert64[j] = first64[j] = 0ull;
-        if (!routed_fixed && slot < routed.experts) {
-            population64[j] = routed.bucket_populations[slot];
-            expert64[j] = routed.expert_ids[slot];
-            first64[j] = routed.bucket_offsets[slot];
+        for (unsigned j = 0; j < 4u; ++j) {
+            const unsigned slot = 4u * lane + j;
+            population64[j] = routed_fixed ? (slot == 0u ? routed.pairs : 0ull) : 0ull;
+            expert64[j] = first64[j] = 0ull;
+            if (!routed_fixed && slot < routed.experts) {
+                population64[j] = routed.bucket_populations[slot];
+                expert64[j] = routed.expert_ids[slot];
+                first64[j] = routed.bucket_offsets[slot];
+            }
         }
     }
     unsigned long long source_here[2] = {~0ull, ~0ull};
@@ -857,14 +870,19 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
         for (unsigned k = 0; k < 2u; ++k)
             if (tid + k * kSweepThreads < routed.pairs) source_here[k] = routed.order[tid + k * kSweepThreads];
     }
+    if constexpr (QT == QT_IQ2_XXS) {
+        if (wave >= 4u) sweep_signs_fill();
+    }
+    if (tid == 0u) lds_store_u32(kTicketAddress, 0u);
 
-    const unsigned units = a.width >> 5;
+    // (shifts and comparisons: a division by a number that only the launch knows is forty dependent instructions)
     SweepLane g;
-    g.lanes_per_row = units / 4u;                                  // 16 .. 64, checked on the host
-    g.rows_per_iter = (g.lanes_per_row % 16u) == 0u && 64u % g.lanes_per_row == 0u
-        ? 64u / g.lanes_per_row : 1u;
-    g.sub = lane / g.lanes_per_row;
-    const unsigned seg = lane % g.lanes_per_row;
+    g.lanes_per_row = a.width >> 7;                                // 16 .. 64, checked on the host
+    g.row_shift = g.lanes_per_row == 16u ? 2u : g.lanes_per_row == 32u ? 1u : 0u;
+    g.rows_per_iter = 1u << g.row_shift;
+    g.sub = (lane >= g.lanes_per_row ? 1u : 0u) + (lane >= 2u * g.lanes_per_row ? 1u : 0u) +
+            (lane >= 3u * g.lanes_per_row ? 1u : 0u);
+    const unsigned seg = lane - g.sub * g.lanes_per_row;
     g.live = g.sub < g.rows_per_iter;
     g.super = seg >> 1;
     g.half = seg & 1u;
@@ -874,151 +892,147 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
     g.scale_shift = 8u * (block_start & 3u);
     g.mag_lane = (lane & 15u) * 16u;
     g.sel_lane = kSelBase + (lane & 31u) * 8u;
-    g.park = kParkBase + wave * kParkBytes;
+    g.park = kParkBase + (tid >> 6) * kParkBytes;      // (in a vector register: the window's stores lose their immediate offsets otherwise)
     g.results = g.park + kWindowBytes;
     g.terms = g.lanes_per_row / 2u;
-    g.row_shift = g.rows_per_iter == 4u ? 2u : g.rows_per_iter == 2u ? 1u : 0u;
     {
         // a line of the window: parity, then the rows of an iteration, then the row's superblocks
-        const unsigned span = 64u >> g.row_shift;                  // lanes of a weight row's slot
-        g.term_slot = ((lane & 1u) * 32u + (lane / span) * (span / 2u) + (lane % span) / 2u) * 4u;
+        const unsigned span_shift = 6u - g.row_shift, span = 64u >> g.row_shift;      // lanes of a weight row's slot
+        g.term_slot = ((lane & 1u) * 32u + (lane >> span_shift) * (span / 2u) + (lane & (span - 1u)) / 2u) * 4u;
     }
-
-    // ---- the launch's work, the same in every wave ----
-    // Slot 0 is the shared expert (no rows of its own when there is none), slot 1 + b bucket b. A
-    // slot of n pairs has n / 4 sweeps of four pairs and one of what is left. Every wave needs the
-    // prefix sums of cost and sweeps over the slots: a scan across its 64 lanes, four slots each,
-    // no barrier and no LDS. (It was a list of all sweeps sorted by their pairs, built by the
-    // workgroup in LDS behind two barriers: 2.5 us of every launch's first 8.5.)
+    const unsigned turn_shift = g.row_shift + (MODE == 2 ? 1u : 0u), turn_rows = 1u << turn_shift;
     const GroupedProblem &extra = a.problem[a.problems > 1u ? 1u : 0u];
     const unsigned extra_pairs = a.problems > 1u ? extra.pairs : 0u;
-    const unsigned extra_cost = bucket_cost<QT>(extra_pairs), extra_sweeps = (extra_pairs + 3u) / 4u;
-    const unsigned buckets = (unsigned)bucket_count;
-    unsigned population[4], cost_here = 0u, sweeps_here = 0u;
-    bool bad = bucket_count > 256ull;
-#pragma unroll
-    for (unsigned j = 0; j < 4u; ++j) {
-        const bool live = 4u * lane + j < bucket_count;
-        bad |= live && (population64[j] > routed.pairs || expert64[j] >= routed.experts || first64[j] > routed.pairs);
-        population[j] = live ? (unsigned)population64[j] : 0u;
-        cost_here += bucket_cost<QT>(population[j]);
-        sweeps_here += (population[j] + 3u) / 4u;
-    }
-    const unsigned all_pairs = (unsigned)group_sum_i32<64>((int)(population[0] + population[1] + population[2] + population[3]));
-    // (the launch wrapper bounds the pairs, and with them what the packed sums below can hold)
-    if (__ballot(bad) != 0ull || all_pairs > routed.pairs || routed.pairs + extra_pairs > kMaxSweeps) {
-        if (tid == 0u) raise_status(a.status, 2);
-        return;
-    }
-    static_assert(kMaxSweeps * sweep_cost<QT>(4u) < 65536u, "a prefix is two 16-bit sums");
-    const unsigned packed = (sweeps_here << 16) | cost_here;
-    const unsigned inclusive = wave_inclusive_sum_u32(packed);
-    const unsigned before = inclusive - packed;
-    const unsigned totals = (unsigned)__builtin_amdgcn_readlane((int)inclusive, 63);
-    const unsigned row_cost = extra_cost + (totals & 0xffffu), all_sweeps = extra_sweeps + (totals >> 16);
-
-    // ---- this workgroup's piece ----
-    const unsigned turn_rows = MODE == 2 ? 2u * g.rows_per_iter : g.rows_per_iter;
-    const unsigned granule = 2u * turn_rows;                       // the ring turns twice a trip through its loop
-    // iterations of a piece: a batch of a few rows leaves a wave a handful of them, and is cut finely
-    const unsigned piece_turns = (unsigned)((unsigned long long)all_sweeps * (a.out_rows / turn_rows) / gridDim.x);
-    auto chunk_turns_of = [&](unsigned n) -> unsigned {
-        unsigned turns = n >= 2u ? kSweepChunkTurns / 2u : kSweepChunkTurns;
-        while (turns > 2u && (turns * (4u * kSweepWaves) > piece_turns || (FUSED && turns * turn_rows > kFusedItemRows)))
-            turns /= 2u;
-        return turns;
-    };
     struct Place {
         unsigned slot, sweep, row;
     };
-    // (integer arithmetic on the scalar unit, one division for both ends)
-    const unsigned long long all_cost = (unsigned long long)row_cost * a.out_rows;
-    const unsigned long long share = uniform64((unsigned long long)((double)all_cost / (double)gridDim.x));
-    const unsigned long long left_over = all_cost - share * gridDim.x;
-    auto place_of = [&](unsigned who) -> Place {        // where the piece of workgroup `who` begins
-        if (who >= gridDim.x) return Place{buckets + 1u, 0u, 0u};
-        unsigned long long at = share * who + (who < left_over ? who : left_over);
-        unsigned slot = 0u, n = extra_pairs;
-        if (at >= (unsigned long long)extra_cost * a.out_rows) {
-            at -= (unsigned long long)extra_cost * a.out_rows;
-            const unsigned long long below = __ballot((unsigned long long)(before & 0xffffu) * a.out_rows <= at);
-            const int holder = 63 - __builtin_clzll(below);
-            at -= (unsigned long long)((unsigned)__builtin_amdgcn_readlane((int)before, holder) & 0xffffu) * a.out_rows;
-            slot = 4u * (unsigned)holder + 1u;
-            n = (unsigned)__builtin_amdgcn_readlane((int)population[0], holder);
+
+    // ---- the launch's work and this workgroup's piece of it, by one wave ----
+    // Slot 0 is the shared expert (no rows of its own when there is none), slot 1 + b bucket b. A
+    // slot of n pairs has n / 4 sweeps of four pairs and one of what is left. The prefix sums of cost and sweeps over the
+    // slots are a scan across the wave's 64 lanes, four slots each, no barrier and no LDS. (It was a list of all sweeps
+    // sorted by their pairs, built by the workgroup in LDS behind two barriers: 2.5 us of every launch's first 8.5.)
+    unsigned warm[2] = {0u, 0u};
+    if (placing) {
+        const unsigned extra_cost = bucket_cost<QT>(extra_pairs), extra_sweeps = (extra_pairs + 3u) / 4u;
+        const unsigned buckets = (unsigned)bucket_count;
+        unsigned population[4], cost_here = 0u, sweeps_here = 0u;
+        bool bad = bucket_count > 256ull;
 #pragma unroll
-            for (unsigned j = 1; j < 4u; ++j) {
-                const unsigned long long rows = (unsigned long long)bucket_cost<QT>(n) * a.out_rows;
-                const unsigned behind = (unsigned)__builtin_amdgcn_readlane((int)population[j], holder);
-                if (slot == 4u * (unsigned)holder + j && at >= rows) {
-                    at -= rows;
-                    ++slot;
-                    n = behind;
+        for (unsigned j = 0; j < 4u; ++j) {
+            const bool live = 4u * lane + j < bucket_count;
+            bad |= live && (population64[j] > routed.pairs || expert64[j] >= routed.experts || first64[j] > routed.pairs);
+            population[j] = live ? (unsigned)population64[j] : 0u;
+            cost_here += bucket_cost<QT>(population[j]);
+            sweeps_here += (population[j] + 3u) / 4u;
+        }
+        const unsigned all_pairs = (unsigned)group_sum_i32<64>((int)(population[0] + population[1] + population[2] + population[3]));
+        // (the launch wrapper bounds the pairs, and with them what the packed sums below can hold)
+        const bool refused = __ballot(bad) != 0ull || all_pairs > routed.pairs || routed.pairs + extra_pairs > kMaxSweeps;
+        if (refused) {
+            if (lane == 0u) raise_status(a.status, 2);
+            lds_store_uint4(kPlaceAddress, make_uint4(0u, 0u, 0u, 1u));
+        } else {
+            static_assert(kMaxSweeps * sweep_cost<QT>(4u) < 65536u, "a prefix is two 16-bit sums");
+            const unsigned packed = (sweeps_here << 16) | cost_here;
+            const unsigned inclusive = wave_inclusive_sum_u32(packed);
+            const unsigned before = inclusive - packed;
+            const unsigned totals = (unsigned)__builtin_amdgcn_readlane((int)inclusive, 63);
+            const unsigned row_cost = extra_cost + (totals & 0xffffu), all_sweeps = extra_sweeps + (totals >> 16);
+#pragma unroll
+            for (unsigned j = 0; j < 4u; ++j)
+                lds_store_uint4(kBucketBase + 16u * (4u * lane + j),
+                                make_uint4((unsigned)expert64[j], (unsigned)first64[j], population[j], 0u));
+
+            const unsigned granule = 2u * turn_rows;                   // the ring turns twice a trip through its loop
+            // iterations of a piece: a batch of a few rows leaves a wave a handful of them, and is cut finely
+            const unsigned piece_turns = uniform((unsigned)((float)all_sweeps * (float)(a.out_rows >> turn_shift) *
+                                                            __builtin_amdgcn_rcpf((float)gridDim.x)));
+            // (integer arithmetic on the scalar unit; any share does whose pieces do not reach past the end)
+            const unsigned long long all_cost = (unsigned long long)row_cost * a.out_rows;
+            const unsigned long long share = (gridDim.x & (gridDim.x - 1u)) == 0u
+                ? all_cost >> (31 - __builtin_clz(gridDim.x)) : uniform64((unsigned long long)((double)all_cost / (double)gridDim.x));
+            const unsigned long long left_over = all_cost - share * gridDim.x;
+            auto place_of = [&](unsigned who) -> Place {        // where the piece of workgroup `who` begins
+                if (who >= gridDim.x) return Place{buckets + 1u, 0u, 0u};
+                unsigned long long at = share * who + (who < left_over ? who : left_over);
+                unsigned slot = 0u, n = extra_pairs;
+                if (at >= (unsigned long long)extra_cost * a.out_rows) {
+                    at -= (unsigned long long)extra_cost * a.out_rows;
+                    const unsigned long long below = __ballot((unsigned long long)(before & 0xffffu) * a.out_rows <= at);
+                    const int holder = 63 - __builtin_clzll(below);
+                    at -= (unsigned long long)((unsigned)__builtin_amdgcn_readlane((int)before, holder) & 0xffffu) * a.out_rows;
+                    slot = 4u * (unsigned)holder + 1u;
+                    n = (unsigned)__builtin_amdgcn_readlane((int)population[0], holder);
+#pragma unroll
+                    for (unsigned j = 1; j < 4u; ++j) {
+                        const unsigned long long rows = (unsigned long long)bucket_cost<QT>(n) * a.out_rows;
+                        const unsigned behind = (unsigned)__builtin_amdgcn_readlane((int)population[j], holder);
+                        if (slot == 4u * (unsigned)holder + j && at >= rows) {
+                            at -= rows;
+                            ++slot;
+                            n = behind;
+                        }
+                    }
+                }
+                const unsigned full = n / 4u;
+                const unsigned sweep_rows = sweep_cost<QT>(4u) * a.out_rows;
+                unsigned sweep = 0u;
+                if (full) {
+                    // (a quotient of at most kMaxSweeps / 4: out by one at most)
+                    sweep = uniform((unsigned)((float)at * __builtin_amdgcn_rcpf((float)sweep_rows)));
+                    if ((unsigned long long)sweep * sweep_rows > at) --sweep;
+                    if ((unsigned long long)(sweep + 1u) * sweep_rows <= at) ++sweep;
+                    if (sweep > full) sweep = full;
+                    at -= (unsigned long long)sweep * sweep_rows;
+                }
+                const unsigned rest = (unsigned)at;
+                unsigned row = sweep < full ? rest / sweep_cost<QT>(4u)
+                    : n % 4u == 1u ? rest / sweep_cost<QT>(1u) : n % 4u == 2u ? rest / sweep_cost<QT>(2u)
+                                                                             : rest / sweep_cost<QT>(3u);
+                if (row > a.out_rows) row = a.out_rows;
+                return Place{uniform(slot), uniform(sweep), uniform(row & ~(granule - 1u))};
+            };
+            Place now{}, end{};
+#pragma unroll 1
+            for (unsigned ends = 0; ends < 2u; ++ends) {      // (the code of one, run twice)
+                now = end;
+                end = place_of(blockIdx.x + ends);
+            }
+            lds_store_uint4(kPlaceAddress, make_uint4(now.slot, now.sweep, now.row, 0u));
+            lds_store_uint4(kPlaceAddress + 16u, make_uint4(end.slot, end.sweep, end.row, piece_turns));
+
+            // The first weight rows of the piece start on their way to the caches (64 bytes apart, so the lanes cover
+            // 4 KB of each stream).
+            if (now.slot <= buckets) {
+                const unsigned bucket = now.slot ? now.slot - 1u : 0u;
+                unsigned expert = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)expert64[0], (int)(bucket >> 2));
+#pragma unroll
+                for (unsigned j = 1; j < 4u; ++j) {
+                    const unsigned other = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)expert64[j], (int)(bucket >> 2));
+                    if ((bucket & 3u) == j) expert = other;
+                }
+                const GroupedProblem &pr = a.problem[now.slot == 0u ? a.problems - 1u : 0u];
+                if (now.slot == 0u) expert = 0u;
+                const unsigned rows_left = a.out_rows - now.row;
+                unsigned long long offset = 64ull * lane;
+                const unsigned long long bytes_left = rows_left * pr.row_bytes;
+                if (bytes_left >= 8ull) {
+                    if (offset + 4ull > bytes_left) offset = bytes_left - 4ull;
+                    const unsigned char *rows = pr.gate + expert * pr.expert_bytes + now.row * pr.row_bytes;
+                    warm[0] = *reinterpret_cast<const unsigned *>(rows + (offset & ~3ull));
+                    if (FUSED) {
+                        warm[1] = *reinterpret_cast<const unsigned *>(pr.up + expert * pr.up_expert_bytes +
+                                                                      now.row * pr.up_row_bytes + (offset & ~3ull));
+                    } else if (offset + 4096ull + 4ull <= bytes_left) {
+                        warm[1] = *reinterpret_cast<const unsigned *>(rows + 4096u + (offset & ~3ull));
+                    }
                 }
             }
         }
-        const unsigned full = n / 4u;
-        const unsigned sweep_rows = sweep_cost<QT>(4u) * a.out_rows;
-        unsigned sweep = 0u;
-        if (full) {
-            sweep = uniform((unsigned)((double)at / (double)sweep_rows));
-            if (sweep > full) sweep = full;
-            at -= (unsigned long long)sweep * sweep_rows;
-        }
-        const unsigned rest = (unsigned)at;
-        unsigned row = sweep < full ? rest / sweep_cost<QT>(4u)
-            : n % 4u == 1u ? rest / sweep_cost<QT>(1u) : n % 4u == 2u ? rest / sweep_cost<QT>(2u)
-                                                                     : rest / sweep_cost<QT>(3u);
-        if (row > a.out_rows) row = a.out_rows;
-        // (the same in every lane: kept in scalar registers, of which the sweeps leave some)
-        return Place{uniform(slot), uniform(sweep), uniform(row & ~(granule - 1u))};
-    };
-    Place now{}, end{};
-#pragma unroll 1
-    for (unsigned ends = 0; ends < 2u; ++ends) {      // (the code of one, run twice)
-        now = end;
-        end = place_of(blockIdx.x + ends);
     }
-
-    // The first weight rows of the piece start on their way to the caches while the tables are
-    // built (64 bytes apart, so the lanes cover 4 KB of each stream).
-    unsigned warm[2] = {0u, 0u};
-    if (now.slot <= buckets) {
-        const unsigned bucket = now.slot ? now.slot - 1u : 0u;
-        unsigned expert = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)expert64[0], (int)(bucket >> 2));
-#pragma unroll
-        for (unsigned j = 1; j < 4u; ++j) {
-            const unsigned other = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)expert64[j], (int)(bucket >> 2));
-            if ((bucket & 3u) == j) expert = other;
-        }
-        const GroupedProblem &pr = a.problem[now.slot == 0u ? a.problems - 1u : 0u];
-        if (now.slot == 0u) expert = 0u;
-        const unsigned rows_left = a.out_rows - now.row;
-        unsigned long long offset = 64ull * lane;
-        const unsigned long long bytes_left = rows_left * pr.row_bytes;
-        if (bytes_left >= 8ull) {
-            if (offset + 4ull > bytes_left) offset = bytes_left - 4ull;
-            const unsigned char *rows = pr.gate + expert * pr.expert_bytes + now.row * pr.row_bytes;
-            warm[0] = *reinterpret_cast<const unsigned *>(rows + (offset & ~3ull));
-            if (FUSED) {
-                warm[1] = *reinterpret_cast<const unsigned *>(pr.up + expert * pr.up_expert_bytes +
-                                                              now.row * pr.up_row_bytes + (offset & ~3ull));
-            } else if (offset + 4096ull + 4ull <= bytes_left) {
-                warm[1] = *reinterpret_cast<const unsigned *>(rows + 4096u + (offset & ~3ull));
-            }
-        }
-    }
-
-    if constexpr (QT == QT_IQ2_XXS) sweep_tables_fill(digits);
-    if (tid == 0u) lds_store_u32(kTicketAddress, 0u);
-    if (wave == 0u) {
-        unsigned sweeps_before = before >> 16;
-#pragma unroll
-        for (unsigned j = 0; j < 4u; ++j) {
-            lds_store_uint4(kBucketBase + 16u * (4u * lane + j),
-                            make_uint4((unsigned)expert64[j], (unsigned)first64[j], population[j], sweeps_before));
-            sweeps_before += (population[j] + 3u) / 4u;
-        }
+    if constexpr (QT == QT_IQ2_XXS) {
+        if (wave < 4u) sweep_levels_fill(digits);
     }
     if (pairs_in_lds) {
         float weight_here[2];
@@ -1033,7 +1047,19 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
                                 make_uint2(source_here[k] < 0xffffffffull ? (unsigned)source_here[k] : 0xffffffffu,
                                            __float_as_uint(weight_here[k])));
     }
-    __syncthreads();
+    // (LDS traffic only: the warming loads may still be on their way)
+    lds_barrier();
+    const uint4 first_place = lds_read_uint4(kPlaceAddress), last_place = lds_read_uint4(kPlaceAddress + 16u);
+    if (uniform(first_place.w)) return;                               // refused
+    Place now{uniform(first_place.x), uniform(first_place.y), uniform(first_place.z)};
+    const Place end{uniform(last_place.x), uniform(last_place.y), uniform(last_place.z)};
+    const unsigned piece_turns = uniform(last_place.w);
+    auto chunk_shift_of = [&](unsigned n) -> unsigned {
+        unsigned shift = n >= 2u ? kSweepChunkShift - 1u : kSweepChunkShift;
+        while (shift > 1u && ((4u * kSweepWaves << shift) > piece_turns || (FUSED && (turn_rows << shift) > kFusedItemRows)))
+            --shift;
+        return shift;
+    };
 #if defined(__HIP_DEVICE_COMPILE__)
     asm volatile("" ::"v"(warm[0]), "v"(warm[1]));
 #endif
@@ -1070,9 +1096,8 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
             continue;
         }
         const unsigned live = n - pass < 4u ? n - pass : 4u;
-        const unsigned chunk_turns = chunk_turns_of(live);
-        const unsigned chunk_rows = chunk_turns * turn_rows;
-        const unsigned chunks = (row_end - row_begin + chunk_rows - 1u) / chunk_rows;
+        const unsigned chunk_shift = chunk_shift_of(live), rows_shift = chunk_shift + turn_shift;
+        const unsigned chunks = (row_end - row_begin + (1u << rows_shift) - 1u) >> rows_shift;
         if (drawn - base < chunks) {
             const unsigned char *gate_e = pr.gate + expert * pr.expert_bytes;
             const unsigned char *up_e = FUSED ? pr.up + expert * pr.up_expert_bytes : nullptr;
@@ -1080,13 +1105,13 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
             const unsigned chunk = drawn - base;
             static_assert(kSweepPairs == 4, "a sweep serves one to four pairs");
             if (live == 4u)
-                drawn = iq2_sweep<MODE, 4, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached, chunk, base, chunk_turns);
+                drawn = iq2_sweep<MODE, 4, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached, chunk, base, chunk_shift);
             else if (live == 3u)
-                drawn = iq2_sweep<MODE, 3, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached, chunk, base, chunk_turns);
+                drawn = iq2_sweep<MODE, 3, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached, chunk, base, chunk_shift);
             else if (live == 2u)
-                drawn = iq2_sweep<MODE, 2, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached, chunk, base, chunk_turns);
+                drawn = iq2_sweep<MODE, 2, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached, chunk, base, chunk_shift);
             else
-                drawn = iq2_sweep<MODE, 1, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached, chunk, base, chunk_turns);
+                drawn = iq2_sweep<MODE, 1, IMAGE, QT>(a, pr, g, gate_e, up_e, first + pass, row_begin, row_end, cached, chunk, base, chunk_shift);
         }
         base += chunks;
     }
