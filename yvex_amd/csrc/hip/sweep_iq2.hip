@@ -653,6 +653,19 @@ __device__ __forceinline__ unsigned iq2_sweep(const GroupedArgs &a, const Groupe
             const unsigned at = g.park + line * 256u + parity * 128u + group * segment_bytes;
             double sum = 0.0;
             unsigned k = 0u;
+            // (long rows of formats that have the registers: two reads on their way before the first addition)
+            const unsigned doubled = !Q4 && g.terms > 16u ? g.terms & ~7u : 0u;
+            if constexpr (!Q4) for (; k < doubled; k += 8u) {
+                const uint4 t = lds_read_uint4(at + 4u * k), u = lds_read_uint4(at + 4u * k + 16u);
+                sum += (double)__uint_as_float(t.x);
+                sum += (double)__uint_as_float(t.y);
+                sum += (double)__uint_as_float(t.z);
+                sum += (double)__uint_as_float(t.w);
+                sum += (double)__uint_as_float(u.x);
+                sum += (double)__uint_as_float(u.y);
+                sum += (double)__uint_as_float(u.z);
+                sum += (double)__uint_as_float(u.w);
+            }
             for (; k + 4u <= g.terms; k += 4u) {
                 const uint4 t = lds_read_uint4(at + 4u * k);
                 sum += (double)__uint_as_float(t.x);
@@ -789,9 +802,14 @@ __device__ __forceinline__ unsigned iq2_sweep(const GroupedArgs &a, const Groupe
     // ---- the end of a fused chunk: SwiGLU of the (gate, up) row sums, coalesced stores ----
     if constexpr (FUSED) {
         const unsigned chunk_rows = (finish - begin) << g.row_shift, chunk_row = row_begin + (begin << g.row_shift);
-        const unsigned outputs = chunk_rows * (unsigned)N;
+        // (consecutive lanes: consecutive rows. A chunk's rows are numbered as if it were whole, which takes no division: 298
+        // -> 296 us of a launch of 32 rows, another 3 by the flush above; the Q4_K sweeps have no registers for either)
+        const unsigned row_bits = chunk_shift + g.row_shift;
+        const unsigned outputs = Q4 ? chunk_rows * (unsigned)N : (unsigned)N << row_bits;
         for (unsigned o = lane; o < outputs; o += 64u) {
-            const unsigned p = o / chunk_rows, local = o % chunk_rows;      // consecutive lanes: consecutive rows
+            const unsigned p = Q4 ? o / chunk_rows : o >> row_bits;
+            const unsigned local = Q4 ? o % chunk_rows : o & ((1u << row_bits) - 1u);
+            if (!Q4 && local >= chunk_rows) continue;
             const float first = __uint_as_float(lds_load_u32(g.results + (p * kFusedItemRows + local) * 4u));
             const float second = __uint_as_float(
                 lds_load_u32(g.results + (((unsigned)N + p) * kFusedItemRows + local) * 4u));
@@ -1054,8 +1072,13 @@ __global__ __launch_bounds__(kSweepThreads) void iq2_sweep_kernel(GroupedArgs a)
     Place now{uniform(first_place.x), uniform(first_place.y), uniform(first_place.z)};
     const Place end{uniform(last_place.x), uniform(last_place.y), uniform(last_place.z)};
     const unsigned piece_turns = uniform(last_place.w);
+    // A wave holds one chunk and has drawn the next, and waves of a launch end 10 to 15 % apart, so short chunks are the
+    // better ones until their ends cost more. A chunk of a plain projection ends in a flush: four turns (of 32 rows, IQ2_XXS
+    // 151.5 us with eight turns, 148.9 with four, 153.4 with two; of 23 rows Q4_K 234.3, 229.5, 236.1; of 96 rows Q2_K 154.5,
+    // 152.5, 163.4). One of gate and up rows ends in the SwiGLU as well: sixteen turns of one pair and eight of
+    // more (32 rows: 293 us; eight of any 305; four 316; sixteen of any 299), of Q4_K eight (429; 433 with sixteen of one pair).
     auto chunk_shift_of = [&](unsigned n) -> unsigned {
-        unsigned shift = n >= 2u ? kSweepChunkShift - 1u : kSweepChunkShift;
+        unsigned shift = !FUSED ? kSweepChunkShift - 2u : QT == QT_Q4_K || n >= 2u ? kSweepChunkShift - 1u : kSweepChunkShift;
         while (shift > 1u && ((4u * kSweepWaves << shift) > piece_turns || (FUSED && (turn_rows << shift) > kFusedItemRows)))
             --shift;
         return shift;
