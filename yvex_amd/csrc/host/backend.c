@@ -160,7 +160,7 @@ int yvex_rocm_upload_queued(yvex_rocm_backend *backend, void *device, const void
 
 /* What every session has of its own on the device: a stream, a status word, and pinned memory for
  * what its synchronous operations publish. Released again where any of it is missing. */
-enum { SESSION_WORDS_BYTES = 256 + YVEX_HIP_ARRIVAL_BYTES };     /* the status word, then the counters */
+enum { SESSION_WORDS_BYTES = 256 + YVEX_HIP_ARRIVAL_BYTES };     /* the status word and its counter, then the counters */
 
 static int session_open(yvex_rocm_backend *backend)
 {

@@ -14,7 +14,8 @@ extern "C" {
 #endif
 
 /* The arguments of yvex_hip_publish, and where the workgroups of a launch count each other: YVEX_HIP_ARRIVAL_BYTES of
- * device memory that belong to one stream, zero before the launch and zero again behind it. */
+ * device memory that belong to one stream, zero before the launch and zero again behind it. The status word that goes with
+ * them starts on eight bytes, and the word behind it counts too. */
 typedef struct {
     uint32_t *arrivals;
     uint32_t *host;
@@ -22,7 +23,7 @@ typedef struct {
     int clear;
 } yvex_hip_publication;
 
-enum { YVEX_HIP_ARRIVAL_BYTES = 17 * 128 };
+enum { YVEX_HIP_ARRIVAL_BYTES = 16 * 128 };
 
 /* yvex_hip_matvec, yvex_hip_matvec_quantizing and yvex_hip_argmax_f32 whose last launch publishes by itself where its kernel
  * can: *published says whether it did, yvex_hip_publish is the caller's to make if not. */
