@@ -15,26 +15,28 @@ def dev(array, device):
 POPULATIONS = [64 + 40, 33, 17, 5]
 
 
-@pytest.mark.parametrize("qtype", ["Q4_K", "Q2_K"])
+@pytest.mark.parametrize("qtype", ["Q4_K", "Q2_K", "IQ2_XXS"])
 @pytest.mark.parametrize("scales,magnitude", [("ordinary", 1.0), ("largest", 2.0 ** 80), ("subnormal", 2.0 ** -108)])
 def test_scales_and_minimums_reach_as_far_as_floats(gpu, oracle, qtype, scales, magnitude):
     """Sub-block scales and minimums at their largest against rows whose codes all have the largest magnitude and one sign,
     (the largest sums there are), with block scales whose products are ordinary, huge or denormal."""
     from yvex_amd import kernels as K
     qt, hidden, intermediate = getattr(oracle, qtype), 256, 512
-    block, heads = {"Q4_K": (144, slice(4, 16)), "Q2_K": (84, slice(0, 16))}[qtype]
-    at = 0 if qtype == "Q4_K" else 80
+    # (IQ2_XXS: codebook entries, signs and group scales at once)
+    block, heads, halves = {"Q4_K": (144, slice(4, 16), (0, 2)), "Q2_K": (84, slice(0, 16), (80, 82)),
+                            "IQ2_XXS": (66, slice(2, 66), (0,))}[qtype]
+    first = qt if qtype == "IQ2_XXS" else oracle.Q4_K
     experts, pairs = len(POPULATIONS), sum(POPULATIONS)
     g = oracle.Generator(45, f"limits.{qtype}")
-    up = dev(g.weights(oracle.Q4_K, experts * intermediate, hidden), gpu)
+    up = dev(g.weights(first, experts * intermediate, hidden), gpu)
     down = g.weights(qt, experts * hidden, intermediate)
     blocks = down.reshape(-1, block)
     blocks[::2, heads] = 255
     if scales != "ordinary":
         bits = (np.full(len(blocks), 0x7800) if scales == "largest" else 1 + np.arange(len(blocks)) * 7 % 1023).astype(np.uint16)
-        for offset in (at, at + 2):
+        for offset in halves:
             blocks[:, offset], blocks[:, offset + 1] = bits & 255, bits >> 8
-    weights = K.expert_weights(up, up, dev(down, gpu), (oracle.Q4_K, oracle.Q4_K, qt), hidden, intermediate)
+    weights = K.expert_weights(up, up, dev(down, gpu), (first, first, qt), hidden, intermediate)
     status = K.new_status(gpu)
     selected = torch.repeat_interleave(torch.arange(experts), torch.tensor(POPULATIONS)).reshape(pairs, 1).to(gpu)
     wl = K.worklist_build(selected, experts, status)

@@ -34,8 +34,6 @@ __device__ __forceinline__ void q4k_bsum_limbs(const uint4 (&b)[2], uint2 &lo, u
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float v32f __attribute__((ext_vector_type(32)));
 static_assert(sizeof(f16x8) == 16, "an operand of a matrix instruction");
 
 // Minimum terms on the f16 matrix instructions. A minimum is at most 63 and a sum of sixteen int8 values at

@@ -9,6 +9,7 @@ namespace yvex {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
 
 __device__ __forceinline__ void lds_write_uint4(unsigned address, uint4 v)
 {

@@ -38,6 +38,12 @@
 //       the sum is rounded to float once, which is what the CPU path computes for a row (double
 //       accumulation over a row's blocks, src/gguf/quant_compute.c:152-172): every value
 //       rounded to bfloat16 afterwards rounds as it does there.
+//       The products of a row's and a token's scale are one V_MFMA_F32_32X32X1_2B_F32 a superblock, the outer products
+//       of both token blocks at once: a product of two floats rounded once, the bits of V_MUL_F32. 363 -> 330 vector and
+//       61 -> 56 LDS instructions a superblock and wave of 64 tokens, and a row's scale stays in its lane's register
+//       (it went through LDS to the lanes that hold the row's sums). 2048 rows of 7168 by eight of 256 experts with uneven routing, us
+//       a layer: 2995 -> 2967. The instruction holds the wave for as long as sixteen multiplications, so it gains half of what it
+//       takes out; at one token block it is level.
 //   Output: accumulator i of lane (r, h) is token r's sum for row 8 (i / 4) + 4 h + i % 4 of the
 //       wave's 32 (gate sums in the first eight, the matching up sums in the last eight when
 //       fused), so a lane stores four consecutive rows of its token, 16 bytes, straight from its
@@ -64,8 +70,7 @@ constexpr unsigned kActPitch = 256u;                       // one Q8_K block's i
 constexpr unsigned kCodeBase = 0u;
 constexpr unsigned kSelBase = 128u;
 constexpr unsigned kLutBase = 65536u;                       // 16 scales x 16 replicas x 16 bytes
-constexpr unsigned kRowScaleBase = kLutBase + 16u * 16u * 16u;   // 8 waves x 2 x 32 floats
-constexpr unsigned kPairInfoBase = kRowScaleBase + kRowWaves * 2u * 128u;   // {out row, route weight} x 64
+constexpr unsigned kPairInfoBase = kLutBase + 16u * 16u * 16u;   // {out row, route weight} x 64
 // Item numbering: first full 64-pair tile of every bucket (257 words), then per class of last,
 // partial, tile (33-63, 1-32 pairs) a count and the list of its buckets (u16).
 constexpr unsigned kTileStartBase = kPairInfoBase + kTileTokens * 8u;
@@ -294,15 +299,14 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
     const unsigned code_lane = kCodeBase + (lane & 15u) * 8u;
     const unsigned sel_lane = kSelBase + (lane & 15u) * 8u;
     const unsigned lut_lane = kLutBase + (lane & 15u) * 16u;
-    const unsigned row_scale_at = kRowScaleBase + wave * 256u;      // + 128 for odd superblocks
     unsigned grids[4], aux[4];           // group records of the superblock being decoded
     unsigned head = 0u;                  // image: fp16 scale | the four group scales of this half << 16
+    float row_scale = 0.0f;              // of the superblock being decoded, of the lane's own row
     uint2 codes[2][2], signs[2][2];      // [chunk & 1]: table words of the chunk's two subgroups
     uint4 limbs[2];                      // [group & 1]: limb words of a group
     v4i a_lo[2], a_hi[2];                // [chunk & 1]: A operands of a K chunk
 
-    // Records of superblock sb out of its window, and the row's scale into LDS for the lanes that
-    // hold this row's sums (zero past the end: such superblocks add nothing). With o = (row start
+    // Records of superblock sb out of its window, and the row's scale (zero past the end: such superblocks add nothing). With o = (row start
     // + 66 sb) mod 4 (0 or 2) the fp16 scale sits o bytes into the window and the lane's 32 code
     // bytes at o + 2 + 32 h: in aligned dwords 8 h + o / 2 onwards, shifted by 2 bytes when o is
     // 0. Aligned dword 16 is the last dword of the fifth piece.
@@ -321,8 +325,7 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
             aux[2] = (unsigned)second[2];
             grids[3] = (unsigned)second[3];
             aux[3] = (unsigned)(h ? third[3] : third[0]);
-            const float mine = sb < superblocks ? 0.125f * f16_bits_to_float(head & 0xffffu) : 0.0f;
-            lds_write_u32(row_scale_at + (sb & 1u) * 128u + r * 4u, __float_as_uint(mine));
+            row_scale = sb < superblocks ? 0.125f * f16_bits_to_float(head & 0xffffu) : 0.0f;
             return;
         }
         const unsigned clamped = sb < last ? sb : last;
@@ -340,7 +343,7 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
         for (unsigned i = 0; i < 8u; ++i) w[i] = o ? d[i + 1u] : d[i];
         w[8] = d[8];           // (the ninth is only part of a record when o is 0)
         // the fp16 scale sits o bytes into the window: in the first dword of the first half's lanes,
-        // which are the ones that publish it
+        // from where those of the second half have it too
         const unsigned scale16 = ((unsigned)first[0] >> (8u * o)) & 0xffffu;
         const unsigned shift = (o + 2u) & 3u;
 #pragma unroll
@@ -349,7 +352,7 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
             aux[g] = __builtin_amdgcn_alignbyte(w[2u * g + 2u], w[2u * g + 1u], shift);
         }
         const float mine = sb < superblocks ? 0.125f * f16_bits_to_float(scale16) : 0.0f;
-        lds_write_u32(h ? kTrashBase : row_scale_at + (sb & 1u) * 128u + r * 4u, __float_as_uint(mine));
+        row_scale = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute((int)(4u * r), (int)__float_as_uint(mine)));
     };
     // table lookups of K chunk c: subgroups 2 (c & 1) and 2 (c & 1) + 1 of group c / 2
     auto lookup = [&](unsigned c) {
@@ -457,8 +460,8 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
     constexpr unsigned kBarrierInFlight = 3u + (R - 2u) * kRoundPieces;
 
     for (unsigned sb = 0; sb < superblocks; ++sb) {
-        float rs[16];                // row scales of the rows this lane holds sums of
-        float ts[NTB];               // activation scales of this lane's token per token block
+        float rs = 0.0f, ts = 0.0f;  // scales of the lane's weight row and of its token (of block h) in this superblock
+        v32f scale;                  // their products, where the sums of that row and token are
         const unsigned stage = kStageBase + (sb % R) * kStageBytes;
 #pragma unroll
         for (unsigned m = 0; m < 8u; ++m) {
@@ -511,29 +514,19 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
                 // chunk 7's lookups are on their way: the next superblock's records replace this
                 // one's (its window has landed: see the counts above)
                 __builtin_amdgcn_s_waitcnt(0x0f70u | (kSettleInFlight & 15u) | ((kSettleInFlight >> 4) << 14));
+                rs = row_scale;
                 settle(sb + 1u);
             }
             if (m == 4u) {
                 // this superblock's token scales, while its stage is still held
-                const unsigned at = stage + T * kActPitch + r * NTB * 4u;
-                if constexpr (NTB == 2u) {
-                    const uint2 v = lds_read_uint2(at);
-                    ts[0] = __uint_as_float(v.x);
-                    ts[1] = __uint_as_float(v.y);
-                } else {
-                    ts[0] = __uint_as_float(lds_read_u32(at));
-                }
+                ts = __uint_as_float(lds_read_u32(stage + T * kActPitch + (r * NTB + (NTB == 2u ? h : 0u)) * 4u));
             }
             if (m == 6u) {
-                // the row scales of this superblock, for the scaling below
+                // the scaling's factors: block h of the instruction is the rows against token block h
+                v32f zero;
 #pragma unroll
-                for (unsigned q = 0; q < 4u; ++q) {
-                    const uint4 v = lds_read_uint4(row_scale_at + (sb & 1u) * 128u + (8u * q + 4u * h) * 4u);
-                    rs[4u * q] = __uint_as_float(v.x);
-                    rs[4u * q + 1u] = __uint_as_float(v.y);
-                    rs[4u * q + 2u] = __uint_as_float(v.z);
-                    rs[4u * q + 3u] = __uint_as_float(v.w);
-                }
+                for (unsigned i = 0; i < 32u; ++i) zero[i] = 0.0f;
+                scale = __builtin_amdgcn_mfma_f32_32x32x1f32(rs, ts, zero, 0, 0, 0);
             }
             if (m == kBarrierSlot) {
                 // Every read of this superblock's stage and of the next one's window has returned
@@ -558,7 +551,7 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
 #pragma unroll
                     for (unsigned i = 0; i < 16u; ++i) {
                         const int total = (sum_hi[tb][i] << 7) + sum_lo[tb][i];
-                        const float term = rs[i] * ts[tb] * (float)total;    // each product rounded to float
+                        const float term = scale[16u * tb + i] * (float)total;    // each product rounded to float
                         acc[tb][i] += (double)term;
                     }
             }
