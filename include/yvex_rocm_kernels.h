@@ -393,6 +393,15 @@ int yvex_hip_mhc_ingress_encoded(const float *rows, const float *mixes, const vo
                                  uint64_t streams, uint64_t width, uint64_t iterations, double rms_epsilon,
                                  double mhc_epsilon, double post_multiplier, float *normalized, float *post,
                                  float *combination, int *status, yvex_hip_stream stream);
+/* yvex_hip_matvec_f32_rows of the mixing function (F32 rows) followed by yvex_hip_mhc_ingress_encoded, in two launches:
+ * the ingress adds the partial sums itself. UNSUPPORTED where yvex_hip_matvec_f32_rows_launches says 1 for the operands. */
+int yvex_hip_mhc_ingress_projecting(const float *rows, const float *function, const void *scale,
+                                    unsigned int scale_qtype, const void *base, unsigned int base_qtype,
+                                    const void *norm, unsigned int norm_qtype, uint64_t row_count,
+                                    uint64_t streams, uint64_t width, uint64_t iterations, double rms_epsilon,
+                                    double mhc_epsilon, double post_multiplier, float *normalized, float *post,
+                                    float *combination, void *scratch, uint64_t scratch_bytes, int *status,
+                                    yvex_hip_stream stream);
 int yvex_hip_mhc_egress(const float *core, const float *rows, const float *post,
                         const float *combination, uint64_t row_count, uint64_t streams,
                         uint64_t width, float *output, int *status, yvex_hip_stream stream);

@@ -626,6 +626,40 @@ def test_ingress_of_few_rows_is_that_of_many(gpu, oracle, streams, width):
     assert int(status.item()) == 1
 
 
+# one and two workgroups a row, 256 and 1024 threads, 16- and 32-row tiles of the projection, two to 56 splits, one to four
+# partial sums a thread
+@pytest.mark.parametrize("streams,width,count", [(2, 512, 8), (4, 1024, 20), (4, 1920, 300), (4, 4096, 8), (4, 4096, 96), (4, 4096, 129),
+                                                 (4, 4096, 333), (7, 1024, 33), (7, 4096, 16), (7, 4096, 130)])
+def test_ingress_that_joins_its_projection_equals_the_launches_apart(gpu, oracle, streams, width, count):
+    from yvex_amd import kernels as K, load_library
+    g, mixing, expanded = oracle.Generator(46, f"projecting.{streams}.{width}"), (streams + 2) * streams, streams * width
+    rows, function = dev(g.normal(count * expanded).reshape(count, expanded), gpu), dev(g.normal(mixing * expanded).reshape(mixing, expanded), gpu)
+    function /= expanded ** 0.5
+    scale, base, norm = (dev(g.normal(n), gpu) for n in (3, mixing, width))
+    lib, status = load_library(), K.new_status(gpu)
+    lib.yvex_hip_matvec_f32_scratch_bytes.restype = C.c_uint64
+    need = lib.yvex_hip_matvec_f32_scratch_bytes(u64(mixing), u64(expanded), u64(count))
+    scratch = torch.zeros(need // 8, dtype=torch.float64, device=gpu)
+    kw = dict(streams=streams, width=width, iterations=20, rms_epsilon=1e-6, mhc_epsilon=1e-6, post_multiplier=2.0)
+
+    def projecting(n):
+        out = [torch.zeros(n, w, device=gpu) for w in (width, streams, streams * streams)]
+        rc = lib.yvex_hip_mhc_ingress_projecting(
+            ptr(rows), ptr(function), ptr(scale), C.c_uint(0), ptr(base), C.c_uint(0), ptr(norm), C.c_uint(0), u64(n), u64(streams),
+            u64(width), u64(20), C.c_double(1e-6), C.c_double(1e-6), C.c_double(2.0), *(ptr(t) for t in out), ptr(scratch), u64(need),
+            ptr(status), C.c_void_p(torch.cuda.current_stream().cuda_stream))
+        return rc, out
+
+    mixes = K.matvec_f32_rows(function, rows, status, scratch=scratch.view(torch.uint8))
+    want = K.mhc_ingress(rows, mixes, scale, base, norm, status=status, **kw)
+    rc, got = projecting(count)
+    assert rc == 0 and int(status.item()) == 0
+    assert all(same_bits(a, b.reshape(a.shape)) for a, b in zip(got, want))
+    assert projecting(7)[0] != 0                   # a batch whose projection is one launch
+    function[mixing - 1, 5] = float("inf")
+    assert projecting(count)[0] == 0 and int(status.item()) == 1
+
+
 def _row_with_mean_square_one(rng, width):
     """bf16 values, one of them 1.5, whose squares add up to `width` within 2^-70, most of them far below a unit in the
     last place of the large ones' squares: what a sum in double rounds to depends on its order."""

@@ -120,6 +120,11 @@ __device__ __forceinline__ float sinkhorn4(float m, unsigned iterations, double 
 // one-row launch is 2.6 us of getting there and back and then waits of one workgroup for itself, by 1 / 96 / 128 rows
 // 9.6 / 11.0 / 11.4 -> 7.7 / 9.8 / 10.4 us, of 7168 values 13.7 / 15.4 / 16.0 -> 10.7 / 13.7 / 15.2. Where two workgroups
 // have to share a compute unit the second pass over the row costs what it gave: 160 rows 11.8 and 14.7, 16.6 and 24.4.
+// With `parts` the mixing projection's sums arrive as its `splits` partial sums (doubles, [split][row][mixing row]), requested ahead
+// of the row and put into LDS behind it; whoever uses a sum adds its parts in their order, as matvec_f32_join_kernel
+// does, whose launch is not needed then: 6.5 us a layer of 96 rows, 4.7 of 333.
+constexpr unsigned kPartsAThread = 4u;    // 63 mixing rows in 64 splits, or in 16 of an expanded row under 8192 values
+
 template <unsigned THREADS, bool SPLIT>
 __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
     const float *__restrict__ rows, const float *__restrict__ mixes, const void *__restrict__ scale_values,
@@ -127,7 +132,7 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
     unsigned base_qtype, unsigned norm_qtype, unsigned streams, unsigned width,
     unsigned iterations, double rms_epsilon, double mhc_epsilon, double post_multiplier,
     float *__restrict__ normalized, float *__restrict__ post, float *__restrict__ combination,
-    int quads, int held, int *status)
+    int quads, int held, const double *__restrict__ parts, unsigned splits, unsigned parts_at, int *status)
 {
     __shared__ float base[64], scale[3];      // (streams + 2) * streams <= 63 mixing rows
     extern __shared__ __align__(16) float collapsed[];   // width values; behind them, where held, the row as bf16
@@ -140,8 +145,25 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
     const bool mixes_only = SPLIT && (blockIdx.x & 1u) != 0u, mixes_here = !SPLIT || mixes_only;
     const unsigned expanded = streams * width, mixing_rows = (streams + 2u) * streams;
     const float *in = rows + row * expanded;
-    const float *mix = mixes + row * mixing_rows;
+    const float *mix = parts ? nullptr : mixes + row * mixing_rows;
     bool bad = false;    // quads: width is a multiple of four and every row starts 16-byte aligned
+    double *const parts_held = reinterpret_cast<double *>(collapsed + parts_at);
+    double part[kPartsAThread];
+    if (parts) {
+        const unsigned long long row_count = SPLIT ? gridDim.x >> 1 : gridDim.x;
+#pragma unroll
+        for (unsigned k = 0; k < kPartsAThread; ++k) {
+            const unsigned at = tid + k * THREADS, z = at / mixing_rows;
+            part[k] = z < splits ? parts[(z * row_count + row) * mixing_rows + (at - z * mixing_rows)] : 0.0;
+        }
+    }
+    auto mix_of = [&](unsigned index) {
+        if (!parts) return mix[index];
+        double sum = parts_held[index];
+        for (unsigned z = 1; z < splits; ++z) sum += parts_held[z * mixing_rows + index];
+        bad |= !finite_f32((float)sum);
+        return (float)sum;
+    };
 
     // mean square of the bf16-rounded residual (a value that is not finite makes the sum not finite)
     double squares = 0.0;
@@ -177,24 +199,29 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
     bad |= !finite_f64(squares);
     if (tid < mixing_rows) {
         base[tid] = coefficient(base_values, base_qtype, tid);
-        bad |= !finite_f32(base[tid]) || !finite_f32(mix[tid]);
+        bad |= !finite_f32(base[tid]) || (!parts && !finite_f32(mix[tid]));
+    }
+    if (parts) {
+#pragma unroll
+        for (unsigned k = 0; k < kPartsAThread; ++k)
+            if (tid + k * THREADS < splits * mixing_rows) parts_held[tid + k * THREADS] = part[k];
     }
     if (tid < 3u) {
         scale[tid] = coefficient(scale_values, scale_qtype, tid);
         bad |= !finite_f32(scale[tid]);
     }
-    // (the barriers inside the sum publish base and scale to the threads that read them below)
+    // (the barriers inside the sum publish base, scale and the partial sums to the threads that read them below)
     const double inverse = 1.0 / sqrt(workgroup_sum<THREADS / 64u>(squares, slots) / (double)expanded + rms_epsilon);
     bad |= !finite_f64(inverse);
 
     // (the two sigmoids of a stream in different wavefronts)
     if (!mixes_only && tid < streams) {
-        const double pre = sigmoid_f64((double)mix[tid] * inverse * (double)scale[0] + (double)base[tid]);
+        const double pre = sigmoid_f64((double)mix_of(tid) * inverse * (double)scale[0] + (double)base[tid]);
         gate[tid] = pre + mhc_epsilon;
     } else if (!mixes_only && tid >= 64u && tid < 64u + streams) {
         const unsigned s = tid - 64u;
         post[row * streams + s] = (float)(post_multiplier * sigmoid_f64(
-            (double)mix[streams + s] * inverse * (double)scale[1] + (double)base[streams + s]));
+            (double)mix_of(streams + s) * inverse * (double)scale[1] + (double)base[streams + s]));
     }
     __syncthreads();
 
@@ -210,7 +237,7 @@ __global__ __launch_bounds__(THREADS) void mhc_ingress_kernel(
         const bool cell = held < cells;
         const unsigned r = cell ? held / streams : 0u, c = cell ? held % streams : 0u;
         const unsigned index = 2u * streams + (cell ? held : 0u);
-        float m = (float)((double)mix[index] * inverse * (double)scale[2] + (double)base[index]);
+        float m = (float)((double)mix_of(index) * inverse * (double)scale[2] + (double)base[index]);
         double maximum = -__builtin_inf(), total = 0.0;
         for (unsigned k = 0; k < streams; ++k)
             maximum = fmax(maximum, (double)__shfl(m, (int)(r * streams + k), kWave));
@@ -442,14 +469,21 @@ static bool envelope_shape_ok(uint64_t row_count, uint64_t streams, uint64_t wid
            row_count <= 0x7fffffffull / ((width + kEnvelopeThreads - 1u) / kEnvelopeThreads);
 }
 
+// The mixing projection that the ingress joins: its F32 weight rows, and scratch memory for the partial sums.
+struct IngressProjection {
+    const float *weights;
+    void *scratch;
+    uint64_t scratch_bytes;
+};
+
 static int launch_mhc_ingress(const float *rows, const float *mixes, const void *scale, unsigned scale_qtype,
                               const void *base, unsigned base_qtype, const void *norm, unsigned norm_qtype,
                               uint64_t row_count, uint64_t streams, uint64_t width, uint64_t iterations,
                               double rms_epsilon, double mhc_epsilon, double post_multiplier,
                               float *normalized, float *post, float *combination, int *status,
-                              yvex_hip_stream stream)
+                              yvex_hip_stream stream, const IngressProjection *projection = nullptr)
 {
-    if (!rows || !mixes || !scale || !base || !norm || !normalized || !post || !combination || !status)
+    if (!rows || (!mixes && !projection) || !scale || !base || !norm || !normalized || !post || !combination || !status)
         return ST_INVALID_ARG;
     const unsigned qtypes[3] = {scale_qtype, base_qtype, norm_qtype};
     const void *const vectors[3] = {scale, base, norm};
@@ -481,13 +515,27 @@ static int launch_mhc_ingress(const float *rows, const float *mixes, const void 
     const bool split = 2u * row_count <= (uint64_t)compute_units(), wide = streams * width >= 8192u;
     const unsigned collapsed_bytes = (unsigned)(width * sizeof(float)), row_bytes = (unsigned)(2u * streams * width);
     const int held = split && quads && streams <= 4u && collapsed_bytes + row_bytes <= kEnvelopeLdsBytes;
-    const unsigned lds = collapsed_bytes + (held ? row_bytes : 0u);
+    const unsigned parts_at = (collapsed_bytes + (held ? row_bytes : 0u) + 7u) & ~7u;
+    unsigned splits = 0u, lds = parts_at;
+    if (projection) {
+        const uint64_t mixing_rows = (streams + 2u) * streams, expanded = streams * width;
+        splits = f32_rows_splits(mixing_rows, expanded, row_count);
+        if (yvex_hip_matvec_f32_rows_launches(projection->weights, mixing_rows, expanded, rows, row_count, expanded,
+                                              projection->scratch, projection->scratch_bytes) != 2u ||
+            splits * mixing_rows > kPartsAThread * (wide ? 1024u : 256u))
+            return ST_UNSUPPORTED;
+        lds += (unsigned)(splits * mixing_rows * sizeof(double));
+        if (lds > kEnvelopeLdsBytes) return ST_UNSUPPORTED;
+        const int rc = launch_f32_rows_parts(projection->weights, mixing_rows, expanded, rows, row_count, expanded,
+                                             (double *)projection->scratch, status, as_stream(stream));
+        if (rc) return rc;
+    }
     const auto kernel = wide ? (split ? mhc_ingress_kernel<1024, true> : mhc_ingress_kernel<1024, false>)
                              : (split ? mhc_ingress_kernel<256, true> : mhc_ingress_kernel<256, false>);
     kernel<<<(unsigned)(split ? 2u * row_count : row_count), wide ? 1024 : 256, lds, as_stream(stream)>>>(
         rows, mixes, scale, base, norm, scale_qtype, base_qtype, norm_qtype, (unsigned)streams, (unsigned)width,
         (unsigned)iterations, rms_epsilon, mhc_epsilon, post_multiplier, normalized, post, combination, quads, held,
-        status);
+        projection ? (const double *)projection->scratch : nullptr, splits, parts_at / 4u, status);
     return check_launch("mhc_ingress");
 }
 
@@ -515,6 +563,21 @@ extern "C" int yvex_hip_mhc_ingress_encoded(const float *rows, const float *mixe
     return launch_mhc_ingress(rows, mixes, scale, scale_qtype, base, base_qtype, norm, norm_qtype, row_count,
                               streams, width, iterations, rms_epsilon, mhc_epsilon, post_multiplier, normalized,
                               post, combination, status, stream);
+}
+
+extern "C" int yvex_hip_mhc_ingress_projecting(const float *rows, const float *function, const void *scale,
+                                               unsigned int scale_qtype, const void *base,
+                                               unsigned int base_qtype, const void *norm,
+                                               unsigned int norm_qtype, uint64_t row_count, uint64_t streams,
+                                               uint64_t width, uint64_t iterations, double rms_epsilon,
+                                               double mhc_epsilon, double post_multiplier, float *normalized,
+                                               float *post, float *combination, void *scratch,
+                                               uint64_t scratch_bytes, int *status, yvex_hip_stream stream)
+{
+    const IngressProjection projection{function, scratch, scratch_bytes};
+    return launch_mhc_ingress(rows, nullptr, scale, scale_qtype, base, base_qtype, norm, norm_qtype, row_count, streams,
+                              width, iterations, rms_epsilon, mhc_epsilon, post_multiplier, normalized, post,
+                              combination, status, stream, &projection);
 }
 
 extern "C" int yvex_hip_mhc_egress(const float *core, const float *rows, const float *post,

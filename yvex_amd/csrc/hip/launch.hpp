@@ -75,6 +75,12 @@ int launch_q4k_rows_staged(const uint8_t *encoded, uint64_t row_count, uint64_t 
                           const float *additive, float *out, uint64_t out_stride, bool output_bf16,
                           int *status, hipStream_t stream);
 
+// The first launch of a split F32 projection (matvec.hip; operands for which yvex_hip_matvec_f32_rows_launches says 2): the
+// partial sums into parts[split][input row][weight row], and how many splits there are.
+unsigned f32_rows_splits(uint64_t row_count, uint64_t row_width, uint64_t input_rows);
+int launch_f32_rows_parts(const float *weights, uint64_t row_count, uint64_t row_width, const float *input,
+                          uint64_t input_rows, uint64_t input_stride, double *parts, int *status, hipStream_t stream);
+
 inline hipStream_t as_stream(yvex_hip_stream s) { return reinterpret_cast<hipStream_t>(s); }
 
 }  // namespace yvex

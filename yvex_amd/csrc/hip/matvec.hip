@@ -1431,7 +1431,7 @@ static ScalarTiles f32_rows_tiles(uint64_t row_count, uint64_t row_width, uint64
 }
 
 // Splits of an F32 projection over a row batch; 0 where it is one launch: a row of too few columns at decode width.
-static unsigned f32_rows_splits(uint64_t row_count, uint64_t row_width, uint64_t input_rows)
+unsigned yvex::f32_rows_splits(uint64_t row_count, uint64_t row_width, uint64_t input_rows)
 {
     if (input_rows < 8u || row_width % 128u) return 0u;
     const unsigned columns = f32_rows_column_splits(row_width);
@@ -1544,6 +1544,14 @@ static int launch_f32_rows_parts(const MatvecArgs &a, yvex_hip_stream stream)
                                        f32_rows_splits(a.row_count, a.row_width, a.input_rows)), 256, 0,
                                   as_stream(stream)>>>(a);
     return check_launch("matvec_f32_rows.parts");
+}
+
+int yvex::launch_f32_rows_parts(const float *weights, uint64_t row_count, uint64_t row_width, const float *input,
+                                uint64_t input_rows, uint64_t input_stride, double *parts, int *status, hipStream_t stream)
+{
+    return ::launch_f32_rows_parts(MatvecArgs{(const unsigned char *)weights, row_count, row_width, row_width * 4u, input,
+                                              input_rows, input_stride, nullptr, nullptr, row_count, 0, status, parts,
+                                              nullptr, 0}, reinterpret_cast<yvex_hip_stream>(stream));
 }
 
 static int launch_f32_rows_split(const MatvecArgs &a, yvex_hip_stream stream)
