@@ -10,7 +10,8 @@
 //     total = fmaf(d_b * d_a, float(dot_b), total)         b = 0 .. 7 in order, floats, from zero
 //     row  += double(total)                                superblock by superblock, rounded to float once
 // A block has a scale of its own, so every matrix instruction starts anew and its sixteen
-// results a lane are brought to float, scaled and chained on the vector ALU (three instructions each).
+// results a lane are brought to float and chained on the vector ALU (two instructions each); the products of the
+// scales come from the matrix cores (scale_products; the 16 x 16 tiles multiply).
 //
 // A workgroup owns 32 weight rows x 32 input rows; its four waves take every fourth superblock
 // (eight blocks, 272 bytes a row) and their partial tiles are added in wave order, so results do
@@ -103,14 +104,30 @@ __device__ __forceinline__ uint4 read16(unsigned address)
 
 constexpr unsigned kStagedPitch = 272u;
 
+// The products d_b * d_a of two neighbouring blocks where their sums are, sixteen of the first and sixteen of the second: two outer
+// products on one V_MFMA_F32_32X32X1_2B_F32, the bits of sixteen multiplications a block. Lane (r, h) brings input row r's
+// scale and that of weight row r's block h of the two. It takes 64 cycles of the matrix cores for 128 of the vector ALU,
+// eleven LDS reads a superblock and sixteen registers (a V_MFMA_F32_32X32X2_F32 a block, 64 cycles for 64, had made the 128 x 128
+// tiles 6 % slower). 450 -> 314 vector instructions a superblock on the 128 x 128 tiles, 466 -> 333 on the 32 x 32 ones. us a call
+// before and after, quantization and completion included: 4096 x 4096 by 40 / 96 / 200 / 333 / 512 / 2048 rows 25.9 / 29.4 / 43.1 / 50.8 /
+// 53.8 / 133.5 -> 23.6 / 27.8 / 36.3 / 47.5 / 50.8 / 126.8, 7168 x 2048 by 700 67 -> 59, 129 280 x 7168 by 3 with its selection
+// 216 -> 208. The kernels that call this are bounded to 256 registers: with more to spend the compiler keeps the products in
+// accumulation registers and moves each out.
+__device__ __forceinline__ v32f scale_products(float d_a, unsigned scale_bits)
+{
+    v32f zero;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) zero[i] = 0.0f;
+    return __builtin_amdgcn_mfma_f32_32x32x1f32(d_a, f16_bits_to_float(scale_bits), zero, 0, 0, 0);
+}
+
 // One superblock out of LDS: lane (r, h)'s weight row at `w_row` (272 bytes), its input row's codes, of which it holds
 // sixteen bytes a block, at `a_row`, and the scales of the input rows that it has sums of, four at a time, at `scales`.
-__device__ __forceinline__ void q80_superblock(unsigned w_row, unsigned a_row, unsigned scales, unsigned h, float scale, double (&acc)[16])
+__device__ __forceinline__ void q80_superblock(unsigned w_row, unsigned a_row, unsigned scale_at, unsigned h, float scale, double (&acc)[16])
 {
-    float d_a[16], total[16];
+    float total[16];
     uint4 lo[2], hi[2] = {};
     v4i tokens[2];
-    unsigned scale_bits[2];
     auto read_block = [&](unsigned c) {
         const unsigned slot = c % 2u;
         const unsigned start_at = c % 2u == 0u ? 34u * c : 34u * c + 2u;      // the lane's window: + 16 h
@@ -123,7 +140,6 @@ __device__ __forceinline__ void q80_superblock(unsigned w_row, unsigned a_row, u
             hi[slot].x = two.x;
             hi[slot].y = two.y;
         } else if (words) hi[slot] = read16(behind);
-        scale_bits[slot] = lds_read_u16(w_row + 34u * c);
         tokens[slot] = lds_read_v4i(a_row + 32u * c);
     };
     auto codes_of = [&](unsigned c) -> v4i {
@@ -138,24 +154,28 @@ __device__ __forceinline__ void q80_superblock(unsigned w_row, unsigned a_row, u
         return codes;
     };
     read_block(0u);
-#pragma unroll
-    for (unsigned q = 0; q < 4u; ++q) {
-        const uint4 d = read16(scales + 32u * q);
-        d_a[4u * q] = __uint_as_float(d.x); d_a[4u * q + 1u] = __uint_as_float(d.y);
-        d_a[4u * q + 2u] = __uint_as_float(d.z); d_a[4u * q + 3u] = __uint_as_float(d.w);
-    }
+    const float d_a = __uint_as_float(lds_read_u32(scale_at));
+    unsigned scale_bits = lds_read_u16(w_row + 34u * h);
+    v32f step;
 #pragma unroll
     for (unsigned c = 0; c < 8u; ++c) {
         const v4i codes = codes_of(c);
-        const float d_w = f16_bits_to_float(scale_bits[c % 2u]);
         if (c + 1u < 8u) read_block(c + 1u);
         __builtin_amdgcn_sched_barrier(0);
         const v16f dot = block_sums(tokens[c % 2u], codes);
         __builtin_amdgcn_sched_barrier(0);
+        if (c % 2u == 0u) {
+            step = scale_products(d_a, scale_bits);
+            if (c < 6u) scale_bits = lds_read_u16(w_row + 34u * (c + 2u + h));
+        }
+        float value[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) value[i] = __builtin_fmaf(dot[i], scale, -67108864.0f * __uint_as_float(kStartBits));
+        if (c % 2u == 0u) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const float step = d_w * d_a[i], value = __builtin_fmaf(dot[i], scale, -67108864.0f * __uint_as_float(kStartBits));
-            total[i] = c == 0u ? step * value : __builtin_fmaf(step, value, total[i]);
+            const float both = step[16u * (c % 2u) + i];
+            total[i] = c == 0u ? both * value[i] : __builtin_fmaf(both, value[i], total[i]);
         }
         // (the compiler would sink all of it behind the last block, and keep every block's sums until then)
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -179,7 +199,7 @@ constexpr unsigned kPlainLdsBytes = kPlainWaves * kPlainWindow;        // (the p
 // superblock ahead, and the bytes pass through a window of LDS of the wave's own. 4096 x 4096 by 32 / 96 rows
 // 17.0 / 25.6 -> 14.2 / 18.3 us, 2048 x 7168 by 32 / 256 21.2 / 34.1 -> 18.3 / 25.9. (Eight waves, two superblocks each, are
 // 1 to 1.5 us behind: the reduction is longer and the device no fuller.)
-__global__ __launch_bounds__(64 * kPlainWaves) void dense_q8_0_kernel(DenseQ80Args g)
+__global__ __launch_bounds__(64 * kPlainWaves, 2) void dense_q8_0_kernel(DenseQ80Args g)
 {
     extern __shared__ __align__(16) unsigned char dense_q8_0_plain_lds[];
     if (lds_address_of(dense_q8_0_plain_lds) != 0u) {   // operands are addressed by absolute LDS offsets
@@ -239,7 +259,7 @@ __global__ __launch_bounds__(64 * kPlainWaves) void dense_q8_0_kernel(DenseQ80Ar
         // the next superblock's bytes travel while this one is worked on
         request(sb + kPlainWaves < g.blocks ? sb + kPlainWaves : sb);
         wave_lds_fence();
-        q80_superblock(window + r * kStagedPitch, window + kPlainAct + r * kStagedPitch + 16u * h, window + kPlainScales + 16u * h, h,
+        q80_superblock(window + r * kStagedPitch, window + kPlainAct + r * kStagedPitch + 16u * h, window + kPlainScales + 4u * r, h,
                        scale, acc);
         wave_lds_fence();
     }
@@ -389,8 +409,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void dense_q8_0_small_kernel(Dens
 // Eight waves, two per SIMD, each 32 weight rows x 32 input rows over the whole row width: no
 // partial tiles. Here the input rows are the A operand and the weight rows the B operand, so lane
 // (r, h) holds weight row r against input rows 8 (i / 4) + 4 h + i % 4: the block's scale is one
-// value a lane (read from the row's bytes in LDS) and the input rows' scales, needed once a
-// superblock, are sixteen broadcast reads.
+// value a lane (read from the row's bytes in LDS), and so is an input row's (scale_products).
 //
 // ROW_BLOCKS = 4: the tile above (512 lanes, 104 KB of LDS, a workgroup a compute unit);
 // ROW_BLOCKS = 2: 64 weight rows, four waves, 70 KB, two workgroups a compute unit, for batches
@@ -405,7 +424,7 @@ constexpr unsigned staged_lds_bytes(unsigned row_blocks, unsigned token_blocks =
 
 
 template <unsigned ROW_BLOCKS, unsigned TOKEN_BLOCKS = 2u>
-__global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS) void dense_q8_0_staged_kernel(DenseQ80Args g)
+__global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS, 2) void dense_q8_0_staged_kernel(DenseQ80Args g)
 {
     constexpr unsigned kStagedThreads = 64u * ROW_BLOCKS * TOKEN_BLOCKS, kStagedRows = 32u * ROW_BLOCKS;
     constexpr unsigned kStagedTokens = 32u * TOKEN_BLOCKS;
@@ -495,22 +514,19 @@ __global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS) void dense_q8_0_sta
         const unsigned w_row = kStagedWeightBase + buffer * kStagedWeightBytes + (32u * row_block + r) * kStagedPitch;
         const unsigned a_tile = kStagedActBase + buffer * kStagedActBytes + 32u * token_block * kStagedPitch;
 
-        float d_a[16], total[16];   // the input rows' scales; the superblock's chain of eight terms
+        const float d_a = __uint_as_float(lds_read_u32(a_tile + r * kStagedPitch + 256u));   // the lane's input row's scale
+        float total[16];            // the superblock's chain of eight terms
 #pragma unroll
-        for (unsigned i = 0; i < 16u; ++i) {
-            const unsigned token = 8u * (i >> 2) + 4u * h + (i & 3u);
-            d_a[i] = __uint_as_float(lds_read_u32(a_tile + token * kStagedPitch + 256u));
-            total[i] = 0.0f;
-        }
+        for (unsigned i = 0; i < 16u; ++i) total[i] = 0.0f;
         // Three stages in flight, or a wave would run its LDS reads, its matrix instruction and the
         // scaling of the results one after the other: in step k the operands of block k are
         // read, block k - 1 is multiplied and the results of block k - 2 are scaled (vector
         // instructions that issue while the matrix pipe works).
         uint4 lo[2], hi[2] = {};
         v4i tokens[2];
-        unsigned scale_bits[2];
+        unsigned scale_bits = 0u;   // of block c + h
         v16i dot[2];
-        float d_w[2];
+        v32f step;                  // the products of the scales of two blocks (scale_products)
 #pragma unroll
         for (unsigned k = 0; k < 10u; ++k) {
             if (k < 8u) {
@@ -519,7 +535,7 @@ __global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS) void dense_q8_0_sta
                 lo[slot] = read16(w_row + 16u * h + (start & ~15u));
                 // (an even block's window is 20 bytes, an odd block's 16: only block 7's fits one piece)
                 hi[slot] = c % 2u == 0u || (start & 15u) ? read16(w_row + 16u * h + (start & ~15u) + 16u) : lo[slot];
-                scale_bits[slot] = lds_read_u16(w_row + 34u * c);
+                if (c % 2u == 0u) scale_bits = lds_read_u16(w_row + 34u * (c + h));
                 tokens[slot] = lds_read_v4i(a_tile + r * kStagedPitch + 16u * (2u * c + h));
             }
             if (k >= 1u && k < 9u) {
@@ -541,14 +557,14 @@ __global__ __launch_bounds__(64 * ROW_BLOCKS * TOKEN_BLOCKS) void dense_q8_0_sta
 #pragma unroll
                 for (int i = 0; i < 16; ++i) zero[i] = 0;
                 dot[slot] = __builtin_amdgcn_mfma_i32_32x32x32_i8(tokens[slot], codes, zero, 0, 0, 0);
-                d_w[slot] = f16_bits_to_float(scale_bits[slot]);
             }
             if (k >= 2u) {
                 const unsigned slot = k % 2u;           // block k - 2
 #pragma unroll
                 for (int i = 0; i < 16; ++i)
-                    total[i] = __builtin_fmaf(d_w[slot] * d_a[i], (float)dot[slot][i], total[i]);
+                    total[i] = __builtin_fmaf(step[16u * slot + i], (float)dot[slot][i], total[i]);
             }
+            if (k % 2u == 1u && k < 9u) step = scale_products(d_a, scale_bits);      // of blocks k - 1 and k
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
@@ -593,9 +609,8 @@ constexpr unsigned kWideLdsBytes = kWideScaleBase + 2u * kWideTokens * 4u;
 // 4096 x 4096 by 2048 rows 136 -> 129 us (532 TOP/s; eight waves of 32 x 64, two a SIMD, before). No pipe is full: the
 // vector ALU is issued to 66 % of the time, the LDS is busy 40 %, nearly half of it bank conflicts (at a pitch of 272 bytes
 // rows r and r + 16 start on one bank, which the reads of less than 16 bytes meet on), the matrix cores 12 %; a wave waits for
-// data 42 % of its time, copies behind a full wait and a barrier a superblock. The products of the scales as one
-// V_MFMA_F32_32X32X2_F32 a block (the same bits): 137 us, it does not run beside vector instructions. Whole 16-byte reads of a
-// window's end: 131 us.
+// data 42 % of its time, copies behind a full wait and a barrier a superblock. (Counters from before
+// scale_products.) Whole 16-byte reads of a window's end: 131 us.
 __global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80Args g)
 {
     extern __shared__ __align__(16) unsigned char dense_q8_0_lds[];
@@ -658,7 +673,7 @@ __global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80A
         if (sb + 1u < g.blocks) copies(sb + 1u);
         q80_superblock(buffer * kWideWeightBytes + (32u * row_block + r) * kStagedPitch,
                        kWideActBase + buffer * kWideActBytes + (32u * token_block + r) * kStagedPitch + 16u * h,
-                       kWideScaleBase + buffer * (kWideTokens * 4u) + (32u * token_block + 4u * h) * 4u, h, scale, acc);
+                       kWideScaleBase + buffer * (kWideTokens * 4u) + (32u * token_block + r) * 4u, h, scale, acc);
         // the next superblock's copies have landed and every wave is done with this one's buffers
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
@@ -703,8 +718,8 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
     // load (measured at 16 superblocks a row, microseconds: 9 on the 16 x 16 tile and 3.8 more for every such workgroup
     // that a compute unit has besides, 14 on the 32-row tile and 18.5 once two such
     // workgroups share a compute unit, 29 on the 64-row staged tile and 43 once two of them share
-    // a compute unit, 35 on the 128-row tile, 54 on the 128 x 128 tile), so the choice is the number of
-    // rounds each shape needs.
+    // a compute unit, 35 on the 128-row tile, 54 on the 128 x 128 tile; scale_products has since made all but the first 4 to
+    // 15 % faster, with the same order among them), so the choice is the number of rounds each shape needs.
     const uint64_t token_tiles32 = (input_rows + 31u) / 32u;
     const uint64_t token_tiles64 = (input_rows + 63u) / 64u;
     if (token_tiles32 > 65535ull) return ST_BOUNDS;
