@@ -719,7 +719,7 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
     // that a compute unit has besides, 14 on the 32-row tile and 18.5 once two such
     // workgroups share a compute unit, 29 on the 64-row staged tile and 43 once two of them share
     // a compute unit, 35 on the 128-row tile, 54 on the 128 x 128 tile; scale_products has since made all but the first 4 to
-    // 15 % faster, with the same order among them), so the choice is the number of rounds each shape needs.
+    // 15 % faster), so the choice is the number of rounds each shape needs.
     const uint64_t token_tiles32 = (input_rows + 31u) / 32u;
     const uint64_t token_tiles64 = (input_rows + 63u) / 64u;
     if (token_tiles32 > 65535ull) return ST_BOUNDS;

@@ -42,8 +42,8 @@
 //       of both token blocks at once: a product of two floats rounded once, the bits of V_MUL_F32. 363 -> 330 vector and
 //       61 -> 56 LDS instructions a superblock and wave of 64 tokens, and a row's scale stays in its lane's register
 //       (it went through LDS to the lanes that hold the row's sums). 2048 rows of 7168 by eight of 256 experts with uneven routing, us
-//       a layer: 2995 -> 2967. The instruction holds the wave for as long as sixteen multiplications, so it gains half of what it
-//       takes out; at one token block it is level.
+//       a layer: 2995 -> 2967 on one box, 3010 -> 3005 on another. The instruction holds the wave for as long as sixteen
+//       multiplications, which takes most of the gain; at one token block it is level.
 //   Output: accumulator i of lane (r, h) is token r's sum for row 8 (i / 4) + 4 h + i % 4 of the
 //       wave's 32 (gate sums in the first eight, the matching up sums in the last eight when
 //       fused), so a lane stores four consecutive rows of its token, 16 bytes, straight from its
