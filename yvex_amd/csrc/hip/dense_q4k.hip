@@ -27,6 +27,7 @@
 #include "launch.hpp"
 #include "grouped.hpp"
 #include "publish.hpp"
+#include "kquant_limbs.hpp"
 
 namespace yvex {
 
@@ -123,10 +124,8 @@ __device__ __forceinline__ void bsum_limbs(const uint4 (&b)[2], uint2 &lo, uint2
 }
 
 template <unsigned NT>
-__global__ __launch_bounds__(256) void dense_q4k_kernel(DenseQ4kArgs g)
+__global__ __launch_bounds__(256, NT == 1u ? 2 : 1) void dense_q4k_kernel(DenseQ4kArgs g)
 {
-    // per wave: d and dmin of its 32 rows for the superblock in hand; then the partial tiles
-    __shared__ __align__(16) float row_scale[4][2][32];
     __shared__ double partial[3][NT][16][64];
     const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const unsigned r = lane & 31u, h = lane >> 5;
@@ -156,16 +155,12 @@ __global__ __launch_bounds__(256) void dense_q4k_kernel(DenseQ4kArgs g)
         SuperInputs<NT> nxt;
         const unsigned ahead = sb + 4u < g.blocks ? sb + 4u : sb;
         load_super<NT>(g, wrow, arow, ahead, h, nxt);
+        __builtin_amdgcn_sched_barrier(0);      // (they would be requested where they are used)
 
         // scales and minima of the eight sub-blocks, four to a dword (ggml get_scale_min_k4)
         const unsigned s0 = cur.scales.x, s1 = cur.scales.y, s2 = cur.scales.z;
         const unsigned sc_pack[2] = {s0 & 0x3f3f3f3fu, (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u)};
         const unsigned mn_pack[2] = {s1 & 0x3f3f3f3fu, ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u)};
-        if (h == 0u) {
-            row_scale[wave][0][r] = f16_bits_to_float(cur.head & 0xffffu);
-            row_scale[wave][1][r] = f16_bits_to_float(cur.head >> 16);
-        }
-
         v16i lo_sum[NT], hi_sum[NT];
 #pragma unroll
         for (unsigned nt = 0; nt < NT; ++nt)
@@ -189,50 +184,24 @@ __global__ __launch_bounds__(256) void dense_q4k_kernel(DenseQ4kArgs g)
                 hi_sum[nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a_hi, b, hi_sum[nt], 0, 0, 0);
             }
         }
-        // minimum term: m_j (bytes 0..7 of the h = 0 half, zeros elsewhere) against the pair sums
-        v4i m_op = {0, 0, 0, 0};
-        if (h == 0u) {
-            m_op[0] = (int)mn_pack[0];
-            m_op[1] = (int)mn_pack[1];
-        }
-        v16i min_lo[NT], min_hi[NT];
+        // minimum term and products of the scales as in rows_q4k.hip: a K step on f16 operands whose float sums are exact, and two
+        // outer products (d on the lanes of half 0, dmin on the others)
+        const f16x8 m_op = bytes_to_f16(mn_pack[0], mn_pack[1]);
+        const float row_scale = f16_bits_to_float(cur.head >> (16u * h) & 0xffffu);
 #pragma unroll
         for (unsigned nt = 0; nt < NT; ++nt) {
-            uint2 bl, bh;
-            bsum_limbs(cur.bsums[nt], bl, bh);
-            v4i b_lo = {0, 0, 0, 0}, b_hi = {0, 0, 0, 0};
-            if (h == 0u) {
-                b_lo[0] = (int)bl.x; b_lo[1] = (int)bl.y;
-                b_hi[0] = (int)bh.x; b_hi[1] = (int)bh.y;
-            }
-            v16i zero;
+            v16f zero16;
+            v32f zero32;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) zero[i] = 0;
-            min_lo[nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(m_op, b_lo, zero, 0, 0, 0);
-            min_hi[nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(m_op, b_hi, zero, 0, 0, 0);
-        }
-        // d and dmin of the sixteen rows this lane accumulates (written above by the wave itself)
-        wave_lds_fence();
-        float d_of[16], dmin_of[16];
-#pragma unroll
-        for (unsigned q4 = 0; q4 < 4u; ++q4) {
-            const float4 d = *reinterpret_cast<const float4 *>(&row_scale[wave][0][8u * q4 + 4u * h]);
-            const float4 m = *reinterpret_cast<const float4 *>(&row_scale[wave][1][8u * q4 + 4u * h]);
-            d_of[4u * q4] = d.x; d_of[4u * q4 + 1u] = d.y; d_of[4u * q4 + 2u] = d.z; d_of[4u * q4 + 3u] = d.w;
-            dmin_of[4u * q4] = m.x; dmin_of[4u * q4 + 1u] = m.y; dmin_of[4u * q4 + 2u] = m.z;
-            dmin_of[4u * q4 + 3u] = m.w;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (unsigned nt = 0; nt < NT; ++nt) {
-            const float da = cur.act_scale[nt];
+            for (int i = 0; i < 16; ++i) zero16[i] = zero32[i] = zero32[i + 16] = 0.0f;
+            const v16f minimum = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                m_op, q4k_bsum_operand(cur.bsums[nt][0], cur.bsums[nt][1], h), zero16, 0, 0, 0);
+            const v32f scale = __builtin_amdgcn_mfma_f32_32x32x1f32(row_scale, cur.act_scale[nt], zero32, 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const int dot = (hi_sum[nt][i] << 3) + lo_sum[nt][i];
-                const int minimum = (min_hi[nt][i] << 7) + min_lo[nt][i];
-                const float left = (da * d_of[i]) * (float)dot;
-                const float right = (da * dmin_of[i]) * (float)minimum;
+                const float left = scale[i] * (float)dot;
+                const float right = scale[i + 16] * minimum[i];
                 acc[nt][i] += (double)(left - right);
             }
         }
