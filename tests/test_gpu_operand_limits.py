@@ -49,3 +49,19 @@ def test_scales_and_minimums_reach_as_far_as_floats(gpu, oracle, qtype, scales, 
     K.moe_down_rows(weights, act, wl, pairs, experts, out[1], status)
     assert int(status.item()) == 0 and bool(torch.isfinite(out[0]).all())
     assert torch.equal(out[0].view(torch.int32), out[1].view(torch.int32))
+
+
+# more 64-token tiles than compute units, a remainder of tokens and of rows, one superblock and fewer than a workgroup's waves
+@pytest.mark.parametrize("rows,width,inputs", [(8200, 256, 70), (8224, 768, 97), (4112, 1536, 190)])
+def test_q4k_tiles_that_share_a_compute_unit_publish_what_single_ones_do(gpu, oracle, rows, width, inputs):
+    """The first 2048 rows alone are few enough tiles for a compute unit each; the order of every sum is the same."""
+    from yvex_amd import kernels as K
+    g, status = oracle.Generator(47, f"paired.{rows}.{width}"), K.new_status(gpu)
+    weights = dev(g.weights(oracle.Q4_K, rows, width), gpu)
+    act = K.q8k_quantize(dev(g.normal(inputs * width).reshape(inputs, width), gpu), status)
+    units, few, tiles = torch.cuda.get_device_properties(gpu).multi_processor_count, 2048, (inputs + 63) // 64
+    assert (rows + 31) // 32 * tiles > units >= few // 32 * tiles and (rows + 127) // 128 * tiles < units
+    assert few // 16 * ((inputs + 31) // 32) > units            # (no 16 x 16 tiles)
+    many, part = (K.matvec(weights[:count * width // 256 * 144], oracle.Q4_K, count, width, act, input_q8=True, input_rows=inputs,
+                           status=status) for count in (rows, few))
+    assert int(status.item()) == 0 and torch.equal(many[:, :few].contiguous().view(torch.int32), part.view(torch.int32))

@@ -123,8 +123,12 @@ __device__ __forceinline__ void bsum_limbs(const uint4 (&b)[2], uint2 &lo, uint2
     hi = make_uint2(u[0], u[1]);
 }
 
-template <unsigned NT>
-__global__ __launch_bounds__(256, NT == 1u ? 2 : 1) void dense_q4k_kernel(DenseQ4kArgs g)
+// A workgroup that has its compute unit to itself requests a superblock ahead, on as many registers as that takes; where 64-token
+// tiles outnumber the compute units (PAIRED) two of them share one on half the registers and cover each other's loads. us a
+// call one way and the other: 7168 x 2048 by 120 rows 36.3 and 29.0, 4096 x 4096 by 150 42.4 and 36.1, 2048 x 7168 by 300 57.9 and
+// 55.3; with a tile a compute unit or fewer 2048 x 7168 by 200 37.0 and 45.2, 4096 x 4096 by 96 30.0 and 32.4, 1024 x 4096 by 300 30.4 and 33.4.
+template <unsigned NT, bool PAIRED = false>
+__global__ __launch_bounds__(256, NT == 1u || PAIRED ? 2 : 1) void dense_q4k_kernel(DenseQ4kArgs g)
 {
     __shared__ double partial[3][NT][16][64];
     const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -155,7 +159,7 @@ __global__ __launch_bounds__(256, NT == 1u ? 2 : 1) void dense_q4k_kernel(DenseQ
         SuperInputs<NT> nxt;
         const unsigned ahead = sb + 4u < g.blocks ? sb + 4u : sb;
         load_super<NT>(g, wrow, arow, ahead, h, nxt);
-        __builtin_amdgcn_sched_barrier(0);      // (they would be requested where they are used)
+        if (!PAIRED) __builtin_amdgcn_sched_barrier(0);      // (they would be requested where they are used)
 
         // scales and minima of the eight sub-blocks, four to a dword (ggml get_scale_min_k4)
         const unsigned s0 = cur.scales.x, s1 = cur.scales.y, s2 = cur.scales.z;
@@ -448,6 +452,8 @@ int launch_q4k_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t r
         // faster ones (2048 x 7168 at 96 rows: 17 us on 32 x 32 tiles, 21 on 16 x 32; at 256 rows 27 us on 32 x 64).
         if (row_tiles * token_tiles32 <= units)
             dense_q4k_kernel<1><<<dim3((unsigned)row_tiles, (unsigned)token_tiles32), 256, 0, stream>>>(g);
+        else if (row_tiles * token_tiles > units)
+            dense_q4k_kernel<2, true><<<dim3((unsigned)row_tiles, (unsigned)token_tiles), 256, 0, stream>>>(g);
         else
             dense_q4k_kernel<2><<<dim3((unsigned)row_tiles, (unsigned)token_tiles), 256, 0, stream>>>(g);
     }
