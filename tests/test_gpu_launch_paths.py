@@ -627,9 +627,10 @@ def test_ingress_of_few_rows_is_that_of_many(gpu, oracle, streams, width):
 
 
 # one and two workgroups a row, 256 and 1024 threads, 16- and 32-row tiles of the projection, two to 56 splits, one to four
-# partial sums a thread
+# partial sums a thread; rows that fit LDS beside their collapsed values and not beside the partial sums as well; the widest row
 @pytest.mark.parametrize("streams,width,count", [(2, 512, 8), (4, 1024, 20), (4, 1920, 300), (4, 4096, 8), (4, 4096, 96), (4, 4096, 129),
-                                                 (4, 4096, 333), (7, 1024, 33), (7, 4096, 16), (7, 4096, 130)])
+                                                 (4, 4096, 333), (7, 1024, 33), (7, 4096, 16), (7, 4096, 130), (4, 11520, 16),
+                                                 (4, 12288, 8), (4, 12288, 96), (3, 14592, 8), (7, 16384, 8)])
 def test_ingress_that_joins_its_projection_equals_the_launches_apart(gpu, oracle, streams, width, count):
     from yvex_amd import kernels as K, load_library
     g, mixing, expanded = oracle.Generator(46, f"projecting.{streams}.{width}"), (streams + 2) * streams, streams * width

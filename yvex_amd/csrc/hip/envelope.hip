@@ -21,7 +21,6 @@ constexpr unsigned kEnvelopeThreads = 256;
 constexpr unsigned kEnvelopeMaxStreams = 7;       // (streams + 2) * streams <= 64 mixing rows
 constexpr unsigned kEnvelopeMaxWidth = 16384;     // the reference's bound (src/graph/moe.c:453-455)
 constexpr unsigned kEnvelopeLdsBytes = 147456;    // a row of floats and what else fits
-static_assert(kEnvelopeMaxWidth * sizeof(float) <= kEnvelopeLdsBytes, "the collapsed row");
 
 __device__ __forceinline__ bool finite_f64(double v)
 {
@@ -513,19 +512,24 @@ static int launch_mhc_ingress(const float *rows, const float *mixes, const void 
     const int quads = width % 4u == 0u && !(((uintptr_t)rows | (uintptr_t)normalized) & 15u) &&
                       !((uintptr_t)norm & (norm_qtype == QT_F32 ? 15u : 7u));
     const bool split = 2u * row_count <= (uint64_t)compute_units(), wide = streams * width >= 8192u;
-    const unsigned collapsed_bytes = (unsigned)(width * sizeof(float)), row_bytes = (unsigned)(2u * streams * width);
-    const int held = split && quads && streams <= 4u && collapsed_bytes + row_bytes <= kEnvelopeLdsBytes;
-    const unsigned parts_at = (collapsed_bytes + (held ? row_bytes : 0u) + 7u) & ~7u;
-    unsigned splits = 0u, lds = parts_at;
+    unsigned splits = 0u, parts_bytes = 0u;
     if (projection) {
         const uint64_t mixing_rows = (streams + 2u) * streams, expanded = streams * width;
         splits = f32_rows_splits(mixing_rows, expanded, row_count);
         if (yvex_hip_matvec_f32_rows_launches(projection->weights, mixing_rows, expanded, rows, row_count, expanded,
-                                              projection->scratch, projection->scratch_bytes) != 2u ||
-            splits * mixing_rows > kPartsAThread * (wide ? 1024u : 256u))
+                                              projection->scratch, projection->scratch_bytes) != 2u)
             return ST_UNSUPPORTED;
-        lds += (unsigned)(splits * mixing_rows * sizeof(double));
-        if (lds > kEnvelopeLdsBytes) return ST_UNSUPPORTED;
+        if (splits * mixing_rows > kPartsAThread * (wide ? 1024u : 256u)) return ST_BOUNDS;    // (never: kPartsAThread)
+        parts_bytes = (unsigned)(splits * mixing_rows * sizeof(double));
+    }
+    // The collapsed row and the partial sums always fit; the row itself is held where there is room for it besides.
+    static_assert(kEnvelopeMaxWidth * sizeof(float) + kPartsAThread * 1024u * sizeof(double) <= kEnvelopeLdsBytes,
+                  "the collapsed row and the partial sums");
+    const unsigned collapsed_bytes = (unsigned)(width * sizeof(float)), row_bytes = (unsigned)(2u * streams * width);
+    const int held = split && quads && streams <= 4u && collapsed_bytes + row_bytes + parts_bytes <= kEnvelopeLdsBytes;
+    const unsigned parts_at = (collapsed_bytes + (held ? row_bytes : 0u) + 7u) & ~7u, lds = parts_at + parts_bytes;
+    if (projection) {
+        const uint64_t mixing_rows = (streams + 2u) * streams, expanded = streams * width;
         const int rc = launch_f32_rows_parts(projection->weights, mixing_rows, expanded, rows, row_count, expanded,
                                              (double *)projection->scratch, status, as_stream(stream));
         if (rc) return rc;
