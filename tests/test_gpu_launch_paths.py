@@ -100,6 +100,33 @@ def test_projections_that_publish_for_themselves(gpu, oracle, qtype, weight_rows
         b.close()
 
 
+# the most work that a launch ends by itself, and a little more: rows a wave of the product that quantizes
+@pytest.mark.parametrize("qtype,weight_rows,width,inputs,launches", [
+    ("Q8_0", 32768, 256, 1, 1), ("Q8_0", 32769, 256, 1, 2), ("Q8_0", 32768, 512, 2, 1), ("Q8_0", 36001, 512, 2, 2)])
+def test_where_projections_publish_for_themselves(gpu, oracle, qtype, weight_rows, width, inputs, launches):
+    from backend_helpers import Backend
+    from yvex_amd import abi, kernels as K
+    assert torch.cuda.get_device_properties(gpu).multi_processor_count == 256
+    qt, g, b, st = getattr(oracle, qtype), oracle.Generator(18, "published.lines"), Backend(), K.new_status(gpu)
+    few = g.weights(qt, 64, width)
+    encoded = np.tile(few, (weight_rows + 63) // 64)[:len(few) // 64 * weight_rows]
+    x = g.normal(inputs * width).reshape(inputs, width)
+    try:
+        _, base = b.resident(encoded)
+        b.workspace(inputs * (width // 256) * 292 + 4096)
+        rows_in, out, facts, err = b.f32(x), b.empty_f32(inputs * weight_rows), abi.OperationFacts(), abi.Error()
+        for _ in range(2):
+            assert b.lib.yvex_rocm_encoded_matvec(b.handle, base, encoded.nbytes, qt, weight_rows, width, encoded.nbytes // weight_rows,
+                                                  inputs, rows_in, None, 0, None, out, 1, C.byref(facts), C.byref(err)) == 0, err.message
+            assert facts.kernel_launches == launches
+        want = K.matvec(dev(encoded, gpu), qt, weight_rows, width, K.q8k_quantize(dev(x, gpu), st), input_q8=True, input_rows=inputs,
+                        status=st).cpu().numpy()
+        got = b.read_f32(out, inputs * weight_rows).reshape(inputs, weight_rows)
+        assert int(st.item()) == 0 and np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    finally:
+        b.close()
+
+
 # a full round of 128 x 128 tiles with ragged edges on both sides, one and three superblocks a row
 @pytest.mark.parametrize("rows,width,inputs", [(2047, 256, 2040), (1921, 768, 2048)])
 def test_q8_0_wide_tiles_are_the_oracles_bits(gpu, oracle, rows, width, inputs):

@@ -1266,7 +1266,11 @@ static int launch_quantizing(MatvecArgs &a, hipStream_t s, Publisher *publisher)
     const unsigned long long groups = (a.row_count + kHeldWaves - 1ull) / kHeldWaves, most = (unsigned long long)compute_units();
     const unsigned grid = (unsigned)(groups < most ? groups : most);
     const unsigned lds = (unsigned)held_bytes(T, a.row_width / 256ull);
-    a.publication = take_publication(publisher, grid);
+    // The launch ends the operation while a wave has up to eight rows: each row's store goes to memory ahead of the next
+    // row's bytes and is waited for with them. us a call, published by the launch and behind it: 32 768 x 4096 by 1 / 2
+    // rows 30.9 / 33.4 and 30.9 / 33.4, x 1024 17.5 / 21.8 and 18.2 / 22.7; 40 960 x 7168 61.7 / 66.9 and 61.0 / 65.8;
+    // 129 280 x 4096 112.2 / 117.7 and 108.3 / 111.3, x 7168 188.4 / 204.2 and 184.4 / 195.8.
+    a.publication = take_publication(publisher, groups, 8ull * most);
     if (a.row_width <= 2048ull) matvec_q8_0_quantizing_kernel<T, 1><<<grid, kHeldThreads, lds, s>>>(a);
     else if (a.row_width <= 4096ull) matvec_q8_0_quantizing_kernel<T, 2><<<grid, kHeldThreads, lds, s>>>(a);
     else matvec_q8_0_quantizing_kernel<T, 4><<<grid, kHeldThreads, lds, s>>>(a);
