@@ -100,9 +100,11 @@ def test_projections_that_publish_for_themselves(gpu, oracle, qtype, weight_rows
         b.close()
 
 
-# the most work that a launch ends by itself, and a little more: rows a wave of the product that quantizes
+# the most work that a launch ends by itself, and a little more: rows a wave of the product that quantizes, a
+# compute unit for each IQ2_XXS tile
 @pytest.mark.parametrize("qtype,weight_rows,width,inputs,launches", [
-    ("Q8_0", 32768, 256, 1, 1), ("Q8_0", 32769, 256, 1, 2), ("Q8_0", 32768, 512, 2, 1), ("Q8_0", 36001, 512, 2, 2)])
+    ("Q8_0", 32768, 256, 1, 1), ("Q8_0", 32769, 256, 1, 2), ("Q8_0", 32768, 512, 2, 1), ("Q8_0", 36001, 512, 2, 2),
+    ("IQ2_XXS", 4096, 512, 16, 2), ("IQ2_XXS", 2048, 512, 17, 2), ("IQ2_XXS", 4100, 512, 7, 3), ("IQ2_XXS", 1376, 1024, 33, 3)])
 def test_where_projections_publish_for_themselves(gpu, oracle, qtype, weight_rows, width, inputs, launches):
     from backend_helpers import Backend
     from yvex_amd import abi, kernels as K

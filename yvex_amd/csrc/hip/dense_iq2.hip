@@ -175,9 +175,13 @@ int launch_iq2_rows_small(const uint8_t *encoded, uint64_t row_count, uint64_t r
         return ST_BOUNDS;
     if (((uintptr_t)encoded & 3u) || ((uintptr_t)act_q8k & 3u)) return ST_INVALID_ARG;
     YVEX_ALLOW_DYNAMIC_LDS(dense_iq2_kernel, kIq2LdsBytes);
+    // A workgroup has its compute unit to itself, and one that publishes keeps it from the next until its stores are in
+    // memory, so a launch ends the operation while it is one round. us a call, published by the launch and behind it:
+    // 1024 x 4096 by 64 rows 17.8 and 18.3 (one round), 4096 x 4096 by 32 / 48 / 64 23.6 / 29.1 / 34.2 and 22.8 / 27.4 / 31.8 (two, three,
+    // four rounds), 16384 x 4096 by 8 34.3 and 31.7, 2048 x 7168 by 64 / 128 27.1 / 41.4 and 26.3 / 38.8.
     dense_iq2_kernel<<<dim3((unsigned)row_tiles, (unsigned)token_tiles), kIq2Threads, kIq2LdsBytes, stream>>>(
         DenseIq2Args{encoded, row_count, row_bytes, (unsigned)(row_width / 256u), (const unsigned char *)act_q8k, input_rows,
-                     out, output_bf16 ? 1 : 0, status, take_publication(publisher, row_tiles * token_tiles)});
+                     out, output_bf16 ? 1 : 0, status, take_publication(publisher, row_tiles * token_tiles, (uint64_t)compute_units())});
     return check_launch("dense_iq2");
 }
 
