@@ -438,7 +438,11 @@ int launch_q4k_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t r
     if (input_rows <= 32u || small_tiles * token_tiles32 <= units) {
         if (small_tiles > 0x7fffffffull || token_tiles16 > 65535ull) return ST_BOUNDS;
         const dim3 grid((unsigned)small_tiles, (unsigned)token_tiles16);
-        g.publication = take_publication(publisher, small_tiles * token_tiles16);
+        // A launch ends the operation while a compute unit has up to five of its tiles: the next ones wait for the stores of
+        // those before them. us a call, published by the launch and behind it: 4096 x 512 by 32 rows (two tiles a compute
+        // unit) 14.6 and 14.9, 16384 x 4096 by 16 (four) 25.6 and 26.5, 8192 x 512 by 32 (four) 17.9 and 17.6; 12288 x 512 / 4096 by 32 (six)
+        // 18.9 / 31.4 and 18.5 / 31.5, 16384 x 512 / 2048 by 32 (eight) 21.1 / 27.3 and 20.1 / 27.1.
+        g.publication = take_publication(publisher, small_tiles * token_tiles16, 5u * units);
         if (small_tiles * token_tiles16 <= units) dense_q4k16_kernel<8><<<grid, 512, 0, stream>>>(g);
         else dense_q4k16_kernel<4><<<grid, 256, 0, stream>>>(g);
     } else {
