@@ -101,11 +101,13 @@ def test_projections_that_publish_for_themselves(gpu, oracle, qtype, weight_rows
 
 
 # the most work that a launch ends by itself, and a little more: rows a wave of the product that quantizes, a
-# compute unit for each IQ2_XXS tile and for five Q4_K ones
+# compute unit for each IQ2_XXS tile and for five Q4_K ones, the
+# longest rows that a wave has two of
 @pytest.mark.parametrize("qtype,weight_rows,width,inputs,launches", [
     ("Q8_0", 32768, 256, 1, 1), ("Q8_0", 32769, 256, 1, 2), ("Q8_0", 32768, 512, 2, 1), ("Q8_0", 36001, 512, 2, 2),
     ("IQ2_XXS", 4096, 512, 16, 2), ("IQ2_XXS", 2048, 512, 17, 2), ("IQ2_XXS", 4100, 512, 7, 3), ("IQ2_XXS", 1376, 1024, 33, 3),
-    ("Q4_K", 20480, 256, 13, 2), ("Q4_K", 20481, 256, 13, 3), ("Q4_K", 10250, 512, 32, 3)])
+    ("Q4_K", 20480, 256, 13, 2), ("Q4_K", 20481, 256, 13, 3), ("Q4_K", 10250, 512, 32, 3),
+    ("Q4_K", 24, 4096, 1, 2), ("Q4_K", 24, 4352, 1, 3), ("Q2_K", 24, 4096, 3, 2), ("Q2_K", 24, 4352, 3, 3), ("IQ2_XXS", 22, 4608, 2, 3)])
 def test_where_projections_publish_for_themselves(gpu, oracle, qtype, weight_rows, width, inputs, launches):
     from backend_helpers import Backend
     from yvex_amd import abi, kernels as K

@@ -979,12 +979,18 @@ static int launch_block_even(const MatvecArgs &a, hipStream_t stream)
     return check_launch("matvec");
 }
 
+// Rows of up to 4096 columns, of which a workgroup has eight or more, end the operation by themselves; longer ones take a wave
+// each, and the four of a workgroup are too little to wait for. us a call, published by the launch and behind it: 8192 x 4096 by
+// 1 / 3 rows Q4_K 15.7 / 22.9 and 16.0 / 22.7, 65536 x 1024 by 1 / 3 17.9 / 30.8 and 18.4 / 31.0, 16384 x 4096 by 1 18.6 and 19.2; but 4096 x 7168 by
+// 1 / 2 / 3 16.5 / 21.5 / 24.0 and 16.4 / 20.5 / 22.5, 1024 x 7168 by 1 13.9 and 13.8, IQ2_XXS 6144 x 7168 by 1 / 3 18.6 / 26.2 and 18.3 / 25.5.
+constexpr uint64_t row_publishing_groups(int lanes_a_row) { return lanes_a_row < 64 ? kPublishingGroups : 0u; }
+
 template <unsigned QT, int L>
 static int launch_dense_row(MatvecArgs &a, hipStream_t stream, Publisher *publisher)
 {
     const unsigned long long grid = (a.row_count + 4ull * (64u / L) - 1ull) / (4ull * (64u / L));
     if (grid > 0x7fffffffull) return ST_BOUNDS;
-    a.publication = take_publication(publisher, grid);
+    a.publication = take_publication(publisher, grid, row_publishing_groups(L));
     dense_row_q8k_kernel<QT, L><<<(unsigned)grid, 256, 0, stream>>>(a);
     return check_launch("matvec.row");
 }
@@ -1004,7 +1010,7 @@ static int launch_dense_fewrows(MatvecArgs &a, hipStream_t stream, Publisher *pu
 {
     const unsigned long long grid = (a.row_count + 4ull * (64u / L) - 1ull) / (4ull * (64u / L));
     if (grid > 0x7fffffffull) return ST_BOUNDS;
-    a.publication = take_publication(publisher, grid);
+    a.publication = take_publication(publisher, grid, row_publishing_groups(L));
     dense_fewrows_q8k_kernel<QT, L><<<(unsigned)grid, 256, 0, stream>>>(a);
     return check_launch("matvec.fewrows");
 }
