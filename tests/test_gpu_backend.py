@@ -294,6 +294,26 @@ def test_select_greedy_rows(backend, oracle):
     assert facts.kernel_launches == 2
 
 
+# either side of the number of rows up to which the selection's launch brings its results to the host itself
+@pytest.mark.parametrize("rows", [16, 17, 300])
+@pytest.mark.parametrize("width", [700, 9000])
+def test_select_greedy_rows_of_batches(backend, oracle, rows, width):
+    b, rng = backend, np.random.default_rng(12)
+    b.workspace(1 << 17)
+    values = rng.standard_normal((rows, width)).astype(np.float32)
+    values[rows - 1, [3, width - 1]] = 9.0
+    bad = values.copy()
+    bad[rows // 2, 5] = np.inf
+    good, bad = b.f32(values), b.f32(bad)
+    _, *want = oracle.argmax_f32(values)
+    for _ in range(3):
+        rc, tokens, best, ties, facts, err = run_greedy(b, good, rows, width)
+        assert rc == 0, err.message
+        assert all(np.array_equal(a, w) for a, w in zip((tokens, best, ties), want)) and ties[rows - 1] == 2
+        rc, tokens, best, ties, _, _ = run_greedy(b, bad, rows, width)
+        assert rc == abi.FORMAT and not tokens.any() and not best.any() and not ties.any()
+
+
 def sweep_image_decision(experts, rows, width, consumer):
     """The decision that asks derived_layout_plan/build for the expert sweeps' image."""
     d = abi.ExecutionDecision()

@@ -303,10 +303,12 @@ static int launch_argmax(const float *values, uint64_t row_count, uint64_t row_w
     if (((uintptr_t)values & 3u) || ((uintptr_t)scratch & 7u)) return ST_INVALID_ARG;
     const uint64_t need = yvex_hip_argmax_scratch_bytes(row_count, row_width);
     hipStream_t s = as_stream(stream);
-    // (what crosses to the host is bounded like what a publishing launch of its own brings there)
-    if (row_count * 16u > YVEX_HIP_PUBLISH_MAX_BYTES) publisher = nullptr;
+    // A publishing launch stores a row's results on the host word by word and waits for them there; a launch of its own
+    // brings those of many rows in whole lines. us a selection, published by the launch and behind it: rows of 1024 values
+    // by 1 / 16 / 64 / 256 / 2048 rows 16.7 / 18.0 / 21.5 / 24.3 / 122.4 and 17.3 / 18.6 / 19.4 / 21.0 / 67.1, of 129 280 by 1 / 16 / 48
+    // 16.0 / 17.7 / 22.5 and 17.2 / 17.7 / 20.5.
     const Selection selection{selected_tokens, selected_values, (unsigned long long *)tie_counts, row_count,
-                              take_publication(publisher, row_count)};
+                              take_publication(publisher, row_count, 16u)};
     if (need && scratch && scratch_bytes >= need) {
         const unsigned spans = (unsigned)((row_width + kSpanElements - 1u) / kSpanElements);
         argmax_spans_kernel<<<dim3(spans, (unsigned)row_count), kSpanThreads, 0, s>>>(
