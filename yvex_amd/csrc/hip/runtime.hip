@@ -66,17 +66,15 @@ __global__ void fill_u32_kernel(uint32_t *dst, uint32_t value, uint64_t count)
 __global__ __launch_bounds__(256) void publish_kernel(const uint32_t *source, unsigned words, int *status, int clear,
                                                       uint32_t *host, uint32_t sequence)
 {
-    int raised = 0;
-    if (threadIdx.x == 0u) {
-        raised = *status;
-        if (clear && raised) *status = 0;
-    }
+    const int raised = threadIdx.x == 0u ? *status : 0;      // (nobody waits for it ahead of the copies)
     if (words) {
         for (unsigned i = threadIdx.x; i < words; i += 256u) host[kPublishedHeadWords + i] = source[i];
         __threadfence_system();      // every thread's host words are out before the sequence number is
         __syncthreads();
     }
-    if (threadIdx.x == 0u) publish_status(host, sequence, raised);
+    if (threadIdx.x != 0u) return;
+    if (clear && raised) *status = 0;
+    publish_status(host, sequence, raised);
 }
 
 // Streaming read of a buffer with 16-byte loads; every lane folds what it read into one word so
