@@ -878,8 +878,9 @@ sequence:
         split = lend && yvex_hip_matvec_f32_rows_launches(
             (const float *)(uintptr_t)envelope_addresses[0], layer->mhc_mixing_rows, expanded,
             (const float *)rows->device_rows->data, row_count, expanded, AT(pair_outputs), need) == 2u;
-        /* the ingress adds the partial sums itself, a launch less; a batch whose intermediate rows come back to the host
-         * keeps its launches apart, here as at the egress */
+        /* the ingress adds the partial sums itself, a launch less. A batch whose intermediate rows come back to the host needs
+         * none of it in memory here (at the egress it does), but waits for its copies anyway, and keeps one launch a
+         * stage, which its callers count */
         joined = split && fused_coefficients && !host_rows;
         if (joined) {
             LAUNCH(yvex_hip_mhc_ingress_projecting((const float *)rows->device_rows->data,
