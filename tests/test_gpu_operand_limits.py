@@ -51,6 +51,39 @@ def test_scales_and_minimums_reach_as_far_as_floats(gpu, oracle, qtype, scales, 
     assert torch.equal(out[0].view(torch.int32), out[1].view(torch.int32))
 
 
+# the same for a plain projection: 16 x 16, 32 x 32 and 32 x 64 tiles, those that share a compute unit, tiles staged through
+# LDS; ragged edges on both sides
+@pytest.mark.parametrize("rows,width,inputs", [(50, 512, 20), (2060, 768, 71), (2078, 512, 100), (8200, 256, 41), (8180, 256, 230)])
+@pytest.mark.parametrize("scales,magnitude", [("ordinary", 1.0), ("largest", 2.0 ** 80), ("subnormal", 2.0 ** -108)])
+def test_q4k_projections_reach_as_far_as_floats(gpu, oracle, rows, width, inputs, scales, magnitude):
+    """Against the kernel of a few input rows, which scales on the vector ALU, for every row of the batch, and the CPU path's
+    bits of some."""
+    from yvex_amd import kernels as K
+    g, status = oracle.Generator(48, f"q4k.limits.{rows}.{inputs}"), K.new_status(gpu)
+    packed = g.weights(oracle.Q4_K, rows, width)
+    blocks = packed.reshape(-1, 144)
+    blocks[::2, 4:16] = 255
+    if scales != "ordinary":
+        bits = (np.full(len(blocks), 0x7800) if scales == "largest" else 1 + np.arange(len(blocks)) * 7 % 1023).astype(np.uint16)
+        for offset in (0, 2):
+            blocks[:, offset], blocks[:, offset + 1] = bits & 255, bits >> 8
+    x = g.normal(inputs * width).reshape(inputs, width)
+    x[::3], x[1::3] = 1.0, -1.0
+    x = (x / np.abs(x).max(axis=1, keepdims=True) * magnitude).astype(np.float32)
+    weights, rows_in = dev(packed, gpu), dev(x, gpu)
+
+    def product(first, count):
+        act = K.q8k_quantize(rows_in[first:first + count].contiguous(), status)
+        return K.matvec(weights, oracle.Q4_K, rows, width, act, input_q8=True, input_rows=count, status=status)
+    got = product(0, inputs)
+    want = torch.cat([product(first, min(3, inputs - first)) for first in range(0, inputs, 3)])
+    assert int(status.item()) == 0 and bool(torch.isfinite(got).all())
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+    picked = [0, inputs // 2, inputs - 1]
+    exact = oracle.q8_matvec(oracle.Q4_K, packed, rows, width, oracle.q8k_quantize(x[picked]), len(picked))
+    assert np.array_equal(got[picked].cpu().numpy().view(np.uint32), exact.view(np.uint32))
+
+
 # more 64-token tiles than compute units, a remainder of tokens and of rows, one superblock and fewer than a workgroup's waves
 @pytest.mark.parametrize("rows,width,inputs", [(8200, 256, 70), (8224, 768, 97), (4112, 1536, 190)])
 def test_q4k_tiles_that_share_a_compute_unit_publish_what_single_ones_do(gpu, oracle, rows, width, inputs):
