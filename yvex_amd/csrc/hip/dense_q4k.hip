@@ -15,8 +15,10 @@
 // operand carries sc_j * nibble (at most 63 * 15 = 945) as two int8 limbs, value = 8 hi + lo
 // with lo = (sc_j mod 8) * nibble and hi = (sc_j div 8) * nibble, both at most 105, so each
 // sub-block costs two matrix instructions per 32 tokens and the int32 accumulators run over the
-// whole superblock without rescaling. The minimum term is one more reduction of depth 8 (the m_j
-// against the pair sums of bsums, in two limbs of base 128) through the same instruction.
+// whole superblock without rescaling. The minimum term is one K step of an f16 instruction whose float
+// sums are exact (kquant_limbs.hpp); on the 16 x 16 tiles it is one more reduction of depth 8, the m_j against the pair sums
+// of bsums in two limbs of base 128, through the int8 instruction. Products of the scales are outer products on
+// the matrix cores (rows_q4k.hip), on the 16 x 16 tiles multiplications.
 //
 // A workgroup owns 32 weight rows x 32 or 64 tokens; its four waves take every fourth
 // superblock and their double-precision partial tiles are added in wave order, so results do not depend on
@@ -88,12 +90,8 @@ __device__ __forceinline__ void load_super(const DenseQ4kArgs &g, const unsigned
     (void)g;
 }
 
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-
-// Two int8 limbs of sc * nibble for the four nibbles of one dword (already shifted so that the
-// wanted nibble of every byte sits in its low four bits), value = 8 hi + lo. The 6-bit scale is
-// split as sc = 8 s_hi + s_lo with both parts in 0..7: a limb byte nibble * s is at most 105, so
-// one 16-bit lane multiply scales two bytes at once without a carry from one into the next.
+// q4k_limbs of a whole scale. (Its two parts as arguments leave the registers of two workgroups a compute unit worse off:
+// 4096 x 4096 by 150 rows 35.3 -> 37.4 us, 2048 x 7168 by 300 54.1 -> 59.1.)
 __device__ __forceinline__ void limbs(unsigned x, unsigned sc, unsigned &lo, unsigned &hi)
 {
     const unsigned nibbles = x & 0x0f0f0f0fu;
@@ -106,21 +104,6 @@ __device__ __forceinline__ v4i as_v4i(uint4 v)
 {
     v4i r = {(int)v.x, (int)v.y, (int)v.z, (int)v.w};
     return r;
-}
-
-// Pair sums of the 16 int16 block sums as two int8 limbs (value = 128 hi + lo, lo in 0..127).
-__device__ __forceinline__ void bsum_limbs(const uint4 (&b)[2], uint2 &lo, uint2 &hi)
-{
-    const unsigned w[8] = {b[0].x, b[0].y, b[0].z, b[0].w, b[1].x, b[1].y, b[1].z, b[1].w};
-    unsigned l[2] = {0u, 0u}, u[2] = {0u, 0u};
-#pragma unroll
-    for (unsigned s = 0; s < 8u; ++s) {
-        const int pair = (int)(short)(w[s] & 0xffffu) + ((int)w[s] >> 16);
-        l[s >> 2] |= ((unsigned)pair & 127u) << (8u * (s & 3u));
-        u[s >> 2] |= ((unsigned)(pair >> 7) & 255u) << (8u * (s & 3u));
-    }
-    lo = make_uint2(l[0], l[1]);
-    hi = make_uint2(u[0], u[1]);
 }
 
 // A workgroup that has its compute unit to itself requests a superblock ahead, on as many registers as that takes; where 64-token
@@ -366,7 +349,7 @@ __global__ __launch_bounds__(64 * WAVES) void dense_q4k16_kernel(DenseQ4kArgs g)
         }
         v4s min_lo, min_hi;
         uint2 bl, bh;
-        bsum_limbs(bsums, bl, bh);
+        q4k_bsum_limbs(bsums, bl, bh);
         v4i b_lo = {0, 0, 0, 0}, b_hi = {0, 0, 0, 0};
         if (q == 0u) {
             b_lo[0] = (int)bl.x; b_lo[1] = (int)bl.y;

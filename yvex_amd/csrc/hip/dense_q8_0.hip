@@ -122,7 +122,8 @@ __device__ __forceinline__ v32f scale_products(float d_a, unsigned scale_bits)
 }
 
 // One superblock out of LDS: lane (r, h)'s weight row at `w_row` (272 bytes), its input row's codes, of which it holds
-// sixteen bytes a block, at `a_row`, and the scales of the input rows that it has sums of, four at a time, at `scales`.
+// sixteen bytes a block, at `a_row`, and that input row's scale, the same for both halves, at `scale_at` (scale_products takes it to
+// the lanes that hold the row's sums).
 __device__ __forceinline__ void q80_superblock(unsigned w_row, unsigned a_row, unsigned scale_at, unsigned h, float scale, double (&acc)[16])
 {
     float total[16];

@@ -1,5 +1,5 @@
 // Q4_K and Q2_K codes times their sub-block scales, and Q8_K block sums, as int8 limbs for the
-// matrix cores (rows_q4k.hip, rows16.hip).
+// matrix cores (dense_q4k.hip, rows_q4k.hip, rows16.hip).
 #pragma once
 #include "common.hpp"
 #include "lds_copy.hpp"
@@ -8,8 +8,10 @@ namespace yvex {
 
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
-// Two int8 limbs of sc * nibble for the four nibbles of one dword, value = 8 hi + lo (see
-// dense_q4k.hip): sc = 8 high + low.
+// Two int8 limbs of sc * nibble for the four nibbles of one dword (already shifted so that the
+// wanted nibble of every byte sits in its low four bits), value = 8 hi + lo. The 6-bit scale is
+// split as sc = 8 high + low with both parts in 0..7: a limb byte nibble * part is at most 105, so
+// one 16-bit lane multiply scales two bytes at once without a carry from one into the next.
 __device__ __forceinline__ void q4k_limbs(unsigned x, unsigned short low, unsigned short high, unsigned &lo, unsigned &hi)
 {
     const unsigned nibbles = x & 0x0f0f0f0fu;
