@@ -148,9 +148,11 @@ def test_q8_0_wide_tiles_are_the_oracles_bits(gpu, oracle, rows, width, inputs):
     assert np.array_equal(got[picked].view(np.uint32), want.view(np.uint32))
 
 
-# a shape of each Q8_0 kernel: the lane chain, 16 x 16, 32 x 32, 256 x 32, 64 x 64, 128 x 64 and 128 x 128 tiles
+# a shape of each Q8_0 kernel: the lane chain, 16 x 16, 32 x 32, 256 x 32, 64 x 64, 128 x 64 and 128 x 128 tiles; 32 x 32 tiles
+# that outnumber the compute units, long rows and not, and two rounds of 64 x 64 ones
 @pytest.mark.parametrize("rows,width,inputs", [(33, 1024, 1), (100, 768, 20), (2047, 512, 95), (65300, 256, 9), (4090, 256, 200),
-                                               (8190, 256, 230), (2047, 512, 2040)])
+                                               (8190, 256, 230), (2047, 512, 2040),
+                                               (2044, 7168, 321), (1022, 4096, 161), (7166, 2048, 130)])
 @pytest.mark.parametrize("scales,magnitude", [("largest", 2.0 ** 95), ("subnormal", 2.0 ** -108)])
 def test_q8_0_block_scales_reach_as_far_as_floats(gpu, oracle, rows, width, inputs, scales, magnitude):
     """Products of a weight and an input block's scale near either end of the float range, the sums of some

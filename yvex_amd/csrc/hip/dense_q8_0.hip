@@ -715,12 +715,14 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
                    (const unsigned char *)act_q8k, input_rows, additive, out, out_stride,
                    output_bf16 ? 1 : 0, status, encoded_second, out_second, {}};
     if (matrices > 1u) publisher = nullptr;       // (workgroups are counted over one matrix)
-    // Which tiles: a pass over the row width costs a workgroup about the same whatever the device's
-    // load (measured at 16 superblocks a row, microseconds: 9 on the 16 x 16 tile and 3.8 more for every such workgroup
-    // that a compute unit has besides, 14 on the 32-row tile and 18.5 once two such
-    // workgroups share a compute unit, 29 on the 64-row staged tile and 43 once two of them share
-    // a compute unit, 35 on the 128-row tile, 54 on the 128 x 128 tile; scale_products has since made all but the first 4 to
-    // 15 % faster), so the choice is the number of rounds each shape needs.
+    // Which tiles: the ones whose launch is the shortest. A pass over the row width takes a workgroup about as long
+    // whatever the device's load, so a launch's time goes by its rounds over the compute units, or by its tiles where
+    // many workgroups share one; either has a part that grows with the row (`long_rows`: 1 at 4096 columns). The numbers are
+    // microseconds, fitted to calls of seventeen matrices of 1024 to 16384 rows of 256 to 14336 columns by 17 to 2048 rows, each on every
+    // kind of tiles: the choice is 0.1 % behind the best one on average and 2.7 % at most, and 6 % at most for eleven other matrices
+    // (1.3 and 24 before, by numbers that did not know the row's length and were older than scale_products). us a call before and
+    // now: 4096 x 4096 by 1400 rows 118.3 and 113.5, 7168 x 7168 by 65 51.8 and 47.0, 2048 x 7168 by 333 52.6 and 48.6, 16384 x 2048 by 320
+    // 70.1 and 62.1, 1024 x 4096 by 160 24.8 and 23.6.
     const uint64_t token_tiles32 = (input_rows + 31u) / 32u;
     const uint64_t token_tiles64 = (input_rows + 63u) / 64u;
     if (token_tiles32 > 65535ull) return ST_BOUNDS;
@@ -737,25 +739,28 @@ int launch_q8_0_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t 
     }
     const uint64_t token_tiles16 = (input_rows + 15u) / 16u, small = matrices * ((row_count + 15u) / 16u) * token_tiles16;
     const uint64_t plain = matrices * row_tiles * token_tiles32;
-    const double plain_cost = !units || plain <= units ? 14.0 : 18.5 * (double)((plain + 2u * units - 1u) / (2u * units));
-    const double small_cost = !units || small <= units ? 9.0 : 4.0 + 3.8 * (double)small / (double)units;
-    // (a batch that offers the staged tiles more than these is not theirs: they take 29 us at least)
-    if (small_cost < plain_cost && small_cost < 29.0 && token_tiles16 <= 65535u && (row_count + 15u) / 16u <= 0x7fffffffull) {
+    const double long_rows = (double)row_width / 4096.0;
+    auto share = [&](uint64_t tiles) { return units && tiles > units ? (double)tiles / (double)units : 1.0; };
+    auto rounds = [&](uint64_t tiles) { return units ? (double)((tiles + units - 1u) / units) : 1.0; };
+    const double plain_cost = 6.9 + 7.4 * long_rows + (2.6 + 3.4 * long_rows) * (share(plain) - 1.0);
+    const double small_cost = share(small) > 1.0 ? 3.8 + 2.9 * long_rows + (1.5 + 1.9 * long_rows) * share(small) : 1.3 + 5.3 * long_rows;
+    const uint64_t tall = matrices * ((row_count + 127u) / 128u) * token_tiles64, low = matrices * ((row_count + 63u) / 64u) * token_tiles64;
+    const uint64_t token_tiles128 = (input_rows + 127u) / 128u, wide = matrices * ((row_count + 127u) / 128u) * token_tiles128;
+    // (two workgroups of the 64-row tiles share a compute unit: the second round costs little)
+    const double low_rounds = rounds(low), low_second = low_rounds > 1.0 ? 2.1 + 5.2 * long_rows : 0.0;
+    const double low_cost = 5.4 + 19.7 * long_rows + low_second + (low_rounds > 2.0 ? (1.5 + 11.3 * long_rows) * (low_rounds - 2.0) : 0.0);
+    const double tall_cost = 5.2 + 30.7 * long_rows + (3.6 + 29.0 * long_rows) * (rounds(tall) - 1.0);
+    const double wide_cost = 5.1 + 44.3 * long_rows + (5.8 + 39.3 * long_rows) * (rounds(wide) - 1.0);
+    const bool staged = aligned16 && units;
+    if (small_cost < plain_cost && (!staged || (small_cost < low_cost && small_cost <= tall_cost)) && token_tiles16 <= 65535u &&
+        (row_count + 15u) / 16u <= 0x7fffffffull) {
         YVEX_ALLOW_DYNAMIC_LDS(dense_q8_0_small_kernel, kSmallLdsBytes);
         g.publication = take_publication(publisher, small);
         dense_q8_0_small_kernel<<<dim3((unsigned)((row_count + 15u) / 16u), (unsigned)token_tiles16, (unsigned)matrices),
                                   64 * kSmallWaves, kSmallLdsBytes, stream>>>(g);
         return check_launch("dense_q8_0_small");
     }
-    if (aligned16 && units) {
-        const uint64_t tall = matrices * ((row_count + 127u) / 128u) * token_tiles64,
-                       low = matrices * ((row_count + 63u) / 64u) * token_tiles64;
-        const double low_share = 43.0 * (double)low / (double)(2u * units);
-        const double low_cost = low <= units ? 29.0 : (low_share > 43.0 ? low_share : 43.0);
-        const double tall_cost = 35.0 * (double)((tall + units - 1u) / units);
-        const uint64_t token_tiles128 = (input_rows + 127u) / 128u;
-        const uint64_t wide = matrices * ((row_count + 127u) / 128u) * token_tiles128;
-        const double wide_cost = 54.0 * (double)((wide + units - 1u) / units);
+    if (staged) {
         // (32-bit offsets into a tile's rows)
         if (wide_cost < plain_cost && wide_cost <= low_cost && wide_cost <= tall_cost &&
             row_bytes <= (1ull << 24) && row_width / 256u * kQ8KBytes <= (1ull << 24)) {
