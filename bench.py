@@ -415,10 +415,11 @@ def prefill_leg(torch, K, MoeLayer, weights, shared, dev, steps: int, warmup: in
     abi_same = bool((torch.from_numpy(abi_layer.output()) == stage_rows.cpu()).all().item())
     abi_unique = int(abi_layer.result.unique_experts)
     abi_eager_ms = abi_layer.timed(steps, warmup, eager=True)
-    abi_graph_ms = abi_layer.timed(steps, max(warmup, 2))
+    abi_ms = abi_layer.timed(steps, max(warmup, 2))
+    abi_graph = bool(abi_layer.result.graph_launches)
     abi_layer.close()
     harness_ms = step_ms
-    step_ms = min(abi_graph_ms, abi_eager_ms)
+    step_ms = call_ms(abi_ms, abi_eager_ms, abi_graph)
     residency = "canonical bytes"
     # IQ2_XXS experts resident as the sweep image only: the matrix-core kernels read it as well
     image = None
@@ -430,7 +431,7 @@ def prefill_leg(torch, K, MoeLayer, weights, shared, dev, steps: int, warmup: in
         image_layer.close()
         del image_layer
         torch.cuda.empty_cache()
-        image = {"graph_ms_per_step": round(image_ms, 4), "rows_identical_to_canonical": image_same}
+        image = {"ms_per_step": round(image_ms, 4), "rows_identical_to_canonical": image_same}
         if not image_same:
             return {"error": "the sweep image and the canonical rows disagree on the matrix-core kernels"}
         # as for the decode step, the faster residency is the leg's figure (same rows bit for bit;
@@ -448,8 +449,8 @@ def prefill_leg(torch, K, MoeLayer, weights, shared, dev, steps: int, warmup: in
         "ms_per_step": round(step_ms, 4), "tokens_per_s": round(rows / (step_ms * 1e-3), 1),
         "residency": residency,
         "c_abi": {"entry": "yvex_rocm_backend_moe_operations_get()->execute_rows + complete_rows",
-                  "graph_ms_per_step": round(abi_graph_ms, 4), "eager_ms_per_step": round(abi_eager_ms, 4),
-                  "rows_identical_to_stage_harness": abi_same,
+                  "default_ms_per_step": round(abi_ms, 4), "eager_ms_per_step": round(abi_eager_ms, 4),
+                  "launch_graph": abi_graph, "rows_identical_to_stage_harness": abi_same,
                   "distinct_routed_experts": abi_unique},
         "c_abi_sweep_image": image,
         "stage_harness_ms_per_step": round(harness_ms, 4),
@@ -468,6 +469,12 @@ def prefill_leg(torch, K, MoeLayer, weights, shared, dev, steps: int, warmup: in
     }
 
 
+def call_ms(default_ms, eager_ms, took_graph):
+    """A step through the C ABI: the call as a caller makes it, or with eager_execution set where that is faster than the launch
+    graph it replays. A layer that takes no graph makes the same launches either way, and the call as it is counts."""
+    return min(default_ms, eager_ms) if took_graph else default_ms
+
+
 def decode_q4k_leg(torch, K, weights, shared, dev, steps: int, warmup: int):
     """The headline batch (32 rows, top-8 of 256 + shared) with Q4_K experts, through the C ABI:
     the decode-width sweeps read Q4_K rows too. Bytes counted: the canonical bytes of the distinct
@@ -480,14 +487,15 @@ def decode_q4k_leg(torch, K, weights, shared, dev, steps: int, warmup: int):
     layer.step(defer=False)
     unique = int(layer.result.unique_experts)
     eager_ms = layer.timed(steps, warmup, eager=True)
-    graph_ms = layer.timed(steps, max(warmup, 2))
+    default_ms = layer.timed(steps, max(warmup, 2))
+    graph = bool(layer.result.graph_launches)
     layer.close()
-    step_ms = min(graph_ms, eager_ms)
+    step_ms = call_ms(default_ms, eager_ms, graph)
     expert_bytes = 3 * INTERMEDIATE * HIDDEN // 256 * 144
     read = (unique + 1) * expert_bytes
     return {"workload": "moe_decode_q4k: 32 rows, top-8 of 256 Q4_K experts + shared, Q8_K activations",
-            "ms_per_step": round(step_ms, 4), "graph_ms_per_step": round(graph_ms, 4),
-            "eager_ms_per_step": round(eager_ms, 4), "distinct_routed_experts": unique,
+            "ms_per_step": round(step_ms, 4), "default_ms_per_step": round(default_ms, 4),
+            "eager_ms_per_step": round(eager_ms, 4), "launch_graph": graph, "distinct_routed_experts": unique,
             "GB_per_s": round(read / (step_ms * 1e-3) / 1e9, 1),
             "hbm_peak_frac": round(read / (step_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}
 
@@ -537,7 +545,9 @@ def model_file_layer_leg(torch, gate, up, dev, steps: int, warmup: int):
         layer.step(defer=False)
         unique = int(layer.result.unique_experts)
         matrix = int(layer.result.tensor_core_launches)
-        ms = min(layer.timed(count, max(warmup, 2)), layer.timed(count, warmup, eager=True))
+        eager_ms = layer.timed(count, warmup, eager=True)
+        ms = layer.timed(count, max(warmup, 2))
+        ms = call_ms(ms, eager_ms, bool(layer.result.graph_launches))
         layer.close()
         read = unique * blocks * (2 * 66 + 84) + 3 * blocks * 8 * 34
         leg = {"ms_per_step": round(ms, 4), "distinct_routed_experts": unique, "matrix_core_launches": matrix,
@@ -571,12 +581,13 @@ def envelope_leg(torch, routed, shared, router, dev, steps: int, warmup: int):
     layer.step(defer=False)
     launches = int(layer.result.kernel_launches)
     eager_ms = layer.timed(steps, warmup, eager=True)
-    graph_ms = layer.timed(steps, max(warmup, 2))
+    default_ms = layer.timed(steps, max(warmup, 2))
+    graph = bool(layer.result.graph_launches)
     layer.close()
     return {"workload": "the decode step with 4 residual streams of 7168 around the layer (24 mixing rows, "
                         "20 Sinkhorn iterations), sweep image",
-            "ms_per_step": round(min(graph_ms, eager_ms), 4), "graph_ms_per_step": round(graph_ms, 4),
-            "eager_ms_per_step": round(eager_ms, 4), "kernel_launches": launches}
+            "ms_per_step": round(call_ms(default_ms, eager_ms, graph), 4), "default_ms_per_step": round(default_ms, 4),
+            "eager_ms_per_step": round(eager_ms, 4), "launch_graph": graph, "kernel_launches": launches}
 
 
 def small_batches_leg(torch, routed, shared, router, dev, steps: int, warmup: int):
@@ -593,7 +604,9 @@ def small_batches_leg(torch, routed, shared, router, dev, steps: int, warmup: in
         layer.step(defer=False)
         unique = int(layer.result.unique_experts)
         layer.timed(steps, warmup)
-        ms = min(layer.timed(steps, max(warmup, 2)), layer.timed(steps, warmup, eager=True))
+        eager_ms = layer.timed(steps, warmup, eager=True)
+        ms = layer.timed(steps, max(warmup, 2))
+        ms = call_ms(ms, eager_ms, bool(layer.result.graph_launches))
         layer.close()
         out[f"rows_{rows}"] = {"us_per_step": round(ms * 1e3, 1), "distinct_routed_experts": unique,
                                "GB_per_s": round((unique + 1) * EXPERT_BYTES / (ms * 1e-3) / 1e9, 1)}
@@ -732,7 +745,7 @@ def main() -> int:
     abi_unique = int(abi_layer.result.unique_experts)
     abi_same = bool((torch.from_numpy(abi_layer.output()) == stage_rows.cpu()).all().item())
     abi_eager_ms = abi_layer.timed(args.steps, args.warmup, eager=True)
-    abi_graph_ms = abi_layer.timed(args.steps, max(args.warmup, 2))
+    abi_ms = abi_layer.timed(args.steps, max(args.warmup, 2))
     graph_facts = (int(abi_layer.result.graph_launches), int(abi_layer.result.graph_replays))
     abi_sync_ms = abi_layer.timed(args.steps, args.warmup, defer=False)
     abi_launches = int(abi_layer.result.kernel_launches)
@@ -741,9 +754,9 @@ def main() -> int:
         print(f"decode step: execute_rows and the stage harness disagree (distinct experts {abi_unique} "
               f"vs {unique}, identical rows {abi_same})", file=sys.stderr)
         return 1
-    step_ms = min(abi_graph_ms, abi_eager_ms)
-    graph_mode = "library launch graph" if graph_facts[0] else "eager launches"
-    launch_mode = (f"execute_rows, {graph_mode if abi_graph_ms <= abi_eager_ms else 'eager launches'}, "
+    took_graph = bool(graph_facts[0])
+    step_ms = call_ms(abi_ms, abi_eager_ms, took_graph)
+    launch_mode = (f"execute_rows, {'library launch graph' if took_graph and step_ms == abi_ms else 'eager launches'}, "
                    "completion deferred to the phase barrier")
     # The same step with the experts resident as the decode sweeps' image: a caller's residency
     # step plans it (derived_layout_plan, 72 bytes a superblock instead of 66) and builds it on the
@@ -756,7 +769,7 @@ def main() -> int:
         image_layer.step(defer=False)
         image_same = bool((torch.from_numpy(image_layer.output()) == stage_rows.cpu()).all().item())
         image_eager_ms = image_layer.timed(args.steps, args.warmup, eager=True)
-        image_graph_ms = image_layer.timed(args.steps, max(args.warmup, 2))
+        image_default_ms = image_layer.timed(args.steps, max(args.warmup, 2))
         image_bytes = sum(t.numel() for t in image_layer.images)
         image_layer.close()
         del image_layer
@@ -775,15 +788,16 @@ def main() -> int:
         torch.cuda.empty_cache()
         image = {"entry": "the same execute_rows over DERIVED_BACKEND views built by "
                           "yvex_rocm_moe_derived_layout_plan + yvex_rocm_moe_sweep_image_build_resident",
-                 "graph_ms_per_step": round(image_graph_ms, 4), "eager_ms_per_step": round(image_eager_ms, 4),
+                 "default_ms_per_step": round(image_default_ms, 4), "eager_ms_per_step": round(image_eager_ms, 4),
                  "image_bytes": image_bytes, "canonical_bytes": (EXPERTS + 1) * EXPERT_BYTES,
                  "rows_identical_to_canonical": image_same,
                  "gate_up_sweep_ms": round(image_sweeps_ms["up"][0], 4),
                  "down_sweep_ms": round(image_sweeps_ms["down"][0], 4)}
-        if min(image_graph_ms, image_eager_ms) < step_ms:
-            step_ms = min(image_graph_ms, image_eager_ms)
+        image_ms = call_ms(image_default_ms, image_eager_ms, took_graph)
+        if image_ms < step_ms:
+            step_ms = image_ms
             launch_mode = ("execute_rows over the sweep image, " +
-                           (graph_mode if image_graph_ms <= image_eager_ms else "eager launches") +
+                           ("library launch graph" if took_graph and image_ms == image_default_ms else "eager launches") +
                            ", completion deferred to the phase barrier")
             sweeps_ms = image_sweeps_ms
     weight_bytes = (unique + 1) * EXPERT_BYTES
@@ -843,7 +857,7 @@ def main() -> int:
         "tokens_per_s": round(ROWS / (step_ms * 1e-3), 1),
         "launch": launch_mode,
         "c_abi": {"entry": "yvex_rocm_backend_moe_operations_get()->execute_rows + complete_rows",
-                  "graph_ms_per_step": round(abi_graph_ms, 4), "eager_ms_per_step": round(abi_eager_ms, 4),
+                  "default_ms_per_step": round(abi_ms, 4), "eager_ms_per_step": round(abi_eager_ms, 4),
                   "completed_every_step_ms": round(abi_sync_ms, 4), "kernel_launches": abi_launches,
                   "graph_launches_replays_last_step": graph_facts,
                   "rows_identical_to_stage_harness": abi_same},
