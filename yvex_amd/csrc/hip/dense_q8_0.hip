@@ -607,11 +607,11 @@ constexpr unsigned kWideLdsBytes = kWideScaleBase + 2u * kWideTokens * 4u;
 //    other's waits and the rate of one wave's instructions (one in 5.5 cycles on this part; two waves issue 4-cycle
 //    instructions in 5.0 cycles each, four in 4.4).
 //  * Copies take a scalar base and a 32-bit offset a lane: a register and no addition each.
-// 4096 x 4096 by 2048 rows 136 -> 129 us (532 TOP/s; eight waves of 32 x 64, two a SIMD, before). No pipe is full: the
-// vector ALU is issued to 66 % of the time, the LDS is busy 40 %, nearly half of it bank conflicts (at a pitch of 272 bytes
-// rows r and r + 16 start on one bank, which the reads of less than 16 bytes meet on), the matrix cores 12 %; a wave waits for
-// data 42 % of its time, copies behind a full wait and a barrier a superblock. (Counters from before
-// scale_products.) Whole 16-byte reads of a window's end: 131 us.
+// 4096 x 4096 by 2048 rows 136 -> 129 us (532 TOP/s; eight waves of 32 x 64, two a SIMD, before). With
+// scale_products 119 us. No pipe is full: the vector ALU is issued to 51 % of the time, the LDS is busy 32 %, nearly half of it bank
+// conflicts (at a pitch of 272 bytes rows r and r + 16 start on one bank, which the reads of less than 16 bytes meet on), the matrix
+// cores 25 %; a wave waits for data 42 % of its time, copies behind a full wait and a barrier a superblock, and for its turn to
+// issue 34 %. Whole 16-byte reads of a window's end, before scale_products: 131 us.
 __global__ __launch_bounds__(kWideThreads) void dense_q8_0_wide_kernel(DenseQ80Args g)
 {
     extern __shared__ __align__(16) unsigned char dense_q8_0_lds[];

@@ -163,7 +163,10 @@ int launch_iq2_sweep(const GroupedArgs &a, unsigned qtype, bool fused, bool imag
 // few it holds (54 us of gate/up and 28 us of Q2_K down rows at width 4096 for one bucket or sixteen), a bucket in two
 // tiles 2.6 and 1.5 us of the whole device. Two tiles in every bucket of 256 are the slower way: 665 us
 // against 600 (width 4096, 24 pairs), 1148 against 935 (7168, fourteen); and beside a launch that is long anyway
-// they gain nothing (1111 uneven rows of Q4_K 2570 us without, 2650 with). Every thread of a block calls this, a thread a
+// they gain nothing (1111 uneven rows of Q4_K 2570 us without, 2650 with). Taken again with products of the scales on the matrix
+// cores in the 64-pair kernels: 420 even rows of 7168 by eight of 256 Q4_K experts 1657 us so, 1815 with two tiles in up to 64
+// buckets or all; of 4096 by six in the model file's formats 666 so, 694 with a bucket never in two; uneven ones within 1 % (2.5 % at 1600
+// rows of Q4_K, two tiles in every bucket). Every thread of a block calls this, a thread a
 // bucket, those without one with 0; `lds` is the address of four words of LDS that hold nothing (the kernels leave no
 // room for static LDS).
 constexpr unsigned kFewPairSeconds = 16u;

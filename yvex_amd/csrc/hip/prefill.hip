@@ -820,7 +820,9 @@ static int launch_mfma(const MfmaArgs &a, hipStream_t stream)
 // bucket holds behind its whole 64-pair tiles if that fits one of their tiles (12 pairs at width 7168, 16 up to about 5000; two tiles
 // where few_pair_limit says so): such a tile takes them 1.3 us of the whole device for the 2 x 2048 x 4096 IQ2_XXS
 // rows of an expert, and the 64-pair kernels, which pay for 32 token columns, 2.3 us; with two of theirs (2.6 us) it
-// is the other way round. A matrix that is alone (no worklist) is theirs where they come out at one round of
+// is the other way round. (Q4_K, and Q2_K down rows, without the few-pair kernels and with the present 64-pair ones: 150 / 420 even rows of
+// 7168 by eight of 256 Q4_K experts 1442 / 1668 -> 1758 / 1899 us a layer, of 4096 by six in the model file's formats 577 / 660 -> 681 / 759; 2048 uneven rows 3460 -> 3519
+// and 1523 -> 1534. Uneven rows of 4096 by six of Q4_K would gain: 1111 rows 1097 -> 1058.) A matrix that is alone (no worklist) is theirs where they come out at one round of
 // their waves: 16 superblocks take 22 to 31 us then, and 45 us as 64-pair items, which are fewer than the
 // compute units up to 1024 rows (4096 x 4096 IQ2_XXS by 128 rows 44 -> 24 us, 2048 x 7168 69 -> 35; 7168 x
 // 7168 by 256 rows, two rounds, 102 us against 70).
