@@ -52,8 +52,9 @@ def test_scales_and_minimums_reach_as_far_as_floats(gpu, oracle, qtype, scales, 
 
 
 # the same for a plain projection: 16 x 16, 32 x 32 and 32 x 64 tiles, those that share a compute unit, tiles staged through
-# LDS; ragged edges on both sides
-@pytest.mark.parametrize("rows,width,inputs", [(50, 512, 20), (2060, 768, 71), (2078, 512, 100), (8200, 256, 41), (8180, 256, 230)])
+# LDS; ragged edges on both sides; more 32 x 64 tiles of long rows than compute units
+@pytest.mark.parametrize("rows,width,inputs", [(50, 512, 20), (2060, 768, 71), (2078, 512, 100), (8200, 256, 41), (8180, 256, 230),
+                                               (2060, 6144, 530), (4100, 11520, 140)])
 @pytest.mark.parametrize("scales,magnitude", [("ordinary", 1.0), ("largest", 2.0 ** 80), ("subnormal", 2.0 ** -108)])
 def test_q4k_projections_reach_as_far_as_floats(gpu, oracle, rows, width, inputs, scales, magnitude):
     """Against the kernel of a few input rows, which scales on the vector ALU, for every row of the batch, and the CPU path's

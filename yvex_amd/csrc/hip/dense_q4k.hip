@@ -108,7 +108,7 @@ __device__ __forceinline__ v4i as_v4i(uint4 v)
 
 // A workgroup that has its compute unit to itself requests a superblock ahead, on as many registers as that takes; where 64-token
 // tiles outnumber the compute units (PAIRED) two of them share one on half the registers and cover each other's loads. us a
-// call one way and the other: 7168 x 2048 by 120 rows 36.3 and 29.0, 4096 x 4096 by 150 42.4 and 36.1, 2048 x 7168 by 300 57.9 and
+// call one way and the other (tiles_share_units has the line): 7168 x 2048 by 120 rows 36.3 and 29.0, 4096 x 4096 by 150 42.4 and 36.1, 2048 x 7168 by 300 57.9 and
 // 55.3; with a tile a compute unit or fewer 2048 x 7168 by 200 37.0 and 45.2, 4096 x 4096 by 96 30.0 and 32.4, 1024 x 4096 by 300 30.4 and 33.4.
 template <unsigned NT, bool PAIRED = false>
 __global__ __launch_bounds__(256, NT == 1u || PAIRED ? 2 : 1) void dense_q4k_kernel(DenseQ4kArgs g)
@@ -400,6 +400,19 @@ __global__ __launch_bounds__(64 * WAVES) void dense_q4k16_kernel(DenseQ4kArgs g)
 
 }  // namespace
 
+// Whether two workgroups of 32 x 64 tiles share a compute unit, where the tiles outnumber them. The longer the row, the nearer a
+// pair's time comes to that of two tiles one behind the other, so a third round of tiles, which is half a pair's, is
+// dearer in pairs from some 6000 columns on, and any from 11 500 (multiples of 8192 apart, which gain in pairs as short rows do). us a call,
+// in pairs and not, 384 / 640 / 896 tiles: 4096 columns 38.6 / 57.8 / 65.9 and 45.3 / 61.5 / 77.6; 5888 48.4 / 76.8 / 88.1 and 54.3 / 77.1 / 97.5; 7424 57.1 / 92.5 / 107.1
+// and 61.3 / 87.4 / 111.0; 11 264 76.1 / 125.2 / 142.3 and 76.4 / 110.1 / 141.8; 12 288 81.4 / 132.9 / 152.5 and 80.9 / 114.1 / 146.7; 8192 (576, 832 tiles) 104.5 / 128.4 and
+// 108.8 / 143.4.
+static bool tiles_share_units(uint64_t tiles, uint64_t units, uint64_t row_width)
+{
+    if (tiles <= units) return false;
+    if (row_width < 6144u || row_width % 8192u == 0u) return true;
+    return row_width < 11520u && (tiles <= 2u * units || tiles > 3u * units);
+}
+
 int launch_q4k_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t row_width,
                           uint64_t row_bytes, const void *act_q8k, uint64_t input_rows,
                           const float *additive, float *out, uint64_t out_stride, bool output_bf16,
@@ -439,7 +452,7 @@ int launch_q4k_rows_dense(const uint8_t *encoded, uint64_t row_count, uint64_t r
         // faster ones (2048 x 7168 at 96 rows: 17 us on 32 x 32 tiles, 21 on 16 x 32; at 256 rows 27 us on 32 x 64).
         if (row_tiles * token_tiles32 <= units)
             dense_q4k_kernel<1><<<dim3((unsigned)row_tiles, (unsigned)token_tiles32), 256, 0, stream>>>(g);
-        else if (row_tiles * token_tiles > units)
+        else if (tiles_share_units(row_tiles * token_tiles, units, row_width))
             dense_q4k_kernel<2, true><<<dim3((unsigned)row_tiles, (unsigned)token_tiles), 256, 0, stream>>>(g);
         else
             dense_q4k_kernel<2><<<dim3((unsigned)row_tiles, (unsigned)token_tiles), 256, 0, stream>>>(g);
