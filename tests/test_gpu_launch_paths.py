@@ -101,8 +101,7 @@ def test_projections_that_publish_for_themselves(gpu, oracle, qtype, weight_rows
 
 
 # the most work that a launch ends by itself, and a little more: rows a wave of the product that quantizes, a
-# compute unit for each IQ2_XXS tile and for five Q4_K ones, the
-# longest rows that a wave has two of
+# compute unit for each IQ2_XXS tile and for five Q4_K ones, the longest rows that a wave has two of
 @pytest.mark.parametrize("qtype,weight_rows,width,inputs,launches", [
     ("Q8_0", 32768, 256, 1, 1), ("Q8_0", 32769, 256, 1, 2), ("Q8_0", 32768, 512, 2, 1), ("Q8_0", 36001, 512, 2, 2),
     ("IQ2_XXS", 4096, 512, 16, 2), ("IQ2_XXS", 2048, 512, 17, 2), ("IQ2_XXS", 4100, 512, 7, 3), ("IQ2_XXS", 1376, 1024, 33, 3),
@@ -493,15 +492,17 @@ def test_row_batches_either_side_of_the_matrix_core_line(gpu, oracle, qtype, sha
 
 
 # the layer as a decoder runs it, deferred and without host copies, whose combine goes straight into the egress; the
-# caller alternates with batches that ask for host copies, each kind eager, captured and replayed
-@pytest.mark.parametrize("down,shared,rows", [(None, None, 1), ("Q2_K", "Q8_0", 5), ("Q2_K", "Q8_0", 75)])
-def test_deferred_layers_with_streams_are_the_oracles(gpu, oracle, down, shared, rows):
+# caller alternates with batches that ask for host copies, each kind eager, captured and replayed; the last is the widest row
+# of a layer, by as many rows as the ingress needs to join its projection
+@pytest.mark.parametrize("down,shared,rows,width", [(None, None, 1, 512), ("Q2_K", "Q8_0", 5, 512), ("Q2_K", "Q8_0", 75, 512),
+                                                    (None, None, 8, 8192)])
+def test_deferred_layers_with_streams_are_the_oracles(gpu, oracle, down, shared, rows, width):
     from backend_helpers import Backend
     from test_gpu_backend import MoeCase, same_as_cpu
     from yvex_amd import abi
     b = Backend()
     try:
-        case = MoeCase(b, oracle, hidden=512, intermediate=512, rows=rows, streams=4, down_qtype=down, shared_qtype=shared)
+        case = MoeCase(b, oracle, hidden=width, intermediate=512, rows=rows, streams=4, down_qtype=down, shared_qtype=shared)
         b.workspace(case.workspace_bytes)
         want, host, done = case.oracle_layer(act_q8=True), case.out, abi.RowBatchResult()
         empty, zeros = abi.RowBatchOutput(), np.zeros_like(case.x)
@@ -523,7 +524,7 @@ def test_deferred_layers_with_streams_are_the_oracles(gpu, oracle, down, shared,
                     assert np.max(np.abs(case.comb - want["combination"])) <= 1e-6
                     same_as_cpu(case.combined, want["combined"])
                     # the egress of the CPU's combined rows with the device's own gates is exact
-                    rc, egress = oracle.mhc_post(want["combined"], case.x, case.post, case.comb, streams=4, width=512)
+                    rc, egress = oracle.mhc_post(want["combined"], case.x, case.post, case.comb, streams=4, width=width)
                     assert rc == 0
                 else:
                     assert not case.combined.any()
