@@ -923,3 +923,22 @@ def test_envelope_flags_non_finite(gpu, oracle):
     with pytest.raises(K.KernelError):     # eight streams would need 80 mixing rows
         K.mhc_egress(dev(core, gpu), dev(rows, gpu), dev(np.ones((3, 8), np.float32), gpu),
                      dev(np.ones((3, 8, 8), np.float32), gpu), streams=8, width=32, status=status)
+
+
+def test_bfloat16_rounding_of_every_upper_half(gpu):
+    """Every upper half of a float with lower halves at and beside the tie (numbers, subnormals, infinities, NaNs) comes
+    out as the reference's integer rounding (kernel_primitives.h:89-99) has it."""
+    import ctypes
+    from yvex_amd import kernels as K
+    lower = np.array([0x0000, 0x0001, 0x7fff, 0x8000, 0x8001, 0xffff], dtype=np.uint32)
+    bits = ((np.arange(65536, dtype=np.uint32)[:, None] << 16) | lower[None, :]).reshape(-1)
+    upper, low = bits >> 16, bits & 0xffff
+    nan = ((bits & 0x7f800000) == 0x7f800000) & ((bits & 0x7fffff) != 0)
+    up = (low > 0x8000) | ((low == 0x8000) & ((upper & 1) == 1))
+    want = np.where(nan, upper | 0x40, upper + up).astype(np.uint32) << 16
+    values, half = dev(bits.view(np.int32), gpu), bits.size // 2
+    out, status = torch.empty_like(values), K.new_status(gpu)
+    K._call("yvex_hip_concat_rows_bf16", K._ptr(values[:half]), K._ptr(values[half:]), ctypes.c_uint64(1),
+            ctypes.c_uint64(half), ctypes.c_uint64(half), K._ptr(out), K._ptr(status), K._stream())
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), want)
+    assert int(status.item()) == 1          # (infinities and NaNs are among them)

@@ -59,7 +59,7 @@ __device__ __forceinline__ float swiglu_bf16_fast(float g, float u, float route_
     const bool finite = finite_f32(v), large = fabsf(v) > 1.0e-30f, inside = fabsf(gv) <= 16.0f;
     const bool clear = (low < 0x8000u - 64u) | (low > 0x8000u + 64u);
     const bool safe = ((double)limit_f32 == limit) & finite & large & inside & clear;
-    if (safe) return bf16_round_number(v);
+    if (safe) return bf16_round(v);
     return swiglu_bf16(g, u, route_weight, limit);
 }
 

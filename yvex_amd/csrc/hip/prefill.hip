@@ -590,7 +590,7 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
                 for (unsigned j = 0; j < 4u; ++j) {
                     value[j] = (float)acc[tb][4u * q + j];
                     good &= finite_f32(value[j]);
-                    if (!a.plain_output) value[j] = bf16_round_number(value[j]);   // (a NaN has just been noted)
+                    if (!a.plain_output) value[j] = bf16_round(value[j]);   // (a NaN has just been noted)
                 }
             }
 #pragma unroll

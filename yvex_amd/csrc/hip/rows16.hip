@@ -759,7 +759,7 @@ __global__ __launch_bounds__((Map16<QT, S>::kThreads)) void rows16_kernel(Rows16
                     } else {
                         value[i] = (float)acc[u][i];
                         good &= finite_f32(value[i]);
-                        if (a.round) value[i] = bf16_round_number(value[i]);      // (a NaN has just been noted)
+                        if (a.round) value[i] = bf16_round(value[i]);      // (a NaN has just been noted)
                     }
                     good &= finite_f32(value[i]);
                 }

@@ -364,7 +364,7 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
                 for (unsigned k = 0; k < 4u; ++k) {
                     value[k] = add ? (float)acc[nt][4u * q4 + k] + extra[k] : (float)acc[nt][4u * q4 + k];
                     fine[k] = finite_f32(value[k]);          // (the rounding below is for numbers)
-                    if (round) value[k] = bf16_round_number(value[k]);
+                    if (round) value[k] = bf16_round(value[k]);
                 }
             }
 #pragma unroll
