@@ -3,10 +3,18 @@
 // A work item is (bucket, tile of up to 64 ordered pairs, tile of 256 weight rows: 128 gate rows
 // and the 128 matching up rows when the SwiGLU is fused). The workgroup has eight waves, two per
 // SIMD; each owns 32 weight rows and multiplies them by all of the item's Q8_K activation rows
-// with V_MFMA_I32_32X32X32_I8. A wave cannot run vector instructions under its own matrix
-// instruction, the other wave of its SIMD can, so two waves a SIMD is the shape that lets decode
-// and scaling arithmetic overlap the matrix pipe, and 256 registers a wave is what decides the
-// tile: 32 rows x 64 tokens of int32 limb sums and double-precision row sums.
+// with V_MFMA_I32_32X32X32_I8. 256 registers a wave are what decides the tile: 32 rows x 64 tokens of int32
+// limb sums and double-precision row sums.
+//
+// What bounds it is not the matrix pipe: vector instructions run under matrix instructions, a wave's own among them (one
+// 32 x 32 x 32 instruction and k byte permutes take max(32, 8 + 4.5 k) cycles with two waves a SIMD), and without its
+// matrix instructions a launch takes as many cycles. It is the issue of everything else, about five cycles a vector or LDS
+// instruction and forty a window copy, and the matrix instructions' power: 1.9 to 2.0 GHz under this kernel, 2.2 without
+// them. The wave's number is kept scalar, and with it every LDS address of a copy and every distance it adds to its
+// lanes' pointers (333 -> 315 vector instructions a superblock: 7168 x 2 x 4096 by 2048 rows 317 -> 301 us, 2048 x 8192 by 2048 122.2 -> 119.4).
+// Two things that look the same and are slower: stages with sixteen bytes between groups of tokens, which make the fragments' places
+// immediate offsets (a copy into LDS that does not start on 64 bytes is split: 582K cycles against 570K), and windows without their
+// spare pieces (64 scattered dwords cost a copy more than 64 pieces of sixteen bytes: 600K against 590K).
 //
 //   A operand (weights): built in registers, one K chunk (32 columns) ahead of its use. Lane
 //       (r, h) = (lane % 32, lane / 32) owns weight row r and the groups 4h .. 4h + 3 of the
@@ -111,6 +119,11 @@ __device__ __forceinline__ void mfma_tables_fill()
         lds_write_uint4(kLutBase + index * 16u, iq2_limb_words(index >> 4));
 }
 
+__device__ __forceinline__ unsigned uniform32(unsigned v)
+{
+    return (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+}
+
 // What one work item needs to know about its place in the problem.
 struct MfmaItem {
     unsigned long long expert, pair0;
@@ -176,7 +189,7 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
     constexpr unsigned T = NTB * 32u;                // token slots of one stage
     constexpr unsigned kStageBytes = T * kActPitch + 256u;
     constexpr unsigned kBarrierSlot = 5u;
-    const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const unsigned tid = threadIdx.x, lane = tid & 63u, wave = uniform32(tid >> 6);
     const unsigned r = lane & 31u, h = lane >> 5;
     constexpr unsigned kItemRows = FUSED_UP ? 128u : 256u;
     const unsigned superblocks = a.width >> 8;
@@ -227,11 +240,13 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
     long long ahead_shift = 0;
     bool ahead = false;
     auto weight_piece = [&](unsigned sb, unsigned k) {
-        const unsigned to = (unsigned)__builtin_amdgcn_readfirstlane(
-            (int)(window_base + (sb & 1u) * kWindowBytes + k * 1024u));
+        const unsigned to = window_base + (sb & 1u) * kWindowBytes + k * 1024u;
         const bool past = sb > last;
         const unsigned record = !past ? sb : ahead ? (sb - superblocks) & 1u : last;
-        const long long offset = (past ? ahead_shift : 0ll) + (long long)(record * (IMAGE ? 72u : 66u));
+        long long offset = (past ? ahead_shift : 0ll) + (long long)(record * (IMAGE ? 72u : 66u));
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+s"(offset));       // (one sum on the scalar unit, one addition a lane)
+#endif
         const unsigned char *from = IMAGE
             ? window_from[k] + offset
             : (const unsigned char *)((unsigned long long)(window_from[k] + offset) & ~3ull);
@@ -245,7 +260,7 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
         const unsigned live = token < it.tokens ? token : it.tokens - 1u;   // padding repeats a row
         const unsigned long long ordered = it.pair0 + live;
         const unsigned long long source = pr.order ? pr.order[ordered] : ordered;
-        const unsigned long long arow = pr.act_by_ordered_pair ? ordered : source / pr.topk;
+        const unsigned long long arow = pr.act_by_ordered_pair ? ordered : (unsigned)source / pr.topk;      // (pairs fit 32 bits)
         return (const unsigned char *)pr.activations + arow * pr.act_stride;
     };
     const unsigned char *copy_from[NTB];
@@ -278,14 +293,14 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
     constexpr unsigned kActPieces = NTB + 1u;
     auto act_piece = [&](unsigned sb, unsigned j) {
         const unsigned base = kStageBase + (sb % R) * kStageBytes;
-        sb = sb < last ? sb : last;
+        unsigned offset = (sb < last ? sb : last) * kQ8KBytes;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+s"(offset));
+#endif
         if (j < NTB) {
-            copy_to_lds_16(copy_from[j] + (unsigned long long)sb * kQ8KBytes,
-                           (unsigned)__builtin_amdgcn_readfirstlane((int)(base + (wave + kRowWaves * j) * 1024u)));
+            copy_to_lds_16(copy_from[j] + offset, base + (wave + kRowWaves * j) * 1024u);
         } else {
-            copy_to_lds_4(scale_from + (unsigned long long)sb * kQ8KBytes,
-                          (unsigned)__builtin_amdgcn_readfirstlane(
-                              (int)(wave == 0u ? base + T * kActPitch : kTrashBase)));
+            copy_to_lds_4(scale_from + offset, wave == 0u ? base + T * kActPitch : kTrashBase);
         }
     };
     // the copies issued after the barrier of superblock sb: the stage and the window just released
@@ -755,7 +770,6 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
     };
     // ---- ... and looked at later. Every lane holds the same values: the item is kept in scalar
     // registers. ----
-    auto uniform32 = [](unsigned v) { return (unsigned)__builtin_amdgcn_readfirstlane((int)v); };
     auto uniform64 = [&](unsigned long long v) {
         return (unsigned long long)uniform32((unsigned)v) | ((unsigned long long)uniform32((unsigned)(v >> 32)) << 32);
     };
