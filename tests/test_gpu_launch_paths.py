@@ -454,6 +454,56 @@ def test_few_pair_kernels_take_second_tiles(gpu, oracle, hidden, intermediate, t
     assert same_bits(out[0], out[1]) and int(status.item()) == 0
 
 
+# more row tiles than workgroups, so that pieces begin and end inside token tiles and pass from tiles of 64 pairs to ones of 33 to
+# 63 and of fewer than 33; rows of an odd number of superblocks, of two and of many
+@pytest.mark.parametrize("hidden,intermediate", [(8192, 512), (1280, 4096)])
+@pytest.mark.parametrize("image", [True, False])
+def test_runs_of_row_tiles_agree_with_the_sweeps(gpu, oracle, hidden, intermediate, image):
+    """A workgroup of the 64-pair kernel goes from row tile to row tile and from token tile to token tile: each pair's rows
+    come out once, the sweeps' bits."""
+    from yvex_amd import kernels as K
+    qt, populations = oracle.IQ2_XXS, [420, 33, 260, 130, 20, 100, 64, 29]
+    experts, pairs = len(populations), sum(populations)
+    g = oracle.Generator(45, f"runs.{hidden}")
+    tensors = [dev(g.weights(qt, experts * r, w), gpu) for r, w in
+               ((intermediate, hidden), (intermediate, hidden), (hidden, intermediate))]
+    weights = K.expert_weights(*tensors, (qt, qt, qt), hidden, intermediate)
+    rows_form = K.expert_weights_image(weights, hidden, intermediate) if image else weights
+    status = K.new_status(gpu)
+    selected = torch.repeat_interleave(torch.arange(experts), torch.tensor(populations))
+    selected = selected[torch.randperm(pairs, generator=torch.Generator().manual_seed(5))].reshape(pairs, 1).to(gpu)
+    wl = K.worklist_build(selected, experts, status)
+    route = dev((0.5 + np.abs(g.normal(pairs))).astype(np.float32), gpu)
+    act = K.q8k_quantize(dev(g.normal(pairs * hidden).reshape(pairs, hidden), gpu), status)
+    mid = [torch.full((pairs, intermediate), float("nan"), device=gpu) for _ in range(2)]
+    K.moe_up(weights, act, True, route, wl, pairs, 1, experts, 10.0, mid[0], status)
+    K.moe_up_rows(rows_form, act, route, wl, pairs, 1, experts, 10.0, mid[1], status)
+    assert same_bits(mid[0], mid[1])
+    mid_q8 = K.q8k_quantize(mid[0], status)
+    out = [torch.full((pairs, hidden), float("nan"), device=gpu) for _ in range(2)]
+    K.moe_down(weights, mid_q8, True, wl, pairs, experts, out[0], status)
+    K.moe_down_rows(rows_form, mid_q8, wl, pairs, experts, out[1], status)
+    assert same_bits(out[0], out[1]) and int(status.item()) == 0
+
+
+# a last row tile of four rows and of 252, one superblock and an odd number of them
+@pytest.mark.parametrize("rows,width,inputs", [(4100, 1280, 2048), (7164, 256, 1025)])
+def test_ragged_row_tiles_run_alone(gpu, oracle, rows, width, inputs):
+    """A projection whose last row tile is not whole holds what the kernels of a few input rows publish."""
+    from yvex_amd import kernels as K
+    qt = oracle.IQ2_XXS
+    g = oracle.Generator(46, f"ragged.{rows}")
+    weights, status = dev(g.weights(qt, rows, width), gpu), K.new_status(gpu)
+    act = K.q8k_quantize(dev(g.normal(inputs * width).reshape(inputs, width), gpu), status)
+    got = K.matvec(weights, qt, rows, width, act, input_q8=True, input_rows=inputs, status=status)
+    stride = width // 256 * 292
+    for at in (0, 61, inputs - 5):
+        few = K.matvec(weights, qt, rows, width, act[at * stride:(at + 5) * stride].contiguous(), input_q8=True, input_rows=5,
+                       status=status)
+        assert same_bits(got[at:at + 5], few)
+    assert int(status.item()) == 0
+
+
 # 16, 32 and 64 input rows a workgroup of the staged kernel (on 256 compute units), ragged on both sides,
 # one chunk and several
 @pytest.mark.parametrize("rows,width,inputs", [(250, 384, 345), (256, 128, 850), (249, 256, 2045)])

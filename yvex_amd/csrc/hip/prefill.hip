@@ -124,29 +124,13 @@ __device__ __forceinline__ unsigned uniform32(unsigned v)
     return (unsigned)__builtin_amdgcn_readfirstlane((int)v);
 }
 
-// What one work item needs to know about its place in the problem.
-struct MfmaItem {
+// Row tiles [row_tile, row_end) of one token tile.
+struct MfmaRun {
     unsigned long long expert, pair0;
-    unsigned tokens, row_tile;
+    unsigned tokens, row_tile, row_end;
 };
 
-// A work item whose bucket record has been requested from memory but not looked at yet.
-struct MfmaItemRequest {
-    int state;                      // 0: requested, 1: the lists are inconsistent (skip it), 2: past the last item
-    bool partial;                   // the bucket's last, partial token tile
-    unsigned bucket, token_tile, row_tile;
-    unsigned long long first, population, expert;
-};
-
-// The item a workgroup runs after the current one.
-struct MfmaNextItem {
-    MfmaItem it;
-    int state;                      // as above (0: it holds the item)
-    bool ahead;                     // the current item's last rounds of copies fetch its first two windows
-    long long shift;                // from a weight row of the current item to the same row of this one
-};
-
-// One work item with NTB live 32-token blocks (NTB is 1 or 2).
+// A run of row tiles against one token tile of NTB live 32-token blocks (NTB is 1 or 2).
 //
 // Time slot (sb, m) = superblock sb, K chunk m: 2 NTB matrix instructions (low and high limb for
 // every token block) on the chunk's operands, which were built during the slot before: the
@@ -174,15 +158,13 @@ struct MfmaNextItem {
 // The loop body is one superblock in one basic block (requests past the end are clamped, and
 // superblocks past the end run with a zero row scale), so nothing leaves registers.
 //
-// Between two items of a workgroup: the item that follows is looked up while the first copies of
-// this one are in flight (`request_next` before them, `resolve_next` once they have landed), and
-// when it has the same shape the loop's last rounds of window copies, which have no superblock
-// of this item left to fetch, fetch its first two windows instead (`prefetched` tells the
-// item that they are there). Its first activation stage cannot come early: the publishing pass
-// uses the stages' memory.
-template <bool FUSED_UP, unsigned NTB, bool IMAGE, class Request, class Resolve>
-__device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it, bool prefetched,
-                                          Request &&request_next, Resolve &&resolve_next, MfmaNextItem &next)
+// From row tile to row tile nothing stops: superblocks are counted through (`step`), the windows fetched ahead are the
+// next tile's, the stages begin again with the token tile's first, and a tile's sums are published between two
+// steps. Only a run opens: where its tokens' rows lie, the first copies' round trip, the first operands, 9 000 to
+// 10 000 cycles that every item paid (36 000 in the loop of eight superblocks, 121 000 in one of 28) while items were dealt out one by
+// one. A tile that is not whole has lanes that repeat a row, and runs alone.
+template <bool FUSED_UP, unsigned NTB, bool IMAGE>
+__device__ __forceinline__ void rows_run(const MfmaArgs &a, const MfmaRun &it)
 {
     const GroupedProblem &pr = a.pr;
     constexpr unsigned R = 4u / NTB;                 // activation stages
@@ -235,15 +217,22 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
         }
     }
     const unsigned window_base = kWindowBase + wave * 2u * kWindowBytes;
-    // Windows past the last superblock: windows 0 and 1 of the next item (by parity, so that a
-    // third one repeats the first) when they are fetched ahead, else the last window again.
-    long long ahead_shift = 0;
-    bool ahead = false;
-    auto weight_piece = [&](unsigned sb, unsigned k) {
-        const unsigned to = window_base + (sb & 1u) * kWindowBytes + k * 1024u;
-        const bool past = sb > last;
-        const unsigned record = !past ? sb : ahead ? (sb - superblocks) & 1u : last;
-        long long offset = (past ? ahead_shift : 0ll) + (long long)(record * (IMAGE ? 72u : 66u));
+    // The window of the step that is asked for next: its superblock, the distance to its row tile, its step.
+    const unsigned steps = (it.row_end - it.row_tile) * superblocks;
+    const unsigned long long tile_bytes = (unsigned long long)kItemRows * pr.row_bytes;
+    unsigned window_sb = 0u, window_step = 0u;
+    unsigned long long window_tile = 0ull;
+    auto window_passed = [&] {                       // (behind the run's last step its bytes are fetched again)
+        const bool more = window_step + 1u < steps, wraps = window_sb == last;
+        ++window_step;
+        if (more) {
+            window_sb = wraps ? 0u : window_sb + 1u;
+            window_tile += wraps ? tile_bytes : 0ull;
+        }
+    };
+    auto weight_piece = [&](unsigned k) {            // the pieces of a window in order
+        const unsigned to = window_base + (window_step & 1u) * kWindowBytes + k * 1024u;
+        unsigned long long offset = window_tile + window_sb * (IMAGE ? 72u : 66u);
 #if defined(__HIP_DEVICE_COMPILE__)
         asm volatile("" : "+s"(offset));       // (one sum on the scalar unit, one addition a lane)
 #endif
@@ -251,6 +240,7 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
             ? window_from[k] + offset
             : (const unsigned char *)((unsigned long long)(window_from[k] + offset) & ~3ull);
         copy_to_lds_16(from, to);
+        if (k == 2u) window_passed();
     };
 
     // ---- activation rows this lane copies: wave w owns the 4-slot groups w (and w + 8) ----
@@ -278,8 +268,8 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
         const unsigned index = wave == 0u ? lane % T : 0u;
         scale_from = token_row((index % NTB) * 32u + index / NTB);
     }
-    // Where each pair's results go and its route weight, for the publishing pass: requested now,
-    // put into LDS once the previous item's publishing pass is over.
+    // Where each pair's results go and its route weight, for the publishing passes: requested now,
+    // put into LDS once the previous run's last one is over.
     const bool info_lane = tid < kTileTokens && tid < it.tokens;
     unsigned info_out = 0u;
     float info_weight = 1.0f;
@@ -289,11 +279,12 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
         info_out = (unsigned)(pr.out_by_source_pair ? source : ordered);
         if (pr.route_weights) info_weight = pr.route_weights[source];
     }
-    auto request = request_next();
     constexpr unsigned kActPieces = NTB + 1u;
-    auto act_piece = [&](unsigned sb, unsigned j) {
-        const unsigned base = kStageBase + (sb % R) * kStageBytes;
-        unsigned offset = (sb < last ? sb : last) * kQ8KBytes;
+    // the stage that is asked for next: its superblock and its place
+    unsigned stage_sb = 0u, stage_to = kStageBase;
+    auto act_piece = [&](unsigned j) {               // the pieces of a stage in order
+        const unsigned base = stage_to;
+        unsigned offset = stage_sb * kQ8KBytes;
 #if defined(__HIP_DEVICE_COMPILE__)
         asm volatile("" : "+s"(offset));
 #endif
@@ -301,13 +292,15 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
             copy_to_lds_16(copy_from[j] + offset, base + (wave + kRowWaves * j) * 1024u);
         } else {
             copy_to_lds_4(scale_from + offset, wave == 0u ? base + T * kActPitch : kTrashBase);
+            stage_sb = stage_sb == last ? 0u : stage_sb + 1u;
+            stage_to = stage_to == kStageBase + (R - 1u) * kStageBytes ? kStageBase : stage_to + kStageBytes;
         }
     };
-    // the copies issued after the barrier of superblock sb: the stage and the window just released
+    // the copies issued after the barrier of a step: the stage and the window just released, R and three steps ahead
     constexpr unsigned kRoundPieces = kActPieces + 3u;
-    auto round_piece = [&](unsigned sb, unsigned j) {
-        if (j < kActPieces) act_piece(sb + R, j);
-        else weight_piece(sb + 3u, j - kActPieces);
+    auto round_piece = [&](unsigned j) {
+        if (j < kActPieces) act_piece(j);
+        else weight_piece(j - kActPieces);
     };
 
     // ---- decode state ----
@@ -325,11 +318,11 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
     // + 66 sb) mod 4 (0 or 2) the fp16 scale sits o bytes into the window and the lane's 32 code
     // bytes at o + 2 + 32 h: in aligned dwords 8 h + o / 2 onwards, shifted by 2 bytes when o is
     // 0. Aligned dword 16 is the last dword of the fifth piece.
-    auto settle = [&](unsigned sb) {
+    auto settle = [&](unsigned step, unsigned sb) {  // (superblock `sb`, which only its parity and the last step need)
         if constexpr (IMAGE) {
             // The lane's record is nine dwords: pieces 3 h and 3 h + 1 whole, and of piece 3 h + 2
             // the first dword (bytes 32-35 of the row's 72) or the last (bytes 68-71).
-            const unsigned at = window_base + (sb & 1u) * kWindowBytes + (3u * h * 32u + r) * 16u;
+            const unsigned at = window_base + (step & 1u) * kWindowBytes + (3u * h * 32u + r) * 16u;
             const v4i first = lds_read_v4i(at), second = lds_read_v4i(at + 512u), third = lds_read_v4i(at + 1024u);
             head = (unsigned)first[0];
             grids[0] = (unsigned)first[1];
@@ -340,15 +333,14 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
             aux[2] = (unsigned)second[2];
             grids[3] = (unsigned)second[3];
             aux[3] = (unsigned)(h ? third[3] : third[0]);
-            row_scale = sb < superblocks ? 0.125f * f16_bits_to_float(head & 0xffffu) : 0.0f;
+            row_scale = step < steps ? 0.125f * f16_bits_to_float(head & 0xffffu) : 0.0f;
             return;
         }
-        const unsigned clamped = sb < last ? sb : last;
-        const unsigned o = (row_misalign + 2u * clamped) & 3u;
+        const unsigned o = (row_misalign + 2u * sb) & 3u;
         // Aligned dwords 8 h .. 8 h + 8 of the window: pieces 2 h and 2 h + 1 whole, and the dword
         // behind them (the first of piece 2, or the last of the fifth piece, which is aligned
         // dword 16). The lane's nine dwords start at dword 8 h + o / 2 of the window.
-        const unsigned at = window_base + (sb & 1u) * kWindowBytes + (2u * h * 32u + r) * 16u;
+        const unsigned at = window_base + (step & 1u) * kWindowBytes + (2u * h * 32u + r) * 16u;
         const v4i first = lds_read_v4i(at), second = lds_read_v4i(at + 512u), third = lds_read_v4i(at + 1024u);
         const unsigned d[9] = {(unsigned)first[0], (unsigned)first[1], (unsigned)first[2], (unsigned)first[3],
                                (unsigned)second[0], (unsigned)second[1], (unsigned)second[2], (unsigned)second[3],
@@ -366,7 +358,7 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
             grids[g] = __builtin_amdgcn_alignbyte(w[2u * g + 1u], w[2u * g], shift);
             aux[g] = __builtin_amdgcn_alignbyte(w[2u * g + 2u], w[2u * g + 1u], shift);
         }
-        const float mine = sb < superblocks ? 0.125f * f16_bits_to_float(scale16) : 0.0f;
+        const float mine = step < steps ? 0.125f * f16_bits_to_float(scale16) : 0.0f;
         row_scale = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute((int)(4u * r), (int)__float_as_uint(mine)));
     };
     // table lookups of K chunk c: subgroups 2 (c & 1) and 2 (c & 1) + 1 of group c / 2
@@ -402,63 +394,36 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
     unsigned frag_at = kStageBase + r * kActPitch + (((8u * h) ^ (r & 15u)) << 4);
 
     // ---- prologue ----
-    // Copies in flight when the loop starts are those of its own schedule: a round (stage sb + R,
-    // window sb + 3) is issued after the barrier of superblock sb, four pieces in slots 6 and 7 and
-    // the rest at the start of the next superblock, so rounds -(R - 1) .. -1 are issued here
-    // (windows 0 and 1 are needed before them; the rounds before -1 repeat window 1, which keeps
-    // the counts below the same for every superblock).
-    lds_barrier();     // every wave is done with the previous item's stages and pair records (its stores may still be on their way)
-    if (prefetched) {      // windows 0 and 1 came with the previous item's last rounds
+    // Copies in flight when the loop starts are those of its own schedule: a round (stage step + R,
+    // window step + 3) is issued after the barrier of a step, four pieces in slots 6 and 7 and
+    // the rest at the start of the next one, so rounds -(R - 1) .. -1 are issued here (windows 0 and 1 are needed before
+    // them; a round before -1 has three copies to where nobody reads in the place of a window, which keeps the counts below the same for
+    // every step).
+    lds_barrier();     // every wave is done with the previous run's stages and pair records (its stores may still be on their way)
 #pragma unroll
-        for (unsigned j = 0; j < kActPieces; ++j) act_piece(0u, j);
-        __builtin_amdgcn_s_waitcnt(0x0f70u);   // vmcnt(0): stage 0 has landed
-    } else {
+    for (unsigned k = 0; k < 3u; ++k) weight_piece(k);
 #pragma unroll
-        for (unsigned k = 0; k < 3u; ++k) weight_piece(0u, k);
+    for (unsigned j = 0; j < kActPieces; ++j) act_piece(j);
 #pragma unroll
-        for (unsigned j = 0; j < kActPieces; ++j) act_piece(0u, j);
-#pragma unroll
-        for (unsigned k = 0; k < 3u; ++k) weight_piece(1u, k);
-        __builtin_amdgcn_s_waitcnt(0x0f73u);   // vmcnt(3): window 0 and stage 0 have landed
-    }
+    for (unsigned k = 0; k < 3u; ++k) weight_piece(k);
+    __builtin_amdgcn_s_waitcnt(0x0f73u);   // vmcnt(3): window 0 and stage 0 have landed
     if (info_lane) lds_write_uint2(kPairInfoBase + tid * 8u, make_uint2(info_out, __float_as_uint(info_weight)));
-    // The next item, and whether its first windows can ride on this item's last rounds: both
-    // items cover whole row tiles of equal geometry (then the same lane copies the same piece of
-    // the same row, one fixed distance on), and the window parity comes out right.
-    resolve_next(request, next);
-    next.ahead = false;
-    next.shift = 0;
-    if (next.state == 0 && superblocks >= 4u && (superblocks & 1u) == 0u &&
-        (!FUSED_UP || (pr.expert_bytes == pr.up_expert_bytes && pr.row_bytes == pr.up_row_bytes)) &&
-        (unsigned long long)(it.row_tile + 1u) * kItemRows <= a.out_rows &&
-        (unsigned long long)(next.it.row_tile + 1u) * kItemRows <= a.out_rows) {
-        next.ahead = true;
-        next.shift = ((long long)next.it.expert - (long long)it.expert) * (long long)pr.expert_bytes +
-                     ((long long)next.it.row_tile - (long long)it.row_tile) * (long long)kItemRows * (long long)pr.row_bytes;
-    }
-    ahead = next.ahead;
-    ahead_shift = next.shift;
-    settle(0u);
+    settle(0u, 0u);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the window's reads have returned before it is refilled
 #pragma unroll
     for (unsigned x = 1; x + 1u < R; ++x) {
 #pragma unroll
-        for (unsigned j = 0; j < kActPieces; ++j) act_piece(x, j);
+        for (unsigned j = 0; j < kActPieces; ++j) act_piece(j);
 #pragma unroll
-        for (unsigned k = 0; k < 3u; ++k) weight_piece(1u, k);
+        for (unsigned k = 0; k < 3u; ++k) copy_to_lds_4(scale_from, kTrashBase);
     }
 #pragma unroll
-    for (unsigned j = 0; j < 4u; ++j) round_piece(0u - 1u, j);
+    for (unsigned j = 0; j < 4u; ++j) round_piece(j);
     lookup(0u);
     lookup(1u);
     build(0u);
     __syncthreads();   // every wave's share of stage 0 has landed
 
-    double acc[NTB][16];            // row sums: float terms added in double, in superblock order
-#pragma unroll
-    for (unsigned tb = 0; tb < NTB; ++tb)
-#pragma unroll
-        for (unsigned i = 0; i < 16u; ++i) acc[tb][i] = 0.0;
     v16i sum_lo[NTB], sum_hi[NTB];   // integer sums of the running superblock
     v4i frag[2][NTB];                // [slot & 1]: re-requested for two slots on as soon as it is used
 #pragma unroll
@@ -466,18 +431,27 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
         frag[0][tb] = lds_read_v4i(frag_at + tb * 32u * kActPitch);
         frag[1][tb] = lds_read_v4i((frag_at ^ 16u) + tb * 32u * kActPitch);
     }
-    // Waits, counted in copies issued later than the one needed:
-    //   * before settle(sb + 1) at slot 5: window sb + 1 belongs to round sb - 2, so one full
-    //     round (sb - 1) may be in flight;
-    //   * at the barrier of superblock sb: stage sb + 1 belongs to round sb + 1 - R, so the
+    // Waits, counted in copies issued later than the one needed (a tile's stores among them make a wait longer, never
+    // shorter), step by step:
+    //   * before settle(step + 1) at slot 5: window step + 1 belongs to round step - 2, so one full
+    //     round (step - 1) may be in flight;
+    //   * at the barrier of a step: stage step + 1 belongs to round step + 1 - R, so the
     //     window of that round and R - 2 full rounds may be in flight.
     constexpr unsigned kSettleInFlight = kRoundPieces;
     constexpr unsigned kBarrierInFlight = 3u + (R - 2u) * kRoundPieces;
 
-    for (unsigned sb = 0; sb < superblocks; ++sb) {
+    unsigned step = 0u, stage = kStageBase;              // the running step and its stage
+    const float limit_f32 = (float)a.limit;
+    const bool whole_quads = (a.out_rows & 3u) == 0u;
+    for (unsigned row_tile = it.row_tile; row_tile < it.row_end; ++row_tile) {
+    double acc[NTB][16];            // row sums: float terms added in double, in superblock order
+#pragma unroll
+    for (unsigned tb = 0; tb < NTB; ++tb)
+#pragma unroll
+        for (unsigned i = 0; i < 16u; ++i) acc[tb][i] = 0.0;
+    for (unsigned sb = 0; sb < superblocks; ++sb, ++step) {
         float rs = 0.0f, ts = 0.0f;  // scales of the lane's weight row and of its token (of block h) in this superblock
         v32f scale;                  // their products, where the sums of that row and token are
-        const unsigned stage = kStageBase + (sb % R) * kStageBytes;
 #pragma unroll
         for (unsigned m = 0; m < 8u; ++m) {
             // ---- 2 NTB matrix instructions with the rest of the slot's work between them, a
@@ -530,7 +504,7 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
                 // one's (its window has landed: see the counts above)
                 __builtin_amdgcn_s_waitcnt(0x0f70u | (kSettleInFlight & 15u) | ((kSettleInFlight >> 4) << 14));
                 rs = row_scale;
-                settle(sb + 1u);
+                settle(step + 1u, sb == last ? 0u : sb + 1u);
             }
             if (m == 4u) {
                 // this superblock's token scales, while its stage is still held
@@ -549,16 +523,17 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
                 // reads this stage again and the next one is complete.
                 __builtin_amdgcn_s_waitcnt(0x0070u | (kBarrierInFlight & 15u) | ((kBarrierInFlight >> 4) << 14));
                 __syncthreads();
-                const unsigned flip = (sb % R == R - 1u) ? 0u - (R - 1u) * kStageBytes : kStageBytes;
+                const unsigned flip = stage == kStageBase + (R - 1u) * kStageBytes ? 0u - (R - 1u) * kStageBytes : kStageBytes;
                 frag_at += flip;
+                stage += flip;
             }
             // ---- the round of copies into the stage and the window just released: two pieces a
             // slot behind the barrier, the rest at the start of the next superblock ----
             if (m > kBarrierSlot) {
-                round_piece(sb, 2u * (m - kBarrierSlot - 1u));
-                round_piece(sb, 2u * (m - kBarrierSlot - 1u) + 1u);
+                round_piece(2u * (m - kBarrierSlot - 1u));
+                round_piece(2u * (m - kBarrierSlot - 1u) + 1u);
             }
-            if (m < kRoundPieces - 4u) round_piece(sb - 1u, 4u + m);
+            if (m < kRoundPieces - 4u) round_piece(4u + m);
             // ---- the superblock's sums are complete: ((0.125 d_w) d_a) (128 hi + lo) ----
             if (m == 7u) {
 #pragma unroll
@@ -578,11 +553,9 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
     // The values go from the registers straight to memory, 16 bytes a lane: the two halves of a
     // wave complete 32 bytes of a token's row per store, the four (two) stores of a token block
     // a whole cache line (half of one), which the L2 merges before it writes them back. No LDS,
-    // no barrier: the stores drain while the next item starts, and copies past the end that are
-    // still in flight land in stages and windows nobody reads before the next item has waited
+    // no barrier: the stores drain while the next tile is worked on; copies past the run's end that are
+    // still in flight land in stages and windows nobody reads before the next run has waited
     // for copies of its own, which the same wave issues later to the same places.
-    const float limit_f32 = (float)a.limit;
-    const bool whole_quads = (a.out_rows & 3u) == 0u;
     bool bad = false;
 #pragma unroll
     for (unsigned tb = 0; tb < NTB; ++tb) {
@@ -591,7 +564,7 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
         float *const out_row = pr.out + (unsigned long long)info.x * a.out_rows;
 #pragma unroll
         for (unsigned q = 0; q < (FUSED_UP ? 2u : 4u); ++q) {
-            const unsigned row = it.row_tile * kItemRows + wave * (FUSED_UP ? 16u : 32u) + 8u * q + 4u * h;
+            const unsigned row = row_tile * kItemRows + wave * (FUSED_UP ? 16u : 32u) + 8u * q + 4u * h;
             float value[4];
             bool good = true;
             if constexpr (FUSED_UP) {
@@ -627,11 +600,10 @@ __device__ __forceinline__ void rows_item(const MfmaArgs &a, const MfmaItem &it,
         }
     }
     if (bad) raise_status(a.status, 1);
-    // An item with another number of token blocks lays its stages out differently, so that its
-    // copies come from other waves than this item's copies to the same bytes: then this item's
-    // last copies land first (the next item's opening barrier makes that hold for every wave).
-    const unsigned blocks_next = next.state != 0 ? 0u : next.it.tokens <= 32u ? 1u : 2u;
-    if (blocks_next != NTB) __builtin_amdgcn_s_waitcnt(0x0070u);   // vmcnt(0)
+    }
+    // (a run with another number of token blocks lays its stages out differently, so that its copies come from other waves
+    // than this run's to the same bytes: all have landed here, and the next run's opening barrier makes that hold for every wave)
+    __builtin_amdgcn_s_waitcnt(0x0070u);   // vmcnt(0)
 }
 
 template <bool FUSED_UP, bool IMAGE>
@@ -651,9 +623,8 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
     // bucket), and the tables built only where there is an item.
     unsigned long long population_here = 0ull;
     if (tid < 256u && tid < buckets) population_here = fixed ? pr.pairs : pr.bucket_populations[tid];
-    // Full 64-pair tiles come first in the item list, then the partial last tiles by size,
-    // largest first: every workgroup, walking the list with the grid's stride, gets the same
-    // share of each kind of item, and the short items come last. Bucket b's first full tile is
+    // Full 64-pair tiles come first in the list of tiles, then the partial last tiles of more than 32
+    // pairs, then those of fewer. Bucket b's first full tile is
     // the number of full tiles before it (a scan over the 256 bucket slots); its place in its
     // class of partial tiles (more than 32 pairs, or fewer) is its rank among the buckets of
     // that class, in bucket order, from ballots and per-wave totals.
@@ -695,123 +666,75 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
         return;
     }
 
-    // weight rows (gate/up row pairs when fused) per work item
+    // The row tiles of all token tiles, a token tile's one after another, are dealt out in one piece of equal cost a
+    // workgroup; a tile of 33 to 64 pairs costs four and one of fewer three (64 experts of 50 / 28 pairs: gate and up
+    // 366 / 277 us, down 221 / 173). Neighbouring pieces read the same weights where a bucket has several
+    // token tiles, so they go to workgroups of one XCD (workgroups are dealt to the eight XCDs in turn).
     constexpr unsigned kItemRows = FUSED_UP ? 128u : 256u;
+    constexpr unsigned kWide = 4u, kNarrow = 3u;                // costs of a row tile
     const unsigned row_tiles = (a.out_rows + kItemRows - 1u) / kItemRows;
-    const unsigned long long full_items = (unsigned long long)lds_read_u32(kTileStartBase + 4u * buckets) * row_tiles;
-    unsigned members[2];
-    unsigned long long items = full_items;
-    for (unsigned c = 0; c < 2u; ++c) {
-        members[c] = lds_read_u32(kClassCountBase + 4u * c);
-        items += (unsigned long long)members[c] * row_tiles;
-    }
-    // Neighbouring items read the same weights (a bucket's token tiles of one row tile), so they go to
-    // workgroups of one XCD (workgroups are dealt to the eight XCDs in turn), whose L2 then fetches them
-    // once: 2048 rows of 7168 with uneven experts, gate/up 1506 -> 1480 us; even experts, whose
-    // buckets are single tiles, are indifferent.
-    const unsigned start = gridDim.x % 8u ? blockIdx.x : (blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
-    if (start >= items) return;
-    mfma_tables_fill();
-    __syncthreads();
-
-    // ---- which bucket, row tile and token tile an item is: the bucket's record is requested... ----
-    auto request_item = [&](unsigned long long item) {
-        MfmaItemRequest q;
-        q.state = 0;
-        q.partial = false;
-        q.bucket = q.token_tile = q.row_tile = 0u;
-        q.first = q.population = q.expert = 0ull;
-        if (item >= items) {
-            q.state = 2;
-            return q;
-        }
-        if (item < full_items) {
-            unsigned low = 0u, high = buckets;   // the last bucket whose first full tile is <= item's
-            while (low + 1u < high) {
-                const unsigned middle = (low + high) >> 1;
-                if ((unsigned long long)lds_read_u32(kTileStartBase + 4u * middle) * row_tiles <= item)
-                    low = middle;
-                else
-                    high = middle;
-            }
-            const unsigned tile_first = lds_read_u32(kTileStartBase + 4u * low);
-            const unsigned bucket_tiles = lds_read_u32(kTileStartBase + 4u * (low + 1u)) - tile_first;
-            const unsigned long long local = item - (unsigned long long)tile_first * row_tiles;
-            if (!bucket_tiles) {
-                q.state = 1;
-                return q;
-            }
-            q.bucket = low;
-            q.token_tile = (unsigned)(local % bucket_tiles);
-            q.row_tile = (unsigned)(local / bucket_tiles);
-        } else {
-            unsigned long long rest = item - full_items;
-            unsigned c = 0u;
-            if (rest >= (unsigned long long)members[0] * row_tiles) {
-                rest -= (unsigned long long)members[0] * row_tiles;
-                c = 1u;
-            }
-            if (!members[c]) {
-                q.state = 1;
-                return q;
-            }
-            q.bucket = lds_read_u16(kClassListBase + (c * 256u + (unsigned)(rest % members[c])) * 2u);
-            q.row_tile = (unsigned)(rest / members[c]);
-            q.partial = true;               // its token tile is the one after the bucket's full tiles
-        }
-        if (q.bucket >= buckets) {
-            q.state = 1;
-            return q;
-        }
-        q.first = fixed ? 0ull : pr.bucket_offsets[q.bucket];
-        q.population = fixed ? pr.pairs : pr.bucket_populations[q.bucket];
-        q.expert = fixed ? 0ull : pr.expert_ids[q.bucket];
-        return q;
+    const unsigned full_tiles = uniform32(lds_read_u32(kTileStartBase + 4u * buckets));
+    const unsigned members[2] = {uniform32(lds_read_u32(kClassCountBase)), uniform32(lds_read_u32(kClassCountBase + 4u))};
+    const unsigned long long wide = (unsigned long long)(full_tiles + members[0]) * row_tiles,
+                             narrow = (unsigned long long)members[1] * row_tiles;
+    const unsigned long long cost = kWide * wide + kNarrow * narrow;
+    const unsigned who = gridDim.x % 8u ? blockIdx.x : (blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
+    auto place_of = [&](unsigned workgroup) {                   // the first row tile of its piece
+        const unsigned long long at = cost / gridDim.x * workgroup + cost % gridDim.x * workgroup / gridDim.x;
+        return at <= kWide * wide ? (at + kWide - 1u) / kWide : wide + (at - kWide * wide + kNarrow - 1u) / kNarrow;
     };
-    // ---- ... and looked at later. Every lane holds the same values: the item is kept in scalar
-    // registers. ----
     auto uniform64 = [&](unsigned long long v) {
         return (unsigned long long)uniform32((unsigned)v) | ((unsigned long long)uniform32((unsigned)(v >> 32)) << 32);
     };
-    auto resolve_item = [&](const MfmaItemRequest &q, MfmaNextItem &out) {
-        out.ahead = false;
-        out.shift = 0;
-        out.state = (int)uniform32((unsigned)q.state);
-        if (out.state == 2) return;
-        const unsigned long long first = uniform64(q.first), population = uniform64(q.population);
-        const unsigned token_tile = uniform32(q.partial ? (unsigned)(population / kTileTokens) : q.token_tile);
-        out.it.expert = uniform64(q.expert);
-        out.it.row_tile = uniform32(q.row_tile);
-        if (out.state != 0 || out.it.expert >= pr.experts || first + population > pr.pairs ||
-            (unsigned long long)token_tile * kTileTokens >= population || out.it.row_tile >= row_tiles) {
-            if (tid == 0u) raise_status(a.status, 2);
-            out.state = 1;
-            return;
-        }
-        const unsigned long long left = population - (unsigned long long)token_tile * kTileTokens;
-        out.it.pair0 = first + (unsigned long long)token_tile * kTileTokens;
-        out.it.tokens = left < kTileTokens ? (unsigned)left : kTileTokens;
-    };
+    unsigned long long at = uniform64(place_of(who));
+    const unsigned long long end = uniform64(place_of(who + 1u));
+    if (at >= end) return;
+    mfma_tables_fill();
+    __syncthreads();
 
-    unsigned long long item = start;
-    MfmaNextItem current;
-    resolve_item(request_item(item), current);
-    bool prefetched = false;
-    while (current.state != 2) {
-        MfmaNextItem next;
-        const unsigned long long following = item + gridDim.x;
-        auto request_next = [&] { return request_item(following); };
-        if (current.state == 0) {
-            if (current.it.tokens <= 32u)
-                rows_item<FUSED_UP, 1u, IMAGE>(a, current.it, prefetched, request_next, resolve_item, next);
-            else
-                rows_item<FUSED_UP, 2u, IMAGE>(a, current.it, prefetched, request_next, resolve_item, next);
+    const bool ragged = a.out_rows % kItemRows != 0u;           // the last row tile is not whole
+    while (at < end) {
+        const unsigned tile = uniform32((unsigned)(at / row_tiles));
+        MfmaRun run;
+        run.row_tile = uniform32((unsigned)(at % row_tiles));
+        const unsigned long long left = end - at;
+        run.row_end = left < row_tiles - run.row_tile ? run.row_tile + (unsigned)left : row_tiles;
+        if (ragged && run.row_end == row_tiles && run.row_end - run.row_tile > 1u) --run.row_end;
+        at += run.row_end - run.row_tile;
+        // which bucket the tile is of, and which of its tiles
+        unsigned bucket, token_tile = 0u;
+        const bool partial = tile >= full_tiles;                // the one behind the bucket's full tiles
+        if (!partial) {
+            unsigned low = 0u, high = buckets;                  // the last bucket whose first full tile is <= tile: it has it
+            while (low + 1u < high) {
+                const unsigned middle = (low + high) >> 1;
+                if (lds_read_u32(kTileStartBase + 4u * middle) <= tile) low = middle;
+                else high = middle;
+            }
+            bucket = low;
+            token_tile = tile - lds_read_u32(kTileStartBase + 4u * low);
         } else {
-            resolve_item(request_next(), next);
+            const unsigned rank = tile - full_tiles, c = rank < members[0] ? 0u : 1u;
+            bucket = lds_read_u16(kClassListBase + (c * 256u + rank - (c ? members[0] : 0u)) * 2u);
         }
-        prefetched = current.state == 0 && next.ahead;
-        current = next;
-        item = following;
+        bucket = uniform32(bucket);
+        if (bucket >= buckets) {
+            if (tid == 0u) raise_status(a.status, 2);
+            continue;
+        }
+        const unsigned long long first = fixed ? 0ull : uniform64(pr.bucket_offsets[bucket]);
+        const unsigned long long population = fixed ? pr.pairs : uniform64(pr.bucket_populations[bucket]);
+        run.expert = fixed ? 0ull : uniform64(pr.expert_ids[bucket]);
+        token_tile = uniform32(partial ? (unsigned)(population / kTileTokens) : token_tile);
+        if (run.expert >= pr.experts || first + population > pr.pairs || (unsigned long long)token_tile * kTileTokens >= population) {
+            if (tid == 0u) raise_status(a.status, 2);
+            continue;
+        }
+        const unsigned long long tokens = population - (unsigned long long)token_tile * kTileTokens;
+        run.pair0 = first + (unsigned long long)token_tile * kTileTokens;
+        run.tokens = tokens < kTileTokens ? (unsigned)tokens : kTileTokens;
+        if (run.tokens <= 32u) rows_run<FUSED_UP, 1u, IMAGE>(a, run);
+        else rows_run<FUSED_UP, 2u, IMAGE>(a, run);
     }
 }
 
