@@ -668,8 +668,11 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
 
     // The row tiles of all token tiles, a token tile's one after another, are dealt out in one piece of equal cost a
     // workgroup; a tile of 33 to 64 pairs costs four and one of fewer three (64 experts of 50 / 28 pairs: gate and up
-    // 366 / 277 us, down 221 / 173). Neighbouring pieces read the same weights where a bucket has several
-    // token tiles, so they go to workgroups of one XCD (workgroups are dealt to the eight XCDs in turn).
+    // 352 / 253 us, down 193 / 141). Where there are enough of the short ones, every workgroup has as many of the long ones as the
+    // next, or one more, and short ones make up the difference (2048 uneven rows, gate and up: a workgroup in twenty
+    // had 5 % more to do than the mean). Neighbouring pieces read the same weights where a bucket has several
+    // token tiles, so they go to workgroups of one XCD (workgroups are dealt to the eight XCDs in turn; not so, 1231 -> 1270 us of 256
+    // experts by 64).
     constexpr unsigned kItemRows = FUSED_UP ? 128u : 256u;
     constexpr unsigned kWide = 4u, kNarrow = 3u;                // costs of a row tile
     const unsigned row_tiles = (a.out_rows + kItemRows - 1u) / kItemRows;
@@ -679,21 +682,35 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
                              narrow = (unsigned long long)members[1] * row_tiles;
     const unsigned long long cost = kWide * wide + kNarrow * narrow;
     const unsigned who = gridDim.x % 8u ? blockIdx.x : (blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
-    auto place_of = [&](unsigned workgroup) {                   // the first row tile of its piece
-        const unsigned long long at = cost / gridDim.x * workgroup + cost % gridDim.x * workgroup / gridDim.x;
-        return at <= kWide * wide ? (at + kWide - 1u) / kWide : wide + (at - kWide * wide + kNarrow - 1u) / kNarrow;
+    auto share_of = [&](unsigned long long all, unsigned workgroup) {       // what the workgroups before have
+        return all / gridDim.x * workgroup + all % gridDim.x * workgroup / gridDim.x;
+    };
+    const bool level = cost / gridDim.x >= kWide * (wide / gridDim.x + 1u);
+    auto narrow_place = [&](unsigned workgroup) {
+        return wide + (share_of(cost, workgroup) - kWide * share_of(wide, workgroup) + kNarrow - 1u) / kNarrow;
+    };
+    auto place_of = [&](unsigned workgroup) {                   // the first row tile of its piece, of its long ones
+        const unsigned long long at = share_of(cost, workgroup);
+        return level ? share_of(wide, workgroup)
+             : at <= kWide * wide ? (at + kWide - 1u) / kWide : wide + (at - kWide * wide + kNarrow - 1u) / kNarrow;
     };
     auto uniform64 = [&](unsigned long long v) {
         return (unsigned long long)uniform32((unsigned)v) | ((unsigned long long)uniform32((unsigned)(v >> 32)) << 32);
     };
     unsigned long long at = uniform64(place_of(who));
-    const unsigned long long end = uniform64(place_of(who + 1u));
-    if (at >= end) return;
+    unsigned long long end = uniform64(place_of(who + 1u));
+    unsigned long long narrow_at = level ? uniform64(narrow_place(who)) : 0ull;
+    const unsigned long long narrow_end = level ? uniform64(narrow_place(who + 1u)) : 0ull;
+    if (at >= end && narrow_at >= narrow_end) return;
     mfma_tables_fill();
     __syncthreads();
 
     const bool ragged = a.out_rows % kItemRows != 0u;           // the last row tile is not whole
-    while (at < end) {
+    while (at < end || narrow_at < narrow_end) {
+        if (at >= end) {
+            at = narrow_at;
+            end = narrow_at = narrow_end;
+        }
         const unsigned tile = uniform32((unsigned)(at / row_tiles));
         MfmaRun run;
         run.row_tile = uniform32((unsigned)(at % row_tiles));
