@@ -55,8 +55,22 @@ __device__ __forceinline__ f16x8 bytes_to_f16(unsigned first, unsigned second)
     return f16x8{pair[0][0], pair[0][1], pair[1][0], pair[1][1], pair[2][0], pair[2][1], pair[3][0], pair[3][1]};
 }
 
+// Four bytes (at most 127) as f16, each twice.
+__device__ __forceinline__ f16x8 byte_pairs_to_f16(unsigned bytes)
+{
+    const f16x2 bias = {(_Float16)1024.0f, (_Float16)1024.0f};
+    f16x2 pair[4];
+#pragma unroll
+    for (unsigned i = 0; i < 4u; ++i) {
+        const unsigned bits = __builtin_amdgcn_perm(0x64646464u, bytes, 0x04000400u + 0x00010001u * i);
+        pair[i] = __builtin_bit_cast(f16x2, bits) - bias;
+    }
+    return f16x8{pair[0][0], pair[0][1], pair[1][0], pair[1][1], pair[2][0], pair[2][1], pair[3][0], pair[3][1]};
+}
+
 // Q4_K: a minimum per 32 values. The sums of two neighbours (at most 4096 in magnitude) in two parts f16 holds, each on
-// half of the K step: multiples of 32 for lanes of half 0, what is left for those of half 1.
+// half of the K step: multiples of 32 for lanes of half 0, what is left for those of half 1. (dense_q4k.hip, whose lanes hold all
+// sixteen sums anyway; on the operands below its tiles are 2 to 3 % slower.)
 __device__ __forceinline__ f16x8 q4k_bsum_operand(const uint4 &b0, const uint4 &b1, unsigned half)
 {
     const unsigned w[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
@@ -70,8 +84,9 @@ __device__ __forceinline__ f16x8 q4k_bsum_operand(const uint4 &b0, const uint4 &
     return out;
 }
 
-// Q2_K: a minimum per 16 values, eight of the sixteen sums a lane.
-__device__ __forceinline__ f16x8 q2k_bsum_operand(const uint4 &b)
+// Eight of a block's sums of sixteen values: a K step of sixteen on both halves of a wave. Q2_K has a minimum for each, Q4_K one for
+// two (rows_q4k.hip: 453 -> 423 vector instructions a superblock and wave of 64 tokens against the operand above).
+__device__ __forceinline__ f16x8 bsum_operand(const uint4 &b)
 {
     const unsigned w[4] = {b.x, b.y, b.z, b.w};
     f16x8 out;

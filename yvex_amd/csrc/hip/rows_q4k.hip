@@ -18,7 +18,9 @@
 // of two floats rounded once, bit for bit what V_MUL_F32 gives (denormals and infinities too), and
 // the row scales need no place in LDS. The sums are kept from being rounded in every turn of the loop
 // for the sake of its last (what the compiler made of it). 600 -> 453 vector instructions a superblock and wave of 64 tokens; 1111
-// rows of 7168 by eight of 256 Q4_K experts with uneven routing 2530 -> 2213 us.
+// rows of 7168 by eight of 256 Q4_K experts with uneven routing 2530 -> 2213 us. A Q4_K minimum meets its sub-block's two sums of
+// sixteen as they lie, twice, instead of their sum in two parts, and the wave's number is scalar: 453 -> 423; 32 experts of 128 pairs, gate and up of
+// 7168 x 2048 434 -> 409 us, down 275 -> 258, Q2_K down rows of 64 by 64 133 -> 125.
 //
 // What differs is how the operands arrive. A lane that fetches its own 16-byte pieces of a
 // 144-byte weight block and of a 292-byte activation block touches up to 64 cache lines per load
@@ -99,7 +101,8 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
 {
     static_assert(QT == QT_Q4_K || (QT == QT_Q2_K && !FUSED), "Q4_K rows, or Q2_K rows of a plain projection");
     const GroupedProblem &pr = g.pr;
-    const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    // (the wave's number kept scalar, and with it the copies' places in LDS)
+    const unsigned tid = threadIdx.x, lane = tid & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const unsigned r = lane & 31u, h = lane >> 5;
     constexpr unsigned kWgRows = FUSED ? 64u : 128u;        // output rows of a workgroup
     constexpr unsigned kWaveRows = FUSED ? 16u : 32u;
@@ -110,7 +113,7 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
         const unsigned live = token < tile.tokens ? token : tile.tokens - 1u;   // padding repeats a row
         const unsigned long long ordered = tile.first + live;
         const unsigned long long source = pr.order ? pr.order[ordered] : ordered;
-        const unsigned long long act_row = pr.act_by_ordered_pair ? ordered : source / pr.topk;
+        const unsigned long long act_row = pr.act_by_ordered_pair ? ordered : (unsigned)source / pr.topk;     // (pairs fit 32 bits)
         return (const unsigned char *)pr.activations + act_row * pr.act_stride;
     };
 
@@ -163,28 +166,22 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
         if constexpr (QT == QT_Q2_K) {
 #pragma unroll
             for (unsigned k = 0; k < kRounds; ++k)
-                copy_to_lds_4(weight_from[k] + w_at, (unsigned)__builtin_amdgcn_readfirstlane((int)(w_to + 256u * k)));
+                copy_to_lds_4(weight_from[k] + w_at, w_to + 256u * k);
         } else {
 #pragma unroll
             for (unsigned k = 0; k < 4u; ++k)
-                copy_to_lds_16(weight_from[k] + w_at, (unsigned)__builtin_amdgcn_readfirstlane((int)(w_to + 1024u * k)));
-            copy_to_lds_16_first32(weight_from[4] + w_at, (unsigned)__builtin_amdgcn_readfirstlane((int)(w_to + 4096u)));
+                copy_to_lds_16(weight_from[k] + w_at, w_to + 1024u * k);
+            copy_to_lds_16_first32(weight_from[4] + w_at, w_to + 4096u);
         }
 #pragma unroll
         for (unsigned k = 0; k < 2u * NT; ++k)
-            copy_to_lds_16(act_from[k] + a_at,
-                           (unsigned)__builtin_amdgcn_readfirstlane(
-                               (int)(kQ4ActBase + buffer * kQ4Tokens * 256u + 16u * (64u * wave + 256u * k))));
+            copy_to_lds_16(act_from[k] + a_at, kQ4ActBase + buffer * kQ4Tokens * 256u + 16u * (64u * wave + 256u * k));
         // (wave 3 and, with one token block, part of the others copy into bytes nobody reads,
         // which is cheaper than a branch around the instruction)
         if (wave == 0u)
-            copy_to_lds_4(extra_from + a_at,
-                          (unsigned)__builtin_amdgcn_readfirstlane((int)(kQ4ScaleBase + buffer * kQ4Tokens * 4u)));
+            copy_to_lds_4(extra_from + a_at, kQ4ScaleBase + buffer * kQ4Tokens * 4u);
         else
-            copy_to_lds_16(extra_from + a_at,
-                           (unsigned)__builtin_amdgcn_readfirstlane(
-                               (int)(wave == 3u ? kQ4TrashBase
-                                                : kQ4BsumBase + buffer * kQ4Tokens * 32u + 1024u * (wave - 1u))));
+            copy_to_lds_16(extra_from + a_at, wave == 3u ? kQ4TrashBase : kQ4BsumBase + buffer * kQ4Tokens * 32u + 1024u * (wave - 1u));
     };
 
     double acc[NT][16];      // row sums: a float term per superblock, added in double in superblock order
@@ -253,7 +250,7 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
             const unsigned sc_low[2] = {sc_pack[0] & 0x07070707u, sc_pack[1] & 0x07070707u};
             const unsigned sc_high[2] = {sc_pack[0] >> 3 & 0x07070707u, sc_pack[1] >> 3 & 0x07070707u};
             scales16 = head.x;
-            m_op = bytes_to_f16(mn_pack[0], mn_pack[1]);     // the same on both halves, against the two parts of the sums
+            m_op = byte_pairs_to_f16(h ? mn_pack[1] : mn_pack[0]);
 #pragma unroll
             for (unsigned j = 0; j < 4u; ++j) {
                 const uint4 q = read16(w_at + 16u + 32u * j + 16u * h);
@@ -286,9 +283,7 @@ __device__ __forceinline__ void rows_q4k_tile(const RowsQ4kArgs &g, const Q4Tile
             const unsigned token = nt * 32u + r;
             const float da = __uint_as_float(lds_read_u32(kQ4ScaleBase + buffer * kQ4Tokens * 4u + 4u * token));
             const unsigned at = kQ4BsumBase + buffer * kQ4Tokens * 32u + 32u * token;
-            f16x8 sums;
-            if constexpr (QT == QT_Q2_K) sums = q2k_bsum_operand(read16(at + 16u * h));  // a minimum per 16 values: the sums as they are
-            else sums = q4k_bsum_operand(read16(at), read16(at + 16u), h);
+            const f16x8 sums = bsum_operand(read16(at + 16u * h));       // eight of the sixteen sums of 16 values
             v16f zero16;
             v32f zero32;
 #pragma unroll
