@@ -676,31 +676,31 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
     constexpr unsigned kItemRows = FUSED_UP ? 128u : 256u;
     constexpr unsigned kWide = 4u, kNarrow = 3u;                // costs of a row tile
     const unsigned row_tiles = (a.out_rows + kItemRows - 1u) / kItemRows;
+    // (in 32 bits: the launch wrapper bounds the row tiles of all token tiles, and a division of 64 bits is a hundred instructions)
     const unsigned full_tiles = uniform32(lds_read_u32(kTileStartBase + 4u * buckets));
     const unsigned members[2] = {uniform32(lds_read_u32(kClassCountBase)), uniform32(lds_read_u32(kClassCountBase + 4u))};
-    const unsigned long long wide = (unsigned long long)(full_tiles + members[0]) * row_tiles,
-                             narrow = (unsigned long long)members[1] * row_tiles;
-    const unsigned long long cost = kWide * wide + kNarrow * narrow;
+    const unsigned wide = (full_tiles + members[0]) * row_tiles, narrow = members[1] * row_tiles, cost = kWide * wide + kNarrow * narrow;
     const unsigned who = gridDim.x % 8u ? blockIdx.x : (blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
-    auto share_of = [&](unsigned long long all, unsigned workgroup) {       // what the workgroups before have
-        return all / gridDim.x * workgroup + all % gridDim.x * workgroup / gridDim.x;
-    };
-    const bool level = cost / gridDim.x >= kWide * (wide / gridDim.x + 1u);
+    const unsigned cost_share = cost / gridDim.x, cost_rest = cost - cost_share * gridDim.x;
+    const unsigned wide_share = wide / gridDim.x, wide_rest = wide - wide_share * gridDim.x;
+    // what the workgroups before have
+    auto cost_before = [&](unsigned workgroup) { return cost_share * workgroup + cost_rest * workgroup / gridDim.x; };
+    auto wide_before = [&](unsigned workgroup) { return wide_share * workgroup + wide_rest * workgroup / gridDim.x; };
+    const bool level = cost_share >= kWide * (wide_share + 1u);
     auto narrow_place = [&](unsigned workgroup) {
-        return wide + (share_of(cost, workgroup) - kWide * share_of(wide, workgroup) + kNarrow - 1u) / kNarrow;
+        return wide + (cost_before(workgroup) - kWide * wide_before(workgroup) + kNarrow - 1u) / kNarrow;
     };
     auto place_of = [&](unsigned workgroup) {                   // the first row tile of its piece, of its long ones
-        const unsigned long long at = share_of(cost, workgroup);
-        return level ? share_of(wide, workgroup)
+        const unsigned at = cost_before(workgroup);
+        return level ? wide_before(workgroup)
              : at <= kWide * wide ? (at + kWide - 1u) / kWide : wide + (at - kWide * wide + kNarrow - 1u) / kNarrow;
     };
     auto uniform64 = [&](unsigned long long v) {
         return (unsigned long long)uniform32((unsigned)v) | ((unsigned long long)uniform32((unsigned)(v >> 32)) << 32);
     };
-    unsigned long long at = uniform64(place_of(who));
-    unsigned long long end = uniform64(place_of(who + 1u));
-    unsigned long long narrow_at = level ? uniform64(narrow_place(who)) : 0ull;
-    const unsigned long long narrow_end = level ? uniform64(narrow_place(who + 1u)) : 0ull;
+    unsigned at = uniform32(place_of(who)), end = uniform32(place_of(who + 1u));
+    unsigned narrow_at = level ? uniform32(narrow_place(who)) : 0u;
+    const unsigned narrow_end = level ? uniform32(narrow_place(who + 1u)) : 0u;
     if (at >= end && narrow_at >= narrow_end) return;
     mfma_tables_fill();
     __syncthreads();
@@ -711,11 +711,10 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
             at = narrow_at;
             end = narrow_at = narrow_end;
         }
-        const unsigned tile = uniform32((unsigned)(at / row_tiles));
+        const unsigned tile = uniform32(at / row_tiles);
         MfmaRun run;
-        run.row_tile = uniform32((unsigned)(at % row_tiles));
-        const unsigned long long left = end - at;
-        run.row_end = left < row_tiles - run.row_tile ? run.row_tile + (unsigned)left : row_tiles;
+        run.row_tile = at - tile * row_tiles;
+        run.row_end = end - at < row_tiles - run.row_tile ? run.row_tile + (end - at) : row_tiles;
         if (ragged && run.row_end == row_tiles && run.row_end - run.row_tile > 1u) --run.row_end;
         at += run.row_end - run.row_tile;
         // which bucket the tile is of, and which of its tiles
@@ -766,6 +765,9 @@ static int launch_mfma_variant(const MfmaArgs &a, hipStream_t stream)
 template <bool FUSED_UP>
 static int launch_mfma(const MfmaArgs &a, hipStream_t stream)
 {
+    // (the kernel counts row tiles in 32 bits; the outputs or the weights of so many are more than the card's memory)
+    const uint64_t token_tiles = a.pr.pairs / kTileTokens + (a.pr.expert_ids ? 256u : 1u);
+    if (token_tiles * ((uint64_t)a.out_rows / (FUSED_UP ? 128u : 256u) + 1u) >= 1ull << 30) return ST_BOUNDS;
     return a.image ? launch_mfma_variant<FUSED_UP, true>(a, stream)
                    : launch_mfma_variant<FUSED_UP, false>(a, stream);
 }
