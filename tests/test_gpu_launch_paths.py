@@ -316,6 +316,30 @@ def test_quantization_forms_the_shared_experts_products(gpu, oracle, rows, share
     assert torch.equal(bytes_of[1], K.q8k_quantize(products, status)) and int(status.item()) == 0
 
 
+@pytest.mark.parametrize("limit", [7.1, 40.1, 1.0e9])
+def test_clamped_product_over_the_range_of_its_exponential(gpu, oracle, limit):
+    # limits that binary32 does not hold, or arguments past 16, take the path in double; its exponential is within 0.6 units in
+    # the last place of binary64, so that bfloat16 results are those of a correctly rounded one
+    from yvex_amd import kernels as K
+    g = oracle.Generator(42, f"swiglu.{limit}")
+    gate = np.concatenate([np.asarray(g.normal(4096, spread), dtype=np.float32).reshape(-1) for spread in (1.0, 8.0, 40.0, 250.0)] +
+                          [np.array([0.0, -0.0, 1e-30, -1e-30, -16.0, 16.0, -87.4, -708.5, -744.0, -746.0, -799.0, -801.0, -3e38, 3e38],
+                                    dtype=np.float32)])
+    up = np.asarray(g.normal(gate.size, 4.0), dtype=np.float32).reshape(-1)
+    status = K.new_status(gpu)
+    out = torch.empty(gate.size, dtype=torch.float32, device=gpu)
+    held = dev(gate, gpu), dev(up, gpu)
+    call("yvex_hip_moe_swiglu_rows", ptr(held[0]), ptr(held[1]), u64(gate.size), C.c_double(limit), ptr(out), ptr(status))
+    gv = np.minimum(gate.astype(np.float64), limit)
+    t = np.exp(-np.abs(gv))
+    product = np.where(gv >= 0.0, gv / (1.0 + t), gv * t / (1.0 + t)) * np.clip(up.astype(np.float64), -limit, limit)
+    with np.errstate(over="ignore"):
+        want = torch.from_numpy(product.astype(np.float32)).to(torch.bfloat16).float()
+    finite = torch.isfinite(want)
+    assert same_bits(out.cpu()[finite], want[finite])
+    assert int(status.item()) == (0 if bool(finite.all()) else 1)
+
+
 @pytest.mark.parametrize("rows,topk,width", [(1, 1, 4), (3, 6, 1028), (9, 8, 7168)])
 def test_combine_goes_straight_into_the_egress(gpu, oracle, rows, topk, width):
     from yvex_amd import kernels as K
