@@ -621,8 +621,9 @@ __global__ __launch_bounds__(kRowThreads) void mfma_iq2_kernel(MfmaArgs a)
 
     // The buckets' populations are requested together (one round trip to memory instead of one per
     // bucket), and the tables built only where there is an item.
-    unsigned long long population_here = 0ull;
-    if (tid < 256u && tid < buckets) population_here = fixed ? pr.pairs : pr.bucket_populations[tid];
+    // (a slot is read whether a bucket uses it or not: the number of buckets is on its way meanwhile)
+    unsigned long long population_here = fixed ? pr.pairs : tid < 256u && tid < pr.experts ? pr.bucket_populations[tid] : 0ull;
+    if (tid >= 256u || tid >= buckets) population_here = 0ull;
     // Full 64-pair tiles come first in the list of tiles, then the partial last tiles of more than 32
     // pairs, then those of fewer. Bucket b's first full tile is
     // the number of full tiles before it (a scan over the 256 bucket slots); its place in its

@@ -224,11 +224,11 @@ __global__ __launch_bounds__((Map16<QT, S>::kThreads)) void rows16_kernel(Rows16
     const unsigned tid = threadIdx.x, lane = tid & 63u, wave = uniform(tid >> 6);
     const Lane16 l{lane & 15u, lane >> 4};
     const bool fixed = pr.expert_ids == nullptr;
+    // ---- the first tile of every bucket (a scan over the 256 bucket slots; a slot is read whether a bucket uses it or not:
+    // the number of buckets is on its way meanwhile) ----
+    const unsigned long long held = fixed ? pr.pairs : tid < 256u && tid < pr.experts ? pr.bucket_populations[tid] : 0ull;
     const unsigned buckets = fixed ? 1u : uniform((unsigned)pr.counts[0]);
-
-    // ---- the first tile of every bucket (a scan over the 256 bucket slots) ----
-    unsigned long long population_here = 0ull;
-    if (tid < 256u && tid < buckets) population_here = fixed ? pr.pairs : pr.bucket_populations[tid];
+    const unsigned long long population_here = tid < 256u && tid < buckets ? held : 0ull;
     {
         const unsigned long long served = a.behind ? population_here % a.behind : population_here;
         const unsigned limit = a.behind ? few_pair_limit(a.tokens, population_here, M::kMisc + 16u) : 0u;
