@@ -316,6 +316,46 @@ def test_quantization_forms_the_shared_experts_products(gpu, oracle, rows, share
     assert torch.equal(bytes_of[1], K.q8k_quantize(products, status)) and int(status.item()) == 0
 
 
+@pytest.mark.parametrize("rows,width,gap", [(1, 256, 0), (3, 256, 1), (5, 768, 0), (7, 2304, 3), (9, 4096, 4)])
+def test_four_blocks_a_wavefront_quantize_as_one_does(gpu, oracle, rows, width, gap):
+    # blocks whose largest magnitude has both signs (the first decides), lies at an end, is zero, or so small that its inverse
+    # is not finite (there only the kernel of one block a wavefront says what is right)
+    from yvex_amd import kernels as K
+    g = oracle.Generator(42, f"four.{rows}.{width}")
+    x = np.asarray(g.normal(rows * width), dtype=np.float32).reshape(-1, 256)
+    places = np.random.default_rng(rows).integers(0, 256, (x.shape[0], 2))
+    for b in range(x.shape[0]):
+        kind = b % 6
+        if kind == 0:
+            x[b] = -0.0 if b % 4 else 0.0
+        elif kind in (1, 2):
+            x[b, places[b, 0]], x[b, places[b, 1]] = 9.0, -9.0
+        elif kind == 3:
+            x[b] = np.where(np.arange(256) % 2 == b % 2, 1.0, -1.0)
+        elif kind == 4:
+            x[b, 255] = -11.0
+    wide = torch.zeros((rows, width + gap), dtype=torch.float32, device=gpu)
+    wide[:, :width] = dev(x.reshape(rows, width), gpu)
+    status = K.new_status(gpu)
+    got = torch.zeros(rows * (width // 256) * 292, dtype=torch.uint8, device=gpu)
+    call("yvex_hip_q8k_quantize", ptr(wide), u64(rows), u64(width), u64(width + gap), ptr(got), ptr(status))
+    assert np.array_equal(got.cpu().numpy(), oracle.q8k_quantize(x.reshape(rows, width))) and int(status.item()) == 0
+    # tiny magnitudes and what is not finite, against the launch that takes a block a wavefront
+    tiny = x.copy()
+    tiny[::2] *= np.float32(1e-38)
+    tiny = dev(tiny.reshape(rows, width), gpu)
+    selected = torch.zeros((rows, 1), dtype=torch.int64, device=gpu)
+    mine, encoded = K.Worklist(rows, 2, gpu), torch.empty_like(got)
+    call("yvex_hip_moe_prepare_routed", ptr(selected), u64(rows), u64(2), u64(1), *K._wl_ptrs(mine), ptr(tiny), u64(width),
+         u64(width), ptr(encoded), ptr(status))
+    assert torch.equal(K.q8k_quantize(tiny, status), encoded) and int(status.item()) == 0
+    for value in (float("inf"), float("nan")):
+        broken, flag = tiny.clone(), K.new_status(gpu)
+        broken[rows - 1, width - 1] = value
+        K.q8k_quantize(broken, flag)
+        assert int(flag.item()) == 1
+
+
 @pytest.mark.parametrize("limit", [7.1, 40.1, 1.0e9])
 def test_clamped_product_over_the_range_of_its_exponential(gpu, oracle, limit):
     # limits that binary32 does not hold, or arguments past 16, take the path in double; its exponential is within 0.6 units in

@@ -1,4 +1,4 @@
-// Q8_K activation quantizer for gfx950: one 64-lane wavefront per 256-value block (q8k.hpp).
+// Q8_K activation quantizer for gfx950: a 64-lane wavefront four blocks of 256 values, or one where other work rides along (q8k.hpp).
 #include "common.hpp"
 #include "q8k.hpp"
 #include "q8_0_rows.hpp"
@@ -12,30 +12,50 @@ __global__ __launch_bounds__(256) void q8k_quantize_kernel(
     unsigned long long input_stride, unsigned char *__restrict__ encoded, int *status)
 {
     const unsigned lane = threadIdx.x & 63u;
-    const unsigned long long task = (unsigned long long)blockIdx.x * 4ull + (threadIdx.x >> 6);
-    if (task >= rows * blocks) return;
-    const unsigned long long row = task / blocks, block = task % blocks;
-    q8k_quantize_block(values + row * input_stride + block * 256ull + lane * 4u, encoded + task * kQ8KBytes,
-                       lane, status);
+    const unsigned long long tasks = rows * blocks;
+    const unsigned long long task = ((unsigned long long)blockIdx.x * 4ull + (threadIdx.x >> 6)) * 4ull + (lane >> 4);
+    const unsigned long long held = task < tasks ? task : tasks - 1ull;
+    // (rows end to end, as the layers' are, need no row number)
+    const float *x = values + held * 256ull;
+    if (input_stride != blocks * 256ull) {
+        const unsigned long long row = held / blocks;
+        x = values + row * input_stride + (held - row * blocks) * 256ull;
+    }
+    float v[4][4];
+#pragma unroll
+    for (unsigned k = 0; k < 4u; ++k) __builtin_memcpy(v[k], x + 4u * (lane & 15u) + 64u * k, 16);
+    q8k_quantize_four(v, encoded + held * kQ8KBytes, lane, task < tasks, status);
 }
 
 // The same for a layer's intermediate rows where a shared expert's gate and up sums come from dense
 // projections: behind the routed pairs' rows the shared rows' values are formed on the way in, the
 // clamped SwiGLU product rounded to bfloat16 (what yvex_hip_moe_swiglu_rows stores). A launch and a
 // round trip of the rows through memory less.
+// Four routed blocks a wavefront as above, behind the workgroups of the shared ones, a block a wavefront: one product in
+// five hundred takes the path in double, and a wavefront of four blocks meets it twice (96 rows 5.5 -> 6.9 us so).
 __global__ __launch_bounds__(256) void q8k_quantize_swiglu_kernel(
     const float *__restrict__ values, unsigned long long rows, unsigned long long blocks,
     unsigned char *__restrict__ encoded, const float *__restrict__ gate, const float *__restrict__ up,
     unsigned long long shared_rows, double limit, unsigned char *__restrict__ shared_encoded, int *status)
 {
     const unsigned lane = threadIdx.x & 63u;
-    const unsigned long long task = (unsigned long long)blockIdx.x * 4ull + (threadIdx.x >> 6);
-    if (task < rows * blocks) {
-        q8k_quantize_block(values + task * 256ull + lane * 4u, encoded + task * kQ8KBytes, lane, status);
+    const unsigned long long shared_tasks = shared_rows * blocks, shared_groups = (shared_tasks + 3ull) / 4ull;
+    if (blockIdx.x >= shared_groups) {
+        const unsigned long long tasks = rows * blocks;
+        const unsigned long long task = ((blockIdx.x - shared_groups) * 4ull + (threadIdx.x >> 6)) * 4ull + (lane >> 4);
+        const unsigned long long held = task < tasks ? task : tasks - 1ull;
+        const float4 *const x = reinterpret_cast<const float4 *>(values + held * 256ull) + (lane & 15u);
+        float v[4][4];
+#pragma unroll
+        for (unsigned k = 0; k < 4u; ++k) {
+            const float4 x4 = x[16u * k];
+            v[k][0] = x4.x, v[k][1] = x4.y, v[k][2] = x4.z, v[k][3] = x4.w;
+        }
+        q8k_quantize_four(v, encoded + held * kQ8KBytes, lane, task < tasks, status);
         return;
     }
-    const unsigned long long shared_task = task - rows * blocks;
-    if (shared_task >= shared_rows * blocks) return;
+    const unsigned long long shared_task = blockIdx.x * 4ull + (threadIdx.x >> 6);
+    if (shared_task >= shared_tasks) return;
     const float4 g = *reinterpret_cast<const float4 *>(gate + shared_task * 256ull + lane * 4u);
     const float4 u = *reinterpret_cast<const float4 *>(up + shared_task * 256ull + lane * 4u);
     const float v[4] = {swiglu_bf16_fast(g.x, u.x, 1.0f, limit, (float)limit),
@@ -130,8 +150,8 @@ extern "C" int yvex_hip_q8k_quantize(const float *values, uint64_t rows, uint64_
         return ST_INVALID_ARG;
     const uint64_t blocks = width / 256u;
     if (rows > UINT64_MAX / blocks) return ST_BOUNDS;
-    const uint64_t tasks = rows * blocks, grid = (tasks + 3u) / 4u;
-    if (grid > 0x7fffffffull) return ST_BOUNDS;
+    const uint64_t tasks = rows * blocks, grid = (tasks + 15u) / 16u;
+    if (grid > 0x1fffffffull) return ST_BOUNDS;
     q8k_quantize_kernel<<<(unsigned)grid, 256, 0, as_stream(stream)>>>(
         values, rows, blocks, input_stride, encoded, status);
     return check_launch("q8k_quantize");
@@ -148,8 +168,8 @@ extern "C" int yvex_hip_q8k_quantize_swiglu(const float *values, uint64_t rows, 
         return ST_INVALID_ARG;
     const uint64_t blocks = width / 256u;
     if (rows > 0xffffffffull || shared_rows > 0xffffffffull) return ST_BOUNDS;
-    const uint64_t grid = ((rows + shared_rows) * blocks + 3u) / 4u;
-    if (grid > 0x7fffffffull) return ST_BOUNDS;
+    const uint64_t grid = (rows * blocks + 15u) / 16u + (shared_rows * blocks + 3u) / 4u;
+    if (grid > 0x1fffffffull) return ST_BOUNDS;
     q8k_quantize_swiglu_kernel<<<(unsigned)grid, 256, 0, as_stream(stream)>>>(
         values, rows, blocks, encoded, gate, up, shared_rows, limit, shared_encoded, status);
     return check_launch("q8k_quantize_swiglu");
