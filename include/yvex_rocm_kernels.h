@@ -329,6 +329,25 @@ unsigned int yvex_hip_moe_down_rows_launches(const yvex_hip_expert_weights *weig
                                              const uint64_t *expert_ids, uint64_t pairs, uint64_t experts,
                                              float *pair_outputs);
 
+/* Both again with a shared expert's rows in the same launch: what yvex_hip_moe_up_rows / _down_rows for the routed experts and
+ * for the shared one (expert_ids == NULL) write, bit for bit. yvex_hip_moe_rows_join says whether the two can go together
+ * (the same format, Q4_K or Q2_K, the same sizes, and rows enough for the 64-pair kernel); where not, the functions
+ * return the code of an unsupported call and launch nothing. Launches: those of the routed experts alone. */
+int yvex_hip_moe_rows_join(const yvex_hip_expert_weights *weights, const uint64_t *expert_ids, uint64_t pairs, uint64_t topk,
+                           uint64_t experts, const yvex_hip_expert_weights *shared, uint64_t shared_rows, int down);
+int yvex_hip_moe_up_rows_joined(const yvex_hip_expert_weights *weights, const void *act_q8k, const float *route_weights,
+                                const uint64_t *order, const uint64_t *expert_ids, const uint64_t *bucket_offsets,
+                                const uint64_t *bucket_populations, const uint64_t *counts, uint64_t pairs, uint64_t topk,
+                                uint64_t experts, double limit, float *intermediate,
+                                const yvex_hip_expert_weights *shared, uint64_t shared_rows, float *shared_intermediate,
+                                int *status, yvex_hip_stream stream);
+int yvex_hip_moe_down_rows_joined(const yvex_hip_expert_weights *weights, const void *intermediate_q8k, const uint64_t *order,
+                                  const uint64_t *expert_ids, const uint64_t *bucket_offsets,
+                                  const uint64_t *bucket_populations, const uint64_t *counts, uint64_t pairs,
+                                  uint64_t experts, float *pair_outputs, const yvex_hip_expert_weights *shared,
+                                  const void *shared_intermediate_q8k, uint64_t shared_rows, float *shared_outputs,
+                                  int *status, yvex_hip_stream stream);
+
 /* The SwiGLU stage of an expert whose gate and up projections ran as dense projections (a shared
  * expert of a format the expert kernels do not take): out[i] = bf16(silu(min(gate[i], limit)) *
  * clamp(up[i], -limit, limit)), the value yvex_moe_grouped_up_rows forms with a route weight of

@@ -429,6 +429,43 @@ def test_sweeps_agree_with_the_matrix_core_kernels(gpu, oracle, qtype, hidden, i
     assert same_bits(out[0], out[1]) and int(status.item()) == 0
 
 
+# a shared tile of one row, a whole one, one and a row; few routed pairs and several tiles a bucket; with the few-pair
+# kernels beside (1100 rows of two superblocks, which a matrix alone has too many of for them)
+@pytest.mark.parametrize("down,hidden,intermediate,rows,topk", [
+    ("Q4_K", 256, 256, 1, 2), ("Q4_K", 256, 256, 64, 1), ("Q2_K", 256, 256, 65, 3), ("Q2_K", 256, 256, 200, 3),
+    ("Q4_K", 1024, 512, 1100, 2)])
+def test_shared_rows_join_the_routed_launch(gpu, oracle, down, hidden, intermediate, rows, topk):
+    """One launch writes what the two it replaces write, bit for bit; an unsuitable pair is refused."""
+    from yvex_amd import kernels as K
+    experts, g = 7, oracle.Generator(42, f"join.{down}.{hidden}.{intermediate}.{rows}")
+    kinds = (oracle.Q4_K, oracle.Q4_K, getattr(oracle, down))
+    shapes = ((intermediate, hidden), (intermediate, hidden), (hidden, intermediate))
+    routed, shared = (K.expert_weights(*(dev(g.weights(qt, n * r, w), gpu) for qt, (r, w) in zip(kinds, shapes)), kinds, hidden,
+                                       intermediate) for n in (experts, 1))
+    status = K.new_status(gpu)
+    logits = dev(g.normal(rows * experts).reshape(rows, experts) - 0.5 * np.arange(experts), gpu)
+    selected, route = K.moe_route_rows(logits.float(), None, topk, K.SIGMOID, True, 1.0, status)
+    wl, pairs = K.worklist_build(selected, experts, status), rows * topk
+    act = K.q8k_quantize(dev(g.normal(rows * hidden).reshape(rows, hidden), gpu), status)
+    assert all(K.moe_rows_join(routed, wl, pairs, topk, experts, shared, rows, way) for way in (0, 1))
+    mid, mid_shared = ([torch.zeros((n, intermediate), device=gpu) for _ in range(2)] for n in (pairs, rows))
+    K.moe_up_rows(routed, act, route, wl, pairs, topk, experts, 10.0, mid[0], status)
+    K.moe_up_rows(shared, act, None, None, rows, 1, 1, 10.0, mid_shared[0], status)
+    K.moe_up_rows_joined(routed, act, route, wl, pairs, topk, experts, 10.0, mid[1], shared, rows, mid_shared[1], status)
+    assert same_bits(mid[0], mid[1]) and same_bits(mid_shared[0], mid_shared[1]) and bool(mid_shared[0].any())
+    mid_q8, shared_q8 = K.q8k_quantize(mid[0], status), K.q8k_quantize(mid_shared[0], status)
+    out, out_shared = ([torch.zeros((n, hidden), device=gpu) for _ in range(2)] for n in (pairs, rows))
+    K.moe_down_rows(routed, mid_q8, wl, pairs, experts, out[0], status)
+    K.moe_down_rows(shared, shared_q8, None, rows, 1, out_shared[0], status)
+    K.moe_down_rows_joined(routed, mid_q8, wl, pairs, experts, out[1], shared, shared_q8, rows, out_shared[1], status)
+    assert same_bits(out[0], out[1]) and same_bits(out_shared[0], out_shared[1]) and bool(out_shared[0].any())
+    assert int(status.item()) == 0
+    other = K.expert_weights(*shared._keep, (oracle.Q4_K, oracle.Q4_K, oracle.IQ2_XXS), hidden, intermediate)
+    assert not K.moe_rows_join(routed, wl, pairs, topk, experts, other, rows, 1)
+    with pytest.raises(Exception):
+        K.moe_down_rows_joined(routed, mid_q8, wl, pairs, experts, out[1], other, shared_q8, rows, out_shared[1], status)
+
+
 # a pair, a remainder of the largest size the few-pair kernels take at the width and one more, 64-pair
 # tiles with and without such remainders; two, three and 32 superblocks a row, ragged row units
 @pytest.mark.parametrize("up,down,hidden,intermediate,tokens,image", [

@@ -206,9 +206,11 @@ __device__ __forceinline__ unsigned few_pair_limit(unsigned few, unsigned long l
 
 // Row-batch expert kernels on the int8 matrix cores (rows_q4k.hip): Q4_K weights, fused gate/up
 // or a plain projection; Q2_K weights, a plain projection (the down experts). A bucket's last tile is left to
-// the kernels below where few_pair_limit says so.
+// the kernels below where few_pair_limit says so. `beside`, or null: a matrix alone of the same formats and sizes, in the
+// same launch.
 int launch_q4k_rows_grouped(const GroupedProblem &problem, unsigned qtype, bool fused, uint64_t width,
-                            uint64_t out_rows, unsigned few, double limit, int *status, hipStream_t stream);
+                            uint64_t out_rows, unsigned few, const GroupedProblem *beside, double limit, int *status,
+                            hipStream_t stream);
 
 // The same problems where few pairs meet (rows16.hip): IQ2_XXS (canonical bytes, or the sweep image) and
 // Q4_K rows, fused gate/up or plain; Q2_K rows, plain. The first: pairs of a full tile, 0 for a problem

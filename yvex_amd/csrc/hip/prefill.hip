@@ -797,14 +797,14 @@ static RowsPlan plan_rows(const GroupedProblem &pr, unsigned qtype, bool fused, 
 }
 
 template <bool FUSED_UP>
-static int launch_rows(MfmaArgs &a, unsigned qtype, hipStream_t stream)
+static int launch_rows(MfmaArgs &a, unsigned qtype, hipStream_t stream, const GroupedProblem *beside = nullptr)
 {
     const RowsPlan plan = plan_rows(a.pr, qtype, FUSED_UP, a.image, a.width, a.out_rows);
     a.few = plan.few;
     if (plan.many) {
         const int rc = qtype == QT_IQ2_XXS
             ? launch_mfma<FUSED_UP>(a, stream)
-            : launch_q4k_rows_grouped(a.pr, qtype, FUSED_UP, a.width, a.out_rows, plan.few, a.limit, a.status, stream);
+            : launch_q4k_rows_grouped(a.pr, qtype, FUSED_UP, a.width, a.out_rows, plan.few, beside, a.limit, a.status, stream);
         if (rc || !plan.few) return rc;
     }
     return launch_rows16_grouped(a.pr, qtype, a.image != 0, FUSED_UP, a.width, a.out_rows, a.pr.expert_ids ? kTileTokens : 0u,
@@ -869,15 +869,26 @@ extern "C" unsigned yvex_hip_moe_down_rows_launches(const yvex_hip_expert_weight
     return (plan.few ? 1u : 0u) + (plan.many ? 1u : 0u);
 }
 
-extern "C" int yvex_hip_moe_up_rows(const yvex_hip_expert_weights *w, const void *act_q8k,
-                                    const float *route_weights, const uint64_t *order,
-                                    const uint64_t *expert_ids, const uint64_t *bucket_offsets,
-                                    const uint64_t *bucket_populations, const uint64_t *counts,
-                                    uint64_t pairs, uint64_t topk, uint64_t experts, double limit,
-                                    float *intermediate, int *status, yvex_hip_stream stream)
+// A shared expert's rows go along with the routed ones' where both are the 64-pair Q4_K and Q2_K kernel's, in the same shape.
+static bool rows_join(const GroupedProblem &routed, const GroupedProblem &alone, const yvex_hip_expert_weights *w,
+                      const yvex_hip_expert_weights *shared, bool fused)
+{
+    const unsigned qtype = fused ? w->gate_qtype : w->down_qtype;
+    if (qtype == QT_IQ2_XXS || qtype != (fused ? shared->gate_qtype : shared->down_qtype) || w->hidden != shared->hidden ||
+        w->intermediate != shared->intermediate)
+        return false;
+    const uint64_t width = fused ? w->hidden : w->intermediate, out_rows = fused ? w->intermediate : w->hidden;
+    const RowsPlan plan = plan_rows(routed, qtype, fused, 0, width, out_rows);
+    const RowsPlan other = plan_rows(alone, qtype, fused, 0, width, out_rows);
+    return plan.many && other.many && !other.few && (uint64_t)routed.pairs + alone.pairs <= 1ull << 21;      // (the grid's second side)
+}
+
+static int prepare_up_rows(MfmaArgs &a, const yvex_hip_expert_weights *w, const void *act_q8k, const float *route_weights,
+                           const WorklistView &wl, uint64_t pairs, uint64_t topk, uint64_t experts, double limit,
+                           float *intermediate, int *status)
 {
     if (!w || !w->gate || !w->up || !act_q8k || !intermediate || !status || !pairs || !topk ||
-        !experts || !(limit > 0.0) || (expert_ids && (!bucket_offsets || !bucket_populations || !counts)))
+        !experts || !(limit > 0.0) || (wl.expert_ids && (!wl.bucket_offsets || !wl.bucket_populations || !wl.counts)))
         return ST_INVALID_ARG;
     if (w->gate_qtype != w->up_qtype || (w->gate_qtype != QT_IQ2_XXS && w->gate_qtype != QT_Q4_K))
         return ST_UNSUPPORTED;
@@ -888,15 +899,49 @@ extern "C" int yvex_hip_moe_up_rows(const yvex_hip_expert_weights *w, const void
     if (w->up_row_bytes != w->gate_row_bytes) return ST_BOUNDS;
     if (w->gate_up_image && (((uintptr_t)w->up & 3u) || (w->up_expert_bytes & 3u))) return ST_INVALID_ARG;
     if (pairs > 0xffffffffull || w->intermediate > 0xffffffffull || w->intermediate % 4u) return ST_BOUNDS;
-    MfmaArgs a{};
-    const WorklistView wl{order, expert_ids, bucket_offsets, bucket_populations, nullptr, counts};
     fill_up_problem(a.pr, w, act_q8k, 1, route_weights, wl, pairs, topk, experts, intermediate);
     a.width = (unsigned)w->hidden;
     a.out_rows = (unsigned)w->intermediate;
     a.limit = limit;
     a.status = status;
     a.image = w->gate_up_image != 0;
-    return launch_rows<true>(a, w->gate_qtype, as_stream(stream));
+    return ST_OK;
+}
+
+static int prepare_down_rows(MfmaArgs &a, const yvex_hip_expert_weights *w, const void *intermediate_q8k, const WorklistView &wl,
+                             uint64_t pairs, uint64_t experts, float *pair_outputs, int *status)
+{
+    if (!w || !w->down || !intermediate_q8k || !pair_outputs || !status || !pairs || !experts ||
+        (wl.expert_ids && (!wl.bucket_offsets || !wl.bucket_populations || !wl.counts)))
+        return ST_INVALID_ARG;
+    if (w->down_qtype != QT_IQ2_XXS && w->down_qtype != QT_Q4_K && w->down_qtype != QT_Q2_K) return ST_UNSUPPORTED;
+    int rc = w->down_image
+        ? check_image_matrix(w->down_qtype, w->intermediate, w->down_row_bytes, w->down, w->down_expert_bytes)
+        : check_matrix(w->down_qtype, w->intermediate, w->down_row_bytes);
+    if (rc) return rc;
+    if (pairs > 0xffffffffull || w->hidden > 0xffffffffull || w->hidden % 4u) return ST_BOUNDS;
+    fill_down_problem(a.pr, w, intermediate_q8k, 1, wl, pairs, experts, pair_outputs);
+    a.width = (unsigned)w->intermediate;
+    a.out_rows = (unsigned)w->hidden;
+    a.limit = 1.0;
+    a.status = status;
+    a.image = w->down_image != 0;
+    return ST_OK;
+}
+
+static const WorklistView kNoWorklist{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+
+extern "C" int yvex_hip_moe_up_rows(const yvex_hip_expert_weights *w, const void *act_q8k,
+                                    const float *route_weights, const uint64_t *order,
+                                    const uint64_t *expert_ids, const uint64_t *bucket_offsets,
+                                    const uint64_t *bucket_populations, const uint64_t *counts,
+                                    uint64_t pairs, uint64_t topk, uint64_t experts, double limit,
+                                    float *intermediate, int *status, yvex_hip_stream stream)
+{
+    MfmaArgs a{};
+    const WorklistView wl{order, expert_ids, bucket_offsets, bucket_populations, nullptr, counts};
+    const int rc = prepare_up_rows(a, w, act_q8k, route_weights, wl, pairs, topk, experts, limit, intermediate, status);
+    return rc ? rc : launch_rows<true>(a, w->gate_qtype, as_stream(stream));
 }
 
 extern "C" int yvex_hip_moe_down_rows(const yvex_hip_expert_weights *w, const void *intermediate_q8k,
@@ -906,22 +951,54 @@ extern "C" int yvex_hip_moe_down_rows(const yvex_hip_expert_weights *w, const vo
                                       uint64_t pairs, uint64_t experts, float *pair_outputs,
                                       int *status, yvex_hip_stream stream)
 {
-    if (!w || !w->down || !intermediate_q8k || !pair_outputs || !status || !pairs || !experts ||
-        (expert_ids && (!bucket_offsets || !bucket_populations || !counts)))
-        return ST_INVALID_ARG;
-    if (w->down_qtype != QT_IQ2_XXS && w->down_qtype != QT_Q4_K && w->down_qtype != QT_Q2_K) return ST_UNSUPPORTED;
-    int rc = w->down_image
-        ? check_image_matrix(w->down_qtype, w->intermediate, w->down_row_bytes, w->down, w->down_expert_bytes)
-        : check_matrix(w->down_qtype, w->intermediate, w->down_row_bytes);
-    if (rc) return rc;
-    if (pairs > 0xffffffffull || w->hidden > 0xffffffffull || w->hidden % 4u) return ST_BOUNDS;
     MfmaArgs a{};
     const WorklistView wl{order, expert_ids, bucket_offsets, bucket_populations, nullptr, counts};
-    fill_down_problem(a.pr, w, intermediate_q8k, 1, wl, pairs, experts, pair_outputs);
-    a.width = (unsigned)w->intermediate;
-    a.out_rows = (unsigned)w->hidden;
-    a.limit = 1.0;
-    a.status = status;
-    a.image = w->down_image != 0;
-    return launch_rows<false>(a, w->down_qtype, as_stream(stream));
+    const int rc = prepare_down_rows(a, w, intermediate_q8k, wl, pairs, experts, pair_outputs, status);
+    return rc ? rc : launch_rows<false>(a, w->down_qtype, as_stream(stream));
+}
+
+extern "C" int yvex_hip_moe_rows_join(const yvex_hip_expert_weights *w, const uint64_t *expert_ids, uint64_t pairs, uint64_t topk,
+                                      uint64_t experts, const yvex_hip_expert_weights *shared, uint64_t shared_rows, int down)
+{
+    if (!w || !shared || !expert_ids || pairs > 0xffffffffull || shared_rows > 0xffffffffull || !shared_rows) return 0;
+    GroupedProblem routed{}, alone{};
+    const WorklistView wl{nullptr, expert_ids, nullptr, nullptr, nullptr, nullptr};
+    if (down) {
+        fill_down_problem(routed, w, nullptr, 1, wl, pairs, experts, nullptr);
+        fill_down_problem(alone, shared, nullptr, 1, kNoWorklist, shared_rows, 1u, nullptr);
+    } else {
+        fill_up_problem(routed, w, nullptr, 1, nullptr, wl, pairs, topk, experts, nullptr);
+        fill_up_problem(alone, shared, nullptr, 1, nullptr, kNoWorklist, shared_rows, 1u, 1u, nullptr);
+    }
+    return rows_join(routed, alone, w, shared, !down);
+}
+
+extern "C" int yvex_hip_moe_up_rows_joined(const yvex_hip_expert_weights *w, const void *act_q8k, const float *route_weights,
+                                           const uint64_t *order, const uint64_t *expert_ids, const uint64_t *bucket_offsets,
+                                           const uint64_t *bucket_populations, const uint64_t *counts, uint64_t pairs,
+                                           uint64_t topk, uint64_t experts, double limit, float *intermediate,
+                                           const yvex_hip_expert_weights *shared, uint64_t shared_rows,
+                                           float *shared_intermediate, int *status, yvex_hip_stream stream)
+{
+    MfmaArgs a{}, alone{};
+    const WorklistView wl{order, expert_ids, bucket_offsets, bucket_populations, nullptr, counts};
+    int rc = prepare_up_rows(a, w, act_q8k, route_weights, wl, pairs, topk, experts, limit, intermediate, status);
+    if (!rc) rc = prepare_up_rows(alone, shared, act_q8k, nullptr, kNoWorklist, shared_rows, 1u, 1u, limit, shared_intermediate, status);
+    if (!rc && (!expert_ids || !rows_join(a.pr, alone.pr, w, shared, true))) rc = ST_UNSUPPORTED;
+    return rc ? rc : launch_rows<true>(a, w->gate_qtype, as_stream(stream), &alone.pr);
+}
+
+extern "C" int yvex_hip_moe_down_rows_joined(const yvex_hip_expert_weights *w, const void *intermediate_q8k, const uint64_t *order,
+                                             const uint64_t *expert_ids, const uint64_t *bucket_offsets,
+                                             const uint64_t *bucket_populations, const uint64_t *counts, uint64_t pairs,
+                                             uint64_t experts, float *pair_outputs, const yvex_hip_expert_weights *shared,
+                                             const void *shared_intermediate_q8k, uint64_t shared_rows, float *shared_outputs,
+                                             int *status, yvex_hip_stream stream)
+{
+    MfmaArgs a{}, alone{};
+    const WorklistView wl{order, expert_ids, bucket_offsets, bucket_populations, nullptr, counts};
+    int rc = prepare_down_rows(a, w, intermediate_q8k, wl, pairs, experts, pair_outputs, status);
+    if (!rc) rc = prepare_down_rows(alone, shared, shared_intermediate_q8k, kNoWorklist, shared_rows, 1u, shared_outputs, status);
+    if (!rc && (!expert_ids || !rows_join(a.pr, alone.pr, w, shared, false))) rc = ST_UNSUPPORTED;
+    return rc ? rc : launch_rows<false>(a, w->down_qtype, as_stream(stream), &alone.pr);
 }

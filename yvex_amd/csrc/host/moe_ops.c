@@ -555,6 +555,7 @@ static int moe_execute_rows(yvex_rocm_backend *backend, const yvex_moe_layer_job
     void *combined_target;
     unsigned long long table_address = 0ull;
     unsigned int matrix_launches[4] = {0};   /* routed up and down, shared up and down */
+    int joined[2] = {0};                     /* shared up and down rows in the routed ones' launches */
     int matrix_allowed = 1, envelope, hash_router, unsupported_width, routed_q8 = 0, shared_q8 = 0, routed_image = 0, shared_image = 0, has_shared, merged, row_batch, shared_row_batch, shared_dense, device_status = 0, rc, defer, host_rows, combined_egress, swiglu_quantized, routed_rows = 0;
     void *status;
     yvex_hip_stream stream;
@@ -835,6 +836,11 @@ sequence:
                                                            (float *)AT(shared_intermediate));
         matrix_launches[3] = yvex_hip_moe_down_rows_launches(&shared, AT(shared_intermediate_q8), NULL, row_count, 1ull,
                                                              (float *)AT(shared_outputs));
+        for (int down = 0; down < 2; ++down) {
+            joined[down] = yvex_hip_moe_rows_join(&routed, (const uint64_t *)AT(expert_ids), pairs, topk, experts, &shared,
+                                                  row_count, down);
+            if (joined[down]) matrix_launches[2 + down] = 0u;
+        }
     }
 #define COUNTED(index)                                                  \
     do {                                                                \
@@ -1055,7 +1061,15 @@ sequence:
             LAUNCH(yvex_hip_q8k_quantize((const float *)activations, row_count, hidden, hidden,
                                          (uint8_t *)AT(input_q8), (int *)status, stream), "rocm.moe.rows.q8");
     }
-    if (row_batch) {
+    if (joined[0]) {
+        LAUNCH(yvex_hip_moe_up_rows_joined(&routed, AT(input_q8), (const float *)AT(weights), (const uint64_t *)AT(order),
+                                           (const uint64_t *)AT(expert_ids), (const uint64_t *)AT(bucket_offsets),
+                                           (const uint64_t *)AT(bucket_populations), (const uint64_t *)AT(counts),
+                                           pairs, topk, experts, layer->activation_limit, (float *)AT(intermediate),
+                                           &shared, row_count, (float *)AT(shared_intermediate), (int *)status, stream),
+               "rocm.moe.rows.up-matrix");
+        COUNTED(0);
+    } else if (row_batch) {
         LAUNCH(yvex_hip_moe_up_rows(&routed, AT(input_q8), (const float *)AT(weights),
                                     (const uint64_t *)AT(order), (const uint64_t *)AT(expert_ids),
                                     (const uint64_t *)AT(bucket_offsets),
@@ -1073,7 +1087,7 @@ sequence:
                            (float *)AT(intermediate), merged ? &shared : NULL, merged ? row_count : 0ull,
                            merged ? (float *)AT(shared_intermediate) : NULL, (int *)status, stream),
            "rocm.moe.rows.up");
-    if (shared_row_batch) {
+    if (shared_row_batch && !joined[0]) {
         LAUNCH(yvex_hip_moe_up_rows(&shared, AT(input_q8), NULL, NULL, NULL, NULL, NULL, NULL, row_count,
                                     1ull, 1ull, layer->activation_limit, (float *)AT(shared_intermediate),
                                     (int *)status, stream), "rocm.moe.rows.shared-up-matrix");
@@ -1088,7 +1102,7 @@ sequence:
                                             row_count * layer->shared_intermediate_width, layer->activation_limit,
                                             (float *)AT(shared_intermediate), (int *)status, stream),
                    "rocm.moe.rows.shared-swiglu");
-    } else if (has_shared && !merged && !shared_rides)
+    } else if (has_shared && !merged && !shared_rides && !joined[0])
         LAUNCH(yvex_hip_moe_up(&shared, shared_q8 ? AT(input_q8) : (void *)(uintptr_t)activations,
                                shared_q8, NULL, NULL, NULL, NULL, NULL, NULL, NULL, row_count, 1ull, 1ull,
                                layer->activation_limit, (float *)AT(shared_intermediate), NULL, 0ull, NULL,
@@ -1121,7 +1135,16 @@ sequence:
                                      layer->shared_intermediate_width, layer->shared_intermediate_width,
                                      (uint8_t *)AT(shared_intermediate_q8), (int *)status, stream),
                "rocm.moe.rows.q8-shared-mid");
-    if (row_batch) {
+    if (joined[1]) {
+        LAUNCH(yvex_hip_moe_down_rows_joined(&routed, AT(intermediate_q8), (const uint64_t *)AT(order),
+                                             (const uint64_t *)AT(expert_ids), (const uint64_t *)AT(bucket_offsets),
+                                             (const uint64_t *)AT(bucket_populations), (const uint64_t *)AT(counts),
+                                             pairs, experts, (float *)AT(pair_outputs), &shared,
+                                             AT(shared_intermediate_q8), row_count, (float *)AT(shared_outputs),
+                                             (int *)status, stream),
+               "rocm.moe.rows.down-matrix");
+        COUNTED(1);
+    } else if (row_batch) {
         LAUNCH(yvex_hip_moe_down_rows(&routed, AT(intermediate_q8), (const uint64_t *)AT(order),
                                       (const uint64_t *)AT(expert_ids), (const uint64_t *)AT(bucket_offsets),
                                       (const uint64_t *)AT(bucket_populations), (const uint64_t *)AT(counts),
@@ -1138,7 +1161,7 @@ sequence:
                              merged ? (shared_q8 ? AT(shared_intermediate_q8) : AT(shared_intermediate)) : NULL,
                              merged ? (float *)AT(shared_outputs) : NULL, (int *)status, stream),
            "rocm.moe.rows.down");
-    if (shared_row_batch) {
+    if (shared_row_batch && !joined[1]) {
         LAUNCH(yvex_hip_moe_down_rows(&shared, AT(shared_intermediate_q8), NULL, NULL, NULL, NULL, NULL,
                                       row_count, 1ull, (float *)AT(shared_outputs), (int *)status, stream),
                "rocm.moe.rows.shared-down-matrix");
@@ -1148,7 +1171,7 @@ sequence:
                                shared.down_row_bytes, AT(shared_intermediate_q8), 1, row_count,
                                layer->shared_intermediate_width, NULL, (float *)AT(shared_outputs), hidden, 1,
                                (int *)status, stream), "rocm.moe.rows.shared-down-dense");
-    else if (has_shared && !merged && !shared_rides)
+    else if (has_shared && !merged && !shared_rides && !joined[1])
         LAUNCH(yvex_hip_moe_down(&shared, shared_q8 ? AT(shared_intermediate_q8) : AT(shared_intermediate),
                                  shared_q8, NULL, NULL, NULL, NULL, NULL, NULL, row_count, 1ull,
                                  (float *)AT(shared_outputs), NULL, 0ull, NULL, NULL, (int *)status, stream),

@@ -370,6 +370,29 @@ def moe_down_rows(w: ExpertWeights, intermediate_q8k, wl, pairs, experts, pair_o
           C.c_uint64(experts), _ptr(pair_outputs), _ptr(status), _stream())
 
 
+def moe_rows_join(w: ExpertWeights, wl, pairs, topk, experts, shared: ExpertWeights, shared_rows, down) -> bool:
+    return bool(load_library().yvex_hip_moe_rows_join(
+        C.byref(w), _ptr(wl.expert_ids), C.c_uint64(pairs), C.c_uint64(topk), C.c_uint64(experts), C.byref(shared),
+        C.c_uint64(shared_rows), C.c_int(int(down))))
+
+
+def moe_up_rows_joined(w: ExpertWeights, act_q8k, route_weights, wl, pairs, topk, experts, limit, intermediate,
+                       shared: ExpertWeights, shared_rows, shared_intermediate, status):
+    """moe_up_rows of the routed experts and of a shared one in one launch, where moe_rows_join says so."""
+    _call("yvex_hip_moe_up_rows_joined", C.byref(w), _ptr(act_q8k), _ptr(route_weights), _ptr(wl.order), _ptr(wl.expert_ids),
+          _ptr(wl.bucket_offsets), _ptr(wl.bucket_populations), _ptr(wl.counts), C.c_uint64(pairs), C.c_uint64(topk),
+          C.c_uint64(experts), C.c_double(limit), _ptr(intermediate), C.byref(shared), C.c_uint64(shared_rows),
+          _ptr(shared_intermediate), _ptr(status), _stream())
+
+
+def moe_down_rows_joined(w: ExpertWeights, intermediate_q8k, wl, pairs, experts, pair_outputs, shared: ExpertWeights,
+                         shared_intermediate_q8k, shared_rows, shared_outputs, status):
+    _call("yvex_hip_moe_down_rows_joined", C.byref(w), _ptr(intermediate_q8k), _ptr(wl.order), _ptr(wl.expert_ids),
+          _ptr(wl.bucket_offsets), _ptr(wl.bucket_populations), _ptr(wl.counts), C.c_uint64(pairs), C.c_uint64(experts),
+          _ptr(pair_outputs), C.byref(shared), _ptr(shared_intermediate_q8k), C.c_uint64(shared_rows), _ptr(shared_outputs),
+          _ptr(status), _stream())
+
+
 def moe_reduce_combine(pair_outputs, rows, topk, hidden, shared, routed, combined, status):
     _call("yvex_hip_moe_reduce_combine", _ptr(pair_outputs), C.c_uint64(rows), C.c_uint64(topk),
           C.c_uint64(hidden), _ptr(shared), _ptr(routed), _ptr(combined), _ptr(status), _stream())
