@@ -733,6 +733,20 @@ def test_f32_tiles_of_32_weight_rows_match_float64(gpu, oracle, qtype, rows, wid
     assert int(status.item()) == 0
 
 
+# one input tile's workgroups test the weights for all: one input tile and several, of both sizes
+@pytest.mark.parametrize("inputs", [8, 40, 1500])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_a_weight_that_is_no_number_is_reported_once_for_all_input_rows(gpu, inputs, value):
+    from yvex_amd import kernels as K
+    weights, x = torch.ones((70, 1024), device=gpu), torch.ones((inputs, 1024), device=gpu)
+    for row, column in ((0, 0), (37, 1023), (69, 500)):
+        held, status = weights.clone(), K.new_status(gpu)
+        assert bool((K.matvec_f32_rows(held, x, status) == 1024.0).all()) and int(status.item()) == 0
+        held[row, column] = value
+        K.matvec_f32_rows(held, x, status)
+        assert int(status.item()) == 1
+
+
 # the shared expert's Q8_0 products beside preparation and quantization: the separate launches' bits, at one and two rows,
 # fewer weight rows than a workgroup has waves, rows between dword boundaries, several rows a wave
 @pytest.mark.parametrize("rows,hidden,middle,experts,topk,offset", [(1, 256, 256, 4, 2, 0), (2, 2048, 768, 16, 4, 2),

@@ -709,7 +709,11 @@ __global__ __launch_bounds__(WAVES * 64) void matvec_f32_tile16_kernel(MatvecArg
 // 32 columns ahead, passes them through a window of LDS of its own (144 bytes a row: the sixteen rows that a read
 // touches lie on different banks) and needs no barrier before the sums are added.
 // 256 x 7168 by 64 / 256 / 512 / 1111 / 2048 rows 18.7 / 38.6 / 62.6 / 136 / 168 us -> 14.0 / 25.0 / 40.8 / 87.0 / 131, with
-// the join.
+// the join. A vector instruction and a matrix instruction on doubles never run together (SQ_VALU_MFMA_COEXEC_CYCLES is zero), so the
+// vector instructions that are left count in full. Weights tested by one input tile's workgroups and conversions in batches:
+// 256 x 7168 by 1111 / 1500 / 2048 rows of a layer 102 / 117 / 160 -> 100 / 110 / 151 us, 256 x 4096 and 24 x 16384 by 333
+// 21.4 and 16.1 -> 20.0 and 15.2, level up to 96. (Two or three chunks ahead instead of one: registers of the second
+// workgroup, 160 -> 181; the eight workgroups of an input tile on one XCD: level.)
 constexpr unsigned kTile32Columns = 32u, kTile32Pitch = kTile32Columns * 4u + 16u, kTile32Waves = 8u;
 
 template <unsigned QT, unsigned INPUTS>
@@ -720,6 +724,9 @@ __global__ __launch_bounds__(kTile32Waves * 64) void matvec_f32_tile32_kernel(Ma
     typedef float v4f __attribute__((ext_vector_type(4)));
     constexpr unsigned kRows = 32u + INPUTS, kWindow = kRows * kTile32Pitch, kTiles = INPUTS / 8u;
     constexpr unsigned kInputLoads = INPUTS / 8u;
+    // Columns whose operands are converted together, ahead of eight matrix instructions that then follow one another: no
+    // vector instruction issues while one of them runs, and between two of them a conversion and its wait states are a gap.
+    constexpr unsigned kBatch = INPUTS == 16u ? 4u : 2u;
     static_assert((WAVES - 1u) * kTiles * 4u * 64u * 8u <= WAVES * kWindow, "the partial sums fit the windows");
     __shared__ __align__(16) unsigned char windows[WAVES * kWindow];
     const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -766,10 +773,13 @@ __global__ __launch_bounds__(kTile32Waves * 64) void matvec_f32_tile32_kernel(Ma
     if (begin < end) request(begin);
     for (unsigned chunk = begin; chunk < end; ++chunk) {
 #pragma unroll
-        for (unsigned k = 0; k < 4u; ++k) {
-            bad |= (unsigned)!finite_f32(weights[k][0]) | (unsigned)!finite_f32(weights[k][1]) |
-                   (unsigned)!finite_f32(weights[k][2]) | (unsigned)!finite_f32(weights[k][3]);
-            *reinterpret_cast<v4f *>(to + 8u * k * kTile32Pitch) = weights[k];
+        for (unsigned k = 0; k < 4u; ++k) *reinterpret_cast<v4f *>(to + 8u * k * kTile32Pitch) = weights[k];
+        // (vector instructions take the time of the matrix cores here: one input tile's workgroups test the weights for all)
+        if (blockIdx.y == 0u) {
+#pragma unroll
+            for (unsigned k = 0; k < 4u; ++k)
+                bad |= (unsigned)!finite_f32(weights[k][0]) | (unsigned)!finite_f32(weights[k][1]) |
+                       (unsigned)!finite_f32(weights[k][2]) | (unsigned)!finite_f32(weights[k][3]);
         }
 #pragma unroll
         for (unsigned k = 0; k < kInputLoads; ++k) *reinterpret_cast<v4f *>(to + (32u + 8u * k) * kTile32Pitch) = inputs[k];
@@ -785,10 +795,23 @@ __global__ __launch_bounds__(kTile32Waves * 64) void matvec_f32_tile32_kernel(Ma
             for (unsigned n = 0; n < INPUTS / 16u; ++n)
                 x[n] = *reinterpret_cast<const v4f *>(from + (32u + 16u * n) * kTile32Pitch + 64u * step);
 #pragma unroll
-            for (unsigned c = 0; c < 4u; ++c)
+            for (unsigned at = 0; at < 4u; at += kBatch) {
+                double wide[kBatch][2], in[kBatch][INPUTS / 16u];
 #pragma unroll
-                for (unsigned t = 0; t < kTiles; ++t)
-                    acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)w[t & 1u][c], (double)x[t >> 1][c], acc[t], 0, 0, 0);
+                for (unsigned c = 0; c < kBatch; ++c) {
+#pragma unroll
+                    for (unsigned m = 0; m < 2u; ++m) wide[c][m] = (double)w[m][at + c];
+#pragma unroll
+                    for (unsigned n = 0; n < INPUTS / 16u; ++n) in[c][n] = (double)x[n][at + c];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (unsigned c = 0; c < kBatch; ++c)
+#pragma unroll
+                    for (unsigned t = 0; t < kTiles; ++t)
+                        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(wide[c][t & 1u], in[c][t >> 1], acc[t], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
