@@ -193,6 +193,12 @@ int yvex_hip_worklist_build(const uint64_t *selected, uint64_t pairs, uint64_t t
                             uint64_t *bucket_offsets, uint64_t *bucket_populations,
                             uint64_t *sweep_offsets, uint64_t *counts, int *status,
                             yvex_hip_stream stream);
+/* yvex_hip_worklist_build and yvex_hip_q8k_quantize of the pairs / topk input rows, which lie end to end, in one launch: the
+ * same words and blocks. For large batches; a small one's are yvex_hip_moe_prepare_routed's. */
+int yvex_hip_worklist_quantize(const uint64_t *selected, uint64_t pairs, uint64_t topk, uint64_t experts,
+                               uint64_t *order, uint64_t *expert_ids, uint64_t *bucket_offsets,
+                               uint64_t *bucket_populations, uint64_t *sweep_offsets, uint64_t *counts,
+                               const float *values, uint64_t width, uint8_t *encoded, int *status, yvex_hip_stream stream);
 
 /* A decode batch's preparation in one launch: yvex_hip_moe_route_rows, yvex_hip_worklist_build and
  * (when values is not NULL) yvex_hip_q8k_quantize of the rows x width input, with the same outputs

@@ -429,6 +429,37 @@ def test_sweeps_agree_with_the_matrix_core_kernels(gpu, oracle, qtype, hidden, i
     assert same_bits(out[0], out[1]) and int(status.item()) == 0
 
 
+# selections that a thread keeps and that it reads again, the order put together in LDS and stored word by word, with and
+# without the table of counts below a word; one row, one expert, a selection that repeats or is no expert
+@pytest.mark.parametrize("rows,experts,topk,fault", [
+    (1, 1, 1, None), (513, 256, 8, None), (2048, 256, 8, None), (2047, 256, 9, None), (3001, 250, 6, None), (4096, 256, 8, None),
+    (4096, 7, 7, None), (1111, 33, 3, "twice"), (1111, 33, 3, "none")])
+def test_worklist_and_quantization_in_one_launch(gpu, oracle, rows, experts, topk, fault):
+    from yvex_amd import kernels as K
+    width, g = 512, oracle.Generator(42, f"large.worklist.{rows}.{experts}.{topk}")
+    keys = g.normal(rows * experts).reshape(rows, experts) - 0.05 * np.arange(experts)
+    chosen = np.argsort(-keys, axis=1)[:, :topk].astype(np.int64)
+    if fault:
+        chosen[700, 2] = chosen[700, 0] if fault == "twice" else experts
+    selected, x = dev(chosen, gpu), dev(g.normal(rows * width).reshape(rows, width), gpu)
+    status = [K.new_status(gpu) for _ in range(2)]
+    wl, q8 = [K.Worklist(rows * topk, experts, gpu) for _ in range(2)], [torch.zeros(rows * 2 * 292, dtype=torch.uint8, device=gpu)] * 2
+    K.worklist_build(selected, experts, status[0], wl[0])
+    q8[0] = K.q8k_quantize(x, status[0]).view(torch.uint8).reshape(-1)
+    call("yvex_hip_worklist_quantize", ptr(selected), u64(rows * topk), u64(topk), u64(experts), ptr(wl[1].order),
+         ptr(wl[1].expert_ids), ptr(wl[1].bucket_offsets), ptr(wl[1].bucket_populations), ptr(wl[1].sweep_offsets),
+         ptr(wl[1].counts), ptr(x), u64(width), ptr(q8[1]), ptr(status[1]))
+    assert torch.equal(q8[0], q8[1]) and [int(s.item()) for s in status] == [2 if fault else 0] * 2
+    if fault:
+        return
+    for name in ("order", "expert_ids", "bucket_populations", "counts"):
+        assert torch.equal(getattr(wl[0], name), getattr(wl[1], name)), name
+    buckets = int(wl[0].counts[0].item())
+    assert torch.equal(wl[0].order, torch.sort(selected.reshape(-1), stable=True)[1])
+    for name in ("bucket_offsets", "sweep_offsets"):
+        assert torch.equal(getattr(wl[0], name)[:buckets + 1], getattr(wl[1], name)[:buckets + 1]), name
+
+
 # a shared tile of one row, a whole one, one and a row; few routed pairs and several tiles a bucket; with the few-pair
 # kernels beside (1100 rows of two superblocks, which a matrix alone has too many of for them)
 @pytest.mark.parametrize("down,hidden,intermediate,rows,topk", [

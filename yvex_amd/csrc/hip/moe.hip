@@ -103,17 +103,28 @@ constexpr unsigned kWorklistMaxRows = 4096u;
 
 __host__ __device__ constexpr unsigned worklist_pitch(unsigned rows) { return (rows + 31u) / 32u | 1u; }
 
-// The whole worklist by one workgroup; shared_words is its dynamic LDS (worklist_lds_bytes). `routed`: the selections
-// in LDS, from a workgroup that has routed the rows itself and need not wait for its stores to come back.
+// The whole worklist by one workgroup of 1024 threads; shared_words is its dynamic LDS (worklist_lds_bytes). `routed`: the
+// selections in LDS, from a workgroup that has routed the rows itself and need not wait for its stores to come back.
+// LARGE: for more rows than kPrepareMaxRoutedRows. One workgroup's round trips to memory, and its stores of single words, bound it there:
+// 16 384 stores that touch a line each are 8 us. So the selections are read once and kept, four threads count an expert's
+// words, and the order is put together in LDS (`ordered`, where it fits) and stored in lines. A decode batch
+// has no use for that, and its launch fetches every instruction to run it once: 96 rows 6.2 us without, 6.7 with.
+// With rows of pairs by a multiplication as well 2048 rows of eight experts 21 -> 15 us, 1111 rows 13 -> 10. (The odd pitch and the counts
+// below a word: 2048 rows 39 -> 22 us before, 4096 rows 872 -> 112.)
+template <bool LARGE>
 __device__ __forceinline__ void worklist_block(
     const unsigned long long *__restrict__ selected, unsigned pairs, unsigned topk,
     unsigned experts, unsigned long long *__restrict__ order,
     unsigned long long *__restrict__ expert_ids, unsigned long long *__restrict__ bucket_offsets,
     unsigned long long *__restrict__ bucket_populations,
     unsigned long long *__restrict__ sweep_offsets, unsigned long long *__restrict__ counts,
-    int *status, unsigned *shared_words, bool with_below, const unsigned *routed = nullptr)
+    int *status, unsigned *shared_words, bool with_below, bool with_ordered = false, const unsigned *routed = nullptr)
 {
     const unsigned rows = pairs / topk;
+    // p / topk, exact while p * topk < 2^32 (4096 rows of 256 choices at most). In place of two divisions a pair: the
+    // preparation of 1 / 96 / 333 rows 9.1 / 6.0 / 7.3 -> 8.8 / 5.7 / 6.4 us
+    const unsigned inverse = topk == 1u ? 0u : 0xffffffffu / topk + 1u;
+    auto row_of = [&](unsigned p) { return inverse ? __umulhi(p, inverse) : p; };
     const unsigned words = (rows + 31u) / 32u;            // bitmap words per expert
     const unsigned pitch = worklist_pitch(rows);          // odd: the experts' words in different banks
     unsigned *bitmap = shared_words;                       // [experts][pitch]
@@ -128,41 +139,85 @@ __device__ __forceinline__ void worklist_block(
         slot[experts + 1536u] = 0u;   // running maximum of the populations (scan[1536])
     }
     __syncthreads();
-    // (Four selections a thread in flight: a large batch's loops are round trips to memory. With the odd
-    // pitch, and the counts below a word stored word by word, 2048 rows of eight experts take 22 us, not
-    // 39, and 4096 rows 112, not 872.)
-    constexpr unsigned kInFlight = 4u;
-    for (unsigned first = tid; first < pairs; first += kInFlight * blockDim.x) {
-        unsigned long long chosen[kInFlight];
+    // A thread's first selections in registers (2048 rows of eight experts have sixteen), the others four at a time, twice
+    constexpr unsigned kKept = LARGE ? 16u : 0u, kInFlight = 4u, threads = 1024u;
+    auto selection = [&](unsigned p) { return routed ? (unsigned long long)routed[p] : selected[p]; };
+    auto mark = [&](unsigned p, unsigned e) {
+        if (e >= experts) {
+            bad = 1u;
+            return;
+        }
+        const unsigned row = row_of(p);
+        const unsigned old = atomicOr(&bitmap[e * pitch + (row >> 5)], 1u << (row & 31u));
+        if (old & (1u << (row & 31u))) bad = 1u;   // duplicate expert inside one row
+    };
+    auto expert_of = [](unsigned long long chosen) { return chosen > 0xffffffffull ? 0xffffffffu : (unsigned)chosen; };
+    unsigned kept[LARGE ? kKept : 1u];
+    if constexpr (LARGE) {
+        unsigned long long chosen[kKept];
 #pragma unroll
-        for (unsigned k = 0; k < kInFlight; ++k) {
-            const unsigned p = first + k * blockDim.x;
-            chosen[k] = routed ? routed[p < pairs ? p : first] : selected[p < pairs ? p : first];
+        for (unsigned k = 0; k < kKept; ++k) {
+            if ((k / kInFlight * kInFlight) * threads >= pairs) break;
+            const unsigned p = tid + k * threads;
+            chosen[k] = selection(p < pairs ? p : pairs - 1u);
         }
 #pragma unroll
-        for (unsigned k = 0; k < kInFlight; ++k) {
-            const unsigned p = first + k * blockDim.x;
-            if (p >= pairs) break;
-            if (chosen[k] >= experts) {
-                bad = 1u;
-                continue;
-            }
-            const unsigned row = p / topk;
-            const unsigned old = atomicOr(&bitmap[(unsigned)chosen[k] * pitch + (row >> 5)], 1u << (row & 31u));
-            if (old & (1u << (row & 31u))) bad = 1u;   // duplicate expert inside one row
+        for (unsigned k = 0; k < kKept; ++k) {
+            if ((k / kInFlight * kInFlight) * threads >= pairs) break;
+            kept[k] = expert_of(chosen[k]);
+            if (tid + k * threads < pairs) mark(tid + k * threads, kept[k]);
         }
     }
+    auto each_behind = [&](auto &&with) {
+        for (unsigned first = kKept * threads + tid; first < pairs; first += kInFlight * threads) {
+            unsigned long long chosen[kInFlight];
+#pragma unroll
+            for (unsigned k = 0; k < kInFlight; ++k) {
+                const unsigned p = first + k * threads;
+                chosen[k] = selection(p < pairs ? p : first);
+            }
+#pragma unroll
+            for (unsigned k = 0; k < kInFlight; ++k)
+                if (first + k * threads < pairs) with(first + k * threads, expert_of(chosen[k]));
+        }
+    };
+    each_behind(mark);
     __syncthreads();
     // rows below each bitmap word that chose the expert (16 bits: at most 4096 rows), kept when
     // the table fits beside the bitmap
     unsigned short *below = reinterpret_cast<unsigned short *>(slot + experts + 1537u);
-    for (unsigned e = tid; e < experts; e += blockDim.x) {
+    [[maybe_unused]] unsigned short *const ordered = below + experts * words;      // [pairs], behind the table
+    if constexpr (LARGE) {
+        unsigned *const part = slot + experts + 64u;       // [4][256], in what the scan leaves free
+        const unsigned e = tid & 255u, from = words * (tid >> 8) / 4u, to = words * ((tid >> 8) + 1u) / 4u;
         unsigned n = 0u;
-        for (unsigned w = 0; w < words; ++w) {
-            if (with_below) below[w * experts + e] = (unsigned short)n;
-            n += __popc(bitmap[e * pitch + w]);
+        if (e < experts) {
+#pragma unroll 4
+            for (unsigned w = from; w < to; ++w) n += __popc(bitmap[e * pitch + w]);
+            part[tid] = n;
         }
-        population[e] = n;
+        __syncthreads();
+        if (e < experts) {
+            unsigned before = 0u;
+            for (unsigned other = e; other < tid; other += 256u) before += part[other];
+            if (tid >= 768u) population[e] = before + n;
+            if (with_below) {
+#pragma unroll 4
+                for (unsigned w = from; w < to; ++w) {
+                    below[w * experts + e] = (unsigned short)before;
+                    before += __popc(bitmap[e * pitch + w]);
+                }
+            }
+        }
+    } else {
+        for (unsigned e = tid; e < experts; e += threads) {
+            unsigned n = 0u;
+            for (unsigned w = 0; w < words; ++w) {
+                if (with_below) below[w * experts + e] = (unsigned short)n;
+                n += __popc(bitmap[e * pitch + w]);
+            }
+            population[e] = n;
+        }
     }
     __syncthreads();
     // Inclusive prefix sums over the experts (<= 256: the first four wavefronts) of population,
@@ -232,27 +287,29 @@ __device__ __forceinline__ void worklist_block(
     if (tid == 0u) counts[1] = scan[1536u];
     // every pair finds its own place: its bucket's start plus the rows below its own that chose
     // the same expert (pairs of a bucket stay in row order, which is the stable order)
-    for (unsigned first = tid; first < pairs; first += kInFlight * blockDim.x) {
-        unsigned long long chosen[kInFlight];
+    auto place = [&](unsigned p, unsigned e) {
+        if (e >= experts) return;
+        const unsigned row = row_of(p), w = row >> 5;
+        const unsigned *mine = bitmap + e * pitch;
+        unsigned before = __popc(mine[w] & ((1u << (row & 31u)) - 1u));
+        if (with_below) before += below[w * experts + e];
+        else
+            for (unsigned other = 0; other < w; ++other) before += __popc(mine[other]);
+        if (LARGE && with_ordered) ordered[offset[e] + before] = (unsigned short)p;
+        else order[offset[e] + before] = p;
+    };
+    if constexpr (LARGE) {
 #pragma unroll
-        for (unsigned k = 0; k < kInFlight; ++k) {
-            const unsigned p = first + k * blockDim.x;
-            chosen[k] = routed ? routed[p < pairs ? p : first] : selected[p < pairs ? p : first];
+        for (unsigned k = 0; k < kKept; ++k) {
+            if ((k / kInFlight * kInFlight) * threads >= pairs) break;
+            if (tid + k * threads < pairs) place(tid + k * threads, kept[k]);
         }
-#pragma unroll
-        for (unsigned k = 0; k < kInFlight; ++k) {
-            const unsigned p = first + k * blockDim.x;
-            if (p >= pairs) break;
-            const unsigned long long e = chosen[k];
-            if (e >= experts) continue;
-            const unsigned row = p / topk, w = row >> 5;
-            const unsigned *mine = bitmap + (unsigned)e * pitch;
-            unsigned before = __popc(mine[w] & ((1u << (row & 31u)) - 1u));
-            if (with_below) before += below[w * experts + (unsigned)e];
-            else
-                for (unsigned other = 0; other < w; ++other) before += __popc(mine[other]);
-            order[offset[e] + before] = p;
-        }
+    }
+    each_behind(place);
+    if (LARGE && with_ordered) {
+        __syncthreads();
+        // (a batch that is refused below leaves places unwritten: every pair number is one all the same)
+        for (unsigned at = tid; at < pairs; at += threads) order[at] = ordered[at] < pairs ? ordered[at] : 0u;
     }
     __syncthreads();
     if (tid == 0u && bad) raise_status(status, 2);
@@ -267,8 +324,46 @@ __global__ __launch_bounds__(1024) void worklist_kernel(
     int *status, int with_below)
 {
     extern __shared__ unsigned shared_words[];
-    worklist_block(selected, pairs, topk, experts, order, expert_ids, bucket_offsets, bucket_populations,
-                   sweep_offsets, counts, status, shared_words, with_below != 0);
+    worklist_block<false>(selected, pairs, topk, experts, order, expert_ids, bucket_offsets, bucket_populations,
+                          sweep_offsets, counts, status, shared_words, with_below != 0);
+}
+
+// A large batch's worklist by the first workgroup and, beside it, the input rows' Q8_K blocks by the others, four a
+// wavefront: neither waits for the other, and the one workgroup takes as long as all the others. (Of the same LDS as the first, one
+// a compute unit, so its waves go on from block to block and ask ahead.) In a layer of 7168 columns, eight of 256 experts,
+// 2048 rows 21.2 and 13.9 us -> 22.5, 1111 rows 14.0 and 8.6 -> 17.9.
+__global__ __launch_bounds__(1024) void worklist_quantize_kernel(
+    const unsigned long long *__restrict__ selected, unsigned pairs, unsigned topk,
+    unsigned experts, unsigned long long *__restrict__ order,
+    unsigned long long *__restrict__ expert_ids, unsigned long long *__restrict__ bucket_offsets,
+    unsigned long long *__restrict__ bucket_populations,
+    unsigned long long *__restrict__ sweep_offsets, unsigned long long *__restrict__ counts,
+    int *status, int with_below, int with_ordered, const float *__restrict__ values, unsigned tasks,
+    unsigned char *__restrict__ encoded)
+{
+    extern __shared__ unsigned shared_words[];
+    if (blockIdx.x == 0u) {
+        worklist_block<true>(selected, pairs, topk, experts, order, expert_ids, bucket_offsets, bucket_populations,
+                             sweep_offsets, counts, status, shared_words, with_below != 0, with_ordered != 0);
+        return;
+    }
+    const unsigned lane = threadIdx.x & 63u, stride = (gridDim.x - 1u) * 64u;
+    unsigned task = (blockIdx.x - 1u) * 64u + 4u * (threadIdx.x >> 6) + (lane >> 4);
+    float v[4][4], ahead[4][4];
+    auto request = [&](unsigned wanted, float (&to)[4][4]) {
+        const unsigned held = wanted < tasks ? wanted : tasks - 1u;
+#pragma unroll
+        for (unsigned k = 0; k < 4u; ++k) __builtin_memcpy(to[k], values + held * 256ull + 4u * (lane & 15u) + 64u * k, 16);
+    };
+    request(task, v);
+    for (unsigned first = (blockIdx.x - 1u) * 64u; first < tasks; first += stride, task += stride) {
+        request(task + stride, ahead);
+        q8k_quantize_four(v, encoded + (task < tasks ? task : tasks - 1u) * (unsigned long long)kQ8KBytes, lane, task < tasks, status);
+#pragma unroll
+        for (unsigned k = 0; k < 4u; ++k)
+#pragma unroll
+            for (unsigned i = 0; i < 4u; ++i) v[k][i] = ahead[k][i];
+    }
 }
 
 // A decode batch's preparation in one launch instead of three: workgroup 0 routes the rows (one
@@ -355,11 +450,11 @@ __global__ __launch_bounds__(1024) void decode_prepare_kernel(
                           chosen + row * topk);
             __syncthreads();   // the selections are read by other waves below, the scores overwritten
         }
-        worklist_block(selected, rows * topk, topk, experts, order, expert_ids, bucket_offsets, bucket_populations,
-                       sweep_offsets, counts, status, shared_words, true, chosen);
+        worklist_block<false>(selected, rows * topk, topk, experts, order, expert_ids, bucket_offsets, bucket_populations,
+                       sweep_offsets, counts, status, shared_words, true, false, chosen);
         return;
     }
-    worklist_block(selected, rows * topk, topk, experts, order, expert_ids, bucket_offsets,
+    worklist_block<false>(selected, rows * topk, topk, experts, order, expert_ids, bucket_offsets,
                    bucket_populations, sweep_offsets, counts, status, shared_words, true);
 }
 
@@ -920,6 +1015,32 @@ extern "C" int yvex_hip_worklist_build(const uint64_t *selected, uint64_t pairs,
         (unsigned long long *)bucket_offsets, (unsigned long long *)bucket_populations,
         (unsigned long long *)sweep_offsets, (unsigned long long *)counts, status, with_below);
     return check_launch("worklist_build");
+}
+
+extern "C" int yvex_hip_worklist_quantize(const uint64_t *selected, uint64_t pairs, uint64_t topk, uint64_t experts,
+                                          uint64_t *order, uint64_t *expert_ids, uint64_t *bucket_offsets,
+                                          uint64_t *bucket_populations, uint64_t *sweep_offsets, uint64_t *counts,
+                                          const float *values, uint64_t width, uint8_t *encoded, int *status,
+                                          yvex_hip_stream stream)
+{
+    if (!selected || !order || !expert_ids || !bucket_offsets || !bucket_populations || !sweep_offsets || !counts ||
+        !status || !pairs || !topk || !experts || experts > 256u || pairs % topk || !values || !encoded || !width || width % 256u)
+        return ST_INVALID_ARG;
+    const uint64_t rows = pairs / topk, tasks = rows * (width / 256u);
+    if (rows > kWorklistMaxRows || tasks > 0x7fffffffull) return ST_BOUNDS;
+    int with_below = 0;
+    size_t lds = worklist_lds_bytes(experts, rows, &with_below);
+    if (lds > kWorklistLdsLimit) return ST_BOUNDS;
+    const bool with_ordered = with_below && pairs <= 65536u && lds + pairs * sizeof(unsigned short) <= kWorklistLdsLimit;
+    if (with_ordered) lds += pairs * sizeof(unsigned short);
+    YVEX_ALLOW_DYNAMIC_LDS(worklist_quantize_kernel, kWorklistLdsLimit);
+    const uint64_t groups = (tasks + 63u) / 64u, others = compute_units() > 1 ? (uint64_t)compute_units() - 1u : 1u;
+    worklist_quantize_kernel<<<1u + (unsigned)(groups < others ? groups : others), 1024, lds, as_stream(stream)>>>(
+        (const unsigned long long *)selected, (unsigned)pairs, (unsigned)topk, (unsigned)experts,
+        (unsigned long long *)order, (unsigned long long *)expert_ids, (unsigned long long *)bucket_offsets,
+        (unsigned long long *)bucket_populations, (unsigned long long *)sweep_offsets, (unsigned long long *)counts, status,
+        with_below, with_ordered, values, (unsigned)tasks, encoded);
+    return check_launch("worklist_quantize");
 }
 
 extern "C" int yvex_hip_moe_prepare_supported(uint64_t rows, uint64_t experts, uint64_t topk)

@@ -1052,14 +1052,22 @@ sequence:
                                            layer->routed_scaling_factor, (uint64_t *)AT(selected),
                                            (float *)AT(weights), (int *)status, stream),
                    "rocm.moe.rows.route");
-        LAUNCH(yvex_hip_worklist_build((const uint64_t *)AT(selected), pairs, topk, experts,
-                                       (uint64_t *)AT(order), (uint64_t *)AT(expert_ids),
-                                       (uint64_t *)AT(bucket_offsets), (uint64_t *)AT(bucket_populations),
-                                       (uint64_t *)AT(sweep_offsets), (uint64_t *)AT(counts), (int *)status,
-                                       stream), "rocm.moe.rows.worklist");
-        if (need_q8)
-            LAUNCH(yvex_hip_q8k_quantize((const float *)activations, row_count, hidden, hidden,
-                                         (uint8_t *)AT(input_q8), (int *)status, stream), "rocm.moe.rows.q8");
+        if (need_q8 && row_count > 512ull)
+            LAUNCH(yvex_hip_worklist_quantize((const uint64_t *)AT(selected), pairs, topk, experts, (uint64_t *)AT(order),
+                                              (uint64_t *)AT(expert_ids), (uint64_t *)AT(bucket_offsets),
+                                              (uint64_t *)AT(bucket_populations), (uint64_t *)AT(sweep_offsets),
+                                              (uint64_t *)AT(counts), (const float *)activations, hidden,
+                                              (uint8_t *)AT(input_q8), (int *)status, stream), "rocm.moe.rows.worklist");
+        else {
+            LAUNCH(yvex_hip_worklist_build((const uint64_t *)AT(selected), pairs, topk, experts,
+                                           (uint64_t *)AT(order), (uint64_t *)AT(expert_ids),
+                                           (uint64_t *)AT(bucket_offsets), (uint64_t *)AT(bucket_populations),
+                                           (uint64_t *)AT(sweep_offsets), (uint64_t *)AT(counts), (int *)status,
+                                           stream), "rocm.moe.rows.worklist");
+            if (need_q8)
+                LAUNCH(yvex_hip_q8k_quantize((const float *)activations, row_count, hidden, hidden,
+                                             (uint8_t *)AT(input_q8), (int *)status, stream), "rocm.moe.rows.q8");
+        }
     }
     if (joined[0]) {
         LAUNCH(yvex_hip_moe_up_rows_joined(&routed, AT(input_q8), (const float *)AT(weights), (const uint64_t *)AT(order),
