@@ -460,6 +460,25 @@ def test_worklist_and_quantization_in_one_launch(gpu, oracle, rows, experts, top
         assert torch.equal(getattr(wl[0], name)[:buckets + 1], getattr(wl[1], name)[:buckets + 1]), name
 
 
+# ranks in one batch of loads and in several, columns in fours and one by one, edges of a workgroup's columns, more rows
+# than a grid has in its second direction
+@pytest.mark.parametrize("rows,topk,hidden", [(1, 1, 4), (3, 8, 1024), (2, 9, 1028), (5, 17, 258), (1, 6, 2050), (65537, 2, 4)])
+def test_reduce_adds_ranks_in_order(gpu, oracle, rows, topk, hidden):
+    from yvex_amd import kernels as K
+    g = oracle.Generator(42, f"reduce.{rows}.{topk}.{hidden}")
+    pairs = dev(g.normal(rows * topk * hidden).reshape(rows, topk, hidden).astype(np.float32), gpu)
+    shared = dev(g.normal(rows * hidden).reshape(rows, hidden).astype(np.float32), gpu)
+    routed, combined, status = torch.zeros_like(shared), torch.zeros_like(shared), K.new_status(gpu)
+    K.moe_reduce_combine(pairs, rows, topk, hidden, shared, routed, combined, status)
+    want = torch.zeros_like(shared)
+    for rank in range(topk):
+        want += pairs[:, rank]
+    assert same_bits(routed, want) and same_bits(combined, (want + shared).to(torch.bfloat16).float()) and int(status.item()) == 0
+    pairs[rows - 1, topk - 1, hidden - 1] = float("nan")
+    K.moe_reduce_combine(pairs, rows, topk, hidden, shared, routed, combined, status)
+    assert int(status.item()) == 1
+
+
 # a shared tile of one row, a whole one, one and a row; few routed pairs and several tiles a bucket; with the few-pair
 # kernels beside (1100 rows of two superblocks, which a matrix alone has too many of for them)
 @pytest.mark.parametrize("down,hidden,intermediate,rows,topk", [
