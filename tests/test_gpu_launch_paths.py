@@ -461,8 +461,8 @@ def test_worklist_and_quantization_in_one_launch(gpu, oracle, rows, experts, top
 
 
 # ranks in one batch of loads and in several, columns in fours and one by one, edges of a workgroup's columns, more rows
-# than a grid has in its second direction
-@pytest.mark.parametrize("rows,topk,hidden", [(1, 1, 4), (3, 8, 1024), (2, 9, 1028), (5, 17, 258), (1, 6, 2050), (65537, 2, 4)])
+# than a grid has in its second direction, outputs that are loaded past the caches
+@pytest.mark.parametrize("rows,topk,hidden", [(1, 1, 4), (3, 8, 1024), (2, 9, 1028), (5, 17, 258), (1, 6, 2050), (65537, 2, 4), (2100, 8, 1028)])
 def test_reduce_adds_ranks_in_order(gpu, oracle, rows, topk, hidden):
     from yvex_amd import kernels as K
     g = oracle.Generator(42, f"reduce.{rows}.{topk}.{hidden}")

@@ -833,8 +833,8 @@ __global__ __launch_bounds__(kGroupedThreads) void grouped_kernel(GroupedArgs a)
 // rank order, so the result does not depend on LANES. The memory bounds it (a pair's outputs are read once and from there); a workgroup's
 // place is its block numbers (a row's and a column's number by 64-bit division were what a thread did first, for as long
 // as its loads took), and up to eight ranks' loads are in flight with the shared row's. Eight ranks of 7168 columns by 2048 rows
-// 107 -> 88 us (6.7 TB/s), 1111 rows 55.6 -> 52, up to 32 rows level (a branch a rank around its load: 1 us more of five rows).
-template <int LANES>
+// 107 -> 88 us (6.7 TB/s), 1111 rows 55.6 -> 52, up to 100 rows level (a branch a rank around its load: 1 us more of five rows). STREAMING: kReduceStreaming.
+template <int LANES, bool STREAMING>
 __global__ __launch_bounds__(256) void reduce_combine_kernel(
     const float *__restrict__ pair_outputs, unsigned long long rows, unsigned topk,
     unsigned long long hidden, const float *__restrict__ shared, float *__restrict__ routed,
@@ -853,8 +853,10 @@ __global__ __launch_bounds__(256) void reduce_combine_kernel(
                 constexpr unsigned kBatch = decltype(batch)::value;
                 Pack part[kBatch];
 #pragma unroll
-                for (unsigned k = 0; k < kBatch; ++k)
-                    part[k] = __builtin_nontemporal_load(reinterpret_cast<const Pack *>(source + (k < live ? k : live - 1u) * hidden));
+                for (unsigned k = 0; k < kBatch; ++k) {
+                    const Pack *const from = reinterpret_cast<const Pack *>(source + (k < live ? k : live - 1u) * hidden);
+                    part[k] = STREAMING ? __builtin_nontemporal_load(from) : *from;
+                }
 #pragma unroll
                 for (unsigned k = 0; k < kBatch; ++k) {
                     if (k >= live) break;
@@ -1284,6 +1286,10 @@ extern "C" int yvex_hip_moe_swiglu_rows(const float *gate, const float *up, uint
     return check_launch("moe_swiglu_rows");
 }
 
+// From here on pair outputs are loaded past the caches: eight ranks of 7168 columns by 100 / 333 / 700 / 1111 / 2048 rows (23 to 470 MB) 7.3 /
+// 17.3 / 33.5 / 49.6 / 93 us so, 7.0 / 17.8 / 34.3 / 54.3 / 105 through them.
+constexpr uint64_t kReduceStreaming = 64ull << 20;
+
 extern "C" int yvex_hip_moe_reduce_combine(const float *pair_outputs, uint64_t rows,
                                            uint64_t topk, uint64_t hidden, const float *shared,
                                            float *routed, float *combined, int *status,
@@ -1299,11 +1305,8 @@ extern "C" int yvex_hip_moe_reduce_combine(const float *pair_outputs, uint64_t r
     if ((rows * hidden / (quads ? 4u : 1u) + 255u) / 256u > 0x7fffffffull) return ST_BOUNDS;
     const uint64_t blocks = (hidden / (quads ? 4u : 1u) + 255u) / 256u;
     const dim3 grid((unsigned)blocks, (unsigned)(rows < 65535u ? rows : 65535u));
-    if (quads)
-        reduce_combine_kernel<4><<<grid, 256, 0, as_stream(stream)>>>(
-            pair_outputs, rows, (unsigned)topk, hidden, shared, routed, combined, status);
-    else
-        reduce_combine_kernel<1><<<grid, 256, 0, as_stream(stream)>>>(
-            pair_outputs, rows, (unsigned)topk, hidden, shared, routed, combined, status);
+    const auto kernel = !quads ? reduce_combine_kernel<1, false>
+                      : rows * topk * hidden * sizeof(float) > kReduceStreaming ? reduce_combine_kernel<4, true> : reduce_combine_kernel<4, false>;
+    kernel<<<grid, 256, 0, as_stream(stream)>>>(pair_outputs, rows, (unsigned)topk, hidden, shared, routed, combined, status);
     return check_launch("moe_reduce_combine");
 }
