@@ -380,7 +380,8 @@ def test_clamped_product_over_the_range_of_its_exponential(gpu, oracle, limit):
     assert int(status.item()) == (0 if bool(finite.all()) else 1)
 
 
-@pytest.mark.parametrize("rows,topk,width", [(1, 1, 4), (3, 6, 1028), (9, 8, 7168)])
+# (the last: pair outputs that are loaded past the caches)
+@pytest.mark.parametrize("rows,topk,width", [(1, 1, 4), (3, 6, 1028), (9, 8, 7168), (300, 8, 7172)])
 def test_combine_goes_straight_into_the_egress(gpu, oracle, rows, topk, width):
     from yvex_amd import kernels as K
     streams = 4

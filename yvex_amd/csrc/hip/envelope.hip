@@ -406,8 +406,8 @@ __global__ __launch_bounds__(kEnvelopeThreads) void mhc_egress_kernel(
 // memory took, and 87 registers kept a larger batch to five waves a SIMD. 4096 columns, six ranks, by 1 / 96 / 333 / 700 /
 // 1111 / 2048 rows 7.5 / 13.8 / 30.7 / 50.6 / 70.7 / 114.5 us with four columns, 3.8 / 10.2 / 25.2 / 47.2 / 69.9 / 117.1 with one;
 // eight ranks of 7168 columns by 2048 rows 209 and 213. The 2 % that 16-byte loads are ahead by at 2048 rows are not worth a
-// second kernel.
-template <unsigned STREAMS>
+// second kernel. STREAMING: kPairsStreaming.
+template <unsigned STREAMS, bool STREAMING>
 __global__ __launch_bounds__(kEnvelopeThreads) void combine_egress_kernel(
     const float *__restrict__ pair_outputs, unsigned topk, const float *__restrict__ shared,
     const float *__restrict__ rows, const float *__restrict__ post, const float *__restrict__ combination,
@@ -435,8 +435,10 @@ __global__ __launch_bounds__(kEnvelopeThreads) void combine_egress_kernel(
     for (unsigned rank = 0; rank < topk; rank += 4u) {
         float part[4];
 #pragma unroll
-        for (unsigned k = 0; k < 4u; ++k)
-            part[k] = source[(unsigned long long)(rank + k < topk ? rank + k : topk - 1u) * width];
+        for (unsigned k = 0; k < 4u; ++k) {
+            const float *const from = source + (unsigned long long)(rank + k < topk ? rank + k : topk - 1u) * width;
+            part[k] = STREAMING ? __builtin_nontemporal_load(from) : *from;
+        }
 #pragma unroll
         for (unsigned k = 0; k < 4u; ++k) {
             if (rank + k >= topk) break;
@@ -605,6 +607,11 @@ extern "C" int yvex_hip_mhc_egress(const float *core, const float *rows, const f
     return check_launch("mhc_egress");
 }
 
+// From here on pair outputs, which nobody reads again, are loaded past the caches: six ranks of 4096 columns by 300 / 500 / 700 / 1111 / 1500 /
+// 2048 rows (29 to 201 MB) 17.1 / 25.5 / 34.5 / 51.9 / 68.7 / 92.7 us so, 16.5 / 25.7 / 35.7 / 55.2 / 72.8 / 95.0 through them, and the ingress of the
+// layer behind 1 to 2 us less, whose rows stay in the caches.
+constexpr uint64_t kPairsStreaming = 64ull << 20;
+
 // Four streams, widths of whole 16-byte pieces; UNSUPPORTED otherwise (the two launches serve those).
 extern "C" int yvex_hip_moe_combine_egress(const float *pair_outputs, uint64_t row_count, uint64_t topk,
                                            uint64_t streams, uint64_t width, const float *shared, const float *rows,
@@ -619,7 +626,8 @@ extern "C" int yvex_hip_moe_combine_egress(const float *pair_outputs, uint64_t r
         (((uintptr_t)pair_outputs | (uintptr_t)shared | (uintptr_t)rows | (uintptr_t)output) & 15u))
         return ST_UNSUPPORTED;
     const unsigned blocks_per_row = (unsigned)((width + kEnvelopeThreads - 1u) / kEnvelopeThreads);
-    combine_egress_kernel<4><<<(unsigned)(row_count * blocks_per_row), kEnvelopeThreads, 0, as_stream(stream)>>>(
+    const auto kernel = row_count * topk * width * sizeof(float) > kPairsStreaming ? combine_egress_kernel<4, true> : combine_egress_kernel<4, false>;
+    kernel<<<(unsigned)(row_count * blocks_per_row), kEnvelopeThreads, 0, as_stream(stream)>>>(
         pair_outputs, (unsigned)topk, shared, rows, post, combination, row_count, (unsigned)width, blocks_per_row,
         output, status);
     return check_launch("moe_combine_egress");
