@@ -461,6 +461,31 @@ def test_worklist_and_quantization_in_one_launch(gpu, oracle, rows, experts, top
         assert torch.equal(getattr(wl[0], name)[:buckets + 1], getattr(wl[1], name)[:buckets + 1]), name
 
 
+# so many choices a row that a row number by multiplication comes out one too high for the last pair: of 32 (96) rows that is the
+# first bit of another expert's words
+@pytest.mark.parametrize("rows,topk", [(32, 11627), (96, 6733)])
+def test_more_choices_a_row_than_experts_reach_no_other_experts_words(gpu, rows, topk):
+    """Such a batch repeats experts and is refused; its lists hold the rows that chose an expert and nothing else."""
+    from yvex_amd import kernels as K
+    experts, width, pairs = 9, 256, rows * topk
+    inverse = 0xffffffff // topk + 1
+    assert ((pairs - 1) * inverse >> 32) == rows and (rows // 32) % 2 == 1
+    selected, x = torch.full((rows, topk), 5, dtype=torch.int64, device=gpu), torch.ones((rows, width), device=gpu)
+    q8 = torch.zeros(rows * 292, dtype=torch.uint8, device=gpu)
+    for quantizing in (False, True):
+        wl, status = K.Worklist(pairs, experts, gpu), K.new_status(gpu)
+        wl.order.zero_()
+        if quantizing:
+            call("yvex_hip_worklist_quantize", ptr(selected), u64(pairs), u64(topk), u64(experts), *K._wl_ptrs(wl), ptr(x),
+                 u64(width), ptr(q8), ptr(status))
+        else:
+            K.worklist_build(selected, experts, status, wl)
+        assert int(status.item()) == 2
+        assert wl.counts.tolist()[:3] == [1, rows, rows] and wl.expert_ids[0].item() == 5
+        assert wl.bucket_populations.tolist() == [rows] + [0] * (experts - 1)
+        assert bool(((wl.order >= 0) & (wl.order < pairs)).all())
+
+
 # ranks in one batch of loads and in several, columns in fours and one by one, edges of a workgroup's columns, more rows
 # than a grid has in its second direction, outputs that are loaded past the caches
 @pytest.mark.parametrize("rows,topk,hidden", [(1, 1, 4), (3, 8, 1024), (2, 9, 1028), (5, 17, 258), (1, 6, 2050), (65537, 2, 4), (2100, 8, 1028)])

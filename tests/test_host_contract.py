@@ -364,3 +364,19 @@ def test_shared_sessions_borrow_the_owner(monkeypatch):
     assert owner.close() == abi.STATE and owner.handle.value
     assert child.close() == 0, child.err.message
     assert owner.close() == 0, owner.err.message
+
+
+def _device(address):
+    return C.c_void_p(address)          # (never touched: the calls below are refused on the host)
+
+
+def _worklist_arguments(pairs, topk, experts=256):
+    """selected, pairs, topk, experts and the worklist's six arrays."""
+    return [_device(0x1000), C.c_uint64(pairs), C.c_uint64(topk), C.c_uint64(experts)] + [_device(0x2000 + 0x1000 * k) for k in range(6)]
+
+
+def test_worklists_of_more_pairs_than_their_kernels_count_are_refused(lib):
+    for pairs in (1 << 31, 1 << 33):
+        lists = _worklist_arguments(pairs, pairs)
+        assert lib.yvex_hip_worklist_build(*lists, _device(0x9000), None) == abi.BOUNDS
+        assert lib.yvex_hip_worklist_quantize(*lists, _device(0xa000), C.c_uint64(256), _device(0xb000), _device(0x9000), None) == abi.BOUNDS

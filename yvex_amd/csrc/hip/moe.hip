@@ -102,6 +102,7 @@ __global__ __launch_bounds__(256) void route_hash_rows_kernel(
 // which is exactly the stable counting sort of pairs by expert (src/graph/worklist.c:380-393).
 
 constexpr unsigned kWorklistMaxRows = 4096u;
+constexpr uint64_t kWorklistMaxPairs = 0x7fffffffull;    // (counted in 32 bits)
 
 __host__ __device__ constexpr unsigned worklist_pitch(unsigned rows) { return (rows + 31u) / 32u | 1u; }
 
@@ -123,10 +124,11 @@ __device__ __forceinline__ void worklist_block(
     int *status, unsigned *shared_words, bool with_below, bool with_ordered = false, const unsigned *routed = nullptr)
 {
     const unsigned rows = pairs / topk;
-    // p / topk, exact while p * topk < 2^32 (4096 rows of 256 choices at most). In place of two divisions a pair: the
-    // preparation of 1 / 96 / 333 rows 9.1 / 6.0 / 7.3 -> 8.8 / 5.7 / 6.4 us
+    // p / topk, exact while p * topk < 2^32 (so for 4096 rows of 256 choices). In place of two divisions a pair: the
+    // preparation of 1 / 96 / 333 rows 9.1 / 6.0 / 7.3 -> 8.8 / 5.7 / 6.4 us. More choices a row repeat an expert and are
+    // refused below; there a row may come out one too high, and the last one's would be another expert's word of the bitmap.
     const unsigned inverse = topk == 1u ? 0u : 0xffffffffu / topk + 1u;
-    auto row_of = [&](unsigned p) { return inverse ? __umulhi(p, inverse) : p; };
+    auto row_of = [&](unsigned p) { return inverse ? min(__umulhi(p, inverse), rows - 1u) : p; };
     const unsigned words = (rows + 31u) / 32u;            // bitmap words per expert
     const unsigned pitch = worklist_pitch(rows);          // odd: the experts' words in different banks
     unsigned *bitmap = shared_words;                       // [experts][pitch]
@@ -1014,7 +1016,7 @@ extern "C" int yvex_hip_worklist_build(const uint64_t *selected, uint64_t pairs,
         !status || !pairs || !topk || !experts || experts > 256u || pairs % topk)
         return ST_INVALID_ARG;
     const uint64_t rows = pairs / topk;
-    if (rows > kWorklistMaxRows) return ST_BOUNDS;
+    if (rows > kWorklistMaxRows || pairs > kWorklistMaxPairs) return ST_BOUNDS;
     int with_below = 0;
     const size_t lds = worklist_lds_bytes(experts, rows, &with_below);
     YVEX_ALLOW_DYNAMIC_LDS(worklist_kernel, kWorklistLdsLimit);
@@ -1037,7 +1039,7 @@ extern "C" int yvex_hip_worklist_quantize(const uint64_t *selected, uint64_t pai
         !status || !pairs || !topk || !experts || experts > 256u || pairs % topk || !values || !encoded || !width || width % 256u)
         return ST_INVALID_ARG;
     const uint64_t rows = pairs / topk, tasks = rows * (width / 256u);
-    if (rows > kWorklistMaxRows || tasks > 0x7fffffffull) return ST_BOUNDS;
+    if (rows > kWorklistMaxRows || pairs > kWorklistMaxPairs || tasks > 0x7fffffffull) return ST_BOUNDS;
     int with_below = 0;
     size_t lds = worklist_lds_bytes(experts, rows, &with_below);
     if (lds > kWorklistLdsLimit) return ST_BOUNDS;
