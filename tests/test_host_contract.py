@@ -380,3 +380,16 @@ def test_worklists_of_more_pairs_than_their_kernels_count_are_refused(lib):
         lists = _worklist_arguments(pairs, pairs)
         assert lib.yvex_hip_worklist_build(*lists, _device(0x9000), None) == abi.BOUNDS
         assert lib.yvex_hip_worklist_quantize(*lists, _device(0xa000), C.c_uint64(256), _device(0xb000), _device(0x9000), None) == abi.BOUNDS
+
+
+def test_worklist_with_quantization_refuses_what_the_quantization_refuses(lib):
+    """Rows and blocks that do not lie on four bytes, and widths whose blocks are not counted."""
+    lists, status = _worklist_arguments(4096 * 8, 8), _device(0x9000)
+    for values, encoded in ((0x10001, 0x20000), (0x10002, 0x20000), (0x10000, 0x20002)):
+        assert lib.yvex_hip_q8k_quantize(_device(values), C.c_uint64(4096), C.c_uint64(512), C.c_uint64(512), _device(encoded),
+                                         status, None) == abi.INVALID_ARG
+        assert lib.yvex_hip_worklist_quantize(*lists, _device(values), C.c_uint64(512), _device(encoded), status,
+                                              None) == abi.INVALID_ARG
+    for width in (1 << 40, 1 << 63):
+        assert lib.yvex_hip_worklist_quantize(*lists, _device(0x10000), C.c_uint64(width), _device(0x20000), status,
+                                              None) == abi.BOUNDS

@@ -1036,10 +1036,11 @@ extern "C" int yvex_hip_worklist_quantize(const uint64_t *selected, uint64_t pai
                                           yvex_hip_stream stream)
 {
     if (!selected || !order || !expert_ids || !bucket_offsets || !bucket_populations || !sweep_offsets || !counts ||
-        !status || !pairs || !topk || !experts || experts > 256u || pairs % topk || !values || !encoded || !width || width % 256u)
+        !status || !pairs || !topk || !experts || experts > 256u || pairs % topk || !values || !encoded || !width || width % 256u ||
+        (((uintptr_t)values | (uintptr_t)encoded) & 3u))
         return ST_INVALID_ARG;
-    const uint64_t rows = pairs / topk, tasks = rows * (width / 256u);
-    if (rows > kWorklistMaxRows || pairs > kWorklistMaxPairs || tasks > 0x7fffffffull) return ST_BOUNDS;
+    const uint64_t rows = pairs / topk, blocks = width / 256u, tasks = rows * blocks;
+    if (rows > kWorklistMaxRows || pairs > kWorklistMaxPairs || blocks > 0x7fffffffull || tasks > 0x7fffffffull) return ST_BOUNDS;
     int with_below = 0;
     size_t lds = worklist_lds_bytes(experts, rows, &with_below);
     if (lds > kWorklistLdsLimit) return ST_BOUNDS;
