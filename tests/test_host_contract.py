@@ -393,3 +393,17 @@ def test_worklist_with_quantization_refuses_what_the_quantization_refuses(lib):
     for width in (1 << 40, 1 << 63):
         assert lib.yvex_hip_worklist_quantize(*lists, _device(0x10000), C.c_uint64(width), _device(0x20000), status,
                                               None) == abi.BOUNDS
+
+
+def test_long_matrices_of_few_pairs_are_not_refused_for_their_row_tiles(lib):
+    """2^29 rows of 256 columns by 20 pairs of eight experts (71 GB of weights, 43 GB of outputs) reach the launch."""
+    import torch
+    from yvex_amd.kernels import ExpertWeights
+    if torch.cuda.device_count():
+        pytest.skip("the call ends at the launch only where there is no device")
+    w = ExpertWeights(gate=0x10000, up=0x10000, gate_qtype=16, up_qtype=16, hidden=256, intermediate=1 << 29, gate_row_bytes=66,
+                      up_row_bytes=66, gate_expert_bytes=66 << 29, up_expert_bytes=66 << 29)
+    for pairs, code in ((20, abi.BACKEND), (1 << 20, abi.BOUNDS)):       # (more outputs than any card holds)
+        lists = [_device(0x2000 + 0x1000 * k) for k in range(5)]
+        assert lib.yvex_hip_moe_up_rows(C.byref(w), _device(0x1000), None, *lists, C.c_uint64(pairs), C.c_uint64(1), C.c_uint64(8),
+                                        C.c_double(10.0), _device(0x8000), _device(0x9000), None) == code

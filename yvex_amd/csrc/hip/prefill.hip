@@ -766,8 +766,11 @@ static int launch_mfma_variant(const MfmaArgs &a, hipStream_t stream)
 template <bool FUSED_UP>
 static int launch_mfma(const MfmaArgs &a, hipStream_t stream)
 {
-    // (the kernel counts row tiles in 32 bits; the outputs or the weights of so many are more than the card's memory)
-    const uint64_t token_tiles = a.pr.pairs / kTileTokens + (a.pr.expert_ids ? 256u : 1u);
+    // (the kernel counts row tiles in 32 bits: whole tiles and one behind them a bucket, of which there are no more than pairs. The
+    // outputs of so many are more than the card's memory)
+    uint64_t buckets = 1u;
+    if (a.pr.expert_ids) buckets = a.pr.experts < a.pr.pairs ? a.pr.experts : a.pr.pairs;
+    const uint64_t token_tiles = a.pr.pairs / kTileTokens + (buckets < 256u ? buckets : 256u);
     if (token_tiles * ((uint64_t)a.out_rows / (FUSED_UP ? 128u : 256u) + 1u) >= 1ull << 30) return ST_BOUNDS;
     return a.image ? launch_mfma_variant<FUSED_UP, true>(a, stream)
                    : launch_mfma_variant<FUSED_UP, false>(a, stream);
