@@ -663,6 +663,53 @@ def test_runs_of_row_tiles_agree_with_the_sweeps(gpu, oracle, hidden, intermedia
     assert same_bits(out[0], out[1]) and int(status.item()) == 0
 
 
+def packed_iq2(rows, width, seed, device):
+    """Random IQ2_XXS rows: any codes, small positive scales."""
+    gen = torch.Generator(device=device).manual_seed(seed)
+    raw = torch.empty((rows * width // 256, 66), dtype=torch.uint8, device=device).random_(generator=gen)
+    scale = torch.rand((raw.shape[0], 1), generator=gen, device=device).mul_(2.5e-4).add_(1e-4).to(torch.float16)
+    raw[:, :2] = scale.view(torch.uint8)
+    return raw.reshape(-1)
+
+
+# long tiles enough for some workgroups only, and for every one; the short ones (17 to 32 pairs, which the few-pair kernels
+# leave to this one) make up the difference; odd numbers of superblocks and row tiles
+@pytest.mark.parametrize("long_ones", [[64, 40, 128, 63, 200], [64, 33] * 12 + [128, 50] * 6], ids=["few", "many"])
+@pytest.mark.parametrize("image", [True, False], ids=["image", "canonical"])
+def test_short_tiles_fill_up_the_shares_of_long_ones(gpu, oracle, long_ones, image):
+    """The 64-pair IQ2_XXS kernel deals long and short tiles out separately where there are short ones enough: every pair's rows
+    come out once, the sweeps' bits."""
+    from yvex_amd import kernels as K
+    hidden, intermediate, qt = 2304, 1280, oracle.IQ2_XXS
+    populations = [n for pair in zip(long_ones + [0] * 48, [17 + k % 16 for k in range(48)]) for n in pair if n]
+    experts, pairs = len(populations), sum(populations)
+    grid = torch.cuda.get_device_properties(gpu).multi_processor_count
+    for out_rows, tile in ((intermediate, 128), (hidden, 256)):
+        tiles = out_rows // tile
+        wide = tiles * sum(n // 64 + (n % 64 > 32) for n in populations)
+        narrow = tiles * sum(17 <= n % 64 <= 32 for n in populations)
+        assert (4 * wide + 3 * narrow) // grid >= 4 * (wide // grid + 1), "long and short tiles are not dealt out separately here"
+    tensors = [packed_iq2(experts * r, w, 7 + k, gpu) for k, (r, w) in
+               enumerate(((intermediate, hidden), (intermediate, hidden), (hidden, intermediate)))]
+    weights = K.expert_weights(*tensors, (qt, qt, qt), hidden, intermediate)
+    rows_form = K.expert_weights_image(weights, hidden, intermediate) if image else weights
+    status, g = K.new_status(gpu), oracle.Generator(47, f"shares.{experts}")
+    selected = torch.repeat_interleave(torch.arange(experts), torch.tensor(populations))
+    selected = selected[torch.randperm(pairs, generator=torch.Generator().manual_seed(6))].reshape(pairs, 1).to(gpu)
+    wl = K.worklist_build(selected, experts, status)
+    route = dev((0.5 + np.abs(g.normal(pairs))).astype(np.float32), gpu)
+    act = K.q8k_quantize(dev(g.normal(pairs * hidden).reshape(pairs, hidden), gpu), status)
+    mid = [torch.full((pairs, intermediate), float("nan"), device=gpu) for _ in range(2)]
+    K.moe_up(weights, act, True, route, wl, pairs, 1, experts, 10.0, mid[0], status)
+    K.moe_up_rows(rows_form, act, route, wl, pairs, 1, experts, 10.0, mid[1], status)
+    assert bool(torch.isfinite(mid[0]).all()) and same_bits(mid[0], mid[1])
+    mid_q8 = K.q8k_quantize(mid[0], status)
+    out = [torch.full((pairs, hidden), float("nan"), device=gpu) for _ in range(2)]
+    K.moe_down(weights, mid_q8, True, wl, pairs, experts, out[0], status)
+    K.moe_down_rows(rows_form, mid_q8, wl, pairs, experts, out[1], status)
+    assert bool(torch.isfinite(out[0]).all()) and same_bits(out[0], out[1]) and int(status.item()) == 0
+
+
 # a last row tile of four rows and of 252, one superblock and an odd number of them
 @pytest.mark.parametrize("rows,width,inputs", [(4100, 1280, 2048), (7164, 256, 1025)])
 def test_ragged_row_tiles_run_alone(gpu, oracle, rows, width, inputs):
