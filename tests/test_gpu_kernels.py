@@ -942,3 +942,20 @@ def test_bfloat16_rounding_of_every_upper_half(gpu):
             ctypes.c_uint64(half), ctypes.c_uint64(half), K._ptr(out), K._ptr(status), K._stream())
     assert np.array_equal(out.cpu().numpy().view(np.uint32), want)
     assert int(status.item()) == 1          # (infinities and NaNs are among them)
+
+
+def test_bfloat16_rounding_of_every_pattern(gpu):
+    """All 2^32 patterns, against the integer rounding (kernel_primitives.h:89-99) on the device."""
+    import ctypes
+    from yvex_amd import kernels as K
+    count, status = 1 << 27, K.new_status(gpu)
+    low = torch.arange(count, dtype=torch.int32, device=gpu)
+    out = torch.empty_like(low)
+    for high in range(32):
+        values = low + (high * count if high < 16 else high * count - (1 << 32))
+        K._call("yvex_hip_concat_rows_bf16", K._ptr(values[:count // 2]), K._ptr(values[count // 2:]), ctypes.c_uint64(1),
+                ctypes.c_uint64(count // 2), ctypes.c_uint64(count // 2), K._ptr(out), K._ptr(status), K._stream())
+        nan = (values & 0x7fffffff) > 0x7f800000
+        want = (values + 0x7fff + ((values >> 16) & 1)) & -0x10000
+        want = torch.where(nan, (values & -0x10000) | 0x400000, want)
+        assert torch.equal(out, want), f"patterns from {high * count:#x}"
