@@ -1,8 +1,8 @@
 // Row-batch (prefill-width) grouped expert projections on the int8 matrix cores of gfx950.
 //
-// A work item is (bucket, tile of up to 64 ordered pairs, tile of 256 weight rows: 128 gate rows
-// and the 128 matching up rows when the SwiGLU is fused). The workgroup has eight waves, two per
-// SIMD; each owns 32 weight rows and multiplies them by all of the item's Q8_K activation rows
+// A workgroup walks runs: one token tile (up to 64 ordered pairs of a bucket) against row tiles of 256 weight rows (128 gate rows
+// and the 128 matching up rows when the SwiGLU is fused), one after another. It has eight waves, two per
+// SIMD; each owns 32 weight rows of a row tile and multiplies them by all of the token tile's Q8_K activation rows
 // with V_MFMA_I32_32X32X32_I8. 256 registers a wave are what decides the tile: 32 rows x 64 tokens of int32
 // limb sums and double-precision row sums.
 //
@@ -399,7 +399,7 @@ __device__ __forceinline__ void rows_run(const MfmaArgs &a, const MfmaRun &it)
     // the rest at the start of the next one, so rounds -(R - 1) .. -1 are issued here (windows 0 and 1 are needed before
     // them; a round before -1 has three copies to where nobody reads in the place of a window, which keeps the counts below the same for
     // every step).
-    lds_barrier();     // every wave is done with the previous run's stages and pair records (its stores may still be on their way)
+    lds_barrier();     // every wave is done with the previous run's stages and pair records (whose copies and stores have all completed: see its end)
 #pragma unroll
     for (unsigned k = 0; k < 3u; ++k) weight_piece(k);
 #pragma unroll
@@ -553,14 +553,12 @@ __device__ __forceinline__ void rows_run(const MfmaArgs &a, const MfmaRun &it)
     // The values go from the registers straight to memory, 16 bytes a lane: the two halves of a
     // wave complete 32 bytes of a token's row per store, the four (two) stores of a token block
     // a whole cache line (half of one), which the L2 merges before it writes them back. No LDS,
-    // no barrier: the stores drain while the next tile is worked on; copies past the run's end that are
-    // still in flight land in stages and windows nobody reads before the next run has waited
-    // for copies of its own, which the same wave issues later to the same places.
+    // no barrier: the stores drain while the next row tile is worked on, those of a run's last one before the run ends.
     bool bad = false;
 #pragma unroll
     for (unsigned tb = 0; tb < NTB; ++tb) {
         const unsigned token = tb * 32u + r;
-        const uint2 info = lds_read_uint2(kPairInfoBase + token * 8u);   // (stale past the item's last token: not used)
+        const uint2 info = lds_read_uint2(kPairInfoBase + token * 8u);   // (stale past the run's last token: not used)
         float *const out_row = pr.out + (unsigned long long)info.x * a.out_rows;
 #pragma unroll
         for (unsigned q = 0; q < (FUSED_UP ? 2u : 4u); ++q) {
@@ -601,8 +599,9 @@ __device__ __forceinline__ void rows_run(const MfmaArgs &a, const MfmaRun &it)
     }
     if (bad) raise_status(a.status, 1);
     }
-    // (a run with another number of token blocks lays its stages out differently, so that its copies come from other waves
-    // than this run's to the same bytes: all have landed here, and the next run's opening barrier makes that hold for every wave)
+    // Every run ends with all of its copies landed and all of its stores complete, whatever the next one looks like. A run with another
+    // number of token blocks needs the former: it lays its stages out differently, so that its copies come from other waves than this run's
+    // to the same bytes; the next run's opening barrier makes it hold for every wave.
     __builtin_amdgcn_s_waitcnt(0x0070u);   // vmcnt(0)
 }
 
