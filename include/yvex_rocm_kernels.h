@@ -194,7 +194,7 @@ int yvex_hip_worklist_build(const uint64_t *selected, uint64_t pairs, uint64_t t
                             uint64_t *sweep_offsets, uint64_t *counts, int *status,
                             yvex_hip_stream stream);
 /* yvex_hip_worklist_build and yvex_hip_q8k_quantize of the pairs / topk input rows, which lie end to end, in one launch: the
- * same words and blocks. For large batches; a small one's are yvex_hip_moe_prepare_routed's. */
+ * same words and blocks. For batches of more rows than yvex_hip_moe_prepare_routed takes. */
 int yvex_hip_worklist_quantize(const uint64_t *selected, uint64_t pairs, uint64_t topk, uint64_t experts,
                                uint64_t *order, uint64_t *expert_ids, uint64_t *bucket_offsets,
                                uint64_t *bucket_populations, uint64_t *sweep_offsets, uint64_t *counts,
@@ -240,7 +240,8 @@ int yvex_hip_moe_prepare_scored(const float *scores, const float *bias, uint64_t
                                 yvex_hip_stream stream);
 
 /* yvex_hip_moe_prepare for rows that are routed already (yvex_hip_matvec_f32_rows_routed): the
- * worklist and the quantization. rows <= 512. */
+ * worklist and the quantization. rows <= YVEX_HIP_PREPARE_ROUTED_MAX_ROWS. */
+#define YVEX_HIP_PREPARE_ROUTED_MAX_ROWS 512u
 int yvex_hip_moe_prepare_routed(const uint64_t *selected, uint64_t rows, uint64_t experts, uint64_t topk,
                                 uint64_t *order, uint64_t *expert_ids, uint64_t *bucket_offsets,
                                 uint64_t *bucket_populations, uint64_t *sweep_offsets, uint64_t *counts,

@@ -376,7 +376,7 @@ __global__ __launch_bounds__(1024) void worklist_quantize_kernel(
 constexpr unsigned kPrepareMaxRows = 128u;
 // Rows that are routed already leave the worklist: as long as its bitmap is small enough for the
 // quantizing workgroups, which get the same LDS, to share a compute unit.
-constexpr unsigned kPrepareMaxRoutedRows = 512u;
+constexpr unsigned kPrepareMaxRoutedRows = YVEX_HIP_PREPARE_ROUTED_MAX_ROWS;
 
 // T: a decode batch of one or two rows whose shared expert holds Q8_0 matrices takes their products with the input rows
 // along (the workgroups behind those that quantize): the routing that the launch waits for occupies one workgroup. One

@@ -863,7 +863,7 @@ sequence:
                                           YVEX_MOE_WEIGHT_FFN_NORM};
         void *flat_targets[3];
         unsigned long long need = 0ull;
-        int k, fused_coefficients = 1, lend, split, joined;
+        int k, fused_coefficients = 1, lend, split, projecting;
         flat_targets[0] = AT(scale);
         flat_targets[1] = AT(base);
         flat_targets[2] = AT(norm);
@@ -887,8 +887,8 @@ sequence:
         /* the ingress adds the partial sums itself, a launch less. A batch whose intermediate rows come back to the host needs
          * none of it in memory here (at the egress it does), but waits for its copies anyway, and keeps one launch a
          * stage, which its callers count */
-        joined = split && fused_coefficients && !host_rows;
-        if (joined) {
+        projecting = split && fused_coefficients && !host_rows;
+        if (projecting) {
             LAUNCH(yvex_hip_mhc_ingress_projecting((const float *)rows->device_rows->data,
                                                    (const float *)(uintptr_t)envelope_addresses[0],
                                                    (const void *)(uintptr_t)envelope_addresses[1],
@@ -917,7 +917,7 @@ sequence:
                                rows->device_rows->data, 0, row_count, expanded, NULL,
                                (float *)AT(mixes), layer->mhc_mixing_rows, 0, (int *)status, stream),
                "rocm.moe.rows.mhc-function");
-        if (fused_coefficients && !joined)
+        if (fused_coefficients && !projecting)
             LAUNCH(yvex_hip_mhc_ingress_encoded((const float *)rows->device_rows->data, (const float *)AT(mixes),
                                                 (const void *)(uintptr_t)envelope_addresses[1],
                                                 views[flat_slots[0]].qtype,
@@ -930,7 +930,7 @@ sequence:
                                                 (float *)AT(normalized), (float *)AT(post),
                                                 (float *)AT(combination), (int *)status, stream),
                    "rocm.moe.rows.mhc-ingress");
-        else if (!joined) {
+        else if (!projecting) {
         for (k = 0; k < 3; ++k)
             LAUNCH(yvex_hip_gather((const uint8_t *)(uintptr_t)envelope_addresses[1 + k],
                                    views[flat_slots[k]].qtype, 1ull, views[flat_slots[k]].row_width,
@@ -1015,7 +1015,7 @@ sequence:
                              yvex_hip_moe_prepare_projecting_supported(&shared_pair, row_count, hidden) &&
                              yvex_hip_q8k_quantize_swiglu_projecting_supported(
                                  shared.down, hidden, shared.down_row_bytes, row_count, layer->shared_intermediate_width);
-    if (routed_rows && row_count <= 512ull) {
+    if (routed_rows && row_count <= YVEX_HIP_PREPARE_ROUTED_MAX_ROWS) {
         LAUNCH(yvex_hip_moe_prepare_routed((const uint64_t *)AT(selected), row_count, experts, topk,
                                            (uint64_t *)AT(order), (uint64_t *)AT(expert_ids),
                                            (uint64_t *)AT(bucket_offsets), (uint64_t *)AT(bucket_populations),
@@ -1052,7 +1052,7 @@ sequence:
                                            layer->routed_scaling_factor, (uint64_t *)AT(selected),
                                            (float *)AT(weights), (int *)status, stream),
                    "rocm.moe.rows.route");
-        if (need_q8 && row_count > 512ull)
+        if (need_q8 && row_count > YVEX_HIP_PREPARE_ROUTED_MAX_ROWS)
             LAUNCH(yvex_hip_worklist_quantize((const uint64_t *)AT(selected), pairs, topk, experts, (uint64_t *)AT(order),
                                               (uint64_t *)AT(expert_ids), (uint64_t *)AT(bucket_offsets),
                                               (uint64_t *)AT(bucket_populations), (uint64_t *)AT(sweep_offsets),
