@@ -6,12 +6,14 @@
 // with V_MFMA_I32_32X32X32_I8. 256 registers a wave are what decides the tile: 32 rows x 64 tokens of int32
 // limb sums and double-precision row sums.
 //
-// What bounds it is not the matrix pipe: vector instructions run under matrix instructions, a wave's own among them (one
-// 32 x 32 x 32 instruction and k byte permutes take max(32, 8 + 4.5 k) cycles with two waves a SIMD), and without its
-// matrix instructions a launch takes as many cycles. It is the issue of everything else, about five cycles a vector or LDS
+// What bounds it is not the matrix pipe: with two waves a SIMD vector instructions run under matrix instructions (a 32 x 32 x 32
+// instruction and k byte permutes take a SIMD max(33, 9 + 4.5 k) cycles), and without its
+// matrix instructions a launch takes as many cycles. A wave alone on its SIMD hides up to seven permutes under its own matrix
+// instruction (46 cycles) and from eight on none (41 + 4.5 k: 77 of eight, 95 of twelve); this loop has 9.6 vector instructions for
+// each, and would have 7.4 with 128 tokens a wave. It is the issue of everything else, about five cycles a vector or LDS
 // instruction and forty a window copy, and the matrix instructions' power: 1.9 to 2.0 GHz under this kernel, 2.2 without
 // them. The wave's number is kept scalar, and with it every LDS address of a copy and every distance it adds to its
-// lanes' pointers (333 -> 315 vector instructions a superblock: 7168 x 2 x 4096 by 2048 rows 317 -> 301 us, 2048 x 8192 by 2048 122.2 -> 119.4).
+// lanes' pointers (330 -> 318 vector instructions a superblock: 7168 x 2 x 4096 by 2048 rows 317 -> 301 us, 2048 x 8192 by 2048 122.2 -> 119.4).
 // Two things that look the same and are slower: stages with sixteen bytes between groups of tokens, which make the fragments' places
 // immediate offsets (a copy into LDS that does not start on 64 bytes is split: 582K cycles against 570K), and windows without their
 // spare pieces (64 scattered dwords cost a copy more than 64 pieces of sixteen bytes: 600K against 590K).

@@ -80,7 +80,7 @@ __device__ __forceinline__ unsigned row_max_u32(unsigned v)
 // * A code is the low byte of 1.5 * 2^23 + inverse * v, whose addition rounds as a conversion to the nearest does (a
 //   magnitude whose inverse is not finite takes conversions and clamps); V_DOT4 adds a lane's codes.
 // us a launch, a block a wavefront and four: 2048 x 4096 values 10.4 and 6.5, 2048 x 7168 16.5 and 12.5, 16 384 x 2048 33.3 and 25.5
-// (6.8 TB/s), 333 x 4096 3.5 and 2.8, 19 x 7168 2.49 and 2.46, one row of 4096 2.5 and 2.2.
+// (6.8 TB/s; the 18 432 x 2048 of a long batch's layer, part of them out of the caches again, 32: 6.1), 333 x 4096 3.5 and 2.8, 19 x 7168 2.49 and 2.46, one row of 4096 2.5 and 2.2.
 __device__ __forceinline__ void q8k_quantize_four(const float (&v)[4][4], unsigned char *__restrict__ out, unsigned lane,
                                                   bool live, int *status)
 {

@@ -89,8 +89,8 @@ constexpr unsigned kResultBytes = 2u * 4u * kFusedItemRows * 4u;
 // Behind them, for each of the sweep's pairs, {the row its results go to, its route weight}. A chunk's end finds them there by
 // the pair: kept in registers through the loop they were what the compiler spilled, and scratch loads wait for the weight
 // rows asked for ahead as well. With swiglu_bf16's exponential out of the loop's registers too, experts of one
-// pair over the image, gate and up of 7168 x 2048: 40 of them 82.5 -> 75.8 us, 168 of them 300 -> 290; 94 of one pair, 47 of
-// two, 16 of three and 3 of four, down: 163 -> 151.
+// pair over the image, gate and up of 7168 x 2048: 40 of them 80 -> 73 us, 168 of them 285 -> 281 (265 to 310 and 257 to 318 by
+// where the experts lie); 94 of one pair, 47 of two, 16 of three and 3 of four, down: 137 -> 134.
 constexpr unsigned kInfoOffset = kWindowBytes + kResultBytes, kInfoBytes = 4u * 8u;
 constexpr unsigned kParkBytes = kInfoOffset + kInfoBytes;
 constexpr unsigned kMaxSweeps = 4096u;
